@@ -262,6 +262,29 @@ def load():
     return lib
 
 
+_host = None
+
+
+def host():
+    """The native host path (chainer_amd/_host.so: arrays, buffers, hot routines), loaded behind the kernel library it calls.  Raises
+    if it has not been built."""
+    global _host
+    if _host is None:
+        load()
+        try:
+            from chainer_amd import _host as module
+        except ImportError as e:
+            raise ImportError('chainer_amd/_host.so is missing or does not load (%s): build it with `make -C chainer_amd/csrc` '
+                              '(or __graft_entry__.build()); there is no fallback path.' % e)
+        module.setup({'exceptions': [None] + [_STATUS_TO_EXC[i] for i in range(1, 9)], 'make_cdesc': _copy_desc, 'byref': ctypes.byref})
+        _host = module
+    return _host
+
+
+def _copy_desc(address):
+    return CArray.from_buffer_copy(CArray.from_address(address))
+
+
 def check(status):
     if status != 0:
         msg = load().hipcx_last_error().decode('utf-8', 'replace')

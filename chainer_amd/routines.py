@@ -10,39 +10,27 @@ import ctypes
 
 import numpy
 
-from chainer_amd import _lib
-from chainer_amd._array import (ndarray, array, current_stream, alloc_bytes, _normalize_axis, _as_shape, _prod,
+from chainer_amd import _array, _lib
+from chainer_amd._array import (ndarray, array, current_stream, alloc_bytes, _normalize_axis, _prod,
                                 contiguous_strides)
+
+_host = _array._host
+
+# The routines a network issues per layer are native (csrc/python/routines.cc): the host work of a call is what bounds them on
+# small arrays.
+from chainer_amd._host import (promote_types, result_type, full, split, concatenate, stack, add, negative, subtract, multiply, divide,  # noqa: E402,F401
+                               reciprocal, exp, log, tanh, sqrt, sigmoid, relu, if_less_else, if_greater_else, maximum, equal, not_equal,
+                               greater, greater_equal, sum, amax, amin, argmax, argmin, dot, linear, conv, conv_bn_act, fixed_batch_norm,
+                               max_pool, average_pool)
 
 # ---------------------------------------------------------------------------------------------
 # dtype rules (CX/dtype.cc:12-60, CX/routines/type_util.cc:11-46)
 # ---------------------------------------------------------------------------------------------
 _KIND = {'b': 0, 'i': 1, 'u': 2, 'f': 3}
-_CATEGORY = {0: 0, 1: 1, 2: 1, 3: 2}  # bool < int/uint < float
 
 
 def _kind(dtype):
     return _KIND[numpy.dtype(dtype).kind]
-
-
-def promote_types(dt1, dt2):
-    dt1, dt2 = numpy.dtype(dt1), numpy.dtype(dt2)
-    k1, k2 = _kind(dt1), _kind(dt2)
-    if k1 == 0:
-        return dt2
-    if k2 == 0:
-        return dt1
-    if k1 == k2:
-        return dt1 if dt1.itemsize >= dt2.itemsize else dt2
-    if k1 == 3:
-        return dt1
-    if k2 == 3:
-        return dt2
-    if k1 == 2:
-        dt1, dt2 = dt2, dt1
-    if dt1.itemsize > dt2.itemsize:
-        return dt1
-    return numpy.dtype('int16')  # signed one level wider than uint8
 
 
 def _scalar_default_dtype(value):
@@ -51,23 +39,6 @@ def _scalar_default_dtype(value):
     if isinstance(value, (int, numpy.integer)):
         return numpy.dtype('int32')
     return numpy.dtype('float32')
-
-
-def result_type(*args):
-    """ResultType over arrays and Python scalars: scalars only matter if of a higher category."""
-    arr_dt = None
-    sc_dt = None
-    for a in args:
-        if isinstance(a, ndarray):
-            arr_dt = a.dtype if arr_dt is None else promote_types(arr_dt, a.dtype)
-        else:
-            d = _scalar_default_dtype(a)
-            sc_dt = d if sc_dt is None else promote_types(sc_dt, d)
-    if arr_dt is not None:
-        if sc_dt is not None and _CATEGORY[_kind(sc_dt)] > _CATEGORY[_kind(arr_dt)]:
-            return sc_dt
-        return arr_dt
-    return sc_dt
 
 
 def _math_result_dtype(dtype):
@@ -87,14 +58,6 @@ def empty(shape, dtype='float32'):
 
 def empty_like(a):
     return ndarray.empty(a.shape, a.dtype)
-
-
-def full(shape, value, dtype=None):
-    if dtype is None:
-        dtype = _scalar_default_dtype(value)
-    out = ndarray.empty(shape, dtype)
-    out.fill(value)
-    return out
 
 
 def zeros(shape, dtype='float32'):
@@ -230,57 +193,6 @@ def squeeze(a, axis=None):
     return a.squeeze(axis)
 
 
-def split(a, indices_or_sections, axis=0):
-    """Split into views (CX/routines/manipulation.cc Split)."""
-    axis = _normalize_axis(axis, a.ndim)
-    dim = a.shape[axis]
-    if isinstance(indices_or_sections, (int, numpy.integer)):
-        n = int(indices_or_sections)
-        if n <= 0 or dim % n != 0:
-            raise _lib.DimensionError('array split does not result in an equal division')
-        step = dim // n
-        bounds = [(i * step, (i + 1) * step) for i in range(n)]
-    else:
-        idx = [_py.min(_py.max(int(i), 0), dim) for i in indices_or_sections]
-        starts = [0] + idx
-        stops = idx + [dim]
-        bounds = [(s, _py.max(s, e)) for s, e in zip(starts, stops)]
-    out = []
-    for s, e in bounds:
-        key = [slice(None)] * a.ndim
-        key[axis] = slice(s, e)
-        out.append(a[tuple(key)])
-    return out
-
-
-def concatenate(arrays, axis=0):
-    """Concatenate = Empty + one CopyKernel per input (CX/routines/manipulation.cc:415-460)."""
-    arrays = list(arrays)
-    if not arrays:
-        raise _lib.DimensionError('Need at least one array to concatenate')
-    axis = _normalize_axis(axis, arrays[0].ndim)
-    dtype = arrays[0].dtype
-    shape = list(arrays[0].shape)
-    total = 0
-    for a in arrays:
-        if a.ndim != len(shape):
-            raise _lib.DimensionError('all the input arrays must have same number of dimensions')
-        for i in range(a.ndim):
-            if i != axis and a.shape[i] != shape[i]:
-                raise _lib.DimensionError('all the input array dimensions except for the concatenation axis must match exactly')
-        total += a.shape[axis]
-        dtype = promote_types(dtype, a.dtype)
-    shape[axis] = total
-    out = ndarray.empty(shape, dtype)
-    pos = 0
-    for a in arrays:
-        key = [slice(None)] * out.ndim
-        key[axis] = slice(pos, pos + a.shape[axis])
-        _lib.call('hipcx_copy', a.desc(), out[tuple(key)].desc(), current_stream())
-        pos += a.shape[axis]
-    return out
-
-
 # ---------------------------------------------------------------------------------------------
 # elementwise
 # ---------------------------------------------------------------------------------------------
@@ -337,168 +249,12 @@ def _binary_as(kernel, x1, scalar, dtype, out=None):
     return out
 
 
-def add(x1, x2, out=None):
-    if _is_scalar(x2):
-        return _binary_as('hipcx_add_as', x1, x2, result_type(x1, x2), out)
-    if _is_scalar(x1):
-        return _binary_as('hipcx_add_as', x2, x1, result_type(x1, x2), out)
-    return _binary('hipcx_add', x1, x2, result_type(x1, x2), out)
-
-
-def negative(x):
-    """Negative = Multiply(x, Scalar{-1}) (CX/routines/arithmetic.cc)."""
-    if x.dtype == numpy.dtype('bool'):
-        raise _lib.DtypeError('Cannot negate a boolean array.')
-    return _binary_as('hipcx_multiply_as', x, -1, x.dtype)
-
-
-def subtract(x1, x2, out=None):
-    dt = result_type(x1, x2)
-    if _kind(dt) == 0:
-        raise _lib.DtypeError('Boolean arguments are not supported in subtract.')
-    if _is_scalar(x2):
-        return _binary_as('hipcx_subtract_as', x1, x2, dt, out)
-    if _is_scalar(x1):
-        # Subtract(Scalar, Array) = Add(-Array, Scalar) (CX/routines/arithmetic.cc)
-        return add(negative(x2), x1)
-    return _binary('hipcx_subtract', x1, x2, dt, out)
-
-
-def multiply(x1, x2, out=None):
-    if _is_scalar(x2):
-        return _binary_as('hipcx_multiply_as', x1, x2, result_type(x1, x2), out)
-    if _is_scalar(x1):
-        return _binary_as('hipcx_multiply_as', x2, x1, result_type(x1, x2), out)
-    return _binary('hipcx_multiply', x1, x2, result_type(x1, x2), out)
-
-
-def _true_divide_dtype(*args):
-    dt = result_type(*args)
-    return dt if _kind(dt) == 3 else numpy.dtype('float32')
-
-
-def divide(x1, x2, out=None):
-    """TrueDivide: integer operands are computed in float32 (CX/routines/arithmetic.cc Divide)."""
-    dt = _true_divide_dtype(x1, x2)
-    if _is_scalar(x2):
-        return _binary_as('hipcx_divide_as', x1, x2, dt, out)
-    if _is_scalar(x1):
-        if out is None:
-            out = ndarray.empty(x2.shape, dt)
-        _lib.call('hipcx_divide_sa', _lib.make_scalar(x1), x2.astype(out.dtype, False).desc(), out.desc(), current_stream())
-        return out
-    return _binary('hipcx_divide', x1, x2, dt, out)
-
-
-def reciprocal(x):
-    """Reciprocal(x) = Scalar{1} / x (CX/routines/arithmetic.cc)."""
-    return divide(1, x)
-
-
-def _unary_math(kernel, x):
-    dt = _math_result_dtype(x.dtype)
-    xc = x.astype(dt, False)
-    out = ndarray.empty(x.shape, dt)
-    _lib.call(kernel, xc.desc(), out.desc(), current_stream())
-    return out
-
-
-def exp(x):
-    return _unary_math('hipcx_exp', x)
-
-
-def log(x):
-    return _unary_math('hipcx_log', x)
-
-
-def tanh(x):
-    return _unary_math('hipcx_tanh', x)
-
-
-def sqrt(x):
-    return _unary_math('hipcx_sqrt', x)
-
-
-def if_less_else(x1, x2, pos, neg):
-    """x1 < x2 ? pos : neg with scalar x2/pos (CX/routines/misc.cc:34-58)."""
-    dt = result_type(pos, neg)
-    out = _empty_for(x1, x1.shape, dt)
-    _lib.call('hipcx_if_less_else_assa', x1.astype(dt, False).desc(), _lib.make_scalar(x2), _lib.make_scalar(pos),
-              neg.astype(dt, False).desc(), out.desc(), current_stream())
-    return out
-
-
-def if_greater_else(x1, x2, pos, neg):
-    dt = result_type(pos, neg)
-    out = ndarray.empty(x1.shape, dt)
-    _lib.call('hipcx_if_greater_else_assa', x1.astype(dt, False).desc(), _lib.make_scalar(x2), _lib.make_scalar(pos),
-              neg.astype(dt, False).desc(), out.desc(), current_stream())
-    return out
-
-
-def maximum(x1, x2):
-    """Maximum(array, scalar) = IfLessElse(x1, x2, x2, x1) (CX/routines/misc.cc:210-216)."""
-    if _is_scalar(x1):
-        x1, x2 = x2, x1
-    if _is_scalar(x2):
-        return if_less_else(x1, x2, x2, x1)
-    dt = result_type(x1, x2)
-    shape = _broadcast_shape(x1.shape, x2.shape)
-    a = x1.broadcast_to(shape).astype(dt, False)
-    b = x2.broadcast_to(shape).astype(dt, False)
-    out = ndarray.empty(shape, dt)
-    # MaximumImpl: x1 > x2 ? x1 : x2 (CX/routines/misc.cc)
-    _lib.call('hipcx_if_greater_else_aaaa', a.desc(), b.desc(), a.desc(), b.desc(), out.desc(), current_stream())
-    return out
-
-
 def minimum(x1, x2):
     if _is_scalar(x1):
         x1, x2 = x2, x1
     if _is_scalar(x2):
         return if_greater_else(x1, x2, x2, x1)
     raise _lib.ChainerxNotImplementedError('minimum(array, array) is not on the supported path')
-
-
-def relu(x):
-    """Relu(x) = Maximum(0, x) in the math dtype of x (CX/routines/activation.cc:80-84)."""
-    return maximum(x.astype(_math_result_dtype(x.dtype), False), 0)
-
-
-def sigmoid(x):
-    """Sigmoid(x) = Reciprocal(1 + Exp(-x)): four kernels (CX/routines/activation.cc:74-78)."""
-    xc = x.astype(_math_result_dtype(x.dtype), False)
-    return reciprocal(add(exp(negative(xc)), 1))
-
-
-def _compare(kernel, x1, x2):
-    if _is_scalar(x2):
-        x2 = full((), x2, x1.dtype)
-    if (_kind(x1.dtype) == 0) != (_kind(x2.dtype) == 0):
-        raise _lib.DtypeError('Comparison of bool and non-bool dtypes is not supported.')
-    dt = promote_types(x1.dtype, x2.dtype)
-    shape = _broadcast_shape(x1.shape, x2.shape)
-    a = x1.broadcast_to(shape).astype(dt, False)
-    b = x2.broadcast_to(shape).astype(dt, False)
-    out = ndarray.empty(shape, 'bool')
-    _lib.call(kernel, a.desc(), b.desc(), out.desc(), current_stream())
-    return out
-
-
-def equal(x1, x2):
-    return _compare('hipcx_equal', x1, x2)
-
-
-def not_equal(x1, x2):
-    return _compare('hipcx_not_equal', x1, x2)
-
-
-def greater(x1, x2):
-    return _compare('hipcx_greater', x1, x2)
-
-
-def greater_equal(x1, x2):
-    return _compare('hipcx_greater_equal', x1, x2)
 
 
 def less(x1, x2):
@@ -844,59 +600,10 @@ def _reduce(kernel, a, axes, out):
     return out
 
 
-def sum(a, axis=None, keepdims=False):
-    """Sum (CX/routines/reduction.cc:28-76): bool/int inputs accumulate and return int64."""
-    axes = _sorted_axes(axis, a.ndim)
-    k = _kind(a.dtype)
-    out_dtype = numpy.dtype('int64') if k in (0, 1, 2) else a.dtype
-    out = _reduced_out(a, axes, keepdims, out_dtype)
-    return _reduce('hipcx_sum', a, axes, out)
-
-
-def amax(a, axis=None, keepdims=False):
-    """AMax (CX/routines/statistics.cc:21-65)."""
-    axes = _sorted_axes(axis, a.ndim)
-    for i in axes:
-        if a.shape[i] == 0:
-            raise _lib.DimensionError('cannot compute the maximum along zero-sized axis')
-    out = _reduced_out(a, axes, keepdims, a.dtype)
-    return _reduce('hipcx_amax', a, axes, out)
-
-
 max = amax
 
 
-def argmax(a, axis=None):
-    """ArgMax (CX/routines/sorting.cc:21-52): int64 result, no keepdims."""
-    axes = _sorted_axes(axis, a.ndim)
-    for i in axes:
-        if a.shape[i] == 0:
-            raise _lib.DimensionError('cannot compute ArgMax for an empty array')
-    out = ndarray.empty([d for i, d in enumerate(a.shape) if i not in axes], 'int64')
-    return _reduce('hipcx_argmax', a, axes, out)
-
-
-def amin(a, axis=None, keepdims=False):
-    """AMin (CX/routines/statistics.cc:66-79)."""
-    axes = _sorted_axes(axis, a.ndim)
-    for i in axes:
-        if a.shape[i] == 0:
-            raise _lib.DimensionError('cannot compute the minimum along zero-sized axis')
-    out = _reduced_out(a, axes, keepdims, a.dtype)
-    return _reduce('hipcx_amin', a, axes, out)
-
-
 min = amin
-
-
-def argmin(a, axis=None):
-    """ArgMin (CX/routines/sorting.cc:54-85): int64 result, no keepdims."""
-    axes = _sorted_axes(axis, a.ndim)
-    for i in axes:
-        if a.shape[i] == 0:
-            raise _lib.DimensionError('cannot compute ArgMin for an empty array')
-    out = ndarray.empty([d for i, d in enumerate(a.shape) if i not in axes], 'int64')
-    return _reduce('hipcx_argmin', a, axes, out)
 
 
 def nanargmax(a, axis=None):
@@ -972,17 +679,8 @@ def log_softmax(x, axis=None):
 def log_softmax_fused(x, axis=None):
     """Opt-in: LogSoftmax (CX/routines/reduction.cc:88-92) through hipcx_log_softmax -- one or two kernels instead of seven.
     Arrays the fused kernel does not take (ndim != 2, another axis, strided rows) go through log_softmax."""
-    xc = x.astype(_math_result_dtype(x.dtype), False)
-    ax = 1 if axis is None else axis
-    axes = _sorted_axes(ax, x.ndim)
-    it = xc.dtype.itemsize
-    if xc.ndim != 2 or axes != (1,) or (xc.shape[1] > 1 and xc.strides[1] != it) or xc.strides[0] < 0:
-        return log_softmax(x, axis)
-    out = ndarray.empty(xc.shape, xc.dtype)
-    nbytes = _lib.load().hipcx_log_softmax_workspace_size(xc.desc())
-    ws, wsp = _workspace(nbytes)
-    _lib.call('hipcx_log_softmax', xc.desc(), out.desc(), wsp, nbytes, current_stream())
-    return out
+    out = _host.log_softmax_direct(x, axis)
+    return log_softmax(x, axis) if out is None else out
 
 
 def softmax(x, axis=None):
@@ -1003,51 +701,6 @@ def _workspace(nbytes):
         return None, ctypes.c_void_p(0)
     ws = alloc_bytes(nbytes)
     return ws, ctypes.c_void_p(ws.data_ptr())
-
-
-def dot(a, b, out_dtype=None):
-    """Dot for 2-D operands (CX/routines/linalg.cc:27-100): k == 0 gives zeros without a kernel."""
-    if a.ndim != 2 or b.ndim != 2:
-        raise _lib.DimensionError('ChainerX dot supports only 2-dimensional arrays.')
-    if a.shape[1] != b.shape[0]:
-        raise _lib.DimensionError('Axis dimension mismatch')
-    dt = numpy.dtype(out_dtype) if out_dtype is not None else result_type(a, b)
-    m, k, n = a.shape[0], a.shape[1], b.shape[1]
-    if k == 0:
-        return zeros((m, n), dt)
-    out = ndarray.empty((m, n), dt)
-    _dot_into(a.astype(dt, False), b.astype(dt, False), out)
-    return out
-
-
-def _dot_into(a, b, out):
-    nbytes = _lib.load().hipcx_dot_workspace_size(a.desc(), b.desc(), out.desc())
-    ws, wsp = _workspace(nbytes)
-    _lib.call('hipcx_dot', a.desc(), b.desc(), out.desc(), wsp, nbytes, current_stream())
-
-
-def linear(x, w, b=None, n_batch_axes=1):
-    """Linear (CX/routines/connection.cc:322-394): DotKernel(x, w.T view) then AddKernel with a stride-0 bias."""
-    if w.ndim != 2:
-        raise _lib.DimensionError('w.ndim should be 2')
-    if b is not None and b.ndim != 1:
-        raise _lib.DimensionError('b.ndim should be 1')
-    n_batch_axes = _normalize_axis(n_batch_axes, x.ndim) if x.ndim > 0 else 0
-    dt = result_type(x, w, b) if b is not None else result_type(x, w)
-    out_dim = _prod(x.shape[:n_batch_axes])
-    m_dim, n_dim = w.shape
-    out_shape = tuple(x.shape[:n_batch_axes]) + (m_dim,)
-    if m_dim == 0 or n_dim == 0:
-        if b is not None:
-            return b.astype(dt, False).broadcast_to(out_shape)
-        return zeros(out_shape, dt)
-    x_matrix = x.reshape(out_dim, n_dim)
-    out_matrix = ndarray.empty((out_dim, m_dim), dt)
-    _dot_into(x_matrix.astype(dt, False), w.transpose().astype(dt, False), out_matrix)
-    if b is not None:
-        b_matrix = b.broadcast_to((out_dim, m_dim))
-        _lib.call('hipcx_add', out_matrix.desc(), b_matrix.astype(dt, False).desc(), out_matrix.desc(), current_stream())
-    return out_matrix.reshape(out_shape)
 
 
 def _pair(v, n=2):
@@ -1090,29 +743,6 @@ def _spatial_out(x, n, c, h, w, dtype):
     return ndarray.empty((n, c, h, w), dtype)
 
 
-def conv(x, w, b=None, stride=1, pad=0, cover_all=False, out_dtype=None):
-    """Conv (CX/routines/connection.cc:140-208): one ConvKernel call with the bias inside.  Any number of spatial axes; the
-    dedicated kernels are the 2-D ones (0 and 1 axes run through them as extents of one, 3 and more through a plain kernel)."""
-    if x.ndim < 2 or w.ndim != x.ndim:
-        raise _lib.DimensionError('Mismatched number of dimensions in input %r and weights %r.' % (x.shape, w.shape))
-    n = x.ndim - 2
-    stride, pad = _pair(stride, n), _pair(pad, n)
-    if w.shape[1] != x.shape[1]:
-        raise _lib.DimensionError('Mismatched number of input channels in input %r and weights %r.' % (x.shape, w.shape))
-    if b is not None and (b.ndim != 1 or b.shape[0] != w.shape[0]):
-        raise _lib.DimensionError('Mismatched bias shape %r for weights %r.' % (b.shape, w.shape))
-    dt = numpy.dtype(out_dtype) if out_dtype is not None else (result_type(x, w, b) if b is not None else result_type(x, w))
-    dims = tuple(conv_out_dim(x.shape[2 + d], w.shape[2 + d], stride[d], pad[d], cover_all) for d in range(n))
-    out = _spatial_out(x, x.shape[0], w.shape[0], dims[0], dims[1], dt) if n == 2 else ndarray.empty((x.shape[0], w.shape[0]) + dims, dt)
-    xc, wc = x.astype(dt, False), w.astype(dt, False)
-    bc = b.astype(dt, False) if b is not None else None
-    nbytes = _lib.load().hipcx_conv_workspace_size(xc.desc(), wc.desc(), out.desc())
-    ws, wsp = _workspace(nbytes)
-    _lib.call('hipcx_conv', xc.desc(), wc.desc(), bc.desc() if bc is not None else None, _i64(stride), _i64(pad),
-              int(bool(cover_all)), out.desc(), wsp, nbytes, current_stream())
-    return out
-
-
 def conv_route(x, w, b=None, stride=1, pad=0, cover_all=False):
     """Which kernel family `conv` runs for these arguments (hipcx_conv_route): 0 general implicit GEMM, 1 float16 NCHW kernels
     with 128-wide tiles, 2 the 7x7 / 2 stem kernel, 3 the float16 1x1 kernel with LDS-direct operand loads.  For tests and
@@ -1125,93 +755,6 @@ def conv_route(x, w, b=None, stride=1, pad=0, cover_all=False):
     xc, wc = x.astype(dt, False), w.astype(dt, False)
     bc = b.astype(dt, False) if b is not None else None
     return int(_lib.load().hipcx_conv_route(xc.desc(), wc.desc(), bc.desc() if bc is not None else None, _i64(stride), _i64(pad), out.desc()))
-
-
-def conv_bn_act(x, w, b=None, stride=1, pad=0, cover_all=False, bn=None, eps=2e-5, residual=None, relu=False):
-    """Opt-in fused block: relu(fixed_batch_norm(conv(x, w, b), *bn, eps, axis=(0, 2, 3)) + residual) in one kernel call.
-    `bn` is None or (gamma, beta, mean, var), one value per output channel.  Not part of the ChainerX routine surface:
-    the reference issues these as separate kernels (which `conv`, `fixed_batch_norm`, `add`, `relu` here do as well)."""
-    if x.ndim != 4 or w.ndim != 4:
-        raise _lib.ChainerxNotImplementedError('only 2-D convolution is on the supported path')
-    stride, pad = _pair(stride), _pair(pad)
-    if w.shape[1] != x.shape[1]:
-        raise _lib.DimensionError('Mismatched number of input channels in input %r and weights %r.' % (x.shape, w.shape))
-    dt = result_type(x, w)
-    oh = conv_out_dim(x.shape[2], w.shape[2], stride[0], pad[0], cover_all)
-    ow = conv_out_dim(x.shape[3], w.shape[3], stride[1], pad[1], cover_all)
-    out = _spatial_out(x, x.shape[0], w.shape[0], oh, ow, dt)
-    xc, wc = x.astype(dt, False), w.astype(dt, False)
-    bc = b.astype(dt, False) if b is not None else None
-    prm = [a.astype(dt, False).desc() for a in bn] if bn is not None else [None] * 4
-    res = residual.astype(dt, False) if residual is not None else None
-    nbytes = _lib.load().hipcx_conv_workspace_size(xc.desc(), wc.desc(), out.desc())
-    ws, wsp = _workspace(nbytes)
-    _lib.call('hipcx_conv_bn_act', xc.desc(), wc.desc(), bc.desc() if bc is not None else None, _i64(stride), _i64(pad),
-              int(bool(cover_all)), prm[0], prm[1], prm[2], prm[3], _lib.make_scalar(float(eps)),
-              res.desc() if res is not None else None, int(bool(relu)), out.desc(), wsp, nbytes, current_stream())
-    return out
-
-
-def fixed_batch_norm(x, gamma, beta, mean, var, eps=2e-5, axis=None):
-    """FixedBatchNorm (CX/routines/normalization.cc:414-424 with PreprocessBatchNorm :61-101)."""
-    for a in (x, gamma, beta, mean, var):
-        if _kind(a.dtype) != 3:
-            raise _lib.DtypeError('BatchNorm only supports floating kind inputs.')
-    axes = _sorted_axes(axis, x.ndim) if axis is not None else (0,)
-    reduced_shape = tuple(1 if i in axes else d for i, d in enumerate(x.shape))
-    size = _prod(reduced_shape)
-    params = []
-    for name, a in (('Gamma', gamma), ('Beta', beta), ('Mean', mean), ('Variance', var)):
-        if a.size != size:
-            raise _lib.DimensionError('%s must have the same size as the reduced input. Actual: %d. Expected: %d.' % (name, a.size, size))
-        params.append(a.reshape(reduced_shape))
-    out = ndarray(alloc_bytes(x.nbytes), 0, x.shape, _dense_strides_like(x), x.dtype)
-    ax = (ctypes.c_int8 * len(axes))(*axes)
-    _lib.call('hipcx_fixed_batch_norm', x.desc(), params[0].desc(), params[1].desc(), params[2].desc(), params[3].desc(),
-              _lib.make_scalar(float(eps)), ax, len(axes), out.desc(), current_stream())
-    return out
-
-
-def _dense_strides_like(x):
-    """Dense strides with the same axis order as x's memory (so a channels-last input gives a channels-last output)."""
-    order = sorted(range(x.ndim), key=lambda i: (-abs(x.strides[i]), i))
-    strides = [0] * x.ndim
-    acc = x.itemsize
-    for i in reversed(order):
-        strides[i] = acc
-        acc *= _py.max(1, x.shape[i])
-    return tuple(strides)
-
-
-def max_pool(x, ksize, stride=None, pad=0, cover_all=False):
-    """MaxPool (CX/routines/pooling.cc:52-123); one or more spatial axes (the dedicated kernels are the 2-D ones)."""
-    if x.ndim < 3:
-        raise _lib.DimensionError('pooling needs at least one spatial axis, got the shape %r' % (x.shape,))
-    n = x.ndim - 2
-    ksize = _pair(ksize, n)
-    stride = ksize if stride is None else _pair(stride, n)
-    pad = _pair(pad, n)
-    dims = tuple(conv_out_dim(x.shape[2 + d], ksize[d], stride[d], pad[d], cover_all) for d in range(n))
-    out = _spatial_out(x, x.shape[0], x.shape[1], dims[0], dims[1], x.dtype) if n == 2 else ndarray.empty(x.shape[:2] + dims, x.dtype)
-    _lib.call('hipcx_max_pool', x.desc(), _i64(ksize), _i64(stride), _i64(pad), int(bool(cover_all)), out.desc(), current_stream())
-    return out
-
-
-def average_pool(x, ksize, stride=None, pad=0, pad_mode='ignore'):
-    """AveragePool (CX/routines/pooling.cc:125-169), float dtypes only; one or more spatial axes."""
-    if _kind(x.dtype) != 3:
-        raise _lib.DtypeError('cannot apply average pooling to non-float arrays')
-    if x.ndim < 3:
-        raise _lib.DimensionError('pooling needs at least one spatial axis, got the shape %r' % (x.shape,))
-    n = x.ndim - 2
-    ksize = _pair(ksize, n)
-    stride = ksize if stride is None else _pair(stride, n)
-    pad = _pair(pad, n)
-    mode = {'zero': 1, 'ignore': 2}[pad_mode]
-    dims = tuple(conv_out_dim(x.shape[2 + d], ksize[d], stride[d], pad[d], False) for d in range(n))
-    out = _spatial_out(x, x.shape[0], x.shape[1], dims[0], dims[1], x.dtype) if n == 2 else ndarray.empty(x.shape[:2] + dims, x.dtype)
-    _lib.call('hipcx_average_pool', x.desc(), _i64(ksize), _i64(stride), _i64(pad), mode, out.desc(), current_stream())
-    return out
 
 
 # ---------------------------------------------------------------------------------------------
@@ -1391,19 +934,17 @@ def take(a, indices, axis, mode=None):
     backend (one 4-byte read-back after the kernel).  mode None -- what the reference's callers pass -- raises it too, but late: the
     kernel records the bad index on the device and the next call that waits for the device (``get`` / ``synchronize``) raises, so
     a loop of take calls never waits for the host and can be captured into a graph."""
+    if mode != 'raise':
+        return _host.take_deferred(a, indices, axis, _BOUNDS[mode])
     if _kind(indices.dtype) not in (1, 2):
         raise _lib.DtypeError('Only arrays of integer dtype can be used as indices.')
     axis = _normalize_axis(axis, a.ndim)
     out_shape = a.shape[:axis] + indices.shape + a.shape[axis + 1:]
     out = ndarray.empty(out_shape, a.dtype)
-    m = _BOUNDS[mode]
-    flag = None
-    flag_ptr = None
-    if m == 1:
-        flag = zeros((1,), 'int32')
-        flag_ptr = ctypes.cast(ctypes.c_void_p(flag.data_ptr), ctypes.POINTER(ctypes.c_int32))
-    _lib.call('hipcx_take', a.desc(), indices.desc(), axis, out.desc(), m, flag_ptr, current_stream())
-    if flag is not None and int(flag.get()[0]) != 0:
+    flag = zeros((1,), 'int32')
+    flag_ptr = ctypes.cast(ctypes.c_void_p(flag.data_ptr), ctypes.POINTER(ctypes.c_int32))
+    _lib.call('hipcx_take', a.desc(), indices.desc(), axis, out.desc(), _BOUNDS[mode], flag_ptr, current_stream())
+    if int(flag.get()[0]) != 0:
         raise _lib.ChainerxIndexError('Index is out of bounds for axis %d with size %d' % (axis, a.shape[axis]))
     return out
 
@@ -1536,13 +1077,7 @@ def conv_grad_weight(w_dtype, w_shape, x, gy, stride=1, pad=0, cover_all=False):
     wdt = numpy.dtype(w_dtype)
     if not COMPOSE_CONV_GRAD_WEIGHT and _kind(wdt) == 3 and tuple(w_shape[:2]) == (gy.shape[1], c):
         # one entry: Im2Col and the gy transpose as one kernel each, then the matrix product
-        xc, gc = x.astype(wdt, False).as_contiguous(), gy.astype(wdt, False).as_contiguous()
-        gw = ndarray.empty(tuple(w_shape), wdt)
-        st, pd = _i64((sh, sw)), _i64((ph, pw))
-        nbytes = _lib.load().hipcx_conv_grad_weight_workspace_size(xc.desc(), gc.desc(), gw.desc(), st, pd, int(bool(cover_all)))
-        ws, wsp = _workspace(nbytes)
-        _lib.call('hipcx_conv_grad_weight', xc.desc(), gc.desc(), st, pd, int(bool(cover_all)), gw.desc(), wsp, nbytes, current_stream())
-        return gw
+        return _host.conv_grad_weight_2d(wdt, w_shape, x, gy, (sh, sw), (ph, pw), cover_all)
     xp = zeros((n, c, h + 2 * ph + (sh - 1 if cover_all else 0), w + 2 * pw + (sw - 1 if cover_all else 0)), x.dtype)
     _copy_into(xp[:, :, ph:ph + h, pw:pw + w], x)
     col_t = ndarray.empty((c, kh, kw, n, oh, ow), x.dtype)
@@ -1609,15 +1144,7 @@ def conv_transpose(x, w, b=None, stride=1, pad=0, out_size=None, out_dtype=None)
     dt = numpy.dtype(out_dtype) if out_dtype is not None else (result_type(x, w, b) if b is not None else result_type(x, w))
     if not COMPOSE_CONV_TRANSPOSE and not ROUTE_CONV_TRANSPOSE_HERE and _kind(dt) == 3:
         # one entry: it picks the flipped forward convolution, the scattered 1x1 convolution or the native composition itself
-        xc, wc = x.astype(dt, False), w.astype(dt, False)
-        bc = b.astype(dt, False) if b is not None else None
-        out = ndarray.empty((x.shape[0], w.shape[1]) + tuple(out_size), dt)
-        st, pd = _i64(stride), _i64(pad)
-        nbytes = _lib.load().hipcx_conv_transpose_workspace_size(xc.desc(), wc.desc(), st, pd, out.desc())
-        ws, wsp = _workspace(nbytes)
-        _lib.call('hipcx_conv_transpose', xc.desc(), wc.desc(), bc.desc() if bc is not None else None, st, pd, out.desc(), wsp, nbytes,
-                  current_stream())
-        return out
+        return _host.conv_transpose_2d(x, w, b, stride, pad, out_size, dt)
     if (not COMPOSE_CONV_TRANSPOSE and stride == (1, 1) and pad[0] <= kh - 1 and pad[1] <= kw - 1 and _kind(dt) == 3
             and tuple(out_size) == tuple(d - 1 + k - 2 * p for d, k, p in zip(x.shape[2:], (kh, kw), pad))):
         # At stride 1 the transposed convolution is a forward convolution with the filters flipped in both spatial axes, their
@@ -1664,37 +1191,20 @@ def var(a, axis=None, keepdims=False):
 COMPOSE_BATCH_NORM = False
 
 
-def _bn_kernel_applies(x, axes, params, same=()):
-    """The dedicated kernels take a C-contiguous x of fewer than 2^31 elements reduced over every axis but 1; the per-channel arrays
-    ``params`` share one dtype, x's or -- for a float16 x -- float32 (the mixed-precision call: parameters and statistics of a
-    float16 network kept in float32); the arrays in ``same`` have x's dtype."""
-    pd = params[0].dtype
-    return (not COMPOSE_BATCH_NORM and x.ndim >= 2 and tuple(axes) == (0,) + tuple(range(2, x.ndim)) and x.is_contiguous and x.size < 2 ** 31
-            and (pd == x.dtype or (x.dtype == numpy.dtype('float16') and pd == numpy.dtype('float32')))
-            and _py.all(a.dtype == pd for a in params) and _py.all(a.dtype == x.dtype for a in same))
-
-
 def batch_norm(x, gamma, beta, running_mean, running_var, eps=2e-5, decay=0.9, axis=None):
     """BatchNorm in training mode through GenericBatchNormKernel (CX/routines/normalization.cc:155-193): batch Mean / Var in the
     promoted dtype, ApplyGenericBatchNorm, then the running statistics are updated in place (the variance with the n/(n-1)
     correction).  Returns (out, state) with state = (x_mean, x_inv_std, beta dtype) for batch_norm_grad."""
+    if not COMPOSE_BATCH_NORM:
+        # the dedicated kernels: two statistics passes, a per-channel finish, one normalising pass
+        direct = _host.batch_norm_direct(x, gamma, beta, running_mean, running_var, eps, decay, axis)
+        if direct is not None:
+            return direct
     if _py.any(_kind(t.dtype) != 3 for t in (x, gamma, beta, running_mean, running_var)):
         raise _lib.DtypeError('BatchNorm requires floating point arrays')
     axes = _sorted_axes((0,) + tuple(range(2, x.ndim)) if axis is None else axis, x.ndim)
     red_shape = tuple(1 if i in axes else d for i, d in enumerate(x.shape))
     interm = result_type(x, gamma, beta)
-    if _bn_kernel_applies(x, axes, (gamma, beta, running_mean, running_var)) and x.size > 0:
-        # the dedicated kernels: two statistics passes, a per-channel finish, one normalising pass
-        out = ndarray.empty(x.shape, x.dtype)
-        x_mean = ndarray.empty(red_shape, interm)  # the state has the promoted dtype (CX/routines/normalization.cc:141-150)
-        inv_std = ndarray.empty(red_shape, interm)
-        ax = (ctypes.c_int8 * len(axes))(*axes)
-        nbytes = _lib.load().hipcx_batch_norm_workspace_size(x.desc(), ax, len(axes))
-        ws, wsp = _workspace(nbytes)
-        _lib.call('hipcx_batch_norm', x.desc(), gamma.reshape(red_shape).desc(), beta.reshape(red_shape).desc(),
-                  running_mean.reshape(red_shape).desc(), running_var.reshape(red_shape).desc(), _lib.make_scalar(float(eps)),
-                  _lib.make_scalar(float(decay)), ax, len(axes), out.desc(), x_mean.desc(), inv_std.desc(), wsp, nbytes, current_stream())
-        return out, (x_mean, inv_std, beta.dtype)
     xc = x.astype(interm, False)
     x_mean = mean(xc, axes, True)
     x_var = var(xc, axes, True)
@@ -1714,21 +1224,13 @@ def batch_norm(x, gamma, beta, running_mean, running_var, eps=2e-5, decay=0.9, a
 def batch_norm_grad(x, gamma, gout, state, axis=None):
     """GenericBatchNormGradKernel (CX/routines/normalization.cc:195-250): returns (gx, ggamma, gbeta)."""
     x_mean, x_inv_std, beta_dtype = state
+    if not COMPOSE_BATCH_NORM:
+        direct = _host.batch_norm_grad_direct(x, gamma, gout, x_mean, x_inv_std, beta_dtype, axis)
+        if direct is not None:
+            return direct
     axes = _sorted_axes((0,) + tuple(range(2, x.ndim)) if axis is None else axis, x.ndim)
     red_shape = tuple(1 if i in axes else d for i, d in enumerate(x.shape))
     interm = x_mean.dtype
-    if (_bn_kernel_applies(x, axes, (gamma, x_mean, x_inv_std), (gout,)) and gout.shape == x.shape and gout.is_contiguous
-            and numpy.dtype(beta_dtype) == gamma.dtype and x.size > 0):
-        gx = ndarray.empty(x.shape, x.dtype)
-        ggamma = ndarray.empty(gamma.shape, gamma.dtype)
-        gbeta = ndarray.empty(gamma.shape, gamma.dtype)
-        ax = (ctypes.c_int8 * len(axes))(*axes)
-        nbytes = _lib.load().hipcx_batch_norm_workspace_size(x.desc(), ax, len(axes))
-        ws, wsp = _workspace(nbytes)
-        _lib.call('hipcx_batch_norm_grad', x.desc(), gamma.reshape(red_shape).desc(), gout.desc(), x_mean.reshape(red_shape).desc(),
-                  x_inv_std.reshape(red_shape).desc(), ax, len(axes), gx.desc(), ggamma.reshape(red_shape).desc(),
-                  gbeta.reshape(red_shape).desc(), wsp, nbytes, current_stream())
-        return gx, ggamma, gbeta
     n = _prod(x.shape) // _py.max(1, _prod(gamma.shape))
     inv_n = 1.0 / n
     gc = gout.astype(interm, False)
@@ -1780,16 +1282,7 @@ def max_pool_grad(x, gout, ksize, stride=None, pad=0, cover_all=False):
     if x.ndim == 4 and x.dtype != numpy.dtype('bool') and gout.dtype == x.dtype and not COMPOSE_POOL_GRADIENTS:
         # one kernel: every input position gathers, in kernel-offset order, gout of the windows whose ArgMax it is -- the bits
         # of the composition below
-        oh = conv_out_dim(x.shape[2], ksize[0], stride[0], pad[0], cover_all)
-        ow = conv_out_dim(x.shape[3], ksize[1], stride[1], pad[1], cover_all)
-        if gout.shape != (x.shape[0], x.shape[1], oh, ow):
-            raise _lib.DimensionError('gout has the wrong shape')
-        gx = ndarray.empty(x.shape, x.dtype)
-        nbytes = _lib.load().hipcx_max_pool_grad_workspace_size(gout.desc())
-        ws, wsp = _workspace(nbytes)
-        _lib.call('hipcx_max_pool_grad', x.desc(), gout.desc(), _i64(ksize), _i64(stride), _i64(pad), int(bool(cover_all)), gx.desc(),
-                  wsp, nbytes, current_stream())
-        return gx
+        return _host.max_pool_grad_2d(x, gout, ksize, stride, pad, cover_all)
     lowest = -numpy.inf if _kind(x.dtype) == 3 else (0 if x.dtype == numpy.dtype('bool') else int(numpy.iinfo(x.dtype).min))
     col = im2col(x, ksize, stride, pad, cover_all, lowest)            # [N, C, kh, kw, oh, ow]
     indices = argmax(col, (2, 3))                                     # [N, C, oh, ow]
@@ -1850,10 +1343,7 @@ def average_pool_grad(x, gout, ksize, stride=None, pad=0, pad_mode='ignore'):
     pad = _pair(pad)
     n, c, oh, ow = gout.shape
     if x.ndim == 4 and _kind(x.dtype) == 3 and gout.dtype == x.dtype and not COMPOSE_POOL_GRADIENTS:
-        gx = ndarray.empty(x.shape, x.dtype)
-        _lib.call('hipcx_average_pool_grad', gout.desc(), _i64(ksize), _i64(stride), _i64(pad), {'zero': 1, 'ignore': 2}[pad_mode],
-                  gx.desc(), current_stream())
-        return gx
+        return _host.average_pool_grad_2d(x, gout, ksize, stride, pad, pad_mode)
     g = gout
     if pad_mode == 'ignore':
         def widths(dim, k, st, p, count):  # GetPadModeIgnorePoolingWidths (pool.cc:197-250)
@@ -1898,30 +1388,7 @@ def lstm_fused(c, x):
     """Opt-in: the Lstm cell through hipcx_lstm_cell -- one kernel instead of ~25; same checks and errors as lstm."""
     if c.ndim != 2 or x.ndim != 2:
         return lstm(c, x)
-    h = ndarray.empty(c.shape, c.dtype)
-    new_c = ndarray.empty(c.shape, c.dtype)
-    _lib.call('hipcx_lstm_cell', c.desc(), x.desc(), h.desc(), new_c.desc(), current_stream())
-    return h, new_c
-
-
-def stack(arrays, axis=0):
-    """Stack = Empty + one CopyKernel per input into a view of the new axis (CX/routines/manipulation.cc Stack)."""
-    arrays = list(arrays)
-    if not arrays:
-        raise _lib.DimensionError('Need at least one array to stack')
-    first = arrays[0]
-    axis = _normalize_axis(axis, first.ndim + 1)
-    dtype = first.dtype
-    for a in arrays:
-        if a.shape != first.shape:
-            raise _lib.DimensionError('All arrays need to have the same shape')
-        dtype = promote_types(dtype, a.dtype)
-    out = ndarray.empty(first.shape[:axis] + (len(arrays),) + first.shape[axis:], dtype)
-    for i, a in enumerate(arrays):
-        key = [slice(None)] * out.ndim
-        key[axis] = i
-        _lib.call('hipcx_copy', a.desc(), out[tuple(key)].desc(), current_stream())
-    return out
+    return _host.lstm_cell(c, x)
 
 
 def clipped_relu(x, z):
@@ -2145,21 +1612,10 @@ def rnn(n_layers, hx, cx, ws, bs, xs, bidirectional, mode, activation=None, trai
     flat_w = [w for group in ws for w in group]
     flat_b = [b for group in bs for b in group]
     xs = list(xs)
-    hy = ndarray.empty(hx.shape, hx.dtype)
-    cy = ndarray.empty(cx.shape, cx.dtype) if m == 1 else None
-    ys = [ndarray.empty((x.shape[0], d * hx.shape[2]), hx.dtype) for x in xs]
-    pw, pb, px, py = (_descriptor_pointers(v) for v in (flat_w, flat_b, xs, ys))
-    L = _lib.load()
-    rbytes = L.hipcx_n_step_rnn_reserve_size(n_layers, d - 1, m, hx.desc(), px, len(xs)) if training else 0
-    reserve, rp = _workspace(rbytes) if training else (None, None)
-    nbytes = L.hipcx_n_step_rnn_workspace_size(n_layers, d - 1, m, int(bool(training)), hx.desc(), px, len(xs))
-    wsb, wsp = _workspace(nbytes)
-    _lib.call('hipcx_n_step_rnn', n_layers, d - 1, m, act, hx.desc(), cx.desc() if m == 1 else None, pw, pb, px, len(xs), hy.desc(),
-              cy.desc() if m == 1 else None, py, rp, rbytes, wsp, nbytes, current_stream())
+    hy, cy, ys, reserve = _host.rnn_forward(n_layers, d - 1, m, act, bool(training), hx, cx, flat_w, flat_b, xs)
     state = None
     if training:
-        state = RnnGradState(reserve=reserve, reserve_ptr=rp, reserve_bytes=rbytes, n_layers=n_layers, directions=d, mode=m, activation=act,
-                             hx=hx, ws=flat_w, bs=flat_b, xs=xs)
+        state = RnnGradState(reserve=reserve, n_layers=n_layers, directions=d, mode=m, activation=act, hx=hx, ws=flat_w, bs=flat_b, xs=xs)
     return (hy, cy), ys, state
 
 
@@ -2168,21 +1624,8 @@ def rnn_backward(state, dhy, dcy, dys):
     produced ``state``.  ``dcy`` and entries of ``dys`` may be None (zeros).  Returns ((dhx, dcx or None), dws, dbs, dxs) with dws / dbs
     flat in the order of the forward call's matrices."""
     st = state
-    dhx = ndarray.empty(st.hx.shape, st.hx.dtype)
-    dcx = ndarray.empty(st.hx.shape, st.hx.dtype) if st.mode == 1 else None
-    dws = [ndarray.empty(w.shape, w.dtype) for w in st.ws]
-    dbs = [ndarray.empty(b.shape, b.dtype) for b in st.bs]
-    dxs = [ndarray.empty(x.shape, x.dtype) for x in st.xs]
-    pw, pb, px, pdw, pdb, pdx = (_descriptor_pointers(v) for v in (st.ws, st.bs, st.xs, dws, dbs, dxs))
-    for a in dys:
-        if a is not None:
-            a.desc()
-    pdy = (ctypes.POINTER(_lib.CArray) * len(dys))(*[ctypes.pointer(a._desc) if a is not None else None for a in dys])
-    nbytes = _lib.load().hipcx_n_step_rnn_workspace_size(st.n_layers, st.directions - 1, st.mode, 1, st.hx.desc(), px, len(st.xs))
-    wsb, wsp = _workspace(nbytes)
-    _lib.call('hipcx_n_step_rnn_backward', st.n_layers, st.directions - 1, st.mode, st.activation, st.hx.desc(), pw, pb, px, len(st.xs),
-              dhy.desc(), dcy.desc() if (dcy is not None and st.mode == 1) else None, pdy, st.reserve_ptr, st.reserve_bytes, dhx.desc(),
-              dcx.desc() if st.mode == 1 else None, pdw, pdb, pdx, wsp, nbytes, current_stream())
+    dhx, dcx, dws, dbs, dxs = _host.rnn_backward(st.n_layers, st.directions - 1, st.mode, st.activation, st.hx, st.ws, st.bs, st.xs, st.reserve,
+                                                 dhy, dcy, dys)
     return (dhx, dcx), dws, dbs, dxs
 
 
@@ -2297,3 +1740,4 @@ def _install_operators():
 
 
 _install_operators()
+_host.setup({'flags': globals()})  # the native routines look the opt-in switches up here
