@@ -158,6 +158,7 @@ SIGNATURES = {
     'hipcx_argmax': (_INT, [_A, _I8P, _INT, _A, _V, _SZ, _V]),
     'hipcx_dot_workspace_size': (_SZ, [_A, _A, _A]),
     'hipcx_dot': (_INT, [_A, _A, _A, _V, _SZ, _V]),
+    'hipcx_dot_bias': (_INT, [_A, _A, _A, _A, _V, _SZ, _V]),
     'hipcx_conv_out_dim': (ctypes.c_int64, [ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, _INT]),
     'hipcx_conv_workspace_size': (_SZ, [_A, _A, _A]),
     'hipcx_conv': (_INT, [_A, _A, _A, _I64P, _I64P, _INT, _A, _V, _SZ, _V]),
@@ -192,6 +193,8 @@ SIGNATURES = {
     'hipcx_log_softmax_workspace_size': (_SZ, [_A]),
     'hipcx_log_softmax': (_INT, [_A, _A, _V, _SZ, _V]),
     'hipcx_lstm_cell': (_INT, [_A, _A, _A, _A, _V]),
+    'hipcx_softmax_cross_entropy_workspace_size': (_SZ, [_A]),
+    'hipcx_softmax_cross_entropy': (_INT, [_A, _A, _A, _V, _SZ, _V]),
     'hipcx_profile_start': (_INT, []),
     'hipcx_profile_stop': (_INT, [_I64P, ctypes.POINTER(ctypes.c_double), ctypes.POINTER(ctypes.c_double),
                                   ctypes.POINTER(ctypes.c_double)]),

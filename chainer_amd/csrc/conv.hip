@@ -198,7 +198,7 @@ void LaunchIGemmImpl(IGemmArgs<T> p, hipStream_t stream) {
 
 // Large float16 products with both operands' reduction index at unit stride (gemm_pp.h).  Returns false when the problem does
 // not qualify: the 128 x 128 kernels below then take it.
-bool TryGemmPp(const hipcx_array* a, const hipcx_array* b, const hipcx_array* out, hipStream_t stream) {
+bool TryGemmPp(const hipcx_array* a, const hipcx_array* b, const hipcx_array* bias, const hipcx_array* out, hipStream_t stream) {
     static const bool enabled = [] { const char* e = getenv("HIPCX_DOT_PP"); return e == nullptr || e[0] != '0'; }();
     static const int band = [] { const char* e = getenv("HIPCX_DOT_PP_BAND"); return e != nullptr && atoi(e) > 0 ? atoi(e) : 8; }();
     if (!enabled) return false;
@@ -226,6 +226,10 @@ bool TryGemmPp(const hipcx_array* a, const hipcx_array* b, const hipcx_array* ou
     p.tiles_m = static_cast<int>(tiles_m);
     p.tiles_n = static_cast<int>(tiles_n);
     p.band = band;
+    if (bias != nullptr) {
+        p.bias = static_cast<const half_t*>(bias->data);
+        p.bias_stride = bias->strides[0] / 2;
+    }
     ProfileScope prof(stream, 2.0 * static_cast<double>(M) * N * K, 2.0 * (static_cast<double>(M) * K + static_cast<double>(N) * K + static_cast<double>(M) * N));
     struct GemmPpTag {};
     EnsureDynamicLds<GemmPpTag>(reinterpret_cast<const void*>(gemm_pp::GemmPpKernel), gemm_pp::kLdsBytes);
@@ -237,7 +241,7 @@ bool TryGemmPp(const hipcx_array* a, const hipcx_array* b, const hipcx_array* ou
 
 // Small-output matrix products (small_dot.h).  Returns false when the problem does not qualify.
 template <typename T>
-bool TrySmallDot(const hipcx_array* a, const hipcx_array* b, const hipcx_array* out, hipStream_t stream) {
+bool TrySmallDot(const hipcx_array* a, const hipcx_array* b, const hipcx_array* bias, const hipcx_array* out, hipStream_t stream) {
     static const bool enabled = [] { const char* e = getenv("HIPCX_SMALL_DOT"); return e == nullptr || e[0] != '0'; }();
     if (!enabled) return false;
     const int64_t M = a->shape[0], K = a->shape[1], N = b->shape[1];
@@ -266,6 +270,10 @@ bool TrySmallDot(const hipcx_array* a, const hipcx_array* b, const hipcx_array* 
     auto dword_ok = [&](const void* ptr, int64_t line_stride) { return reinterpret_cast<uintptr_t>(ptr) % 4 == 0 && (line_stride * it) % 4 == 0; };
     p.a_vec = (p.a_k == 1 && dword_ok(a->data, p.a_row)) ? 1 : 0;
     p.b_vec = (p.b_k == 1 && dword_ok(b->data, p.b_col)) ? 1 : 0;
+    if (bias != nullptr) {
+        p.bias = bias->data;
+        p.bias_stride = bias->strides[0] / it;
+    }
     p.tiles_n = static_cast<int>((N + 31) / 32);
     int64_t blocks = ((M + 31) / 32) * p.tiles_n;
     ProfileScope prof(stream, 2.0 * M * N * K, static_cast<double>(it) * (M * K + K * N + M * N));
@@ -1434,24 +1442,9 @@ void LaunchBatchedProduct(int dtype, const void* a, int64_t a_row, int64_t a_sli
     else run(float{});
 }
 
-extern "C" {
-
-size_t hipcx_dot_workspace_size(const hipcx_array* a, const hipcx_array* b, const hipcx_array* out) {
-    try {
-        if (out != nullptr && !IsFloatDtype(out->dtype)) return 0;
-        DotStaging st = PlanDotStaging(a, b, out);
-        size_t split = 0;
-        if (a != nullptr && b != nullptr && out != nullptr && a->ndim == 2 && b->ndim == 2) {
-            split = SplitKBytes(a->shape[0], b->shape[1], PlanSplitK(a->shape[0], b->shape[1], a->shape[1], out->dtype));
-        }
-        return RoundUpTo(st.a_bytes + st.b_bytes, 256) + split;
-    } catch (...) {
-        return 0;
-    }
-}
-
-int hipcx_dot(const hipcx_array* a, const hipcx_array* b, const hipcx_array* out, void* workspace, size_t workspace_bytes,
-              void* stream) {
+// Dot, and Add of a stride-0 row (may be null) in its epilogue.
+static int DotBias(const hipcx_array* a, const hipcx_array* b, const hipcx_array* bias, const hipcx_array* out, void* workspace,
+                   size_t workspace_bytes, void* stream) {
     return Guard([&] {
         ValidateArray(a, "a");
         ValidateArray(b, "b");
@@ -1463,24 +1456,40 @@ int hipcx_dot(const hipcx_array* a, const hipcx_array* b, const hipcx_array* out
         HIPCX_REQUIRE(a->dtype == out->dtype && b->dtype == out->dtype, HIPCX_DTYPE_ERROR,
                       "a and b must have out's dtype (cast with hipcx_copy first)");
         HIPCX_REQUIRE(m < (1LL << 31) && n < (1LL << 31) && k < (1LL << 31), HIPCX_NOT_IMPLEMENTED_ERROR, "extent too large");
+        if (bias != nullptr) {
+            ValidateArray(bias, "bias");
+            HIPCX_REQUIRE(bias->ndim == 1 && bias->shape[0] == n, HIPCX_DIMENSION_ERROR, "dot: one bias element per column is needed");
+            HIPCX_REQUIRE(bias->dtype == out->dtype, HIPCX_DTYPE_ERROR, "bias must have out's dtype (cast with hipcx_copy first)");
+        }
         if (m == 0 || n == 0) return;
         hipStream_t st = AsStream(stream);
+        auto add_bias = [&] {
+            if (bias == nullptr) return;
+            hipcx_array row = *out;
+            row.data = bias->data;
+            row.strides[0] = 0;
+            row.strides[1] = bias->strides[0];
+            int s = hipcx_add(out, &row, out, stream);
+            if (s != HIPCX_OK) throw Error(s, hipcx_last_error());
+        };
         if (k == 0) {  // the routine normally short-circuits this (CX/routines/linalg.cc:59-61)
             hipcx_scalar zero{HIPCX_KIND_INT, 0, 0, 0.0};
             int s = hipcx_fill(out, zero, stream);
             if (s != HIPCX_OK) throw Error(s, hipcx_last_error());
+            add_bias();
             return;
         }
         if (!IsFloatDtype(out->dtype)) {  // integers and bool: int_dot.hip
             IntDot(a, b, out, st);
+            add_bias();
             return;
         }
         auto fill = [&](auto& p) {
             using T = std::remove_cv_t<std::remove_pointer_t<decltype(p.out)>>;
             p.x = static_cast<const T*>(a->data);
             p.w = static_cast<const T*>(b->data);
-            p.bias = nullptr;
-            p.bias_stride = 0;
+            p.bias = bias != nullptr ? static_cast<const T*>(bias->data) : nullptr;
+            p.bias_stride = bias != nullptr ? bias->strides[0] / ItemSize(out->dtype) : 0;
             p.out = static_cast<T*>(out->data);
             p.N = static_cast<int>(m);
             p.C = static_cast<int>(k);
@@ -1556,15 +1565,15 @@ int hipcx_dot(const hipcx_array* a, const hipcx_array* b, const hipcx_array* out
             }
         }
         if (out->dtype == HIPCX_FLOAT16) {
-            if (slices == 1 && TryGemmPp(a, b, out, st)) return;
-            if (slices == 1 && TrySmallDot<half_t>(a, b, out, st)) return;
+            if (slices == 1 && TryGemmPp(a, b, bias, out, st)) return;
+            if (slices == 1 && TrySmallDot<half_t>(a, b, bias, out, st)) return;
             IGemmArgs<half_t> p{};
             fill(p);
             p.ksplit = slices;
             p.partial = partial;
             LaunchIGemmImpl(p, st);
         } else if (out->dtype == HIPCX_FLOAT32) {
-            if (slices == 1 && TrySmallDot<float>(a, b, out, st)) return;
+            if (slices == 1 && TrySmallDot<float>(a, b, bias, out, st)) return;
             IGemmArgs<float> p{};
             fill(p);
             p.ksplit = slices;
@@ -1576,5 +1585,31 @@ int hipcx_dot(const hipcx_array* a, const hipcx_array* b, const hipcx_array* out
             LaunchF64(p, st);
         }
     });
+}
+
+extern "C" {
+
+size_t hipcx_dot_workspace_size(const hipcx_array* a, const hipcx_array* b, const hipcx_array* out) {
+    try {
+        if (out != nullptr && !IsFloatDtype(out->dtype)) return 0;
+        DotStaging st = PlanDotStaging(a, b, out);
+        size_t split = 0;
+        if (a != nullptr && b != nullptr && out != nullptr && a->ndim == 2 && b->ndim == 2) {
+            split = SplitKBytes(a->shape[0], b->shape[1], PlanSplitK(a->shape[0], b->shape[1], a->shape[1], out->dtype));
+        }
+        return RoundUpTo(st.a_bytes + st.b_bytes, 256) + split;
+    } catch (...) {
+        return 0;
+    }
+}
+
+int hipcx_dot(const hipcx_array* a, const hipcx_array* b, const hipcx_array* out, void* workspace, size_t workspace_bytes,
+              void* stream) {
+    return DotBias(a, b, nullptr, out, workspace, workspace_bytes, stream);
+}
+
+int hipcx_dot_bias(const hipcx_array* a, const hipcx_array* b, const hipcx_array* bias, const hipcx_array* out, void* workspace,
+                   size_t workspace_bytes, void* stream) {
+    return DotBias(a, b, bias, out, workspace, workspace_bytes, stream);
 }
 }

@@ -123,6 +123,42 @@ __global__ __launch_bounds__(NT) void LogSoftmaxRowKernel(const T* x, T* out, in
     }
 }
 
+// ---- LogSoftmax, short rows: LPR lanes of a wave hold a row of at most 16 * LPR elements (MAXE per lane), 64 / LPR rows to a wave.
+// A wave per row leaves most lanes without an element when rows are classes (10, 16, ...) and is bounded by the launch of its
+// workgroups: [65536, 16] float32 ran 65536 of them. ----
+template <typename T, int LPR>
+__global__ __launch_bounds__(256) void LogSoftmaxShortRowKernel(const T* x, T* out, int64_t rows, int n, int64_t x_row, int64_t o_row) {
+    using C = compute_t<T>;
+    constexpr int MAXE = 4;
+    const int64_t row = static_cast<int64_t>(blockIdx.x) * (256 / LPR) + threadIdx.x / LPR;
+    const int lane = threadIdx.x % LPR;
+    if (row >= rows) return;  // whole groups of LPR lanes leave: the shuffles below stay inside a group
+    const T* xr = x + row * x_row;
+    C v[MAXE];
+    C m = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < MAXE; ++i) {
+        const int e = i * LPR + lane;
+        v[i] = e < n ? static_cast<C>(xr[e]) : static_cast<C>(-INFINITY);
+        if (e < n) m = MaxNan(m, v[i]);
+    }
+#pragma unroll
+    for (int d = LPR / 2; d >= 1; d >>= 1) m = MaxNan(m, static_cast<C>(__shfl_xor(m, d, LPR)));
+    C s = 0;
+#pragma unroll
+    for (int i = 0; i < MAXE; ++i) {
+        if (i * LPR + lane < n) s += ExpOf<C>(v[i] - m);
+    }
+#pragma unroll
+    for (int d = LPR / 2; d >= 1; d >>= 1) s += static_cast<C>(__shfl_xor(s, d, LPR));
+    const C lse = m + LogOf<C>(s);
+    T* orow = out + row * o_row;
+#pragma unroll
+    for (int i = 0; i < MAXE; ++i) {
+        if (i * LPR + lane < n) orow[i * LPR + lane] = static_cast<T>(v[i] - lse);
+    }
+}
+
 // ---- LogSoftmax, long rows: pass 1 leaves (max, sum of exp(x - max)) per (row, segment); pass 2 merges a row's
 // segments, then rewrites its own segment ----
 constexpr int kSegThreads = 256;
@@ -232,7 +268,20 @@ void RunLogSoftmax(const hipcx_array* x, const hipcx_array* out, const LsmShape&
     const int vec_ok = reinterpret_cast<uintptr_t>(xp) % 16 == 0 && reinterpret_cast<uintptr_t>(op) % 16 == 0 && sh.x_row % V == 0 && sh.o_row % V == 0;
     const int64_t packs = (sh.n + V - 1) / V;
     const unsigned rows = static_cast<unsigned>(sh.rows);
-    if (packs <= 64) {
+    auto short_rows = [&](auto lpr) {
+        constexpr int LPR = decltype(lpr)::value;
+        const int64_t blocks = (sh.rows + 256 / LPR - 1) / (256 / LPR);
+        hipLaunchKernelGGL((LogSoftmaxShortRowKernel<T, LPR>), dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, xp, op, sh.rows,
+                           static_cast<int>(sh.n), sh.x_row, sh.o_row);
+    };
+    // up to four elements to a lane: beyond 128 of them a row fills a wave with 16-byte loads
+    if (sh.n <= 16) {
+        short_rows(std::integral_constant<int, 4>{});
+    } else if (sh.n <= 64) {
+        short_rows(std::integral_constant<int, 16>{});
+    } else if (sh.n <= 128) {
+        short_rows(std::integral_constant<int, 32>{});
+    } else if (packs <= 64) {
         hipLaunchKernelGGL((LogSoftmaxRowKernel<T, 64, 1>), dim3(rows), dim3(64), 0, stream, xp, op, sh.n, sh.x_row, sh.o_row, vec_ok);
     } else if (packs <= 256) {
         hipLaunchKernelGGL((LogSoftmaxRowKernel<T, 256, 1>), dim3(rows), dim3(256), 0, stream, xp, op, sh.n, sh.x_row, sh.o_row, vec_ok);
@@ -258,6 +307,129 @@ void RunLogSoftmax(const hipcx_array* x, const hipcx_array* out, const LsmShape&
                            static_cast<int>(nseg), vec_ok);
     }
     CheckLaunch("log_softmax");
+}
+
+// ---- softmax cross entropy ----
+// A group of LPR lanes walks a row twice (maximum; sum of exponentials), the second time out of L1 / L2; what a row contributes is the
+// score of its label.  The chain multiplies every score with a 0 / 1 mask, so a score of -inf elsewhere in the row turns the sum into
+// NaN (0 * inf): the smallest other score is kept to see that.  One workgroup does a small batch alone ([100, 10]: 15 launches of
+// 2.1-3.6 us, 41 us together -> one of 4 us); larger batches leave partial sums for XentFinishKernel.
+struct XentArgs {
+    const void* x;
+    const void* t;
+    void* out;
+    double* partial;  // {sum of scores, number of labels} per workgroup, or null: one workgroup writes the result itself
+    int64_t rows, n, x_row, t_stride;
+    int t_dtype;
+};
+
+__device__ __forceinline__ int64_t LoadLabel(const void* t, int64_t i, int dtype) {
+    switch (dtype) {
+        case HIPCX_INT8: return static_cast<const int8_t*>(t)[i];
+        case HIPCX_INT16: return static_cast<const int16_t*>(t)[i];
+        case HIPCX_INT32: return static_cast<const int32_t*>(t)[i];
+        case HIPCX_UINT8: return static_cast<const uint8_t*>(t)[i];
+        default: return static_cast<const int64_t*>(t)[i];
+    }
+}
+
+// -sum / count with the roundings of Sum, Sum, Divide(-1, .) and Multiply.
+template <typename T>
+__device__ __forceinline__ T XentResult(double sum, double count) {
+    using C = compute_t<T>;
+    const C s = static_cast<C>(static_cast<T>(sum)), n = static_cast<C>(static_cast<T>(count));
+    const C factor = static_cast<C>(static_cast<T>(C(-1) / n));
+    return static_cast<T>(s * factor);
+}
+
+// Adds up (a, b) of all threads of a workgroup; valid in thread 0.
+template <int NT>
+__device__ __forceinline__ void BlockSum2(double& a, double& b, double (*scratch)[2]) {
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) {
+        a += ShflDown(a, d);
+        b += ShflDown(b, d);
+    }
+    if ((threadIdx.x & 63) == 0) {
+        scratch[threadIdx.x >> 6][0] = a;
+        scratch[threadIdx.x >> 6][1] = b;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < NT / 64; ++w) {
+            a += scratch[w][0];
+            b += scratch[w][1];
+        }
+    }
+}
+
+constexpr int kXentThreads = 1024;
+
+template <typename T, int LPR>
+__global__ __launch_bounds__(kXentThreads) void XentKernel(XentArgs p) {
+    using C = compute_t<T>;
+    __shared__ double scratch[kXentThreads / 64][2];
+    const int lane = threadIdx.x % LPR;
+    double sum = 0, count = 0;
+    for (int64_t row = static_cast<int64_t>(blockIdx.x) * (kXentThreads / LPR) + threadIdx.x / LPR; row < p.rows;
+         row += static_cast<int64_t>(gridDim.x) * (kXentThreads / LPR)) {
+        const T* xr = static_cast<const T*>(p.x) + row * p.x_row;
+        const int64_t label = LoadLabel(p.t, row * p.t_stride, p.t_dtype);
+        C m = -INFINITY, least = INFINITY;
+        for (int64_t e = lane; e < p.n; e += LPR) {
+            const C v = static_cast<C>(xr[e]);
+            m = MaxNan(m, v);
+            if (e != label) least = v < least ? v : least;
+        }
+#pragma unroll
+        for (int d = LPR / 2; d >= 1; d >>= 1) {
+            m = MaxNan(m, static_cast<C>(__shfl_xor(m, d, LPR)));
+            const C o = static_cast<C>(__shfl_xor(least, d, LPR));
+            least = o < least ? o : least;
+        }
+        C s = 0;
+        for (int64_t e = lane; e < p.n; e += LPR) s += ExpOf<C>(static_cast<C>(xr[e]) - m);
+#pragma unroll
+        for (int d = LPR / 2; d >= 1; d >>= 1) s += static_cast<C>(__shfl_xor(s, d, LPR));
+        if (lane == 0) {
+            const C lse = m + LogOf<C>(s);
+            const bool counts = label >= 0 && label < p.n;
+            C score = counts ? static_cast<C>(static_cast<T>(static_cast<C>(xr[label]) - lse)) : C(0);
+            if (p.n > (counts ? 1 : 0)) score += static_cast<C>(static_cast<T>(least - lse)) * C(0);
+            sum += static_cast<double>(score);
+            count += counts ? 1.0 : 0.0;
+        }
+    }
+    BlockSum2<kXentThreads>(sum, count, scratch);
+    if (threadIdx.x == 0) {
+        if (p.partial != nullptr) {
+            p.partial[2 * blockIdx.x] = sum;
+            p.partial[2 * blockIdx.x + 1] = count;
+        } else {
+            *static_cast<T*>(p.out) = XentResult<T>(sum, count);
+        }
+    }
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void XentFinishKernel(XentArgs p, int n_partial) {
+    __shared__ double scratch[4][2];
+    double sum = 0, count = 0;
+    for (int i = threadIdx.x; i < n_partial; i += 256) {
+        sum += p.partial[2 * i];
+        count += p.partial[2 * i + 1];
+    }
+    BlockSum2<256>(sum, count, scratch);
+    if (threadIdx.x == 0) *static_cast<T*>(p.out) = XentResult<T>(sum, count);
+}
+
+// Workgroups for a batch: one while it is at most a few thousand elements (a second launch costs more than it saves), then one per
+// eight of its row slots, up to two to a compute unit.
+int XentBlocks(int64_t rows, int64_t n) {
+    if (rows * n <= 16384) return 1;
+    const int64_t lpr = n <= 16 ? 16 : 64;
+    const int64_t blocks = (rows * lpr + kXentThreads - 1) / kXentThreads;
+    return static_cast<int>(blocks < 512 ? blocks : 512);
 }
 
 // ---- Lstm cell ----
@@ -316,6 +488,57 @@ int hipcx_log_softmax(const hipcx_array* x, const hipcx_array* out, void* worksp
         VisitFloatDtype(x->dtype, [&](auto tag) {
             using T = typename decltype(tag)::type;
             RunLogSoftmax<T>(x, out, sh, workspace, workspace_bytes, AsStream(stream));
+        });
+    });
+}
+
+size_t hipcx_softmax_cross_entropy_workspace_size(const hipcx_array* x) {
+    if (x == nullptr || x->ndim != 2) return 0;
+    const int blocks = XentBlocks(x->shape[0], x->shape[1]);
+    return blocks > 1 ? static_cast<size_t>(blocks) * 2 * sizeof(double) : 0;
+}
+
+int hipcx_softmax_cross_entropy(const hipcx_array* x, const hipcx_array* t, const hipcx_array* out, void* workspace, size_t workspace_bytes,
+                                void* stream) {
+    return Guard([&] {
+        ValidateArray(x, "x");
+        ValidateArray(t, "t");
+        ValidateArray(out, "out");
+        HIPCX_REQUIRE(IsFloatDtype(x->dtype) && out->dtype == x->dtype, HIPCX_DTYPE_ERROR, "softmax_cross_entropy: x and out need one float dtype");
+        HIPCX_REQUIRE(!IsFloatDtype(t->dtype) && t->dtype != HIPCX_BOOL, HIPCX_DTYPE_ERROR, "softmax_cross_entropy: labels need an integer dtype");
+        HIPCX_REQUIRE(x->ndim == 2 && t->ndim == 1 && t->shape[0] == x->shape[0] && TotalSize(out) == 1, HIPCX_DIMENSION_ERROR,
+                      "softmax_cross_entropy: x [B, n], t [B] and an out of one element are needed");
+        const int64_t it = ItemSize(x->dtype);
+        HIPCX_REQUIRE((x->shape[1] <= 1 || x->strides[1] == it) && x->strides[0] % it == 0 && t->strides[0] % ItemSize(t->dtype) == 0,
+                      HIPCX_NOT_IMPLEMENTED_ERROR, "softmax_cross_entropy: rows must be dense along axis 1");
+        XentArgs p{};
+        p.x = x->data;
+        p.t = t->data;
+        p.out = out->data;
+        p.rows = x->shape[0];
+        p.n = x->shape[1];
+        p.x_row = x->strides[0] / it;
+        p.t_stride = t->strides[0] / ItemSize(t->dtype);
+        p.t_dtype = t->dtype;
+        const int blocks = p.rows > 0 ? XentBlocks(p.rows, p.n) : 1;
+        if (blocks > 1) {
+            const size_t need = static_cast<size_t>(blocks) * 2 * sizeof(double);
+            HIPCX_REQUIRE(workspace != nullptr && workspace_bytes >= need, HIPCX_CHAINERX_ERROR,
+                          "softmax_cross_entropy: workspace of " + std::to_string(need) + " bytes required");
+            p.partial = static_cast<double*>(workspace);
+        }
+        VisitFloatDtype(x->dtype, [&](auto tag) {
+            using T = typename decltype(tag)::type;
+            if (p.n <= 16) {
+                hipLaunchKernelGGL((XentKernel<T, 16>), dim3(blocks), dim3(kXentThreads), 0, AsStream(stream), p);
+            } else {
+                hipLaunchKernelGGL((XentKernel<T, 64>), dim3(blocks), dim3(kXentThreads), 0, AsStream(stream), p);
+            }
+            CheckLaunch("softmax_cross_entropy");
+            if (blocks > 1) {
+                hipLaunchKernelGGL((XentFinishKernel<T>), dim3(1), dim3(256), 0, AsStream(stream), p, blocks);
+                CheckLaunch("softmax_cross_entropy_finish");
+            }
         });
     });
 }

@@ -32,6 +32,8 @@ struct GemmArgs {
     int lda, ldb, ldc;  // elements
     int tiles_m, tiles_n;
     int band;  // tile rows per band of the tile order
+    const half_t* bias;  // one element per column of c, added before the rounding; may be null
+    int64_t bias_stride;
 };
 
 // Raw buffer descriptor (base, no stride, size in bytes, 32-bit untyped data) as four scalars.
@@ -206,7 +208,11 @@ __global__ __launch_bounds__(512) void GemmPpKernel(GemmArgs p) {
                 if (n >= p.N) continue;  // N % 4 == 0: a group of four is inside or outside
                 PVecH<4> o;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) o.e[e] = static_cast<half_t>(acc[i][j][q * 4 + e]);
+                for (int e = 0; e < 4; ++e) {
+                    float v = acc[i][j][q * 4 + e];
+                    if (p.bias != nullptr) v += static_cast<float>(p.bias[(n + e) * p.bias_stride]);
+                    o.e[e] = static_cast<half_t>(v);
+                }
                 *reinterpret_cast<PVecH<4>*>(crow + n) = o;
             }
         }

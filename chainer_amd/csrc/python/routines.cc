@@ -190,17 +190,12 @@ UNARY_ROUTINE(Log, log)
 UNARY_ROUTINE(Tanh, tanh)
 UNARY_ROUTINE(Sqrt, sqrt)
 
-// Sigmoid(x) = Reciprocal(1 + Exp(-x)): four kernels (CX/routines/activation.cc:74-78).
+// Sigmoid(x) = Reciprocal(1 + Exp(-x)) (CX/routines/activation.cc:74-78), its four steps in one kernel.
 HOST_FN(Sigmoid) {
     HOST_TRY;
     HOST_ARGS("sigmoid", 1, "x");
-    Array* x = AsArray(arg[0], "x");
-    const int code = MathDtype(x->d.dtype);
-    Ref xc = Cast(x, code);
-    Ref neg = NegativeOf(xc.arr());
-    Ref e = Unary(hipcx_exp, neg.arr());
-    Ref one_more = BinaryScalar(hipcx_add_as, e.arr(), IntScalar(1), code, nullptr);
-    return DivideScalar(IntScalar(1), one_more.arr(), code, nullptr).release();
+    auto fn = [](const hipcx_array* x, const hipcx_array* out, void* stream) { return hipcx_unary(HIPCX_UNARY_SIGMOID, x, out, stream); };
+    return Unary(fn, AsArray(arg[0], "x")).release();
     HOST_CATCH(nullptr);
 }
 
@@ -581,7 +576,7 @@ HOST_FN(Dot) {
     HOST_CATCH(nullptr);
 }
 
-// Linear (CX/routines/connection.cc:322-394): DotKernel(x, w.T view) then AddKernel with a stride-0 bias.
+// Linear (CX/routines/connection.cc:322-394): DotKernel(x, w.T view), AddKernel with a stride-0 bias in its epilogue.
 HOST_FN(Linear) {
     HOST_TRY;
     HOST_ARGS("linear", 2, "x", "w", "b", "n_batch_axes");
@@ -610,11 +605,17 @@ HOST_FN(Linear) {
     std::swap(wt.shape[0], wt.shape[1]);
     std::swap(wt.strides[0], wt.strides[1]);
     Ref out = Empty(2, matrix_shape, code);
-    DotInto(xm.d(), &wt, out.d());
-    if (b != nullptr) {
-        Ref bc = Operand(b, 2, matrix_shape, code);
+    if (b == nullptr) {
+        DotInto(xm.d(), &wt, out.d());
+    } else {
+        Ref bc = Cast(b, code);
+        if (bc.arr()->d.shape[0] != m) {  // a bias of one element is broadcast; other lengths raise
+            const int64_t bias_shape[1] = {m};
+            bc = BroadcastTo(bc.arr(), 1, bias_shape);
+        }
+        Workspace ws(hipcx_dot_workspace_size(xm.d(), &wt, out.d()));
         void* stream = Stream();
-        Call([&] { return hipcx_add(out.d(), bc.d(), out.d(), stream); });
+        Call([&] { return hipcx_dot_bias(xm.d(), &wt, bc.d(), out.d(), ws.ptr, ws.bytes, stream); });
     }
     return Reshape(out.arr(), n_batch + 1, out_shape).release();
     HOST_CATCH(nullptr);
@@ -1111,10 +1112,35 @@ HOST_FN(LogSoftmaxDirect) {
     HOST_CATCH(nullptr);
 }
 
+// The loss of the routine below in one call, or None for operands its kernel does not take.
+HOST_FN(SoftmaxCrossEntropyDirect) {
+    HOST_TRY;
+    HOST_ARGS("softmax_cross_entropy", 2, "x", "t");
+    Array *x0 = AsArray(arg[0], "x"), *t = AsArray(arg[1], "t");
+    static const int64_t kMax[10] = {0, 0, 127, 32767, INT32_MAX, INT64_MAX, 255, 0, 0, 0};  // of the integer dtypes
+    if (x0->d.ndim != 2 || t->d.ndim != 1 || t->d.shape[0] != x0->d.shape[0] || x0->d.shape[0] == 0 || x0->d.shape[1] == 0 ||
+        x0->d.shape[1] - 1 > kMax[t->d.dtype]) {
+        Py_RETURN_NONE;
+    }
+    Ref x = Cast(x0, MathDtype(x0->d.dtype));
+    const hipcx_array* d = x.d();
+    if (d->shape[1] > 1 && d->strides[1] != ItemSize(d->dtype)) Py_RETURN_NONE;
+    Ref out = Empty(0, nullptr, d->dtype);
+    Workspace ws(hipcx_softmax_cross_entropy_workspace_size(d));
+    void* stream = Stream();
+    Call([&] { return hipcx_softmax_cross_entropy(d, &t->d, out.d(), ws.ptr, ws.bytes, stream); });
+    return out.release();
+    HOST_CATCH(nullptr);
+}
+
+// The Lstm cell of 2-D arrays with dense rows through hipcx_lstm_cell, or None for other calls.
 HOST_FN(LstmCell) {
     HOST_TRY;
     HOST_ARGS("lstm_cell", 2, "c", "x");
     Array *c = AsArray(arg[0], "c"), *x = AsArray(arg[1], "x");
+    for (const Array* a : {c, x}) {
+        if (a->d.ndim != 2 || (a->d.shape[1] > 1 && a->d.strides[1] != ItemSize(a->d.dtype)) || a->d.strides[0] < 0) Py_RETURN_NONE;
+    }
     Ref h = EmptyLike(c, c->d.dtype), new_c = EmptyLike(c, c->d.dtype);
     void* stream = Stream();
     Call([&] { return hipcx_lstm_cell(&c->d, &x->d, h.d(), new_c.d(), stream); });
@@ -1275,6 +1301,7 @@ PyMethodDef kRoutines[] = {
         ROUTINE("batch_norm_grad_direct", BatchNormGradDirect, nullptr),
         ROUTINE("take_deferred", TakeDeferred, nullptr),
         ROUTINE("log_softmax_direct", LogSoftmaxDirect, nullptr),
+        ROUTINE("softmax_cross_entropy_direct", SoftmaxCrossEntropyDirect, nullptr),
         ROUTINE("lstm_cell", LstmCell, nullptr),
         ROUTINE("rnn_forward", RnnForward, nullptr),
         ROUTINE("rnn_backward", RnnBackward, nullptr),

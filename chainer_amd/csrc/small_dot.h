@@ -24,6 +24,8 @@ struct SmallDotArgs {
     unsigned a_bytes, b_bytes;  // spans, for the buffer descriptors
     int a_vec, b_vec;           // k is the unit-stride axis of the operand and 16-byte runs are dword aligned
     int tiles_n;
+    const void* bias;     // one element per column of out, added to the rounded product (Dot, then Add); may be null
+    int64_t bias_stride;  // elements
     int nw;  // SmallDotRowsKernel: waves per workgroup = ways the reduction axis is split
 };
 
@@ -38,6 +40,14 @@ __device__ __forceinline__ void SmallDotTile(int tiles_m, int& tm, int& tn) {
     const int tile = xcd * q + min(xcd, r) + loc;
     tn = tile / tiles_m;
     tm = tile - tn * tiles_m;
+}
+
+// One element of the product, with the bias of a Linear layer: Dot rounds its result, then Add adds the bias and rounds again.
+template <typename T>
+__device__ __forceinline__ void StoreDot(const SmallDotArgs& p, T* out, int m, int n, float s) {
+    T v = static_cast<T>(s);
+    if (p.bias != nullptr) v = static_cast<T>(static_cast<float>(v) + static_cast<float>(static_cast<const T*>(p.bias)[n * p.bias_stride]));
+    out[m * p.o_row + n * p.o_col] = v;
 }
 
 template <typename T>
@@ -217,7 +227,7 @@ __global__ __launch_bounds__(512) void SmallDotKernel(SmallDotArgs p) {
 #pragma unroll
         for (int w = 0; w < NW; ++w) s += part[w][row * 33 + col];
         int om = tm * 32 + row, on = tn * 32 + col;
-        if (om < p.M && on < p.N) out[om * p.o_row + on * p.o_col] = static_cast<T>(s);
+        if (om < p.M && on < p.N) StoreDot<T>(p, out, om, on, s);
     }
 }
 
@@ -323,7 +333,7 @@ __global__ __launch_bounds__(512) void SmallDotRowsKernel(SmallDotArgs p) {
         float s = 0.f;
         for (int w = 0; w < p.nw; ++w) s += part[w * (32 * 33) + row * 33 + col];
         const int om = tm * 32 + row, on = tn * 32 + col;
-        if (om < p.M && on < p.N) out[om * p.o_row + on * p.o_col] = static_cast<T>(s);
+        if (om < p.M && on < p.N) StoreDot<T>(p, out, om, on, s);
     }
 }
 

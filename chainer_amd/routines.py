@@ -2,8 +2,9 @@
 
 Each function mirrors one routine of ``CX/routines/*.cc``: the same dtype promotion, broadcasting,
 output allocation and -- most importantly -- the same decomposition into kernel calls, one
-``hipcx_*`` call per ``CallKernel<...>`` of the reference.  Nothing is fused here that the
-reference does not fuse; the fused entry points live in ``chainer_amd.fused`` and are opt-in.
+``hipcx_*`` call per ``CallKernel<...>`` of the reference.  A chain that belongs to one routine (Linear's Dot and Add, Sigmoid,
+LogSoftmax, the Lstm cell, softmax cross entropy) runs as one kernel where its arrays allow; nothing is fused across routines
+except by the opt-in ``conv_bn_act``.
 """
 import builtins as _py
 import ctypes
@@ -671,16 +672,18 @@ def logsumexp(x, axis=None, keepdims=False):
 
 
 def log_softmax(x, axis=None):
-    """LogSoftmax = x - LogSumExp(x, axis or 1, keepdims) (CX/routines/reduction.cc:88-92): seven kernels."""
+    """LogSoftmax = x - LogSumExp(x, axis or 1, keepdims) (CX/routines/reduction.cc:88-92): hipcx_log_softmax (one or two kernels) along
+    the dense axis 1 of a matrix, seven kernels otherwise."""
+    out = _host.log_softmax_direct(x, axis)
+    if out is not None:
+        return out
     xc = x.astype(_math_result_dtype(x.dtype), False)
     return subtract(xc, logsumexp(xc, 1 if axis is None else axis, True))
 
 
 def log_softmax_fused(x, axis=None):
-    """Opt-in: LogSoftmax (CX/routines/reduction.cc:88-92) through hipcx_log_softmax -- one or two kernels instead of seven.
-    Arrays the fused kernel does not take (ndim != 2, another axis, strided rows) go through log_softmax."""
-    out = _host.log_softmax_direct(x, axis)
-    return log_softmax(x, axis) if out is None else out
+    """LogSoftmax through hipcx_log_softmax, which log_softmax takes by itself for every array the kernel covers."""
+    return log_softmax(x, axis)
 
 
 def softmax(x, axis=None):
@@ -1362,7 +1365,8 @@ def average_pool_grad(x, gout, ksize, stride=None, pad=0, pad_mode='ignore'):
 # composite routines
 # ---------------------------------------------------------------------------------------------
 def lstm(c, x):
-    """Lstm cell (CX/routines/connection.cc:396-446), equal batch sizes: gates are stride-4 views of x."""
+    """Lstm cell (CX/routines/connection.cc:396-446), equal batch sizes: gates are stride-4 views of x.  hipcx_lstm_cell for matrices
+    with dense rows, ~25 kernels otherwise."""
     if x.shape[0] > c.shape[0]:
         raise _lib.DimensionError('The batch size of x must be equal to or less than the size of c')
     if x.shape[1] != 4 * c.shape[1]:
@@ -1373,6 +1377,9 @@ def lstm(c, x):
         raise _lib.DtypeError('Datatypes of c and x should be equal')
     if x.shape[0] != c.shape[0]:
         raise _lib.ChainerxNotImplementedError('ragged batches are not on the supported path')
+    fused = _host.lstm_cell(c, x)
+    if fused is not None:
+        return fused
     xr = x.reshape((x.shape[0], x.shape[1] // 4, 4) + tuple(x.shape[2:]))
     gates = [g.squeeze(2) for g in split(xr, 4, 2)]
     a = tanh(gates[0])
@@ -1385,10 +1392,8 @@ def lstm(c, x):
 
 
 def lstm_fused(c, x):
-    """Opt-in: the Lstm cell through hipcx_lstm_cell -- one kernel instead of ~25; same checks and errors as lstm."""
-    if c.ndim != 2 or x.ndim != 2:
-        return lstm(c, x)
-    return _host.lstm_cell(c, x)
+    """The Lstm cell through hipcx_lstm_cell, which lstm takes by itself for every call the kernel covers."""
+    return lstm(c, x)
 
 
 def clipped_relu(x, z):
@@ -1703,7 +1708,11 @@ def n_step_birnn(n_layers, hx, ws, bs, xs, activation='tanh', kernel=False):
 
 def softmax_cross_entropy(x, t):
     """Chainer's F.softmax_cross_entropy forward for chainerx arrays with the default reduce='mean', normalize=True
-    (chainer/functions/loss/softmax_cross_entropy.py:123-130): a Python-level composition, 15 kernel calls."""
+    (chainer/functions/loss/softmax_cross_entropy.py:123-130): one or two kernels for a matrix with dense rows and labels whose dtype
+    holds every class, the reference's composition (15 kernel calls) otherwise."""
+    loss = _host.softmax_cross_entropy_direct(x, t)
+    if loss is not None:
+        return loss
     score = log_softmax(x, 1)
     mask = equal(t[:, None], arange(score.shape[1], dtype=t.dtype)).astype(score.dtype)
     return multiply(sum(multiply(score, mask)), divide(-1, sum(mask)))

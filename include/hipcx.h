@@ -202,7 +202,9 @@ enum hipcx_unary_op {
     HIPCX_UNARY_SINH, HIPCX_UNARY_COSH, HIPCX_UNARY_ARCSINH, HIPCX_UNARY_ARCCOSH,
     HIPCX_UNARY_SIN, HIPCX_UNARY_COS, HIPCX_UNARY_TAN, HIPCX_UNARY_ARCSIN, HIPCX_UNARY_ARCCOS, HIPCX_UNARY_ARCTAN,
     HIPCX_UNARY_CEIL, HIPCX_UNARY_FLOOR,
-    HIPCX_UNARY_SQUARE, HIPCX_UNARY_ABS, HIPCX_UNARY_SIGN
+    HIPCX_UNARY_SQUARE, HIPCX_UNARY_ABS, HIPCX_UNARY_SIGN,
+    HIPCX_UNARY_SIGMOID /* the Sigmoid routine (CX/routines/activation.cc:74-78: Multiply by -1, Exp, Add 1, Divide 1 by it) in one
+                           pass, rounded to the array's dtype after every one of those steps: the bits of the chain */
 };
 int hipcx_unary(int op, const hipcx_array* x, const hipcx_array* out, void* stream);
 
@@ -290,6 +292,10 @@ int hipcx_sum_static_scratch(const hipcx_array* a, const int8_t* axis, int naxis
  * accumulator of the array dtype, i.e. sums modulo 2^bits; bool is "any of the conjunctions") by a plain tiled kernel -- the cuda
  * backend raises for them (CX/cuda/cuda_device/dot.cu:74-76). */
 size_t hipcx_dot_workspace_size(const hipcx_array* a, const hipcx_array* b, const hipcx_array* out);
+/* hipcx_dot followed by AddKernel with a stride-0 row, as the Linear routine issues them (CX/routines/connection.cc:379-392), with the
+ * addition in the product's epilogue: `bias` has one element per column of out.  Workspace as for hipcx_dot. */
+int hipcx_dot_bias(const hipcx_array* a, const hipcx_array* b, const hipcx_array* bias, const hipcx_array* out, void* workspace,
+                   size_t workspace_bytes, void* stream);
 int hipcx_dot(const hipcx_array* a, const hipcx_array* b, const hipcx_array* out, void* workspace, size_t workspace_bytes,
               void* stream);
 /* Output extent of a convolution/pooling window (CX/routines/connection.cc:37-49). Returns -1 if not positive. */
@@ -401,6 +407,14 @@ int hipcx_n_step_rnn_backward(int n_layers, int bidirectional, int mode, int act
 size_t hipcx_log_softmax_workspace_size(const hipcx_array* x);
 int hipcx_log_softmax(const hipcx_array* x, const hipcx_array* out, void* workspace, size_t workspace_bytes, void* stream);
 int hipcx_lstm_cell(const hipcx_array* c, const hipcx_array* x, const hipcx_array* h_out, const hipcx_array* c_out, void* stream);
+/* hipcx_softmax_cross_entropy: F.softmax_cross_entropy for chainerx arrays (chainer/functions/loss/softmax_cross_entropy.py:123-130:
+ *   LogSoftmax, a one-hot mask from Equal(t[:, None], Arange(n)), -sum(score * mask) / sum(mask); about 15 kernels) as one kernel, or
+ *   two for large batches.  x [B, n] float, dense along axis 1; t [B], an integer dtype that can hold n - 1; out: one element of x's
+ *   dtype.  A label outside [0, n) selects nothing and does not count, as in the mask; the values summed are rounded to x's dtype
+ *   where the chain stores them, sums run in double.  `workspace`: hipcx_softmax_cross_entropy_workspace_size(x) bytes. */
+size_t hipcx_softmax_cross_entropy_workspace_size(const hipcx_array* x);
+int hipcx_softmax_cross_entropy(const hipcx_array* x, const hipcx_array* t, const hipcx_array* out, void* workspace, size_t workspace_bytes,
+                                void* stream);
 
 /* Measurement aid (no counterpart in the reference): between start and stop every implicit-GEMM launch made by
  * hipcx_dot / hipcx_conv from the calling process is bracketed by a pair of HIP events on its stream.  stop waits for them
