@@ -269,16 +269,16 @@ __device__ __forceinline__ T FromLaneAbove(T v) {
 }
 
 template <typename In>
-struct alignas(sizeof(In) * 4) Group4 {
+struct Group4 {
     In v[4];
 };
 
-template <bool ALIGNED, typename In>
+// One load of up to 16 bytes at any address: rows of odd length start anywhere, and the hardware takes vector loads there too
+// ([333, 1001] float16 along axis 1, bound by latency, 4.0 -> 3.7 us).
+template <typename In>
 __device__ __forceinline__ Group4<In> LoadGroup(const In* p) {
-    if (ALIGNED) return *reinterpret_cast<const Group4<In>*>(p);
     Group4<In> q;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) q.v[j] = p[j];
+    __builtin_memcpy(&q, p, sizeof(q));
     return q;
 }
 
@@ -331,7 +331,7 @@ __device__ __forceinline__ typename Op::Acc MergeRows(typename Op::Acc acc) {
     return d;
 }
 
-template <typename Impl, bool ALIGNED>
+template <typename Impl>
 __global__ __launch_bounds__(kRowThreads) void RowReduceKernel(ReduceGeom g, int64_t span, int blocks_per_row, void* partials) {
     using R = typename Impl::Row;  // the same reduction with indices counted from the block's first element
     using In = typename R::In;
@@ -467,7 +467,7 @@ __global__ __launch_bounds__(kRowThreads) void RowReduceKernel(ReduceGeom g, int
         const int local = it * kElemsPerIter + tid * 4;
         Acc gv = R::Empty();
         if (grp < G) {
-            const Group4<In> q = LoadGroup<ALIGNED>(at(grp * 4));
+            const Group4<In> q = LoadGroup(at(grp * 4));
             Acc p0 = R::Map(q.v[0], local);
             R::Reduce(R::Map(q.v[1], local + 1), p0);
             Acc p1 = R::Map(q.v[2], local + 2);
@@ -513,12 +513,12 @@ __global__ __launch_bounds__(kRowThreads) void RowReduceKernel(ReduceGeom g, int
     for (; it + kLoadBatch <= plain_iters; it += kLoadBatch) {
         Group4<In> q[kLoadBatch];
 #pragma unroll
-        for (int u = 0; u < kLoadBatch; ++u) q[u] = LoadGroup<ALIGNED>(xrow + static_cast<int64_t>(it + u) * kElemsPerIter);
+        for (int u = 0; u < kLoadBatch; ++u) q[u] = LoadGroup(xrow + static_cast<int64_t>(it + u) * kElemsPerIter);
         __builtin_amdgcn_sched_barrier(0);  // all loads in flight before anything waits for the first
         plain(it, q, std::integral_constant<int, kLoadBatch>());
     }
     for (; it < plain_iters; ++it) {
-        const Group4<In> q = LoadGroup<ALIGNED>(xrow + static_cast<int64_t>(it) * kElemsPerIter);
+        const Group4<In> q = LoadGroup(xrow + static_cast<int64_t>(it) * kElemsPerIter);
         plain(it, &q, std::integral_constant<int, 1>());
     }
     for (; it < iters; ++it) guarded(it);
@@ -645,97 +645,173 @@ __global__ __launch_bounds__(256) void GenericReduceKernel(ReduceGeom g) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// Column kernels: one strided reduced axis, few outputs against its length (sums over the batch axis, bias gradients).
-// The reduced sequence is cut into `nslices` aligned slices of 2^level 32-element blocks.  Pass 1: one thread per
-// (slice, output), outputs fastest (coalesced for an inner kept axis), runs the reference loop over its slice -- whose
-// result is exactly the node the sequential binary counter would hold for those blocks.  Pass 2: one thread per output
-// pushes the slice nodes through the counter, then walks on through the blocks after the last slice (at least one is
-// always left, so the tail and the final fold happen exactly where the reference has them).
+// Column kernels: one strided reduced axis (sums over the batch axis, bias gradients, axis 0 of a matrix).
+//
+// Bound by memory: every element is read once.  A thread owns V neighbouring outputs (one 16-byte load per row) and one 32-element
+// chunk of the reduced axis; 256 / CL threads of a workgroup hold consecutive chunks of the same outputs and their chunk results are
+// merged in LDS as the aligned binary tree the native counter builds, so a workgroup leaves the node of a slice of 256 / CL chunks.
+// The last chunk takes the groups short of a full one and the up to three leftover elements.  ColumnFinishKernel merges the slice
+// nodes (an aligned tree as well; missing nodes at the end are padding, which a merge passes through).
+// 4096 x 4096 float32 along axis 0: 64 us (a thread per output and slice, one serial pass over the slice nodes) -> 18 us.
+// Rows of any alignment take the vector loads (the hardware reads 16 bytes from any address); where V does not divide a row, its last
+// vector starts V before the end and repeats a few outputs of its neighbour, which costs less than a branch around every load.
 // ---------------------------------------------------------------------------------------------
-template <typename Impl>
-__global__ __launch_bounds__(256) void ColumnSliceKernel(ReduceGeom g, int level, int nslices, void* partials) {
+template <typename In, int V>
+struct Row16 {
+    In v[V];
+};
+
+template <typename Impl, int V, int CL>
+__global__ __launch_bounds__(256) void ColumnChunkKernel(ReduceGeom g, int64_t nchunks, int nslices, int64_t inner, int64_t vecs_per_row, int64_t col_blocks,
+                                                         void* partials) {
     using In = typename Impl::In;
     using Acc = typename Impl::Acc;
-    const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (t >= g.n_out * nslices) return;
-    const int64_t slice = t / g.n_out;
-    const int64_t o = t - slice * g.n_out;
-    int64_t in_off, out_off;
-    OutOffsets(g, o, in_off, out_off);
-    const int64_t stride = g.red_stride[0];
-    const int64_t count = static_cast<int64_t>(32) << level;
-    const int64_t i_begin = slice * count;
-    const char* ptr = g.in + in_off + i_begin * stride;
-    Acc accum = Impl::Identity();
-    Acc tree[32];
-    for (int64_t r = 0; r < count; r += 4) {
-        if (r != 0 && r % 32 == 0) {
-            int lvl = 0;
-            for (int64_t k = r >> 1; k % 32 == 0; k >>= 1, ++lvl) Impl::Reduce(tree[lvl], accum);
-            tree[lvl] = accum;
-            accum = Impl::Identity();
+    constexpr int RL = 256 / CL;
+    static_assert(CL * V <= 256, "one thread folds a column of nodes");
+    __shared__ Acc nodes[RL][CL * V];
+    const int cl = threadIdx.x % CL, rl = threadIdx.x / CL;
+    const int64_t slice = blockIdx.x / col_blocks;
+    const int64_t unit = (blockIdx.x - slice * col_blocks) * CL + cl;  // V outputs of one row of the innermost kept axis
+    const int64_t outer = unit / vecs_per_row;
+    const int64_t c = (unit - outer * vecs_per_row) * V;
+    const int64_t o0 = outer * inner + (c + V <= inner ? c : inner - V);
+    const int64_t chunk = slice * RL + rl;
+    Acc acc[V];
+#pragma unroll
+    for (int v = 0; v < V; ++v) acc[v] = Impl::Empty();
+    if (o0 < g.n_out && chunk < nchunks) {
+        int64_t in_off, out_off;
+        OutOffsets(g, o0, in_off, out_off);
+        const int64_t stride = g.red_stride[0];
+        const int64_t i0 = chunk * 32;
+        const char* ptr = g.in + in_off + i0 * stride;
+        const int64_t main_len = g.red_len - g.red_len % 4;
+        const int64_t left = main_len - i0;
+        const int groups = left >= 32 ? 8 : static_cast<int>(left / 4);
+#pragma unroll
+        for (int v = 0; v < V; ++v) acc[v] = Impl::Identity();
+        auto load = [](const char* q) {
+            Row16<In, V> r;
+            __builtin_memcpy(&r, q, sizeof(r));
+            return r;
+        };
+        auto fold = [&](const Row16<In, V>* r, int64_t i) {
+#pragma unroll
+            for (int v = 0; v < V; ++v) {
+                Acc p0 = Impl::Map(r[0].v[v], i);
+                Impl::Reduce(Impl::Map(r[1].v[v], i + 1), p0);
+                Acc p1 = Impl::Map(r[2].v[v], i + 2);
+                Impl::Reduce(Impl::Map(r[3].v[v], i + 3), p1);
+                Impl::Reduce(p1, p0);
+                Impl::Reduce(p0, acc[v]);
+            }
+        };
+        if (groups == 8) {
+#pragma unroll 1
+            for (int b = 0; b < 32; b += 16) {  // 16 rows in flight at a time
+                Row16<In, V> r[16];
+#pragma unroll
+                for (int k = 0; k < 16; ++k) {
+                    r[k] = load(ptr);
+                    ptr += stride;
+                }
+#pragma unroll
+                for (int k = 0; k < 4; ++k) fold(r + 4 * k, i0 + b + 4 * k);
+            }
+        } else {
+#pragma unroll 1
+            for (int k = 0; k < groups; ++k) {
+                Row16<In, V> r[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    r[e] = load(ptr);
+                    ptr += stride;
+                }
+                fold(r, i0 + 4 * k);
+            }
         }
-        const int64_t i = i_begin + r;
-        Acc p0 = Impl::Map(*reinterpret_cast<const In*>(ptr), i);
-        Impl::Reduce(Impl::Map(*reinterpret_cast<const In*>(ptr + stride), i + 1), p0);
-        Acc p1 = Impl::Map(*reinterpret_cast<const In*>(ptr + 2 * stride), i + 2);
-        Impl::Reduce(Impl::Map(*reinterpret_cast<const In*>(ptr + 3 * stride), i + 3), p1);
-        Impl::Reduce(p1, p0);
-        Impl::Reduce(p0, accum);
-        ptr += 4 * stride;
+        if (chunk == nchunks - 1) {
+#pragma unroll 1
+            for (int64_t i = main_len; i < g.red_len; ++i, ptr += stride) {
+                const Row16<In, V> r = load(ptr);
+#pragma unroll
+                for (int v = 0; v < V; ++v) Impl::Reduce(Impl::Map(r.v[v], i), acc[v]);
+            }
+        }
     }
-    for (int lvl = 0; lvl < level; ++lvl) Impl::Reduce(tree[lvl], accum);  // 2^level blocks: every lower level is pending
-    reinterpret_cast<Acc*>(partials)[slice * g.n_out + o] = accum;
+#pragma unroll
+    for (int v = 0; v < V; ++v) nodes[rl][cl * V + v] = acc[v];
+    __syncthreads();
+    const int t = threadIdx.x;
+    if (t >= CL * V) return;
+    Acc a[RL];
+#pragma unroll
+    for (int r = 0; r < RL; ++r) a[r] = nodes[r][t];
+#pragma unroll
+    for (int s = 1; s < RL; s <<= 1) {
+#pragma unroll
+        for (int r = 0; r < RL; r += 2 * s) {
+            Impl::Reduce(a[r], a[r + s]);
+            a[r] = a[r + s];
+        }
+    }
+    const int64_t unit_t = (blockIdx.x - slice * col_blocks) * CL + t / V;
+    const int64_t outer_t = unit_t / vecs_per_row;
+    const int64_t c_t = (unit_t - outer_t * vecs_per_row) * V;
+    const int64_t o = outer_t * inner + (c_t + V <= inner ? c_t : inner - V) + t % V;
+    if (o >= g.n_out) return;
+    if (nslices == 1) {
+        int64_t in_off, out_off;
+        OutOffsets(g, o, in_off, out_off);
+        *reinterpret_cast<typename Impl::Out*>(g.out + out_off) = Impl::MapOut(a[0]);
+    } else {
+        static_cast<Acc*>(partials)[slice * g.n_out + o] = a[0];
+    }
 }
 
-template <typename Impl>
-__global__ __launch_bounds__(256) void ColumnFinishKernel(ReduceGeom g, int level, int nslices, const void* partials) {
-    using In = typename Impl::In;
+// SL threads share an output; each first merges an aligned run of 2^run_level slice nodes.
+template <typename Impl, int SL>
+__global__ __launch_bounds__(256) void ColumnFinishKernel(ReduceGeom g, int nslices, int run_level, const void* partials) {
     using Acc = typename Impl::Acc;
-    const int64_t o = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (o >= g.n_out) return;
-    int64_t in_off, out_off;
-    OutOffsets(g, o, in_off, out_off);
-    const int64_t stride = g.red_stride[0];
-    const Acc* part = reinterpret_cast<const Acc*>(partials);
-    Acc tree[48];
-    Acc accum;
-    for (int s = 0; s < nslices; ++s) {  // the boundary merges of the reference at the end of every slice
-        accum = part[static_cast<int64_t>(s) * g.n_out + o];
-        int lvl = level;
-        for (int t = s; t & 1; t >>= 1, ++lvl) Impl::Reduce(tree[lvl], accum);
-        tree[lvl] = accum;
-    }
-    const int64_t len = g.red_len;
-    const int64_t main_len = len - (len % 4);
-    const int64_t i0 = static_cast<int64_t>(nslices) * (static_cast<int64_t>(32) << level);
-    const char* ptr = g.in + in_off + i0 * stride;
-    int64_t i = i0;
-    accum = Impl::Identity();
-    while (i < main_len) {
-        if (i != i0 && i % 32 == 0) {
+    constexpr int CF = 256 / SL;
+    __shared__ Acc nodes[SL][CF];
+    const int c = threadIdx.x % CF, sl = threadIdx.x / CF;
+    const int64_t o = static_cast<int64_t>(blockIdx.x) * CF + c;
+    const Acc* part = static_cast<const Acc*>(partials);
+    Acc acc = Impl::Empty();
+    if (o < g.n_out) {
+        const int64_t first = static_cast<int64_t>(sl) << run_level;
+        const int64_t count = nslices - first < (1LL << run_level) ? nslices - first : (1LL << run_level);
+        if (run_level == 0) {
+            if (count > 0) acc = part[first * g.n_out + o];
+        } else {
+            Acc tree[24];
+            for (int64_t s = 0; s < count; ++s) {
+                Acc node = part[(first + s) * g.n_out + o];
+                int lvl = 0;
+                for (int64_t k = s; k & 1; k >>= 1, ++lvl) Impl::Reduce(tree[lvl], node);
+                tree[lvl] = node;
+            }
             int lvl = 0;
-            for (int64_t k = i >> 1; k % 32 == 0; k >>= 1, ++lvl) Impl::Reduce(tree[lvl], accum);
-            tree[lvl] = accum;
-            accum = Impl::Identity();
-        }
-        Acc p0 = Impl::Map(*reinterpret_cast<const In*>(ptr), i);
-        Impl::Reduce(Impl::Map(*reinterpret_cast<const In*>(ptr + stride), i + 1), p0);
-        Acc p1 = Impl::Map(*reinterpret_cast<const In*>(ptr + 2 * stride), i + 2);
-        Impl::Reduce(Impl::Map(*reinterpret_cast<const In*>(ptr + 3 * stride), i + 3), p1);
-        Impl::Reduce(p1, p0);
-        Impl::Reduce(p0, accum);
-        ptr += 4 * stride;
-        i += 4;
-    }
-    for (; i < len; ++i, ptr += stride) Impl::Reduce(Impl::Map(*reinterpret_cast<const In*>(ptr), i), accum);
-    {
-        int lvl = 0;
-        for (int64_t k = (len / 4 - 1) / 8; k > 0; k >>= 1, ++lvl) {
-            if (k & 1) Impl::Reduce(tree[lvl], accum);
+            for (int64_t k = count > 0 ? count : 0; k > 0; k >>= 1, ++lvl) {
+                if (k & 1) Impl::Reduce(tree[lvl], acc);
+            }
         }
     }
-    *reinterpret_cast<typename Impl::Out*>(g.out + out_off) = Impl::MapOut(accum);
+    nodes[sl][c] = acc;
+    for (int s = 1; s < SL; s <<= 1) {
+        __syncthreads();
+        if (sl % (2 * s) == 0) {
+            Acc later = nodes[sl + s][c];
+            Impl::Reduce(nodes[sl][c], later);
+            nodes[sl][c] = later;
+        }
+    }
+    if (sl == 0 && o < g.n_out) {
+        int64_t in_off, out_off;
+        OutOffsets(g, o, in_off, out_off);
+        *reinterpret_cast<typename Impl::Out*>(g.out + out_off) = Impl::MapOut(nodes[0][c]);
+    }
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -744,13 +820,15 @@ __global__ __launch_bounds__(256) void ColumnFinishKernel(ReduceGeom g, int leve
 struct ReducePlan {
     ReduceGeom g;
     bool row_path = false;
-    bool aligned = false;
     int64_t span = 0;
     int blocks_per_row = 1;
     size_t acc_size = 0;
     bool column_path = false;
-    int col_level = 0;    // a slice is 2^col_level blocks of 32 elements
-    int col_slices = 0;
+    int col_vec = 1;      // outputs per thread: 16 bytes of the innermost kept axis, or 1
+    int col_lanes = 64;   // threads along the outputs: 16 or 64 (then 16 or 4 chunks of 32 elements to a workgroup)
+    int64_t col_chunks = 0;
+    int col_slices = 0;   // workgroups along the reduced axis
+    int64_t col_inner = 1, col_vecs_per_row = 1, col_blocks = 0;
 };
 
 ReduceGeom MakeGeom(const hipcx_array* a, const int8_t* axis, int naxis, const hipcx_array* out) {
@@ -852,42 +930,35 @@ ReducePlan MakePlan(const hipcx_array* a, const int8_t* axis, int naxis, const h
         } else {
             pl.span = span;
             pl.blocks_per_row = static_cast<int>(bpr);
-            bool al = reinterpret_cast<uintptr_t>(g.in) % (4 * it) == 0;
-            for (int d = 0; d < g.n_keep; ++d) al = al && g.keep_in_stride[d] % (4 * it) == 0;
-            al = al && g.seg_stride % (4 * it) == 0;
-            pl.aligned = al;
         }
     }
-    // Column path: one strided reduced axis that is long against the number of outputs (one thread per output would walk it alone).
-    if (!pl.row_path && g.n_red == 1 && g.red_len >= 512 && g.n_out > 0 && g.n_out < (1LL << 28)) {
-        const int64_t main_len = g.red_len - g.red_len % 4;
-        const int64_t nblocks = (main_len + 31) / 32;
-        // Serial work of the longest thread: a slice in pass 1 (times the rounds the chip needs for all slice threads), then
-        // in pass 2 the slice nodes plus the blocks behind the last slice.  Take the slice size that minimises it.
-        const int64_t resident = static_cast<int64_t>(NumCUs()) * 2048;
-        int best_level = -1;
-        int64_t best_cost = g.red_len;  // the generic kernel's: one thread walks everything
-        for (int level = 0; level < 24; ++level) {
-            const int64_t slices = (nblocks - 1) >> level;  // at least one block stays behind the last slice
-            if (slices < 2) break;
-            if (slices > (1 << 20) || g.n_out * slices >= (1LL << 36)) continue;
-            const int64_t slice_len = static_cast<int64_t>(32) << level;
-            const int64_t rounds = (g.n_out * slices + resident - 1) / resident;
-            const int64_t left = g.red_len - slices * slice_len;
-            const int64_t cost = slice_len * rounds + slices + left;
-            if (cost < best_cost) best_cost = cost, best_level = level;
-        }
-        if (best_level >= 0 && 2 * best_cost <= g.red_len) {
+    // Column path: one strided reduced axis of at least a chunk (below that a thread per output reads its few rows itself).
+    if (!pl.row_path && g.n_red == 1 && g.red_stride[0] != it && g.red_len >= 32 && g.n_out > 0 && g.n_out < (1LL << 28)) {
+        const int64_t chunks = (g.red_len / 4 + 7) / 8;
+        const int last = g.n_keep - 1;
+        pl.col_inner = last >= 0 ? g.keep_shape[last] : 1;
+        // a vector needs neighbouring outputs next to each other in memory, and rows worth one
+        const int vec = static_cast<int>(16 / it < 8 ? 16 / it : 8);
+        pl.col_vec = last >= 0 && g.keep_in_stride[last] == it && pl.col_inner >= vec ? vec : 1;
+        pl.col_vecs_per_row = (pl.col_inner + pl.col_vec - 1) / pl.col_vec;
+        // 16 lanes of 16 bytes are a 256-byte piece of a row and leave 16 chunks to a workgroup; few chunks, or outputs read one by
+        // one, take 64 lanes and 4 chunks (one thread folds a column of nodes: 64 lanes hold at most four outputs each)
+        pl.col_lanes = (chunks <= 4 && pl.col_vec <= 4) || pl.col_vec == 1 ? 64 : 16;
+        const int64_t units = g.n_out / pl.col_inner * pl.col_vecs_per_row;
+        pl.col_blocks = (units + pl.col_lanes - 1) / pl.col_lanes;
+        const int64_t per_slice = 256 / pl.col_lanes;
+        const int64_t slices = (chunks + per_slice - 1) / per_slice;
+        if (slices < (1LL << 30) && pl.col_blocks * slices < (1LL << 31)) {
             pl.column_path = true;
-            pl.col_level = best_level;
-            pl.col_slices = static_cast<int>((nblocks - 1) >> best_level);
+            pl.col_chunks = chunks;
+            pl.col_slices = static_cast<int>(slices);
         }
     }
     return pl;
 }
 
 size_t WorkspaceBytes(const ReducePlan& pl) {
-    if (pl.column_path) return static_cast<size_t>(pl.g.n_out) * pl.col_slices * pl.acc_size;
+    if (pl.column_path) return pl.col_slices > 1 ? static_cast<size_t>(pl.g.n_out) * pl.col_slices * pl.acc_size : 0;
     if (!pl.row_path || pl.blocks_per_row == 1) return 0;
     return static_cast<size_t>(pl.g.n_out) * pl.blocks_per_row * pl.acc_size;
 }
@@ -905,11 +976,7 @@ void Run(const hipcx_array* a, const int8_t* axis, int naxis, const hipcx_array*
         HIPCX_REQUIRE(need == 0 || reinterpret_cast<uintptr_t>(workspace) % 16 == 0, HIPCX_CHAINERX_ERROR,
                       "workspace must be 16-byte aligned");
         dim3 grid(static_cast<unsigned>(g.n_out * pl.blocks_per_row)), block(kRowThreads);
-        if (pl.aligned) {
-            hipLaunchKernelGGL((RowReduceKernel<Impl, true>), grid, block, 0, stream, g, pl.span, pl.blocks_per_row, workspace);
-        } else {
-            hipLaunchKernelGGL((RowReduceKernel<Impl, false>), grid, block, 0, stream, g, pl.span, pl.blocks_per_row, workspace);
-        }
+        hipLaunchKernelGGL((RowReduceKernel<Impl>), grid, block, 0, stream, g, pl.span, pl.blocks_per_row, workspace);
         CheckLaunch("row_reduce");
         if (pl.blocks_per_row > 1) {
             hipLaunchKernelGGL((RowFinalizeKernel<Impl>), dim3(static_cast<unsigned>(g.n_out)), block, 0, stream, g, pl.blocks_per_row,
@@ -920,15 +987,38 @@ void Run(const hipcx_array* a, const int8_t* axis, int naxis, const hipcx_array*
     }
     if (pl.column_path) {
         size_t need = WorkspaceBytes(pl);
-        HIPCX_REQUIRE(workspace != nullptr && workspace_bytes >= need, HIPCX_CHAINERX_ERROR,
+        HIPCX_REQUIRE(need == 0 || (workspace != nullptr && workspace_bytes >= need), HIPCX_CHAINERX_ERROR,
                       "reduction workspace too small: need " + std::to_string(need) + " bytes");
-        HIPCX_REQUIRE(reinterpret_cast<uintptr_t>(workspace) % 16 == 0, HIPCX_CHAINERX_ERROR, "workspace must be 16-byte aligned");
-        const int64_t threads = g.n_out * pl.col_slices;
-        hipLaunchKernelGGL((ColumnSliceKernel<Impl>), dim3(static_cast<unsigned>((threads + 255) / 256)), dim3(256), 0, stream, g, pl.col_level,
-                           pl.col_slices, workspace);
-        CheckLaunch("column_reduce_slices");
-        hipLaunchKernelGGL((ColumnFinishKernel<Impl>), dim3(static_cast<unsigned>((g.n_out + 255) / 256)), dim3(256), 0, stream, g, pl.col_level,
-                           pl.col_slices, workspace);
+        HIPCX_REQUIRE(need == 0 || reinterpret_cast<uintptr_t>(workspace) % 16 == 0, HIPCX_CHAINERX_ERROR, "workspace must be 16-byte aligned");
+        const dim3 grid(static_cast<unsigned>(pl.col_blocks * pl.col_slices)), block(256);
+        constexpr int VEC = 16 / sizeof(typename Impl::In) < 8 ? 16 / sizeof(typename Impl::In) : 8;
+        auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, grid, block, 0, stream, g, pl.col_chunks, pl.col_slices, pl.col_inner, pl.col_vecs_per_row, pl.col_blocks, workspace);
+        };
+        if (pl.col_vec == 1) {
+            launch(ColumnChunkKernel<Impl, 1, 64>);
+        } else if (pl.col_lanes == 16) {
+            launch(ColumnChunkKernel<Impl, VEC, 16>);
+        } else {
+            if constexpr (VEC <= 4) launch(ColumnChunkKernel<Impl, VEC, 64>);
+        }
+        CheckLaunch("column_reduce_chunks");
+        if (pl.col_slices == 1) return;
+        // as many threads to an output as there are slice nodes, up to 256
+        auto finish = [&](auto kernel, int sl) {
+            int level = 0;
+            while ((static_cast<int64_t>(sl) << level) < pl.col_slices) ++level;
+            const int64_t per_block = 256 / sl;
+            hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>((g.n_out + per_block - 1) / per_block)), block, 0, stream, g, pl.col_slices, level,
+                               workspace);
+        };
+        if (pl.col_slices <= 16) {
+            finish(ColumnFinishKernel<Impl, 16>, 16);
+        } else if (pl.col_slices <= 64) {
+            finish(ColumnFinishKernel<Impl, 64>, 64);
+        } else {
+            finish(ColumnFinishKernel<Impl, 256>, 256);
+        }
         CheckLaunch("column_reduce_finish");
         return;
     }
