@@ -42,6 +42,8 @@ struct LinspaceOp {
         double value = n == 1 ? start : (start * static_cast<double>(n - 1 - i) + stop * static_cast<double>(i)) / static_cast<double>(n - 1);
         if constexpr (std::is_same<T, bool>::value) {
             return value != 0.0;
+        } else if constexpr (std::is_integral<T>::value) {
+            return static_cast<T>(static_cast<int64_t>(value));  // negative values wrap in an unsigned array
         } else {
             return static_cast<compute_t<T>>(value);
         }
