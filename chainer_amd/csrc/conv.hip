@@ -239,51 +239,151 @@ bool TryGemmPp(const hipcx_array* a, const hipcx_array* b, const hipcx_array* bi
     return true;
 }
 
-// Small-output matrix products (small_dot.h).  Returns false when the problem does not qualify.
+// Workgroups that share a tile's reduction: while tiles leave compute units without one, but at least 896 bytes of a row each.
+int PlanSmallDotSplit(int64_t m, int64_t n, int64_t k, int dtype) {
+    const int64_t tiles = ((m + 31) / 32) * ((n + 31) / 32), lines = (k * ItemSize(dtype) + 127) / 128;
+    const int64_t s = std::min<int64_t>({NumCUs() / tiles, lines / 7, 32});
+    return s > 1 ? static_cast<int>(s) : 1;
+}
+
+// Splitting pays for the extra pass over the partial sums (3-4 us) once a tile's reduction takes longer than that on one compute unit:
+// 0.11 us per 128 bytes of its rows in float32 (16 MFMAs), 0.065 us in float16 (fetching the lines).
+int SmallDotSplit(int64_t m, int64_t n, int64_t k, int dtype) {
+    const int64_t lines = (k * ItemSize(dtype) + 127) / 128;
+    return lines >= (dtype == HIPCX_FLOAT32 ? 48 : 80) ? PlanSmallDotSplit(m, n, k, dtype) : 1;
+}
+
+size_t SmallDotPartialBytes(int64_t m, int64_t n, int64_t k, int dtype) {
+    const int split = SmallDotSplit(m, n, k, dtype);
+    return split > 1 ? static_cast<size_t>(split) * m * n * sizeof(float) : 0;
+}
+
+bool SmallDotShape(int64_t m, int64_t n, int64_t k) { return ((m + 127) / 128) * ((n + 127) / 128) < 128 && k >= 64; }
+
+// Fills in the operands; false when their strides or spans rule the kernels out.
 template <typename T>
-bool TrySmallDot(const hipcx_array* a, const hipcx_array* b, const hipcx_array* bias, const hipcx_array* out, hipStream_t stream) {
-    static const bool enabled = [] { const char* e = getenv("HIPCX_SMALL_DOT"); return e == nullptr || e[0] != '0'; }();
-    if (!enabled) return false;
+bool SmallDotOperands(const hipcx_array* a, const hipcx_array* b, SmallDotArgs* p, int* a_mode, int* b_mode) {
     const int64_t M = a->shape[0], K = a->shape[1], N = b->shape[1];
     const int64_t it = sizeof(T);
-    if (((M + 127) / 128) * ((N + 127) / 128) >= 128 || K < 64) return false;
-    for (const hipcx_array* x : {a, b, out}) {
+    for (const hipcx_array* x : {a, b}) {
         if (x->strides[0] < 0 || x->strides[1] < 0 || x->strides[0] % it || x->strides[1] % it) return false;
     }
+    p->a = a->data;
+    p->b = b->data;
+    p->M = static_cast<int>(M);
+    p->N = static_cast<int>(N);
+    p->K = static_cast<int>(K);
+    p->a_row = a->strides[0] / it;
+    p->a_k = a->strides[1] / it;
+    p->b_k = b->strides[0] / it;
+    p->b_col = b->strides[1] / it;
+    int64_t a_span = ((M - 1) * p->a_row + (K - 1) * p->a_k + 1) * it, b_span = ((K - 1) * p->b_k + (N - 1) * p->b_col + 1) * it;
+    if (a_span >= (1LL << 31) - 256 || b_span >= (1LL << 31) - 256) return false;
+    auto mode = [&](const void* ptr, int64_t k_stride, int64_t line_stride, int64_t* span) {
+        if (k_stride != 1 && K > 1) return static_cast<int>(kElements);
+        if (reinterpret_cast<uintptr_t>(ptr) % 4 == 0 && line_stride * it % 4 == 0) {
+            *span = (*span + 3) / 4 * 4;  // a last half element shares its (aligned) dword with the two bytes behind it
+            return static_cast<int>(kPieces);
+        }
+        return static_cast<int>(kOddPieces);
+    };
+    *a_mode = mode(a->data, p->a_k, p->a_row, &a_span);
+    *b_mode = mode(b->data, p->b_k, p->b_col, &b_span);
+    p->a_bytes = static_cast<unsigned>(a_span);
+    p->b_bytes = static_cast<unsigned>(b_span);
+    p->tiles_m = static_cast<int>((M + 31) / 32);
+    p->tiles_n = static_cast<int>((N + 31) / 32);
+    return true;
+}
+
+template <typename T, int AM, int BM, int P>
+void LaunchSmallDotPieces(const SmallDotArgs& p, dim3 grid, hipStream_t stream) {
+    constexpr int kWaveBytes = std::max<int>((P == 4) * ((AM != kElements) + (BM != kElements)) * kSmallDotStage, kSmallDotPart * sizeof(float));
+    struct SmallDotTag {};
+    EnsureDynamicLds<SmallDotTag>(reinterpret_cast<const void*>(SmallDotMixedKernel<T, AM, BM, P>), kSmallDotMaxWaves * kWaveBytes);
+    hipLaunchKernelGGL((SmallDotMixedKernel<T, AM, BM, P>), grid, dim3(64 * p.nw), p.nw * kWaveBytes, stream, p);
+    CheckLaunch("small_dot_mixed");
+}
+
+template <typename T, int AM, int BM>
+void LaunchSmallDotMixed(const SmallDotArgs& p, dim3 grid, int pieces, hipStream_t stream) {
+    if constexpr (AM != kOddPieces && BM != kOddPieces && (AM != kPieces || BM != kPieces)) {
+        if (pieces == 1) return LaunchSmallDotPieces<T, AM, BM, 1>(p, grid, stream);
+    }
+    LaunchSmallDotPieces<T, AM, BM, 4>(p, grid, stream);
+}
+
+// `batch` products (SmallDotArgs::outs) of p.ksplit workgroups per tile.
+template <typename T>
+void LaunchSmallDot(SmallDotArgs p, int a_mode, int b_mode, int batch, hipStream_t stream) {
+    const dim3 grid(static_cast<unsigned>(p.tiles_m * p.tiles_n * p.ksplit), static_cast<unsigned>(batch));
+    const bool latency_bound = static_cast<int64_t>(p.tiles_m) * p.tiles_n <= NumCUs();
+    const int lines = (p.K * static_cast<int>(sizeof(T)) + 127) / 128;
+    // with more tiles than compute units and a reduction of any length the whole lines of SmallDotMixedKernel are faster
+    // ([128,650] . [650,2600] 13.9 -> 13.4 us)
+    if (a_mode == kPieces && b_mode == kPieces && (latency_bound || lines <= 7)) {
+        hipLaunchKernelGGL((SmallDotKernel<T>), grid, dim3(512), 0, stream, p);
+        CheckLaunch("small_dot");
+        return;
+    }
+    // Elements wait for their own loads: chunks of 32 bytes, six of them in flight, beat whole lines while latency is what counts
+    // ([32,1000] . [1000,2048] float16 14.3 -> 5.5 us, [20,2600] . [2600,650] float32 13.4 -> 9.3); rows of odd pitch gain from whole
+    // lines at any size.
+    const int pieces = latency_bound && a_mode != kOddPieces && b_mode != kOddPieces ? 1 : 4;
+    // eight waves keep more loads in flight; four, one per SIMD, once there is a workgroup for every compute unit
+    const int chunk = pieces == 1 ? 32 : 128, chunks = (p.K * static_cast<int>(sizeof(T)) + chunk - 1) / chunk;
+    const int per_split = (chunks + p.ksplit - 1) / p.ksplit;
+    const int most = static_cast<int>(grid.x) * batch <= NumCUs() ? kSmallDotMaxWaves : 4;
+    const int per_wave = (per_split + most - 1) / most;
+    p.nw = (per_split + per_wave - 1) / per_wave;
+    auto with_a = [&](auto a_tag) {
+        constexpr int AM = decltype(a_tag)::value;
+        if (b_mode == kElements) return LaunchSmallDotMixed<T, AM, kElements>(p, grid, pieces, stream);
+        if constexpr (sizeof(T) == 2) {
+            if (b_mode == kOddPieces) return LaunchSmallDotMixed<T, AM, kOddPieces>(p, grid, pieces, stream);
+        }
+        LaunchSmallDotMixed<T, AM, kPieces>(p, grid, pieces, stream);
+    };
+    if (a_mode == kPieces) return with_a(std::integral_constant<int, kPieces>{});
+    if (a_mode == kElements) return with_a(std::integral_constant<int, kElements>{});
+    if constexpr (sizeof(T) == 2) with_a(std::integral_constant<int, kOddPieces>{});
+}
+
+// Small-output matrix products (small_dot.h).  Returns false when the problem does not qualify.  `partial` holds
+// SmallDotPartialBytes bytes; without it the reduction is not split.
+template <typename T>
+bool TrySmallDot(const hipcx_array* a, const hipcx_array* b, const hipcx_array* bias, const hipcx_array* out, float* partial, hipStream_t stream) {
+    static const bool enabled = [] { const char* e = getenv("HIPCX_SMALL_DOT"); return e == nullptr || e[0] != '0'; }();
+    const int64_t M = a->shape[0], K = a->shape[1], N = b->shape[1];
+    const int64_t it = sizeof(T);
+    if (!enabled || !SmallDotShape(M, N, K)) return false;
+    if (out->strides[0] < 0 || out->strides[1] < 0 || out->strides[0] % it || out->strides[1] % it) return false;
     SmallDotArgs p{};
-    p.a = a->data;
-    p.b = b->data;
+    int a_mode = 0, b_mode = 0;
+    if (!SmallDotOperands<T>(a, b, &p, &a_mode, &b_mode)) return false;
     p.out = out->data;
-    p.M = static_cast<int>(M);
-    p.N = static_cast<int>(N);
-    p.K = static_cast<int>(K);
-    p.a_row = a->strides[0] / it;
-    p.a_k = a->strides[1] / it;
-    p.b_k = b->strides[0] / it;
-    p.b_col = b->strides[1] / it;
     p.o_row = out->strides[0] / it;
     p.o_col = out->strides[1] / it;
-    int64_t a_span = ((M - 1) * p.a_row + (K - 1) * p.a_k + 1) * it, b_span = ((K - 1) * p.b_k + (N - 1) * p.b_col + 1) * it;
-    if (a_span >= (1LL << 31) || b_span >= (1LL << 31)) return false;
-    p.a_bytes = static_cast<unsigned>(a_span);
-    p.b_bytes = static_cast<unsigned>(b_span);
-    auto dword_ok = [&](const void* ptr, int64_t line_stride) { return reinterpret_cast<uintptr_t>(ptr) % 4 == 0 && (line_stride * it) % 4 == 0; };
-    p.a_vec = (p.a_k == 1 && dword_ok(a->data, p.a_row)) ? 1 : 0;
-    p.b_vec = (p.b_k == 1 && dword_ok(b->data, p.b_col)) ? 1 : 0;
     if (bias != nullptr) {
         p.bias = bias->data;
         p.bias_stride = bias->strides[0] / it;
     }
-    p.tiles_n = static_cast<int>((N + 31) / 32);
-    int64_t blocks = ((M + 31) / 32) * p.tiles_n;
     ProfileScope prof(stream, 2.0 * M * N * K, static_cast<double>(it) * (M * K + K * N + M * N));
+    if (M <= 4 && a_mode == kPieces && b_mode == kPieces) {
+        const dim3 grid(static_cast<unsigned>((N + 3) / 4));
+        if (M == 1) hipLaunchKernelGGL((SmallDotVectorKernel<T, 1>), grid, dim3(256), 0, stream, p);
+        else if (M == 2) hipLaunchKernelGGL((SmallDotVectorKernel<T, 2>), grid, dim3(256), 0, stream, p);
+        else hipLaunchKernelGGL((SmallDotVectorKernel<T, 4>), grid, dim3(256), 0, stream, p);
+        CheckLaunch("small_dot_vector");
+        return true;
+    }
     static const bool rows_ok = [] { const char* e = getenv("HIPCX_SMALL_DOT_ROWS"); return e == nullptr || e[0] != '0'; }();
     // whole-line loads regrouped through LDS pay off once the product is large enough to be bandwidth-bound (measured: the
     // 10000-column projection of the language model gains 15 %, the 2600- and 1000-column layers lose 10 %)
-    if (rows_ok && p.a_vec && p.b_vec && 2.0 * M * N * K >= 1e9) {
+    if (rows_ok && a_mode == kPieces && b_mode == kPieces && 2.0 * M * N * K >= 1e9) {
         // Waves per workgroup = ways K is split: the choice that leaves the busiest SIMD the least matrix work
         // (wave-tiles are dealt over 4 SIMDs per CU; a wave's share is whole 128-byte steps).
-        const int64_t steps = (K * it + 127) / 128;
+        const int64_t blocks = static_cast<int64_t>(p.tiles_m) * p.tiles_n, steps = (K * it + 127) / 128;
         const int64_t simds = static_cast<int64_t>(NumCUs()) * 4;
         int best_nw = 1;
         int64_t best_cost = -1;
@@ -301,8 +401,13 @@ bool TrySmallDot(const hipcx_array* a, const hipcx_array* b, const hipcx_array* 
         CheckLaunch("small_dot_rows");
         return true;
     }
-    hipLaunchKernelGGL((SmallDotKernel<T>), dim3(static_cast<unsigned>(blocks)), dim3(512), 0, stream, p);
-    CheckLaunch("small_dot");
+    p.ksplit = partial != nullptr ? SmallDotSplit(M, N, K, DtypeOf<T>::value) : 1;
+    p.partial = p.ksplit > 1 ? partial : nullptr;
+    LaunchSmallDot<T>(p, a_mode, b_mode, 1, stream);
+    if (p.ksplit > 1) {
+        hipLaunchKernelGGL((SmallDotSumKernel<T>), dim3(static_cast<unsigned>((M * N + 255) / 256)), dim3(256), 0, stream, p);
+        CheckLaunch("small_dot_sum");
+    }
     return true;
 }
 
@@ -1348,7 +1453,7 @@ DotStaging PlanDotStaging(const hipcx_array* a, const hipcx_array* b, const hipc
     if (a_fast && b_fast) return st;
     // worth it only when the product is large against the copies; small outputs have their own kernel (any layout)
     if (2.0 * m * n * k < 2e8) return st;
-    if (((m + 127) / 128) * ((n + 127) / 128) < 128 && k >= 64) return st;
+    if (SmallDotShape(m, n, k)) return st;
     const int64_t epv = 16 / it;
     st.kpad = (k + epv - 1) / epv * epv;
     // a changed pitch on one side needs the same (zero-padded) k extent on the other
@@ -1564,16 +1669,24 @@ static int DotBias(const hipcx_array* a, const hipcx_array* b, const hipcx_array
                 }
             }
         }
+        // the same piece of the workspace serves a small product's partial sums
+        float* small_partial = nullptr;
+        if (slices == 1 && staged_bytes == 0 && out->dtype != HIPCX_FLOAT64 && SmallDotShape(m, n, k)) {
+            const size_t need = SmallDotPartialBytes(m, n, k, out->dtype);
+            if (need > 0 && workspace != nullptr && workspace_bytes >= need && reinterpret_cast<uintptr_t>(workspace) % 16 == 0) {
+                small_partial = static_cast<float*>(workspace);
+            }
+        }
         if (out->dtype == HIPCX_FLOAT16) {
             if (slices == 1 && TryGemmPp(a, b, bias, out, st)) return;
-            if (slices == 1 && TrySmallDot<half_t>(a, b, bias, out, st)) return;
+            if (slices == 1 && TrySmallDot<half_t>(a, b, bias, out, small_partial, st)) return;
             IGemmArgs<half_t> p{};
             fill(p);
             p.ksplit = slices;
             p.partial = partial;
             LaunchIGemmImpl(p, st);
         } else if (out->dtype == HIPCX_FLOAT32) {
-            if (slices == 1 && TrySmallDot<float>(a, b, bias, out, st)) return;
+            if (slices == 1 && TrySmallDot<float>(a, b, bias, out, small_partial, st)) return;
             IGemmArgs<float> p{};
             fill(p);
             p.ksplit = slices;
@@ -1594,8 +1707,10 @@ size_t hipcx_dot_workspace_size(const hipcx_array* a, const hipcx_array* b, cons
         if (out != nullptr && !IsFloatDtype(out->dtype)) return 0;
         DotStaging st = PlanDotStaging(a, b, out);
         size_t split = 0;
-        if (a != nullptr && b != nullptr && out != nullptr && a->ndim == 2 && b->ndim == 2) {
-            split = SplitKBytes(a->shape[0], b->shape[1], PlanSplitK(a->shape[0], b->shape[1], a->shape[1], out->dtype));
+        if (a != nullptr && b != nullptr && out != nullptr && a->ndim == 2 && b->ndim == 2 && a->shape[1] > 0 && a->shape[0] > 0 && b->shape[1] > 0) {
+            const int64_t m = a->shape[0], n = b->shape[1], k = a->shape[1];
+            split = SplitKBytes(m, n, PlanSplitK(m, n, k, out->dtype));
+            if (split == 0 && out->dtype != HIPCX_FLOAT64 && SmallDotShape(m, n, k)) split = SmallDotPartialBytes(m, n, k, out->dtype);
         }
         return RoundUpTo(st.a_bytes + st.b_bytes, 256) + split;
     } catch (...) {

@@ -1,17 +1,26 @@
-// Matrix product for small outputs (batch-sized Linear layers: 100-128 rows, K up to a few thousand):
-// out[M,N] = a[M,K] . b[K,N] with M*N so small that 128x128 tiles would occupy a handful of CUs.
+// Matrix products with small outputs (batch-sized Linear layers, recurrent steps, weight gradients of small layers):
+// out[M,N] = a[M,K] . b[K,N] with so few elements that 128x128 tiles would occupy a handful of compute units.
 //
-// A workgroup owns one 32x32 tile of `out`; its 8 waves split the reduction axis, each feeding the MFMA straight
-// from global memory (operands this small live in L2; no LDS staging), and the 8 partial tiles are summed through
-// LDS.  For float the reduction index is dealt to the v_mfma_f32_32x32x2_f32 steps so that a lane's four steps use
-// four consecutive k (one 16-byte load when k is the contiguous axis of the operand, which is the case for
-// Linear's x and W^T view); for float16 a lane's v_mfma_f32_32x32x16_f16 operand is 8 consecutive k.
+// A workgroup owns one 32x32 tile of `out`; its waves split the reduction axis -- and, with ksplit > 1, so do several workgroups, whose
+// sums another kernel adds up -- each feeding the MFMA from global memory on its own (operands this small live in the caches), and
+// the partial tiles are summed through LDS.  Four kernels, by where the operands lie (chosen in TrySmallDot):
+//   SmallDotKernel        k is the unit-stride axis of both operands (Linear's x and W^T): straight from global memory, bound by the
+//                         latency of a few loads.
+//   SmallDotRowsKernel    the same for products of 1 GFLOP and more, whole 128-byte lines regrouped through LDS.
+//   SmallDotMixedKernel   an operand whose k axis is not the unit-stride one (dG . Wh of a recurrent network, x^T . gy), or float16 rows
+//                         of odd pitch.
+//   SmallDotVectorKernel  M <= 4 (one image, one sentence): a wave per output column, K across the lanes, where the MFMA would work on
+//                         32 rows.
+// For float the reduction index is dealt to the v_mfma_f32_32x32x2_f32 steps so that a lane's four steps use four consecutive k (one
+// 16-byte load when k is the contiguous axis of the operand); for float16 a lane's v_mfma_f32_32x32x16_f16 operand is 8 consecutive k.
 // Rows / columns beyond M / N and the tail of K are served as zeros by the buffer bounds check or explicit masks.
 #pragma once
 
 #include "nchw_conv.h"
 
 namespace hipcx {
+
+constexpr int kSmallDotMaxBatch = 4;
 
 struct SmallDotArgs {
     const void* a;
@@ -22,19 +31,22 @@ struct SmallDotArgs {
     int64_t b_k, b_col;  // element strides of b along k and n
     int64_t o_row, o_col;
     unsigned a_bytes, b_bytes;  // spans, for the buffer descriptors
-    int a_vec, b_vec;           // k is the unit-stride axis of the operand and 16-byte runs are dword aligned
-    int tiles_n;
+    int tiles_m, tiles_n;
     const void* bias;     // one element per column of out, added to the rounded product (Dot, then Add); may be null
     int64_t bias_stride;  // elements
-    int nw;  // SmallDotRowsKernel: waves per workgroup = ways the reduction axis is split
+    int nw;               // waves per workgroup = ways a workgroup's share of the reduction is split (SmallDotKernel: 8)
+    int ksplit;           // workgroups per tile along the reduction (not SmallDotRowsKernel)
+    float* partial;       // not null: [ksplit][M][N] sums go there instead of to out
+    // blockIdx.y: products that share their shapes and strides, a and b at constant distances (elements), outputs anywhere
+    // (not SmallDotRowsKernel)
+    int64_t a_batch, b_batch;
+    void* outs[kSmallDotMaxBatch];
 };
 
 // Workgroups are dealt to the 8 XCDs round-robin, and each XCD has its own L2: give every XCD one contiguous range of
 // tiles, row tiles fastest, so that the workgroups sharing a slice of b (the weights) share an L2 and the whole of b is
 // fetched into the L2s once instead of once per XCD.
-__device__ __forceinline__ void SmallDotTile(int tiles_m, int& tm, int& tn) {
-    const int nblk = gridDim.x;
-    const int bid = blockIdx.x;
+__device__ __forceinline__ void SmallDotTile(int nblk, int bid, int tiles_m, int& tm, int& tn) {
     const int xcd = bid & 7, loc = bid >> 3;
     const int q = nblk >> 3, r = nblk & 7;
     const int tile = xcd * q + min(xcd, r) + loc;
@@ -48,6 +60,16 @@ __device__ __forceinline__ void StoreDot(const SmallDotArgs& p, T* out, int m, i
     T v = static_cast<T>(s);
     if (p.bias != nullptr) v = static_cast<T>(static_cast<float>(v) + static_cast<float>(static_cast<const T*>(p.bias)[n * p.bias_stride]));
     out[m * p.o_row + n * p.o_col] = v;
+}
+
+// Where an element of a tile goes.
+template <typename T>
+__device__ __forceinline__ void StoreTileElement(const SmallDotArgs& p, int split, T* out, int m, int n, float s) {
+    if (p.partial != nullptr) {
+        p.partial[(static_cast<int64_t>(split) * p.M + m) * p.N + n] = s;
+    } else {
+        StoreDot<T>(p, out, m, n, s);
+    }
 }
 
 template <typename T>
@@ -64,36 +86,6 @@ struct SmallDotTraits<half_t> {
     static constexpr int PER_LANE = 8;
     static constexpr int STEPS_IN_FLIGHT = 2;  // per register stage (two stages)
 };
-
-// PER_LANE consecutive-k elements of one operand row/column as raw dwords; `contig`: k is the unit-stride axis.
-template <typename T>
-__device__ __forceinline__ Bytes16 LoadRun(__amdgpu_buffer_rsrc_t r, const T* base, int64_t line_off, int64_t kstride, int k, int kend, bool line_ok,
-                                           bool contig) {
-    constexpr int PL = SmallDotTraits<T>::PER_LANE;
-    Bytes16 v = Bytes16(0);
-    if (!line_ok) return v;
-    if (contig && k + PL <= kend) {
-        return __builtin_amdgcn_raw_buffer_load_b128(r, static_cast<int>((line_off + k) * static_cast<int64_t>(sizeof(T))), 0, 0);
-    }
-    T e[PL];
-#pragma unroll
-    for (int i = 0; i < PL; ++i) e[i] = (k + i < kend) ? base[line_off + (k + i) * kstride] : T(0);
-    if constexpr (sizeof(T) == 4) {
-        v.x = __builtin_bit_cast(unsigned, e[0]);
-        v.y = __builtin_bit_cast(unsigned, e[1]);
-        v.z = __builtin_bit_cast(unsigned, e[2]);
-        v.w = __builtin_bit_cast(unsigned, e[3]);
-    } else {
-        auto pk = [](T lo, T hi) {
-            return static_cast<unsigned>(__builtin_bit_cast(unsigned short, lo)) | (static_cast<unsigned>(__builtin_bit_cast(unsigned short, hi)) << 16);
-        };
-        v.x = pk(e[0], e[1]);
-        v.y = pk(e[2], e[3]);
-        v.z = pk(e[4], e[5]);
-        v.w = pk(e[6], e[7]);
-    }
-    return v;
-}
 
 // The same run when k is the unit-stride axis, without a branch: lines beyond the operand come back as zeros from the
 // buffer bounds check, elements beyond kend (they belong to the next line) are masked.  Loads written this way can all be
@@ -131,29 +123,31 @@ __global__ __launch_bounds__(512) void SmallDotKernel(SmallDotArgs p) {
     const int lr = lane & 31;
     const int g = lane >> 5;
     int tm, tn;
-    SmallDotTile((p.M + 31) / 32, tm, tn);
+    const int tiles = p.tiles_m * p.tiles_n;
+    const int split = blockIdx.x / tiles;
+    SmallDotTile(tiles, blockIdx.x - split * tiles, p.tiles_m, tm, tn);
     const int m = tm * 32 + lr;
     const int n = tn * 32 + lr;
-    const T* a = static_cast<const T*>(p.a);
-    const T* b = static_cast<const T*>(p.b);
-    const __amdgpu_buffer_rsrc_t ar = MakeRsrc(p.a, p.a_bytes);
-    const __amdgpu_buffer_rsrc_t br = MakeRsrc(p.b, p.b_bytes);
-    const bool a_contig = p.a_vec != 0, b_contig = p.b_vec != 0;
+    const int batch = blockIdx.y;
+    const __amdgpu_buffer_rsrc_t ar = MakeRsrc(static_cast<const T*>(p.a) + batch * p.a_batch, p.a_bytes);
+    const __amdgpu_buffer_rsrc_t br = MakeRsrc(static_cast<const T*>(p.b) + batch * p.b_batch, p.b_bytes);
     const bool m_ok = m < p.M, n_ok = n < p.N;
     const int64_t a_off = static_cast<int64_t>(m) * p.a_row;
     const int64_t b_off = static_cast<int64_t>(n) * p.b_col;
 
     // this wave's share of K, in whole group steps
     const int groups = (p.K + KG - 1) / KG;
-    const int per_wave = (groups + NW - 1) / NW;
-    const int k_begin = wave * per_wave * KG;
-    const int k_end = min(p.K, k_begin + per_wave * KG);
+    const int per_split = (groups + p.ksplit - 1) / p.ksplit;
+    const int split_end = min(groups, (split + 1) * per_split);
+    const int per_wave = (per_split + NW - 1) / NW;
+    const int k_begin = (split * per_split + wave * per_wave) * KG;
+    const int k_end = min(p.K, min(split_end, split * per_split + (wave + 1) * per_wave) * KG);
 
     float16_t acc;
 #pragma unroll
     for (int v = 0; v < 16; ++v) acc[v] = 0.f;
     constexpr int U = SmallDotTraits<T>::STEPS_IN_FLIGHT;
-    if (a_contig && b_contig) {  // Linear's x and W^T: every operand load is one branch-free 16-byte buffer load
+    {
         // Two register stages of U group steps: the loads of the next stage are issued before the MFMAs of the current one,
         // so that a wave's matrix work overlaps its own loads (all waves of a workgroup run in lockstep otherwise).
         // Stages made of whole runs inside K need no masking, so nothing but the MFMAs depends on a load and the waits
@@ -203,31 +197,19 @@ __global__ __launch_bounds__(512) void SmallDotKernel(SmallDotArgs p) {
             Bytes16 tb = LoadRunContig<T>(br, b_off, kk, k_end, n_ok);
             MfmaTile<T>(ta, tb, acc);
         }
-    } else {
-        for (int k = k_begin; k < k_end; k += 2 * KG) {
-            Bytes16 av[2], bv[2];
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                int kk = k + u * KG + g * PL;
-                av[u] = LoadRun<T>(ar, a, a_off, p.a_k, kk, k_end, m_ok, a_contig);
-                bv[u] = LoadRun<T>(br, b, b_off, p.b_k, kk, k_end, n_ok, b_contig);
-            }
-#pragma unroll
-            for (int u = 0; u < 2; ++u) MfmaTile<T>(av[u], bv[u], acc);
-        }
     }
     // lane holds column lr, rows 8*(v/4) + 4*g + v%4
 #pragma unroll
     for (int v = 0; v < 16; ++v) part[wave][(8 * (v / 4) + 4 * g + (v % 4)) * 33 + lr] = acc[v];
     __syncthreads();
-    T* out = static_cast<T*>(p.out);
+    T* out = static_cast<T*>(gridDim.y > 1 ? p.outs[batch] : p.out);
     for (int e = tid; e < 32 * 32; e += 512) {
         int row = e >> 5, col = e & 31;
         float s = 0.f;
 #pragma unroll
         for (int w = 0; w < NW; ++w) s += part[w][row * 33 + col];
         int om = tm * 32 + row, on = tn * 32 + col;
-        if (om < p.M && on < p.N) StoreDot<T>(p, out, om, on, s);
+        if (om < p.M && on < p.N) StoreTileElement<T>(p, split, out, om, on, s);
     }
 }
 
@@ -251,7 +233,7 @@ __global__ __launch_bounds__(512) void SmallDotRowsKernel(SmallDotArgs p) {
     const int piece = lane & 7;
     const int sub = lane >> 3;  // row within a group of 8
     int tm, tn;
-    SmallDotTile((p.M + 31) / 32, tm, tn);
+    SmallDotTile(gridDim.x, blockIdx.x, p.tiles_m, tm, tn);
     const __amdgpu_buffer_rsrc_t ar = MakeRsrc(p.a, p.a_bytes);
     const __amdgpu_buffer_rsrc_t br = MakeRsrc(p.b, p.b_bytes);
     char* wa = lds + wave * REGION;
@@ -334,6 +316,270 @@ __global__ __launch_bounds__(512) void SmallDotRowsKernel(SmallDotArgs p) {
         for (int w = 0; w < p.nw; ++w) s += part[w * (32 * 33) + row * 33 + col];
         const int om = tm * 32 + row, on = tn * 32 + col;
         if (om < p.M && on < p.N) StoreDot<T>(p, out, om, on, s);
+    }
+}
+
+// How SmallDotMixedKernel reads an operand.  kPieces: rows of contiguous k as 16-byte pieces; kElements: another axis is the unit-stride
+// one, element by element with that axis across the lanes -- whole lines too, already in the MFMA layout; kOddPieces: float16 rows of odd
+// pitch, whose last elements share a dword with what lies behind the array: pieces, but the chunk that holds the end of K by elements.
+enum SmallDotMode { kPieces, kElements, kOddPieces };
+
+constexpr int kSmallDotMaxWaves = 8;
+constexpr int kSmallDotPart = 32 * 33;  // floats of a wave's partial tile
+
+constexpr int kSmallDotPitch = 144;  // bytes of a row staged in LDS: the 16-byte reads of 8 consecutive rows start in different banks
+constexpr int kSmallDotStage = 32 * kSmallDotPitch;
+
+// One lane's share of a chunk of an operand: P pieces of 16 bytes.
+template <int P>
+struct SmallDotShare {
+    Bytes16 v[P];
+};
+
+// PL consecutive elements of k at byte `line` (negative: a row beyond the operand).  WHOLE: as one load, which may reach beyond K.
+template <typename T, bool WHOLE>
+__device__ __forceinline__ Bytes16 LoadPiece(__amdgpu_buffer_rsrc_t r, int line, int k_stride_bytes, int k, int K) {
+    constexpr int PL = 16 / sizeof(T);
+    constexpr int kOut = 0x7fffffff;
+    if constexpr (WHOLE) {
+        return __builtin_amdgcn_raw_buffer_load_b128(r, line >= 0 && k < K ? line + k * static_cast<int>(sizeof(T)) : kOut, 0, 0);
+    } else {
+        Bytes16 v;
+        if constexpr (sizeof(T) == 4) {
+#pragma unroll
+            for (int e = 0; e < PL; ++e) v[e] = __builtin_amdgcn_raw_buffer_load_b32(r, line >= 0 && k + e < K ? line + (k + e) * k_stride_bytes : kOut, 0, 0);
+        } else {
+            unsigned short s[PL];
+#pragma unroll
+            for (int e = 0; e < PL; ++e) s[e] = __builtin_amdgcn_raw_buffer_load_b16(r, line >= 0 && k + e < K ? line + (k + e) * k_stride_bytes : kOut, 0, 0);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = s[2 * e] | (static_cast<unsigned>(s[2 * e + 1]) << 16);
+        }
+        return v;
+    }
+}
+
+// The first K - k elements of a piece, zeros in place of what follows K in the memory of a row.
+template <typename T>
+__device__ __forceinline__ Bytes16 MaskPiece(Bytes16 v, int k, int K) {
+    constexpr int PD = 4 / sizeof(T);  // elements per dword
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+        const int left = K - (k + d * PD);
+        v[d] = left >= PD ? v[d] : (left == 1 && PD == 2 ? v[d] & 0xffffu : 0u);
+    }
+    return v;
+}
+
+// The reduction is dealt out in chunks of 128 bytes per row.  Pieces are loaded as whole lines (8 lanes to a row, 8 rows to an instruction)
+// and turned round through a piece of LDS that belongs to the wave (no barrier); elements come as they are used.  Two chunks are in flight
+// while a third is multiplied.  [20,2600] . [2600,650] float32, row-major b: 34 -> 9.3 us (several workgroups per tile and the pass over
+// their sums included), [64,333] . [333,777] float16 8.5 -> 6.4.
+template <typename T, int AM, int BM, int P>
+__global__ __launch_bounds__(64 * kSmallDotMaxWaves) __attribute__((amdgpu_waves_per_eu(3, 8))) void SmallDotMixedKernel(SmallDotArgs p) {
+    constexpr int PL = 16 / sizeof(T);
+    constexpr int KC = 2 * P * PL;      // k per chunk
+    constexpr int D = P == 1 ? 6 : 2;   // chunks in flight
+    constexpr bool A_LDS = P == 4 && AM != kElements, B_LDS = P == 4 && BM != kElements;
+    extern __shared__ __align__(16) char lds[];
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: the loop below runs on scalar control flow
+    const int lr = lane & 31;
+    const int g = lane >> 5;
+    const int piece = lane & 7, sub = lane >> 3;
+    const int tiles = p.tiles_m * p.tiles_n;
+    const int split = blockIdx.x / tiles;
+    int tm, tn;
+    SmallDotTile(tiles, blockIdx.x - split * tiles, p.tiles_m, tm, tn);
+    const int batch = blockIdx.y;
+    const __amdgpu_buffer_rsrc_t ar = MakeRsrc(static_cast<const T*>(p.a) + batch * p.a_batch, p.a_bytes);
+    const __amdgpu_buffer_rsrc_t br = MakeRsrc(static_cast<const T*>(p.b) + batch * p.b_batch, p.b_bytes);
+    const int a_ks = static_cast<int>(p.a_k * sizeof(T)), b_ks = static_cast<int>(p.b_k * sizeof(T));
+    // rows this lane reads: in the MFMA layout its own (lr), as whole lines every eighth one
+    auto line_of = [](int row, int rows, int64_t stride) { return row < rows ? static_cast<int>(row * stride * static_cast<int64_t>(sizeof(T))) : -1; };
+    int a_line[4], b_line[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        a_line[j] = line_of(tm * 32 + (A_LDS ? j * 8 + sub : lr), p.M, p.a_row);
+        b_line[j] = line_of(tn * 32 + (B_LDS ? j * 8 + sub : lr), p.N, p.b_col);
+    }
+    char* const stage = lds + wave * ((A_LDS ? kSmallDotStage : 0) + (B_LDS ? kSmallDotStage : 0));
+
+    // this wave's chunks
+    const int chunks = (p.K + KC - 1) / KC;
+    const int per_split = (chunks + p.ksplit - 1) / p.ksplit;
+    const int s_begin = split * per_split, s_end = min(chunks, s_begin + per_split);
+    const int per_wave = (max(s_end - s_begin, 0) + p.nw - 1) / p.nw;
+    const int begin = s_begin + wave * per_wave, end = min(s_end, begin + per_wave);
+
+    float16_t acc;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[v] = 0.f;
+    SmallDotShare<P> av[D], bv[D];
+    auto load_operand = [&](auto mode_tag, SmallDotShare<P>& x, __amdgpu_buffer_rsrc_t r, const int (&line)[4], int ks, int c) {
+        constexpr int MODE = decltype(mode_tag)::value;
+        constexpr bool LDS = P == 4 && MODE != kElements;
+        const int k0 = c * KC + (LDS ? piece * PL : g * P * PL);
+        if (MODE == kPieces || (MODE == kOddPieces && (c + 1) * KC <= p.K)) {
+#pragma unroll
+            for (int j = 0; j < P; ++j) x.v[j] = LoadPiece<T, true>(r, line[LDS ? j : 0], ks, k0 + (LDS ? 0 : j * PL), p.K);
+        } else {
+#pragma unroll
+            for (int j = 0; j < P; ++j) x.v[j] = LoadPiece<T, false>(r, line[LDS ? j : 0], ks, k0 + (LDS ? 0 : j * PL), p.K);
+        }
+    };
+    auto load = [&](int i, int c) {
+        load_operand(std::integral_constant<int, AM>{}, av[i], ar, a_line, a_ks, c);
+        load_operand(std::integral_constant<int, BM>{}, bv[i], br, b_line, b_ks, c);
+    };
+    // the chunk in the MFMA layout: lane (lr, g) holds pieces g * P .. of its row
+    auto arrange = [&](auto mode_tag, SmallDotShare<P>& x, char* area, int c) {
+        constexpr int MODE = decltype(mode_tag)::value;
+        constexpr bool LDS = P == 4 && MODE != kElements;
+        if (MODE == kPieces && (c + 1) * KC > p.K) {
+            const int k0 = c * KC + (LDS ? piece * PL : g * P * PL);
+#pragma unroll
+            for (int j = 0; j < P; ++j) x.v[j] = MaskPiece<T>(x.v[j], k0 + (LDS ? 0 : j * PL), p.K);
+        }
+        if constexpr (LDS) {
+#pragma unroll
+            for (int j = 0; j < P; ++j) *reinterpret_cast<Bytes16*>(area + (j * 8 + sub) * kSmallDotPitch + piece * 16) = x.v[j];
+        }
+    };
+    auto fragment = [&](bool in_lds, const SmallDotShare<P>& x, const char* area, int j) {
+        return in_lds ? *reinterpret_cast<const Bytes16*>(area + lr * kSmallDotPitch + (g * P + j) * 16) : x.v[j];
+    };
+    auto multiply = [&](int i, int c, auto&& next) {
+        char* const b_area = stage + (A_LDS ? kSmallDotStage : 0);
+        arrange(std::integral_constant<int, AM>{}, av[i], stage, c);
+        arrange(std::integral_constant<int, BM>{}, bv[i], b_area, c);
+        if constexpr (A_LDS || B_LDS) __builtin_amdgcn_wave_barrier();
+        Bytes16 fa[P], fb[P];
+#pragma unroll
+        for (int j = 0; j < P; ++j) {
+            fa[j] = fragment(A_LDS, av[i], stage, j);
+            fb[j] = fragment(B_LDS, bv[i], b_area, j);
+        }
+        if constexpr (A_LDS && B_LDS) next();  // (else the registers of a chunk are its fragments)
+        if constexpr (A_LDS || B_LDS) __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int j = 0; j < P; ++j) MfmaTile<T>(fa[j], fb[j], acc);
+        if constexpr (!(A_LDS && B_LDS)) next();
+    };
+    if (begin < end) {
+#pragma unroll
+        for (int i = 0; i < D; ++i) {
+            if (begin + i < end) load(i, begin + i);
+        }
+        int c = begin;
+        // no conditional loads while a whole round of them is left: the waits then cover one chunk, not what was issued behind it
+        for (; c + 2 * D <= end; c += D) {
+#pragma unroll
+            for (int i = 0; i < D; ++i) multiply(i, c + i, [&] { load(i, c + i + D); });
+        }
+        if (c + D < end) {
+#pragma unroll
+            for (int i = 0; i < D; ++i) {
+                multiply(i, c + i, [&] {
+                    if (c + i + D < end) load(i, c + i + D);
+                });
+            }
+            c += D;
+        }
+#pragma unroll
+        for (int i = 0; i < D; ++i) {
+            if (c + i < end) multiply(i, c + i, [] {});
+        }
+    }
+    if constexpr (A_LDS || B_LDS) __syncthreads();  // the staging areas become the partial tiles
+    // lane holds column lr, rows 8*(v/4) + 4*g + v%4
+    float* const part = reinterpret_cast<float*>(lds);
+    float* const mine = part + wave * kSmallDotPart;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) mine[(8 * (v / 4) + 4 * g + (v % 4)) * 33 + lr] = acc[v];
+    __syncthreads();
+    T* out = static_cast<T*>(gridDim.y > 1 ? p.outs[batch] : p.out);
+    for (int e = tid; e < 32 * 32; e += 64 * p.nw) {
+        const int row = e >> 5, col = e & 31;
+        const int om = tm * 32 + row, on = tn * 32 + col;
+        if (om >= p.M || on >= p.N) continue;
+        float s = 0.f;
+        for (int w = 0; w < p.nw; ++w) s += part[w * kSmallDotPart + row * 33 + col];
+        StoreTileElement<T>(p, split, out, om, on, s);
+    }
+}
+
+// Sums the partial products of ksplit > 1.
+template <typename T>
+__global__ __launch_bounds__(256) void SmallDotSumKernel(SmallDotArgs p) {
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+    const int64_t total = static_cast<int64_t>(p.M) * p.N;
+    if (i >= total) return;
+    float s = 0.f;
+#pragma unroll 4
+    for (int k = 0; k < p.ksplit; ++k) s += p.partial[k * total + i];
+    const int m = static_cast<int>(i / p.N);
+    StoreDot<T>(p, static_cast<T*>(p.out), m, static_cast<int>(i - static_cast<int64_t>(m) * p.N), s);
+}
+
+// M <= 4 rows against rows of K contiguous elements (b_k == 1, a_k == 1): a wave per output column, 64 x 16 bytes of K per step, the
+// rows of `a` out of L1.  Bound by one pass over b: [1,784] . [784,1000] float32 7.7 -> 3 us.
+template <typename T, int MR>
+__global__ __launch_bounds__(256) void SmallDotVectorKernel(SmallDotArgs p) {
+    constexpr int PL = 16 / sizeof(T);
+    constexpr int U = 4;  // steps in flight
+    const int lane = threadIdx.x & 63;
+    const int n = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (n >= p.N) return;
+    const __amdgpu_buffer_rsrc_t ar = MakeRsrc(p.a, p.a_bytes);
+    const __amdgpu_buffer_rsrc_t br = MakeRsrc(p.b, p.b_bytes);
+    const int b_line = static_cast<int>(n * p.b_col * static_cast<int64_t>(sizeof(T)));
+    float acc[MR];
+#pragma unroll
+    for (int r = 0; r < MR; ++r) acc[r] = 0.f;
+    for (int k0 = lane * PL; k0 - lane * PL < p.K; k0 += U * 64 * PL) {  // (uniform trip count)
+        Bytes16 bv[U], av[U][MR];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int k = k0 + u * 64 * PL;
+            const bool in = k < p.K;
+            bv[u] = __builtin_amdgcn_raw_buffer_load_b128(br, in ? b_line + k * static_cast<int>(sizeof(T)) : 0x7fffffff, 0, 0);
+#pragma unroll
+            for (int r = 0; r < MR; ++r) {
+                const int line = static_cast<int>(r * p.a_row * static_cast<int64_t>(sizeof(T)));
+                av[u][r] = __builtin_amdgcn_raw_buffer_load_b128(ar, in && r < p.M ? line + k * static_cast<int>(sizeof(T)) : 0x7fffffff, 0, 0);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int k = k0 + u * 64 * PL;
+            struct Piece {
+                T e[PL];
+            };
+            const Piece bp = __builtin_bit_cast(Piece, bv[u]);
+#pragma unroll
+            for (int r = 0; r < MR; ++r) {
+                const Piece ap = __builtin_bit_cast(Piece, av[u][r]);
+#pragma unroll
+                for (int e = 0; e < PL; ++e) {
+                    const float product = static_cast<float>(ap.e[e]) * static_cast<float>(bp.e[e]);
+                    acc[r] += k + e < p.K ? product : 0.f;  // (what follows K may be anything)
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) {
+#pragma unroll
+        for (int r = 0; r < MR; ++r) acc[r] += __shfl_xor(acc[r], d, 64);
+    }
+    if (lane == 0) {
+#pragma unroll
+        for (int r = 0; r < MR; ++r) {
+            if (r < p.M) StoreDot<T>(p, static_cast<T*>(p.out), r, n, acc[r]);
+        }
     }
 }
 
