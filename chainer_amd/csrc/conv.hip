@@ -15,6 +15,7 @@
 #include "nchw_conv.h"
 #include "pw_conv.h"
 #include "stem_conv.h"
+#include "dot_parts.h"
 #include "small_dot.h"
 
 namespace hipcx {
@@ -1185,6 +1186,42 @@ void CheckConv(const hipcx_array* x, const hipcx_array* w, const hipcx_array* b,
 }
 
 }  // namespace
+
+int DotPartSplits(int64_t m, int64_t n, int64_t k) {
+    // M <= 4 rows have a kernel of their own, GFLOPs the one for whole lines
+    return SmallDotShape(m, n, k) && m > 4 && 2.0 * m * n * k < 1e9 ? PlanSmallDotSplit(m, n, k, HIPCX_FLOAT32) : 1;
+}
+
+void DotParts(const hipcx_array* a, const hipcx_array* b, float* parts, int splits, hipStream_t stream) {
+    SmallDotArgs p{};
+    int a_mode = 0, b_mode = 0;
+    HIPCX_REQUIRE(SmallDotOperands<float>(a, b, &p, &a_mode, &b_mode), HIPCX_NOT_IMPLEMENTED_ERROR, "DotParts: operands out of range");
+    p.ksplit = splits;
+    p.partial = parts;
+    ProfileScope prof(stream, 2.0 * p.M * p.N * p.K, 4.0 * (static_cast<double>(p.M) * p.K + static_cast<double>(p.K) * p.N + static_cast<double>(p.M) * p.N * splits));
+    LaunchSmallDot<float>(p, a_mode, b_mode, 1, stream);
+}
+
+bool DotSeveral(const hipcx_array* a0, int64_t a_distance, const hipcx_array* b, const hipcx_array* const* outs, int n, hipStream_t stream) {
+    const int64_t M = a0->shape[0], K = a0->shape[1], N = b->shape[1];
+    SmallDotArgs p{};
+    int a_mode = 0, b_mode = 0;
+    if (n > kSmallDotMaxBatch || !SmallDotShape(M, N, K) || SmallDotSplit(M, N, K, HIPCX_FLOAT32) > 1) return false;
+    if (!SmallDotOperands<float>(a0, b, &p, &a_mode, &b_mode)) return false;
+    for (int i = 0; i < n; ++i) {
+        if (outs[i]->strides[0] != outs[0]->strides[0] || outs[i]->strides[1] != outs[0]->strides[1]) return false;
+        p.outs[i] = outs[i]->data;
+    }
+    if (outs[0]->strides[0] < 0 || outs[0]->strides[1] < 0 || outs[0]->strides[0] % 4 || outs[0]->strides[1] % 4) return false;
+    p.out = outs[0]->data;
+    p.o_row = outs[0]->strides[0] / 4;
+    p.o_col = outs[0]->strides[1] / 4;
+    p.a_batch = a_distance;
+    p.ksplit = 1;
+    ProfileScope prof(stream, 2.0 * M * N * K * n, 4.0 * n * (M * K + K * N + M * N));
+    LaunchSmallDot<float>(p, a_mode, b_mode, n, stream);
+    return true;
+}
 }  // namespace hipcx
 
 namespace hipcx {

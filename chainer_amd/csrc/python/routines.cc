@@ -362,13 +362,18 @@ HOST_FN(Split) {
     HOST_CATCH(nullptr);
 }
 
-// One CopyKernel per input into a view of the result.
-void CopyInto(Array* a, const hipcx_array& view) {
+// Every input into its view of the result.
+void CopyInto(const std::vector<Ref>& arrays, const std::vector<hipcx_array>& views) {
     void* stream = Stream();
-    Call([&] { return hipcx_copy(&a->d, &view, stream); });
+    std::vector<const hipcx_array*> from, to;
+    for (size_t i = 0; i < views.size(); ++i) {
+        from.push_back(&arrays[i].arr()->d);
+        to.push_back(&views[i]);
+    }
+    Call([&] { return hipcx_copy_many(from.data(), to.data(), static_cast<int>(from.size()), stream); });
 }
 
-// Concatenate = Empty + one CopyKernel per input (CX/routines/manipulation.cc:415-460).
+// Concatenate = Empty + a copy of every input (CopyKernel, CX/routines/manipulation.cc:415-460).
 HOST_FN(Concatenate) {
     HOST_TRY;
     HOST_ARGS("concatenate", 1, "arrays", "axis");
@@ -394,16 +399,18 @@ HOST_FN(Concatenate) {
     }
     Ref out = Empty(n, shape, code);
     hipcx_array view = out.arr()->d;
+    std::vector<hipcx_array> views;
     for (const Ref& r : arrays) {
         view.shape[axis] = r.arr()->d.shape[axis];
-        CopyInto(r.arr(), view);
+        views.push_back(view);
         view.data = static_cast<char*>(view.data) + view.shape[axis] * view.strides[axis];
     }
+    CopyInto(arrays, views);
     return out.release();
     HOST_CATCH(nullptr);
 }
 
-// Stack = Empty + one CopyKernel per input into a view of the new axis (CX/routines/manipulation.cc Stack).
+// Stack = Empty + a copy of every input into a view of the new axis (CX/routines/manipulation.cc Stack).
 HOST_FN(Stack) {
     HOST_TRY;
     HOST_ARGS("stack", 1, "arrays", "axis");
@@ -425,10 +432,12 @@ HOST_FN(Stack) {
     view.ndim = n;
     const int64_t step = view.strides[axis];
     for (int i = axis; i < n; ++i) view.shape[i] = view.shape[i + 1], view.strides[i] = view.strides[i + 1];
-    for (const Ref& r : arrays) {
-        CopyInto(r.arr(), view);
+    std::vector<hipcx_array> views;
+    for (size_t i = 0; i < arrays.size(); ++i) {
+        views.push_back(view);
         view.data = static_cast<char*>(view.data) + step;
     }
+    CopyInto(arrays, views);
     return out.release();
     HOST_CATCH(nullptr);
 }

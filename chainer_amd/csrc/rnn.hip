@@ -22,9 +22,11 @@
 // The reference's cuda backend gets these numbers from cuDNN (CX/cuda/cuda_device/rnn.cu); every other backend from autograd over the
 // composition.  Sums run in another order than either: equal to float32 tolerance.
 #include <algorithm>
+#include <utility>
 #include <vector>
 
 #include "common.h"
+#include "dot_parts.h"
 
 extern "C" {
 size_t hipcx_n_step_lstm_workspace_size(int n_layers, const hipcx_array* hx, const hipcx_array* const* xs, int n_steps);
@@ -42,10 +44,11 @@ int NumGates(int mode) { return mode == kLstm ? 4 : (mode == kGru ? 3 : 1); }   
 int ReserveGates(int mode) { return mode == kRnn ? 1 : 4; }  // saved values per unit and row: LSTM i f g o; GRU r z n hh; RNN h
 
 struct CellArgs {
-    int mode, relu;
+    int relu;
     int Bt, H;
     const float* xw;    // [Bt][G*H]: this step's rows of the input projection
-    const float* hw;    // [Bt][G*H]: h . Wh^T
+    const float* hw;    // [splits][Bt][G*H]: h . Wh^T in parts of the reduction
+    int splits;
     const float* bx;    // [G*H]
     const float* bh;    // [G*H]
     float* h;           // [B][H] state, rows < Bt updated in place
@@ -59,18 +62,34 @@ struct CellArgs {
 
 __device__ __forceinline__ float Sigmoid(float v) { return 1.0f / (1.0f + expf(-v)); }  // CX/routines/activation.cc:74-78
 
+// sum[g] of the parts p[s * stride + g * H], s < splits, in that order.
+template <int G>
+__device__ __forceinline__ void SumParts(const float* p, int splits, int64_t stride, int H, float (&sum)[G]) {
+#pragma unroll
+    for (int g = 0; g < G; ++g) sum[g] = 0.f;
+#pragma unroll 4
+    for (int s = 0; s < splits; ++s) {
+#pragma unroll
+        for (int g = 0; g < G; ++g) sum[g] += p[s * stride + g * H];
+    }
+}
+
+// A step's cells.  Bound by the latency of a few loads; the product h . Wh^T arrives in the parts its reduction was split into.
+template <int MODE>
 __global__ __launch_bounds__(256) void RnnCellKernel(CellArgs p) {
+    constexpr int G = MODE == kLstm ? 4 : (MODE == kGru ? 3 : 1);
     const int total = p.Bt * p.H;
-    const int GH = p.H * (p.mode == kLstm ? 4 : (p.mode == kGru ? 3 : 1));
+    const int GH = p.H * G;
     for (int idx = blockIdx.x * 256 + threadIdx.x; idx < total; idx += gridDim.x * 256) {
         const int r = idx / p.H, u = idx - r * p.H;
         const float* xw = p.xw + static_cast<int64_t>(r) * GH + u;
-        const float* hw = p.hw + static_cast<int64_t>(r) * GH + u;
-        auto pre = [&](int g) { return (xw[g * p.H] + p.bx[g * p.H + u]) + (hw[g * p.H] + p.bh[g * p.H + u]); };  // Linear(x) + Linear(h)
+        float hw[G];
+        SumParts<G>(p.hw + static_cast<int64_t>(r) * GH + u, p.splits, static_cast<int64_t>(p.Bt) * GH, p.H, hw);
+        auto pre = [&](int g) { return (xw[g * p.H] + p.bx[g * p.H + u]) + (hw[g] + p.bh[g * p.H + u]); };  // Linear(x) + Linear(h)
         float* hs = p.h + static_cast<int64_t>(r) * p.H + u;
         const float h_old = *hs;
         float h_new;
-        if (p.mode == kLstm) {
+        if constexpr (MODE == kLstm) {
             float* cs = p.c + static_cast<int64_t>(r) * p.H + u;
             const float c_old = *cs;
             const float gi = Sigmoid(pre(0)), gf = Sigmoid(pre(1)), gg = tanhf(pre(2)), go = Sigmoid(pre(3));
@@ -82,9 +101,9 @@ __global__ __launch_bounds__(256) void RnnCellKernel(CellArgs p) {
                 q[0] = gi, q[p.H] = gf, q[2 * p.H] = gg, q[3 * p.H] = go;
                 p.cprev[idx] = c_old;
             }
-        } else if (p.mode == kGru) {
+        } else if constexpr (MODE == kGru) {
             const float gr = Sigmoid(pre(0)), gz = Sigmoid(pre(1));
-            const float hh = hw[2 * p.H] + p.bh[2 * p.H + u];
+            const float hh = hw[2] + p.bh[2 * p.H + u];
             const float gn = tanhf((xw[2 * p.H] + p.bx[2 * p.H + u]) + gr * hh);
             h_new = (1.0f - gz) * gn + gz * h_old;
             if (p.gates != nullptr) {
@@ -103,12 +122,14 @@ __global__ __launch_bounds__(256) void RnnCellKernel(CellArgs p) {
 }
 
 struct CellGradArgs {
-    int mode, relu;
+    int relu;
     int Bt, H;
     const float* dy;  // this step's rows of the gradient of the layer's output, this direction's columns
     int64_t dy_stride;
-    float* dh;        // [B][H]: in, the gradient of the state after the step; out, the part of the gradient of the state before
-                      // the step that does not pass through Wh (GRU: dh * z, else 0) -- the caller adds dGh . Wh
+    float* dh;        // [B][H]: the part of the gradient of the state after the step that did not pass through Wh in the step behind it;
+                      // out, the same for the step before (GRU: dh * z, else 0)
+    const float* parts;  // [splits][part_rows][H]: the other part, dGh . Wh of the step behind, in parts of its reduction
+    int splits, part_rows;
     float* dc;        // [B][H] (LSTM), updated in place
     const float* gates;
     const float* hprev;
@@ -117,13 +138,25 @@ struct CellGradArgs {
     float* dgh;       // [Bt][G*H]: gradient of h . Wh^T + bh (the same array as dgx unless GRU)
 };
 
+// Rows from Bt to part_rows, which the step does not hold, only take in their parts.
+template <int MODE>
 __global__ __launch_bounds__(256) void RnnCellGradKernel(CellGradArgs p) {
-    const int total = p.Bt * p.H;
+    const int total = max(p.Bt, p.part_rows) * p.H;
     for (int idx = blockIdx.x * 256 + threadIdx.x; idx < total; idx += gridDim.x * 256) {
         const int r = idx / p.H, u = idx - r * p.H;
         float* dhs = p.dh + static_cast<int64_t>(r) * p.H + u;
-        const float dh = *dhs + p.dy[static_cast<int64_t>(r) * p.dy_stride + u];
-        if (p.mode == kLstm) {
+        float after = *dhs;
+        if (r < p.part_rows) {
+            float sum[1];
+            SumParts<1>(p.parts + idx, p.splits, static_cast<int64_t>(p.part_rows) * p.H, p.H, sum);
+            after += sum[0];
+        }
+        if (r >= p.Bt) {
+            *dhs = after;
+            continue;
+        }
+        const float dh = after + p.dy[static_cast<int64_t>(r) * p.dy_stride + u];
+        if constexpr (MODE == kLstm) {
             const float* q = p.gates + static_cast<int64_t>(r) * 4 * p.H + u;
             const float gi = q[0], gf = q[p.H], gg = q[2 * p.H], go = q[3 * p.H];
             const float c_old = p.cprev[idx];
@@ -137,7 +170,7 @@ __global__ __launch_bounds__(256) void RnnCellGradKernel(CellGradArgs p) {
             g[3 * p.H] = dh * tc * go * (1.0f - go);
             *dcs = dc * gf;
             *dhs = 0.0f;
-        } else if (p.mode == kGru) {
+        } else if constexpr (MODE == kGru) {
             const float* q = p.gates + static_cast<int64_t>(r) * 4 * p.H + u;
             const float gr = q[0], gz = q[p.H], gn = q[2 * p.H], hh = q[3 * p.H];
             const float h_old = p.hprev[idx];
@@ -155,6 +188,14 @@ __global__ __launch_bounds__(256) void RnnCellGradKernel(CellGradArgs p) {
             *dhs = 0.0f;
         }
     }
+}
+
+// f<mode> for the mode of a call
+template <typename F>
+void VisitMode(int mode, F&& f) {
+    if (mode == kLstm) f(std::integral_constant<int, kLstm>{});
+    else if (mode == kGru) f(std::integral_constant<int, kGru>{});
+    else f(std::integral_constant<int, kRnn>{});
 }
 
 size_t Round256(size_t v) { return (v + 255) / 256 * 256; }
@@ -279,8 +320,33 @@ public:
         HIPCX_REQUIRE(scratch_off_ + need <= bytes_, HIPCX_CHAINERX_ERROR, "n_step_rnn workspace too small for a sum");
         CheckStatus(hipcx_sum(&a, &axis, 1, &out, base_ + scratch_off_, bytes_ - scratch_off_, stream_));
     }
+    // a . b in splits > 1 parts (DotPartSplits) at `parts`, or whole there
+    void DotInParts(const hipcx_array& a, const hipcx_array& b, float* parts, int splits) {
+        if (splits == 1) return Dot(a, b, Matrix(parts, a.shape[0], b.shape[1], b.shape[1]));
+        if (!dry_) DotParts(&a, &b, parts, splits, hip_stream());
+    }
+    // outs[i] = a_i . b for left operands `distance` elements apart
+    void DotEach(const hipcx_array& a0, int64_t distance, const hipcx_array& b, const hipcx_array* const* outs, int n) {
+        if (!dry_ && DotSeveral(&a0, distance, &b, outs, n, hip_stream())) return;
+        hipcx_array a = a0;
+        for (int i = 0; i < n; ++i) {
+            Dot(a, b, *outs[i]);
+            a.data = static_cast<float*>(a.data) + distance;
+        }
+    }
+    // Copies run together, at the next FlushCopies()
     void Copy(const hipcx_array& a, const hipcx_array& out) {
-        if (!dry_) CheckStatus(hipcx_copy(&a, &out, stream_));
+        copies_.push_back(a);
+        copies_.push_back(out);
+    }
+    void FlushCopies() {
+        std::vector<const hipcx_array*> from, to;
+        for (size_t i = 0; i < copies_.size(); i += 2) {
+            from.push_back(&copies_[i]);
+            to.push_back(&copies_[i + 1]);
+        }
+        if (!dry_) CheckStatus(hipcx_copy_many(from.data(), to.data(), static_cast<int>(from.size()), stream_));
+        copies_.clear();
     }
     void Add(const hipcx_array& a, const hipcx_array& b, const hipcx_array& out) {
         if (!dry_) CheckStatus(hipcx_add(&a, &b, &out, stream_));
@@ -297,13 +363,22 @@ private:
     void* stream_;
     bool dry_;
     size_t used_ = 0, scratch_off_ = 0, scratch_need_ = 0;
+    std::vector<hipcx_array> copies_;
 };
+
+// Most floats that DotInParts needs over the steps of a pass for [bt, k] . [k, n].
+int64_t PartFloats(const RnnPlan& pl, int64_t n, int64_t k) {
+    int64_t most = 0;
+    for (int64_t bt : pl.bt) most = std::max(most, DotPartSplits(bt, n, k) * bt * n);
+    return most;
+}
 
 struct PackedWeights {
     std::vector<float*> wx, wh, bx, bh;  // per layer-direction: [G*H][in], [G*H][H], [G*H], [G*H]
 };
 
 // Stacks the matrices and biases of every layer-direction, gate-major: rows [g*H, (g+1)*H) of wx are ws[idx][g], of wh ws[idx][G + g].
+// bs null: the matrices alone, which is all the backward pass reads.
 PackedWeights PackWeights(Pass& pass, const RnnPlan& pl, const hipcx_array* const* ws, const hipcx_array* const* bs) {
     PackedWeights pw;
     const int G = pl.G;
@@ -311,18 +386,16 @@ PackedWeights PackWeights(Pass& pass, const RnnPlan& pl, const hipcx_array* cons
         const int64_t in = pl.In(idx / pl.D);
         pw.wx.push_back(pass.Take(G * pl.H * in));
         pw.wh.push_back(pass.Take(G * pl.H * pl.H));
-        pw.bx.push_back(pass.Take(G * pl.H));
-        pw.bh.push_back(pass.Take(G * pl.H));
+        pw.bx.push_back(bs != nullptr ? pass.Take(G * pl.H) : nullptr);
+        pw.bh.push_back(bs != nullptr ? pass.Take(G * pl.H) : nullptr);
         if (pass.dry()) continue;
         for (int g = 0; g < 2 * G; ++g) {
             const hipcx_array* w = ws[idx * 2 * G + g];
-            const hipcx_array* b = bs[idx * 2 * G + g];
             const bool xside = g < G;
             const int64_t cols = xside ? in : pl.H;
             float* wdst = (xside ? pw.wx[idx] : pw.wh[idx]) + static_cast<int64_t>(g % G) * pl.H * cols;
-            float* bdst = (xside ? pw.bx[idx] : pw.bh[idx]) + static_cast<int64_t>(g % G) * pl.H;
             pass.Copy(*w, Matrix(wdst, pl.H, cols, cols));
-            pass.Copy(*b, Vector(bdst, pl.H));
+            if (bs != nullptr) pass.Copy(*bs[idx * 2 * G + g], Vector((xside ? pw.bx[idx] : pw.bh[idx]) + static_cast<int64_t>(g % G) * pl.H, pl.H));
         }
     }
     return pw;
@@ -393,7 +466,7 @@ void RunForward(Pass& pass, const RnnPlan& pl, int activation, const hipcx_array
         if (pl.L > 2) y_buf[1] = pass.Take(rows * DH);
     }
     float* xw_all = pass.Take(rows * GH);
-    float* hw = pass.Take(B * GH);
+    float* hw = pass.Take(PartFloats(pl, GH, H));
     float* h_state = pass.Take(B * H);
     float* c_state = pl.mode == kLstm ? pass.Take(B * H) : nullptr;
     pass.StartScratch();
@@ -404,17 +477,19 @@ void RunForward(Pass& pass, const RnnPlan& pl, int activation, const hipcx_array
         float* y_out = l + 1 == pl.L ? nullptr : (reserve != nullptr ? reinterpret_cast<float*>(reserve + pl.r_y[l]) : y_buf[l & 1]);
         for (int d = 0; d < pl.D; ++d) {
             const int idx = l * pl.D + d;
-            // the input projection of every step at once
-            pass.Dot(Matrix(x_in, rows, in, in), Matrix(pw.wx[idx], in, GH, 1, in), Matrix(xw_all, rows, GH, GH));
             pass.Copy(StateSlice(hx, idx), Matrix(h_state, B, H, H));
             if (pl.mode == kLstm) pass.Copy(StateSlice(cx, idx), Matrix(c_state, B, H, H));
+            pass.FlushCopies();
+            // the input projection of every step at once
+            pass.Dot(Matrix(x_in, rows, in, in), Matrix(pw.wx[idx], in, GH, 1, in), Matrix(xw_all, rows, GH, GH));
             for (int s = 0; s < pl.T; ++s) {
                 const int t = d == 0 ? s : pl.T - 1 - s;
                 const int64_t bt = pl.bt[t], r0 = pl.row_start[t];
-                pass.Dot(Matrix(h_state, bt, H, H), Matrix(pw.wh[idx], H, GH, 1, H), Matrix(hw, bt, GH, GH));
+                const int splits = DotPartSplits(bt, GH, H);
+                pass.DotInParts(Matrix(h_state, bt, H, H), Matrix(pw.wh[idx], H, GH, 1, H), hw, splits);
                 if (pass.dry()) continue;
                 CellArgs a{};
-                a.mode = pl.mode, a.relu = activation == 1;
+                a.splits = splits, a.relu = activation == 1;
                 a.Bt = static_cast<int>(bt), a.H = static_cast<int>(H);
                 a.xw = xw_all + r0 * GH;
                 a.hw = hw;
@@ -432,11 +507,14 @@ void RunForward(Pass& pass, const RnnPlan& pl, int activation, const hipcx_array
                     a.hprev = reinterpret_cast<float*>(reserve + pl.r_hprev[idx]) + r0 * H;
                     a.cprev = pl.mode == kLstm ? reinterpret_cast<float*>(reserve + pl.r_cprev[idx]) + r0 * H : nullptr;
                 }
-                hipLaunchKernelGGL(RnnCellKernel, dim3(CellBlocks(bt * H)), dim3(256), 0, pass.hip_stream(), a);
+                VisitMode(pl.mode, [&](auto mode) {
+                    hipLaunchKernelGGL(RnnCellKernel<decltype(mode)::value>, dim3(CellBlocks(bt * H)), dim3(256), 0, pass.hip_stream(), a);
+                });
                 CheckLaunch("rnn_cell");
             }
             pass.Copy(Matrix(h_state, B, H, H), StateSlice(hy, idx));
             if (pl.mode == kLstm) pass.Copy(Matrix(c_state, B, H, H), StateSlice(cy, idx));
+            pass.FlushCopies();
         }
     }
     pass.CheckFits();
@@ -448,7 +526,7 @@ void RunBackward(Pass& pass, const RnnPlan& pl, int activation, const hipcx_arra
                  const hipcx_array* dhx, const hipcx_array* dcx, const hipcx_array* const* dws, const hipcx_array* const* dbs,
                  const hipcx_array* const* dxs) {
     const int64_t B = pl.B, H = pl.H, GH = pl.G * H, DH = pl.D * H, rows = pl.rows;
-    PackedWeights pw = PackWeights(pass, pl, ws, bs);
+    PackedWeights pw = PackWeights(pass, pl, ws, nullptr);
     float* x_all = pass.Take(rows * pl.I);
     float* dy_cur = pass.Take(rows * pl.max_in);   // gradient of the current layer's output rows [rows][D*H]
     float* dx_acc = pass.Take(rows * pl.max_in);   // gradient of its input rows [rows][in]
@@ -457,7 +535,8 @@ void RunBackward(Pass& pass, const RnnPlan& pl, int activation, const hipcx_arra
     float* dgh_all = pl.mode == kGru ? pass.Take(rows * GH) : dgx_all;
     float* dh = pass.Take(B * H);
     float* dc = pl.mode == kLstm ? pass.Take(B * H) : nullptr;
-    float* tmp = pass.Take(B * H);
+    float* parts = pass.Take(PartFloats(pl, H, GH));
+    float* db = pass.Take(pl.L * pl.D * 2 * GH);
     pass.StartScratch();
     for (int t = 0; t < pl.T; ++t) pass.Copy(*xs[t], Matrix(x_all + pl.row_start[t] * pl.I, pl.bt[t], pl.I, pl.I));
     for (int t = 0; t < pl.T; ++t) {
@@ -465,6 +544,14 @@ void RunBackward(Pass& pass, const RnnPlan& pl, int activation, const hipcx_arra
         if (dys[t] != nullptr) pass.Copy(*dys[t], dst);
         else pass.Zero(dst);
     }
+    std::vector<std::pair<hipcx_array, hipcx_array>> db_copies;
+    auto launch_cells = [&](const CellGradArgs& a) {
+        VisitMode(pl.mode, [&](auto mode) {
+            const int64_t cells = static_cast<int64_t>(std::max(a.Bt, a.part_rows)) * H;
+            hipLaunchKernelGGL(RnnCellGradKernel<decltype(mode)::value>, dim3(CellBlocks(cells)), dim3(256), 0, pass.hip_stream(), a);
+        });
+        CheckLaunch("rnn_cell_grad");
+    };
     for (int l = pl.L - 1; l >= 0; --l) {
         const int64_t in = pl.In(l);
         const float* x_in = l == 0 ? x_all : reinterpret_cast<const float*>(reserve + pl.r_y[l - 1]);
@@ -478,12 +565,14 @@ void RunBackward(Pass& pass, const RnnPlan& pl, int activation, const hipcx_arra
                 if (dcy != nullptr) pass.Copy(StateSlice(dcy, idx), Matrix(dc, B, H, H));
                 else pass.Zero(Matrix(dc, B, H, H));
             }
+            pass.FlushCopies();
+            CellGradArgs a{};  // the step behind the last one has no parts
             for (int s = pl.T - 1; s >= 0; --s) {  // the forward order of this direction, backwards
                 const int t = d == 0 ? s : pl.T - 1 - s;
                 const int64_t bt = pl.bt[t], r0 = pl.row_start[t];
+                const int splits = DotPartSplits(bt, H, GH);
                 if (!pass.dry()) {
-                    CellGradArgs a{};
-                    a.mode = pl.mode, a.relu = activation == 1;
+                    a.relu = activation == 1;
                     a.Bt = static_cast<int>(bt), a.H = static_cast<int>(H);
                     a.dy = dy_cur + r0 * DH + d * H;
                     a.dy_stride = DH;
@@ -493,23 +582,27 @@ void RunBackward(Pass& pass, const RnnPlan& pl, int activation, const hipcx_arra
                     a.cprev = cprev != nullptr ? cprev + r0 * H : nullptr;
                     a.dgx = dgx_all + r0 * GH;
                     a.dgh = dgh_all + r0 * GH;
-                    hipLaunchKernelGGL(RnnCellGradKernel, dim3(CellBlocks(bt * H)), dim3(256), 0, pass.hip_stream(), a);
-                    CheckLaunch("rnn_cell_grad");
+                    launch_cells(a);
                 }
                 // dh of the state before the step: what the cell left there plus dGh . Wh
-                pass.Dot(Matrix(dgh_all + r0 * GH, bt, GH, GH), Matrix(pw.wh[idx], GH, H, H), Matrix(tmp, bt, H, H));
-                pass.Add(Matrix(dh, bt, H, H), Matrix(tmp, bt, H, H), Matrix(dh, bt, H, H));
+                pass.DotInParts(Matrix(dgh_all + r0 * GH, bt, GH, GH), Matrix(pw.wh[idx], GH, H, H), parts, splits);
+                a.parts = parts, a.splits = splits, a.part_rows = static_cast<int>(bt);
             }
+            a.Bt = 0;
+            if (!pass.dry()) launch_cells(a);
             pass.Copy(Matrix(dh, B, H, H), StateSlice(dhx, idx));
             if (pl.mode == kLstm) pass.Copy(Matrix(dc, B, H, H), StateSlice(dcx, idx));
-            // parameter gradients over all rows at once
-            for (int g = 0; g < pl.G; ++g) {
-                const hipcx_array gx_t = Matrix(dgx_all + g * H, H, rows, 1, GH);  // dGx[:, g]^T
-                const hipcx_array gh_t = Matrix(dgh_all + g * H, H, rows, 1, GH);
-                pass.Dot(gx_t, Matrix(x_in, rows, in, in), *dws[idx * 2 * pl.G + g]);
-                pass.Dot(gh_t, Matrix(hprev, rows, H, H), *dws[idx * 2 * pl.G + pl.G + g]);
-                pass.SumRows(Matrix(dgx_all + g * H, rows, H, GH), *dbs[idx * 2 * pl.G + g]);
-                pass.SumRows(Matrix(dgh_all + g * H, rows, H, GH), *dbs[idx * 2 * pl.G + pl.G + g]);
+            pass.FlushCopies();
+            // parameter gradients over all rows at once: dGx[:, g]^T . x and dGh[:, g]^T . h for all gates g in a launch each
+            pass.DotEach(Matrix(dgx_all, H, rows, 1, GH), H, Matrix(x_in, rows, in, in), dws + idx * 2 * pl.G, pl.G);
+            pass.DotEach(Matrix(dgh_all, H, rows, 1, GH), H, Matrix(hprev, rows, H, H), dws + idx * 2 * pl.G + pl.G, pl.G);
+            // the biases' are column sums of all gates at once; they go to their arrays at the end
+            float* const db_x = db + static_cast<int64_t>(idx) * 2 * GH;
+            float* const db_h = dgh_all == dgx_all ? db_x : db_x + GH;
+            pass.SumRows(Matrix(dgx_all, rows, GH, GH), Vector(db_x, GH));
+            if (db_h != db_x) pass.SumRows(Matrix(dgh_all, rows, GH, GH), Vector(db_h, GH));
+            for (int g = 0; g < 2 * pl.G; ++g) {
+                db_copies.emplace_back(Vector((g < pl.G ? db_x : db_h) + (g % pl.G) * H, H), *dbs[idx * 2 * pl.G + g]);
             }
             // gradient of the layer's input rows; the second direction adds to the first
             if (d == 0) {
@@ -522,6 +615,8 @@ void RunBackward(Pass& pass, const RnnPlan& pl, int activation, const hipcx_arra
         std::swap(dy_cur, dx_acc);  // the layer below produced these rows
     }
     for (int t = 0; t < pl.T; ++t) pass.Copy(Matrix(dy_cur + pl.row_start[t] * pl.I, pl.bt[t], pl.I, pl.I), *dxs[t]);
+    for (const auto& c : db_copies) pass.Copy(c.first, c.second);
+    pass.FlushCopies();
     pass.CheckFits();
 }
 

@@ -187,6 +187,7 @@ int hipcx_greater_equal(const hipcx_array* x1, const hipcx_array* x2, const hipc
 
 /* ---- creation: CX/kernels/creation.h, misc.h ---- */
 int hipcx_copy(const hipcx_array* a, const hipcx_array* out, void* stream);                       /* CopyKernel creation.h:16 (dtype-casting) */
+int hipcx_copy_many(const hipcx_array* const* as, const hipcx_array* const* outs, int n, void* stream);  /* n copies, none of which reads what another writes */
 int hipcx_fill(const hipcx_array* out, hipcx_scalar value, void* stream);                         /* FillKernel misc.h:9 */
 int hipcx_arange(hipcx_scalar start, hipcx_scalar step, const hipcx_array* out, void* stream);    /* ArangeKernel creation.h:11 */
 
