@@ -197,49 +197,6 @@ void LaunchIGemmImpl(IGemmArgs<T> p, hipStream_t stream) {
 }
 
 
-// Large float16 products with both operands' reduction index at unit stride (gemm_pp.h).  Returns false when the problem does
-// not qualify: the 128 x 128 kernels below then take it.
-bool TryGemmPp(const hipcx_array* a, const hipcx_array* b, const hipcx_array* bias, const hipcx_array* out, hipStream_t stream) {
-    static const bool enabled = [] { const char* e = getenv("HIPCX_DOT_PP"); return e == nullptr || e[0] != '0'; }();
-    static const int band = [] { const char* e = getenv("HIPCX_DOT_PP_BAND"); return e != nullptr && atoi(e) > 0 ? atoi(e) : 8; }();
-    if (!enabled) return false;
-    const int64_t M = a->shape[0], K = a->shape[1], N = b->shape[1];
-    if (K % 32 != 0 || K < gemm_pp::kMinK || N % 4 != 0) return false;
-    // a: rows of K contiguous halves; b: columns of K contiguous halves (the view Linear hands over, or a staged copy)
-    if (a->strides[1] != 2 || b->strides[0] != 2 || out->strides[1] != 2) return false;
-    const int64_t lda = a->strides[0] / 2, ldb = b->strides[1] / 2, ldc = out->strides[0] / 2;
-    if (a->strides[0] % 16 != 0 || b->strides[1] % 16 != 0 || out->strides[0] % 8 != 0 || lda < K || ldb < K || ldc < N) return false;
-    if (reinterpret_cast<uintptr_t>(a->data) % 16 != 0 || reinterpret_cast<uintptr_t>(b->data) % 16 != 0 || reinterpret_cast<uintptr_t>(out->data) % 8 != 0) return false;
-    if (256 * lda * 2 >= (1LL << 31) || 256 * ldb * 2 >= (1LL << 31)) return false;  // 32-bit offsets inside a tile's rows
-    const int64_t tiles_m = (M + 255) / 256, tiles_n = (N + 255) / 256;
-    // enough 256 x 256 tiles to occupy most of the chip; smaller products fill it better with 128 x 128 tiles
-    if (tiles_m * tiles_n < (NumCUs() * 3) / 4 || tiles_m * tiles_n >= (1LL << 24)) return false;
-    gemm_pp::GemmArgs p{};
-    p.a = static_cast<const half_t*>(a->data);
-    p.b = static_cast<const half_t*>(b->data);
-    p.c = static_cast<half_t*>(out->data);
-    p.M = static_cast<int>(M);
-    p.N = static_cast<int>(N);
-    p.K = static_cast<int>(K);
-    p.lda = static_cast<int>(lda);
-    p.ldb = static_cast<int>(ldb);
-    p.ldc = static_cast<int>(ldc);
-    p.tiles_m = static_cast<int>(tiles_m);
-    p.tiles_n = static_cast<int>(tiles_n);
-    p.band = band;
-    if (bias != nullptr) {
-        p.bias = static_cast<const half_t*>(bias->data);
-        p.bias_stride = bias->strides[0] / 2;
-    }
-    ProfileScope prof(stream, 2.0 * static_cast<double>(M) * N * K, 2.0 * (static_cast<double>(M) * K + static_cast<double>(N) * K + static_cast<double>(M) * N));
-    struct GemmPpTag {};
-    EnsureDynamicLds<GemmPpTag>(reinterpret_cast<const void*>(gemm_pp::GemmPpKernel), gemm_pp::kLdsBytes);
-    const unsigned grid = static_cast<unsigned>((tiles_m * tiles_n + 7) / 8 * 8);
-    hipLaunchKernelGGL(gemm_pp::GemmPpKernel, dim3(grid), dim3(512), gemm_pp::kLdsBytes, stream, p);
-    CheckLaunch("gemm_pp");
-    return true;
-}
-
 // Workgroups that share a tile's reduction: while tiles leave compute units without one, but at least 896 bytes of a row each.
 int PlanSmallDotSplit(int64_t m, int64_t n, int64_t k, int dtype) {
     const int64_t tiles = ((m + 31) / 32) * ((n + 31) / 32), lines = (k * ItemSize(dtype) + 127) / 128;
@@ -327,10 +284,10 @@ void LaunchSmallDot(SmallDotArgs p, int a_mode, int b_mode, int batch, hipStream
         CheckLaunch("small_dot");
         return;
     }
-    // Elements wait for their own loads: chunks of 32 bytes, six of them in flight, beat whole lines while latency is what counts
-    // ([32,1000] . [1000,2048] float16 14.3 -> 5.5 us, [20,2600] . [2600,650] float32 13.4 -> 9.3); rows of odd pitch gain from whole
-    // lines at any size.
-    const int pieces = latency_bound && a_mode != kOddPieces && b_mode != kOddPieces ? 1 : 4;
+    // Elements come as they are used: chunks of 32 bytes, six of them in flight, beat whole lines ([32,1000] . [1000,2048] float16 14.3 -> 5.5 us,
+    // [200,4000] . [4000,4000] 174 -> 51, [20,2600] . [2600,650] float32 13.4 -> 9.3); rows of odd pitch gain from whole lines at any size.
+    const bool elements = a_mode == kElements || b_mode == kElements, odd = a_mode == kOddPieces || b_mode == kOddPieces;
+    const int pieces = (latency_bound || elements) && !odd ? 1 : 4;
     // eight waves keep more loads in flight; four, one per SIMD, once there is a workgroup for every compute unit
     const int chunk = pieces == 1 ? 32 : 128, chunks = (p.K * static_cast<int>(sizeof(T)) + chunk - 1) / chunk;
     const int per_split = (chunks + p.ksplit - 1) / p.ksplit;
@@ -1521,6 +1478,121 @@ int PlanSplitK(int64_t m, int64_t n, int64_t k, int dtype) {
 size_t SplitKBytes(int64_t m, int64_t n, int slices) { return slices > 1 ? static_cast<size_t>(slices) * m * n * sizeof(float) : 0; }
 }  // namespace
 
+namespace {
+// Large float16 products (gemm_pp.h): whether they take this one, in how many slices of the reduction, and the workspace for it: operands whose
+// reduction axis is not the unit-stride one (or whose rows are not dword-aligned) laid out anew, then the partial sums.
+struct GemmPpPlan {
+    int slices = 0;  // 0: left to the other kernels
+    bool stage_a = false, stage_b = false;
+    int64_t pitch = 0;  // of a staged row, elements
+    size_t a_bytes = 0, b_bytes = 0, partial_bytes = 0;
+    size_t Total() const { return a_bytes + b_bytes + partial_bytes; }
+};
+
+// The estimates, in us, are fits to measured products.  256 x 256 tiles: 0.85 for a chunk of 32 k, 5 for a tile's start and end, one tile at a time on
+// a compute unit, the result at 5 TB/s (nothing else runs meanwhile), partial sums written and read at 4 TB/s, staging at 3.5 TB/s.  The 128 x 128
+// kernel: 450 TFLOP/s on rows of 16-byte pieces, 350 of 8.  The 32 x 32 tiles of small outputs: 130, a third of it for operands read element by element.
+// The large tiles have to win by a fifth.
+GemmPpPlan PlanGemmPp(const hipcx_array* a, const hipcx_array* b, const hipcx_array* out) {
+    GemmPpPlan pl;
+    static const bool enabled = [] { const char* e = getenv("HIPCX_DOT_PP"); return e == nullptr || e[0] != '0'; }();
+    if (!enabled || a == nullptr || b == nullptr || out == nullptr || out->dtype != HIPCX_FLOAT16 || a->ndim != 2 || b->ndim != 2) return pl;
+    const int64_t m = a->shape[0], k = a->shape[1], n = b->shape[1];
+    if (k < gemm_pp::kMinK || m < 64 || n < 64) return pl;
+    for (const hipcx_array* x : {a, b, out}) {
+        if (x->strides[0] % 2 != 0 || x->strides[1] % 2 != 0) return pl;
+    }
+    if (out->strides[1] != 2 || out->strides[0] < 2 * n || out->strides[0] >= (1LL << 31)) return pl;
+    const int64_t tiles = ((m + 255) / 256) * ((n + 255) / 256), chunks = (k + 31) / 32;
+    pl.pitch = (k + 7) / 8 * 8;
+    if (tiles >= (1LL << 20) || 512 * pl.pitch >= (1LL << 31)) return pl;  // 32-bit offsets inside a tile's rows
+    auto fits = [&](const void* ptr, int64_t line, int64_t k_stride) {
+        return k_stride == 2 && reinterpret_cast<uintptr_t>(ptr) % 4 == 0 && line % 4 == 0 && line >= 2 * k && 128 * line + 2 * k < (1LL << 30);
+    };
+    pl.stage_a = !fits(a->data, a->strides[0], a->strides[1]);
+    pl.stage_b = !fits(b->data, b->strides[1], b->strides[0]);
+    const double flops = 2.0 * m * n * k, out_us = 2.0 * m * n / 5e6;
+    auto stage_us = [&](bool needed, int64_t lines) { return needed ? 2.0 + 4.0 * lines * k / 3.5e6 : 0.0; };
+    const bool small = SmallDotShape(m, n, k), rows = a->strides[1] == 2 && b->strides[0] == 2;
+    const bool wide = rows && k % 8 == 0 && a->strides[0] % 16 == 0 && b->strides[1] % 16 == 0;
+    double other;
+    if (small) other = std::max(8.0, flops / (rows ? 130e6 : 45e6));
+    else other = 4.0 + out_us + flops / (!rows || wide ? 450e6 : 350e6) + stage_us(a->strides[1] != 2, m) + stage_us(b->strides[0] != 2, n);
+    // (on equal terms they may be level: most of the time of short reductions goes into the result)
+    double least = (wide && k % 32 == 0 && tiles >= (NumCUs() * 3) / 4 ? 1.05 : 0.8) * other;
+    for (int s = 1; s <= 16 && chunks / s >= 8 * (s > 1); ++s) {
+        // every slice has work for the pipeline's prologue
+        if (chunks - (s - 1) * ((chunks + s - 1) / s) < gemm_pp::kMinK / 32) continue;
+        const int64_t rounds = (tiles * s + NumCUs() - 1) / NumCUs();
+        const double t = rounds * (((chunks + s - 1) / s) * 0.85 + 5.0) + (s > 1 ? 2.0 + 8.0 * s * m * n / 4e6 : out_us) + stage_us(pl.stage_a, m) + stage_us(pl.stage_b, n);
+        if (t < least) least = t, pl.slices = s;
+    }
+    pl.a_bytes = pl.stage_a ? RoundUpTo(static_cast<size_t>(m * pl.pitch * 2), 256) : 0;
+    pl.b_bytes = pl.stage_b ? RoundUpTo(static_cast<size_t>(n * pl.pitch * 2), 256) : 0;
+    pl.partial_bytes = SplitKBytes(m, n, pl.slices);
+    return pl;
+}
+
+bool TryGemmPp(const hipcx_array* a, const hipcx_array* b, const hipcx_array* bias, const hipcx_array* out, void* workspace, size_t workspace_bytes,
+               hipStream_t stream) {
+    static const int band = [] { const char* e = getenv("HIPCX_DOT_PP_BAND"); return e != nullptr && atoi(e) > 0 ? atoi(e) : 8; }();
+    const int64_t M = a->shape[0], K = a->shape[1], N = b->shape[1];
+    const GemmPpPlan space = PlanGemmPp(a, b, out);
+    const int slices = space.slices;
+    if (slices == 0) return false;
+    if (space.Total() > 0 && (workspace == nullptr || workspace_bytes < space.Total() || reinterpret_cast<uintptr_t>(workspace) % 16 != 0)) return false;
+    char* const ws = static_cast<char*>(workspace);
+    gemm_pp::GemmArgs p{};
+    p.a = static_cast<const half_t*>(a->data);
+    p.b = static_cast<const half_t*>(b->data);
+    p.c = static_cast<half_t*>(out->data);
+    p.M = static_cast<int>(M);
+    p.N = static_cast<int>(N);
+    p.K = static_cast<int>(K);
+    p.lda = static_cast<int>(a->strides[0] / 2);
+    p.ldb = static_cast<int>(b->strides[1] / 2);
+    p.ldc = static_cast<int>(out->strides[0] / 2);
+    if (space.stage_a) {
+        half_t* const to = reinterpret_cast<half_t*>(ws);
+        StageMatrix<half_t>(p.a, a->strides[0] / 2, a->strides[1] / 2, to, space.pitch, M, K, stream);
+        p.a = to, p.lda = static_cast<int>(space.pitch);
+    }
+    if (space.stage_b) {
+        half_t* const to = reinterpret_cast<half_t*>(ws + space.a_bytes);
+        StageMatrix<half_t>(p.b, b->strides[1] / 2, b->strides[0] / 2, to, space.pitch, N, K, stream);
+        p.b = to, p.ldb = static_cast<int>(space.pitch);
+    }
+    p.tiles_m = static_cast<int>((M + 255) / 256);
+    p.tiles_n = static_cast<int>((N + 255) / 256);
+    p.slices = slices;
+    p.slice_chunks = static_cast<int>(((K + 31) / 32 + slices - 1) / slices);
+    p.partial = slices > 1 ? reinterpret_cast<float*>(ws + space.a_bytes + space.b_bytes) : nullptr;
+    p.band = band;
+    if (bias != nullptr) {
+        p.bias = static_cast<const half_t*>(bias->data);
+        p.bias_stride = bias->strides[0] / 2;
+    }
+    ProfileScope prof(stream, 2.0 * static_cast<double>(M) * N * K, 2.0 * (static_cast<double>(M) * K + static_cast<double>(N) * K + static_cast<double>(M) * N));
+    const unsigned grid = static_cast<unsigned>((static_cast<int64_t>(p.tiles_m) * p.tiles_n * slices + 7) / 8 * 8);
+    auto launch = [&](auto direct) {
+        constexpr bool DIRECT = decltype(direct)::value;
+        struct GemmPpTag {};
+        EnsureDynamicLds<GemmPpTag>(reinterpret_cast<const void*>(gemm_pp::GemmPpKernel<DIRECT>), gemm_pp::kLdsBytes);
+        hipLaunchKernelGGL(gemm_pp::GemmPpKernel<DIRECT>, dim3(grid), dim3(512), gemm_pp::kLdsBytes, stream, p);
+    };
+    // short reductions: see the epilogue
+    if (slices == 1 && K <= 256 && N % 4 == 0 && p.ldc % 4 == 0 && Aligned(p.c, 8)) launch(std::true_type{});
+    else launch(std::false_type{});
+    CheckLaunch("gemm_pp");
+    if (slices > 1) {
+        const int64_t threads = M * ((N + 7) / 8);
+        hipLaunchKernelGGL(gemm_pp::GemmSumKernel, dim3(static_cast<unsigned>((threads + 255) / 256)), dim3(256), 0, stream, p);
+        CheckLaunch("gemm_pp sum");
+    }
+    return true;
+}
+}  // namespace
+
 // out[m][n] = sum over b < batch, k < depth of a[b][m][k] * bt[b][n][k]: one matrix product per batch entry, accumulated.  Rows of a_b
 // and bt_b are dense along k; a_row / bt_row are their row strides and a_slice / bt_slice the distances between batch entries, in
 // elements.  out is row-major [m][n].  Float partial sums go to `partial` when BatchedProductSlices(...) > 1
@@ -1653,6 +1725,7 @@ static int DotBias(const hipcx_array* a, const hipcx_array* b, const hipcx_array
             p.M = m;
             p.Kg = static_cast<int>(k);
         };
+        if (out->dtype == HIPCX_FLOAT16 && TryGemmPp(a, b, bias, out, workspace, workspace_bytes, st)) return;
         // operands in another layout than the MFMA kernels read are staged in the workspace first
         hipcx_array a_st = *a, b_st = *b;
         const int64_t k_given = k;  // the reduction extent the workspace query saw (staging may pad it)
@@ -1715,7 +1788,6 @@ static int DotBias(const hipcx_array* a, const hipcx_array* b, const hipcx_array
             }
         }
         if (out->dtype == HIPCX_FLOAT16) {
-            if (slices == 1 && TryGemmPp(a, b, bias, out, st)) return;
             if (slices == 1 && TrySmallDot<half_t>(a, b, bias, out, small_partial, st)) return;
             IGemmArgs<half_t> p{};
             fill(p);
@@ -1749,7 +1821,9 @@ size_t hipcx_dot_workspace_size(const hipcx_array* a, const hipcx_array* b, cons
             split = SplitKBytes(m, n, PlanSplitK(m, n, k, out->dtype));
             if (split == 0 && out->dtype != HIPCX_FLOAT64 && SmallDotShape(m, n, k)) split = SmallDotPartialBytes(m, n, k, out->dtype);
         }
-        return RoundUpTo(st.a_bytes + st.b_bytes, 256) + split;
+        const size_t need = RoundUpTo(st.a_bytes + st.b_bytes, 256) + split;
+        const GemmPpPlan pp = PlanGemmPp(a, b, out);
+        return pp.slices > 0 ? std::max(need, pp.Total()) : need;
     } catch (...) {
         return 0;
     }

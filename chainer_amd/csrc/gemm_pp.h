@@ -11,6 +11,11 @@
 // two groups of four (one of each on every SIMD) that alternate between a memory phase (issue the loads of the chunk two
 // ahead, read the 12 fragments of the current chunk) and an MFMA phase (16 MFMAs on registers), half a period apart and
 // separated by workgroup barriers: while one wave of a SIMD multiplies, the other one feeds.
+// k may be any number: the last chunk is masked in registers; rows need dword alignment only.  Where tiles leave compute units idle the
+// reduction is split over `slices` workgroups, whose float sums GemmSumKernel adds up.
+// Bound by the matrix pipes and, in short reductions, by writing c.  us, against 128 x 128 tiles over padded copies of the operands:
+// [4480,650] . [650,10000] 126 -> 95, [4480,10000] . [10000,650] 188 -> 115, [10000,4480] . [4480,650] with a and b transposed 198 -> 130;
+// [4096,4096]^2 126 (1089 TFLOP/s).
 // Tiles are ordered so that the 32 workgroups an XCD runs at a time cover `band` tile rows x 32 / band tile columns: they
 // share operand rows in that XCD's L2.
 #pragma once
@@ -29,8 +34,11 @@ struct GemmArgs {
     const half_t* b;
     half_t* c;
     int M, N, K;
-    int lda, ldb, ldc;  // elements
+    int lda, ldb, ldc;  // elements; rows of a and b start at multiples of 4 bytes
     int tiles_m, tiles_n;
+    int slices;         // workgroups per tile along k
+    int slice_chunks;   // chunks of 32 k of a slice (the last one may have fewer), at least kMinK / 32
+    float* partial;     // slices > 1: [slices][M][N] sums go there, GemmSumKernel makes c of them
     int band;  // tile rows per band of the tile order
     const half_t* bias;  // one element per column of c, added before the rounding; may be null
     int64_t bias_stride;
@@ -60,7 +68,17 @@ __device__ __forceinline__ void WaitVmcnt() {
 constexpr int kStages = 3;
 constexpr int kLdsBytes = kStages * 2 * 256 * 64;
 constexpr int kMinK = 32 * (kStages - 1);  // the pipeline's prologue issues kStages - 1 chunks
+// Rows of a wave's 32 x 64 block on its way out, a float for partial sums: 16 bytes of padding keep the banks apart.
+constexpr int kOutPitch = 64 * 4 + 16;
+static_assert(8 * 32 * kOutPitch <= kLdsBytes, "the eight waves' blocks fit the ring");
 
+template <typename T>
+struct __attribute__((packed, aligned(2))) OutPiece {  // 16 bytes of c, whose rows may start anywhere
+    T e[16 / sizeof(T)];
+};
+
+// DIRECT: c leaves straight from the registers (one slice, rows of c aligned to 8 bytes, N % 4 == 0).
+template <bool DIRECT>
 __global__ __launch_bounds__(512) void GemmPpKernel(GemmArgs p) {
     constexpr int NSTAGE = kStages, AHEAD = NSTAGE - 1;
     constexpr int TILE_B = 256 * 64;  // bytes of one operand tile in a stage
@@ -71,10 +89,15 @@ __global__ __launch_bounds__(512) void GemmPpKernel(GemmArgs p) {
 
     // ---- tile of this workgroup: XCD x (workgroup ids go round-robin to the 8 XCDs) walks a contiguous range of the tile
     // order; inside it bands of `band` tile rows are walked column by column ----
-    const int total = p.tiles_m * p.tiles_n;
+    const int tiles = p.tiles_m * p.tiles_n;
+    const int total = tiles * p.slices;
     const int per = (total + 7) / 8;
-    const int logical = (static_cast<int>(blockIdx.x) % 8) * per + static_cast<int>(blockIdx.x) / 8;
+    int logical = (static_cast<int>(blockIdx.x) % 8) * per + static_cast<int>(blockIdx.x) / 8;
     if (logical >= total) return;
+    const int slice = logical / tiles;
+    logical -= slice * tiles;
+    const int k0 = slice * p.slice_chunks * 32;
+    const int k_left = p.K - k0;
     int tile_m, tile_n;
     {
         const int band_tiles = p.band * p.tiles_n;
@@ -93,8 +116,10 @@ __global__ __launch_bounds__(512) void GemmPpKernel(GemmArgs p) {
     const int r = lane & 31, h = lane >> 5;
 
     // ---- global -> LDS loads: a wave instruction covers 16 rows x 64 bytes; lane = 4 * row + position ----
-    const int4_t ra = RawRsrc(p.a + static_cast<int64_t>(m0) * p.lda, static_cast<unsigned>(min(p.M - m0, 256)) * static_cast<unsigned>(p.lda) * 2u);
-    const int4_t rb = RawRsrc(p.b + static_cast<int64_t>(n0) * p.ldb, static_cast<unsigned>(min(p.N - n0, 256)) * static_cast<unsigned>(p.ldb) * 2u);
+    // what lies behind the last element of the last row is out of the buffers' bounds (an odd end shares its dword with 2 more bytes)
+    auto span = [&](int rows, int ld) { return ((static_cast<unsigned>(rows - 1) * static_cast<unsigned>(ld) + k_left) * 2u + 3u) & ~3u; };
+    const int4_t ra = RawRsrc(p.a + static_cast<int64_t>(m0) * p.lda + k0, span(min(p.M - m0, 256), p.lda));
+    const int4_t rb = RawRsrc(p.b + static_cast<int64_t>(n0) * p.ldb + k0, span(min(p.N - n0, 256), p.ldb));
     int voa[LPO], vob[LPO];
 #pragma unroll
     for (int i = 0; i < LPO; ++i) {
@@ -162,8 +187,23 @@ __global__ __launch_bounds__(512) void GemmPpKernel(GemmArgs p) {
                     acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8_t, fn[t][j]), __builtin_bit_cast(half8_t, fm[t][i]), acc[i][j], 0, 0, 0);
     };
 
-    // ---- pipeline (the host guarantees K % 32 == 0 and K / 32 >= AHEAD) ----
-    const int nc = p.K / 32;
+    // The last chunk's elements from k = K on are the next row's: zeros instead, in both operands (they may be NaN or Inf).
+    auto mask_tail = [&](int valid) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int d = 0; d < 4; ++d) {
+                const int left = valid - (t * 16 + h * 8 + d * 2);
+                const unsigned mask = left >= 2 ? 0xffffffffu : (left == 1 ? 0xffffu : 0u);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) fm[t][i][d] &= mask;
+#pragma unroll
+                for (int j = 0; j < 2; ++j) fn[t][j][d] &= mask;
+            }
+    };
+
+    // ---- pipeline (the host guarantees nc >= AHEAD) ----
+    const int nc = min(p.slice_chunks, (k_left + 31) / 32);
 #pragma unroll
     for (int c = 0; c < AHEAD; ++c) issue(c);
     WaitVmcnt<(AHEAD - 1) * LPC>();  // this wave's share of chunk 0 has landed
@@ -175,6 +215,9 @@ __global__ __launch_bounds__(512) void GemmPpKernel(GemmArgs p) {
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (ISSUE) issue(c + AHEAD);  // into the stage both groups finished reading a phase ago
         read_frags(c);
+        if constexpr (!ISSUE && WAIT == 0) {
+            if (c * 32 + 32 > k_left) mask_tail(k_left - c * 32);
+        }
         WaitVmcnt<WAIT>();  // chunk c + 1 (this wave's share) must have landed before the barrier behind which it is read
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_barrier();
@@ -194,27 +237,125 @@ __global__ __launch_bounds__(512) void GemmPpKernel(GemmArgs p) {
     });
     if (grp == 0) __builtin_amdgcn_s_barrier();
 
-    // ---- epilogue: lane holds m = r, n = 8 * (v / 4) + 4 * h + v % 4 of each 32 x 32 block ----
+    // ---- epilogue: lane holds m = r, n = 8 * (v / 4) + 4 * h + v % 4 of each 32 x 32 block.  DIRECT stores them as they are, 8 bytes each, and
+    // relies on the caches to put lines together; else the blocks pass through LDS (a piece per wave, free now), so that a row of 64 columns
+    // leaves in whole lines at any address.  That costs a tile about 1 us of latency and saves the traffic: [4480,650] . [650,10000] 100 -> 94 us,
+    // but [8192,128] . [128,8192], which has little else to do, 57 -> 61 ----
+    if constexpr (DIRECT) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int m = m0 + wm * 128 + i * 32 + r;
-        if (m >= p.M) continue;
-        half_t* const crow = p.c + static_cast<int64_t>(m) * p.ldc;
+        for (int i = 0; i < 4; ++i) {
+            const int m = m0 + wm * 128 + i * 32 + r;
+            if (m >= p.M) continue;
+            half_t* const crow = p.c + static_cast<int64_t>(m) * p.ldc;
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
+            for (int j = 0; j < 2; ++j) {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int n = n0 + wn * 64 + j * 32 + q * 8 + h * 4;
-                if (n >= p.N) continue;  // N % 4 == 0: a group of four is inside or outside
-                PVecH<4> o;
+                for (int q = 0; q < 4; ++q) {
+                    const int n = n0 + wn * 64 + j * 32 + q * 8 + h * 4;
+                    if (n >= p.N) continue;  // N % 4 == 0: a group of four is inside or outside
+                    PVecH<4> o;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    float v = acc[i][j][q * 4 + e];
-                    if (p.bias != nullptr) v += static_cast<float>(p.bias[(n + e) * p.bias_stride]);
-                    o.e[e] = static_cast<half_t>(v);
+                    for (int e = 0; e < 4; ++e) {
+                        float v = acc[i][j][q * 4 + e];
+                        if (p.bias != nullptr) v += static_cast<float>(p.bias[(n + e) * p.bias_stride]);
+                        o.e[e] = static_cast<half_t>(v);
+                    }
+                    *reinterpret_cast<PVecH<4>*>(crow + n) = o;
                 }
-                *reinterpret_cast<PVecH<4>*>(crow + n) = o;
             }
+        }
+        return;
+    }
+    char* const mine = lds + wave * 32 * kOutPitch;
+    float bias[2][16];
+    if (p.bias != nullptr && p.slices == 1) {  // one load for the wave's 64 columns, then to where the lanes need them
+        const int n = n0 + wn * 64 + lane;
+        const float v = n < p.N ? static_cast<float>(p.bias[n * p.bias_stride]) : 0.f;
+        __builtin_memcpy(mine + lane * 4, &v, 4);
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) __builtin_memcpy(&bias[j][q * 4], mine + (j * 32 + 8 * q + 4 * h) * 4, 16);
+        __builtin_amdgcn_wave_barrier();
+    }
+    auto store = [&](auto tag, auto* c, int64_t ld) {
+        using T = decltype(tag);
+        constexpr int E = 16 / static_cast<int>(sizeof(T)), LANES = 64 / E, ROWS = 64 / LANES;  // lanes of a row, rows of an instruction
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    T o[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        float v = acc[i][j][q * 4 + e];
+                        if constexpr (sizeof(T) == 2) {
+                            if (p.bias != nullptr) v += bias[j][q * 4 + e];
+                        }
+                        o[e] = static_cast<T>(v);
+                    }
+                    __builtin_memcpy(mine + r * kOutPitch + (j * 32 + q * 8 + h * 4) * sizeof(T), o, sizeof(o));
+                }
+            __builtin_amdgcn_wave_barrier();
+            const int n = n0 + wn * 64 + (lane % LANES) * E;
+#pragma unroll
+            for (int s = 0; s < 32 / ROWS; ++s) {
+                const int row = s * ROWS + lane / LANES;
+                const int m = m0 + wm * 128 + i * 32 + row;
+                OutPiece<T> o;
+                __builtin_memcpy(&o, mine + row * kOutPitch + (lane % LANES) * 16, 16);
+                if (m < p.M) {
+                    T* const to = c + static_cast<int64_t>(m) * ld + n;
+                    if (n + E <= p.N) {
+                        *reinterpret_cast<OutPiece<T>*>(to) = o;
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < E; ++e) {
+                            if (n + e < p.N) to[e] = o.e[e];
+                        }
+                    }
+                }
+            }
+            __builtin_amdgcn_wave_barrier();
+        }
+    };
+    if (p.slices > 1) store(float{}, p.partial + static_cast<int64_t>(slice) * p.M * p.N, p.N);
+    else store(half_t{}, p.c, p.ldc);
+}
+
+// c = the sum of the slices (from the first on), plus the bias, rounded once.  Bound by memory: 8 columns of a row per thread.
+__global__ __launch_bounds__(256) void GemmSumKernel(GemmArgs p) {
+    const int groups = (p.N + 7) / 8;
+    const int64_t g = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+    const int64_t m = g / groups;
+    const int n = static_cast<int>(g - m * groups) * 8;
+    if (m >= p.M) return;
+    const float* from = p.partial + m * p.N + n;
+    const int64_t slice = static_cast<int64_t>(p.M) * p.N;
+    half_t* const to = p.c + m * p.ldc + n;
+    if (n + 8 <= p.N) {
+        float sum[8] = {};
+        for (int s = 0; s < p.slices; ++s, from += slice) {
+            const OutPiece<float> lo = *reinterpret_cast<const OutPiece<float>*>(from), hi = *reinterpret_cast<const OutPiece<float>*>(from + 4);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sum[e] += lo.e[e], sum[4 + e] += hi.e[e];
+        }
+        OutPiece<half_t> o;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            if (p.bias != nullptr) sum[e] += static_cast<float>(p.bias[(n + e) * p.bias_stride]);
+            o.e[e] = static_cast<half_t>(sum[e]);
+        }
+        *reinterpret_cast<OutPiece<half_t>*>(to) = o;
+    } else {
+        for (int e = 0; n + e < p.N; ++e) {
+            float sum = 0.f;
+            for (int s = 0; s < p.slices; ++s) sum += from[s * slice + e];
+            if (p.bias != nullptr) sum += static_cast<float>(p.bias[(n + e) * p.bias_stride]);
+            to[e] = static_cast<half_t>(sum);
         }
     }
 }

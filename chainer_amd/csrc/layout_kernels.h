@@ -97,38 +97,61 @@ inline void LaunchToChannelsLast(const ToChannelsLastArgs& a, hipStream_t stream
     CheckLaunch("to_channels_last");
 }
 
-// dst[r][c] (dense, row pitch dst_pitch elements, columns c >= cols zero-filled up to dst_pitch) = src[r * sr + c * sc]:
+// dst[r][c] (dense, row pitch dst_pitch elements, a multiple of 16 bytes; columns c >= cols zero-filled up to dst_pitch) = src[r * sr + c * sc]:
 // brings a matrix operand whose reduction axis is not the unit-stride one into the layout the MFMA kernels read.
-// 64x64 tiles through LDS; reads walk the source's faster axis, writes walk dst rows.
+// Bound by memory.  A thread moves a block of E x E elements (E = 16 bytes' worth) by 16-byte accesses at any address and turns it
+// round in registers; 8 x 8 threads make a wave's block, so that reads and writes both cover whole 128-byte lines without a detour
+// through LDS.  [4480,10000] float16 transposed: 55 -> 40 us, against 64 x 64 tiles of single elements in LDS.
+enum StageRead { kStageColumns, kStageRows, kStageElements };  // src's unit-stride axis: c, r, neither
+
 template <typename T>
-__global__ __launch_bounds__(256) void StageMatrixKernel(const T* src, int64_t sr, int64_t sc, T* dst, int64_t dst_pitch, int rows, int cols,
-                                                         int read_rows_fast) {
-    constexpr int TILE = 64;
-    __shared__ T tile[TILE][TILE + 2];
-    const int r0 = blockIdx.y * TILE, c0 = blockIdx.x * TILE;
-    const int tid = threadIdx.x;
-    for (int e = tid; e < TILE * TILE; e += 256) {
-        // consecutive threads take consecutive rows when the source is contiguous along r, consecutive columns otherwise
-        const int rl = read_rows_fast ? e % TILE : e / TILE;
-        const int cl = read_rows_fast ? e / TILE : e % TILE;
-        const int r = r0 + rl, c = c0 + cl;
-        tile[rl][cl] = (r < rows && c < cols) ? src[r * sr + c * sc] : T(0);
+struct __attribute__((packed, aligned(1))) StagePiece {
+    T e[16 / sizeof(T)];
+};
+
+template <typename T, int READ>
+__global__ __launch_bounds__(256) void StageMatrixKernel(const T* src, int64_t sr, int64_t sc, T* dst, int64_t dst_pitch, int rows, int cols) {
+    constexpr int E = 16 / static_cast<int>(sizeof(T)), TILE = 8 * E;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int r0 = blockIdx.y * TILE + (lane & 7) * E;
+    const int64_t c0 = (static_cast<int64_t>(blockIdx.x) * 4 + wave) * TILE + (lane >> 3) * E;
+    if (r0 >= rows || c0 >= dst_pitch) return;
+    StagePiece<T> in[E], out[E];  // in: by column where the source's rows are the unit-stride axis
+    if (r0 + E <= rows && c0 + E <= cols && READ != kStageElements) {
+#pragma unroll
+        for (int i = 0; i < E; ++i) in[i] = *reinterpret_cast<const StagePiece<T>*>(READ == kStageRows ? src + r0 + (c0 + i) * sc : src + (r0 + i) * sr + c0);
+    } else {
+#pragma unroll
+        for (int i = 0; i < E; ++i)
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                const int r = r0 + (READ == kStageRows ? e : i);
+                const int64_t c = c0 + (READ == kStageRows ? i : e);
+                in[i].e[e] = r < rows && c < cols ? src[r * sr + c * sc] : T(0);
+            }
     }
-    __syncthreads();
-    for (int e = tid; e < TILE * TILE; e += 256) {
-        const int rl = e / TILE, cl = e % TILE;
-        const int r = r0 + rl, c = c0 + cl;
-        if (r < rows && c < dst_pitch) dst[r * dst_pitch + c] = tile[rl][cl];
+#pragma unroll
+    for (int i = 0; i < E; ++i)
+#pragma unroll
+        for (int e = 0; e < E; ++e) out[i].e[e] = READ == kStageRows ? in[e].e[i] : in[i].e[e];
+#pragma unroll
+    for (int i = 0; i < E; ++i) {
+        if (r0 + i < rows) *reinterpret_cast<StagePiece<T>*>(dst + (r0 + i) * dst_pitch + c0) = out[i];
     }
 }
 
 template <typename T>
 void StageMatrix(const T* src, int64_t sr, int64_t sc, T* dst, int64_t dst_pitch, int64_t rows, int64_t cols, hipStream_t stream) {
-    const int64_t asr = sr < 0 ? -sr : sr, asc = sc < 0 ? -sc : sc;
-    dim3 grid(static_cast<unsigned>((dst_pitch + 63) / 64), static_cast<unsigned>((rows + 63) / 64));
+    constexpr int TILE = 128 / static_cast<int>(sizeof(T));
+    dim3 grid(static_cast<unsigned>((dst_pitch + 4 * TILE - 1) / (4 * TILE)), static_cast<unsigned>((rows + TILE - 1) / TILE));
     HIPCX_REQUIRE(grid.y < 65536, HIPCX_NOT_IMPLEMENTED_ERROR, "matrix operand has too many rows to stage in one launch");
-    hipLaunchKernelGGL((StageMatrixKernel<T>), grid, dim3(256), 0, stream, src, sr, sc, dst, dst_pitch, static_cast<int>(rows),
-                       static_cast<int>(cols), asr < asc ? 1 : 0);
+    auto launch = [&](auto read) {
+        hipLaunchKernelGGL((StageMatrixKernel<T, decltype(read)::value>), grid, dim3(256), 0, stream, src, sr, sc, dst, dst_pitch, static_cast<int>(rows),
+                           static_cast<int>(cols));
+    };
+    if (sc == 1) launch(std::integral_constant<int, kStageColumns>{});
+    else if (sr == 1) launch(std::integral_constant<int, kStageRows>{});
+    else launch(std::integral_constant<int, kStageElements>{});
     CheckLaunch("stage_matrix");
 }
 
