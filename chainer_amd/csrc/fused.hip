@@ -5,6 +5,8 @@
 // Both evaluate the same float operations in the same order as the chain (Exp/Tanh/Log are the same device functions the
 // separate kernels call; no contraction), so for float32/float64 the Lstm cell is bit-identical to the chain and LogSoftmax
 // differs only through the order of the row sum.  float16 computes in float and rounds once.
+#include <algorithm>
+
 #include "common.h"
 
 namespace hipcx {
@@ -256,14 +258,15 @@ LsmShape CheckLogSoftmax(const hipcx_array* x, const hipcx_array* out) {
     HIPCX_REQUIRE((x->shape[1] <= 1 || (x->strides[1] == it && out->strides[1] == it)) && x->strides[0] % it == 0 && out->strides[0] % it == 0 &&
                           x->strides[0] >= 0 && out->strides[0] >= 0,
                   HIPCX_NOT_IMPLEMENTED_ERROR, "log_softmax: rows must be dense along axis 1");
-    HIPCX_REQUIRE(x->shape[0] < (1LL << 31) / 1024, HIPCX_NOT_IMPLEMENTED_ERROR, "log_softmax: too many rows for one launch");
     return LsmShape{x->shape[0], x->shape[1], x->strides[0] / it, out->strides[0] / it};
 }
 
+// Rows of one launch: a grid holds less than 2^32 threads, at most 256 of them (and two or more segments) to a row.  More rows than
+// these take several launches, each of them far longer than its start.
+constexpr int64_t kRowsPerLaunch = int64_t{1} << 21;
+
 template <typename T>
-void RunLogSoftmax(const hipcx_array* x, const hipcx_array* out, const LsmShape& sh, void* workspace, size_t workspace_bytes, hipStream_t stream) {
-    const T* xp = static_cast<const T*>(x->data);
-    T* op = static_cast<T*>(out->data);
+void RunLogSoftmax(const T* xp, T* op, const LsmShape& sh, void* workspace, size_t workspace_bytes, hipStream_t stream) {
     constexpr int V = 16 / sizeof(T);
     const int vec_ok = reinterpret_cast<uintptr_t>(xp) % 16 == 0 && reinterpret_cast<uintptr_t>(op) % 16 == 0 && sh.x_row % V == 0 && sh.o_row % V == 0;
     const int64_t packs = (sh.n + V - 1) / V;
@@ -487,7 +490,12 @@ int hipcx_log_softmax(const hipcx_array* x, const hipcx_array* out, void* worksp
         if (sh.rows == 0 || sh.n == 0) return;
         VisitFloatDtype(x->dtype, [&](auto tag) {
             using T = typename decltype(tag)::type;
-            RunLogSoftmax<T>(x, out, sh, workspace, workspace_bytes, AsStream(stream));
+            for (int64_t row = 0; row < sh.rows; row += kRowsPerLaunch) {
+                LsmShape part = sh;
+                part.rows = std::min(kRowsPerLaunch, sh.rows - row);
+                RunLogSoftmax<T>(static_cast<const T*>(x->data) + row * sh.x_row, static_cast<T*>(out->data) + row * sh.o_row, part, workspace,
+                                 workspace_bytes, AsStream(stream));
+            }
         });
     });
 }

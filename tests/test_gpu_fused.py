@@ -131,6 +131,19 @@ def test_log_softmax_fused_views_and_special_values():
                       chx.routines.current_stream())
 
 
+@pytest.mark.parametrize('cols', [2, 130])  # several rows to a wave, a wave per row
+def test_log_softmax_of_more_rows_than_a_launch_takes(cols):
+    """Per-pixel class scores: 32 images of 256 x 256 pixels are 2^21 rows."""
+    import chainer_amd as chx
+    period, repeats = 1031, 2035  # 2098085 rows
+    x = (np.random.default_rng(cols).standard_normal((period, cols)) * 3).astype('float16')
+    X = chx.array(x)[None].broadcast_to((repeats, period, cols)).copy().reshape((repeats * period, cols))
+    got = chx.log_softmax(X, 1)
+    ref = O.log_softmax(x, 1)
+    for lo, hi in ((0, 50), (2 ** 21 - 50, 2 ** 21 + 50), (repeats * period - 50, repeats * period)):
+        assert_close(got[lo:hi].get(), ref[np.arange(lo, hi) % period], None, 'log_softmax rows %d to %d' % (lo, hi))
+
+
 @pytest.mark.parametrize('dt', ['float32', 'float64', 'float16'])
 def test_lstm_cell_fused(dt):
     import chainer_amd as chx
