@@ -1098,7 +1098,8 @@ HOST_FN(TakeDeferred) {
 // ---------------------------------------------------------------------------------------------
 // fused, opt-in
 // ---------------------------------------------------------------------------------------------
-// LogSoftmax of a 2-D array along its unit-stride axis 1 through hipcx_log_softmax, or None for other calls.
+// LogSoftmax of a 2-D array along its unit-stride axis 1 through hipcx_log_softmax, or None for other calls: an axis without elements is
+// an error that the chain's AMax raises.
 HOST_FN(LogSoftmaxDirect) {
     HOST_TRY;
     HOST_ARGS("log_softmax", 1, "x", "axis");
@@ -1112,7 +1113,10 @@ HOST_FN(LogSoftmaxDirect) {
     }
     Ref x = Cast(x0, MathDtype(x0->d.dtype));
     const hipcx_array* d = x.d();
-    if (d->ndim != 2 || n != 1 || axes[0] != 1 || (d->shape[1] > 1 && d->strides[1] != ItemSize(d->dtype)) || d->strides[0] < 0) Py_RETURN_NONE;
+    if (d->ndim != 2 || n != 1 || axes[0] != 1 || d->shape[1] == 0 || (d->shape[1] > 1 && d->strides[1] != ItemSize(d->dtype)) ||
+        d->strides[0] < 0) {
+        Py_RETURN_NONE;
+    }
     Ref out = EmptyLike(x.arr(), d->dtype);
     Workspace ws(hipcx_log_softmax_workspace_size(d));
     void* stream = Stream();

@@ -682,7 +682,10 @@ def log_softmax(x, axis=None):
 
 
 def log_softmax_fused(x, axis=None):
-    """LogSoftmax through hipcx_log_softmax, which log_softmax takes by itself for every array the kernel covers."""
+    """log_softmax, which takes hipcx_log_softmax by itself for every array the kernel covers -- and, as the kernel does, an empty
+    result for rows without elements, where the routine raises AMax's DimensionError."""
+    if x.ndim == 2 and x.shape[1] == 0 and _sorted_axes(1 if axis is None else axis, 2) == (1,):
+        return ndarray.empty(x.shape, _math_result_dtype(x.dtype))
     return log_softmax(x, axis)
 
 

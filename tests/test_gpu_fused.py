@@ -131,6 +131,16 @@ def test_log_softmax_fused_views_and_special_values():
                       chx.routines.current_stream())
 
 
+def test_log_softmax_of_rows_without_elements():
+    """AMax along an axis of length 0 is a DimensionError (CX/routines/statistics.cc:21-65); no rows at all are an empty result."""
+    import chainer_amd as chx
+    for axis in (None, 1, -1):
+        with pytest.raises(chx.DimensionError, match='zero-sized'):
+            chx.log_softmax(chx.zeros((4, 0), 'float32'), axis)
+    assert chx.log_softmax(chx.zeros((0, 4), 'float32'), 1).shape == (0, 4)
+    assert chx.log_softmax_fused(chx.zeros((4, 0), 'float32')).shape == (4, 0)
+
+
 @pytest.mark.parametrize('cols', [2, 130])  # several rows to a wave, a wave per row
 def test_log_softmax_of_more_rows_than_a_launch_takes(cols):
     """Per-pixel class scores: 32 images of 256 x 256 pixels are 2^21 rows."""
