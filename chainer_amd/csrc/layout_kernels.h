@@ -143,11 +143,15 @@ __global__ __launch_bounds__(256) void StageMatrixKernel(const T* src, int64_t s
 template <typename T>
 void StageMatrix(const T* src, int64_t sr, int64_t sc, T* dst, int64_t dst_pitch, int64_t rows, int64_t cols, hipStream_t stream) {
     constexpr int TILE = 128 / static_cast<int>(sizeof(T));
-    dim3 grid(static_cast<unsigned>((dst_pitch + 4 * TILE - 1) / (4 * TILE)), static_cast<unsigned>((rows + TILE - 1) / TILE));
-    HIPCX_REQUIRE(grid.y < 65536, HIPCX_NOT_IMPLEMENTED_ERROR, "matrix operand has too many rows to stage in one launch");
+    // row tiles lie along the grid's y axis; more rows than it holds take several launches
+    constexpr int64_t kMaxRows = int64_t{65535} * TILE;
     auto launch = [&](auto read) {
-        hipLaunchKernelGGL((StageMatrixKernel<T, decltype(read)::value>), grid, dim3(256), 0, stream, src, sr, sc, dst, dst_pitch, static_cast<int>(rows),
-                           static_cast<int>(cols));
+        for (int64_t r0 = 0; r0 < rows; r0 += kMaxRows) {
+            const int64_t count = rows - r0 < kMaxRows ? rows - r0 : kMaxRows;
+            const dim3 grid(static_cast<unsigned>((dst_pitch + 4 * TILE - 1) / (4 * TILE)), static_cast<unsigned>((count + TILE - 1) / TILE));
+            hipLaunchKernelGGL((StageMatrixKernel<T, decltype(read)::value>), grid, dim3(256), 0, stream, src + r0 * sr, sr, sc, dst + r0 * dst_pitch,
+                               dst_pitch, static_cast<int>(count), static_cast<int>(cols));
+        }
     };
     if (sc == 1) launch(std::integral_constant<int, kStageColumns>{});
     else if (sr == 1) launch(std::integral_constant<int, kStageRows>{});

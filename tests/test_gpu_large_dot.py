@@ -41,3 +41,20 @@ def test_bias(m, k, n):
     expected = x.astype(np.float32) @ w.T.astype(np.float32) + bias
     got = chx.to_numpy(chx.linear(chx.array(x), chx.array(w), chx.array(bias)))
     np.testing.assert_allclose(got.astype(np.float32), expected, rtol=1e-3)
+
+
+@pytest.mark.parametrize('dt,rows', [('float32', 2500000), ('float16', 4300000)])  # 65535 tiles of rows are 2097120 and 4194240
+@pytest.mark.parametrize('layout', ['r', 'c'])
+def test_more_rows_to_lay_out_anew_than_a_launch_takes(dt, rows, layout):
+    period = 100
+    rng = np.random.default_rng(7)
+    x = rng.integers(-2, 3, (period, 65)).astype(dt)  # 65 columns: rows that the matrix kernels do not read as they are
+    w = rng.integers(-2, 3, (64, 65)).astype(dt)
+    X = chx.array(x)[None].broadcast_to((rows // period, period, 65)).copy().reshape((rows, 65))
+    if layout == 'c':
+        X = X.T.copy().T
+    got = chx.linear(X, chx.array(w))
+    expected = (x.astype(np.float32) @ w.T.astype(np.float32)).astype(dt)
+    cut = 65535 * 128 // x.itemsize
+    for lo, hi in ((0, 150), (cut // 2 - 75, cut // 2 + 75), (cut - 75, cut + 75), (rows - 150, rows)):
+        np.testing.assert_array_equal(got[lo:hi].get(), expected[np.arange(lo, hi) % period])
