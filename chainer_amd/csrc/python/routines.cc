@@ -1130,7 +1130,7 @@ HOST_FN(SoftmaxCrossEntropyDirect) {
     HOST_TRY;
     HOST_ARGS("softmax_cross_entropy", 2, "x", "t");
     Array *x0 = AsArray(arg[0], "x"), *t = AsArray(arg[1], "t");
-    static const int64_t kMax[10] = {0, 0, 127, 32767, INT32_MAX, INT64_MAX, 255, 0, 0, 0};  // of the integer dtypes
+    static const int64_t kMax[10] = {-1, -1, 127, 32767, INT32_MAX, INT64_MAX, 255, -1, -1, -1};  // the last class a label dtype can name
     if (x0->d.ndim != 2 || t->d.ndim != 1 || t->d.shape[0] != x0->d.shape[0] || x0->d.shape[0] == 0 || x0->d.shape[1] == 0 ||
         x0->d.shape[1] - 1 > kMax[t->d.dtype]) {
         Py_RETURN_NONE;

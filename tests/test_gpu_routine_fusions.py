@@ -38,6 +38,16 @@ def test_softmax_cross_entropy_label_dtypes(t_dtype):
         assert_close(chx.softmax_cross_entropy(chx.array(x), chx.array(t)).get().reshape(1), np.asarray(ref).reshape(1), what=t_dtype)
 
 
+@pytest.mark.parametrize('cols', [1, 2])
+def test_softmax_cross_entropy_float_labels(cols):
+    """The chain compares labels of any numeric dtype with Arange(n) of that dtype."""
+    import chainer_amd as chx
+    x = np.random.default_rng(6).standard_normal((20, cols)).astype('float32')
+    t = np.array([0, 1] * 10).astype('float32')
+    ref = O.softmax_cross_entropy(x, t)
+    assert_close(chx.softmax_cross_entropy(chx.array(x), chx.array(t)).get().reshape(1), np.asarray(ref).reshape(1), what='float labels')
+
+
 @pytest.mark.parametrize('dt', ['float16', 'float32', 'float64'])
 @pytest.mark.parametrize('cols', [1, 4, 16, 17, 64, 65, 128, 129])
 def test_log_softmax_short_rows(dt, cols):
