@@ -334,18 +334,21 @@ inline void LaunchEwVec(const EwPlan& p, const Op& op, hipStream_t stream, int64
     int64_t cols = nd > 0 ? p.shape[nd - 1] : 1;
     int64_t rows = nd > 0 ? p.total / cols : 1;
     const int64_t cvecs = (cols + VEC - 1) / VEC;
-    // a launch counts its vectors in 31 bits: larger problems are cut in two along their outermost axis
+    // a launch counts its vectors in 31 bits: larger problems are cut in two along their outermost axis (of more than one entry, which
+    // it may have been cut down to); along the inner axis, so that the second part starts as well aligned as the first
     if (rows * cvecs >= (int64_t{1} << 31) - kEwThreads * kEwUnroll) {
+        int d = 0;
+        while (p.shape[d] == 1) ++d;  // (the product of the extents is far from 1)
+        const int64_t first = d == nd - 1 ? p.shape[d] / 2 / VEC * VEC : p.shape[d] / 2;
+        const int64_t per_entry = p.total / p.shape[d];
         for (int half = 0; half < 2; ++half) {
             EwPlan q = p;
-            const int64_t first = p.shape[0] / 2 / VEC * VEC;
-            HIPCX_REQUIRE(first > 0, HIPCX_NOT_IMPLEMENTED_ERROR, "array too large for one launch");
-            q.shape[0] = half == 0 ? first : p.shape[0] - first;
-            q.total = p.total / p.shape[0] * q.shape[0];
+            q.shape[d] = half == 0 ? first : p.shape[d] - first;
+            q.total = per_entry * q.shape[d];
             if (half == 1) {
-                for (int i = 0; i < p.nops; ++i) q.ptr[i] += first * p.strides[i][0];
+                for (int i = 0; i < p.nops; ++i) q.ptr[i] += first * p.strides[i][d];
             }
-            LaunchEwVec<Op, VEC>(q, op, stream, index_base + (half == 1 ? p.total / p.shape[0] * first : 0));
+            LaunchEwVec<Op, VEC>(q, op, stream, index_base + (half == 1 ? per_entry * first : 0));
         }
         return;
     }

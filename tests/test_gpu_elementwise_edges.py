@@ -34,3 +34,22 @@ def test_odd_widths(dt, rows, cols):
         assert_exact(chx.relu(X).get(), np.maximum(x, 0).astype(dt), 'relu')
         assert_exact(X.astype('float32').get(), x.astype('float32'), 'cast')
         assert_exact(chx.where(chx.greater(X, B), X, 1).get(), np.where(x > b, x, np.array(1, dt)), 'bool condition')
+
+
+def test_more_elements_than_a_launch_counts():
+    """2^32 vectors in two rows that the operands walk apart: cut between the rows, then inside each."""
+    import torch
+    import chainer_amd as chx
+    cols = (1 << 35) + 5
+    if torch.cuda.mem_get_info()[0] < 3 * cols:
+        pytest.skip('needs %d bytes of device memory' % (3 * cols))
+    out = None
+    try:
+        out = chx.array(np.array([[3], [-7]], 'int8')).broadcast_to((2, cols)).copy()
+        for row, value in enumerate((3, -7)):
+            for lo in (0, cols // 4 - 500, cols // 2 - 500, 3 * (cols // 4) - 500, cols - 1000):
+                assert_exact(out[row, lo:lo + 1000].get(), np.full(1000, value, 'int8'), 'row %d from %d' % (row, lo))
+    finally:
+        del out
+        chx.synchronize()
+        chx.free_unused_blocks()
