@@ -48,9 +48,11 @@ def _require_device():
 
 
 def _start_device():
-    """Before the first allocation or stream look-up: checks for a device and initialises PyTorch's side of the runtime."""
+    """Before the first allocation or stream look-up: checks for a device, initialises PyTorch's side of the runtime and takes its
+    stream functions, which a build of PyTorch without device support does not have."""
     _require_device()
     torch().cuda.init()
+    _host.setup({'raw_stream': torch()._C._cuda_getCurrentRawStream, 'get_device': torch()._C._cuda_getDevice})
 
 
 def current_stream():
@@ -193,7 +195,6 @@ _host.setup({
     'dtypes': [None] + [dt for dt, _ in sorted(_DTYPE_CODES.items(), key=lambda item: item[1])],
     'np_dtype': numpy.dtype, 'np_bool': numpy.bool_, 'np_integer': numpy.integer, 'np_floating': numpy.floating,
     'require_device': _start_device,
-    'raw_stream': torch()._C._cuda_getCurrentRawStream, 'get_device': torch()._C._cuda_getDevice,
 })
 
 

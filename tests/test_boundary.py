@@ -11,6 +11,7 @@ import ctypes
 import os
 import re
 import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -230,6 +231,25 @@ def test_no_device_means_loud_failure():
         chx.array(np.zeros(3, np.float32))
     with pytest.raises(chx.BackendError):
         chx.zeros((3,), 'float32')
+
+
+def test_import_needs_no_device_build_of_torch():
+    """A PyTorch without device support has no stream functions: the package imports there and fails when it is used."""
+    code = """
+import torch
+torch.cuda.is_available = lambda: False
+for name in ('_cuda_getCurrentRawStream', '_cuda_getDevice'):
+    if hasattr(torch._C, name):
+        delattr(torch._C, name)
+import chainer_amd as chx
+try:
+    chx.zeros((2,), 'float32')
+except chx.BackendError as e:
+    print('refused:', e)
+"""
+    r = subprocess.run([sys.executable, '-c', code], capture_output=True, text=True, cwd=ROOT)
+    assert r.returncode == 0, r.stderr[-2000:]
+    assert 'refused: no HIP device' in r.stdout
 
 
 def test_bench_rejects_more_than_one_gpu():
