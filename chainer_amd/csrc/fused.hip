@@ -313,20 +313,30 @@ void RunLogSoftmax(const T* xp, T* op, const LsmShape& sh, void* workspace, size
 }
 
 // ---- softmax cross entropy ----
-// A group of LPR lanes walks a row twice (maximum; sum of exponentials), the second time out of L1 / L2; what a row contributes is the
-// score of its label.  The chain multiplies every score with a 0 / 1 mask, so a score of -inf elsewhere in the row turns the sum into
-// NaN (0 * inf): the smallest other score is kept to see that.  One workgroup does a small batch alone ([100, 10]: 15 launches of
-// 2.1-3.6 us, 41 us together -> one of 4 us); larger batches leave partial sums for XentFinishKernel.
+// What a row contributes is the score of its label, x[label] - (max + log(sum of exponentials)).  The chain multiplies every score
+// with a 0 / 1 mask, so a score of -inf elsewhere in the row turns the sum into NaN (0 * inf): the smallest other score is kept to see
+// that.  Every element is read once, 16 bytes per access at any address, and held in registers between the maximum and the sum.
+// Three shapes (PlanXent); us, against a wave to a row with one element per lane and step, twice over (and the chain of 15 kernels):
+//   XentKernel       short rows in the registers of 16 lanes or a wave.  One workgroup does a small batch alone; others leave partial
+//                    sums for XentFinishKernel.  Bound by the latency of a few loads and the exponentials behind them.  float32
+//                    [100,10] 4.5 -> 4.4 (53), [1000,10] 18 -> 6.0 (60), [900,18] 70 -> 6.1 (60), [128,1000] 10.4 -> 6.6 (60),
+//                    [20000,1500] 58 -> 38 (332).
+//   XentBlockKernel  longer rows, a workgroup to a row: bound by memory and, at few packs to a thread, by its three reductions.
+//                    [4480,10000] 121 -> 72 (482).  Rows too few to fill the chip are cut into segments, each a workgroup's, which
+//                    XentMergeKernel puts together in double: [128,10000] 51 -> 12 (65), [1,1000000] 3878 -> 11 (65).
 struct XentArgs {
     const void* x;
     const void* t;
     void* out;
-    double* partial;  // {sum of scores, number of labels} per workgroup, or null: one workgroup writes the result itself
+    double* partial;  // XentBlockKernel with segments: {maximum, sum, least other} of each; else {sum of scores, labels} per workgroup, or
+                      // null: one workgroup writes the result itself
     int64_t rows, n, x_row, t_stride;
     int t_dtype;
+    int nseg;         // segments of a row
+    int64_t seg_len;  // elements, a multiple of 16 bytes
 };
 
-__device__ __forceinline__ int64_t LoadLabel(const void* t, int64_t i, int dtype) {
+__device__ __forceinline__ int64_t LoadInteger(const void* t, int64_t i, int dtype) {
     switch (dtype) {
         case HIPCX_INT8: return static_cast<const int8_t*>(t)[i];
         case HIPCX_INT16: return static_cast<const int16_t*>(t)[i];
@@ -334,6 +344,12 @@ __device__ __forceinline__ int64_t LoadLabel(const void* t, int64_t i, int dtype
         case HIPCX_UINT8: return static_cast<const uint8_t*>(t)[i];
         default: return static_cast<const int64_t*>(t)[i];
     }
+}
+
+// The label of a row, -1 where it names no class.
+__device__ __forceinline__ int64_t LoadLabel(const XentArgs& p, int64_t row) {
+    const int64_t label = LoadInteger(p.t, row * p.t_stride, p.t_dtype);
+    return label >= 0 && label < p.n ? label : -1;
 }
 
 // -sum / count with the roundings of Sum, Sum, Divide(-1, .) and Multiply.
@@ -366,73 +382,280 @@ __device__ __forceinline__ void BlockSum2(double& a, double& b, double (*scratch
     }
 }
 
-constexpr int kXentThreads = 1024;
+template <typename T, int V>
+struct __attribute__((packed, aligned(sizeof(T)))) AnyPack {
+    T e[V];
+};
 
-template <typename T, int LPR>
-__global__ __launch_bounds__(kXentThreads) void XentKernel(XentArgs p) {
+// Elements [lo, end) of a row (end >= V), U packs of V to a lane, LANES lanes side by side.  The last pack moves back to end at `end`:
+// its first skip[u] elements are not this lane's (all V beyond the end).
+template <typename T, int V, int U, int LANES>
+struct XentShare {
     using C = compute_t<T>;
-    __shared__ double scratch[kXentThreads / 64][2];
+    C v[U][V];
+    int skip[U];
+
+    __device__ __forceinline__ void Load(const T* xr, int64_t lo, int64_t end, int lane) {
+        AnyPack<T, V> p[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int64_t first = lo + static_cast<int64_t>(u * LANES + lane) * V;
+            const int64_t from = first < end - V ? first : end - V;
+            skip[u] = static_cast<int>(first - from < V ? first - from : V);
+            p[u] = *reinterpret_cast<const AnyPack<T, V>*>(xr + from);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int j = 0; j < V; ++j) v[u][j] = static_cast<C>(p[u].e[j]);
+    }
+
+    // The maximum, and the least of the elements other than `label`.
+    __device__ __forceinline__ void Extremes(int64_t lo, int64_t end, int lane, int64_t label, C& m, C& least) const {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (u > 0 && lo + u * LANES * V >= end) break;  // (the same for all lanes)
+            const int64_t first = lo + static_cast<int64_t>(u * LANES + lane) * V;
+            const int64_t at = label - (first < end - V ? first : end - V);
+#pragma unroll
+            for (int j = 0; j < V; ++j) {
+                if (j < skip[u]) continue;
+                m = MaxNan(m, v[u][j]);
+                if (j != at && v[u][j] < least) least = v[u][j];
+            }
+        }
+    }
+
+    __device__ __forceinline__ C SumExp(int64_t lo, int64_t end, C m) const {
+        C s = 0;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (u > 0 && lo + u * LANES * V >= end) break;
+#pragma unroll
+            for (int j = 0; j < V; ++j) s += j >= skip[u] ? ExpOf<C>(v[u][j] - m) : C(0);
+        }
+        return s;
+    }
+};
+
+// Adds a row's contribution, with the roundings of LogSoftmax, Multiply and Sum.
+template <typename T>
+__device__ __forceinline__ void XentAddRow(const T* xr, int64_t n, int64_t label, compute_t<T> m, compute_t<T> s, compute_t<T> least, double& sum,
+                                           double& count) {
+    using C = compute_t<T>;
+    const C lse = m + LogOf<C>(s);
+    const bool counts = label >= 0;
+    C score = counts ? static_cast<C>(static_cast<T>(static_cast<C>(xr[label]) - lse)) : C(0);
+    if (n > (counts ? 1 : 0)) score += static_cast<C>(static_cast<T>(least - lse)) * C(0);
+    sum += static_cast<double>(score);
+    count += counts ? 1.0 : 0.0;
+}
+
+// The workgroup's {sum of scores, labels}, or the result itself.
+template <typename T, int NT>
+__device__ __forceinline__ void XentStore(const XentArgs& p, double sum, double count) {
+    __shared__ double scratch[NT / 64][2];
+    BlockSum2<NT>(sum, count, scratch);
+    if (threadIdx.x != 0) return;
+    if (p.partial != nullptr) {
+        p.partial[2 * blockIdx.x] = sum;
+        p.partial[2 * blockIdx.x + 1] = count;
+    } else {
+        *static_cast<T*>(p.out) = XentResult<T>(sum, count);
+    }
+}
+
+// E elements of a row to each of LPR lanes.
+template <typename T, int LPR, int E, int NT>
+__global__ __launch_bounds__(NT) void XentKernel(XentArgs p) {
+    using C = compute_t<T>;
+    constexpr int V = E * sizeof(T) < 16 ? E : 16 / sizeof(T), U = E / V;
     const int lane = threadIdx.x % LPR;
     double sum = 0, count = 0;
-    for (int64_t row = static_cast<int64_t>(blockIdx.x) * (kXentThreads / LPR) + threadIdx.x / LPR; row < p.rows;
-         row += static_cast<int64_t>(gridDim.x) * (kXentThreads / LPR)) {
+    for (int64_t row = static_cast<int64_t>(blockIdx.x) * (NT / LPR) + threadIdx.x / LPR; row < p.rows; row += static_cast<int64_t>(gridDim.x) * (NT / LPR)) {
         const T* xr = static_cast<const T*>(p.x) + row * p.x_row;
-        const int64_t label = LoadLabel(p.t, row * p.t_stride, p.t_dtype);
+        const int64_t label = LoadLabel(p, row);
+        XentShare<T, V, U, LPR> share;
+        share.Load(xr, 0, p.n, lane);
         C m = -INFINITY, least = INFINITY;
-        for (int64_t e = lane; e < p.n; e += LPR) {
-            const C v = static_cast<C>(xr[e]);
-            m = MaxNan(m, v);
-            if (e != label) least = v < least ? v : least;
-        }
+        share.Extremes(0, p.n, lane, label, m, least);
 #pragma unroll
         for (int d = LPR / 2; d >= 1; d >>= 1) {
             m = MaxNan(m, static_cast<C>(__shfl_xor(m, d, LPR)));
             const C o = static_cast<C>(__shfl_xor(least, d, LPR));
             least = o < least ? o : least;
         }
-        C s = 0;
-        for (int64_t e = lane; e < p.n; e += LPR) s += ExpOf<C>(static_cast<C>(xr[e]) - m);
+        C s = share.SumExp(0, p.n, m);
 #pragma unroll
         for (int d = LPR / 2; d >= 1; d >>= 1) s += static_cast<C>(__shfl_xor(s, d, LPR));
+        if (lane == 0) XentAddRow<T>(xr, p.n, label, m, s, least, sum, count);
+    }
+    XentStore<T, NT>(p, sum, count);
+}
+
+// s * exp(m - to) of a part of a row; a part of -inf alone has no terms (or the whole row has none, and the score becomes NaN).
+__device__ __forceinline__ double Rescaled(double s, double m, double to) { return m == -INFINITY ? 0.0 : s * exp(m - to); }
+
+constexpr int kXentThreads = 256;
+
+// U packs of a row to a thread at a time.
+template <typename T, int U>
+__global__ __launch_bounds__(kXentThreads) void XentBlockKernel(XentArgs p) {
+    using C = compute_t<T>;
+    constexpr int V = 16 / sizeof(T);
+    constexpr int64_t CHUNK = kXentThreads * U * V;
+    __shared__ C scratch[kXentThreads / 64];
+    double sum = 0, count = 0;
+    for (int64_t part = blockIdx.x; part < p.rows * p.nseg; part += gridDim.x) {
+        const int64_t row = part / p.nseg, lo = (part - row * p.nseg) * p.seg_len, hi = min(p.n, lo + p.seg_len);
+        const T* xr = static_cast<const T*>(p.x) + row * p.x_row;
+        const int64_t label = LoadLabel(p, row);
+        C m = -INFINITY, least = INFINITY;
+        double s = 0;  // of exp(x - m), so far
+        for (int64_t from = lo; from < hi; from += CHUNK) {
+            const int64_t end = min(hi, from + CHUNK);
+            XentShare<T, V, U, kXentThreads> share;
+            share.Load(xr, from, end, threadIdx.x);
+            C mc = -INFINITY;
+            share.Extremes(from, end, threadIdx.x, label, mc, least);
+            mc = BlockReduce<C, kXentThreads, true>(mc, scratch);
+            const C sc = BlockReduce<C, kXentThreads, false>(share.SumExp(from, end, mc), scratch);
+            const C both = MaxNan(m, mc);
+            s = hi - lo <= CHUNK && mc != static_cast<C>(-INFINITY) ? static_cast<double>(sc) : Rescaled(s, m, both) + Rescaled(sc, mc, both);
+            m = both;
+        }
+        least = -BlockReduce<C, kXentThreads, true>(-least, scratch);
+        if (threadIdx.x == 0) {
+            if (p.nseg > 1) {
+                p.partial[3 * part] = m;
+                p.partial[3 * part + 1] = s;
+                p.partial[3 * part + 2] = least;
+            } else {
+                XentAddRow<T>(xr, p.n, label, m, static_cast<C>(s), least, sum, count);
+            }
+        }
+    }
+    if (p.nseg == 1) XentStore<T, kXentThreads>(p, sum, count);
+}
+
+// The result of rows in segments: LPR lanes put a row together.
+template <typename T, int LPR>
+__global__ __launch_bounds__(1024) void XentMergeKernel(XentArgs p) {
+    using C = compute_t<T>;
+    const int lane = threadIdx.x % LPR;
+    double sum = 0, count = 0;
+    for (int64_t row = threadIdx.x / LPR; row < p.rows; row += 1024 / LPR) {
+        const double* part = p.partial + 3 * row * p.nseg;
+        double m = -INFINITY, least = INFINITY, s = 0;
+#pragma unroll 4
+        for (int i = lane; i < p.nseg; i += LPR) {
+            m = MaxNan(m, part[3 * i]);
+            least = part[3 * i + 2] < least ? part[3 * i + 2] : least;
+        }
+#pragma unroll
+        for (int d = LPR / 2; d >= 1; d >>= 1) {
+            m = MaxNan(m, __shfl_xor(m, d, LPR));
+            const double o = __shfl_xor(least, d, LPR);
+            least = o < least ? o : least;
+        }
+#pragma unroll 4
+        for (int i = lane; i < p.nseg; i += LPR) s += Rescaled(part[3 * i + 1], part[3 * i], m);
+#pragma unroll
+        for (int d = LPR / 2; d >= 1; d >>= 1) s += __shfl_xor(s, d, LPR);
         if (lane == 0) {
-            const C lse = m + LogOf<C>(s);
-            const bool counts = label >= 0 && label < p.n;
-            C score = counts ? static_cast<C>(static_cast<T>(static_cast<C>(xr[label]) - lse)) : C(0);
-            if (p.n > (counts ? 1 : 0)) score += static_cast<C>(static_cast<T>(least - lse)) * C(0);
-            sum += static_cast<double>(score);
-            count += counts ? 1.0 : 0.0;
+            XentAddRow<T>(static_cast<const T*>(p.x) + row * p.x_row, p.n, LoadLabel(p, row), static_cast<C>(m),
+                          static_cast<C>(s), static_cast<C>(least), sum, count);
         }
     }
-    BlockSum2<kXentThreads>(sum, count, scratch);
-    if (threadIdx.x == 0) {
-        if (p.partial != nullptr) {
-            p.partial[2 * blockIdx.x] = sum;
-            p.partial[2 * blockIdx.x + 1] = count;
-        } else {
-            *static_cast<T*>(p.out) = XentResult<T>(sum, count);
-        }
-    }
+    p.partial = nullptr;
+    XentStore<T, 1024>(p, sum, count);
 }
 
 template <typename T>
 __global__ __launch_bounds__(256) void XentFinishKernel(XentArgs p, int n_partial) {
-    __shared__ double scratch[4][2];
     double sum = 0, count = 0;
     for (int i = threadIdx.x; i < n_partial; i += 256) {
         sum += p.partial[2 * i];
         count += p.partial[2 * i + 1];
     }
-    BlockSum2<256>(sum, count, scratch);
-    if (threadIdx.x == 0) *static_cast<T*>(p.out) = XentResult<T>(sum, count);
+    p.partial = nullptr;
+    XentStore<T, 256>(p, sum, count);
 }
 
-// Workgroups for a batch: one while it is at most a few thousand elements (a second launch costs more than it saves), then one per
-// eight of its row slots, up to two to a compute unit.
-int XentBlocks(int64_t rows, int64_t n) {
-    if (rows * n <= 16384) return 1;
-    const int64_t lpr = n <= 16 ? 16 : 64;
-    const int64_t blocks = (rows * lpr + kXentThreads - 1) / kXentThreads;
-    return static_cast<int>(blocks < 512 ? blocks : 512);
+struct XentPlan {
+    int blocks = 1;
+    int nseg = 0;  // 0: XentKernel
+    int64_t seg_len = 0;
+    size_t Bytes() const { return nseg > 1 ? static_cast<size_t>(blocks) * 3 * sizeof(double) : blocks > 1 ? static_cast<size_t>(blocks) * 2 * sizeof(double) : 0; }
+};
+
+// Rows of at most 64 elements or 4 KB, 8 KB where there are four for every compute unit: XentKernel.  A row takes a group of lanes 1 us
+// and more, a second launch 2: the batch is one workgroup's alone while that means no more than two rows one after the other of 16 lanes
+// each, or one of 64 ([256,10] 6.9 us alone, 6.0 in two launches; [64,1000] 15 and 6.5).  Else a workgroup of four waves to every four
+// (16 short) rows, up to eight to a compute unit.
+// Longer rows: a workgroup each once there is one for every compute unit ([20000,1500] float32 would take 71 us so, 38 as waves), else
+// segments of 8 KB and more, up to four to a compute unit ([1,1000000] with 4 KB: 21 us, 11 with 8: the merge is one workgroup's).
+XentPlan PlanXent(int64_t rows, int64_t n, int64_t item) {
+    XentPlan pl;
+    if (n <= 64 || n * item <= (rows >= 4 * NumCUs() ? 8192 : 4096)) {
+        const int64_t lpr = n <= 64 ? 16 : 64;
+        if (rows * lpr > (n <= 64 ? 2048 : 1024)) pl.blocks = static_cast<int>(std::min<int64_t>((rows * lpr + 255) / 256, int64_t{8} * NumCUs()));
+        return pl;
+    }
+    if (rows >= NumCUs()) {
+        pl.nseg = 1;
+        pl.seg_len = n;
+        pl.blocks = static_cast<int>(std::min<int64_t>(rows, int64_t{8} * NumCUs()));
+        return pl;
+    }
+    const int64_t vec = 16 / item, most = (n * item + 8191) / 8192;
+    const int64_t segments = std::min<int64_t>((int64_t{4} * NumCUs() + rows - 1) / rows, most);
+    pl.seg_len = ((n + segments - 1) / segments + vec - 1) / vec * vec;
+    pl.nseg = static_cast<int>((n + pl.seg_len - 1) / pl.seg_len);
+    pl.blocks = static_cast<int>(rows) * pl.nseg;
+    return pl;
+}
+
+// f(E) for the least power of two E of at least n / lanes elements to a lane.
+template <int E, int MOST, typename F>
+void ForElementsPerLane(int64_t n, int lanes, F&& f) {
+    if constexpr (E < MOST) {
+        if (n > static_cast<int64_t>(E) * lanes) return ForElementsPerLane<2 * E, MOST>(n, lanes, f);
+    }
+    f(std::integral_constant<int, E>{});
+}
+
+template <typename T>
+void LaunchXent(const XentArgs& p, const XentPlan& plan, hipStream_t stream) {
+    constexpr int V = 16 / sizeof(T);
+    const dim3 grid(plan.blocks);
+    if (plan.nseg > 0) {
+        const int64_t packs = (p.seg_len + V - 1) / V;
+        if (packs <= 2 * kXentThreads) hipLaunchKernelGGL((XentBlockKernel<T, 2>), grid, dim3(kXentThreads), 0, stream, p);
+        else if (packs <= 4 * kXentThreads) hipLaunchKernelGGL((XentBlockKernel<T, 4>), grid, dim3(kXentThreads), 0, stream, p);
+        else hipLaunchKernelGGL((XentBlockKernel<T, 8>), grid, dim3(kXentThreads), 0, stream, p);
+    } else if (p.n <= 64) {
+        ForElementsPerLane<1, 4>(p.n, 16, [&](auto e) {
+            constexpr int E = decltype(e)::value;
+            if (plan.blocks == 1) hipLaunchKernelGGL((XentKernel<T, 16, E, 1024>), grid, dim3(1024), 0, stream, p);
+            else hipLaunchKernelGGL((XentKernel<T, 16, E, 256>), grid, dim3(256), 0, stream, p);
+        });
+    } else {
+        ForElementsPerLane<2, 8 * V>(p.n, 64, [&](auto e) {
+            constexpr int E = decltype(e)::value;
+            if (plan.blocks == 1) hipLaunchKernelGGL((XentKernel<T, 64, E, 1024>), grid, dim3(1024), 0, stream, p);
+            else hipLaunchKernelGGL((XentKernel<T, 64, E, 256>), grid, dim3(256), 0, stream, p);
+        });
+    }
+    CheckLaunch("softmax_cross_entropy");
+    if (plan.nseg > 1) {
+        if (plan.nseg <= 16) hipLaunchKernelGGL((XentMergeKernel<T, 16>), dim3(1), dim3(1024), 0, stream, p);
+        else hipLaunchKernelGGL((XentMergeKernel<T, 64>), dim3(1), dim3(1024), 0, stream, p);
+        CheckLaunch("softmax_cross_entropy_merge");
+    } else if (plan.blocks > 1) {
+        hipLaunchKernelGGL((XentFinishKernel<T>), dim3(1), dim3(256), 0, stream, p, plan.blocks);
+        CheckLaunch("softmax_cross_entropy_finish");
+    }
 }
 
 // ---- Lstm cell ----
@@ -501,9 +724,8 @@ int hipcx_log_softmax(const hipcx_array* x, const hipcx_array* out, void* worksp
 }
 
 size_t hipcx_softmax_cross_entropy_workspace_size(const hipcx_array* x) {
-    if (x == nullptr || x->ndim != 2) return 0;
-    const int blocks = XentBlocks(x->shape[0], x->shape[1]);
-    return blocks > 1 ? static_cast<size_t>(blocks) * 2 * sizeof(double) : 0;
+    if (x == nullptr || x->ndim != 2 || x->shape[0] == 0 || x->shape[1] == 0) return 0;
+    return PlanXent(x->shape[0], x->shape[1], ItemSize(x->dtype)).Bytes();
 }
 
 int hipcx_softmax_cross_entropy(const hipcx_array* x, const hipcx_array* t, const hipcx_array* out, void* workspace, size_t workspace_bytes,
@@ -528,26 +750,16 @@ int hipcx_softmax_cross_entropy(const hipcx_array* x, const hipcx_array* t, cons
         p.x_row = x->strides[0] / it;
         p.t_stride = t->strides[0] / ItemSize(t->dtype);
         p.t_dtype = t->dtype;
-        const int blocks = p.rows > 0 ? XentBlocks(p.rows, p.n) : 1;
-        if (blocks > 1) {
-            const size_t need = static_cast<size_t>(blocks) * 2 * sizeof(double);
-            HIPCX_REQUIRE(workspace != nullptr && workspace_bytes >= need, HIPCX_CHAINERX_ERROR,
-                          "softmax_cross_entropy: workspace of " + std::to_string(need) + " bytes required");
+        if (p.n == 0) p.rows = 0;  // nothing to read, no label counts
+        const XentPlan plan = p.rows > 0 ? PlanXent(p.rows, p.n, it) : XentPlan();
+        p.nseg = plan.nseg;
+        p.seg_len = plan.seg_len;
+        if (plan.Bytes() > 0) {
+            HIPCX_REQUIRE(workspace != nullptr && workspace_bytes >= plan.Bytes(), HIPCX_CHAINERX_ERROR,
+                          "softmax_cross_entropy: workspace of " + std::to_string(plan.Bytes()) + " bytes required");
             p.partial = static_cast<double*>(workspace);
         }
-        VisitFloatDtype(x->dtype, [&](auto tag) {
-            using T = typename decltype(tag)::type;
-            if (p.n <= 16) {
-                hipLaunchKernelGGL((XentKernel<T, 16>), dim3(blocks), dim3(kXentThreads), 0, AsStream(stream), p);
-            } else {
-                hipLaunchKernelGGL((XentKernel<T, 64>), dim3(blocks), dim3(kXentThreads), 0, AsStream(stream), p);
-            }
-            CheckLaunch("softmax_cross_entropy");
-            if (blocks > 1) {
-                hipLaunchKernelGGL((XentFinishKernel<T>), dim3(1), dim3(256), 0, AsStream(stream), p, blocks);
-                CheckLaunch("softmax_cross_entropy_finish");
-            }
-        });
+        VisitFloatDtype(x->dtype, [&](auto tag) { LaunchXent<typename decltype(tag)::type>(p, plan, AsStream(stream)); });
     });
 }
 

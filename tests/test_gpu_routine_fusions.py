@@ -27,6 +27,40 @@ def test_softmax_cross_entropy(dt, rows, cols):
         assert np.isnan(chx.softmax_cross_entropy(chx.array(x), chx.array(t)).get())
 
 
+@pytest.mark.parametrize('dt', ['float16', 'float32', 'float64'])
+@pytest.mark.parametrize('rows,cols', [(64, 100), (65, 100), (256, 16), (257, 16), (5, 511), (5, 513), (3, 1024), (3, 1025), (2, 2049), (70, 2051),
+                                       (1, 16385), (2, 40003), (255, 3000), (256, 3001), (258, 33001), (1, 700001),
+                                       (1030, 1025), (1030, 2047), (1030, 2049)])
+def test_softmax_cross_entropy_of_long_rows(dt, rows, cols):
+    """Rows in a wave's registers, in a workgroup's, in segments of several; rows that start anywhere, labels at their ends."""
+    import chainer_amd as chx
+    rng = np.random.default_rng(rows * 31 + cols)
+    wide = np.full((rows, cols + 3), np.nan, dt)
+    x = wide[:, 1:1 + cols]
+    x[...] = (3 * rng.standard_normal((rows, cols))).astype(dt)
+    t = rng.integers(0, cols, rows).astype('int64')
+    t[0], t[-1] = cols - 1, 0
+    if rows > 2:
+        t[1], t[2] = cols, -1  # name no class
+        x[2] += 5
+    x64 = x.astype(np.float64)
+    top = x64.max(1)
+    lse = top + np.log(np.exp(x64 - top[:, None]).sum(1))
+    named = (t >= 0) & (t < cols)
+    expected = (lse - x64[np.arange(rows), np.where(named, t, 0)])[named].mean()
+    X, t_dev = chx.array(wide)[:, 1:1 + cols], chx.array(t)
+    got = float(chx.softmax_cross_entropy(X, t_dev).get())
+    # float16: a score of about 10 keeps 10 bits, the sum and the number of labels (rounded as the chain rounds them) 10 each
+    assert abs(got - expected) <= {'float16': 4e-3, 'float32': 2e-6, 'float64': 1e-13}[dt] * expected, (got, expected)
+    for at, value in ((cols // 2, -np.inf), (cols - 2, np.nan), (1, np.inf)):
+        y = wide.copy()
+        y[-1, 1 + at] = value
+        assert np.isnan(float(chx.softmax_cross_entropy(chx.array(y)[:, 1:1 + cols], t_dev).get())), value
+    y = wide.copy()
+    y[0, 1:1 + cols] = -np.inf
+    assert np.isnan(float(chx.softmax_cross_entropy(chx.array(y)[:, 1:1 + cols], t_dev).get()))
+
+
 @pytest.mark.parametrize('t_dtype', ['int8', 'uint8', 'int64'])
 def test_softmax_cross_entropy_label_dtypes(t_dtype):
     import chainer_amd as chx
