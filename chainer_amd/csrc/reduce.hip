@@ -661,20 +661,15 @@ struct Row16 {
     In v[V];
 };
 
+// The node of a slice, of output t in the workgroup's threads t < CL * V (o0: this thread's first output).
 template <typename Impl, int V, int CL>
-__global__ __launch_bounds__(256) void ColumnChunkKernel(ReduceGeom g, int64_t nchunks, int nslices, int64_t inner, int64_t vecs_per_row, int64_t col_blocks,
-                                                         void* partials) {
+__device__ __forceinline__ typename Impl::Acc ColumnSliceNode(const ReduceGeom& g, int64_t slice, int64_t nchunks, int64_t o0,
+                                                              typename Impl::Acc (*nodes)[CL * V]) {
     using In = typename Impl::In;
     using Acc = typename Impl::Acc;
     constexpr int RL = 256 / CL;
     static_assert(CL * V <= 256, "one thread folds a column of nodes");
-    __shared__ Acc nodes[RL][CL * V];
     const int cl = threadIdx.x % CL, rl = threadIdx.x / CL;
-    const int64_t slice = blockIdx.x / col_blocks;
-    const int64_t unit = (blockIdx.x - slice * col_blocks) * CL + cl;  // V outputs of one row of the innermost kept axis
-    const int64_t outer = unit / vecs_per_row;
-    const int64_t c = (unit - outer * vecs_per_row) * V;
-    const int64_t o0 = outer * inner + (c + V <= inner ? c : inner - V);
     const int64_t chunk = slice * RL + rl;
     Acc acc[V];
 #pragma unroll
@@ -743,7 +738,7 @@ __global__ __launch_bounds__(256) void ColumnChunkKernel(ReduceGeom g, int64_t n
     for (int v = 0; v < V; ++v) nodes[rl][cl * V + v] = acc[v];
     __syncthreads();
     const int t = threadIdx.x;
-    if (t >= CL * V) return;
+    if (t >= CL * V) return Impl::Empty();
     Acc a[RL];
 #pragma unroll
     for (int r = 0; r < RL; ++r) a[r] = nodes[r][t];
@@ -755,6 +750,44 @@ __global__ __launch_bounds__(256) void ColumnChunkKernel(ReduceGeom g, int64_t n
             a[r] = a[r + s];
         }
     }
+    return a[0];
+}
+
+// RUNS: a workgroup takes an aligned run of 2^run_level slices, one after the other, and leaves the node of the run (the one that
+// ColumnFinishKernel would make of theirs): fewer partial results, where the memory for them is limited.  nslices counts runs then.
+template <typename Impl, int V, int CL, bool RUNS = false>
+__global__ __launch_bounds__(256) void ColumnChunkKernel(ReduceGeom g, int64_t nchunks, int nslices, int64_t inner, int64_t vecs_per_row, int64_t col_blocks,
+                                                         void* partials, int run_level) {
+    using Acc = typename Impl::Acc;
+    constexpr int RL = 256 / CL;
+    __shared__ Acc nodes[RL][CL * V];
+    const int64_t slice = blockIdx.x / col_blocks;
+    const int64_t unit = (blockIdx.x - slice * col_blocks) * CL + threadIdx.x % CL;  // V outputs of one row of the innermost kept axis
+    const int64_t outer = unit / vecs_per_row;
+    const int64_t c = (unit - outer * vecs_per_row) * V;
+    const int64_t o0 = outer * inner + (c + V <= inner ? c : inner - V);
+    Acc node;
+    if constexpr (RUNS) {
+        const int64_t first = slice << run_level, left = (nchunks + RL - 1) / RL - first;
+        const int64_t count = left < (int64_t{1} << run_level) ? left : int64_t{1} << run_level;
+        Acc tree[24];
+        for (int64_t s = 0; s < count; ++s) {
+            if (s > 0) __syncthreads();  // the nodes of the slice before are read
+            node = ColumnSliceNode<Impl, V, CL>(g, first + s, nchunks, o0, nodes);
+            int lvl = 0;
+            for (int64_t k = s; k & 1; k >>= 1, ++lvl) Impl::Reduce(tree[lvl], node);
+            tree[lvl] = node;
+        }
+        node = Impl::Empty();
+        int lvl = 0;
+        for (int64_t k = count; k > 0; k >>= 1, ++lvl) {
+            if (k & 1) Impl::Reduce(tree[lvl], node);
+        }
+    } else {
+        node = ColumnSliceNode<Impl, V, CL>(g, slice, nchunks, o0, nodes);
+    }
+    const int t = threadIdx.x;
+    if (t >= CL * V) return;
     const int64_t unit_t = (blockIdx.x - slice * col_blocks) * CL + t / V;
     const int64_t outer_t = unit_t / vecs_per_row;
     const int64_t c_t = (unit_t - outer_t * vecs_per_row) * V;
@@ -763,9 +796,9 @@ __global__ __launch_bounds__(256) void ColumnChunkKernel(ReduceGeom g, int64_t n
     if (nslices == 1) {
         int64_t in_off, out_off;
         OutOffsets(g, o, in_off, out_off);
-        *reinterpret_cast<typename Impl::Out*>(g.out + out_off) = Impl::MapOut(a[0]);
+        *reinterpret_cast<typename Impl::Out*>(g.out + out_off) = Impl::MapOut(node);
     } else {
-        static_cast<Acc*>(partials)[slice * g.n_out + o] = a[0];
+        static_cast<Acc*>(partials)[slice * g.n_out + o] = node;
     }
 }
 
@@ -828,6 +861,7 @@ struct ReducePlan {
     int col_lanes = 64;   // threads along the outputs: 16 or 64 (then 16 or 4 chunks of 32 elements to a workgroup)
     int64_t col_chunks = 0;
     int col_slices = 0;   // workgroups along the reduced axis
+    int col_run_level = -1;  // not negative: each takes an aligned run of 2^col_run_level slices (V = 1, 64 lanes)
     int64_t col_inner = 1, col_vecs_per_row = 1, col_blocks = 0;
 };
 
@@ -963,10 +997,27 @@ size_t WorkspaceBytes(const ReducePlan& pl) {
     return static_cast<size_t>(pl.g.n_out) * pl.blocks_per_row * pl.acc_size;
 }
 
-template <typename Impl>
+// A column plan whose partial results fit in `bytes`: longer runs of the reduced axis to a workgroup.  Only outputs by the hundred
+// thousand, or an axis of millions, need that; both still fill the chip.
+void FitColumnPlan(ReducePlan* pl, size_t bytes) {
+    if (!pl->column_path || WorkspaceBytes(*pl) <= bytes) return;
+    const int64_t slices = (pl->col_chunks + 3) / 4;
+    pl->col_vec = 1;
+    pl->col_lanes = 64;
+    pl->col_vecs_per_row = pl->col_inner;
+    pl->col_blocks = (pl->g.n_out + 63) / 64;
+    for (pl->col_run_level = 0;; ++pl->col_run_level) {
+        pl->col_slices = static_cast<int>(((slices - 1) >> pl->col_run_level) + 1);
+        if (WorkspaceBytes(*pl) <= bytes) return;  // (one slice needs none)
+    }
+}
+
+// FIT: what the workspace holds bounds the number of partial results, not the other way round.
+template <typename Impl, bool FIT = false>
 void Run(const hipcx_array* a, const int8_t* axis, int naxis, const hipcx_array* out, void* workspace, size_t workspace_bytes,
          hipStream_t stream) {
     ReducePlan pl = MakePlan(a, axis, naxis, out, sizeof(typename Impl::Acc));
+    if constexpr (FIT) FitColumnPlan(&pl, workspace_bytes);
     const ReduceGeom& g = pl.g;
     if (g.n_out == 0) return;
     if (pl.row_path) {
@@ -993,9 +1044,12 @@ void Run(const hipcx_array* a, const int8_t* axis, int naxis, const hipcx_array*
         const dim3 grid(static_cast<unsigned>(pl.col_blocks * pl.col_slices)), block(256);
         constexpr int VEC = 16 / sizeof(typename Impl::In) < 8 ? 16 / sizeof(typename Impl::In) : 8;
         auto launch = [&](auto kernel) {
-            hipLaunchKernelGGL(kernel, grid, block, 0, stream, g, pl.col_chunks, pl.col_slices, pl.col_inner, pl.col_vecs_per_row, pl.col_blocks, workspace);
+            hipLaunchKernelGGL(kernel, grid, block, 0, stream, g, pl.col_chunks, pl.col_slices, pl.col_inner, pl.col_vecs_per_row, pl.col_blocks, workspace,
+                               pl.col_run_level);
         };
-        if (pl.col_vec == 1) {
+        if (pl.col_run_level >= 0) {
+            if constexpr (FIT) launch(ColumnChunkKernel<Impl, 1, 64, true>);
+        } else if (pl.col_vec == 1) {
             launch(ColumnChunkKernel<Impl, 1, 64>);
         } else if (pl.col_lanes == 16) {
             launch(ColumnChunkKernel<Impl, VEC, 16>);
@@ -1062,6 +1116,30 @@ StaticScratchSlot& StaticScratchOfCurrentDevice() {
     return slot;
 }
 
+template <bool FIT>
+int SumInto(const hipcx_array* a, const int8_t* axis, int naxis, const hipcx_array* out, void* workspace, size_t workspace_bytes, void* stream) {
+    return Guard([&] {
+        ValidateArray(a, "a");
+        ValidateArray(out, "out");
+        hipStream_t st = AsStream(stream);
+        const int in = a->dtype, od = out->dtype;
+        // Out dtypes the routines produce: the input's float dtype, int64 for bool/int/uint inputs,
+        // float32/float64 for Mean of integers (CX/routines/reduction.cc:34-49, statistics.cc:111-116).
+        auto for_out = [&](auto in_tag) {
+            using In = typename decltype(in_tag)::type;
+            switch (od) {
+                case HIPCX_INT64: Run<SumImpl<In, int64_t>, FIT>(a, axis, naxis, out, workspace, workspace_bytes, st); break;
+                case HIPCX_FLOAT16: Run<SumImpl<In, half_t>, FIT>(a, axis, naxis, out, workspace, workspace_bytes, st); break;
+                case HIPCX_FLOAT32: Run<SumImpl<In, float>, FIT>(a, axis, naxis, out, workspace, workspace_bytes, st); break;
+                case HIPCX_FLOAT64: Run<SumImpl<In, double>, FIT>(a, axis, naxis, out, workspace, workspace_bytes, st); break;
+                default:
+                    throw Error(HIPCX_NOT_IMPLEMENTED_ERROR, std::string("hip sum: unsupported output dtype ") + DtypeName(od));
+            }
+        };
+        VisitDtype(in, for_out);
+    });
+}
+
 }  // namespace
 }  // namespace hipcx
 
@@ -1082,37 +1160,21 @@ size_t hipcx_reduce_workspace_size(const hipcx_array* a, const int8_t* axis, int
 
 int hipcx_sum(const hipcx_array* a, const int8_t* axis, int naxis, const hipcx_array* out, void* workspace, size_t workspace_bytes,
               void* stream) {
-    return Guard([&] {
-        ValidateArray(a, "a");
-        ValidateArray(out, "out");
-        hipStream_t st = AsStream(stream);
-        const int in = a->dtype, od = out->dtype;
-        // Out dtypes the routines produce: the input's float dtype, int64 for bool/int/uint inputs,
-        // float32/float64 for Mean of integers (CX/routines/reduction.cc:34-49, statistics.cc:111-116).
-        auto for_out = [&](auto in_tag) {
-            using In = typename decltype(in_tag)::type;
-            switch (od) {
-                case HIPCX_INT64: Run<SumImpl<In, int64_t>>(a, axis, naxis, out, workspace, workspace_bytes, st); break;
-                case HIPCX_FLOAT16: Run<SumImpl<In, half_t>>(a, axis, naxis, out, workspace, workspace_bytes, st); break;
-                case HIPCX_FLOAT32: Run<SumImpl<In, float>>(a, axis, naxis, out, workspace, workspace_bytes, st); break;
-                case HIPCX_FLOAT64: Run<SumImpl<In, double>>(a, axis, naxis, out, workspace, workspace_bytes, st); break;
-                default:
-                    throw Error(HIPCX_NOT_IMPLEMENTED_ERROR, std::string("hip sum: unsupported output dtype ") + DtypeName(od));
-            }
-        };
-        VisitDtype(in, for_out);
-    });
+    return SumInto<false>(a, axis, naxis, out, workspace, workspace_bytes, stream);
 }
 
 // hipcx_sum for callers that can neither allocate a workspace nor have one allocated for them: the per-block / per-slice
-// partial results go to the library's own static device array.  Same kernels and launch plan as hipcx_sum, hence the same bits.
+// partial results go to the library's own static device array.  Same kernels as hipcx_sum and the same tree of sums, hence the same
+// bits; the launch plan differs where a strided axis has more partial results than the array holds (FitColumnPlan).
 // Every partial is written before it is read, so nothing has to be cleared between calls; calls from different streams or host
 // threads on one device share the array and are chained through an event (see StaticScratchSlot) -- except under stream capture.
 int hipcx_sum_static_scratch(const hipcx_array* a, const int8_t* axis, int naxis, const hipcx_array* out, void* stream) {
     int status = Guard([&] {
         ValidateArray(a, "a");
         ValidateArray(out, "out");
-        const size_t need = hipcx_reduce_workspace_size(a, axis, naxis, out);
+        ReducePlan pl = MakePlan(a, axis, naxis, out, 16);
+        FitColumnPlan(&pl, HIPCX_STATIC_SCRATCH_BYTES);
+        const size_t need = WorkspaceBytes(pl);
         HIPCX_REQUIRE(need <= HIPCX_STATIC_SCRATCH_BYTES, HIPCX_CHAINERX_ERROR,
                       "sum_static_scratch: this reduction needs " + std::to_string(need) + " bytes of partial results, the static scratch holds " +
                               std::to_string(static_cast<size_t>(HIPCX_STATIC_SCRATCH_BYTES)) + "; use hipcx_sum with a workspace");
@@ -1133,7 +1195,7 @@ int hipcx_sum_static_scratch(const hipcx_array* a, const int8_t* axis, int naxis
         status = Guard([&] { HIPCX_CHECK_HIP(hipStreamWaitEvent(s, slot->done, 0)); });
         if (status != HIPCX_OK) return status;
     }
-    status = hipcx_sum(a, axis, naxis, out, slot->address, HIPCX_STATIC_SCRATCH_BYTES, stream);
+    status = SumInto<true>(a, axis, naxis, out, slot->address, HIPCX_STATIC_SCRATCH_BYTES, stream);
     if (chained) {
         int recorded = Guard([&] { HIPCX_CHECK_HIP(hipEventRecord(slot->done, s)); });
         if (recorded == HIPCX_OK) {

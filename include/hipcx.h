@@ -281,8 +281,9 @@ int hipcx_any(const hipcx_array* a, const int8_t* axis, int naxis, const hipcx_a
 /* hipcx_sum without a workspace argument.  No counterpart in the reference: it is for callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc) and so cannot provide the workspace
  * hipcx_sum asks for.  The partial results live in a static device array of HIPCX_STATIC_SCRATCH_BYTES inside the library (one
- * copy per device, held until the process ends); the call allocates and frees nothing.  Reductions whose
- * hipcx_reduce_workspace_size exceeds that are refused with HIPCX_CHAINERX_ERROR.  Results are bit-identical to hipcx_sum's.
+ * copy per device, held until the process ends); the call allocates and frees nothing.  Sums over a strided axis are cut into as
+ * many parts as have room there; sums over dense rows whose hipcx_reduce_workspace_size exceeds it are refused with
+ * HIPCX_CHAINERX_ERROR.  Results are bit-identical to hipcx_sum's.
  * Calls that overlap on one device share the array and race: issue them on one stream, or serialise them. */
 #define HIPCX_STATIC_SCRATCH_BYTES (4u << 20)
 int hipcx_sum_static_scratch(const hipcx_array* a, const int8_t* axis, int naxis, const hipcx_array* out, void* stream);

@@ -40,6 +40,32 @@ def test_static_scratch_sum_matches_workspace_sum_on_consecutive_calls():
     assert needs[2] > 0 and needs[3] > 0, needs
 
 
+@pytest.mark.parametrize('rows,cols,dt,step', [(546, 219264, 'float32', 1), (1111, 300001, 'float16', 1), (1024, 140000, 'int8', 2),
+                                               (2051, 70001, 'float64', 2), (40000002, 2, 'float32', 2), (3000001, 700, 'int8', 7)])
+def test_static_scratch_sum_over_a_strided_axis_takes_any_size(rows, cols, dt, step):
+    """More partial results than the static array holds: by many outputs, by a long axis; outputs side by side in memory and apart."""
+    import chainer_amd as chx
+    rng = np.random.default_rng(79)
+    period = 1001
+    x = rng.integers(-50, 50, (period, cols)).astype(dt) if dt == 'int8' else rng.standard_normal((period, cols)).astype(dt)
+    whole = rows // period
+    X = chx.array(x)
+    if whole > 1:
+        X = X[None].broadcast_to((whole, period, cols)).copy().reshape((whole * period, cols))
+    X = chx.concatenate([X[:min(rows, whole * period)], X[:rows - whole * period]], 0)
+    assert X.shape == (rows, cols)
+    X = X[:, ::step]
+    ref = chx.sum(X, axis=0)
+    out = chx.ndarray.empty(ref.shape, ref.dtype)
+    out.fill(0)
+    from chainer_amd import _lib
+    from chainer_amd._array import current_stream
+    ax = (ctypes.c_int8 * 1)(0)
+    assert _lib.load().hipcx_reduce_workspace_size(X.desc(), ax, 1, out.desc()) > (4 << 20)
+    _lib.call('hipcx_sum_static_scratch', X.desc(), ax, 1, out.desc(), current_stream())
+    assert_exact(out.get(), ref.get(), 'sum_static_scratch')
+
+
 def test_static_scratch_sum_refuses_reductions_beyond_its_size():
     import chainer_amd as chx
     from chainer_amd import _lib
