@@ -70,13 +70,11 @@ def test_static_scratch_sum_refuses_reductions_beyond_its_size():
     import chainer_amd as chx
     from chainer_amd import _lib
     from chainer_amd._array import current_stream
-    # many outputs x many slices of a long strided axis: more partial results than the static array holds
-    X = chx.zeros((4096, 16384), 'float64')
-    out = chx.ndarray.empty((16384,), 'float64')
-    ax = (ctypes.c_int8 * 1)(0)
-    need = _lib.load().hipcx_reduce_workspace_size(X.desc(), ax, 1, out.desc())
-    if need <= (4 << 20):
-        pytest.skip('this launch plan fits the static scratch (%d bytes)' % need)
+    # many dense rows, each of them several workgroups' work: more partial results than the static array holds
+    X = chx.zeros((1, 131072), 'int8').broadcast_to((200000, 131072))
+    out = chx.ndarray.empty((200000,), 'int64')
+    ax = (ctypes.c_int8 * 1)(1)
+    assert _lib.load().hipcx_reduce_workspace_size(X.desc(), ax, 1, out.desc()) > (4 << 20)
     with pytest.raises(chx.ChainerxError, match='static scratch'):
         _lib.call('hipcx_sum_static_scratch', X.desc(), ax, 1, out.desc(), current_stream())
 
