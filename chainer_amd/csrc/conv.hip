@@ -307,18 +307,42 @@ void LaunchSmallDot(SmallDotArgs p, int a_mode, int b_mode, int batch, hipStream
     if constexpr (sizeof(T) == 2) with_a(std::integral_constant<int, kOddPieces>{});
 }
 
+// Which kernel of small_dot.h takes a product.
+enum SmallDotPath { kNoSmallDot, kSmallDotVector, kSmallDotLines, kSmallDotTiles };
+
+template <typename T>
+SmallDotPath PlanSmallDot(const hipcx_array* a, const hipcx_array* b, SmallDotArgs* p, int* a_mode, int* b_mode) {
+    static const bool enabled = [] { const char* e = getenv("HIPCX_SMALL_DOT"); return e == nullptr || e[0] != '0'; }();
+    static const bool rows_ok = [] { const char* e = getenv("HIPCX_SMALL_DOT_ROWS"); return e == nullptr || e[0] != '0'; }();
+    const int64_t M = a->shape[0], K = a->shape[1], N = b->shape[1];
+    if (!enabled || !SmallDotShape(M, N, K) || !SmallDotOperands<T>(a, b, p, a_mode, b_mode)) return kNoSmallDot;
+    if (*a_mode != kPieces || *b_mode != kPieces) return kSmallDotTiles;
+    if (M <= 4) return kSmallDotVector;
+    // whole-line loads regrouped through LDS pay off once the product is large enough to be bandwidth-bound (measured: the
+    // 10000-column projection of the language model gains 15 %, the 2600- and 1000-column layers lose 10 %)
+    return rows_ok && 2.0 * M * N * K >= 1e9 ? kSmallDotLines : kSmallDotTiles;
+}
+
+// Bytes of partial sums for a small product: only tiles are split along the reduction.
+size_t SmallDotWorkspace(const hipcx_array* a, const hipcx_array* b, int dtype) {
+    if (dtype != HIPCX_FLOAT16 && dtype != HIPCX_FLOAT32) return 0;
+    SmallDotArgs p{};
+    int a_mode = 0, b_mode = 0;
+    const SmallDotPath path = dtype == HIPCX_FLOAT16 ? PlanSmallDot<half_t>(a, b, &p, &a_mode, &b_mode) : PlanSmallDot<float>(a, b, &p, &a_mode, &b_mode);
+    return path == kSmallDotTiles ? SmallDotPartialBytes(a->shape[0], b->shape[1], a->shape[1], dtype) : 0;
+}
+
 // Small-output matrix products (small_dot.h).  Returns false when the problem does not qualify.  `partial` holds
 // SmallDotPartialBytes bytes; without it the reduction is not split.
 template <typename T>
 bool TrySmallDot(const hipcx_array* a, const hipcx_array* b, const hipcx_array* bias, const hipcx_array* out, float* partial, hipStream_t stream) {
-    static const bool enabled = [] { const char* e = getenv("HIPCX_SMALL_DOT"); return e == nullptr || e[0] != '0'; }();
     const int64_t M = a->shape[0], K = a->shape[1], N = b->shape[1];
     const int64_t it = sizeof(T);
-    if (!enabled || !SmallDotShape(M, N, K)) return false;
     if (out->strides[0] < 0 || out->strides[1] < 0 || out->strides[0] % it || out->strides[1] % it) return false;
     SmallDotArgs p{};
     int a_mode = 0, b_mode = 0;
-    if (!SmallDotOperands<T>(a, b, &p, &a_mode, &b_mode)) return false;
+    const SmallDotPath path = PlanSmallDot<T>(a, b, &p, &a_mode, &b_mode);
+    if (path == kNoSmallDot) return false;
     p.out = out->data;
     p.o_row = out->strides[0] / it;
     p.o_col = out->strides[1] / it;
@@ -327,7 +351,7 @@ bool TrySmallDot(const hipcx_array* a, const hipcx_array* b, const hipcx_array* 
         p.bias_stride = bias->strides[0] / it;
     }
     ProfileScope prof(stream, 2.0 * M * N * K, static_cast<double>(it) * (M * K + K * N + M * N));
-    if (M <= 4 && a_mode == kPieces && b_mode == kPieces) {
+    if (path == kSmallDotVector) {
         const dim3 grid(static_cast<unsigned>((N + 3) / 4));
         if (M == 1) hipLaunchKernelGGL((SmallDotVectorKernel<T, 1>), grid, dim3(256), 0, stream, p);
         else if (M == 2) hipLaunchKernelGGL((SmallDotVectorKernel<T, 2>), grid, dim3(256), 0, stream, p);
@@ -335,10 +359,7 @@ bool TrySmallDot(const hipcx_array* a, const hipcx_array* b, const hipcx_array* 
         CheckLaunch("small_dot_vector");
         return true;
     }
-    static const bool rows_ok = [] { const char* e = getenv("HIPCX_SMALL_DOT_ROWS"); return e == nullptr || e[0] != '0'; }();
-    // whole-line loads regrouped through LDS pay off once the product is large enough to be bandwidth-bound (measured: the
-    // 10000-column projection of the language model gains 15 %, the 2600- and 1000-column layers lose 10 %)
-    if (rows_ok && a_mode == kPieces && b_mode == kPieces && 2.0 * M * N * K >= 1e9) {
+    if (path == kSmallDotLines) {
         // Waves per workgroup = ways K is split: the choice that leaves the busiest SIMD the least matrix work
         // (wave-tiles are dealt over 4 SIMDs per CU; a wave's share is whole 128-byte steps).
         const int64_t blocks = static_cast<int64_t>(p.tiles_m) * p.tiles_n, steps = (K * it + 127) / 128;
@@ -1781,8 +1802,8 @@ static int DotBias(const hipcx_array* a, const hipcx_array* b, const hipcx_array
         }
         // the same piece of the workspace serves a small product's partial sums
         float* small_partial = nullptr;
-        if (slices == 1 && staged_bytes == 0 && out->dtype != HIPCX_FLOAT64 && SmallDotShape(m, n, k)) {
-            const size_t need = SmallDotPartialBytes(m, n, k, out->dtype);
+        if (slices == 1 && staged_bytes == 0) {
+            const size_t need = SmallDotWorkspace(a, b, out->dtype);
             if (need > 0 && workspace != nullptr && workspace_bytes >= need && reinterpret_cast<uintptr_t>(workspace) % 16 == 0) {
                 small_partial = static_cast<float*>(workspace);
             }
@@ -1819,7 +1840,7 @@ size_t hipcx_dot_workspace_size(const hipcx_array* a, const hipcx_array* b, cons
         if (a != nullptr && b != nullptr && out != nullptr && a->ndim == 2 && b->ndim == 2 && a->shape[1] > 0 && a->shape[0] > 0 && b->shape[1] > 0) {
             const int64_t m = a->shape[0], n = b->shape[1], k = a->shape[1];
             split = SplitKBytes(m, n, PlanSplitK(m, n, k, out->dtype));
-            if (split == 0 && out->dtype != HIPCX_FLOAT64 && SmallDotShape(m, n, k)) split = SmallDotPartialBytes(m, n, k, out->dtype);
+            if (split == 0 && a->dtype == out->dtype && b->dtype == out->dtype) split = SmallDotWorkspace(a, b, out->dtype);
         }
         const size_t need = RoundUpTo(st.a_bytes + st.b_bytes, 256) + split;
         const GemmPpPlan pp = PlanGemmPp(a, b, out);

@@ -99,6 +99,25 @@ def test_conv_out_dim_entry_point():
     assert lib.hipcx_conv_out_dim(112, 3, 2, 0, 1) == 56 and lib.hipcx_conv_out_dim(112, 3, 2, 0, 0) == 55
 
 
+def test_dot_workspace_is_asked_for_by_the_kernels_that_split():
+    """Partial sums of small products belong to the tiles that split the reduction: not to the kernel of at most four rows, nor to the one
+    that reads whole lines."""
+    from chainer_amd import _lib
+    lib = _lib.load()
+
+    def array(shape, strides):
+        return _lib.CArray(0x10000, 8, 2, (ctypes.c_int64 * 10)(*shape), (ctypes.c_int64 * 10)(*strides))  # float32, never read
+
+    def need(m, k, n, b_dense):
+        a, out = array((m, k), (4 * k, 4)), array((m, n), (4 * n, 4))
+        b = array((k, n), (4, 4 * k) if b_dense else (4 * n, 4))
+        return lib.hipcx_dot_workspace_size(ctypes.byref(a), ctypes.byref(b), ctypes.byref(out))
+
+    assert need(1, 8192, 1000, True) == 0 and need(4, 8192, 1000, True) == 0
+    assert need(128, 4000, 1000, True) == 0  # 1.02 GFLOP
+    assert need(20, 8192, 1000, True) > 0 and need(1, 8192, 1000, False) > 0
+
+
 def test_oracle_library_loads():
     from oracle import native
     L = native.lib()
