@@ -37,9 +37,9 @@ struct SmallDotArgs {
     int nw;               // waves per workgroup = ways a workgroup's share of the reduction is split (SmallDotKernel: 8)
     int ksplit;           // workgroups per tile along the reduction (not SmallDotRowsKernel)
     float* partial;       // not null: [ksplit][M][N] sums go there instead of to out
-    // blockIdx.y: products that share their shapes and strides, a and b at constant distances (elements), outputs anywhere
-    // (not SmallDotRowsKernel)
-    int64_t a_batch, b_batch;
+    // blockIdx.y: products of one b that share their shapes and strides, left operands at a constant distance (elements), outputs
+    // anywhere (not SmallDotRowsKernel)
+    int64_t a_batch;
     void* outs[kSmallDotMaxBatch];
 };
 
@@ -130,7 +130,7 @@ __global__ __launch_bounds__(512) void SmallDotKernel(SmallDotArgs p) {
     const int n = tn * 32 + lr;
     const int batch = blockIdx.y;
     const __amdgpu_buffer_rsrc_t ar = MakeRsrc(static_cast<const T*>(p.a) + batch * p.a_batch, p.a_bytes);
-    const __amdgpu_buffer_rsrc_t br = MakeRsrc(static_cast<const T*>(p.b) + batch * p.b_batch, p.b_bytes);
+    const __amdgpu_buffer_rsrc_t br = MakeRsrc(p.b, p.b_bytes);
     const bool m_ok = m < p.M, n_ok = n < p.N;
     const int64_t a_off = static_cast<int64_t>(m) * p.a_row;
     const int64_t b_off = static_cast<int64_t>(n) * p.b_col;
@@ -395,7 +395,7 @@ __global__ __launch_bounds__(64 * kSmallDotMaxWaves) __attribute__((amdgpu_waves
     SmallDotTile(tiles, blockIdx.x - split * tiles, p.tiles_m, tm, tn);
     const int batch = blockIdx.y;
     const __amdgpu_buffer_rsrc_t ar = MakeRsrc(static_cast<const T*>(p.a) + batch * p.a_batch, p.a_bytes);
-    const __amdgpu_buffer_rsrc_t br = MakeRsrc(static_cast<const T*>(p.b) + batch * p.b_batch, p.b_bytes);
+    const __amdgpu_buffer_rsrc_t br = MakeRsrc(p.b, p.b_bytes);
     const int a_ks = static_cast<int>(p.a_k * sizeof(T)), b_ks = static_cast<int>(p.b_k * sizeof(T));
     // rows this lane reads: in the MFMA layout its own (lr), as whole lines every eighth one
     auto line_of = [](int row, int rows, int64_t stride) { return row < rows ? static_cast<int>(row * stride * static_cast<int64_t>(sizeof(T))) : -1; };
