@@ -10,7 +10,9 @@
 
 #include <cstdint>
 #include <cstring>
+#include <exception>
 #include <initializer_list>
+#include <new>
 
 #include "hipcx.h"
 
@@ -86,13 +88,22 @@ private:
     PyObject* p_ = nullptr;
 };
 
-// Thrown when a Python exception is set; every function called by the interpreter ends in CATCH.
+// Thrown when a Python exception is set; every function called by the interpreter ends in CATCH.  Nothing of C++ leaves one: the
+// standard containers' exceptions become Python's.
 struct PyError {};
 #define HOST_TRY try {
-#define HOST_CATCH(value)          \
-    }                              \
-    catch (const host::PyError&) { \
-        return value;              \
+#define HOST_CATCH(value)                                \
+    }                                                    \
+    catch (const host::PyError&) {                       \
+        return value;                                    \
+    }                                                    \
+    catch (const std::bad_alloc&) {                      \
+        PyErr_NoMemory();                                \
+        return value;                                    \
+    }                                                    \
+    catch (const std::exception& e) {                    \
+        PyErr_SetString(PyExc_RuntimeError, e.what());   \
+        return value;                                    \
     }
 
 [[noreturn]] void Raise(int status, const char* format, ...);

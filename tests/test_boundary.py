@@ -271,6 +271,26 @@ except chx.BackendError as e:
     assert 'refused: no HIP device' in r.stdout
 
 
+def test_running_out_of_host_memory_is_an_exception():
+    """2^40 views of an empty axis: what the native routines allocate ends in MemoryError, not in the end of the process."""
+    code = """
+import resource
+import chainer_amd as chx
+class Buffer(object):
+    def data_ptr(self):
+        return 0
+a = chx.ndarray(Buffer(), 0, (0,), (4,), 'float32')
+used = int(open('/proc/self/statm').read().split()[0]) * resource.getpagesize()
+resource.setrlimit(resource.RLIMIT_AS, (used + (1 << 30), resource.RLIM_INFINITY))
+try:
+    chx.split(a, 1 << 40, 0)
+except MemoryError:
+    print('MemoryError')
+"""
+    r = subprocess.run([sys.executable, '-c', code], capture_output=True, text=True, cwd=ROOT)
+    assert r.returncode == 0 and 'MemoryError' in r.stdout, (r.returncode, r.stderr[-2000:])
+
+
 def test_bench_rejects_more_than_one_gpu():
     r = subprocess.run(['python', os.path.join(ROOT, 'bench.py'), '--gpus', '2'], capture_output=True, text=True)
     assert r.returncode != 0 and 'one GPU' in (r.stderr + r.stdout)
