@@ -1838,9 +1838,12 @@ size_t hipcx_dot_workspace_size(const hipcx_array* a, const hipcx_array* b, cons
         DotStaging st = PlanDotStaging(a, b, out);
         size_t split = 0;
         if (a != nullptr && b != nullptr && out != nullptr && a->ndim == 2 && b->ndim == 2 && a->shape[1] > 0 && a->shape[0] > 0 && b->shape[1] > 0) {
-            const int64_t m = a->shape[0], n = b->shape[1], k = a->shape[1];
-            split = SplitKBytes(m, n, PlanSplitK(m, n, k, out->dtype));
-            if (split == 0 && a->dtype == out->dtype && b->dtype == out->dtype) split = SmallDotWorkspace(a, b, out->dtype);
+            const int64_t m = a->shape[0], n = b->shape[1], k = a->shape[1], it = ItemSize(out->dtype);
+            // the 128 x 128 tiles split the reduction of operands laid out (or staged) for them, else the small product's tiles do
+            const bool fast = (st.a || OperandIsFast(a->data, a->strides[0], a->strides[1], k, it)) &&
+                              (st.b || OperandIsFast(b->data, b->strides[1], b->strides[0], k, it));
+            if (fast) split = SplitKBytes(m, n, PlanSplitK(m, n, k, out->dtype));
+            if (split == 0 && !st.a && !st.b && a->dtype == out->dtype && b->dtype == out->dtype) split = SmallDotWorkspace(a, b, out->dtype);
         }
         const size_t need = RoundUpTo(st.a_bytes + st.b_bytes, 256) + split;
         const GemmPpPlan pp = PlanGemmPp(a, b, out);

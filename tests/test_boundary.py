@@ -116,6 +116,8 @@ def test_dot_workspace_is_asked_for_by_the_kernels_that_split():
     assert need(1, 8192, 1000, True) == 0 and need(4, 8192, 1000, True) == 0
     assert need(128, 4000, 1000, True) == 0  # 1.02 GFLOP
     assert need(20, 8192, 1000, True) > 0 and need(1, 8192, 1000, False) > 0
+    # the 128 x 128 tiles would split this reduction in 19, but do not read a row-major b; the small product's tiles do, in 22
+    assert need(64, 5000, 64, False) == 22 * 64 * 64 * 4
 
 
 def test_oracle_library_loads():
