@@ -8,8 +8,7 @@ Every figure is device time between two events recorded on the launch stream aro
 (after warm-up), divided by `iters`; the sweep section also replays ten calls captured into one HIP graph and keeps the
 smaller figure, because the host needs longer to issue a call than the shortest kernels run.  Bandwidth figures divide the *algorithmic* bytes of the operation (each operand
 once, no temporaries) by that time; the fraction is taken against the published peaks (8 TB/s HBM, 2.5 PFLOP/s dense
-fp16 MFMA, 157.3 TFLOP/s fp32 MFMA).  Chains of kernels (log_softmax = 7 launches, softmax_cross_entropy, the LSTM
-cell) are timed as the chain and priced against the bytes a single fused pass would move.
+fp16 MFMA, 157.3 TFLOP/s fp32 MFMA).
 
 `run(sections, cpu=namespace)` additionally times each operation on a CPU implementation of the same routine names that
 the caller passes in (bench.py passes its single-threaded restatement of the ChainerX native backend; bounded sample
@@ -120,20 +119,13 @@ def section_sweep(chx, oracle, with_cpu):
             ('sum axis1', lambda: chx.sum(X, 1), n * s + rows * s, 1, (lambda: oracle.sum(small, 1)) if with_cpu else None),
             ('max axis1', lambda: chx.amax(X, 1), n * s + rows * s, 1, (lambda: oracle.amax(small, 1)) if with_cpu else None),
             ('argmax axis1', lambda: chx.argmax(X, 1), n * s + rows * 8, 1, (lambda: oracle.argmax(small, 1)) if with_cpu else None),
-            ('log_softmax axis1', lambda: chx.log_softmax(X, 1), (2 if shape[1] * s <= 65536 else 3) * n * s, 7,
+            ('log_softmax axis1', lambda: chx.log_softmax(X, 1), (2 if shape[1] * s <= 65536 else 3) * n * s, 1 if shape[1] * s <= 65536 else 2,
              (lambda: oracle.log_softmax(small, 1)) if with_cpu else None),
-            ('log_softmax axis1, fused opt-in entry', lambda: chx.log_softmax_fused(X, 1), (2 if shape[1] * s <= 65536 else 3) * n * s,
-             1 if shape[1] * s <= 65536 else 2, None),
         ]
         for name, fn, nbytes, launches, cfn in ops:
             t = op_time(fn)
             cpu = cpu_time(cfn) * scale if cfn is not None else None
-            note = None
-            if 'fused' in name:
-                note = 'hipcx_log_softmax: one read + one write for rows up to 64 KiB, two reads + one write beyond; not the drop-in kernel boundary'
-            elif launches > 1:
-                note = ('7 kernel launches as the ChainerX routine decomposes it (moves 8*N*4 bytes: ceiling %.0f%% of the '
-                        'fused-ideal figure used here)' % (100.0 * nbytes / (8 * n * s)))
+            note = 'one read + one write for rows up to 64 KiB, two reads + one write beyond' if 'softmax' in name else None
             bw_row('sweep', name, shape, t, nbytes, launches, cpu, note)
 
 
@@ -149,7 +141,7 @@ def section_mlp(chx, oracle, with_cpu):
     graph = graph_time(fn)
     flops = 2 * 100 * (784 * 1000 + 1000 * 1000 + 1000 * 10)
     row = dict(section='mlp', op='forward+loss', batch=100, eager_us=round(eager * 1e6, 1), graph_replay_us=round(graph * 1e6, 1),
-               kernel_launches=3 + 3 + 2 + 15, GFLOP=round(flops / 1e9, 4), TFLOPs_graph=round(flops / graph / 1e12, 2))
+               kernel_launches=3 + 2 + 1, GFLOP=round(flops / 1e9, 4), TFLOPs_graph=round(flops / graph / 1e12, 2))
     if with_cpu:
         row['cpu_native_1core_us'] = round(cpu_time(lambda: cfg.mlp_forward(oracle, p, x, t)) * 1e6, 1)
     emit(**row)
@@ -233,14 +225,10 @@ def section_lstm(chx, oracle, with_cpu):
     graph = graph_time(fn, 5)
     flops = 60.57e9 + 58.24e9
     row = dict(section='lstm', op='35-step forward', batch=128, eager_ms=round(eager * 1e3, 2), graph_replay_ms=round(graph * 1e3, 2),
-               TFLOPs_graph=round(flops / graph / 1e12, 2), tokens_per_s_graph=round(128 * 35 / graph, 0), kernel_launches=35 * 86 + 7,
-               note='eager time is host launch overhead (~3000 kernel calls); take runs in the default bounds mode (mode=None, what the '
+               TFLOPs_graph=round(flops / graph / 1e12, 2), tokens_per_s_graph=round(128 * 35 / graph, 0), kernel_launches=4 + 35 * 10 + 1,
+               note='take runs in the default bounds mode (mode=None, what the '
                     'reference caller passes): an out-of-range id is recorded on the device and raised by the next get / synchronize')
     emit(**row)
-    fused = graph_time(lambda: cfg.lstm_lm_forward(chx, pd, I, chx.zeros, None, True), 5)
-    emit(section='lstm', op='35-step forward, fused opt-in Lstm cell and LogSoftmax', batch=128, graph_replay_ms=round(fused * 1e3, 2),
-         TFLOPs_graph=round(flops / fused / 1e12, 2), tokens_per_s_graph=round(128 * 35 / fused, 0), kernel_launches=35 * 14 + 1,
-         note='hipcx_lstm_cell and hipcx_log_softmax replace the ~25-kernel cell and the 7-kernel LogSoftmax chains; not the drop-in kernel boundary')
     # NStepLstm at the same size: 2 layers x 35 steps, batch 128, 650 units (float32)
     rng = np.random.default_rng(5)
     u = 650

@@ -384,8 +384,8 @@ def lstm_lm_input(seed=5, batch=128, seq=35, vocab=10000):
 
 def lstm_lm_forward(F, p, ids, zeros, take_mode=None, fused=False):
     """Runs the sequence; returns log-probabilities of the last step and the final (h, c) of both layers.
-    ``zeros(shape, dtype)`` makes the initial state on the same backend as ``F``.  ``fused`` takes the opt-in one-kernel
-    Lstm cell and LogSoftmax (``F.lstm_fused``, ``F.log_softmax_fused``) instead of the routine chains."""
+    ``zeros(shape, dtype)`` makes the initial state on the same backend as ``F``.  ``fused`` calls ``F.lstm_fused`` and
+    ``F.log_softmax_fused``, which run the kernels that ``F.lstm`` and ``F.log_softmax`` of this backend run for these arrays."""
     lstm = F.lstm_fused if fused else F.lstm
     log_softmax = F.log_softmax_fused if fused else F.log_softmax
     batch, seq = ids.shape

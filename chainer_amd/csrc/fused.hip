@@ -1,8 +1,10 @@
-// Opt-in fused entries for two routine chains that the reference runs as many small kernels:
+// Routine chains that the reference runs as many small kernels, as one or two; the routines take them wherever their arrays allow:
 //   * LogSoftmax (CX/routines/reduction.cc:78-92): AMax, Subtract, Exp, Sum, Log, Add, Subtract -- 5 reads and 3 writes of
 //     the array -- as one read + one write when a row fits in a workgroup's registers, two reads + one write otherwise;
+//   * softmax cross entropy (chainer/functions/loss/softmax_cross_entropy.py:123-130): LogSoftmax and a masked mean, about 15 kernels,
+//     as one read;
 //   * the Lstm cell (CX/routines/connection.cc:396-446): ~25 strided elementwise kernels as one.
-// Both evaluate the same float operations in the same order as the chain (Exp/Tanh/Log are the same device functions the
+// They evaluate the same float operations in the same order as the chain (Exp/Tanh/Log are the same device functions the
 // separate kernels call; no contraction), so for float32/float64 the Lstm cell is bit-identical to the chain and LogSoftmax
 // differs only through the order of the row sum.  float16 computes in float and rounds once.
 #include <algorithm>

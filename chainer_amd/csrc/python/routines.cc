@@ -1096,7 +1096,7 @@ HOST_FN(TakeDeferred) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// fused, opt-in
+// routine chains as one kernel call
 // ---------------------------------------------------------------------------------------------
 // LogSoftmax of a 2-D array along its unit-stride axis 1 through hipcx_log_softmax, or None for other calls: an axis without elements is
 // an error that the chain's AMax raises.

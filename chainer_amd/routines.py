@@ -1395,7 +1395,7 @@ def lstm(c, x):
 
 
 def lstm_fused(c, x):
-    """The Lstm cell through hipcx_lstm_cell, which lstm takes by itself for every call the kernel covers."""
+    """lstm, which takes hipcx_lstm_cell by itself for every call the kernel covers."""
     return lstm(c, x)
 
 
