@@ -92,7 +92,7 @@ extern "C" int hipcx_copy_many(const hipcx_array* const* as, const hipcx_array* 
                 continue;
             }
             if (size == 0) continue;
-            if (p.n == kMaxSegments || bytes + size >= (int64_t{1} << 40)) flush();
+            if (p.n == kMaxSegments || bytes + size >= (int64_t{1} << 37)) flush();  // (a grid holds less than 2^32 threads)
             p.seg[p.n].src = static_cast<const char*>(as[i]->data);
             p.seg[p.n].dst = static_cast<char*>(outs[i]->data);
             p.seg[p.n++].bytes = size;

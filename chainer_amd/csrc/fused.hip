@@ -789,14 +789,19 @@ int hipcx_lstm_cell(const hipcx_array* c, const hipcx_array* x, const hipcx_arra
         const int64_t B = c->shape[0], H = c->shape[1];
         const int64_t total = B * H;
         if (total == 0) return;
-        HIPCX_REQUIRE(H < (1LL << 31) && (total + 255) / 256 < (1LL << 31), HIPCX_NOT_IMPLEMENTED_ERROR, "lstm_cell: problem too large for one launch");
+        HIPCX_REQUIRE(H < (1LL << 31), HIPCX_NOT_IMPLEMENTED_ERROR, "lstm_cell: problem too large for one launch");
         const int vec_ok = reinterpret_cast<uintptr_t>(x->data) % (4 * it) == 0 && x->strides[0] % (4 * it) == 0;
+        const int64_t rows = std::max<int64_t>(1, (int64_t{1} << 31) / H);  // of one launch: a grid holds less than 2^32 threads
         VisitFloatDtype(c->dtype, [&](auto tag) {
             using T = typename decltype(tag)::type;
-            hipLaunchKernelGGL(LstmCellKernel<T>, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0, AsStream(stream),
-                               static_cast<const T*>(c->data), static_cast<const T*>(x->data), static_cast<T*>(h_out->data),
-                               static_cast<T*>(c_out->data), total, static_cast<int>(H), c->strides[0] / it, x->strides[0] / it,
-                               h_out->strides[0] / it, c_out->strides[0] / it, vec_ok);
+            const int64_t c_row = c->strides[0] / it, x_row = x->strides[0] / it, h_row = h_out->strides[0] / it, co_row = c_out->strides[0] / it;
+            for (int64_t b = 0; b < B; b += rows) {
+                const int64_t part = std::min(rows, B - b) * H;
+                hipLaunchKernelGGL(LstmCellKernel<T>, dim3(static_cast<unsigned>((part + 255) / 256)), dim3(256), 0, AsStream(stream),
+                                   static_cast<const T*>(c->data) + b * c_row, static_cast<const T*>(x->data) + b * x_row,
+                                   static_cast<T*>(h_out->data) + b * h_row, static_cast<T*>(c_out->data) + b * co_row, part, static_cast<int>(H),
+                                   c_row, x_row, h_row, co_row, vec_ok);
+            }
         });
         CheckLaunch("lstm_cell");
     });

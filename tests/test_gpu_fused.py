@@ -187,6 +187,27 @@ def test_lstm_cell_fused(dt):
     assert_close(cn.get(), c_ref, None, 'lstm strided c')
 
 
+def test_lstm_of_more_units_than_a_launch_takes():
+    import torch
+    import chainer_amd as chx
+    rows, units = (1 << 20) + 3, 4096
+    if torch.cuda.mem_get_info()[0] < 5 * rows * units:
+        pytest.skip('needs %d bytes of device memory' % (5 * rows * units))
+    rng = np.random.default_rng(14)
+    c, x = rng.standard_normal((1, units)).astype('float16'), (rng.standard_normal((1, 4 * units)) * 2).astype('float16')
+    h_ref, c_ref = O.lstm(c, x)
+    h = cn = None
+    try:
+        h, cn = chx.lstm(chx.array(c).broadcast_to((rows, units)), chx.array(x).broadcast_to((rows, 4 * units)))
+        for lo in (0, (1 << 19) - 1, (1 << 20) - 1, rows - 2):
+            assert_close(h[lo:lo + 2].get(), np.repeat(h_ref, 2, 0), None, 'h of row %d' % lo)
+            assert_close(cn[lo:lo + 2].get(), np.repeat(c_ref, 2, 0), None, 'c of row %d' % lo)
+    finally:
+        del h, cn
+        chx.synchronize()
+        chx.free_unused_blocks()
+
+
 def test_lstm_cell_fused_errors():
     """Shape and dtype errors of the Lstm routine (CX/routines/connection.cc:398-416)."""
     import chainer_amd as chx
