@@ -20,6 +20,7 @@
 // GenericReduceKernel: any strides; one thread per output element runs the reference loop
 // literally.  Consecutive threads take consecutive outputs, so reducing over outer axes of a
 // dense array (a "column" reduction) is coalesced.
+#include <algorithm>
 #include <mutex>
 
 #include "common.h"
@@ -37,6 +38,7 @@ constexpr int kElemsPerIter = kRowThreads * 4;  // 1024 elements = 32 chunks = 4
 constexpr int kMaxIters = 64;                   // iterations per block -> span <= 65536 elements
 constexpr int kMaxNodes = kMaxIters * 16;       // LDS nodes per block: one per row of 16 lanes (two chunks) and iteration
 constexpr int kMaxPartials = 1024;              // blocks per row handled by the finalize pass
+constexpr int64_t kBlocksPerLaunch = (1 << 24) - 1;  // of 256: a grid holds less than 2^32 threads, of more some do not run (without an error)
 
 // ---------------------------------------------------------------------------------------------
 // Reduction functors.  Acc is what travels through the tree.
@@ -332,18 +334,19 @@ __device__ __forceinline__ typename Op::Acc MergeRows(typename Op::Acc acc) {
 }
 
 template <typename Impl>
-__global__ __launch_bounds__(kRowThreads) void RowReduceKernel(ReduceGeom g, int64_t span, int blocks_per_row, void* partials) {
+__global__ __launch_bounds__(kRowThreads) void RowReduceKernel(ReduceGeom g, int64_t row0, int64_t span, int blocks_per_row, void* partials) {
     using R = typename Impl::Row;  // the same reduction with indices counted from the block's first element
     using In = typename R::In;
     using Acc = typename R::Acc;
     __shared__ Acc nodes[kMaxNodes];
     __shared__ Acc wave_nodes[kMaxNodes / 64];
 
-    int64_t row = blockIdx.x;
+    int64_t row = row0 + blockIdx.x;
     int blk = 0;
     if (blocks_per_row != 1) {
-        row = blockIdx.x / static_cast<unsigned>(blocks_per_row);
-        blk = static_cast<int>(blockIdx.x - static_cast<unsigned>(row) * static_cast<unsigned>(blocks_per_row));
+        const unsigned r = blockIdx.x / static_cast<unsigned>(blocks_per_row);
+        row = row0 + r;
+        blk = static_cast<int>(blockIdx.x - r * static_cast<unsigned>(blocks_per_row));
     }
     int64_t in_off, out_off;
     OutOffsets(g, row, in_off, out_off);
@@ -560,10 +563,10 @@ __global__ __launch_bounds__(kRowThreads) void RowReduceKernel(ReduceGeom g, int
 
 // second pass: tree over the per-block partials of each row (blocks_per_row <= kMaxPartials)
 template <typename Impl>
-__global__ __launch_bounds__(kRowThreads) void RowFinalizeKernel(ReduceGeom g, int blocks_per_row, const void* partials) {
+__global__ __launch_bounds__(kRowThreads) void RowFinalizeKernel(ReduceGeom g, int64_t row0, int blocks_per_row, const void* partials) {
     using Acc = typename Impl::Acc;
     __shared__ Acc nodes[kMaxPartials];
-    const int64_t row = blockIdx.x;
+    const int64_t row = row0 + blockIdx.x;
     const int tid = threadIdx.x;
     int n = 1;
     while (n < blocks_per_row) n <<= 1;
@@ -590,10 +593,10 @@ __global__ __launch_bounds__(kRowThreads) void RowFinalizeKernel(ReduceGeom g, i
 // Generic kernel: the reference loop, one output per thread
 // ---------------------------------------------------------------------------------------------
 template <typename Impl>
-__global__ __launch_bounds__(256) void GenericReduceKernel(ReduceGeom g) {
+__global__ __launch_bounds__(256) void GenericReduceKernel(ReduceGeom g, int64_t o0) {
     using In = typename Impl::In;
     using Acc = typename Impl::Acc;
-    const int64_t o = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    const int64_t o = o0 + static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (o >= g.n_out) return;
     int64_t in_off, out_off;
     OutOffsets(g, o, in_off, out_off);
@@ -804,12 +807,12 @@ __global__ __launch_bounds__(256) void ColumnChunkKernel(ReduceGeom g, int64_t n
 
 // SL threads share an output; each first merges an aligned run of 2^run_level slice nodes.
 template <typename Impl, int SL>
-__global__ __launch_bounds__(256) void ColumnFinishKernel(ReduceGeom g, int nslices, int run_level, const void* partials) {
+__global__ __launch_bounds__(256) void ColumnFinishKernel(ReduceGeom g, int64_t first_out, int nslices, int run_level, const void* partials) {
     using Acc = typename Impl::Acc;
     constexpr int CF = 256 / SL;
     __shared__ Acc nodes[SL][CF];
     const int c = threadIdx.x % CF, sl = threadIdx.x / CF;
-    const int64_t o = static_cast<int64_t>(blockIdx.x) * CF + c;
+    const int64_t o = first_out + static_cast<int64_t>(blockIdx.x) * CF + c;
     const Acc* part = static_cast<const Acc*>(partials);
     Acc acc = Impl::Empty();
     if (o < g.n_out) {
@@ -982,7 +985,7 @@ ReducePlan MakePlan(const hipcx_array* a, const int8_t* axis, int naxis, const h
         pl.col_blocks = (units + pl.col_lanes - 1) / pl.col_lanes;
         const int64_t per_slice = 256 / pl.col_lanes;
         const int64_t slices = (chunks + per_slice - 1) / per_slice;
-        if (slices < (1LL << 30) && pl.col_blocks * slices < (1LL << 31)) {
+        if (pl.col_blocks * slices <= kBlocksPerLaunch) {
             pl.column_path = true;
             pl.col_chunks = chunks;
             pl.col_slices = static_cast<int>(slices);
@@ -1026,13 +1029,16 @@ void Run(const hipcx_array* a, const int8_t* axis, int naxis, const hipcx_array*
                       "reduction workspace too small: need " + std::to_string(need) + " bytes");
         HIPCX_REQUIRE(need == 0 || reinterpret_cast<uintptr_t>(workspace) % 16 == 0, HIPCX_CHAINERX_ERROR,
                       "workspace must be 16-byte aligned");
-        dim3 grid(static_cast<unsigned>(g.n_out * pl.blocks_per_row)), block(kRowThreads);
-        hipLaunchKernelGGL((RowReduceKernel<Impl>), grid, block, 0, stream, g, pl.span, pl.blocks_per_row, workspace);
-        CheckLaunch("row_reduce");
-        if (pl.blocks_per_row > 1) {
-            hipLaunchKernelGGL((RowFinalizeKernel<Impl>), dim3(static_cast<unsigned>(g.n_out)), block, 0, stream, g, pl.blocks_per_row,
-                               workspace);
-            CheckLaunch("row_reduce_finalize");
+        const int64_t rows = std::max<int64_t>(1, kBlocksPerLaunch / pl.blocks_per_row);  // of one launch
+        for (int64_t r0 = 0; r0 < g.n_out; r0 += rows) {
+            const int64_t count = std::min(rows, g.n_out - r0);
+            const dim3 grid(static_cast<unsigned>(count * pl.blocks_per_row)), block(kRowThreads);
+            hipLaunchKernelGGL((RowReduceKernel<Impl>), grid, block, 0, stream, g, r0, pl.span, pl.blocks_per_row, workspace);
+            CheckLaunch("row_reduce");
+            if (pl.blocks_per_row > 1) {
+                hipLaunchKernelGGL((RowFinalizeKernel<Impl>), dim3(static_cast<unsigned>(count)), block, 0, stream, g, r0, pl.blocks_per_row, workspace);
+                CheckLaunch("row_reduce_finalize");
+            }
         }
         return;
     }
@@ -1063,8 +1069,10 @@ void Run(const hipcx_array* a, const int8_t* axis, int naxis, const hipcx_array*
             int level = 0;
             while ((static_cast<int64_t>(sl) << level) < pl.col_slices) ++level;
             const int64_t per_block = 256 / sl;
-            hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>((g.n_out + per_block - 1) / per_block)), block, 0, stream, g, pl.col_slices, level,
-                               workspace);
+            for (int64_t o = 0; o < g.n_out; o += kBlocksPerLaunch * per_block) {
+                const int64_t blocks = std::min(kBlocksPerLaunch, (g.n_out - o + per_block - 1) / per_block);
+                hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), block, 0, stream, g, o, pl.col_slices, level, workspace);
+            }
         };
         if (pl.col_slices <= 16) {
             finish(ColumnFinishKernel<Impl, 16>, 16);
@@ -1076,9 +1084,10 @@ void Run(const hipcx_array* a, const int8_t* axis, int naxis, const hipcx_array*
         CheckLaunch("column_reduce_finish");
         return;
     }
-    int64_t blocks = (g.n_out + 255) / 256;
-    HIPCX_REQUIRE(blocks < (1LL << 31), HIPCX_NOT_IMPLEMENTED_ERROR, "too many outputs for one launch");
-    hipLaunchKernelGGL((GenericReduceKernel<Impl>), dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, g);
+    for (int64_t o0 = 0; o0 < g.n_out; o0 += kBlocksPerLaunch * 256) {
+        const int64_t blocks = std::min(kBlocksPerLaunch, (g.n_out - o0 + 255) / 256);
+        hipLaunchKernelGGL((GenericReduceKernel<Impl>), dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, g, o0);
+    }
     CheckLaunch("generic_reduce");
 }
 

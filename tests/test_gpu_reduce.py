@@ -206,3 +206,28 @@ def test_reduce_over_a_long_strided_axis(dt):
         X = chx.array(x)
         assert_exact(chx.sum(X[:, ::3].T, 1).get(), O.sum(x[:, ::3].T, 1), 'sum over the strided axis of a view')
         assert_exact(chx.sum(X[:, ::3], 1).get(), O.sum(x[:, ::3], 1), 'sum over a stepped axis')
+
+
+def test_more_outputs_than_a_grid_has_threads_for():
+    """2^24 rows, a workgroup of 256 threads to each; 2^32 outputs, a thread to each."""
+    import torch
+    import chainer_amd as chx
+    rng = np.random.default_rng(23)
+    row = rng.integers(-100, 101, 300).astype('int8')
+    row[77] = 120
+    rows = (1 << 24) + 5
+    X = chx.array(row[None]).broadcast_to((rows, 300))
+    assert np.all(chx.sum(X, 1).get() == row.astype('int64').sum())
+    assert np.all(chx.argmax(X, 1).get() == row.argmax())
+    outputs = (1 << 32) + 5
+    if torch.cuda.mem_get_info()[0] < 2 * outputs:
+        pytest.skip('needs %d bytes of device memory' % (2 * outputs))
+    out = None
+    try:
+        out = chx.amax(chx.array(row[None, :2]).broadcast_to((outputs, 2)), 1)
+        for lo in (0, (1 << 31) - 500, (1 << 32) - 1000, outputs - 1000):
+            assert np.all(out[lo:lo + 1000].get() == row[:2].max()), lo
+    finally:
+        del out
+        chx.synchronize()
+        chx.free_unused_blocks()
