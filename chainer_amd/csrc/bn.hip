@@ -277,7 +277,8 @@ void RunBn(const hipcx_array* x, const hipcx_array* const params[4], hipcx_scala
             int64_t lds = max_rows * 4 * static_cast<int64_t>(sizeof(C));
             int64_t blocks = (total + span - 1) / span;
             const int stream_in = vec_ok && total * it > StreamingThresholdBytes() ? 1 : 0;
-            if (lds <= 48 * 1024 && blocks < (1LL << 31) && L < (1LL << 30)) {
+            static_assert(kBnFlatThreads == 256, "kBlocksPerLaunch");
+            if (lds <= 48 * 1024 && blocks <= kBlocksPerLaunch && L < (1LL << 30)) {
                 if (vec_ok) {
                     hipLaunchKernelGGL((BnChannelsFirstKernel<T, VEC>), dim3(static_cast<unsigned>(blocks)), dim3(kBnFlatThreads),
                                        static_cast<size_t>(lds), stream, xp, op, g, b, m, v_, eps, static_cast<int>(Cn), L, ps / it, total,

@@ -242,6 +242,18 @@ inline int DivUp(int64_t a, int64_t b) { return static_cast<int>((a + b - 1) / b
 // Number of compute units of the current device (cached); used to size grid-stride launches.
 int NumCUs();
 
+// Workgroups of 256 threads along a grid's x axis: a grid holds less than 2^32 threads, and of more some do not run, without an error.
+constexpr int64_t kBlocksPerLaunch = (1 << 24) - 1;
+
+// f(grid, first) for every launch of `threads` threads in workgroups of 256, the first of them being thread `first`.
+template <typename F>
+inline void ForLaunches(int64_t threads, F&& f) {
+    for (int64_t first = 0; first < threads; first += kBlocksPerLaunch * 256) {
+        const int64_t blocks = (threads - first + 255) / 256;
+        f(dim3(static_cast<unsigned>(blocks < kBlocksPerLaunch ? blocks : kBlocksPerLaunch)), first);
+    }
+}
+
 // Input size beyond which a streaming kernel loads without allocating in the caches.  A large tensor read front to back with
 // allocating loads pushes out what the memory-side cache (256 MB on this part) still holds of it and of its neighbours in the
 // network; the threshold (75 MB) is the measured optimum over a ResNet-50 forward pass.  HIPCX_STREAM_MB overrides (0 = never).

@@ -81,7 +81,7 @@ void LaunchShape(IGemmArgs<T> p, bool fast16, bool fast8, hipStream_t stream) {
     p.tiles_m = static_cast<int>((p.M + BM - 1) / BM);
     p.tiles_n = (p.K + BN - 1) / BN;
     int64_t total = static_cast<int64_t>(p.tiles_m) * p.tiles_n;
-    HIPCX_REQUIRE(total < (1LL << 30), HIPCX_NOT_IMPLEMENTED_ERROR, "problem too large for one launch");
+    HIPCX_REQUIRE(total <= kBlocksPerLaunch - 7, HIPCX_NOT_IMPLEMENTED_ERROR, "problem too large for one launch");
     int per = static_cast<int>((total + 7) / 8);
     // wide products: a row of concurrent tiles would read more second-operand panels than an XCD's L2 holds
     static const int band_env = [] { const char* e = getenv("HIPCX_IGEMM_BAND"); return e != nullptr ? atoi(e) : 8; }();
@@ -147,8 +147,26 @@ bool FastOk(const IGemmArgs<T>& p, int lb) {
     return true;
 }
 
+// f(problem) for the whole problem, or for groups of its images that have at most max_pixels output positions each.
+template <typename T, typename F>
+void ForImageGroups(const IGemmArgs<T>& p, int64_t max_pixels, F&& f) {
+    if (p.M <= max_pixels) return f(p);
+    const int64_t plane = static_cast<int64_t>(p.OH) * p.OW, group = max_pixels / plane;
+    HIPCX_REQUIRE(group > 0, HIPCX_NOT_IMPLEMENTED_ERROR, "image too large for one launch");
+    for (int64_t n = 0; n < p.N; n += group) {
+        IGemmArgs<T> q = p;
+        q.N = static_cast<int>(p.N - n < group ? p.N - n : group);
+        q.M = q.N * plane;
+        q.x += n * p.xsN;
+        q.out += n * p.osN;
+        f(q);
+    }
+}
+
 template <typename T>
 void LaunchIGemmImpl(IGemmArgs<T> p, hipStream_t stream) {
+    constexpr int64_t kMaxPixels = (int64_t{1} << 31) - 256;  // the kernels count a tile's first position in 31 bits
+    if (p.M > kMaxPixels) return ForImageGroups(p, kMaxPixels, [&](const IGemmArgs<T>& q) { LaunchIGemmImpl(q, stream); });
     if (p.M == 0 || p.K == 0) return;
     if (p.C_logical == 0) {
         p.C_logical = p.C;
@@ -560,12 +578,16 @@ void LaunchF64(IGemmArgs<double> p, hipStream_t stream) {
     if (total == 0) return;
     if (total * p.Kg < (1 << 16) || p.Kg == 0) {  // a few thousand multiply-adds: not worth mostly empty tiles
         int64_t blocks = (total + 255) / 256;
+        HIPCX_REQUIRE(blocks <= kBlocksPerLaunch, HIPCX_NOT_IMPLEMENTED_ERROR, "problem too large for one launch");
         hipLaunchKernelGGL(ConvNaiveF64Kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, p);
         CheckLaunch("conv_f64");
         return;
     }
     const int64_t tiles_m = (p.M + kF64TileM - 1) / kF64TileM, tiles_n = (p.K + kF64TileN - 1) / kF64TileN;
-    HIPCX_REQUIRE(tiles_m * tiles_n < (1LL << 31) && tiles_m < (1LL << 31), HIPCX_NOT_IMPLEMENTED_ERROR, "problem too large for one launch");
+    if (tiles_m * tiles_n > kBlocksPerLaunch) {
+        HIPCX_REQUIRE(tiles_n <= kBlocksPerLaunch, HIPCX_NOT_IMPLEMENTED_ERROR, "problem too large for one launch");
+        return ForImageGroups(p, kBlocksPerLaunch / tiles_n * kF64TileM, [&](const IGemmArgs<double>& q) { LaunchF64(q, stream); });
+    }
     p.tiles_m = static_cast<int>(tiles_m);
     p.tiles_n = static_cast<int>(tiles_n);
     ProfileScope prof(stream, 2.0 * static_cast<double>(p.M) * p.K * p.Kg,

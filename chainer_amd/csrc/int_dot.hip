@@ -114,7 +114,14 @@ void IntDot(const hipcx_array* a, const hipcx_array* b, const hipcx_array* out, 
     VisitDtype(out->dtype, [&](auto tag) {
         using T = typename decltype(tag)::type;
         if constexpr (!std::is_floating_point<T>::value && !std::is_same<T, half_t>::value) {
-            hipLaunchKernelGGL((IntDotKernel<T>), dim3(static_cast<unsigned>(tiles_n), static_cast<unsigned>(tiles_m)), dim3(256), 0, stream, p);
+            for (int64_t first = 0; first < tiles_n; first += kBlocksPerLaunch) {
+                IntDotArgs q = p;
+                q.b = static_cast<const T*>(p.b) + first * kTile * p.b_col;
+                q.out = static_cast<T*>(p.out) + first * kTile * p.o_col;
+                q.n = p.n - first * kTile;
+                const int64_t tiles = tiles_n - first < kBlocksPerLaunch ? tiles_n - first : kBlocksPerLaunch;
+                hipLaunchKernelGGL((IntDotKernel<T>), dim3(static_cast<unsigned>(tiles), static_cast<unsigned>(tiles_m)), dim3(256), 0, stream, q);
+            }
         } else {
             throw Error(HIPCX_DTYPE_ERROR, "IntDot: integer or bool dtype required");
         }

@@ -15,6 +15,7 @@ struct ToChannelsLastArgs {
     int Ho, Wo;          // output plane extents
     int step_h, step_w;  // input pixel = (h * step_h, w * step_w)
     int64_t xsN, xsC, xsH, xsW;  // elements
+    int64_t first_tile;  // of 64 pixels
     int vec_in;          // 1: plane is dense along pixels (xsW == 1, xsH == Wo, steps 1) and 16-byte loads are aligned
 };
 
@@ -28,7 +29,7 @@ __global__ __launch_bounds__(256) void ToChannelsLastKernel(ToChannelsLastArgs a
     T* out = static_cast<T*>(a.out);
     const int tid = threadIdx.x;
     const int64_t plane = static_cast<int64_t>(a.Ho) * a.Wo;
-    const int64_t p0 = static_cast<int64_t>(blockIdx.x) * TILE;
+    const int64_t p0 = (a.first_tile + blockIdx.x) * TILE;
     const int c0 = blockIdx.y * TILE;
     const int n = blockIdx.z;
     const T* xn = x + n * a.xsN;
@@ -88,12 +89,17 @@ __global__ __launch_bounds__(256) void ToChannelsLastKernel(ToChannelsLastArgs a
 }
 
 template <typename T>
-inline void LaunchToChannelsLast(const ToChannelsLastArgs& a, hipStream_t stream) {
+inline void LaunchToChannelsLast(ToChannelsLastArgs a, hipStream_t stream) {
     int64_t plane = static_cast<int64_t>(a.Ho) * a.Wo;
     if (plane == 0 || a.N == 0 || a.Cpad == 0) return;
-    dim3 grid(static_cast<unsigned>((plane + 63) / 64), static_cast<unsigned>((a.Cpad + 63) / 64), static_cast<unsigned>(a.N));
+    dim3 grid(1, static_cast<unsigned>((a.Cpad + 63) / 64), static_cast<unsigned>(a.N));
     HIPCX_REQUIRE(grid.y <= 65535 && grid.z <= 65535, HIPCX_NOT_IMPLEMENTED_ERROR, "too many channels or images for the layout kernel");
-    hipLaunchKernelGGL((ToChannelsLastKernel<T>), grid, dim3(256), 0, stream, a);
+    const int64_t tiles = (plane + 63) / 64;
+    for (a.first_tile = 0; a.first_tile < tiles; a.first_tile += kBlocksPerLaunch) {
+        const int64_t left = tiles - a.first_tile;
+        grid.x = static_cast<unsigned>(left < kBlocksPerLaunch ? left : kBlocksPerLaunch);
+        hipLaunchKernelGGL((ToChannelsLastKernel<T>), grid, dim3(256), 0, stream, a);
+    }
     CheckLaunch("to_channels_last");
 }
 

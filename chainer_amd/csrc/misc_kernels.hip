@@ -51,9 +51,9 @@ struct LinspaceOp {
 };
 
 template <typename T>
-__global__ __launch_bounds__(256) void DiagflatKernel(const char* v, int64_t v_stride, int64_t nv, T* out, int64_t n, int64_t row_start,
-                                                      int64_t col_start) {
-    int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+__global__ __launch_bounds__(256) void DiagflatKernel(const char* v, int64_t v_stride, int64_t nv, T* out, int64_t first, int64_t n,
+                                                      int64_t row_start, int64_t col_start) {
+    int64_t i = first + static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
     if (i >= n * n) return;
     int64_t row = i / n, col = i - row * n;
     int64_t j = row - row_start;
@@ -76,9 +76,9 @@ struct ScanArgs {
 };
 
 template <typename In, typename Out>
-__global__ __launch_bounds__(256) void CumsumKernel(ScanArgs s) {
+__global__ __launch_bounds__(256) void CumsumKernel(ScanArgs s, int64_t first) {
     using Acc = std::conditional_t<std::is_same<Out, half_t>::value, float, Out>;
-    int64_t line = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+    int64_t line = first + static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
     if (line >= s.lines) return;
     int64_t in_off = 0, out_off = 0, r = line;
     for (int d = s.n_outer - 1; d >= 0; --d) {
@@ -172,12 +172,12 @@ int hipcx_diagflat(const hipcx_array* v, int64_t k, const hipcx_array* out, void
         const int64_t absk = k < 0 ? -k : k;
         HIPCX_REQUIRE(out->shape[1] == n && n == v->shape[0] + absk, HIPCX_DIMENSION_ERROR, "diagflat: out must be [len(v) + |k|]^2");
         if (n == 0) return;
-        HIPCX_REQUIRE((n * n + 255) / 256 < (1LL << 31), HIPCX_NOT_IMPLEMENTED_ERROR, "diagflat: output too large for one launch");
         VisitDtype(out->dtype, [&](auto tag) {
             using T = typename decltype(tag)::type;
-            hipLaunchKernelGGL(DiagflatKernel<T>, dim3(static_cast<unsigned>((n * n + 255) / 256)), dim3(256), 0, AsStream(stream),
-                               static_cast<const char*>(v->data), v->strides[0], v->shape[0], static_cast<T*>(out->data), n, k >= 0 ? 0 : -k,
-                               k >= 0 ? k : 0);
+            ForLaunches(n * n, [&](dim3 grid, int64_t first) {
+                hipLaunchKernelGGL(DiagflatKernel<T>, grid, dim3(256), 0, AsStream(stream), static_cast<const char*>(v->data), v->strides[0],
+                                   v->shape[0], static_cast<T*>(out->data), first, n, k >= 0 ? 0 : -k, k >= 0 ? k : 0);
+            });
         });
         CheckLaunch("diagflat");
     });
@@ -205,19 +205,20 @@ int hipcx_cumsum(const hipcx_array* a, int8_t axis, const hipcx_array* out, void
         s.len = a->shape[axis];
         s.in_axis_stride = a->strides[axis];
         s.out_axis_stride = out->strides[axis];
-        HIPCX_REQUIRE((s.lines + 255) / 256 < (1LL << 31), HIPCX_NOT_IMPLEMENTED_ERROR, "cumsum: too many lines for one launch");
-        dim3 grid(static_cast<unsigned>((s.lines + 255) / 256)), block(256);
+        const dim3 block(256);
         hipStream_t st = AsStream(stream);
         // Out dtypes the routine produces: the input's float dtype, int64 for bool / integer inputs (CX/routines/reduction.cc:115-127)
         VisitDtype(a->dtype, [&](auto in_tag) {
             using In = typename decltype(in_tag)::type;
-            switch (out->dtype) {
-                case HIPCX_INT64: hipLaunchKernelGGL((CumsumKernel<In, int64_t>), grid, block, 0, st, s); break;
-                case HIPCX_FLOAT16: hipLaunchKernelGGL((CumsumKernel<In, half_t>), grid, block, 0, st, s); break;
-                case HIPCX_FLOAT32: hipLaunchKernelGGL((CumsumKernel<In, float>), grid, block, 0, st, s); break;
-                case HIPCX_FLOAT64: hipLaunchKernelGGL((CumsumKernel<In, double>), grid, block, 0, st, s); break;
-                default: throw Error(HIPCX_NOT_IMPLEMENTED_ERROR, std::string("hip cumsum: unsupported output dtype ") + DtypeName(out->dtype));
-            }
+            ForLaunches(s.lines, [&](dim3 grid, int64_t first) {
+                switch (out->dtype) {
+                    case HIPCX_INT64: hipLaunchKernelGGL((CumsumKernel<In, int64_t>), grid, block, 0, st, s, first); break;
+                    case HIPCX_FLOAT16: hipLaunchKernelGGL((CumsumKernel<In, half_t>), grid, block, 0, st, s, first); break;
+                    case HIPCX_FLOAT32: hipLaunchKernelGGL((CumsumKernel<In, float>), grid, block, 0, st, s, first); break;
+                    case HIPCX_FLOAT64: hipLaunchKernelGGL((CumsumKernel<In, double>), grid, block, 0, st, s, first); break;
+                    default: throw Error(HIPCX_NOT_IMPLEMENTED_ERROR, std::string("hip cumsum: unsupported output dtype ") + DtypeName(out->dtype));
+                }
+            });
         });
         CheckLaunch("cumsum");
     });

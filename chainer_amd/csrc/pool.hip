@@ -849,9 +849,9 @@ void RunPoolGrad(const PoolGradArgs& p, hipStream_t stream) {
     if constexpr (!IS_MAX) {
         const bool whole_plane = p.OH == 1 && p.OW == 1 && p.kh == p.H && p.kw == p.W && p.ph == 0 && p.pw == 0;
         const bool dense = p.dsW == 1 && p.dsH == p.W && p.dsC == static_cast<int64_t>(p.H) * p.W && p.dsN == p.dsC * p.C;
-        if (whole_plane && dense && reinterpret_cast<uintptr_t>(p.gx) % 16 == 0) {
-            constexpr int V = 16 / sizeof(T);
-            const int64_t threads = (total + V - 1) / V;
+        constexpr int V = 16 / sizeof(T);
+        const int64_t threads = (total + V - 1) / V;
+        if (whole_plane && dense && reinterpret_cast<uintptr_t>(p.gx) % 16 == 0 && threads <= kBlocksPerLaunch * 256) {
             const dim3 blocks(static_cast<unsigned>((threads + 255) / 256));
             if (total + 16 < (1LL << 31)) {
                 hipLaunchKernelGGL((GlobalAvgPoolGradKernel<T, unsigned>), blocks, dim3(256), 0, stream, p, static_cast<unsigned>(total));

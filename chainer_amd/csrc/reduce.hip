@@ -38,7 +38,6 @@ constexpr int kElemsPerIter = kRowThreads * 4;  // 1024 elements = 32 chunks = 4
 constexpr int kMaxIters = 64;                   // iterations per block -> span <= 65536 elements
 constexpr int kMaxNodes = kMaxIters * 16;       // LDS nodes per block: one per row of 16 lanes (two chunks) and iteration
 constexpr int kMaxPartials = 1024;              // blocks per row handled by the finalize pass
-constexpr int64_t kBlocksPerLaunch = (1 << 24) - 1;  // of 256: a grid holds less than 2^32 threads, of more some do not run (without an error)
 
 // ---------------------------------------------------------------------------------------------
 // Reduction functors.  Acc is what travels through the tree.
@@ -1084,10 +1083,7 @@ void Run(const hipcx_array* a, const int8_t* axis, int naxis, const hipcx_array*
         CheckLaunch("column_reduce_finish");
         return;
     }
-    for (int64_t o0 = 0; o0 < g.n_out; o0 += kBlocksPerLaunch * 256) {
-        const int64_t blocks = std::min(kBlocksPerLaunch, (g.n_out - o0 + 255) / 256);
-        hipLaunchKernelGGL((GenericReduceKernel<Impl>), dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, g, o0);
-    }
+    ForLaunches(g.n_out, [&](dim3 grid, int64_t o0) { hipLaunchKernelGGL((GenericReduceKernel<Impl>), grid, dim3(256), 0, stream, g, o0); });
     CheckLaunch("generic_reduce");
 }
 

@@ -134,8 +134,8 @@ __global__ __launch_bounds__(256) void TakeRowsKernel(TakeArgs t) {
 // reference's order (float results are bit-identical; float16 rounds after every addition, as Float16::operator+= does).
 // In TakeArgs terms: `a` is the accumulated array (with the axis), `out` is b (with the index axes).
 template <typename T>
-__global__ __launch_bounds__(256) void AddAtKernel(TakeArgs t) {
-    const int64_t w = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+__global__ __launch_bounds__(256) void AddAtKernel(TakeArgs t, int64_t first) {
+    const int64_t w = first + static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
     if (w >= t.total) return;
     const int64_t r = w % t.right.total;
     const int64_t l = w / t.right.total;
@@ -337,15 +337,13 @@ extern "C" int hipcx_add_at(const hipcx_array* a, const hipcx_array* indices, in
         t.total = t.left.total * t.right.total;
         const bool nothing_to_add = t.total == 0 || t.index.total == 0;
         HIPCX_REQUIRE(nothing_to_add || t.axis_dim > 0, HIPCX_INDEX_ERROR, "add_at: cannot index an axis of extent 0");
-        HIPCX_REQUIRE((t.total + 255) / 256 < (1LL << 31), HIPCX_NOT_IMPLEMENTED_ERROR, "add_at: problem too large for one launch");
         // every argument is accepted: only now is out written, first as a copy of a
         int copied = hipcx_copy(a, out, stream);
         HIPCX_REQUIRE(copied == HIPCX_OK, copied, hipcx_last_error());
         if (nothing_to_add) return;
-        dim3 grid(static_cast<unsigned>((t.total + 255) / 256)), block(256);
         VisitDtype(out->dtype, [&](auto tag) {
             using T = typename decltype(tag)::type;
-            hipLaunchKernelGGL(AddAtKernel<T>, grid, block, 0, AsStream(stream), t);
+            ForLaunches(t.total, [&](dim3 grid, int64_t first) { hipLaunchKernelGGL(AddAtKernel<T>, grid, dim3(256), 0, AsStream(stream), t, first); });
         });
         CheckLaunch("add_at");
     });
