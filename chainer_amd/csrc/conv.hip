@@ -223,7 +223,9 @@ int PlanSmallDotSplit(int64_t m, int64_t n, int64_t k, int dtype) {
 }
 
 // Splitting pays for the extra pass over the partial sums (3-4 us) once a tile's reduction takes longer than that on one compute unit:
-// 0.11 us per 128 bytes of its rows in float32 (16 MFMAs), 0.065 us in float16 (fetching the lines).
+// 0.11 us per 128 bytes of its rows in float32 (16 MFMAs), 0.065 us in float16 (fetching the lines).  Against 1 to 32 parts on 206 products of
+// 650 to 10007 terms the choice is within 10 % of the best for 162.  Not so for float16 operands read element by element, 0.27 us per 128 bytes:
+// [20,3500] . [3500,650] row-major takes 17.6 us in one part and 8.1 in eight.
 int SmallDotSplit(int64_t m, int64_t n, int64_t k, int dtype) {
     const int64_t lines = (k * ItemSize(dtype) + 127) / 128;
     return lines >= (dtype == HIPCX_FLOAT32 ? 48 : 80) ? PlanSmallDotSplit(m, n, k, dtype) : 1;
@@ -1535,7 +1537,9 @@ struct GemmPpPlan {
 // The estimates, in us, are fits to measured products.  256 x 256 tiles: 0.85 for a chunk of 32 k, 5 for a tile's start and end, one tile at a time on
 // a compute unit, the result at 5 TB/s (nothing else runs meanwhile), partial sums written and read at 4 TB/s, staging at 3.5 TB/s.  The 128 x 128
 // kernel: 450 TFLOP/s on rows of 16-byte pieces, 350 of 8.  The 32 x 32 tiles of small outputs: 130, a third of it for operands read element by element.
-// The large tiles have to win by a fifth.
+// The large tiles have to win by a fifth.  Against every choice on 84 products (28 shapes in three layouts) the one made is within 10 % of the best
+// for 62.  Farthest off: a round of large tiles that is not full is priced too high ([1793,642] . [642,2563] 45.8 us, 24.0 on large tiles), small
+// tiles over operands read element by element too (1024^3 with a row-major b 27.5 us, 15.8 on small tiles).
 GemmPpPlan PlanGemmPp(const hipcx_array* a, const hipcx_array* b, const hipcx_array* out) {
     GemmPpPlan pl;
     static const bool enabled = [] { const char* e = getenv("HIPCX_DOT_PP"); return e == nullptr || e[0] != '0'; }();

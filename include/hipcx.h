@@ -355,7 +355,7 @@ int hipcx_conv_bn_act(const hipcx_array* x, const hipcx_array* w, const hipcx_ar
                       hipcx_scalar eps, const hipcx_array* residual, int relu, const hipcx_array* out, void* workspace,
                       size_t workspace_bytes, void* stream);
 
-/* Opt-in fused entries for two routine chains.  No single kernel of the reference corresponds to either.
+/* Two routine chains as one or two kernels.  No single kernel of the reference corresponds to either.
  *
  * hipcx_log_softmax: LogSoftmax along axis 1 of a 2-D array (CX/routines/reduction.cc:78-92: AMaxKernel, SubtractKernel,
  *   ExpKernel, SumKernel, LogKernel, AddKernel, SubtractKernel -- 5 reads and 3 writes of the array) as one read and one
