@@ -591,17 +591,18 @@ struct XentPlan {
     size_t Bytes() const { return nseg > 1 ? static_cast<size_t>(blocks) * 3 * sizeof(double) : blocks > 1 ? static_cast<size_t>(blocks) * 2 * sizeof(double) : 0; }
 };
 
-// Rows of at most 64 elements or 4 KB, 8 KB where there are four for every compute unit: XentKernel.  A row takes a group of lanes 1 us
-// and more, a second launch 2: the batch is one workgroup's alone while that means no more than two rows one after the other of 16 lanes
-// each, or one of 64 ([256,10] 6.9 us alone, 6.0 in two launches; [64,1000] 15 and 6.5).  Else a workgroup of four waves to every four
-// (16 short) rows, up to eight to a compute unit.
+// Rows of at most 64 elements or 4 KB, 8 KB where there are four for every compute unit: XentKernel.  One workgroup does the batch alone
+// while that costs no more than a second launch and the memory for partial sums between the two, 2 us on the device and 5 on the host:
+// [512,10] float32 9.7 us alone, 6.0 in two; [256,40] 7.3, [64,256] 8.1, [32,1000] 9.4 against 6.0-6.5.  Else a workgroup of four waves
+// to every four (16 short) rows, up to eight to a compute unit.
 // Longer rows: a workgroup each once there is one for every compute unit ([20000,1500] float32 would take 71 us so, 38 as waves), else
 // segments of 8 KB and more, up to four to a compute unit ([1,1000000] with 4 KB: 21 us, 11 with 8: the merge is one workgroup's).
 XentPlan PlanXent(int64_t rows, int64_t n, int64_t item) {
     XentPlan pl;
     if (n <= 64 || n * item <= (rows >= 4 * NumCUs() ? 8192 : 4096)) {
         const int64_t lpr = n <= 64 ? 16 : 64;
-        if (rows * lpr > (n <= 64 ? 2048 : 1024)) pl.blocks = static_cast<int>(std::min<int64_t>((rows * lpr + 255) / 256, int64_t{8} * NumCUs()));
+        const int64_t alone = n <= 16 ? 512 : n <= 64 ? 256 : n <= 256 ? 64 : 32;  // rows
+        if (rows > alone) pl.blocks = static_cast<int>(std::min<int64_t>((rows * lpr + 255) / 256, int64_t{8} * NumCUs()));
         return pl;
     }
     if (rows >= NumCUs()) {

@@ -30,7 +30,8 @@ def test_softmax_cross_entropy(dt, rows, cols):
 @pytest.mark.parametrize('dt', ['float16', 'float32', 'float64'])
 @pytest.mark.parametrize('rows,cols', [(64, 100), (65, 100), (256, 16), (257, 16), (5, 511), (5, 513), (3, 1024), (3, 1025), (2, 2049), (70, 2051),
                                        (1, 16385), (2, 40003), (255, 3000), (256, 3001), (258, 33001), (1, 700001),
-                                       (1030, 1025), (1030, 2047), (1030, 2049)])
+                                       (1030, 1025), (1030, 2047), (1030, 2049), (512, 10), (513, 10), (256, 40), (257, 40), (64, 256), (65, 256), (32, 257),
+                                       (33, 257)])
 def test_softmax_cross_entropy_of_long_rows(dt, rows, cols):
     """Rows in a wave's registers, in a workgroup's, in segments of several; rows that start anywhere, labels at their ends."""
     import chainer_amd as chx
