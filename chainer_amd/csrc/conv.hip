@@ -346,10 +346,12 @@ SmallDotPath PlanSmallDot(const hipcx_array* a, const hipcx_array* b, SmallDotAr
 // Bytes of partial sums for a small product: only tiles are split along the reduction.
 size_t SmallDotWorkspace(const hipcx_array* a, const hipcx_array* b, int dtype) {
     if (dtype != HIPCX_FLOAT16 && dtype != HIPCX_FLOAT32) return 0;
+    const size_t bytes = SmallDotPartialBytes(a->shape[0], b->shape[1], a->shape[1], dtype);
+    if (bytes == 0) return 0;  // most products
     SmallDotArgs p{};
     int a_mode = 0, b_mode = 0;
     const SmallDotPath path = dtype == HIPCX_FLOAT16 ? PlanSmallDot<half_t>(a, b, &p, &a_mode, &b_mode) : PlanSmallDot<float>(a, b, &p, &a_mode, &b_mode);
-    return path == kSmallDotTiles ? SmallDotPartialBytes(a->shape[0], b->shape[1], a->shape[1], dtype) : 0;
+    return path == kSmallDotTiles ? bytes : 0;
 }
 
 // Small-output matrix products (small_dot.h).  Returns false when the problem does not qualify.  `partial` holds
