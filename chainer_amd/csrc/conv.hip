@@ -11,6 +11,7 @@
 #include "gemm_pp.h"
 #include "igemm.h"
 #include "igemm_pipe.h"
+#include "igemm_split.h"
 #include "layout_kernels.h"
 #include "nchw_conv.h"
 #include "pw_conv.h"
@@ -57,24 +58,6 @@ struct ProfileScope {
     }
 };
 
-// Raises a kernel's dynamic LDS limit when a launch needs more than it has been given so far.  The limit is a property of the
-// function on one device; several host threads may launch the same kernel, so the bookkeeping is per kernel instantiation
-// (the Tag type), per device, and serialised (the reference serialises its launchers on a mutex too, CX/cuda/elementwise.cuh:38).
-template <typename Tag>
-void EnsureDynamicLds(const void* kernel, int lds_bytes) {
-    constexpr int kMaxDevices = 64;
-    static std::mutex mu;
-    static int configured[kMaxDevices] = {};
-    int dev = 0;
-    HIPCX_CHECK_HIP(hipGetDevice(&dev));
-    HIPCX_REQUIRE(dev >= 0 && dev < kMaxDevices, HIPCX_DEVICE_ERROR, "device index out of range");
-    std::lock_guard<std::mutex> lock(mu);
-    if (lds_bytes > configured[dev]) {
-        HIPCX_CHECK_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes));
-        configured[dev] = lds_bytes;
-    }
-}
-
 template <typename T, int WM, int WN, bool PM>
 void LaunchShape(IGemmArgs<T> p, bool fast16, bool fast8, hipStream_t stream) {
     constexpr int BM = 64 * WM, BN = 64 * WN;
@@ -100,6 +83,13 @@ void LaunchShape(IGemmArgs<T> p, bool fast16, bool fast8, hipStream_t stream) {
     double x_elems = static_cast<double>(p.N) * (p.xsN > 0 ? p.xsN : 1);
     bool fits32 = x_elems < 2147483647.0 && static_cast<double>(p.K) * p.wsK < 2147483647.0;
     static const bool use_pipe = [] { const char* e = getenv("HIPCX_IGEMM_PIPE"); return e != nullptr && e[0] == '1'; }();
+    // float32 on the bfloat16 pipes wherever its layout allows.  us before -> after: [4480,650] . [650,10000] 593 -> 398, [4480,10000] . [10000,650]
+    // 704 -> 441, [4096,4096]^2 1123 -> 734, [8192,100] . [100,3000] 76 -> 47; 3x3 convolutions of 256 images 64 -> 64 at 32^2 234 -> 167,
+    // 128 -> 128 at 16^2 204 -> 148, 256 -> 256 at 8^2 224 -> 156.  Relative error (2-norm) against 64 bits: 4.57e-7 -> 3.89e-7, 1.04e-6 -> 9.3e-7,
+    // 1.15e-6 -> 1.0e-6, 1.8e-7 -> 1.5e-7; 4.24e-7 -> 3.57e-7, 5.88e-7 -> 5.02e-7, 8.07e-7 -> 6.96e-7.
+    static const bool use_split = [] { const char* e = getenv("HIPCX_IGEMM_SPLIT"); return e == nullptr || e[0] != '0'; }();
+    bool split = false;
+    if constexpr (sizeof(T) == 4) split = use_split && (fast16 || fast8) && IGemmSplit<WM, WN>(p, fast16 ? 16 : 8, PM, grid, stream);
     HIPCX_REQUIRE(p.batch == 0 || ((fast16 || fast8) && !PM), HIPCX_NOT_IMPLEMENTED_ERROR, "batched products need operands in the MFMA layout");
     if ((fast16 || fast8) && fits32 && use_pipe && p.batch == 0) {
         constexpr int lds_bytes = PipeLdsBytes<T, WM, WN, PM>();
@@ -114,6 +104,8 @@ void LaunchShape(IGemmArgs<T> p, bool fast16, bool fast8, hipStream_t stream) {
             EnsureDynamicLds<Tag8>(reinterpret_cast<const void*>(kern), lds_bytes);
             hipLaunchKernelGGL(kern, grid, block, lds_bytes, stream, p);
         }
+    } else if (split) {
+        // on the bfloat16 pipes
     } else if (fast16) {
         hipLaunchKernelGGL((IGemmFastKernel<T, WM, WN, 16, PM>), grid, block, 0, stream, p);
     } else if (fast8) {
@@ -1466,6 +1458,25 @@ int hipcx_conv_bn_act(const hipcx_array* x, const hipcx_array* w, const hipcx_ar
 }  // extern "C"
 
 namespace {
+// Matrix products with few 128x128 output tiles and a long reduction axis (weight gradients: M x N = filters, reduction = batch x
+// pixels): slices of the reduction run as separate workgroups.  Returns the number of slices (1: no split).
+int PlanSplitK(int64_t m, int64_t n, int64_t k, int dtype) {
+    static const bool enabled = [] { const char* e = getenv("HIPCX_DOT_SPLITK"); return e == nullptr || e[0] != '0'; }();
+    if (!enabled || (dtype != HIPCX_FLOAT16 && dtype != HIPCX_FLOAT32)) return 1;
+    const int64_t tiles = ((m + 127) / 128) * ((n + 127) / 128);
+    const int64_t steps = k * ItemSize(dtype) / 128;  // reduction steps of 128 bytes per row
+    if (k < 4096 || tiles > NumCUs() || m * n < 64 * 64 || steps < 16) return 1;  // up to one tile per compute unit: a second workgroup per unit still hides latency
+    int64_t s = (2 * NumCUs() + tiles - 1) / tiles;
+    static const int64_t min_steps = [] { const char* e = getenv("HIPCX_DOT_SPLITK_MINSTEPS"); int v = e ? atoi(e) : 0; return v >= 1 && v <= 4096 ? v : 8; }();
+    if (s > steps / min_steps) s = steps / min_steps;  // a slice of fewer steps costs more in partial sums than it gains
+    static const int64_t max_slices = [] { const char* e = getenv("HIPCX_DOT_SPLITK_MAX"); int v = e ? atoi(e) : 0; return v >= 2 && v <= 1024 ? v : 256; }();
+    if (s > max_slices) s = max_slices;
+    return s < 2 ? 1 : static_cast<int>(s);
+}
+size_t SplitKBytes(int64_t m, int64_t n, int slices) { return slices > 1 ? static_cast<size_t>(slices) * m * n * sizeof(float) : 0; }
+}  // namespace
+
+namespace {
 // The MFMA kernels read both operands with the reduction index k as the unit-stride axis, rows 16-byte aligned.  An operand
 // laid out otherwise (a plain row-major b, a transposed a, odd pitches) is first copied into that layout -- one pass over
 // the operand instead of an element-gather kernel for the whole product.
@@ -1492,9 +1503,12 @@ DotStaging PlanDotStaging(const hipcx_array* a, const hipcx_array* b, const hipc
     const bool a_fast = OperandIsFast(a->data, a->strides[0], a->strides[1], k, it);
     const bool b_fast = OperandIsFast(b->data, b->strides[1], b->strides[0], k, it);
     if (a_fast && b_fast) return st;
-    // worth it only when the product is large against the copies; small outputs have their own kernel (any layout)
-    if (2.0 * m * n * k < 2e8) return st;
-    if (SmallDotShape(m, n, k)) return st;
+    // worth it only when the product is large against the copies; small outputs have their own kernel (any layout), which takes elements as they
+    // lie but at the float pipe's rate: from 7 GFLOP on a float32 product whose reduction is split is faster staged, on the bfloat16 pipes
+    // ([1000,8192]^T . [8192,1000] 217 -> 155 us, [1000,4500]^T . [4500,784] 117 -> 110; [500,8192]^T . [8192,500] would go from 60 to 74).
+    const double flops = 2.0 * m * n * k;
+    if (flops < 2e8) return st;
+    if (SmallDotShape(m, n, k) && !(out->dtype == HIPCX_FLOAT32 && flops >= 7e9 && PlanSplitK(m, n, k, out->dtype) > 1)) return st;
     const int64_t epv = 16 / it;
     st.kpad = (k + epv - 1) / epv * epv;
     // a changed pitch on one side needs the same (zero-padded) k extent on the other
@@ -1504,25 +1518,6 @@ DotStaging PlanDotStaging(const hipcx_array* a, const hipcx_array* b, const hipc
     st.b_bytes = st.b ? RoundUpTo(static_cast<size_t>(n * st.kpad * it), 256) : 0;
     return st;
 }
-}  // namespace
-
-namespace {
-// Matrix products with few 128x128 output tiles and a long reduction axis (weight gradients: M x N = filters, reduction = batch x
-// pixels): slices of the reduction run as separate workgroups.  Returns the number of slices (1: no split).
-int PlanSplitK(int64_t m, int64_t n, int64_t k, int dtype) {
-    static const bool enabled = [] { const char* e = getenv("HIPCX_DOT_SPLITK"); return e == nullptr || e[0] != '0'; }();
-    if (!enabled || (dtype != HIPCX_FLOAT16 && dtype != HIPCX_FLOAT32)) return 1;
-    const int64_t tiles = ((m + 127) / 128) * ((n + 127) / 128);
-    const int64_t steps = k * ItemSize(dtype) / 128;  // reduction steps of 128 bytes per row
-    if (k < 4096 || tiles > NumCUs() || m * n < 64 * 64 || steps < 16) return 1;  // up to one tile per compute unit: a second workgroup per unit still hides latency
-    int64_t s = (2 * NumCUs() + tiles - 1) / tiles;
-    static const int64_t min_steps = [] { const char* e = getenv("HIPCX_DOT_SPLITK_MINSTEPS"); int v = e ? atoi(e) : 0; return v >= 1 && v <= 4096 ? v : 8; }();
-    if (s > steps / min_steps) s = steps / min_steps;  // a slice of fewer steps costs more in partial sums than it gains
-    static const int64_t max_slices = [] { const char* e = getenv("HIPCX_DOT_SPLITK_MAX"); int v = e ? atoi(e) : 0; return v >= 2 && v <= 1024 ? v : 256; }();
-    if (s > max_slices) s = max_slices;
-    return s < 2 ? 1 : static_cast<int>(s);
-}
-size_t SplitKBytes(int64_t m, int64_t n, int slices) { return slices > 1 ? static_cast<size_t>(slices) * m * n * sizeof(float) : 0; }
 }  // namespace
 
 namespace {

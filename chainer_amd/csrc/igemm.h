@@ -15,9 +15,29 @@
 // padded by 16 bytes so that the 16-byte fragment reads of 16 consecutive rows hit distinct banks.
 #pragma once
 
+#include <mutex>
+
 #include "common.h"
 
 namespace hipcx {
+
+// Raises a kernel's dynamic LDS limit when a launch needs more than it has been given so far.  The limit is a property of the
+// function on one device; several host threads may launch the same kernel, so the bookkeeping is per kernel instantiation
+// (the Tag type), per device, and serialised (the reference serialises its launchers on a mutex too, CX/cuda/elementwise.cuh:38).
+template <typename Tag>
+void EnsureDynamicLds(const void* kernel, int lds_bytes) {
+    constexpr int kMaxDevices = 64;
+    static std::mutex mu;
+    static int configured[kMaxDevices] = {};
+    int dev = 0;
+    HIPCX_CHECK_HIP(hipGetDevice(&dev));
+    HIPCX_REQUIRE(dev >= 0 && dev < kMaxDevices, HIPCX_DEVICE_ERROR, "device index out of range");
+    std::lock_guard<std::mutex> lock(mu);
+    if (lds_bytes > configured[dev]) {
+        HIPCX_CHECK_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes));
+        configured[dev] = lds_bytes;
+    }
+}
 
 template <typename T>
 struct IGemmArgs {
@@ -75,6 +95,10 @@ template <>
 struct BytesOf<8> {
     using type = Bytes8;
 };
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t MakeRsrc(const void* ptr, unsigned bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(ptr), 0, static_cast<int>(bytes), 0x00020000);
+}
 
 // XCD-aware tile order: hardware deals consecutive workgroup ids round-robin to the 8 XCDs, each
 // with its own L2.  Remap so that every XCD walks a contiguous range of tiles; with the channel

@@ -77,10 +77,6 @@ struct NchwConvArgs {
     int out_ev;   // pixels per output store: the largest of 8, 4, 2, 1 that divides P (a run then stays inside one image)
 };
 
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t MakeRsrc(const void* ptr, unsigned bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(ptr), 0, static_cast<int>(bytes), 0x00020000);
-}
-
 template <int N>
 struct alignas(2 * N) PVecH {
     half_t e[N];

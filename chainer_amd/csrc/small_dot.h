@@ -16,7 +16,7 @@
 // Rows / columns beyond M / N and the tail of K are served as zeros by the buffer bounds check or explicit masks.
 #pragma once
 
-#include "nchw_conv.h"
+#include "igemm.h"
 
 namespace hipcx {
 

@@ -1,0 +1,89 @@
+"""float32 products and convolutions on the bfloat16 matrix pipes (igemm_split.hip): edges of tiles and steps, rows of 8- and 16-byte pieces, split
+reductions, both orientations of the result, and operands whose tile is computed again on the float pipe."""
+import numpy as np
+import pytest
+
+import chainer_amd as chx
+
+pytestmark = pytest.mark.gpu
+
+# A sum of K float products in any order, each and each partial sum rounded once, is within K 2^-24 of the sum of magnitudes (to first order); what the
+# split leaves out of a product is below 2^-25 of it.
+_EPS = 2.0 ** -24
+
+
+def _check(got, x, w):
+    x, w = x.astype(np.float64), w.astype(np.float64)
+    bound = (x.shape[1] + 4) * _EPS * (np.abs(x) @ np.abs(w.T)) + 1e-300
+    np.testing.assert_array_less(np.abs(got.astype(np.float64) - x @ w.T), bound)
+
+
+@pytest.mark.parametrize('m,k,n', [(2048, 64, 1024), (2049, 650, 1153), (1793, 66, 1025), (4000, 17 * 2, 700), (4097, 2, 640), (1500, 4098, 1300), (300, 4096, 300)])
+def test_products(m, k, n):
+    rng = np.random.default_rng(k)
+    # magnitudes over thirty powers of two: every part of an operand matters
+    x = rng.standard_normal((m, k), dtype=np.float32) * np.exp2(rng.integers(-15, 16, (m, k))).astype(np.float32)
+    w = rng.standard_normal((n, k), dtype=np.float32)
+    _check(chx.linear(chx.array(x), chx.array(w)).get(), x, w)
+    xt = chx.array(np.ascontiguousarray(x.T)).T  # laid out anew
+    _check(chx.linear(xt, chx.array(w)).get(), x, w)
+
+
+def test_reduction_of_transposed_operands_is_split():
+    rng = np.random.default_rng(1)
+    x, g = rng.standard_normal((6001, 1000), dtype=np.float32), rng.standard_normal((6001, 700), dtype=np.float32)
+    _check(chx.dot(chx.array(x).T, chx.array(g)).get(), x.T, g.T)
+
+
+@pytest.mark.parametrize('shape,filters,kernel,stride,pad', [
+    ((16, 16, 33, 31), 64, 3, 1, 1), ((16, 32, 17, 17), 130, 3, 2, 1), ((8, 48, 20, 20), 96, 5, 1, 2), ((64, 20, 28, 28), 72, 1, 1, 0),
+    ((3, 64, 40, 40), 256, (1, 3), 1, (0, 1)), ((40, 64, 9, 9), 70, 2, 1, 0)])
+def test_convolutions(shape, filters, kernel, stride, pad):
+    rng = np.random.default_rng(filters)
+    kh, kw = (kernel, kernel) if isinstance(kernel, int) else kernel
+    ph, pw = (pad, pad) if isinstance(pad, int) else pad
+    x = rng.standard_normal(shape, dtype=np.float32)
+    w = rng.standard_normal((filters, shape[1], kh, kw), dtype=np.float32)
+    got = chx.conv(chx.array(x), chx.array(w), None, stride, pad).get()
+    padded = np.pad(x, ((0, 0), (0, 0), (ph, ph), (pw, pw)))
+    windows = np.lib.stride_tricks.sliding_window_view(padded, (kh, kw), (2, 3))[:, :, ::stride, ::stride]  # [n, c, oh, ow, kh, kw]
+    n, _, oh, ow = windows.shape[:4]
+    assert got.shape == (n, filters, oh, ow)
+    rows = windows.transpose(0, 2, 3, 1, 4, 5).reshape(n * oh * ow, -1)
+    _check(got.transpose(0, 2, 3, 1).reshape(n * oh * ow, filters), rows, w.reshape(filters, -1))
+
+
+@pytest.mark.parametrize('value', [np.inf, -np.inf, np.nan, 3.4e38, -3.39e38, 1e-37, 2.0 ** -149, 2.0 ** -111])
+def test_values_that_do_not_split(value):
+    """One such value among ordinary ones, and a row of nothing else: finite results are as close as any, the others the same."""
+    rng = np.random.default_rng(3)
+    m, k, n = 2100, 130, 1100
+    x = rng.standard_normal((m, k), dtype=np.float32)
+    w = rng.standard_normal((n, k), dtype=np.float32)
+    x[5, 7] = value
+    x[700] = value
+    w[:, 7] *= 0.5
+    w[300] = 0
+    w[301] = 0
+    w[301, 7] = 1
+    got = chx.linear(chx.array(x), chx.array(w)).get().astype(np.float64)
+    with np.errstate(all='ignore'):
+        exact = x.astype(np.float64) @ w.T.astype(np.float64)
+        magnitude = np.abs(x).astype(np.float64) @ np.abs(w.T).astype(np.float64)
+        bound = (k + 4) * _EPS * magnitude + 2 * k * 2.0 ** -150  # each product and sum also rounds to a multiple of 2^-149
+    special = ~np.isfinite(exact)
+    np.testing.assert_array_equal(np.isnan(got)[special], np.isnan(exact)[special])
+    np.testing.assert_array_equal(got[special & ~np.isnan(exact)], exact[special & ~np.isnan(exact)])
+    inside = magnitude < 3.4e38  # no sum of any of the products overflows
+    np.testing.assert_array_less(np.abs(got - exact)[inside], bound[inside])
+    overflows = np.isfinite(exact) & (np.abs(exact) > 3.5e38)
+    assert not np.isfinite(got[overflows]).any()
+
+
+def test_sums_that_overflow_in_part():
+    """A product whose upper parts alone are beyond the largest float, but whose value is not."""
+    x, w = np.zeros((2048, 64), np.float32), np.zeros((1024, 64), np.float32)
+    x[:, 3], w[:, 3] = np.float32(2 - 2 ** -9) * np.float32(2) ** 100, np.float32(2) ** 27  # bfloat16(x) rounds up to a power of two
+    got = chx.linear(chx.array(x), chx.array(w)).get()
+    np.testing.assert_array_equal(got, np.full_like(got, x[0, 3] * w[0, 3]))
+    assert np.isfinite(got).all()
