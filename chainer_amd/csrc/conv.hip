@@ -1183,21 +1183,6 @@ void CheckConv(const hipcx_array* x, const hipcx_array* w, const hipcx_array* b,
 
 }  // namespace
 
-int DotPartSplits(int64_t m, int64_t n, int64_t k) {
-    // M <= 4 rows have a kernel of their own, GFLOPs the one for whole lines
-    return SmallDotShape(m, n, k) && m > 4 && 2.0 * m * n * k < 1e9 ? PlanSmallDotSplit(m, n, k, HIPCX_FLOAT32) : 1;
-}
-
-void DotParts(const hipcx_array* a, const hipcx_array* b, float* parts, int splits, hipStream_t stream) {
-    SmallDotArgs p{};
-    int a_mode = 0, b_mode = 0;
-    HIPCX_REQUIRE(SmallDotOperands<float>(a, b, &p, &a_mode, &b_mode), HIPCX_NOT_IMPLEMENTED_ERROR, "DotParts: operands out of range");
-    p.ksplit = splits;
-    p.partial = parts;
-    ProfileScope prof(stream, 2.0 * p.M * p.N * p.K, 4.0 * (static_cast<double>(p.M) * p.K + static_cast<double>(p.K) * p.N + static_cast<double>(p.M) * p.N * splits));
-    LaunchSmallDot<float>(p, a_mode, b_mode, 1, stream);
-}
-
 bool DotSeveral(const hipcx_array* a0, int64_t a_distance, const hipcx_array* b, const hipcx_array* const* outs, int n, hipStream_t stream) {
     const int64_t M = a0->shape[0], K = a0->shape[1], N = b->shape[1];
     SmallDotArgs p{};

@@ -3,8 +3,8 @@
 // v_mfma_f32_32x32x16_bf16 does sixteen times the multiply-adds of v_mfma_f32_32x32x2_f32 in a clock.  A float is the sum of three
 // bfloat16 numbers, exactly: x1 = bf16(x), x2 = bf16(x - x1), x3 = x - x1 - x2 (24 significant bits = 3 x 8; rounding to nearest leaves
 // remainders of at most half a unit, which have 16 and 8 bits).  Of the nine products of two such sums six are computed, smallest
-// first, x3 w1, x1 w3, x2 w2, x2 w1, x1 w2, x1 w1, into one float accumulator; what is left out is below 2^-25 of x w, less than the rounding of
-// one float product, and of either sign.  A bfloat16 product is exact in float32, so the only roundings are the accumulator's, and those are
+// first, x3 w1, x1 w3, x2 w2, x2 w1, x1 w2, x1 w1, into one float accumulator; what is left out is at most 2^-23 of x w and 2^-27 in the mean, below the
+// mean rounding of a float product, and of either sign.  A bfloat16 product is exact in float32, so the only roundings are the accumulator's, and those are
 // fewer than the float pipe's (six per 16 terms instead of one per term).  Against 64-bit sums the results are closer than the float pipe's: see
 // LaunchShape.
 //

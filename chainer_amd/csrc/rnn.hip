@@ -3,22 +3,23 @@
 // directions, with the gradients of a forward pass that kept its reserve.
 //
 // The forward pass computes what the routine composition computes (GruImpl / LstmImpl / RnnImpl, n_step_rnn.cc:57-131; the layer
-// and direction wiring of NStepRnnImpl, :362-426).  Per layer and direction:
-//   * the x-side matrices are stacked once into [G*H][in] (G gates, gate-major rows) and every time step's input projection is one
-//     product  XW = X_all [rows, in] . Wx^T  over the rows of all steps (rows = sum of the steps' batch sizes);
-//   * a time step is the recurrent product  HW = h[:Bt] . Wh^T  and one cell kernel that adds the biases, applies the gate
-//     functions and updates h (and c) in place for the Bt rows the step holds; rows beyond Bt keep their state, as in
-//     OneDirectionalLoop (:133-175).  The backward direction walks the steps from the last to the first on its own state.
-//   * the outputs go to columns [d*H, (d+1)*H) of the layer's output rows, which are the next layer's input (the Concatenate of
+// and direction wiring of NStepRnnImpl, :362-426).  A time step of a layer-direction -- its products and its cells -- is one launch (RnnStepKernel), shared
+// by all layer-directions that can advance at that point: both directions of a layer, or all layers of a one-directional network as a wavefront
+// (layer l at step s - l).  Rows beyond a step's batch keep their state, as in OneDirectionalLoop (:133-175); the backward direction walks the
+// steps from the last to the first on its own state.
+//   * Small launches take the products with the layer's input along; else they are one product  XW = X_all [rows, in] . Wx^T  over the rows of
+//     all steps of a layer (rows = sum of the steps' batch sizes).
+//   * The state before a step is the output of the step before, where it lies; hy and cy are updated in place.
+//   * The outputs go to columns [d*H, (d+1)*H) of the layer's output rows, which are the next layer's input (the Concatenate of
 //     :398-404), or to the caller's ys[t] for the top layer.
-// With a reserve (training) the cell kernel also stores what the gradient needs: the gate activations, the state rows before the
-// step, and the outputs of the lower layers.  The one-direction LSTM without reserve is handed to hipcx_n_step_lstm (lstm.hip), which
-// keeps the gates in MFMA accumulators.
+// With a reserve (training) the steps also store what the gradient needs: the gate activations, the state rows before the
+// step, and the outputs of the lower layers.  Large one-direction LSTMs without reserve are handed to hipcx_n_step_lstm (lstm.hip).
 //
-// The backward pass is backpropagation through time written out over the same buffers: per step one cell-gradient kernel (gate
-// pre-activation gradients from dh, dc, dy and the saved activations), one product with Wh for dh of the step before; per layer
+// The backward pass is backpropagation through time written out over the same buffers, the same layer-directions together: per step one
+// cell-gradient kernel (gate pre-activation gradients from dh, dc, dy and the saved activations) and one launch of products (RnnBackKernel: with Wh for
+// dh of the step before; in a wavefront with Wx too, for dy of the layer below); per layer
 // and direction the weight gradients as products over all rows at once (dWx[g] = dG[:, g]^T . X_all, dWh[g] = dG[:, g]^T . Hprev_all),
-// the bias gradients as column sums, and the input gradient dX_all = dG . Wx, which is the dy of the layer below.
+// the bias gradients as column sums, and the input gradient dX_all = dG . Wx of the lowest layer (without a wavefront of every layer).
 // The reference's cuda backend gets these numbers from cuDNN (CX/cuda/cuda_device/rnn.cu); every other backend from autograd over the
 // composition.  Sums run in another order than either: equal to float32 tolerance.
 #include <algorithm>
@@ -27,6 +28,7 @@
 
 #include "common.h"
 #include "dot_parts.h"
+#include "small_dot.h"
 
 extern "C" {
 size_t hipcx_n_step_lstm_workspace_size(int n_layers, const hipcx_array* hx, const hipcx_array* const* xs, int n_steps);
@@ -43,150 +45,482 @@ enum RnnMode { kGru = 0, kLstm = 1, kRnn = 2 };  // the `mode` argument of RnnKe
 int NumGates(int mode) { return mode == kLstm ? 4 : (mode == kGru ? 3 : 1); }        // matrices per side; ws holds twice as many
 int ReserveGates(int mode) { return mode == kRnn ? 1 : 4; }  // saved values per unit and row: LSTM i f g o; GRU r z n hh; RNN h
 
-struct CellArgs {
-    int relu;
-    int Bt, H;
-    const float* xw;    // [Bt][G*H]: this step's rows of the input projection
-    const float* hw;    // [splits][Bt][G*H]: h . Wh^T in parts of the reduction
-    int splits;
-    const float* bx;    // [G*H]
-    const float* bh;    // [G*H]
-    float* h;           // [B][H] state, rows < Bt updated in place
-    float* c;           // [B][H] (LSTM)
-    float* y;           // output rows
-    int64_t y_stride;
-    float* gates;       // reserve, this step's rows [Bt][GR*H]; null: inference
-    float* hprev;       // reserve [Bt][H]
-    float* cprev;       // reserve [Bt][H] (LSTM)
-};
-
 __device__ __forceinline__ float Sigmoid(float v) { return 1.0f / (1.0f + expf(-v)); }  // CX/routines/activation.cc:74-78
 
-// sum[g] of the parts p[s * stride + g * H], s < splits, in that order.
-template <int G>
-__device__ __forceinline__ void SumParts(const float* p, int splits, int64_t stride, int H, float (&sum)[G]) {
-#pragma unroll
-    for (int g = 0; g < G; ++g) sum[g] = 0.f;
-#pragma unroll 4
-    for (int s = 0; s < splits; ++s) {
-#pragma unroll
-        for (int g = 0; g < G; ++g) sum[g] += p[s * stride + g * H];
-    }
+// Keeps a value that is the same for all lanes in scalar registers from here on.  Kernel arguments are otherwise fetched where they are first used, one
+// dependent round trip to memory after the other; pinned together they come in one.
+template <typename... T>
+__device__ __forceinline__ void Pin(const T&... values) {
+    (..., [](const auto& v) { asm volatile("" ::"s"(v)); }(values));
 }
 
-// A step's cells.  Bound by the latency of a few loads; the product h . Wh^T arrives in the parts its reduction was split into.
+constexpr int kMaxJobs = 4;    // layer-directions that a launch advances by a step; their descriptors travel as kernel arguments
+constexpr int kStepWaves = 8;  // per workgroup; they split the reduction
+constexpr int kChunk = 32;     // terms of it that a wave takes at a time: a line of 128 bytes per row
+constexpr int kPitch = 4 * kChunk + 16;  // bytes of a staged row: fragment reads of 16 rows start in different banks
+constexpr int kPartFloats = 32 * 33;     // a wave's sums
+
+struct __attribute__((packed, aligned(4))) Floats4 {
+    Bytes16 v;
+};
+__device__ __forceinline__ Bytes16 Load4(const float* p) { return reinterpret_cast<const Floats4*>(p)->v; }
+
+// The run of 4 terms from k on of a row of K.  Of a row of 4 and more, what lies beyond it comes from in front of the run instead (16 bytes inside the
+// row, wherever k is); KeepRun drops that.  Shorter rows are read one by one.
+__device__ __forceinline__ int RunStart(int k, int K) { return K >= 4 ? min(k, K - 4) : k; }
+// The runs from k on of four rows.
+__device__ __forceinline__ void LoadRuns(const float* const (&row)[4], int k, int K, Bytes16 (&v)[4]) {
+    if (K >= 4) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = Load4(row[j] + RunStart(k, K));
+        return;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[j][e] = __float_as_uint(row[j][min(k + e, K - 1)]);
+}
+__device__ __forceinline__ void KeepRun(Bytes16& v, int k, int K) {
+    const int at = RunStart(k, K);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = (at + e >= k) & (at + e < K) ? v[e] : 0u;
+}
+
+// One step of one layer-direction.  Matrices are dense [units][columns], vectors dense.
+struct StepJob {
+    const float* x;  // [bt] rows of the layer's input; null: its projection is in xw
+    int64_t x_stride;
+    int in;
+    int bt;
+    int prev_rows;       // the state before the step of rows below it is in h_prev (the outputs of the step before), of the others in h0
+    const float* h_prev;
+    int64_t h_prev_stride;
+    const float* h0;     // [B][H]
+    const float* xw;     // [bt][G*H]
+    const float* wx[4];  // per gate
+    const float* wh[4];
+    const float* bx[4];
+    const float* bh[4];
+    float* y;            // [bt] output rows
+    int64_t y_stride;
+    float* hy;           // the state after the last step of each row: rows < bt are written
+    int64_t hy_row, hy_col;
+    float* cy;           // (LSTM) the same, and the state before the step
+    int64_t cy_row, cy_col;
+    float* gates;        // reserve, this step's rows [bt][GR*H]; null: inference
+    float* hprev;        // reserve [bt][H]
+    float* cprev;        // reserve [bt][H] (LSTM)
+};
+
+struct StepArgs {
+    int relu;
+    int H;
+    StepJob job[kMaxJobs];
+};
+
+// The products x . Wx^T and h . Wh^T of a step and the cells in one launch.  A workgroup owns 32 rows and the gates of 8 (RNN: 32) units, so that the
+// sums of its eight waves, which split the reduction, meet in LDS and the cells run on them: gate pre-activations never reach memory.  GRU keeps
+// the sums of the two sides apart, as its last gate needs them (and takes the columns of a fourth gate, which nobody reads).
+// A wave reads whole lines (8 lanes to a row) two chunks ahead and turns them round in LDS of its own: read straight into the MFMA layout, 32 rows to
+// an instruction, the loads alone took 14 us a step at [20,1300] . [1300,2600], 64 clocks an instruction.
+// Bound by latency (launch, first loads, the waves' sums): a launch advances every layer-direction that can go (blockIdx.y), and whatever the cells
+// read is loaded ahead of the products.  Two layers of 650 LSTM units, 20 rows, 35 steps: 70 launches
+// each of a product (4.9 us) and of cells (4.5) -> 36 of 13.4, x's products (88 us) and the packing of the weights included.
 template <int MODE>
-__global__ __launch_bounds__(256) void RnnCellKernel(CellArgs p) {
+__global__ __launch_bounds__(64 * kStepWaves) void RnnStepKernel(StepArgs p) {
     constexpr int G = MODE == kLstm ? 4 : (MODE == kGru ? 3 : 1);
-    const int total = p.Bt * p.H;
-    const int GH = p.H * G;
-    for (int idx = blockIdx.x * 256 + threadIdx.x; idx < total; idx += gridDim.x * 256) {
-        const int r = idx / p.H, u = idx - r * p.H;
-        const float* xw = p.xw + static_cast<int64_t>(r) * GH + u;
-        float hw[G];
-        SumParts<G>(p.hw + static_cast<int64_t>(r) * GH + u, p.splits, static_cast<int64_t>(p.Bt) * GH, p.H, hw);
-        auto pre = [&](int g) { return (xw[g * p.H] + p.bx[g * p.H + u]) + (hw[g] + p.bh[g * p.H + u]); };  // Linear(x) + Linear(h)
-        float* hs = p.h + static_cast<int64_t>(r) * p.H + u;
-        const float h_old = *hs;
+    constexpr int C = G == 1 ? 1 : 4;  // columns of a unit
+    constexpr int UNITS = 32 / C;
+    constexpr int SIDES = MODE == kGru ? 2 : 1;
+    constexpr int CELLS = 32 * UNITS / (64 * kStepWaves) > 1 ? 32 * UNITS / (64 * kStepWaves) : 1;  // of a thread
+    static_assert(SIDES * kPartFloats * 4 <= 2 * 32 * kPitch, "the sums fit the staging areas");
+    __shared__ __align__(16) char lds[kStepWaves * 2 * 32 * kPitch];
+    const StepJob& args = p.job[blockIdx.y];
+    const float* const x_rows = args.x;
+    const float* const xw_rows = args.xw;
+    const float* const h_prev = args.h_prev;
+    const float* const h0 = args.h0;
+    const int64_t x_stride = args.x_stride, h_prev_stride = args.h_prev_stride, y_stride = args.y_stride;
+    const int bt = args.bt, prev_rows = args.prev_rows, in = x_rows != nullptr ? args.in : 0;
+    float *const y = args.y, *const hy = args.hy, *const gates = args.gates, *const hprev = args.hprev;
+    const int64_t hy_row = args.hy_row, hy_col = args.hy_col;
+    float* const cy = MODE == kLstm ? args.cy : nullptr;
+    float* const cprev = MODE == kLstm ? args.cprev : nullptr;
+    const int64_t cy_row = MODE == kLstm ? args.cy_row : 0, cy_col = MODE == kLstm ? args.cy_col : 0;
+    const float *const wx0 = args.wx[0], *const wx1 = args.wx[G > 1], *const wx2 = args.wx[G > 2 ? 2 : 0], *const wx3 = args.wx[G > 3 ? 3 : 0];
+    const float *const wh0 = args.wh[0], *const wh1 = args.wh[G > 1], *const wh2 = args.wh[G > 2 ? 2 : 0], *const wh3 = args.wh[G > 3 ? 3 : 0];
+    const float *const bx0 = args.bx[0], *const bx1 = args.bx[G > 1], *const bx2 = args.bx[G > 2 ? 2 : 0], *const bx3 = args.bx[G > 3 ? 3 : 0];
+    const float *const bh0 = args.bh[0], *const bh1 = args.bh[G > 1], *const bh2 = args.bh[G > 2 ? 2 : 0], *const bh3 = args.bh[G > 3 ? 3 : 0];
+    Pin(x_rows, xw_rows, h_prev, h0, x_stride, h_prev_stride, y_stride, bt, prev_rows, in, y, hy, gates, hprev, hy_row, hy_col, cy, cprev, cy_row, cy_col);
+    Pin(wx0, wx1, wx2, wx3, wh0, wh1, wh2, wh3, bx0, bx1, bx2, bx3, bh0, bh1, bh2, bh3);
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lr = lane & 31, half = lane >> 5;
+    const int H = p.H;
+    const int tiles_m = (bt + 31) / 32, tiles = tiles_m * ((H + UNITS - 1) / UNITS);
+    if (static_cast<int>(blockIdx.x) >= tiles) return;
+    int tm, tn;
+    SmallDotTile(tiles, blockIdx.x, tiles_m, tm, tn);
+
+    // what this thread's cells read
+    float xw[CELLS][G], b_x[CELLS][G], b_h[CELLS][G], h_old[CELLS], c_old[CELLS];
+    auto cell_at = [&](int i, int& r, int& u) {
+        const int e = tid + i * 64 * kStepWaves;
+        r = tm * 32 + e / UNITS, u = tn * UNITS + e % UNITS;
+        return e < 32 * UNITS && r < bt && u < H;
+    };
+    auto state_row = [&](int r) -> const float* { return r < prev_rows ? h_prev + r * h_prev_stride : h0 + static_cast<int64_t>(r) * H; };
+#pragma unroll
+    for (int i = 0; i < CELLS; ++i) {
+        int r, u;
+        if (!cell_at(i, r, u)) continue;
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            xw[i][g] = xw_rows != nullptr ? xw_rows[(static_cast<int64_t>(r) * G + g) * H + u] : 0.f;
+            b_x[i][g] = (g == 0 ? bx0 : (g == 1 ? bx1 : (g == 2 ? bx2 : bx3)))[u];
+            b_h[i][g] = (g == 0 ? bh0 : (g == 1 ? bh1 : (g == 2 ? bh2 : bh3)))[u];
+        }
+        h_old[i] = state_row(r)[u];
+        if constexpr (MODE == kLstm) c_old[i] = cy[r * cy_row + u * cy_col];
+    }
+
+    // ---- products: this lane's piece (4 k) of every eighth row of x and h and of the matrices' rows that are the columns (rows and columns beyond the
+    // problem repeat the last one: nobody reads what comes of them) ----
+    const int piece = (lane & 7) * 4, eighth = lane >> 3;
+    const int gate = eighth % C;  // of this lane's columns j * 8 + eighth
+    const float* const w_x = gate == 0 ? wx0 : (gate == 1 ? wx1 : (gate == 2 ? wx2 : wx3));
+    const float* const w_h = gate == 0 ? wh0 : (gate == 1 ? wh1 : (gate == 2 ? wh2 : wh3));
+    const float *x_row[4], *h_row[4], *wx_row[4], *wh_row[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int row = min(tm * 32 + j * 8 + eighth, bt - 1);
+        const int64_t unit = min(tn * UNITS + (j * 8 + eighth) / C, H - 1);
+        x_row[j] = x_rows + row * x_stride;
+        h_row[j] = state_row(row);
+        wx_row[j] = w_x + unit * in;
+        wh_row[j] = w_h + unit * H;
+    }
+    const int chunks_x = (in + kChunk - 1) / kChunk, chunks = chunks_x + (H + kChunk - 1) / kChunk;
+    const int per_wave = (chunks + kStepWaves - 1) / kStepWaves;
+    const int begin = min(chunks, wave * per_wave), n = min(chunks, begin + per_wave) - begin;
+    float16_t acc[SIDES];
+#pragma unroll
+    for (int s = 0; s < SIDES; ++s)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[s][v] = 0.f;
+    Bytes16 av[2][4], bv[2][4];
+    auto load = [&](int st, int c) {
+        const int i = begin + c;
+        if (i < chunks_x) {
+            LoadRuns(x_row, i * kChunk + piece, in, av[st]);
+            LoadRuns(wx_row, i * kChunk + piece, in, bv[st]);
+        } else {
+            LoadRuns(h_row, (i - chunks_x) * kChunk + piece, H, av[st]);
+            LoadRuns(wh_row, (i - chunks_x) * kChunk + piece, H, bv[st]);
+        }
+    };
+    char* const stage = lds + wave * 2 * 32 * kPitch;
+    auto multiply = [&](int st, int c) {
+        const int i = begin + c;
+        const bool x = i < chunks_x;
+        const int k = (x ? i : i - chunks_x) * kChunk, K = x ? in : H;
+        if (k + kChunk > K) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) KeepRun(av[st][j], k + piece, K), KeepRun(bv[st][j], k + piece, K);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            *reinterpret_cast<Bytes16*>(stage + (j * 8 + eighth) * kPitch + piece * 4) = av[st][j];
+            *reinterpret_cast<Bytes16*>(stage + (32 + j * 8 + eighth) * kPitch + piece * 4) = bv[st][j];
+        }
+        if (c + 2 < n) load(st, c + 2);
+        __builtin_amdgcn_wave_barrier();
+        Bytes16 fa[4], fb[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            fa[q] = *reinterpret_cast<const Bytes16*>(stage + lr * kPitch + (2 * q + half) * 16);
+            fb[q] = *reinterpret_cast<const Bytes16*>(stage + (32 + lr) * kPitch + (2 * q + half) * 16);
+        }
+        if (SIDES == 1 || x) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) MfmaTile<float>(fa[q], fb[q], acc[0]);
+        } else {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) MfmaTile<float>(fa[q], fb[q], acc[SIDES - 1]);
+        }
+        __builtin_amdgcn_wave_barrier();
+    };
+    if (n > 0) load(0, 0);
+    if (n > 1) load(1, 1);
+    for (int c = 0; c < n; c += 2) {
+        multiply(0, c);
+        if (c + 1 < n) multiply(1, c + 1);
+    }
+    __syncthreads();  // the staging areas become the sums
+    float* const part = reinterpret_cast<float*>(lds);
+    // lane holds column lr, rows 8 * (v / 4) + 4 * half + v % 4
+#pragma unroll
+    for (int s = 0; s < SIDES; ++s)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) part[(s * kStepWaves + wave) * kPartFloats + (8 * (v / 4) + 4 * half + v % 4) * 33 + lr] = acc[s][v];
+    __syncthreads();
+
+#pragma unroll
+    for (int i = 0; i < CELLS; ++i) {
+        int r, u;
+        if (!cell_at(i, r, u)) continue;
+        const int at = (r - tm * 32) * 33 + (u - tn * UNITS) * C;
+        float sum[SIDES][G];
+#pragma unroll
+        for (int s = 0; s < SIDES; ++s)
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                sum[s][g] = 0.f;
+#pragma unroll
+                for (int w = 0; w < kStepWaves; ++w) sum[s][g] += part[(s * kStepWaves + w) * kPartFloats + at + g];
+            }
+        if constexpr (MODE == kGru) {
+#pragma unroll
+            for (int g = 0; g < G; ++g) xw[i][g] += sum[0][g];
+        }
+        const int64_t idx = static_cast<int64_t>(r) * H + u;
+        auto pre = [&](int g) { return (xw[i][g] + b_x[i][g]) + (sum[SIDES - 1][g] + b_h[i][g]); };  // Linear(x) + Linear(h)
         float h_new;
         if constexpr (MODE == kLstm) {
-            float* cs = p.c + static_cast<int64_t>(r) * p.H + u;
-            const float c_old = *cs;
             const float gi = Sigmoid(pre(0)), gf = Sigmoid(pre(1)), gg = tanhf(pre(2)), go = Sigmoid(pre(3));
-            const float c_new = gg * gi + gf * c_old;
+            const float c_new = gg * gi + gf * c_old[i];
             h_new = go * tanhf(c_new);
-            *cs = c_new;
-            if (p.gates != nullptr) {
-                float* q = p.gates + static_cast<int64_t>(r) * 4 * p.H + u;
-                q[0] = gi, q[p.H] = gf, q[2 * p.H] = gg, q[3 * p.H] = go;
-                p.cprev[idx] = c_old;
+            cy[r * cy_row + u * cy_col] = c_new;
+            if (gates != nullptr) {
+                float* q = gates + static_cast<int64_t>(r) * 4 * H + u;
+                q[0] = gi, q[H] = gf, q[2 * H] = gg, q[3 * H] = go;
+                cprev[idx] = c_old[i];
             }
         } else if constexpr (MODE == kGru) {
             const float gr = Sigmoid(pre(0)), gz = Sigmoid(pre(1));
-            const float hh = hw[2] + p.bh[2 * p.H + u];
-            const float gn = tanhf((xw[2 * p.H] + p.bx[2 * p.H + u]) + gr * hh);
-            h_new = (1.0f - gz) * gn + gz * h_old;
-            if (p.gates != nullptr) {
-                float* q = p.gates + static_cast<int64_t>(r) * 4 * p.H + u;
-                q[0] = gr, q[p.H] = gz, q[2 * p.H] = gn, q[3 * p.H] = hh;
+            const float hh = sum[SIDES - 1][2] + b_h[i][2];
+            const float gn = tanhf((xw[i][2] + b_x[i][2]) + gr * hh);
+            h_new = (1.0f - gz) * gn + gz * h_old[i];
+            if (gates != nullptr) {
+                float* q = gates + static_cast<int64_t>(r) * 4 * H + u;
+                q[0] = gr, q[H] = gz, q[2 * H] = gn, q[3 * H] = hh;
             }
         } else {
             const float s = pre(0);
             h_new = p.relu ? fmaxf(s, 0.0f) : tanhf(s);
-            if (p.gates != nullptr) p.gates[idx] = h_new;
+            if (gates != nullptr) gates[idx] = h_new;
         }
-        if (p.gates != nullptr) p.hprev[idx] = h_old;
-        *hs = h_new;
-        p.y[static_cast<int64_t>(r) * p.y_stride + u] = h_new;
+        if (gates != nullptr) hprev[idx] = h_old[i];
+        hy[r * hy_row + u * hy_col] = h_new;
+        y[r * y_stride + u] = h_new;
     }
 }
 
-struct CellGradArgs {
-    int relu;
-    int Bt, H;
-    const float* dy;  // this step's rows of the gradient of the layer's output, this direction's columns
+struct CellGradJob {
+    int bt;
+    const float* dy;     // this step's rows of the gradient of the layer's output, this direction's columns: dy_splits parts dy_part floats apart
     int64_t dy_stride;
-    float* dh;        // [B][H]: the part of the gradient of the state after the step that did not pass through Wh in the step behind it;
-                      // out, the same for the step before (GRU: dh * z, else 0)
+    int dy_splits;
+    int64_t dy_part;
+    float* dh;           // [B][H]: the part of the gradient of the state after the step that did not pass through Wh in the step behind it;
+                         // out, the same for the step before (GRU: dh * z, else 0)
     const float* parts;  // [splits][part_rows][H]: the other part, dGh . Wh of the step behind, in parts of its reduction
     int splits, part_rows;
-    float* dc;        // [B][H] (LSTM), updated in place
+    float* dc;           // [B][H] (LSTM), updated in place
     const float* gates;
     const float* hprev;
     const float* cprev;
-    float* dgx;       // [Bt][G*H]: gradient of x . Wx^T + bx
-    float* dgh;       // [Bt][G*H]: gradient of h . Wh^T + bh (the same array as dgx unless GRU)
+    float* dgx;          // [bt][G*H]: gradient of x . Wx^T + bx
+    float* dgh;          // [bt][G*H]: gradient of h . Wh^T + bh (the same array as dgx unless GRU)
 };
 
-// Rows from Bt to part_rows, which the step does not hold, only take in their parts.
+struct CellGradArgs {
+    int relu;
+    int H;
+    CellGradJob job[kMaxJobs];
+};
+
+// sum of p[s * stride], s < splits, in that order
+__device__ __forceinline__ float SumParts(const float* p, int splits, int64_t stride) {
+    float sum = 0.f;
+#pragma unroll 8
+    for (int s = 0; s < splits; ++s) sum += p[s * stride];
+    return sum;
+}
+
+// Rows from bt to part_rows, which the step does not hold, only take in their parts.  blockIdx.y: the layer-direction.
 template <int MODE>
 __global__ __launch_bounds__(256) void RnnCellGradKernel(CellGradArgs p) {
-    const int total = max(p.Bt, p.part_rows) * p.H;
+    const CellGradJob& args = p.job[blockIdx.y];
+    const int bt = args.bt, splits = args.splits, part_rows = args.part_rows, dy_splits = args.dy_splits;
+    const int64_t dy_stride = args.dy_stride, dy_part = args.dy_part;
+    const float *const dy = args.dy, *const parts = args.parts, *const gates = args.gates, *const hprev = args.hprev, *const cprev = args.cprev;
+    float *const dh_state = args.dh, *const dc_state = args.dc, *const dgx = args.dgx, *const dgh = args.dgh;
+    Pin(bt, splits, part_rows, dy_splits, dy_stride, dy_part, dy, parts, gates, hprev, cprev, dh_state, dc_state, dgx, dgh);
+    const int H = p.H;
+    const int total = max(bt, part_rows) * H;
     for (int idx = blockIdx.x * 256 + threadIdx.x; idx < total; idx += gridDim.x * 256) {
-        const int r = idx / p.H, u = idx - r * p.H;
-        float* dhs = p.dh + static_cast<int64_t>(r) * p.H + u;
+        const int r = idx / H, u = idx - r * H;
+        float* dhs = dh_state + idx;
         float after = *dhs;
-        if (r < p.part_rows) {
-            float sum[1];
-            SumParts<1>(p.parts + idx, p.splits, static_cast<int64_t>(p.part_rows) * p.H, p.H, sum);
-            after += sum[0];
-        }
-        if (r >= p.Bt) {
+        if (r < part_rows) after += SumParts(parts + idx, splits, static_cast<int64_t>(part_rows) * H);
+        if (r >= bt) {
             *dhs = after;
             continue;
         }
-        const float dh = after + p.dy[static_cast<int64_t>(r) * p.dy_stride + u];
+        const float dh = after + SumParts(dy + r * dy_stride + u, dy_splits, dy_part);
         if constexpr (MODE == kLstm) {
-            const float* q = p.gates + static_cast<int64_t>(r) * 4 * p.H + u;
-            const float gi = q[0], gf = q[p.H], gg = q[2 * p.H], go = q[3 * p.H];
-            const float c_old = p.cprev[idx];
+            const float* q = gates + static_cast<int64_t>(r) * 4 * H + u;
+            const float gi = q[0], gf = q[H], gg = q[2 * H], go = q[3 * H];
+            const float c_old = cprev[idx];
             const float tc = tanhf(gg * gi + gf * c_old);
-            float* dcs = p.dc + static_cast<int64_t>(r) * p.H + u;
+            float* dcs = dc_state + idx;
             const float dc = *dcs + dh * go * (1.0f - tc * tc);
-            float* g = p.dgx + static_cast<int64_t>(r) * 4 * p.H + u;
+            float* g = dgx + static_cast<int64_t>(r) * 4 * H + u;
             g[0] = dc * gg * gi * (1.0f - gi);
-            g[p.H] = dc * c_old * gf * (1.0f - gf);
-            g[2 * p.H] = dc * gi * (1.0f - gg * gg);
-            g[3 * p.H] = dh * tc * go * (1.0f - go);
+            g[H] = dc * c_old * gf * (1.0f - gf);
+            g[2 * H] = dc * gi * (1.0f - gg * gg);
+            g[3 * H] = dh * tc * go * (1.0f - go);
             *dcs = dc * gf;
             *dhs = 0.0f;
         } else if constexpr (MODE == kGru) {
-            const float* q = p.gates + static_cast<int64_t>(r) * 4 * p.H + u;
-            const float gr = q[0], gz = q[p.H], gn = q[2 * p.H], hh = q[3 * p.H];
-            const float h_old = p.hprev[idx];
+            const float* q = gates + static_cast<int64_t>(r) * 4 * H + u;
+            const float gr = q[0], gz = q[H], gn = q[2 * H], hh = q[3 * H];
+            const float h_old = hprev[idx];
             const float dn_pre = dh * (1.0f - gz) * (1.0f - gn * gn);
             const float dz_pre = dh * (h_old - gn) * gz * (1.0f - gz);
             const float dr_pre = dn_pre * hh * gr * (1.0f - gr);
-            float* gx = p.dgx + static_cast<int64_t>(r) * 3 * p.H + u;
-            float* gh = p.dgh + static_cast<int64_t>(r) * 3 * p.H + u;
-            gx[0] = dr_pre, gx[p.H] = dz_pre, gx[2 * p.H] = dn_pre;
-            gh[0] = dr_pre, gh[p.H] = dz_pre, gh[2 * p.H] = dn_pre * gr;
+            float* gx = dgx + static_cast<int64_t>(r) * 3 * H + u;
+            float* gh = dgh + static_cast<int64_t>(r) * 3 * H + u;
+            gx[0] = dr_pre, gx[H] = dz_pre, gx[2 * H] = dn_pre;
+            gh[0] = dr_pre, gh[H] = dz_pre, gh[2 * H] = dn_pre * gr;
             *dhs = dh * gz;
         } else {
-            const float h_new = p.gates[idx];
-            p.dgx[idx] = p.relu ? (h_new > 0.0f ? dh : 0.0f) : dh * (1.0f - h_new * h_new);
+            const float h_new = gates[idx];
+            dgx[idx] = p.relu ? (h_new > 0.0f ? dh : 0.0f) : dh * (1.0f - h_new * h_new);
             *dhs = 0.0f;
         }
+    }
+}
+
+// What a step's gate gradients mean for the state before it and, where the layer below runs a step behind, for the layer's input.
+struct BackJob {
+    int bt;
+    const float* dgh;    // [bt][G*H]
+    const float* dgx;
+    const float* wh[4];  // per gate [H][H]
+    const float* wx[4];  // per gate [H][in]
+    int in;              // 0: the input's gradient is not wanted
+    float* dh_parts;     // [splits][bt][H]
+    float* dx_parts;     // [splits][bt][in]
+};
+
+struct BackArgs {
+    int G, H;
+    int subs;  // parts of a gate's reduction; splits = G * subs
+    BackJob job[kMaxJobs];
+};
+
+// The products dGh . Wh and dGx . Wx of a step, in parts of the reduction which the cell kernel adds up: a workgroup owns 32 rows, 32 columns and a
+// part of one gate's units, its eight waves split that.  The rows come as whole lines, turned round in LDS; the matrices, whose rows are k, element by
+// element with the columns across the lanes: whole lines too, already in the MFMA layout.  Bound by latency like the forward step.
+__global__ __launch_bounds__(64 * kStepWaves) void RnnBackKernel(BackArgs p) {
+    __shared__ __align__(16) char lds[kStepWaves * 32 * kPitch];
+    const BackJob& args = p.job[blockIdx.y];
+    const int bt = args.bt, in = args.in;
+    const float *const dgh = args.dgh, *const dgx = args.dgx;
+    const float *const wh0 = args.wh[0], *const wh1 = args.wh[1], *const wh2 = args.wh[2], *const wh3 = args.wh[3];
+    const float *const wx0 = args.wx[0], *const wx1 = args.wx[1], *const wx2 = args.wx[2], *const wx3 = args.wx[3];
+    float *const dh_parts = args.dh_parts, *const dx_parts = args.dx_parts;
+    Pin(bt, in, dgh, dgx, wh0, wh1, wh2, wh3, wx0, wx1, wx2, wx3, dh_parts, dx_parts);
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lr = lane & 31, half = lane >> 5;
+    const int H = p.H, splits = p.G * p.subs;
+    const int tiles_m = (bt + 31) / 32, tiles_h = (H + 31) / 32, tiles_n = tiles_h + (in + 31) / 32;
+    const int tiles = tiles_m * tiles_n;
+    if (static_cast<int>(blockIdx.x) >= tiles * splits) return;
+    const int split = blockIdx.x / tiles;
+    int tm, tn;
+    SmallDotTile(tiles, blockIdx.x - split * tiles, tiles_m, tm, tn);
+    const bool state = tn < tiles_h;
+    const int N = state ? H : in;
+    const int n0 = (state ? tn : tn - tiles_h) * 32;
+    const int gate = split / p.subs, sub = split - gate * p.subs;
+    const float* const w_h = gate == 0 ? wh0 : (gate == 1 ? wh1 : (gate == 2 ? wh2 : wh3));
+    const float* const w_x = gate == 0 ? wx0 : (gate == 1 ? wx1 : (gate == 2 ? wx2 : wx3));
+    const int piece = (lane & 7) * 4, eighth = lane >> 3, col = min(n0 + lr, N - 1);
+    const float* a[4];  // every eighth row
+#pragma unroll
+    for (int j = 0; j < 4; ++j) a[j] = (state ? dgh : dgx) + (static_cast<int64_t>(min(tm * 32 + j * 8 + eighth, bt - 1)) * p.G + gate) * H;
+    const float* const b = (state ? w_h : w_x) + col;
+
+    const int chunks = (H + kChunk - 1) / kChunk, per_sub = (chunks + p.subs - 1) / p.subs;
+    const int sub_begin = min(chunks, sub * per_sub), sub_end = min(chunks, sub_begin + per_sub);
+    const int per_wave = (sub_end - sub_begin + kStepWaves - 1) / kStepWaves;
+    const int begin = min(sub_end, sub_begin + wave * per_wave), end = min(sub_end, begin + per_wave);
+    float16_t acc;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[v] = 0.f;
+    char* const stage = lds + wave * 32 * kPitch;
+    Bytes16 av[2][4], bv[2][4];
+    auto load = [&](int st, int c) {
+        const int k = c * kChunk;
+        LoadRuns(a, k + piece, H, av[st]);
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) bv[st][q][e] = __float_as_uint(b[static_cast<int64_t>(min(k + (2 * q + half) * 4 + e, H - 1)) * N]);
+    };
+    auto multiply = [&](int st, int c) {
+        const int k = c * kChunk;
+        if (k + kChunk > H) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                KeepRun(av[st][j], k + piece, H);
+                // to where the matrices' elements are
+                Bytes16 v = av[st][j];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int shift = k + piece - RunStart(k + piece, H);  // the run was read that much too early
+                    av[st][j][e] = e + shift < 4 ? (shift == 0 ? v[e] : (shift == 1 ? v[(e + 1) & 3] : (shift == 2 ? v[(e + 2) & 3] : v[(e + 3) & 3]))) : 0u;
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) bv[st][q][e] = k + (2 * q + half) * 4 + e < H ? bv[st][q][e] : 0u;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) *reinterpret_cast<Bytes16*>(stage + (j * 8 + eighth) * kPitch + piece * 4) = av[st][j];
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const Bytes16 fa = *reinterpret_cast<const Bytes16*>(stage + lr * kPitch + (2 * q + half) * 16);
+            MfmaTile<float>(fa, bv[st][q], acc);
+        }
+        if (c + 2 < end) load(st, c + 2);
+        __builtin_amdgcn_wave_barrier();
+    };
+    if (begin < end) load(0, begin);
+    if (begin + 1 < end) load(1, begin + 1);
+    for (int c = begin; c < end; c += 2) {
+        multiply(0, c);
+        if (c + 1 < end) multiply(1, c + 1);
+    }
+    __syncthreads();  // the staging areas become the sums
+    float* const part = reinterpret_cast<float*>(lds);
+#pragma unroll
+    for (int v = 0; v < 16; ++v) part[wave * kPartFloats + (8 * (v / 4) + 4 * half + v % 4) * 33 + lr] = acc[v];
+    __syncthreads();
+    float* const out = (state ? dh_parts : dx_parts) + static_cast<int64_t>(split) * bt * N;
+    for (int e = tid; e < 32 * 32; e += 64 * kStepWaves) {
+        const int row = e >> 5, c = e & 31;
+        if (tm * 32 + row >= bt || n0 + c >= N) continue;
+        float s = 0.f;
+#pragma unroll
+        for (int w = 0; w < kStepWaves; ++w) s += part[w * kPartFloats + row * 33 + c];
+        out[static_cast<int64_t>(tm * 32 + row) * N + n0 + c] = s;
     }
 }
 
@@ -320,11 +654,6 @@ public:
         HIPCX_REQUIRE(scratch_off_ + need <= bytes_, HIPCX_CHAINERX_ERROR, "n_step_rnn workspace too small for a sum");
         CheckStatus(hipcx_sum(&a, &axis, 1, &out, base_ + scratch_off_, bytes_ - scratch_off_, stream_));
     }
-    // a . b in splits > 1 parts (DotPartSplits) at `parts`, or whole there
-    void DotInParts(const hipcx_array& a, const hipcx_array& b, float* parts, int splits) {
-        if (splits == 1) return Dot(a, b, Matrix(parts, a.shape[0], b.shape[1], b.shape[1]));
-        if (!dry_) DotParts(&a, &b, parts, splits, hip_stream());
-    }
     // outs[i] = a_i . b for left operands `distance` elements apart
     void DotEach(const hipcx_array& a0, int64_t distance, const hipcx_array& b, const hipcx_array* const* outs, int n) {
         if (!dry_ && DotSeveral(&a0, distance, &b, outs, n, hip_stream())) return;
@@ -340,6 +669,7 @@ public:
         copies_.push_back(out);
     }
     void FlushCopies() {
+        if (copies_.empty()) return;
         std::vector<const hipcx_array*> from, to;
         for (size_t i = 0; i < copies_.size(); i += 2) {
             from.push_back(&copies_[i]);
@@ -366,39 +696,23 @@ private:
     std::vector<hipcx_array> copies_;
 };
 
-// Most floats that DotInParts needs over the steps of a pass for [bt, k] . [k, n].
-int64_t PartFloats(const RnnPlan& pl, int64_t n, int64_t k) {
-    int64_t most = 0;
-    for (int64_t bt : pl.bt) most = std::max(most, DotPartSplits(bt, n, k) * bt * n);
-    return most;
+// The x-side matrices of a layer-direction stacked gate-major into [G*H][in]: rows [g*H, (g+1)*H) are ws[idx][g].
+float* PackInputWeights(Pass& pass, const RnnPlan& pl, const hipcx_array* const* ws, int idx) {
+    const int64_t in = pl.In(idx / pl.D);
+    float* const packed = pass.Take(pl.G * pl.H * in);
+    if (pass.dry()) return packed;
+    for (int g = 0; g < pl.G; ++g) pass.Copy(*ws[idx * 2 * pl.G + g], Matrix(packed + g * pl.H * in, pl.H, in, in));
+    return packed;
 }
 
-struct PackedWeights {
-    std::vector<float*> wx, wh, bx, bh;  // per layer-direction: [G*H][in], [G*H][H], [G*H], [G*H]
-};
-
-// Stacks the matrices and biases of every layer-direction, gate-major: rows [g*H, (g+1)*H) of wx are ws[idx][g], of wh ws[idx][G + g].
-// bs null: the matrices alone, which is all the backward pass reads.
-PackedWeights PackWeights(Pass& pass, const RnnPlan& pl, const hipcx_array* const* ws, const hipcx_array* const* bs) {
-    PackedWeights pw;
-    const int G = pl.G;
-    for (int idx = 0; idx < pl.L * pl.D; ++idx) {
-        const int64_t in = pl.In(idx / pl.D);
-        pw.wx.push_back(pass.Take(G * pl.H * in));
-        pw.wh.push_back(pass.Take(G * pl.H * pl.H));
-        pw.bx.push_back(bs != nullptr ? pass.Take(G * pl.H) : nullptr);
-        pw.bh.push_back(bs != nullptr ? pass.Take(G * pl.H) : nullptr);
-        if (pass.dry()) continue;
-        for (int g = 0; g < 2 * G; ++g) {
-            const hipcx_array* w = ws[idx * 2 * G + g];
-            const bool xside = g < G;
-            const int64_t cols = xside ? in : pl.H;
-            float* wdst = (xside ? pw.wx[idx] : pw.wh[idx]) + static_cast<int64_t>(g % G) * pl.H * cols;
-            pass.Copy(*w, Matrix(wdst, pl.H, cols, cols));
-            if (bs != nullptr) pass.Copy(*bs[idx * 2 * G + g], Vector((xside ? pw.bx[idx] : pw.bh[idx]) + static_cast<int64_t>(g % G) * pl.H, pl.H));
-        }
-    }
-    return pw;
+// An array's data where it is dense, else of a dense copy (there is always room for one: the caller's strides are not known to a dry run).
+const float* Dense(Pass& pass, const hipcx_array* a) {
+    int64_t n = 1;
+    for (int i = 0; i < a->ndim; ++i) n *= a->shape[i];
+    float* const copy = pass.Take(n);
+    if (pass.dry() || IsContiguous(a)) return static_cast<const float*>(a->data);
+    pass.Copy(*a, a->ndim == 1 ? Vector(copy, n) : Matrix(copy, a->shape[0], a->shape[1], a->shape[1]));
+    return copy;
 }
 
 void CheckParameters(const RnnPlan& pl, const hipcx_array* const* ws, const hipcx_array* const* bs, const char* what) {
@@ -453,90 +767,210 @@ unsigned CellBlocks(int64_t items) {
     return static_cast<unsigned>(b > cap ? cap : (b < 1 ? 1 : b));
 }
 
+// Layer-directions that advance together are the two directions of a layer or, as a wavefront, all layers of a one-directional network, layer l a step
+// behind layer l - 1.  The latter needs the products with the layers' inputs to be part of the steps, which then read twice as much but are fewer: it
+// pays to the largest launches tried, four workgroups (32 rows, 8 or 32 units each) to a compute unit (us, forward and backward, products over
+// all steps -> in the steps: 2 x 650 LSTM units, 20 rows, 35 steps 1671 -> 1190; 2 x 649, 128 rows 3883 -> 3486; 3 x 600 GRU units, 128 rows 3235 ->
+// 2566).  Two directions advance together either way, and only small launches gain (2 x 200 GRU units, 20 rows 806 -> 804; 2 x 400, 64 rows 1971 -> 2118).
+bool Narrow(const RnnPlan& pl) {
+    const int64_t units = pl.G == 1 ? 32 : 8, rows = (*std::max_element(pl.bt.begin(), pl.bt.end()) + 31) / 32;
+    const int64_t jobs = pl.D == 2 ? 2 : pl.L, most = pl.D == 2 ? NumCUs() / 2 : 4 * NumCUs();
+    return jobs <= kMaxJobs && rows * ((pl.H + units - 1) / units) * jobs <= most;
+}
+
+// f(jobs), for each launch of a pass: the (layer, direction, step) that it runs.  A direction's step s is time step s or T - 1 - s.
+struct Turn {
+    int layer, direction, s;
+};
+template <typename F>
+void ForEachTurn(const RnnPlan& pl, bool wavefront, int first_layer, int last_layer, F&& f) {
+    std::vector<Turn> turns;
+    if (wavefront) {
+        for (int s = 0; s < pl.T + pl.L - 1; ++s) {
+            turns.clear();
+            for (int l = std::max(0, s - pl.T + 1); l < pl.L && l <= s; ++l) turns.push_back({l, 0, s - l});
+            f(turns);
+        }
+        return;
+    }
+    for (int l = first_layer; l <= last_layer; ++l) {
+        for (int s = 0; s < pl.T; ++s) {
+            turns.clear();
+            for (int d = 0; d < pl.D; ++d) turns.push_back({l, d, s});
+            f(turns);
+        }
+    }
+}
+
 // ---- forward ----
 void RunForward(Pass& pass, const RnnPlan& pl, int activation, const hipcx_array* hx, const hipcx_array* cx, const hipcx_array* const* ws,
                 const hipcx_array* const* bs, const hipcx_array* const* xs, const hipcx_array* hy, const hipcx_array* cy,
                 const hipcx_array* const* ys, char* reserve) {
     const int64_t B = pl.B, H = pl.H, GH = pl.G * H, DH = pl.D * H, rows = pl.rows;
-    PackedWeights pw = PackWeights(pass, pl, ws, bs);
-    float* x_all = pass.Take(rows * pl.I);
-    float* y_buf[2] = {nullptr, nullptr};
-    if (reserve == nullptr && pl.L > 1) {
-        y_buf[0] = pass.Take(rows * DH);
-        if (pl.L > 2) y_buf[1] = pass.Take(rows * DH);
+    const int chains = pl.L * pl.D;
+    const bool narrow = Narrow(pl), wavefront = narrow && pl.D == 1;
+    std::vector<const float*> wx, wh, bx, bh;
+    for (int idx = 0; idx < chains; ++idx) {
+        for (int g = 0; g < 2 * pl.G; ++g) {
+            (g < pl.G ? wx : wh).push_back(Dense(pass, ws[idx * 2 * pl.G + g]));
+            (g < pl.G ? bx : bh).push_back(Dense(pass, bs[idx * 2 * pl.G + g]));
+        }
     }
-    float* xw_all = pass.Take(rows * GH);
-    float* hw = pass.Take(PartFloats(pl, GH, H));
-    float* h_state = pass.Take(B * H);
-    float* c_state = pl.mode == kLstm ? pass.Take(B * H) : nullptr;
+    float* const x_all = pass.Take(rows * pl.I);
+    std::vector<float*> y_buf;  // outputs of the layers below the top
+    for (int l = 0; l + 1 < pl.L; ++l) {
+        if (reserve != nullptr) y_buf.push_back(reinterpret_cast<float*>(reserve + pl.r_y[l]));
+        else y_buf.push_back(l < 2 || wavefront ? pass.Take(rows * DH) : y_buf[l - 2]);
+    }
+    float* xw_all[2] = {nullptr, nullptr};
+    if (!narrow) {
+        for (int d = 0; d < pl.D; ++d) xw_all[d] = pass.Take(rows * GH);
+    }
+    float* const h0 = pass.Take(chains * B * H);
+    std::vector<float*> wx_packed;
+    for (int idx = 0; idx < chains && !narrow; ++idx) wx_packed.push_back(PackInputWeights(pass, pl, ws, idx));
     pass.StartScratch();
-    for (int t = 0; t < pl.T; ++t) pass.Copy(*xs[t], Matrix(x_all + pl.row_start[t] * pl.I, pl.bt[t], pl.I, pl.I));
-    for (int l = 0; l < pl.L; ++l) {
-        const int64_t in = pl.In(l);
-        const float* x_in = l == 0 ? x_all : (reserve != nullptr ? reinterpret_cast<float*>(reserve + pl.r_y[l - 1]) : y_buf[(l - 1) & 1]);
-        float* y_out = l + 1 == pl.L ? nullptr : (reserve != nullptr ? reinterpret_cast<float*>(reserve + pl.r_y[l]) : y_buf[l & 1]);
-        for (int d = 0; d < pl.D; ++d) {
-            const int idx = l * pl.D + d;
-            pass.Copy(StateSlice(hx, idx), Matrix(h_state, B, H, H));
-            if (pl.mode == kLstm) pass.Copy(StateSlice(cx, idx), Matrix(c_state, B, H, H));
-            pass.FlushCopies();
-            // the input projection of every step at once
-            pass.Dot(Matrix(x_in, rows, in, in), Matrix(pw.wx[idx], in, GH, 1, in), Matrix(xw_all, rows, GH, GH));
-            for (int s = 0; s < pl.T; ++s) {
-                const int t = d == 0 ? s : pl.T - 1 - s;
-                const int64_t bt = pl.bt[t], r0 = pl.row_start[t];
-                const int splits = DotPartSplits(bt, GH, H);
-                pass.DotInParts(Matrix(h_state, bt, H, H), Matrix(pw.wh[idx], H, GH, 1, H), hw, splits);
-                if (pass.dry()) continue;
-                CellArgs a{};
-                a.splits = splits, a.relu = activation == 1;
-                a.Bt = static_cast<int>(bt), a.H = static_cast<int>(H);
-                a.xw = xw_all + r0 * GH;
-                a.hw = hw;
-                a.bx = pw.bx[idx], a.bh = pw.bh[idx];
-                a.h = h_state, a.c = c_state;
-                if (y_out != nullptr) {
-                    a.y = y_out + r0 * DH + d * H;
-                    a.y_stride = DH;
-                } else {
-                    a.y = static_cast<float*>(ys[t]->data) + d * H;
-                    a.y_stride = ys[t]->strides[0] / 4;
-                }
-                if (reserve != nullptr) {
-                    a.gates = reinterpret_cast<float*>(reserve + pl.r_gates[idx]) + r0 * pl.GR * H;
-                    a.hprev = reinterpret_cast<float*>(reserve + pl.r_hprev[idx]) + r0 * H;
-                    a.cprev = pl.mode == kLstm ? reinterpret_cast<float*>(reserve + pl.r_cprev[idx]) + r0 * H : nullptr;
-                }
-                VisitMode(pl.mode, [&](auto mode) {
-                    hipLaunchKernelGGL(RnnCellKernel<decltype(mode)::value>, dim3(CellBlocks(bt * H)), dim3(256), 0, pass.hip_stream(), a);
-                });
-                CheckLaunch("rnn_cell");
+    // the steps read rows of xs where they are if their columns are dense; the products over all steps need them in one array
+    bool x_in_place = narrow;
+    for (int t = 0; t < pl.T; ++t) x_in_place = x_in_place && (xs[t]->strides[1] == 4 || pl.I == 1) && xs[t]->strides[0] % 4 == 0;
+    for (int t = 0; t < pl.T && !x_in_place; ++t) pass.Copy(*xs[t], Matrix(x_all + pl.row_start[t] * pl.I, pl.bt[t], pl.I, pl.I));
+    for (int idx = 0; idx < chains; ++idx) {
+        pass.Copy(StateSlice(hx, idx), Matrix(h0 + idx * B * H, B, H, H));
+        pass.Copy(StateSlice(hx, idx), StateSlice(hy, idx));
+        if (pl.mode == kLstm) pass.Copy(StateSlice(cx, idx), StateSlice(cy, idx));
+    }
+    pass.FlushCopies();
+    // output rows of layer l at step t, direction d's columns, and their stride
+    auto y_at = [&](int l, int d, int t, int64_t* stride) {
+        if (l + 1 < pl.L) {
+            *stride = DH;
+            return y_buf[l] + pl.row_start[t] * DH + d * H;
+        }
+        *stride = ys[t]->strides[0] / 4;
+        return static_cast<float*>(ys[t]->data) + d * H;
+    };
+    std::vector<int64_t> seen(chains, 0);  // rows that some step of a layer-direction has held
+    auto launch = [&](const std::vector<Turn>& turns) {
+        StepArgs a{};
+        a.relu = activation == 1;
+        a.H = static_cast<int>(H);
+        int64_t most = 0;
+        for (size_t i = 0; i < turns.size(); ++i) {
+            const int l = turns[i].layer, d = turns[i].direction, s = turns[i].s, idx = l * pl.D + d;
+            const int t = d == 0 ? s : pl.T - 1 - s;
+            const int64_t bt = pl.bt[t], r0 = pl.row_start[t];
+            StepJob& j = a.job[i];
+            j.bt = static_cast<int>(bt);
+            j.in = static_cast<int>(pl.In(l));
+            if (narrow && l == 0) {
+                j.x = x_in_place ? static_cast<const float*>(xs[t]->data) : x_all + r0 * pl.I;
+                j.x_stride = x_in_place ? xs[t]->strides[0] / 4 : pl.I;
+            } else if (narrow) {
+                j.x = y_at(l - 1, 0, t, &j.x_stride);
+            } else {
+                j.xw = xw_all[d] + r0 * GH;
             }
-            pass.Copy(Matrix(h_state, B, H, H), StateSlice(hy, idx));
-            if (pl.mode == kLstm) pass.Copy(Matrix(c_state, B, H, H), StateSlice(cy, idx));
-            pass.FlushCopies();
+            j.h0 = h0 + idx * B * H;
+            if (s > 0) {
+                const int before = d == 0 ? t - 1 : t + 1;
+                j.prev_rows = static_cast<int>(std::min(bt, pl.bt[before]));
+                j.h_prev = y_at(l, d, before, &j.h_prev_stride);
+                if (const int64_t back = std::min(bt, seen[idx]); back > j.prev_rows) {  // rows that an earlier step held and the last one did not
+                    const hipcx_array state = StateSlice(hy, idx);
+                    hipcx_array from = state;
+                    from.data = static_cast<char*>(state.data) + j.prev_rows * state.strides[0];
+                    from.shape[0] = back - j.prev_rows;
+                    pass.Copy(from, Matrix(h0 + (idx * B + j.prev_rows) * H, back - j.prev_rows, H, H));
+                }
+            }
+            seen[idx] = std::max(seen[idx], bt);
+            for (int g = 0; g < pl.G; ++g) {
+                j.wx[g] = wx[idx * pl.G + g], j.wh[g] = wh[idx * pl.G + g];
+                j.bx[g] = bx[idx * pl.G + g], j.bh[g] = bh[idx * pl.G + g];
+            }
+            j.y = y_at(l, d, t, &j.y_stride);
+            const hipcx_array h_out = StateSlice(hy, idx);
+            j.hy = static_cast<float*>(h_out.data), j.hy_row = h_out.strides[0] / 4, j.hy_col = h_out.strides[1] / 4;
+            if (pl.mode == kLstm) {
+                const hipcx_array c_out = StateSlice(cy, idx);
+                j.cy = static_cast<float*>(c_out.data), j.cy_row = c_out.strides[0] / 4, j.cy_col = c_out.strides[1] / 4;
+            }
+            if (reserve != nullptr) {
+                j.gates = reinterpret_cast<float*>(reserve + pl.r_gates[idx]) + r0 * pl.GR * H;
+                j.hprev = reinterpret_cast<float*>(reserve + pl.r_hprev[idx]) + r0 * H;
+                j.cprev = pl.mode == kLstm ? reinterpret_cast<float*>(reserve + pl.r_cprev[idx]) + r0 * H : nullptr;
+            }
+            const int64_t units = pl.G == 1 ? 32 : 8;
+            most = std::max(most, (bt + 31) / 32 * ((H + units - 1) / units));
+        }
+        pass.FlushCopies();
+        if (pass.dry()) return;
+        VisitMode(pl.mode, [&](auto mode) {
+            hipLaunchKernelGGL(RnnStepKernel<decltype(mode)::value>, dim3(static_cast<unsigned>(most), static_cast<unsigned>(turns.size())),
+                               dim3(64 * kStepWaves), 0, pass.hip_stream(), a);
+        });
+        CheckLaunch("rnn_step");
+    };
+    if (narrow) {
+        ForEachTurn(pl, wavefront, 0, pl.L - 1, launch);
+    } else {
+        for (int l = 0; l < pl.L; ++l) {
+            const int64_t in = pl.In(l);
+            const float* const x_in = l == 0 ? x_all : y_buf[l - 1];
+            // the input projection of every step at once
+            for (int d = 0; d < pl.D; ++d) {
+                pass.Dot(Matrix(x_in, rows, in, in), Matrix(wx_packed[l * pl.D + d], in, GH, 1, in), Matrix(xw_all[d], rows, GH, GH));
+            }
+            ForEachTurn(pl, false, l, l, launch);
         }
     }
     pass.CheckFits();
 }
 
 // ---- backward ----
+// Parts of a gate's units in RnnBackKernel: two workgroups to a compute unit while each has 96 units or more (2 x 650 LSTM units, 20 rows, whole pass:
+// one workgroup 1383 us, two 1190, four 1251; from 200 units on, 3 x 200 LSTM units, 128 rows: 2095, from 96 on 1960).
+int BackSubs(const RnnPlan& pl, bool wavefront) {
+    const int64_t rows = (*std::max_element(pl.bt.begin(), pl.bt.end()) + 31) / 32;
+    const int64_t tiles = rows * (wavefront ? 2 * pl.L - 1 : pl.D) * ((pl.H + 31) / 32) * pl.G;
+    return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(2 * NumCUs() / tiles, pl.H / 96)));
+}
+
 void RunBackward(Pass& pass, const RnnPlan& pl, int activation, const hipcx_array* const* ws, const hipcx_array* const* bs,
                  const hipcx_array* const* xs, const hipcx_array* dhy, const hipcx_array* dcy, const hipcx_array* const* dys, const char* reserve,
                  const hipcx_array* dhx, const hipcx_array* dcx, const hipcx_array* const* dws, const hipcx_array* const* dbs,
                  const hipcx_array* const* dxs) {
     const int64_t B = pl.B, H = pl.H, GH = pl.G * H, DH = pl.D * H, rows = pl.rows;
-    PackedWeights pw = PackWeights(pass, pl, ws, nullptr);
+    const int chains = pl.L * pl.D;
+    const bool wavefront = Narrow(pl) && pl.D == 1;
+    const int together = wavefront ? pl.L : pl.D;  // layer-directions that advance together
+    const int subs = BackSubs(pl, wavefront), splits = pl.G * subs;
+    const int64_t most_rows = *std::max_element(pl.bt.begin(), pl.bt.end());
+    std::vector<const float*> wx, wh;
+    for (int idx = 0; idx < chains; ++idx) {
+        for (int g = 0; g < 2 * pl.G; ++g) {
+            if (g >= pl.G) wh.push_back(Dense(pass, ws[idx * 2 * pl.G + g]));
+            else wx.push_back(wavefront && idx > 0 ? Dense(pass, ws[idx * 2 * pl.G + g]) : nullptr);
+        }
+    }
+    std::vector<float*> wx_packed(chains, nullptr);  // for the gradients of a layer's input over all steps
+    for (int idx = 0; idx < chains; ++idx) {
+        if (!wavefront || idx == 0) wx_packed[idx] = PackInputWeights(pass, pl, ws, idx);
+    }
     float* x_all = pass.Take(rows * pl.I);
     float* dy_cur = pass.Take(rows * pl.max_in);   // gradient of the current layer's output rows [rows][D*H]
     float* dx_acc = pass.Take(rows * pl.max_in);   // gradient of its input rows [rows][in]
     float* dx_tmp = pl.D == 2 ? pass.Take(rows * pl.max_in) : nullptr;
-    float* dgx_all = pass.Take(rows * GH);
-    float* dgh_all = pl.mode == kGru ? pass.Take(rows * GH) : dgx_all;
-    float* dh = pass.Take(B * H);
-    float* dc = pl.mode == kLstm ? pass.Take(B * H) : nullptr;
-    float* parts = pass.Take(PartFloats(pl, H, GH));
-    float* db = pass.Take(pl.L * pl.D * 2 * GH);
+    std::vector<float*> dgx_all, dgh_all, dh, dc, dh_parts, dx_parts;  // per layer-direction that advances together
+    for (int i = 0; i < together; ++i) {
+        dgx_all.push_back(pass.Take(rows * GH));
+        dgh_all.push_back(pl.mode == kGru ? pass.Take(rows * GH) : dgx_all[i]);
+        dh_parts.push_back(pass.Take(splits * most_rows * H));
+        dx_parts.push_back(wavefront && i > 0 ? pass.Take(splits * most_rows * H) : nullptr);
+    }
+    float* const dh_all = pass.Take(chains * B * H);
+    float* const dc_all = pl.mode == kLstm ? pass.Take(chains * B * H) : nullptr;
+    float* db = pass.Take(chains * 2 * GH);
     pass.StartScratch();
     for (int t = 0; t < pl.T; ++t) pass.Copy(*xs[t], Matrix(x_all + pl.row_start[t] * pl.I, pl.bt[t], pl.I, pl.I));
     for (int t = 0; t < pl.T; ++t) {
@@ -544,75 +978,123 @@ void RunBackward(Pass& pass, const RnnPlan& pl, int activation, const hipcx_arra
         if (dys[t] != nullptr) pass.Copy(*dys[t], dst);
         else pass.Zero(dst);
     }
+    for (int idx = 0; idx < chains; ++idx) {
+        pass.Copy(StateSlice(dhy, idx), Matrix(dh_all + idx * B * H, B, H, H));
+        if (pl.mode != kLstm) continue;
+        if (dcy != nullptr) pass.Copy(StateSlice(dcy, idx), Matrix(dc_all + idx * B * H, B, H, H));
+        else pass.Zero(Matrix(dc_all + idx * B * H, B, H, H));
+    }
+    pass.FlushCopies();
     std::vector<std::pair<hipcx_array, hipcx_array>> db_copies;
-    auto launch_cells = [&](const CellGradArgs& a) {
+    auto launch_cells = [&](const CellGradArgs& a, size_t jobs) {
+        if (pass.dry()) return;
+        int64_t cells = 0;
+        for (size_t i = 0; i < jobs; ++i) cells = std::max(cells, std::max(a.job[i].bt, a.job[i].part_rows) * H);
         VisitMode(pl.mode, [&](auto mode) {
-            const int64_t cells = static_cast<int64_t>(std::max(a.Bt, a.part_rows)) * H;
-            hipLaunchKernelGGL(RnnCellGradKernel<decltype(mode)::value>, dim3(CellBlocks(cells)), dim3(256), 0, pass.hip_stream(), a);
+            hipLaunchKernelGGL(RnnCellGradKernel<decltype(mode)::value>, dim3(CellBlocks(cells), static_cast<unsigned>(jobs)), dim3(256), 0,
+                               pass.hip_stream(), a);
         });
         CheckLaunch("rnn_cell_grad");
     };
-    for (int l = pl.L - 1; l >= 0; --l) {
+    // rows that the step behind a layer-direction's next one left parts for (none behind the last)
+    std::vector<int> part_rows(together, 0);
+    auto slot = [&](const Turn& turn) { return wavefront ? turn.layer : turn.direction; };
+    auto cell_state = [&](CellGradJob& j, int idx, int i) {
+        j.dh = dh_all + idx * B * H;
+        j.dc = pl.mode == kLstm ? dc_all + idx * B * H : nullptr;
+        j.parts = dh_parts[i], j.splits = splits, j.part_rows = part_rows[i];
+    };
+    auto launch = [&](const std::vector<Turn>& turns) {
+        CellGradArgs a{};
+        BackArgs b{};
+        a.relu = activation == 1;
+        a.H = b.H = static_cast<int>(H);
+        b.G = pl.G, b.subs = subs;
+        int64_t most = 0;
+        for (size_t n = 0; n < turns.size(); ++n) {
+            const int l = turns[n].layer, d = turns[n].direction, i = slot(turns[n]), idx = l * pl.D + d;
+            const int s = turns[n].s;
+            const int t = d == 0 ? s : pl.T - 1 - s;
+            const int64_t bt = pl.bt[t], r0 = pl.row_start[t];
+            CellGradJob& j = a.job[n];
+            j.bt = static_cast<int>(bt);
+            cell_state(j, idx, i);
+            if (wavefront && l + 1 < pl.L) {  // the layer above has just left its input's gradient for this step
+                j.dy = dx_parts[l + 1], j.dy_stride = H, j.dy_splits = splits, j.dy_part = bt * H;
+            } else {
+                j.dy = dy_cur + r0 * DH + d * H, j.dy_stride = DH, j.dy_splits = 1;
+            }
+            j.gates = reinterpret_cast<const float*>(reserve + pl.r_gates[idx]) + r0 * pl.GR * H;
+            j.hprev = reinterpret_cast<const float*>(reserve + pl.r_hprev[idx]) + r0 * H;
+            j.cprev = pl.mode == kLstm ? reinterpret_cast<const float*>(reserve + pl.r_cprev[idx]) + r0 * H : nullptr;
+            j.dgx = dgx_all[i] + r0 * GH;
+            j.dgh = dgh_all[i] + r0 * GH;
+            // dh of the state before the step: what the cell left there plus dGh . Wh
+            BackJob& q = b.job[n];
+            q.bt = j.bt;
+            q.dgh = j.dgh, q.dgx = j.dgx;
+            q.in = wavefront && l > 0 ? static_cast<int>(H) : 0;
+            for (int g = 0; g < pl.G; ++g) q.wh[g] = wh[idx * pl.G + g], q.wx[g] = wx[idx * pl.G + g];
+            q.dh_parts = dh_parts[i], q.dx_parts = dx_parts[i];
+            part_rows[i] = j.bt;
+            most = std::max(most, (bt + 31) / 32 * ((H + 31) / 32 + (q.in + 31) / 32) * splits);
+        }
+        launch_cells(a, turns.size());
+        if (pass.dry()) return;
+        hipLaunchKernelGGL(RnnBackKernel, dim3(static_cast<unsigned>(most), static_cast<unsigned>(turns.size())), dim3(64 * kStepWaves), 0,
+                           pass.hip_stream(), b);
+        CheckLaunch("rnn_back");
+    };
+    // the forward turns of layers first .. last (all of them as a wavefront), backwards, and what is left of the last parts
+    auto run = [&](int first, int last) {
+        std::vector<std::vector<Turn>> turns;
+        ForEachTurn(pl, wavefront, first, last, [&](const std::vector<Turn>& t) { turns.push_back(t); });
+        std::fill(part_rows.begin(), part_rows.end(), 0);
+        for (size_t n = turns.size(); n-- > 0;) launch(turns[n]);
+        CellGradArgs a{};
+        a.H = static_cast<int>(H);
+        for (int i = 0; i < together; ++i) cell_state(a.job[i], wavefront ? i : first * pl.D + i, i);
+        launch_cells(a, together);
+    };
+    // parameter gradients of a layer over all rows, and unless `dx` is null those of its input rows there
+    auto finish = [&](int l, float* dx) {
         const int64_t in = pl.In(l);
         const float* x_in = l == 0 ? x_all : reinterpret_cast<const float*>(reserve + pl.r_y[l - 1]);
         for (int d = 0; d < pl.D; ++d) {
-            const int idx = l * pl.D + d;
-            const float* gates = reinterpret_cast<const float*>(reserve + pl.r_gates[idx]);
+            const int idx = l * pl.D + d, i = wavefront ? l : d;
             const float* hprev = reinterpret_cast<const float*>(reserve + pl.r_hprev[idx]);
-            const float* cprev = pl.mode == kLstm ? reinterpret_cast<const float*>(reserve + pl.r_cprev[idx]) : nullptr;
-            pass.Copy(StateSlice(dhy, idx), Matrix(dh, B, H, H));
-            if (pl.mode == kLstm) {
-                if (dcy != nullptr) pass.Copy(StateSlice(dcy, idx), Matrix(dc, B, H, H));
-                else pass.Zero(Matrix(dc, B, H, H));
-            }
-            pass.FlushCopies();
-            CellGradArgs a{};  // the step behind the last one has no parts
-            for (int s = pl.T - 1; s >= 0; --s) {  // the forward order of this direction, backwards
-                const int t = d == 0 ? s : pl.T - 1 - s;
-                const int64_t bt = pl.bt[t], r0 = pl.row_start[t];
-                const int splits = DotPartSplits(bt, H, GH);
-                if (!pass.dry()) {
-                    a.relu = activation == 1;
-                    a.Bt = static_cast<int>(bt), a.H = static_cast<int>(H);
-                    a.dy = dy_cur + r0 * DH + d * H;
-                    a.dy_stride = DH;
-                    a.dh = dh, a.dc = dc;
-                    a.gates = gates + r0 * pl.GR * H;
-                    a.hprev = hprev + r0 * H;
-                    a.cprev = cprev != nullptr ? cprev + r0 * H : nullptr;
-                    a.dgx = dgx_all + r0 * GH;
-                    a.dgh = dgh_all + r0 * GH;
-                    launch_cells(a);
-                }
-                // dh of the state before the step: what the cell left there plus dGh . Wh
-                pass.DotInParts(Matrix(dgh_all + r0 * GH, bt, GH, GH), Matrix(pw.wh[idx], GH, H, H), parts, splits);
-                a.parts = parts, a.splits = splits, a.part_rows = static_cast<int>(bt);
-            }
-            a.Bt = 0;
-            if (!pass.dry()) launch_cells(a);
-            pass.Copy(Matrix(dh, B, H, H), StateSlice(dhx, idx));
-            if (pl.mode == kLstm) pass.Copy(Matrix(dc, B, H, H), StateSlice(dcx, idx));
-            pass.FlushCopies();
-            // parameter gradients over all rows at once: dGx[:, g]^T . x and dGh[:, g]^T . h for all gates g in a launch each
-            pass.DotEach(Matrix(dgx_all, H, rows, 1, GH), H, Matrix(x_in, rows, in, in), dws + idx * 2 * pl.G, pl.G);
-            pass.DotEach(Matrix(dgh_all, H, rows, 1, GH), H, Matrix(hprev, rows, H, H), dws + idx * 2 * pl.G + pl.G, pl.G);
+            // dGx[:, g]^T . x and dGh[:, g]^T . h for all gates g in a launch each
+            pass.DotEach(Matrix(dgx_all[i], H, rows, 1, GH), H, Matrix(x_in, rows, in, in), dws + idx * 2 * pl.G, pl.G);
+            pass.DotEach(Matrix(dgh_all[i], H, rows, 1, GH), H, Matrix(hprev, rows, H, H), dws + idx * 2 * pl.G + pl.G, pl.G);
             // the biases' are column sums of all gates at once; they go to their arrays at the end
             float* const db_x = db + static_cast<int64_t>(idx) * 2 * GH;
-            float* const db_h = dgh_all == dgx_all ? db_x : db_x + GH;
-            pass.SumRows(Matrix(dgx_all, rows, GH, GH), Vector(db_x, GH));
-            if (db_h != db_x) pass.SumRows(Matrix(dgh_all, rows, GH, GH), Vector(db_h, GH));
+            float* const db_h = dgh_all[i] == dgx_all[i] ? db_x : db_x + GH;
+            pass.SumRows(Matrix(dgx_all[i], rows, GH, GH), Vector(db_x, GH));
+            if (db_h != db_x) pass.SumRows(Matrix(dgh_all[i], rows, GH, GH), Vector(db_h, GH));
             for (int g = 0; g < 2 * pl.G; ++g) {
                 db_copies.emplace_back(Vector((g < pl.G ? db_x : db_h) + (g % pl.G) * H, H), *dbs[idx * 2 * pl.G + g]);
             }
-            // gradient of the layer's input rows; the second direction adds to the first
-            if (d == 0) {
-                pass.Dot(Matrix(dgx_all, rows, GH, GH), Matrix(pw.wx[idx], GH, in, in), Matrix(dx_acc, rows, in, in));
-            } else {
-                pass.Dot(Matrix(dgx_all, rows, GH, GH), Matrix(pw.wx[idx], GH, in, in), Matrix(dx_tmp, rows, in, in));
-                pass.Add(Matrix(dx_acc, rows, in, in), Matrix(dx_tmp, rows, in, in), Matrix(dx_acc, rows, in, in));
-            }
+            // the second direction adds to the first
+            if (dx == nullptr) continue;
+            float* const to = d == 0 ? dx : dx_tmp;
+            pass.Dot(Matrix(dgx_all[i], rows, GH, GH), Matrix(wx_packed[idx], GH, in, in), Matrix(to, rows, in, in));
+            if (d == 1) pass.Add(Matrix(dx, rows, in, in), Matrix(dx_tmp, rows, in, in), Matrix(dx, rows, in, in));
         }
-        std::swap(dy_cur, dx_acc);  // the layer below produced these rows
+    };
+    if (wavefront) {
+        run(0, pl.L - 1);
+        for (int l = pl.L - 1; l >= 0; --l) finish(l, l == 0 ? dx_acc : nullptr);
+        std::swap(dy_cur, dx_acc);
+    } else {
+        for (int l = pl.L - 1; l >= 0; --l) {
+            run(l, l);
+            finish(l, dx_acc);
+            std::swap(dy_cur, dx_acc);  // the layer below produced these rows
+        }
+    }
+    for (int idx = 0; idx < chains; ++idx) {
+        pass.Copy(Matrix(dh_all + idx * B * H, B, H, H), StateSlice(dhx, idx));
+        if (pl.mode == kLstm) pass.Copy(Matrix(dc_all + idx * B * H, B, H, H), StateSlice(dcx, idx));
     }
     for (int t = 0; t < pl.T; ++t) pass.Copy(Matrix(dy_cur + pl.row_start[t] * pl.I, pl.bt[t], pl.I, pl.I), *dxs[t]);
     for (const auto& c : db_copies) pass.Copy(c.first, c.second);
@@ -620,7 +1102,7 @@ void RunBackward(Pass& pass, const RnnPlan& pl, int activation, const hipcx_arra
     pass.CheckFits();
 }
 
-bool FastLstmApplies(const RnnPlan& pl, const void* reserve) { return pl.mode == kLstm && pl.D == 1 && reserve == nullptr; }
+bool FastLstmApplies(const RnnPlan& pl, bool training) { return pl.mode == kLstm && pl.D == 1 && !training && !Narrow(pl); }
 
 }  // namespace
 }  // namespace hipcx
@@ -641,7 +1123,7 @@ size_t hipcx_n_step_rnn_workspace_size(int n_layers, int bidirectional, int mode
                                        int n_steps) {
     try {
         const RnnPlan pl = MakePlan(n_layers, bidirectional, mode, hx, xs, n_steps);
-        if (!training && pl.mode == kLstm && pl.D == 1) return hipcx_n_step_lstm_workspace_size(n_layers, hx, xs, n_steps);
+        if (FastLstmApplies(pl, training != 0)) return hipcx_n_step_lstm_workspace_size(n_layers, hx, xs, n_steps);
         // a dry run over stand-ins for the caller's arrays: dense arrays of the right shapes
         std::vector<hipcx_array> w, b, y;
         std::vector<const hipcx_array*> pw, pb, py;
@@ -694,7 +1176,7 @@ int hipcx_n_step_rnn(int n_layers, int bidirectional, int mode, int activation, 
                       "n_step_rnn: workspace must be 256-byte aligned device memory");
         HIPCX_REQUIRE(reserve == nullptr || (reserve_bytes >= pl.reserve_total && reinterpret_cast<uintptr_t>(reserve) % 256 == 0),
                       HIPCX_CHAINERX_ERROR, "n_step_rnn: reserve too small or not 256-byte aligned: need " + std::to_string(pl.reserve_total) + " bytes");
-        if (FastLstmApplies(pl, reserve)) {
+        if (FastLstmApplies(pl, reserve != nullptr)) {
             CheckStatus(hipcx_n_step_lstm(n_layers, hx, cx, ws, bs, xs, n_steps, hy, cy, ys, workspace, workspace_bytes, stream));
             return;
         }

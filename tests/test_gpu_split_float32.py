@@ -8,7 +8,7 @@ import chainer_amd as chx
 pytestmark = pytest.mark.gpu
 
 # A sum of K float products in any order, each and each partial sum rounded once, is within K 2^-24 of the sum of magnitudes (to first order); what the
-# split leaves out of a product is below 2^-25 of it.
+# split leaves out of a product is at most 2^-23 of it.
 _EPS = 2.0 ** -24
 
 
