@@ -12,19 +12,16 @@
 #include "igemm.h"
 #include "igemm_pipe.h"
 #include "igemm_split.h"
+#include "launch_profile.h"
 #include "layout_kernels.h"
 #include "nchw_conv.h"
 #include "pw_conv.h"
 #include "stem_conv.h"
 #include "dot_parts.h"
-#include "small_dot.h"
 
 namespace hipcx {
 namespace {
 
-// Optional event bracketing of every implicit-GEMM launch (hipcx_profile_start/stop): the events are
-// recorded on the launch stream right before and after the kernel, so their elapsed time is the
-// kernel's own duration and excludes the filter repack and any host work.
 struct ProfileRecord {  // one bracketed launch
     double ms, flops, bytes;
 };
@@ -38,25 +35,25 @@ struct ProfileState {
 ProfileState g_profile;
 std::mutex g_profile_mutex;  // launches from several host threads may record into one profiling window
 
-struct ProfileScope {
-    hipStream_t stream;
-    hipEvent_t stop = nullptr;
-    ProfileScope(hipStream_t s, double flops, double bytes) : stream(s) {
-        std::lock_guard<std::mutex> lock(g_profile_mutex);
-        if (!g_profile.on) return;
-        hipEvent_t start = nullptr;
-        HIPCX_CHECK_HIP(hipEventCreate(&start));
-        HIPCX_CHECK_HIP(hipEventCreate(&stop));
-        g_profile.events.emplace_back(start, stop);
-        g_profile.records.push_back(ProfileRecord{0.0, flops, bytes});
-        g_profile.flops += flops;
-        g_profile.bytes += bytes;
-        HIPCX_CHECK_HIP(hipEventRecord(start, stream));
-    }
-    ~ProfileScope() {
-        if (stop != nullptr) (void)hipEventRecord(stop, stream);
-    }
-};
+}  // namespace
+
+ProfileScope::ProfileScope(hipStream_t s, double flops, double bytes) : stream(s) {
+    std::lock_guard<std::mutex> lock(g_profile_mutex);
+    if (!g_profile.on) return;
+    hipEvent_t start = nullptr;
+    HIPCX_CHECK_HIP(hipEventCreate(&start));
+    HIPCX_CHECK_HIP(hipEventCreate(&stop));
+    g_profile.events.emplace_back(start, stop);
+    g_profile.records.push_back(ProfileRecord{0.0, flops, bytes});
+    g_profile.flops += flops;
+    g_profile.bytes += bytes;
+    HIPCX_CHECK_HIP(hipEventRecord(start, stream));
+}
+ProfileScope::~ProfileScope() {
+    if (stop != nullptr) (void)hipEventRecord(stop, stream);
+}
+
+namespace {
 
 template <typename T, int WM, int WN, bool PM>
 void LaunchShape(IGemmArgs<T> p, bool fast16, bool fast8, hipStream_t stream) {
@@ -206,203 +203,6 @@ void LaunchIGemmImpl(IGemmArgs<T> p, hipStream_t stream) {
     }
 }
 
-
-// Workgroups that share a tile's reduction: while tiles leave compute units without one, but at least 896 bytes of a row each.
-int PlanSmallDotSplit(int64_t m, int64_t n, int64_t k, int dtype) {
-    const int64_t tiles = ((m + 31) / 32) * ((n + 31) / 32), lines = (k * ItemSize(dtype) + 127) / 128;
-    const int64_t s = std::min<int64_t>({NumCUs() / tiles, lines / 7, 32});
-    return s > 1 ? static_cast<int>(s) : 1;
-}
-
-// Splitting pays for the extra pass over the partial sums (3-4 us) once a tile's reduction takes longer than that on one compute unit:
-// 0.11 us per 128 bytes of its rows in float32 (16 MFMAs), 0.065 us in float16 (fetching the lines).  Against 1 to 32 parts on 206 products of
-// 650 to 10007 terms the choice is within 10 % of the best for 162.  Not so for float16 operands read element by element, 0.27 us per 128 bytes:
-// [20,3500] . [3500,650] row-major takes 17.6 us in one part and 8.1 in eight.
-int SmallDotSplit(int64_t m, int64_t n, int64_t k, int dtype) {
-    const int64_t lines = (k * ItemSize(dtype) + 127) / 128;
-    return lines >= (dtype == HIPCX_FLOAT32 ? 48 : 80) ? PlanSmallDotSplit(m, n, k, dtype) : 1;
-}
-
-size_t SmallDotPartialBytes(int64_t m, int64_t n, int64_t k, int dtype) {
-    const int split = SmallDotSplit(m, n, k, dtype);
-    return split > 1 ? static_cast<size_t>(split) * m * n * sizeof(float) : 0;
-}
-
-bool SmallDotShape(int64_t m, int64_t n, int64_t k) { return ((m + 127) / 128) * ((n + 127) / 128) < 128 && k >= 64; }
-
-// Fills in the operands; false when their strides or spans rule the kernels out.
-template <typename T>
-bool SmallDotOperands(const hipcx_array* a, const hipcx_array* b, SmallDotArgs* p, int* a_mode, int* b_mode) {
-    const int64_t M = a->shape[0], K = a->shape[1], N = b->shape[1];
-    const int64_t it = sizeof(T);
-    for (const hipcx_array* x : {a, b}) {
-        if (x->strides[0] < 0 || x->strides[1] < 0 || x->strides[0] % it || x->strides[1] % it) return false;
-    }
-    p->a = a->data;
-    p->b = b->data;
-    p->M = static_cast<int>(M);
-    p->N = static_cast<int>(N);
-    p->K = static_cast<int>(K);
-    p->a_row = a->strides[0] / it;
-    p->a_k = a->strides[1] / it;
-    p->b_k = b->strides[0] / it;
-    p->b_col = b->strides[1] / it;
-    int64_t a_span = ((M - 1) * p->a_row + (K - 1) * p->a_k + 1) * it, b_span = ((K - 1) * p->b_k + (N - 1) * p->b_col + 1) * it;
-    if (a_span >= (1LL << 31) - 256 || b_span >= (1LL << 31) - 256) return false;
-    auto mode = [&](const void* ptr, int64_t k_stride, int64_t line_stride, int64_t* span) {
-        if (k_stride != 1 && K > 1) return static_cast<int>(kElements);
-        if (reinterpret_cast<uintptr_t>(ptr) % 4 == 0 && line_stride * it % 4 == 0) {
-            *span = (*span + 3) / 4 * 4;  // a last half element shares its (aligned) dword with the two bytes behind it
-            return static_cast<int>(kPieces);
-        }
-        return static_cast<int>(kOddPieces);
-    };
-    *a_mode = mode(a->data, p->a_k, p->a_row, &a_span);
-    *b_mode = mode(b->data, p->b_k, p->b_col, &b_span);
-    p->a_bytes = static_cast<unsigned>(a_span);
-    p->b_bytes = static_cast<unsigned>(b_span);
-    p->tiles_m = static_cast<int>((M + 31) / 32);
-    p->tiles_n = static_cast<int>((N + 31) / 32);
-    return true;
-}
-
-template <typename T, int AM, int BM, int P>
-void LaunchSmallDotPieces(const SmallDotArgs& p, dim3 grid, hipStream_t stream) {
-    constexpr int kWaveBytes = std::max<int>((P == 4) * ((AM != kElements) + (BM != kElements)) * kSmallDotStage, kSmallDotPart * sizeof(float));
-    struct SmallDotTag {};
-    EnsureDynamicLds<SmallDotTag>(reinterpret_cast<const void*>(SmallDotMixedKernel<T, AM, BM, P>), kSmallDotMaxWaves * kWaveBytes);
-    hipLaunchKernelGGL((SmallDotMixedKernel<T, AM, BM, P>), grid, dim3(64 * p.nw), p.nw * kWaveBytes, stream, p);
-    CheckLaunch("small_dot_mixed");
-}
-
-template <typename T, int AM, int BM>
-void LaunchSmallDotMixed(const SmallDotArgs& p, dim3 grid, int pieces, hipStream_t stream) {
-    if constexpr (AM != kOddPieces && BM != kOddPieces && (AM != kPieces || BM != kPieces)) {
-        if (pieces == 1) return LaunchSmallDotPieces<T, AM, BM, 1>(p, grid, stream);
-    }
-    LaunchSmallDotPieces<T, AM, BM, 4>(p, grid, stream);
-}
-
-// `batch` products (SmallDotArgs::outs) of p.ksplit workgroups per tile.
-template <typename T>
-void LaunchSmallDot(SmallDotArgs p, int a_mode, int b_mode, int batch, hipStream_t stream) {
-    const dim3 grid(static_cast<unsigned>(p.tiles_m * p.tiles_n * p.ksplit), static_cast<unsigned>(batch));
-    const bool latency_bound = static_cast<int64_t>(p.tiles_m) * p.tiles_n <= NumCUs();
-    const int lines = (p.K * static_cast<int>(sizeof(T)) + 127) / 128;
-    // with more tiles than compute units and a reduction of any length the whole lines of SmallDotMixedKernel are faster
-    // ([128,650] . [650,2600] 13.9 -> 13.4 us)
-    if (a_mode == kPieces && b_mode == kPieces && (latency_bound || lines <= 7)) {
-        hipLaunchKernelGGL((SmallDotKernel<T>), grid, dim3(512), 0, stream, p);
-        CheckLaunch("small_dot");
-        return;
-    }
-    // Elements come as they are used: chunks of 32 bytes, six of them in flight, beat whole lines ([32,1000] . [1000,2048] float16 14.3 -> 5.5 us,
-    // [200,4000] . [4000,4000] 174 -> 51, [20,2600] . [2600,650] float32 13.4 -> 9.3); rows of odd pitch gain from whole lines at any size.
-    const bool elements = a_mode == kElements || b_mode == kElements, odd = a_mode == kOddPieces || b_mode == kOddPieces;
-    const int pieces = (latency_bound || elements) && !odd ? 1 : 4;
-    // eight waves keep more loads in flight; four, one per SIMD, once there is a workgroup for every compute unit
-    const int chunk = pieces == 1 ? 32 : 128, chunks = (p.K * static_cast<int>(sizeof(T)) + chunk - 1) / chunk;
-    const int per_split = (chunks + p.ksplit - 1) / p.ksplit;
-    const int most = static_cast<int>(grid.x) * batch <= NumCUs() ? kSmallDotMaxWaves : 4;
-    const int per_wave = (per_split + most - 1) / most;
-    p.nw = (per_split + per_wave - 1) / per_wave;
-    auto with_a = [&](auto a_tag) {
-        constexpr int AM = decltype(a_tag)::value;
-        if (b_mode == kElements) return LaunchSmallDotMixed<T, AM, kElements>(p, grid, pieces, stream);
-        if constexpr (sizeof(T) == 2) {
-            if (b_mode == kOddPieces) return LaunchSmallDotMixed<T, AM, kOddPieces>(p, grid, pieces, stream);
-        }
-        LaunchSmallDotMixed<T, AM, kPieces>(p, grid, pieces, stream);
-    };
-    if (a_mode == kPieces) return with_a(std::integral_constant<int, kPieces>{});
-    if (a_mode == kElements) return with_a(std::integral_constant<int, kElements>{});
-    if constexpr (sizeof(T) == 2) with_a(std::integral_constant<int, kOddPieces>{});
-}
-
-// Which kernel of small_dot.h takes a product.
-enum SmallDotPath { kNoSmallDot, kSmallDotVector, kSmallDotLines, kSmallDotTiles };
-
-template <typename T>
-SmallDotPath PlanSmallDot(const hipcx_array* a, const hipcx_array* b, SmallDotArgs* p, int* a_mode, int* b_mode) {
-    static const bool enabled = [] { const char* e = getenv("HIPCX_SMALL_DOT"); return e == nullptr || e[0] != '0'; }();
-    static const bool rows_ok = [] { const char* e = getenv("HIPCX_SMALL_DOT_ROWS"); return e == nullptr || e[0] != '0'; }();
-    const int64_t M = a->shape[0], K = a->shape[1], N = b->shape[1];
-    if (!enabled || !SmallDotShape(M, N, K) || !SmallDotOperands<T>(a, b, p, a_mode, b_mode)) return kNoSmallDot;
-    if (*a_mode != kPieces || *b_mode != kPieces) return kSmallDotTiles;
-    if (M <= 4) return kSmallDotVector;
-    // whole-line loads regrouped through LDS pay off once the product is large enough to be bandwidth-bound (measured: the
-    // 10000-column projection of the language model gains 15 %, the 2600- and 1000-column layers lose 10 %)
-    return rows_ok && 2.0 * M * N * K >= 1e9 ? kSmallDotLines : kSmallDotTiles;
-}
-
-// Bytes of partial sums for a small product: only tiles are split along the reduction.
-size_t SmallDotWorkspace(const hipcx_array* a, const hipcx_array* b, int dtype) {
-    if (dtype != HIPCX_FLOAT16 && dtype != HIPCX_FLOAT32) return 0;
-    const size_t bytes = SmallDotPartialBytes(a->shape[0], b->shape[1], a->shape[1], dtype);
-    if (bytes == 0) return 0;  // most products
-    SmallDotArgs p{};
-    int a_mode = 0, b_mode = 0;
-    const SmallDotPath path = dtype == HIPCX_FLOAT16 ? PlanSmallDot<half_t>(a, b, &p, &a_mode, &b_mode) : PlanSmallDot<float>(a, b, &p, &a_mode, &b_mode);
-    return path == kSmallDotTiles ? bytes : 0;
-}
-
-// Small-output matrix products (small_dot.h).  Returns false when the problem does not qualify.  `partial` holds
-// SmallDotPartialBytes bytes; without it the reduction is not split.
-template <typename T>
-bool TrySmallDot(const hipcx_array* a, const hipcx_array* b, const hipcx_array* bias, const hipcx_array* out, float* partial, hipStream_t stream) {
-    const int64_t M = a->shape[0], K = a->shape[1], N = b->shape[1];
-    const int64_t it = sizeof(T);
-    if (out->strides[0] < 0 || out->strides[1] < 0 || out->strides[0] % it || out->strides[1] % it) return false;
-    SmallDotArgs p{};
-    int a_mode = 0, b_mode = 0;
-    const SmallDotPath path = PlanSmallDot<T>(a, b, &p, &a_mode, &b_mode);
-    if (path == kNoSmallDot) return false;
-    p.out = out->data;
-    p.o_row = out->strides[0] / it;
-    p.o_col = out->strides[1] / it;
-    if (bias != nullptr) {
-        p.bias = bias->data;
-        p.bias_stride = bias->strides[0] / it;
-    }
-    ProfileScope prof(stream, 2.0 * M * N * K, static_cast<double>(it) * (M * K + K * N + M * N));
-    if (path == kSmallDotVector) {
-        const dim3 grid(static_cast<unsigned>((N + 3) / 4));
-        if (M == 1) hipLaunchKernelGGL((SmallDotVectorKernel<T, 1>), grid, dim3(256), 0, stream, p);
-        else if (M == 2) hipLaunchKernelGGL((SmallDotVectorKernel<T, 2>), grid, dim3(256), 0, stream, p);
-        else hipLaunchKernelGGL((SmallDotVectorKernel<T, 4>), grid, dim3(256), 0, stream, p);
-        CheckLaunch("small_dot_vector");
-        return true;
-    }
-    if (path == kSmallDotLines) {
-        // Waves per workgroup = ways K is split: the choice that leaves the busiest SIMD the least matrix work
-        // (wave-tiles are dealt over 4 SIMDs per CU; a wave's share is whole 128-byte steps).
-        const int64_t blocks = static_cast<int64_t>(p.tiles_m) * p.tiles_n, steps = (K * it + 127) / 128;
-        const int64_t simds = static_cast<int64_t>(NumCUs()) * 4;
-        int best_nw = 1;
-        int64_t best_cost = -1;
-        for (int nw : {1, 2, 3, 4, 6, 8}) {
-            if (nw > steps) break;
-            int64_t rounds = (blocks * nw + simds - 1) / simds;
-            int64_t cost = rounds * ((steps + nw - 1) / nw) * 8 + nw;  // + the partial-sum pass
-            if (best_cost < 0 || cost < best_cost) best_cost = cost, best_nw = nw;
-        }
-        p.nw = best_nw;
-        const int lds_bytes = best_nw * 2 * 32 * 144;
-        struct RowsTag {};
-        EnsureDynamicLds<RowsTag>(reinterpret_cast<const void*>(SmallDotRowsKernel<T>), 8 * 2 * 32 * 144);
-        hipLaunchKernelGGL((SmallDotRowsKernel<T>), dim3(static_cast<unsigned>(blocks)), dim3(64 * best_nw), lds_bytes, stream, p);
-        CheckLaunch("small_dot_rows");
-        return true;
-    }
-    p.ksplit = partial != nullptr ? SmallDotSplit(M, N, K, DtypeOf<T>::value) : 1;
-    p.partial = p.ksplit > 1 ? partial : nullptr;
-    LaunchSmallDot<T>(p, a_mode, b_mode, 1, stream);
-    if (p.ksplit > 1) {
-        hipLaunchKernelGGL((SmallDotSumKernel<T>), dim3(static_cast<unsigned>((M * N + 255) / 256)), dim3(256), 0, stream, p);
-        CheckLaunch("small_dot_sum");
-    }
-    return true;
-}
 
 // float64 (no MFMA path yet): one thread per output element, fma in reduction order.
 __global__ void ConvNaiveF64Kernel(IGemmArgs<double> p) {
@@ -1183,26 +983,6 @@ void CheckConv(const hipcx_array* x, const hipcx_array* w, const hipcx_array* b,
 
 }  // namespace
 
-bool DotSeveral(const hipcx_array* a0, int64_t a_distance, const hipcx_array* b, const hipcx_array* const* outs, int n, hipStream_t stream) {
-    const int64_t M = a0->shape[0], K = a0->shape[1], N = b->shape[1];
-    SmallDotArgs p{};
-    int a_mode = 0, b_mode = 0;
-    if (n > kSmallDotMaxBatch || !SmallDotShape(M, N, K) || SmallDotSplit(M, N, K, HIPCX_FLOAT32) > 1) return false;
-    if (!SmallDotOperands<float>(a0, b, &p, &a_mode, &b_mode)) return false;
-    for (int i = 0; i < n; ++i) {
-        if (outs[i]->strides[0] != outs[0]->strides[0] || outs[i]->strides[1] != outs[0]->strides[1]) return false;
-        p.outs[i] = outs[i]->data;
-    }
-    if (outs[0]->strides[0] < 0 || outs[0]->strides[1] < 0 || outs[0]->strides[0] % 4 || outs[0]->strides[1] % 4) return false;
-    p.out = outs[0]->data;
-    p.o_row = outs[0]->strides[0] / 4;
-    p.o_col = outs[0]->strides[1] / 4;
-    p.a_batch = a_distance;
-    p.ksplit = 1;
-    ProfileScope prof(stream, 2.0 * M * N * K * n, 4.0 * n * (M * K + K * N + M * N));
-    LaunchSmallDot<float>(p, a_mode, b_mode, n, stream);
-    return true;
-}
 }  // namespace hipcx
 
 namespace hipcx {
@@ -1817,14 +1597,14 @@ static int DotBias(const hipcx_array* a, const hipcx_array* b, const hipcx_array
             }
         }
         if (out->dtype == HIPCX_FLOAT16) {
-            if (slices == 1 && TrySmallDot<half_t>(a, b, bias, out, small_partial, st)) return;
+            if (slices == 1 && TrySmallDot(a, b, bias, out, small_partial, st)) return;
             IGemmArgs<half_t> p{};
             fill(p);
             p.ksplit = slices;
             p.partial = partial;
             LaunchIGemmImpl(p, st);
         } else if (out->dtype == HIPCX_FLOAT32) {
-            if (slices == 1 && TrySmallDot<float>(a, b, bias, out, small_partial, st)) return;
+            if (slices == 1 && TrySmallDot(a, b, bias, out, small_partial, st)) return;
             IGemmArgs<float> p{};
             fill(p);
             p.ksplit = slices;

@@ -6,7 +6,7 @@
 // the partial tiles are summed through LDS.  Four kernels, by where the operands lie (chosen in TrySmallDot):
 //   SmallDotKernel        k is the unit-stride axis of both operands (Linear's x and W^T): straight from global memory, bound by the
 //                         latency of a few loads.
-//   SmallDotRowsKernel    the same for products of 1 GFLOP and more, whole 128-byte lines regrouped through LDS.
+//   SmallDotLinesKernel   the same for more or longer tiles: whole 128-byte lines regrouped through LDS.
 //   SmallDotMixedKernel   an operand whose k axis is not the unit-stride one (dG . Wh of a recurrent network, x^T . gy), or float16 rows
 //                         of odd pitch.
 //   SmallDotVectorKernel  M <= 4 (one image, one sentence): a wave per output column, K across the lanes, where the MFMA would work on
@@ -35,10 +35,10 @@ struct SmallDotArgs {
     const void* bias;     // one element per column of out, added to the rounded product (Dot, then Add); may be null
     int64_t bias_stride;  // elements
     int nw;               // waves per workgroup = ways a workgroup's share of the reduction is split (SmallDotKernel: 8)
-    int ksplit;           // workgroups per tile along the reduction (not SmallDotRowsKernel)
+    int ksplit;           // workgroups per tile along the reduction
     float* partial;       // not null: [ksplit][M][N] sums go there instead of to out
     // blockIdx.y: products of one b that share their shapes and strides, left operands at a constant distance (elements), outputs
-    // anywhere (not SmallDotRowsKernel)
+    // anywhere
     int64_t a_batch;
     void* outs[kSmallDotMaxBatch];
 };
@@ -213,112 +213,6 @@ __global__ __launch_bounds__(512) void SmallDotKernel(SmallDotArgs p) {
     }
 }
 
-// The same product when k is the unit-stride axis of both operands (Linear: x rows and W rows).  Lanes load whole
-// 128-byte lines -- 8 lanes x 16 bytes per row, 8 rows per instruction -- instead of 32-byte pieces of 32 rows, and the
-// wave regroups them into the MFMA operand layout through its own LDS region (no workgroup barrier in the loop).
-// The loads of step s+1 are in flight while step s is multiplied.  p.nw waves split K in whole 128-byte steps.
-template <typename T>
-__global__ __launch_bounds__(512) void SmallDotRowsKernel(SmallDotArgs p) {
-    constexpr int PL = 16 / sizeof(T);   // elements per 16-byte piece
-    constexpr int KS = 8 * PL;           // k per step: one 128-byte line per row
-    constexpr int PITCH = 144;           // bytes per staged row: 16 consecutive rows start on 16 different bank groups
-    constexpr int REGION = 2 * 32 * PITCH;
-    extern __shared__ __align__(16) char lds[];
-
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int lr = lane & 31;
-    const int g = lane >> 5;
-    const int piece = lane & 7;
-    const int sub = lane >> 3;  // row within a group of 8
-    int tm, tn;
-    SmallDotTile(gridDim.x, blockIdx.x, p.tiles_m, tm, tn);
-    const __amdgpu_buffer_rsrc_t ar = MakeRsrc(p.a, p.a_bytes);
-    const __amdgpu_buffer_rsrc_t br = MakeRsrc(p.b, p.b_bytes);
-    char* wa = lds + wave * REGION;
-    char* wb = wa + 32 * PITCH;
-
-    const int steps = (p.K + KS - 1) / KS;
-    const int per_wave = (steps + p.nw - 1) / p.nw;
-    const int k_begin = wave * per_wave * KS;
-    const int k_end = min(p.K, k_begin + per_wave * KS);
-
-    int abase[4], bbase[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int m = tm * 32 + j * 8 + sub, n = tn * 32 + j * 8 + sub;
-        abase[j] = m < p.M ? static_cast<int>((static_cast<int64_t>(m) * p.a_row + piece * PL) * static_cast<int64_t>(sizeof(T))) : -1;
-        bbase[j] = n < p.N ? static_cast<int>((static_cast<int64_t>(n) * p.b_col + piece * PL) * static_cast<int64_t>(sizeof(T))) : -1;
-    }
-    Bytes16 areg[4], breg[4];
-    auto load_step = [&](int k) {
-        const int koff = k * static_cast<int>(sizeof(T));
-        const bool inside = k + piece * PL < k_end;  // pieces wholly beyond the share (or K) come back as zeros
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            areg[j] = __builtin_amdgcn_raw_buffer_load_b128(ar, (abase[j] >= 0 && inside) ? abase[j] + koff : 0x7fffffff, 0, 0);
-            breg[j] = __builtin_amdgcn_raw_buffer_load_b128(br, (bbase[j] >= 0 && inside) ? bbase[j] + koff : 0x7fffffff, 0, 0);
-        }
-    };
-    auto mask_piece = [](Bytes16 v, int c) {  // keep the first c elements of the piece (they end at K; what follows is the next row)
-        if constexpr (sizeof(T) == 4) {
-            v.y = c > 1 ? v.y : 0u;
-            v.z = c > 2 ? v.z : 0u;
-            v.w = c > 3 ? v.w : 0u;
-        } else {
-            auto m = [c](int d) { return c > 2 * d + 1 ? 0xffffffffu : (c > 2 * d ? 0x0000ffffu : 0u); };
-            v.x &= m(0);
-            v.y &= m(1);
-            v.z &= m(2);
-            v.w &= m(3);
-        }
-        return v;
-    };
-    auto stage_step = [&](int k) {
-        const int c = k_end - (k + piece * PL);
-        char* da = wa + sub * PITCH + piece * 16;
-        char* db = wb + sub * PITCH + piece * 16;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            *reinterpret_cast<Bytes16*>(da + j * 8 * PITCH) = c < PL ? mask_piece(areg[j], c) : areg[j];
-            *reinterpret_cast<Bytes16*>(db + j * 8 * PITCH) = c < PL ? mask_piece(breg[j], c) : breg[j];
-        }
-    };
-
-    float16_t acc;
-#pragma unroll
-    for (int v = 0; v < 16; ++v) acc[v] = 0.f;
-    if (k_begin < k_end) {
-        load_step(k_begin);
-        for (int k = k_begin; k < k_end; k += KS) {
-            stage_step(k);                           // waits for this step's loads only
-            if (k + KS < k_end) load_step(k + KS);   // next step in flight during the MFMAs below
-            __builtin_amdgcn_wave_barrier();
-#pragma unroll
-            for (int gs = 0; gs < 4; ++gs) {
-                const Bytes16 fa = *reinterpret_cast<const Bytes16*>(wa + lr * PITCH + (2 * gs + g) * 16);
-                const Bytes16 fb = *reinterpret_cast<const Bytes16*>(wb + lr * PITCH + (2 * gs + g) * 16);
-                MfmaTile<T>(fa, fb, acc);
-            }
-            __builtin_amdgcn_wave_barrier();
-        }
-    }
-    __syncthreads();  // every wave is done with its staging region: it becomes the partial-sum area
-    float* part = reinterpret_cast<float*>(lds);
-#pragma unroll
-    for (int v = 0; v < 16; ++v) part[wave * (32 * 33) + (8 * (v / 4) + 4 * g + (v % 4)) * 33 + lr] = acc[v];
-    __syncthreads();
-    T* out = static_cast<T*>(p.out);
-    for (int e = tid; e < 32 * 32; e += 64 * p.nw) {
-        const int row = e >> 5, col = e & 31;
-        float s = 0.f;
-        for (int w = 0; w < p.nw; ++w) s += part[w * (32 * 33) + row * 33 + col];
-        const int om = tm * 32 + row, on = tn * 32 + col;
-        if (om < p.M && on < p.N) StoreDot<T>(p, out, om, on, s);
-    }
-}
-
 // How SmallDotMixedKernel reads an operand.  kPieces: rows of contiguous k as 16-byte pieces; kElements: another axis is the unit-stride
 // one, element by element with that axis across the lanes -- whole lines too, already in the MFMA layout; kOddPieces: float16 rows of odd
 // pitch, whose last elements share a dword with what lies behind the array: pieces, but the chunk that holds the end of K by elements.
@@ -371,7 +265,128 @@ __device__ __forceinline__ Bytes16 MaskPiece(Bytes16 v, int k, int K) {
     return v;
 }
 
-// The reduction is dealt out in chunks of 128 bytes per row.  Pieces are loaded as whole lines (8 lanes to a row, 8 rows to an instruction)
+// Both operands in pieces.  A wave takes chunks of 128 bytes per row: whole lines (8 lanes to a row, 8 rows to an instruction), turned round in LDS of
+// its own.  Two chunks are in flight while a third is multiplied; the loads' offsets are constants plus a scalar, and only the chunk that holds the end
+// of K looks at it.  Bound by the matrix pipe and by the delivery of operands (64 rows for 1024 outputs) in about equal parts.  us, against one chunk in
+// flight and three or more waves to a tile: float32 [1024,1024]^2 33.4 -> 26.5, [1000,784] . [784,1000] 27.4 -> 22.6, [256,1024] . [1024,1024] 11.4 ->
+// 9.6 (against SmallDotKernel); float16 15.4 -> 10.5, 13.3 -> 11.0, 6.6 -> 5.1, [37,2048] . [2048,1000] 9.8 -> 6.1.
+template <typename T>
+__global__ __launch_bounds__(64 * kSmallDotMaxWaves) __attribute__((amdgpu_waves_per_eu(2, 8))) void SmallDotLinesKernel(SmallDotArgs p) {
+    constexpr int PL = 16 / sizeof(T);
+    constexpr int KC = 8 * PL;  // k per chunk
+    constexpr int kOut = 0x7fffffff;
+    extern __shared__ __align__(16) char lds[];
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: the loop below runs on scalar control flow
+    const int lr = lane & 31;
+    const int g = lane >> 5;
+    const int piece = lane & 7, sub = lane >> 3;
+    const int tiles = p.tiles_m * p.tiles_n;
+    const int split = blockIdx.x / tiles;
+    int tm, tn;
+    SmallDotTile(tiles, blockIdx.x - split * tiles, p.tiles_m, tm, tn);
+    const int batch = blockIdx.y;
+    const __amdgpu_buffer_rsrc_t ar = MakeRsrc(static_cast<const T*>(p.a) + batch * p.a_batch, p.a_bytes);
+    const __amdgpu_buffer_rsrc_t br = MakeRsrc(p.b, p.b_bytes);
+    int a_line[4], b_line[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int m = tm * 32 + j * 8 + sub, n = tn * 32 + j * 8 + sub;
+        a_line[j] = m < p.M ? static_cast<int>((m * p.a_row + piece * PL) * static_cast<int64_t>(sizeof(T))) : kOut;
+        b_line[j] = n < p.N ? static_cast<int>((n * p.b_col + piece * PL) * static_cast<int64_t>(sizeof(T))) : kOut;
+    }
+    char* const a_stage = lds + wave * 2 * kSmallDotStage;
+    char* const to = a_stage + sub * kSmallDotPitch + piece * 16;
+    const char* const from = a_stage + lr * kSmallDotPitch + g * 16;
+
+    // this wave's chunks
+    const int chunks = (p.K + KC - 1) / KC;
+    const int per_split = (chunks + p.ksplit - 1) / p.ksplit;
+    const int s_begin = split * per_split, s_end = min(chunks, s_begin + per_split);
+    const int per_wave = (max(s_end - s_begin, 0) + p.nw - 1) / p.nw;
+    const int begin = s_begin + wave * per_wave, end = min(s_end, begin + per_wave);
+
+    float16_t acc;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[v] = 0.f;
+    Bytes16 av[2][4], bv[2][4];
+    auto load = [&](int st, int c) {
+        if ((c + 1) * KC <= p.K) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                av[st][j] = __builtin_amdgcn_raw_buffer_load_b128(ar, a_line[j], c * 128, 0);
+                bv[st][j] = __builtin_amdgcn_raw_buffer_load_b128(br, b_line[j], c * 128, 0);
+            }
+        } else {  // pieces beyond K are not read
+            const bool in = c * KC + piece * PL < p.K;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                av[st][j] = __builtin_amdgcn_raw_buffer_load_b128(ar, in & (a_line[j] != kOut) ? a_line[j] + c * 128 : kOut, 0, 0);
+                bv[st][j] = __builtin_amdgcn_raw_buffer_load_b128(br, in & (b_line[j] != kOut) ? b_line[j] + c * 128 : kOut, 0, 0);
+            }
+        }
+    };
+    auto multiply = [&](int st, int c, auto&& next) {
+        if ((c + 1) * KC > p.K) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                av[st][j] = MaskPiece<T>(av[st][j], c * KC + piece * PL, p.K);
+                bv[st][j] = MaskPiece<T>(bv[st][j], c * KC + piece * PL, p.K);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            *reinterpret_cast<Bytes16*>(to + j * 8 * kSmallDotPitch) = av[st][j];
+            *reinterpret_cast<Bytes16*>(to + kSmallDotStage + j * 8 * kSmallDotPitch) = bv[st][j];
+        }
+        next();
+        __builtin_amdgcn_wave_barrier();
+        Bytes16 fa[4], fb[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            fa[q] = *reinterpret_cast<const Bytes16*>(from + q * 32);
+            fb[q] = *reinterpret_cast<const Bytes16*>(from + kSmallDotStage + q * 32);
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) MfmaTile<T>(fa[q], fb[q], acc);
+        __builtin_amdgcn_wave_barrier();
+    };
+    if (begin < end) {
+        load(0, begin);
+        if (begin + 1 < end) load(1, begin + 1);
+        int c = begin;
+        for (; c + 3 < end; c += 2) {
+            multiply(0, c, [&] { load(0, c + 2); });
+            multiply(1, c + 1, [&] { load(1, c + 3); });
+        }
+        // one, two or three are left
+        multiply(0, c, [&] {
+            if (c + 2 < end) load(0, c + 2);
+        });
+        if (c + 1 < end) multiply(1, c + 1, [] {});
+        if (c + 2 < end) multiply(0, c + 2, [] {});
+    }
+    __syncthreads();  // the staging areas become the partial tiles
+    // lane holds column lr, rows 8*(v/4) + 4*g + v%4
+    float* const part = reinterpret_cast<float*>(lds);
+    float* const mine = part + wave * kSmallDotPart;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) mine[(8 * (v / 4) + 4 * g + (v % 4)) * 33 + lr] = acc[v];
+    __syncthreads();
+    T* out = static_cast<T*>(gridDim.y > 1 ? p.outs[batch] : p.out);
+    for (int e = tid; e < 32 * 32; e += 64 * p.nw) {
+        const int row = e >> 5, col = e & 31;
+        const int om = tm * 32 + row, on = tn * 32 + col;
+        if (om >= p.M || on >= p.N) continue;
+        float s = 0.f;
+        for (int w = 0; w < p.nw; ++w) s += part[w * kSmallDotPart + row * 33 + col];
+        StoreTileElement<T>(p, split, out, om, on, s);
+    }
+}
+
+// The reduction is dealt out in chunks of 128 bytes per row.  Pieces are loaded as whole lines
 // and turned round through a piece of LDS that belongs to the wave (no barrier); elements come as they are used.  Two chunks are in flight
 // while a third is multiplied.  [20,2600] . [2600,650] float32, row-major b: 34 -> 9.3 us (several workgroups per tile and the pass over
 // their sums included), [64,333] . [333,777] float16 8.5 -> 6.4.

@@ -1,0 +1,238 @@
+// The small matrix product: which kernel of small_dot.h takes it, in how many parts, and the launches.
+#include <algorithm>
+#include <cstdlib>
+
+#include "dot_parts.h"
+#include "launch_profile.h"
+#include "small_dot.h"
+
+namespace hipcx {
+
+bool SmallDotShape(int64_t m, int64_t n, int64_t k) { return ((m + 127) / 128) * ((n + 127) / 128) < 128 && k >= 64; }
+
+namespace {
+
+// Workgroups that share a tile's reduction: while tiles leave compute units without one, but at least 896 bytes of a row each.
+int PlanSmallDotSplit(int64_t m, int64_t n, int64_t k, int dtype) {
+    const int64_t tiles = ((m + 31) / 32) * ((n + 31) / 32), lines = (k * ItemSize(dtype) + 127) / 128;
+    const int64_t s = std::min<int64_t>({NumCUs() / tiles, lines / 7, 32});
+    return s > 1 ? static_cast<int>(s) : 1;
+}
+
+// Splitting pays for the extra pass over the partial sums (3-4 us) once a tile's reduction takes longer than that on one compute unit:
+// 0.11 us per 128 bytes of its rows in float32 (16 MFMAs), 0.065 us in float16 (fetching the lines).  Against 1 to 32 parts on 206 products of
+// 650 to 10007 terms the choice is within 10 % of the best for 162.  Not so for float16 operands read element by element, 0.27 us per 128 bytes:
+// [20,3500] . [3500,650] row-major takes 17.6 us in one part and 8.1 in eight.
+int SmallDotSplit(int64_t m, int64_t n, int64_t k, int dtype) {
+    const int64_t lines = (k * ItemSize(dtype) + 127) / 128;
+    return lines >= (dtype == HIPCX_FLOAT32 ? 48 : 80) ? PlanSmallDotSplit(m, n, k, dtype) : 1;
+}
+
+size_t SmallDotPartialBytes(int64_t m, int64_t n, int64_t k, int dtype) {
+    const int split = SmallDotSplit(m, n, k, dtype);
+    return split > 1 ? static_cast<size_t>(split) * m * n * sizeof(float) : 0;
+}
+
+// Fills in the operands; false when their strides or spans rule the kernels out.
+template <typename T>
+bool SmallDotOperands(const hipcx_array* a, const hipcx_array* b, SmallDotArgs* p, int* a_mode, int* b_mode) {
+    const int64_t M = a->shape[0], K = a->shape[1], N = b->shape[1];
+    const int64_t it = sizeof(T);
+    for (const hipcx_array* x : {a, b}) {
+        if (x->strides[0] < 0 || x->strides[1] < 0 || x->strides[0] % it || x->strides[1] % it) return false;
+    }
+    p->a = a->data;
+    p->b = b->data;
+    p->M = static_cast<int>(M);
+    p->N = static_cast<int>(N);
+    p->K = static_cast<int>(K);
+    p->a_row = a->strides[0] / it;
+    p->a_k = a->strides[1] / it;
+    p->b_k = b->strides[0] / it;
+    p->b_col = b->strides[1] / it;
+    int64_t a_span = ((M - 1) * p->a_row + (K - 1) * p->a_k + 1) * it, b_span = ((K - 1) * p->b_k + (N - 1) * p->b_col + 1) * it;
+    if (a_span >= (1LL << 31) - 256 || b_span >= (1LL << 31) - 256) return false;
+    auto mode = [&](const void* ptr, int64_t k_stride, int64_t line_stride, int64_t* span) {
+        if (k_stride != 1 && K > 1) return static_cast<int>(kElements);
+        if (reinterpret_cast<uintptr_t>(ptr) % 4 == 0 && line_stride * it % 4 == 0) {
+            *span = (*span + 3) / 4 * 4;  // a last half element shares its (aligned) dword with the two bytes behind it
+            return static_cast<int>(kPieces);
+        }
+        return static_cast<int>(kOddPieces);
+    };
+    *a_mode = mode(a->data, p->a_k, p->a_row, &a_span);
+    *b_mode = mode(b->data, p->b_k, p->b_col, &b_span);
+    p->a_bytes = static_cast<unsigned>(a_span);
+    p->b_bytes = static_cast<unsigned>(b_span);
+    p->tiles_m = static_cast<int>((M + 31) / 32);
+    p->tiles_n = static_cast<int>((N + 31) / 32);
+    return true;
+}
+
+template <typename T, int AM, int BM, int P>
+void LaunchSmallDotPieces(const SmallDotArgs& p, dim3 grid, hipStream_t stream) {
+    constexpr int kWaveBytes = std::max<int>((P == 4) * ((AM != kElements) + (BM != kElements)) * kSmallDotStage, kSmallDotPart * sizeof(float));
+    struct SmallDotTag {};
+    EnsureDynamicLds<SmallDotTag>(reinterpret_cast<const void*>(SmallDotMixedKernel<T, AM, BM, P>), kSmallDotMaxWaves * kWaveBytes);
+    hipLaunchKernelGGL((SmallDotMixedKernel<T, AM, BM, P>), grid, dim3(64 * p.nw), p.nw * kWaveBytes, stream, p);
+    CheckLaunch("small_dot_mixed");
+}
+
+template <typename T, int AM, int BM>
+void LaunchSmallDotMixed(const SmallDotArgs& p, dim3 grid, int pieces, hipStream_t stream) {
+    if constexpr (AM != kOddPieces && BM != kOddPieces) {
+        if (pieces == 1) return LaunchSmallDotPieces<T, AM, BM, 1>(p, grid, stream);
+    }
+    LaunchSmallDotPieces<T, AM, BM, 4>(p, grid, stream);
+}
+
+// Whether whole lines regrouped through LDS (SmallDotLinesKernel) beat loads straight into the MFMA layout (SmallDotKernel) for `groups` workgroups of
+// `k` terms each: once most compute units have a tile of some length, or a tile is long.  us, SmallDotKernel and lines: float32 128 tiles
+// of 784 terms 7.2 and 8.6, 164 of 650 7.1 and 8.2, 256 of 1024 11.4 and 9.6, 484 of 300 9.0 and 8.6; float16 64 of 2048 9.8 and 6.1, 128 of 1000 5.0
+// and 5.3, 484 of 300 4.7 and 5.6.
+bool TakesLines(int64_t groups, int64_t k, int item) { return (groups > NumCUs() * 3 / 4 && k * item > 7 * 128) || k >= 1536; }
+
+// Their waves: eight keep most loads in flight while a compute unit has one or two tiles (328 float32 tiles of 21 chunks: 12.3 us, 12.8 with four, 16.6
+// with two); beyond, what leaves the busiest SIMD the fewest chunks, fewer waves on near terms (626 tiles of 21 chunks: 17.6 us with two, 18.2 with three, 16.5 with four; 1252 of
+// 21: 26.9, 26.5, 29.0; 1504 of 25: 34.1, 37.9, 35.3).
+int LinesWaves(int64_t groups, int chunks) {
+    if (groups <= 2 * NumCUs()) return std::min(kSmallDotMaxWaves, chunks);
+    const int64_t per_unit = (groups + NumCUs() - 1) / NumCUs();
+    auto cost = [&](int nw) { return (per_unit * nw + 3) / 4 * ((chunks + nw - 1) / nw); };
+    int best = 2;
+    for (int nw : {3, 4}) {
+        if (10 * cost(nw) < 9 * cost(best)) best = nw;
+    }
+    return std::min(best, chunks);
+}
+
+// `batch` products (SmallDotArgs::outs) of p.ksplit workgroups per tile.
+template <typename T>
+void LaunchSmallDot(SmallDotArgs p, int a_mode, int b_mode, int batch, hipStream_t stream) {
+    const int64_t tiles = static_cast<int64_t>(p.tiles_m) * p.tiles_n;
+    const dim3 grid(static_cast<unsigned>(tiles * p.ksplit), static_cast<unsigned>(batch));
+    if (a_mode == kPieces && b_mode == kPieces) {
+        const int chunks = ((p.K * static_cast<int>(sizeof(T)) + 127) / 128 + p.ksplit - 1) / p.ksplit;
+        const int64_t groups = tiles * p.ksplit * batch;
+        if (!TakesLines(groups, p.K / p.ksplit, sizeof(T))) {
+            hipLaunchKernelGGL((SmallDotKernel<T>), grid, dim3(512), 0, stream, p);
+            CheckLaunch("small_dot");
+            return;
+        }
+        p.nw = LinesWaves(groups, chunks);
+        constexpr int kWaveBytes = 2 * kSmallDotStage;
+        struct LinesTag {};
+        EnsureDynamicLds<LinesTag>(reinterpret_cast<const void*>(SmallDotLinesKernel<T>), kSmallDotMaxWaves * kWaveBytes);
+        hipLaunchKernelGGL((SmallDotLinesKernel<T>), grid, dim3(64 * p.nw), p.nw * kWaveBytes, stream, p);
+        CheckLaunch("small_dot_lines");
+        return;
+    }
+    // Elements come as they are used: chunks of 32 bytes, six of them in flight, beat whole lines ([32,1000] . [1000,2048] float16 14.3 -> 5.5 us,
+    // [200,4000] . [4000,4000] 174 -> 51, [20,2600] . [2600,650] float32 13.4 -> 9.3); rows of odd pitch gain from whole lines at any size.
+    const bool elements = a_mode == kElements || b_mode == kElements, odd = a_mode == kOddPieces || b_mode == kOddPieces;
+    const int pieces = elements && !odd ? 1 : 4;
+    // eight waves keep more loads in flight; four, one per SIMD, once there is a workgroup for every compute unit
+    const int chunk = pieces == 1 ? 32 : 128, chunks = (p.K * static_cast<int>(sizeof(T)) + chunk - 1) / chunk;
+    const int per_split = (chunks + p.ksplit - 1) / p.ksplit;
+    const int most = static_cast<int>(grid.x) * batch <= NumCUs() ? kSmallDotMaxWaves : 4;
+    const int per_wave = (per_split + most - 1) / most;
+    p.nw = (per_split + per_wave - 1) / per_wave;
+    auto with_a = [&](auto a_tag) {
+        constexpr int AM = decltype(a_tag)::value;
+        if (b_mode == kElements) return LaunchSmallDotMixed<T, AM, kElements>(p, grid, pieces, stream);
+        if constexpr (sizeof(T) == 2) {
+            if (b_mode == kOddPieces) return LaunchSmallDotMixed<T, AM, kOddPieces>(p, grid, pieces, stream);
+        }
+        if constexpr (AM != kPieces) LaunchSmallDotMixed<T, AM, kPieces>(p, grid, pieces, stream);
+    };
+    if (a_mode == kPieces) return with_a(std::integral_constant<int, kPieces>{});
+    if (a_mode == kElements) return with_a(std::integral_constant<int, kElements>{});
+    if constexpr (sizeof(T) == 2) with_a(std::integral_constant<int, kOddPieces>{});
+}
+
+// Which kernel of small_dot.h takes a product.
+enum SmallDotPath { kNoSmallDot, kSmallDotVector, kSmallDotTiles, kSmallDotWhole };  // (whole: tiles whose reduction is not split)
+
+template <typename T>
+SmallDotPath PlanSmallDot(const hipcx_array* a, const hipcx_array* b, SmallDotArgs* p, int* a_mode, int* b_mode) {
+    static const bool enabled = [] { const char* e = getenv("HIPCX_SMALL_DOT"); return e == nullptr || e[0] != '0'; }();
+    const int64_t M = a->shape[0], K = a->shape[1], N = b->shape[1];
+    if (!enabled || !SmallDotShape(M, N, K) || !SmallDotOperands<T>(a, b, p, a_mode, b_mode)) return kNoSmallDot;
+    if (*a_mode != kPieces || *b_mode != kPieces) return kSmallDotTiles;
+    if (M <= 4) return kSmallDotVector;
+    return 2.0 * M * N * K >= 1e9 ? kSmallDotWhole : kSmallDotTiles;  // enough tiles, or enough of them long, to keep the chip busy
+}
+
+template <typename T>
+bool TryTyped(const hipcx_array* a, const hipcx_array* b, const hipcx_array* bias, const hipcx_array* out, float* partial, hipStream_t stream) {
+    const int64_t M = a->shape[0], K = a->shape[1], N = b->shape[1];
+    const int64_t it = sizeof(T);
+    if (out->strides[0] < 0 || out->strides[1] < 0 || out->strides[0] % it || out->strides[1] % it) return false;
+    SmallDotArgs p{};
+    int a_mode = 0, b_mode = 0;
+    const SmallDotPath path = PlanSmallDot<T>(a, b, &p, &a_mode, &b_mode);
+    if (path == kNoSmallDot) return false;
+    p.out = out->data;
+    p.o_row = out->strides[0] / it;
+    p.o_col = out->strides[1] / it;
+    if (bias != nullptr) {
+        p.bias = bias->data;
+        p.bias_stride = bias->strides[0] / it;
+    }
+    ProfileScope prof(stream, 2.0 * M * N * K, static_cast<double>(it) * (M * K + K * N + M * N));
+    if (path == kSmallDotVector) {
+        const dim3 grid(static_cast<unsigned>((N + 3) / 4));
+        if (M == 1) hipLaunchKernelGGL((SmallDotVectorKernel<T, 1>), grid, dim3(256), 0, stream, p);
+        else if (M == 2) hipLaunchKernelGGL((SmallDotVectorKernel<T, 2>), grid, dim3(256), 0, stream, p);
+        else hipLaunchKernelGGL((SmallDotVectorKernel<T, 4>), grid, dim3(256), 0, stream, p);
+        CheckLaunch("small_dot_vector");
+        return true;
+    }
+    p.ksplit = partial != nullptr && path == kSmallDotTiles ? SmallDotSplit(M, N, K, DtypeOf<T>::value) : 1;
+    p.partial = p.ksplit > 1 ? partial : nullptr;
+    LaunchSmallDot<T>(p, a_mode, b_mode, 1, stream);
+    if (p.ksplit > 1) {
+        hipLaunchKernelGGL((SmallDotSumKernel<T>), dim3(static_cast<unsigned>((M * N + 255) / 256)), dim3(256), 0, stream, p);
+        CheckLaunch("small_dot_sum");
+    }
+    return true;
+}
+
+}  // namespace
+
+size_t SmallDotWorkspace(const hipcx_array* a, const hipcx_array* b, int dtype) {
+    if (dtype != HIPCX_FLOAT16 && dtype != HIPCX_FLOAT32) return 0;
+    const size_t bytes = SmallDotPartialBytes(a->shape[0], b->shape[1], a->shape[1], dtype);
+    if (bytes == 0) return 0;  // most products
+    SmallDotArgs p{};
+    int a_mode = 0, b_mode = 0;
+    const SmallDotPath path = dtype == HIPCX_FLOAT16 ? PlanSmallDot<half_t>(a, b, &p, &a_mode, &b_mode) : PlanSmallDot<float>(a, b, &p, &a_mode, &b_mode);
+    return path == kSmallDotTiles ? bytes : 0;
+}
+
+bool TrySmallDot(const hipcx_array* a, const hipcx_array* b, const hipcx_array* bias, const hipcx_array* out, float* partial, hipStream_t stream) {
+    return out->dtype == HIPCX_FLOAT16 ? TryTyped<half_t>(a, b, bias, out, partial, stream) : TryTyped<float>(a, b, bias, out, partial, stream);
+}
+
+bool DotSeveral(const hipcx_array* a0, int64_t a_distance, const hipcx_array* b, const hipcx_array* const* outs, int n, hipStream_t stream) {
+    const int64_t M = a0->shape[0], K = a0->shape[1], N = b->shape[1];
+    SmallDotArgs p{};
+    int a_mode = 0, b_mode = 0;
+    if (n > kSmallDotMaxBatch || !SmallDotShape(M, N, K) || SmallDotSplit(M, N, K, HIPCX_FLOAT32) > 1) return false;
+    if (!SmallDotOperands<float>(a0, b, &p, &a_mode, &b_mode)) return false;
+    for (int i = 0; i < n; ++i) {
+        if (outs[i]->strides[0] != outs[0]->strides[0] || outs[i]->strides[1] != outs[0]->strides[1]) return false;
+        p.outs[i] = outs[i]->data;
+    }
+    if (outs[0]->strides[0] < 0 || outs[0]->strides[1] < 0 || outs[0]->strides[0] % 4 || outs[0]->strides[1] % 4) return false;
+    p.out = outs[0]->data;
+    p.o_row = outs[0]->strides[0] / 4;
+    p.o_col = outs[0]->strides[1] / 4;
+    p.a_batch = a_distance;
+    p.ksplit = 1;
+    ProfileScope prof(stream, 2.0 * M * N * K * n, 4.0 * n * (M * K + K * N + M * N));
+    LaunchSmallDot<float>(p, a_mode, b_mode, n, stream);
+    return true;
+}
+
+}  // namespace hipcx
