@@ -16,6 +16,7 @@
 #include "layout_kernels.h"
 #include "nchw_conv.h"
 #include "pw_conv.h"
+#include "small_conv.h"
 #include "stem_conv.h"
 #include "dot_parts.h"
 
@@ -533,6 +534,25 @@ struct FusedTail {
     int relu = 0;
 };
 
+// w[K][C][R][S] (element strides wsK, wsC, wsR, wsS) -> wp[C/8][R*S][K][8].
+__global__ __launch_bounds__(256) void NchwRepackFiltersKernel(const half_t* w, half_t* wp, int K, int C, int RS, int S, int64_t wsK,
+                                                               int64_t wsC, int64_t wsR, int64_t wsS) {
+    int64_t idx = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;  // one 16-byte group each
+    int64_t total = static_cast<int64_t>(C / 8) * RS * K;
+    if (idx >= total) return;
+    int k = static_cast<int>(idx % K);
+    int64_t t = idx / K;
+    int tap = static_cast<int>(t % RS);
+    int cg = static_cast<int>(t / RS);
+    int r = tap / S, s = tap - r * S;
+    struct alignas(16) G {
+        half_t e[8];
+    } grp;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) grp.e[j] = w[k * wsK + (cg * 8 + j) * wsC + r * wsR + s * wsS];
+    *reinterpret_cast<G*>(wp + idx * 8) = grp;
+}
+
 void RunNchw(const hipcx_array* x, const hipcx_array* w, const hipcx_array* b, const NchwPlan& pl, const int64_t* stride,
              const hipcx_array* out, char* workspace, hipStream_t stream, const FusedTail& tail = FusedTail{}) {
     NchwConvArgs a{};
@@ -574,6 +594,13 @@ void RunNchw(const hipcx_array* x, const hipcx_array* w, const hipcx_array* b, c
     if (pl.taps == 9) {
         a.div_wchunks = FastDiv(a.W / pl.npx);
         a.div_percg = FastDiv(pl.nrow * (a.W / pl.npx));
+    }
+    if (IsContiguous(w) && Aligned(w->data, 16) && SmallConvTakes(a, pl.taps)) {
+        ProfileScope prof(stream, 2.0 * a.M * a.K * RS * a.C,
+                          2.0 * (static_cast<double>(a.N) * a.C * a.H * a.W + static_cast<double>(a.K) * RS * a.C + static_cast<double>(a.M) * a.K));
+        a.wp = static_cast<const half_t*>(w->data);
+        SmallConv(a, pl.taps, stream);
+        return;
     }
     // single-pixel loads of a stride-2 layer over an even width fetch whole dwords (the wanted pixel and its odd neighbour)
     const bool pair_load = pl.taps == 1 && pl.npx == 1 && a.stride == 2 && a.W % 2 == 0;

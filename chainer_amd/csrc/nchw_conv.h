@@ -623,23 +623,4 @@ void NchwConvKernel(NchwConvArgs p) {
     }
 }
 
-// w[K][C][R][S] (element strides wsK, wsC, wsR, wsS) -> wp[C/8][R*S][K][8].
-__global__ __launch_bounds__(256) void NchwRepackFiltersKernel(const half_t* w, half_t* wp, int K, int C, int RS, int S, int64_t wsK,
-                                                               int64_t wsC, int64_t wsR, int64_t wsS) {
-    int64_t idx = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;  // one 16-byte group each
-    int64_t total = static_cast<int64_t>(C / 8) * RS * K;
-    if (idx >= total) return;
-    int k = static_cast<int>(idx % K);
-    int64_t t = idx / K;
-    int tap = static_cast<int>(t % RS);
-    int cg = static_cast<int>(t / RS);
-    int r = tap / S, s = tap - r * S;
-    struct alignas(16) G {
-        half_t e[8];
-    } grp;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) grp.e[j] = w[k * wsK + (cg * 8 + j) * wsC + r * wsR + s * wsS];
-    *reinterpret_cast<G*>(wp + idx * 8) = grp;
-}
-
 }  // namespace hipcx

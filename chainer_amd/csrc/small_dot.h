@@ -323,8 +323,8 @@ __global__ __launch_bounds__(64 * kSmallDotMaxWaves) __attribute__((amdgpu_waves
             const bool in = c * KC + piece * PL < p.K;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                av[st][j] = __builtin_amdgcn_raw_buffer_load_b128(ar, in & (a_line[j] != kOut) ? a_line[j] + c * 128 : kOut, 0, 0);
-                bv[st][j] = __builtin_amdgcn_raw_buffer_load_b128(br, in & (b_line[j] != kOut) ? b_line[j] + c * 128 : kOut, 0, 0);
+                av[st][j] = __builtin_amdgcn_raw_buffer_load_b128(ar, (in & (a_line[j] != kOut)) ? a_line[j] + c * 128 : kOut, 0, 0);
+                bv[st][j] = __builtin_amdgcn_raw_buffer_load_b128(br, (in & (b_line[j] != kOut)) ? b_line[j] + c * 128 : kOut, 0, 0);
             }
         }
     };
