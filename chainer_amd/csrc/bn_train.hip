@@ -10,9 +10,11 @@
 // reference's float16 arithmetic come out the same -- a sum past 65504 is inf, the statistics and the output that follow from it
 // are inf / NaN -- and finite results differ from the composition's only by the order of the float additions inside a sum.
 //
+// Channels that fit the registers of a workgroup take all of it in one launch (BnChannelKernel, BnChannelGradKernel).  Else:
 // Statistics: grid (C, S).  Block (c, s) walks images s, s + S, ... of channel c with 16-byte loads, reduces over the block and
 // stores one partial; the finish kernel adds a channel's S partials in order (deterministic).
 #include "elementwise.h"
+#include "igemm.h"
 
 namespace hipcx {
 namespace {
@@ -132,6 +134,29 @@ struct BnFinishArgs {
     double eps, decay;
 };
 
+// Reciprocal(Sqrt(var + eps)) with eps as a scalar of the array dtype (CX/routines/normalization.cc:141)
+template <typename C, typename P>
+__device__ __forceinline__ C InvStd(C var, double eps) {
+    if constexpr (std::is_same<C, float>::value) {
+        return Rnd<P>(1.0f / Rnd<P>(sqrtf(Rnd<P>(var + Rnd<P>(static_cast<float>(eps))))));
+    } else {
+        return 1.0 / sqrt(var + eps);
+    }
+}
+
+// The state handed out and the running statistics: running *= decay; running += (inv_decay [* count / (count - 1)]) * statistic, scalars in the array
+// dtype (CX/routines/normalization.cc:185-190)
+template <typename C, typename P>
+__device__ __forceinline__ void StoreState(const BnFinishArgs& p, int c, C mean, C var, C inv_std, C old_mean, C old_var) {
+    static_cast<P*>(p.mean_out)[c * p.mo_stride] = static_cast<P>(mean);
+    static_cast<P*>(p.inv_std_out)[c * p.io_stride] = static_cast<P>(inv_std);
+    const C decay = Rnd<P>(static_cast<C>(p.decay));
+    const C inv_decay = Rnd<P>(static_cast<C>(1.0 - p.decay));
+    const C inv_decay_adjusted = Rnd<P>(static_cast<C>((1.0 - p.decay) * (p.count / (p.count - 1.0 > 1.0 ? p.count - 1.0 : 1.0))));
+    static_cast<P*>(p.running_mean)[c * p.rm_stride] = static_cast<P>(Rnd<P>(old_mean * decay) + Rnd<P>(inv_decay * mean));
+    static_cast<P*>(p.running_var)[c * p.rv_stride] = static_cast<P>(Rnd<P>(old_var * decay) + Rnd<P>(inv_decay_adjusted * var));
+}
+
 // STEP 0: mean from the sums.  STEP 1: variance -> inv_std, state outputs, running statistics (CX/routines/normalization.cc:176-191).
 template <typename T, typename P, int STEP>
 __global__ __launch_bounds__(256) void BnFinishKernel(BnFinishArgs p) {
@@ -149,24 +174,10 @@ __global__ __launch_bounds__(256) void BnFinishKernel(BnFinishArgs p) {
     }
     const C mean = static_cast<const C*>(p.mean)[c];
     const C var = Rnd<P>(Rnd<P>(sum) / n);
-    // Reciprocal(Sqrt(var + eps)) with eps as a scalar of the array dtype (CX/routines/normalization.cc:141)
-    C inv_std;
-    if constexpr (std::is_same<C, float>::value) {
-        inv_std = Rnd<P>(1.0f / Rnd<P>(sqrtf(Rnd<P>(var + Rnd<P>(static_cast<float>(p.eps))))));
-    } else {
-        inv_std = 1.0 / sqrt(var + p.eps);
-    }
+    const C inv_std = InvStd<C, P>(var, p.eps);
     static_cast<C*>(p.inv_std)[c] = inv_std;
-    static_cast<P*>(p.mean_out)[c * p.mo_stride] = static_cast<P>(mean);
-    static_cast<P*>(p.inv_std_out)[c * p.io_stride] = static_cast<P>(inv_std);
-    // running *= decay; running += (inv_decay [* count / (count - 1)]) * statistic, scalars in the array dtype (CX/routines/normalization.cc:185-190)
-    const C decay = Rnd<P>(static_cast<C>(p.decay));
-    const C inv_decay = Rnd<P>(static_cast<C>(1.0 - p.decay));
-    const C inv_decay_adjusted = Rnd<P>(static_cast<C>((1.0 - p.decay) * (p.count / (p.count - 1.0 > 1.0 ? p.count - 1.0 : 1.0))));
-    P* rm = static_cast<P*>(p.running_mean) + c * p.rm_stride;
-    P* rv = static_cast<P*>(p.running_var) + c * p.rv_stride;
-    *rm = static_cast<P>(Rnd<P>(static_cast<C>(*rm) * decay) + Rnd<P>(inv_decay * mean));
-    *rv = static_cast<P>(Rnd<P>(static_cast<C>(*rv) * decay) + Rnd<P>(inv_decay_adjusted * var));
+    StoreState<C, P>(p, c, mean, var, inv_std, static_cast<C>(static_cast<const P*>(p.running_mean)[c * p.rm_stride]),
+                     static_cast<C>(static_cast<const P*>(p.running_var)[c * p.rv_stride]));
 }
 
 struct BnApplyArgs {
@@ -268,6 +279,159 @@ __global__ __launch_bounds__(256) void BnApplyKernel(BnApplyArgs p) {
             }
         }
         *reinterpret_cast<Vec<T, VEC>*>(out + v * VEC) = o;
+    }
+}
+
+// ---------------------------------------------------------------------------------------------
+// A channel's values in the registers of one workgroup: the statistics, the state and the result in one launch that reads x (and g) once, where the
+// kernels above are five launches that read x three times, and three that read x and g twice.  A thread keeps NV vectors; loads past the channel's end
+// repeat its last vector, so that none is conditional, and count as nothing.  Bound by memory and, for small channels, by the latency of a load and
+// two sums over the workgroup.  us, forward / gradient, float16 with float32 parameters: [32,256,14,14] 14.1 / 9.9 -> 4.8 / 4.9, [32,512,28,28] 27.0 /
+// 26.0 -> 13.2 / 19.3, [32,256,56,56] 42.5 / 42.6 -> 21.0 / 36.7, [2,64,56,56] 15.3 / 10.4 -> 5.1 / 5.1.
+// ---------------------------------------------------------------------------------------------
+template <typename C, int THREADS>
+__device__ __forceinline__ C BlockTotal(C v, C* lds) {  // the same for every thread
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+    __syncthreads();  // lds may still be read by a previous call
+    if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = v;
+    __syncthreads();
+    C r = C(0);
+#pragma unroll
+    for (int w = 0; w < THREADS / 64; ++w) r += lds[w];
+    return r;
+}
+
+// Offsets (elements) of a thread's vectors, and how many of them are its own.
+template <int VEC, int NV, int THREADS>
+__device__ __forceinline__ int ChannelVectors(int N, int C, uint32_t L, uint32_t (&off)[NV]) {
+    const uint32_t lv = L / VEC, items = static_cast<uint32_t>(N) * lv;
+    int own = 0;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        const uint32_t idx = i * THREADS + threadIdx.x, at = min(idx, items - 1);
+        own += idx < items;
+        const uint32_t n = at / lv, v = at - n * lv;
+        off[i] = (n * static_cast<uint32_t>(C) + blockIdx.x) * L + v * VEC;
+    }
+    return own;
+}
+
+// Keeps the compiler from carrying what it made of a vector (twice its registers) from one phase to the next.
+template <typename V>
+__device__ __forceinline__ void Forget(V& v) {
+    using Raw = std::conditional_t<sizeof(V) == 16, Bytes16, std::conditional_t<sizeof(V) == 8, Bytes8, std::conditional_t<sizeof(V) == 4, unsigned, unsigned short>>>;
+    Raw r = __builtin_bit_cast(Raw, v);
+    asm volatile("" : "+v"(r));
+    v = __builtin_bit_cast(V, r);
+}
+
+template <typename T, typename P, int VEC, int NV, int THREADS>
+__global__ __launch_bounds__(THREADS) void BnChannelKernel(BnFinishArgs f, BnApplyArgs p, int N) {
+    using C = compute_t<T>;
+    __shared__ C lds[THREADS / 64];
+    const int c = blockIdx.x;
+    const T* x = static_cast<const T*>(p.x);
+    T* out = static_cast<T*>(p.out);
+    uint32_t off[NV];
+    const int own = ChannelVectors<VEC, NV, THREADS>(N, p.C, static_cast<uint32_t>(p.L), off);
+    Vec<T, VEC> xv[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) xv[i] = *reinterpret_cast<const Vec<T, VEC>*>(x + off[i]);
+    const C gamma = static_cast<C>(static_cast<const P*>(p.gamma)[c * p.gamma_stride]), beta = static_cast<C>(static_cast<const P*>(p.beta)[c * p.beta_stride]);
+    P* const rm = static_cast<P*>(f.running_mean) + c * f.rm_stride;
+    P* const rv = static_cast<P*>(f.running_var) + c * f.rv_stride;
+    const C old_mean = static_cast<C>(*rm), old_var = static_cast<C>(*rv);
+    const C n = static_cast<C>(f.count);
+    C a = C(0);
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        C t = C(0);
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) t += static_cast<C>(xv[i].v[e]);
+        a += i < own ? t : C(0);
+    }
+    const C mean = Rnd<P>(Rnd<P>(BlockTotal<C, THREADS>(a, lds)) / n);
+    a = C(0);
+#pragma unroll
+    for (int i = 0; i < NV; ++i) Forget(xv[i]);
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        C t = C(0);
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) {
+            const C d = Rnd<P>(static_cast<C>(xv[i].v[e]) - mean);
+            t += Rnd<P>(d * d);
+        }
+        a += i < own ? t : C(0);
+    }
+    const C var = Rnd<P>(Rnd<P>(BlockTotal<C, THREADS>(a, lds)) / n);
+    const C inv_std = InvStd<C, P>(var, f.eps);
+    if (threadIdx.x == 0) StoreState<C, P>(f, c, mean, var, inv_std, old_mean, old_var);
+#pragma unroll
+    for (int i = 0; i < NV; ++i) Forget(xv[i]);
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        Vec<T, VEC> o;
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) {
+            const C t = Rnd<P>(Rnd<P>(static_cast<C>(xv[i].v[e]) - mean) * inv_std);
+            o.v[e] = static_cast<T>(Rnd<P>(t * gamma) + beta);
+        }
+        if (i < own) *reinterpret_cast<Vec<T, VEC>*>(out + off[i]) = o;
+    }
+}
+
+template <typename T, typename P, int VEC, int NV, int THREADS>
+__global__ __launch_bounds__(THREADS) void BnChannelGradKernel(BnApplyArgs p, int N) {
+    using C = compute_t<T>;
+    __shared__ C lds[THREADS / 64];
+    const int c = blockIdx.x;
+    const T* x = static_cast<const T*>(p.x);
+    const T* g = static_cast<const T*>(p.g);
+    T* out = static_cast<T*>(p.out);
+    uint32_t off[NV];
+    const int own = ChannelVectors<VEC, NV, THREADS>(N, p.C, static_cast<uint32_t>(p.L), off);
+    Vec<T, VEC> xv[NV], gv[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        xv[i] = *reinterpret_cast<const Vec<T, VEC>*>(x + off[i]);
+        gv[i] = *reinterpret_cast<const Vec<T, VEC>*>(g + off[i]);
+    }
+    const C m = LoadState<T, P>(p.mean, c, p.state_in_array_dtype, p.mean_stride), is = LoadState<T, P>(p.inv_std, c, p.state_in_array_dtype, p.inv_stride);
+    const C gamma = static_cast<C>(static_cast<const P*>(p.gamma)[c * p.gamma_stride]);
+    C a0 = C(0), a1 = C(0);
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        C t0 = C(0), t1 = C(0);
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) {
+            const C ge = static_cast<C>(gv[i].v[e]);
+            t0 += ge;
+            t1 += Rnd<P>(ge * Rnd<P>(Rnd<P>(static_cast<C>(xv[i].v[e]) - m) * is));
+        }
+        a0 += i < own ? t0 : C(0);
+        a1 += i < own ? t1 : C(0);
+    }
+    const C sg = BlockTotal<C, THREADS>(a0, lds), sgx = BlockTotal<C, THREADS>(a1, lds);
+    if (threadIdx.x == 0) {
+        static_cast<P*>(p.gbeta)[c * p.gb_stride] = static_cast<P>(sg);
+        static_cast<P*>(p.ggamma)[c * p.gg_stride] = static_cast<P>(sgx);
+    }
+#pragma unroll
+    for (int i = 0; i < NV; ++i) Forget(xv[i]), Forget(gv[i]);
+    const C gbeta = Rnd<P>(sg), ggamma = Rnd<P>(sgx);
+    const C inv_n = Rnd<P>(static_cast<C>(1.0 / p.count)), scale = Rnd<P>(gamma * is);
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        Vec<T, VEC> o;
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) {
+            const C x_hat = Rnd<P>(Rnd<P>(static_cast<C>(xv[i].v[e]) - m) * is);
+            const C t = Rnd<P>(Rnd<P>(Rnd<P>(x_hat * ggamma) + gbeta) * inv_n);
+            o.v[e] = static_cast<T>(scale * Rnd<P>(static_cast<C>(gv[i].v[e]) - t));
+        }
+        if (i < own) *reinterpret_cast<Vec<T, VEC>*>(out + off[i]) = o;
     }
 }
 
@@ -399,6 +563,34 @@ void LaunchApply(const BnApplyArgs& a, bool vec, hipStream_t stream) {
     CheckLaunch("batch_norm apply");
 }
 
+// f(VEC, NV, THREADS) as constants for channels that one workgroup's registers hold: NV vectors for each of its threads.  False if they do not.  The
+// gradient, which keeps two arrays, has half the threads and twice the registers where the channel is large; the largest, whose registers spill, need
+// a channel for every compute unit to be faster than three launches (us, [32,256,56,56] 42.6 -> 36.7, but [32,128,56,56] 26.0 -> 29.6).
+template <typename T, bool GRAD, typename F>
+bool VisitChannelShape(const BnTrainGeom& g, int width, F&& f) {
+    if constexpr (sizeof(T) > 4) {
+        return false;  // (float64 keeps the general kernels)
+    } else {
+        constexpr int FULL = 16 / sizeof(T);
+        const int64_t items = static_cast<int64_t>(g.N) * (g.L / width);
+        auto with = [&](auto vec) {
+            constexpr auto vec_c = decltype(vec){};
+            auto call = [&](auto nv, auto threads) { f(vec_c, nv, threads); };
+            using std::integral_constant;
+            if (items <= 4 * 256) call(integral_constant<int, 4>{}, integral_constant<int, 256>{});
+            else if (items <= 8 * 256 && g.C >= NumCUs()) call(integral_constant<int, 8>{}, integral_constant<int, 256>{});
+            else if (items <= 4 * 1024) call(integral_constant<int, 4>{}, integral_constant<int, 1024>{});
+            else if (items <= 8 * 1024) call(integral_constant<int, GRAD ? 16 : 8>{}, integral_constant<int, GRAD ? 512 : 1024>{});
+            else if (items <= 25 * 512 && (!GRAD || g.C >= NumCUs())) call(integral_constant<int, GRAD ? 25 : 13>{}, integral_constant<int, GRAD ? 512 : 1024>{});
+            else return false;
+            return true;
+        };
+        if (width == FULL) return with(std::integral_constant<int, FULL>{});
+        if (width == FULL / 2 && FULL >= 4) return with(std::integral_constant<int, FULL / 2>{});
+        return with(std::integral_constant<int, 1>{});
+    }
+}
+
 void CheckWorkspace(void* workspace, size_t workspace_bytes, size_t need) {
     HIPCX_REQUIRE(workspace != nullptr && workspace_bytes >= need, HIPCX_CHAINERX_ERROR,
                   "batch_norm workspace too small: need " + std::to_string(need) + " bytes");
@@ -495,6 +687,12 @@ int hipcx_batch_norm(const hipcx_array* x, const hipcx_array* gamma, const hipcx
         VisitBnDtypes(x->dtype, pd, [&](auto tag, auto ptag) {
             using T = typename decltype(tag)::type;
             using P = typename decltype(ptag)::type;
+            const bool done = VisitChannelShape<T, false>(g, widths.stat, [&](auto vec, auto nv, auto threads) {
+                hipLaunchKernelGGL((BnChannelKernel<T, P, decltype(vec)::value, decltype(nv)::value, decltype(threads)::value>),
+                                   dim3(static_cast<unsigned>(g.C)), dim3(decltype(threads)::value), 0, st, f, a, g.N);
+                CheckLaunch("batch_norm channels");
+            });
+            if (done) return;
             LaunchStat<T, P, 0>(s, widths.stat, st);
             hipLaunchKernelGGL((BnFinishKernel<T, P, 0>), dim3(cblocks), dim3(256), 0, st, f);
             LaunchStat<T, P, 1>(s, widths.stat, st);
@@ -558,6 +756,12 @@ int hipcx_batch_norm_grad(const hipcx_array* x, const hipcx_array* gamma, const 
         VisitBnDtypes(x->dtype, pd, [&](auto tag, auto ptag) {
             using T = typename decltype(tag)::type;
             using P = typename decltype(ptag)::type;
+            const bool done = VisitChannelShape<T, true>(g, widths.stat, [&](auto vec, auto nv, auto threads) {
+                hipLaunchKernelGGL((BnChannelGradKernel<T, P, decltype(vec)::value, decltype(nv)::value, decltype(threads)::value>),
+                                   dim3(static_cast<unsigned>(g.C)), dim3(decltype(threads)::value), 0, st, a, g.N);
+                CheckLaunch("batch_norm_grad channels");
+            });
+            if (done) return;
             LaunchStat<T, P, 2>(s, widths.stat, st);
             hipLaunchKernelGGL((BnGradFinishKernel<T, P>), dim3(cblocks), dim3(256), 0, st, a);
             CheckLaunch("batch_norm_grad finish");
