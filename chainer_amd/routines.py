@@ -1172,10 +1172,10 @@ def conv_transpose(x, w, b=None, stride=1, pad=0, out_size=None, out_dtype=None)
             bb = b.astype(dt, False).reshape((1, -1, 1, 1)).broadcast_to(out.shape)
             _lib.call('hipcx_add', out.desc(), bb.desc(), out.desc(), current_stream())
         return out
-    # TensorDot(w, x) over the input channels; x goes in channels-last so that both Dot operands have the reduction index as
+    # TensorDot(w, x) over the input channels; both are copied channels-last so that both Dot operands have the reduction index as
     # their unit-stride axis
-    w2 = w.transpose((1, 2, 3, 0)).reshape((w.shape[1] * kh * kw, ci))
-    x2 = x.transpose((0, 2, 3, 1)).reshape((n * h * wd, ci))
+    w2 = w.transpose((1, 2, 3, 0)).copy().reshape((w.shape[1] * kh * kw, ci))
+    x2 = x.transpose((0, 2, 3, 1)).copy().reshape((n * h * wd, ci))
     col = dot(w2, x2.T, dt).reshape((w.shape[1], kh, kw, n, h, wd))   # [C_out, kh, kw, N, H, W]
     col = col.transpose((3, 0, 1, 2, 4, 5))                            # batch axis rolled to the top
     out = col2im(col, stride, pad, out_size)

@@ -45,3 +45,13 @@ def test_special_values_stay_where_they_are(n, c, h, w, k, size, stride):
     f = np.ones((k, c, size, size), np.float16)
     pad = size // 2
     np.testing.assert_array_equal(chx.conv(chx.array(x), chx.array(f), None, stride, pad).get(), O.conv(x, f, None, stride, pad))
+
+
+@pytest.mark.parametrize('size', [1, 3])
+def test_filters_that_are_a_view(size):
+    rng = np.random.default_rng(size)
+    x, f = (rng.standard_normal(s).astype(np.float16) for s in ((2, 64, 7, 7), (64, 40, size, size)))
+    view = chx.array(f).transpose((1, 0, 2, 3))[:, :, ::-1, ::-1]
+    X, pad = chx.array(x), size // 2
+    np.testing.assert_array_equal(chx.conv(X, view, None, 1, pad).get(), chx.conv(X, view.copy(), None, 1, pad).get())
+    assert_close(chx.conv(X, view, None, 1, pad).get(), O.conv(x, f.transpose((1, 0, 2, 3))[:, :, ::-1, ::-1], None, 1, pad), 2e-3, 'conv')
