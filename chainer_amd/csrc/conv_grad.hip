@@ -18,6 +18,7 @@
 // an inf or NaN and, after the product, GradWeightChannelFixupKernel computes the flagged channels' filter taps again the
 // reference's way (the sum over the Im2Col windows, padding multiplied as zeros).  With finite data that kernel's workgroups read
 // one flag each and exit.
+#include "batched_product.h"
 #include "common.h"
 
 namespace hipcx {
@@ -335,18 +336,59 @@ void LaunchBatchedProduct(int dtype, const void* a, int64_t a_row, int64_t a_sli
                           int64_t r_stride = 0, int64_t s_stride = 0);
 
 namespace {
-// A 1x1 filter at stride 1 without padding: gw[k][c] = sum over images of gy_n [K, pixels] @ x_n [C, pixels]^T, which the MFMA kernel
-// reads from gy and x where they lie (rows along the pixels, one matrix per image) -- no Im2Col, no transposed copy of gy.
-// Taken when the planes are whole 16-byte granules and long enough to fill reduction steps (14x14 planes in float16 are 8-byte
-// granules and 3 1/16 steps long: measured no faster than the Im2Col route).
-bool DirectPointwise(const GradWeightPlan& pl, const hipcx_array* x, const hipcx_array* gy, const hipcx_array* gw) {
+// The product behind a weight gradient and the float sums it splits into.  float16 within 2 GiB runs in batched_product.hip.
+struct Product {
+    BatchedOperands o{};  // (of the data type: float32 operands too)
+    int dtype = 0;
+    bool half = false;
+    size_t partial_bytes = 0;
+};
+
+Product PlanProduct(const void* a, int64_t a_row, int64_t a_slice, const void* b, int64_t b_row, int64_t b_slice, int64_t m, int64_t n, int64_t depth, int64_t batch,
+                    void* out, int dtype, int taps_r = 0, int taps_s = 0, int64_t r_stride = 0, int64_t s_stride = 0) {
+    Product pr;
+    BatchedOperands& o = pr.o;
+    o.a = static_cast<const half_t*>(a), o.b = static_cast<const half_t*>(b), o.out = static_cast<half_t*>(out);
+    o.M = static_cast<int>(m), o.N = static_cast<int>(n), o.depth = static_cast<int>(depth), o.batch = static_cast<int>(batch);
+    o.a_row = a_row, o.a_slice = a_slice, o.b_row = b_row, o.b_slice = b_slice;
+    o.taps_r = taps_r, o.taps_s = taps_s, o.r_stride = r_stride, o.s_stride = s_stride;
+    pr.dtype = dtype;
+    pr.half = dtype == HIPCX_FLOAT16 && std::max(std::max(m, n), depth) < (1LL << 31) && HalfProductApplies(o);
+    if (pr.half) {
+        const int slices = HalfProductSlices(m, n, depth, batch);
+        pr.partial_bytes = slices > 1 ? static_cast<size_t>(slices) * m * n * sizeof(float) : 0;
+    } else {
+        pr.partial_bytes = BatchedProductPartialBytes(m, n, depth, o.batch, dtype);
+    }
+    return pr;
+}
+
+void RunProduct(const Product& pr, void* partial, hipStream_t stream) {
+    const BatchedOperands& o = pr.o;
+    float* const sums = pr.partial_bytes ? static_cast<float*>(partial) : nullptr;
+    if (pr.half) HalfProduct(o, sums, HalfProductSlices(o.M, o.N, o.depth, o.batch), stream);
+    else LaunchBatchedProduct(pr.dtype, o.a, o.a_row, o.a_slice, o.b, o.b_row, o.b_slice, o.M, o.N, o.depth, o.batch, o.out, sums, stream, o.taps_r, o.taps_s, o.r_stride, o.s_stride);
+}
+
+// A 1x1 filter at stride 1 without padding: gw[k][c] = sum over images of gy_n [K, pixels] @ x_n [C, pixels]^T, which the matrix kernels
+// read from gy and x where they lie (rows along the pixels, one matrix per image) -- no Im2Col, no transposed copy of gy.
+Product PlanPointwise(const GradWeightPlan& pl, const void* x, const void* gy, void* gw, int dtype) {
+    const GradWeightArgs& a = pl.a;
+    const int64_t pixels = static_cast<int64_t>(a.H) * a.W;
+    return PlanProduct(gy, pixels, a.K * pixels, x, pixels, a.C * pixels, a.K, a.C, pixels, a.N, gw, dtype);
+}
+
+// float16 planes of an even number of pixels, 32 at least, are read in place.  The general kernel takes whole 16-byte granules, long enough to fill
+// reduction steps.
+bool DirectPointwise(const GradWeightPlan& pl, const Product& pr, const hipcx_array* x, const hipcx_array* gy, const hipcx_array* gw) {
     static const bool enabled = [] { const char* e = getenv("HIPCX_GRAD_WEIGHT_DIRECT"); return e == nullptr || e[0] != '0'; }();
     const GradWeightArgs& a = pl.a;
     if (!enabled || a.kh != 1 || a.kw != 1 || a.sh != 1 || a.sw != 1 || a.ph != 0 || a.pw != 0 || a.OH != a.H || a.OW != a.W) return false;
     const int64_t pixels = static_cast<int64_t>(a.H) * a.W;
-    if (pixels < 256 || a.N < 1) return false;
-    return BatchedProductApplies(gy->data, pixels, static_cast<int64_t>(a.K) * pixels, x->data, pixels, static_cast<int64_t>(a.C) * pixels, pixels,
-                                 gw->data, gw->dtype);
+    if (a.N < 1) return false;
+    if (pr.half) return true;
+    return pixels >= 256 && BatchedProductApplies(gy->data, pixels, static_cast<int64_t>(a.K) * pixels, x->data, pixels, static_cast<int64_t>(a.C) * pixels,
+                                                  pixels, gw->data, gw->dtype);
 }
 
 // Filters larger than 1x1 at stride 1: shifted zero-padded copies of x instead of Im2Col (see the top of the file).
@@ -356,6 +398,11 @@ struct ShiftedPlan {
     int64_t depth = 0, plane = 0;  // OH*Wp; Hp*Wp
     size_t xs_bytes = 0, gyp_bytes = 0, partial_bytes = 0, flag_bytes = 0;
 };
+
+Product ShiftedProduct(const ShiftedPlan& sp, const GradWeightArgs& g, void* gw, int dtype) {
+    return PlanProduct(sp.a.gyp, sp.depth, g.K * sp.depth, sp.a.xs, sp.plane, g.C * sp.plane, g.K, static_cast<int64_t>(g.C) * g.kh * g.kw, sp.depth, g.N, gw, dtype, g.kh,
+                       g.kw, sp.a.Wp, static_cast<int64_t>(g.N) * g.C * sp.plane);
+}
 
 ShiftedPlan PlanShifted(const GradWeightPlan& pl, int dtype) {
     ShiftedPlan sp;
@@ -378,9 +425,20 @@ ShiftedPlan PlanShifted(const GradWeightPlan& pl, int dtype) {
     sp.plane = Hp * Wp;
     sp.xs_bytes = RoundUp256(static_cast<size_t>(xs_elems * it));
     sp.gyp_bytes = RoundUp256(static_cast<size_t>(gyp_elems * it));
-    sp.partial_bytes = BatchedProductPartialBytes(g.K, static_cast<int64_t>(g.C) * g.kh * g.kw, sp.depth, g.N, dtype);
+    sp.partial_bytes = ShiftedProduct(sp, g, nullptr, dtype).partial_bytes;
     sp.ok = true;
     return sp;
+}
+
+// The product of the staged operands, whose rows are the pixels of all images.  float16 of an even number of pixels only, and of 1 GFLOP or 2048 pixels at
+// least: the rest are Dots.  (us of the call, batch 8, as
+// product and as Dot: 1024 to 512 channels on 7 x 7, 392 pixels, 15.5, 11.9; 512 to 256 on 14 x 14, 1568 pixels, 18.4, 14.1; 256 to 128 on 28 x 28,
+// 6272 pixels, 20, 33; 1024 to 2048 on 7 x 7, 1.6 GFLOP, 18, 22.5.)
+Product StagedProduct(const GradWeightPlan& pl, void* gw, int dtype) {
+    const int64_t np = pl.gy_t.shape[1];
+    Product pr = PlanProduct(pl.a.gy_t, np, 0, pl.a.col_t, np, 0, pl.a.K, pl.col_view.shape[1], np, 1, gw, dtype);
+    pr.half = pr.half && (np >= 2048 || 2.0 * pl.a.K * pl.col_view.shape[1] * np >= 1e9);
+    return pr;
 }
 
 template <typename T>
@@ -417,8 +475,10 @@ size_t hipcx_conv_grad_weight_workspace_size(const hipcx_array* x, const hipcx_a
         hipcx_array out = GwAsMatrix(gw);
         // Which path the call takes depends on the alignment of the data pointers, which a caller sizing its workspace from
         // descriptors alone may not have yet: the answer covers both.
-        const size_t direct = BatchedProductPartialBytes(pl.a.K, pl.a.C, static_cast<int64_t>(pl.a.H) * pl.a.W, pl.a.N, gw->dtype) + 256;
-        const size_t staged = pl.col_bytes + pl.gyt_bytes + hipcx_dot_workspace_size(&pl.gy_t, &pl.col_view, &out);
+        const int64_t pixels = static_cast<int64_t>(pl.a.H) * pl.a.W;
+        const Product in_place = PlanPointwise(pl, nullptr, nullptr, nullptr, gw->dtype), copied = StagedProduct(pl, nullptr, gw->dtype);
+        const size_t direct = std::max(in_place.partial_bytes, BatchedProductPartialBytes(pl.a.K, pl.a.C, pixels, pl.a.N, gw->dtype)) + 256;
+        const size_t staged = pl.col_bytes + pl.gyt_bytes + std::max(hipcx_dot_workspace_size(&pl.gy_t, &pl.col_view, &out), copied.half ? copied.partial_bytes : 0);
         const ShiftedPlan sp = PlanShifted(pl, gw->dtype);
         const size_t shifted = sp.ok ? sp.xs_bytes + sp.gyp_bytes + sp.partial_bytes + sp.flag_bytes + 256 : 0;
         return std::max(std::max(direct, staged), shifted);
@@ -443,15 +503,12 @@ int hipcx_conv_grad_weight(const hipcx_array* x, const hipcx_array* gy, const in
             HIPCX_REQUIRE(rc == HIPCX_OK, rc, hipcx_last_error());
             return;
         }
-        if (DirectPointwise(pl, x, gy, gw)) {
-            const int64_t pixels = static_cast<int64_t>(pl.a.H) * pl.a.W;
-            const size_t partial_bytes = BatchedProductPartialBytes(pl.a.K, pl.a.C, pixels, pl.a.N, gw->dtype);
-            HIPCX_REQUIRE(partial_bytes == 0 || (workspace != nullptr && workspace_bytes >= partial_bytes), HIPCX_CHAINERX_ERROR,
-                          "conv_grad_weight workspace too small: need " + std::to_string(partial_bytes) + " bytes");
+        const Product in_place = PlanPointwise(pl, x->data, gy->data, gw->data, gw->dtype);
+        if (DirectPointwise(pl, in_place, x, gy, gw)) {
+            HIPCX_REQUIRE(in_place.partial_bytes == 0 || (workspace != nullptr && workspace_bytes >= in_place.partial_bytes), HIPCX_CHAINERX_ERROR,
+                          "conv_grad_weight workspace too small: need " + std::to_string(in_place.partial_bytes) + " bytes");
             HIPCX_REQUIRE(reinterpret_cast<uintptr_t>(workspace) % 16 == 0, HIPCX_CHAINERX_ERROR, "workspace must be 16-byte aligned");
-            LaunchBatchedProduct(gw->dtype, gy->data, pixels, static_cast<int64_t>(pl.a.K) * pixels, x->data, pixels,
-                                 static_cast<int64_t>(pl.a.C) * pixels, pl.a.K, pl.a.C, pixels, pl.a.N, gw->data,
-                                 partial_bytes ? static_cast<float*>(workspace) : nullptr, AsStream(stream));
+            RunProduct(in_place, workspace, AsStream(stream));
             return;
         }
         ShiftedPlan sp = PlanShifted(pl, gw->dtype);
@@ -467,10 +524,7 @@ int hipcx_conv_grad_weight(const hipcx_array* x, const hipcx_array* gy, const in
             if (gw->dtype == HIPCX_FLOAT16) RunShiftedCopies<half_t>(sp.a, st);
             else RunShiftedCopies<float>(sp.a, st);
             const GradWeightArgs& g = pl.a;
-            LaunchBatchedProduct(gw->dtype, sp.a.gyp, sp.depth, static_cast<int64_t>(g.K) * sp.depth, sp.a.xs, sp.plane,
-                                 static_cast<int64_t>(g.C) * sp.plane, g.K, static_cast<int64_t>(g.C) * g.kh * g.kw, sp.depth, g.N, gw->data,
-                                 sp.partial_bytes ? reinterpret_cast<float*>(ws + sp.xs_bytes + sp.gyp_bytes) : nullptr, st, g.kh, g.kw, sp.a.Wp,
-                                 static_cast<int64_t>(g.N) * g.C * sp.plane);
+            RunProduct(ShiftedProduct(sp, g, gw->data, gw->dtype), ws + sp.xs_bytes + sp.gyp_bytes, st);
             if (gw->dtype == HIPCX_FLOAT16) RunChannelFixup<half_t>(g, sp.a.nonfinite, gw->data, st);
             else RunChannelFixup<float>(g, sp.a.nonfinite, gw->data, st);
             return;
@@ -490,6 +544,11 @@ int hipcx_conv_grad_weight(const hipcx_array* x, const hipcx_array* gy, const in
             using T = typename decltype(tag)::type;
             RunLayouts<T>(pl.a, st);
         });
+        const Product copied = StagedProduct(pl, gw->data, gw->dtype);
+        if (copied.half && workspace_bytes >= pl.col_bytes + pl.gyt_bytes + copied.partial_bytes) {
+            RunProduct(copied, ws + pl.col_bytes + pl.gyt_bytes, st);
+            return;
+        }
         int rc = hipcx_dot(&pl.gy_t, &pl.col_view, &out, ws + pl.col_bytes + pl.gyt_bytes, dot_bytes, stream);
         HIPCX_REQUIRE(rc == HIPCX_OK, rc, hipcx_last_error());
     });
