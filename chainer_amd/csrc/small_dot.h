@@ -1,7 +1,7 @@
 // Matrix products with small outputs (batch-sized Linear layers, recurrent steps, weight gradients of small layers):
 // out[M,N] = a[M,K] . b[K,N] with so few elements that 128x128 tiles would occupy a handful of compute units.
 //
-// A workgroup owns one 32x32 tile of `out`; its waves split the reduction axis -- and, with ksplit > 1, so do several workgroups, whose
+// A workgroup owns one 32x32 tile of `out` (SmallDotLinesKernel: 16 to 64 columns); its waves split the reduction axis -- and, with ksplit > 1, so do several workgroups, whose
 // sums another kernel adds up -- each feeding the MFMA from global memory on its own (operands this small live in the caches), and
 // the partial tiles are summed through LDS.  Four kernels, by where the operands lie (chosen in TrySmallDot):
 //   SmallDotKernel        k is the unit-stride axis of both operands (Linear's x and W^T): straight from global memory, bound by the
@@ -265,23 +265,38 @@ __device__ __forceinline__ Bytes16 MaskPiece(Bytes16 v, int k, int K) {
     return v;
 }
 
-// Both operands in pieces.  A wave takes chunks of 128 bytes per row: whole lines (8 lanes to a row, 8 rows to an instruction), turned round in LDS of
-// its own.  Two chunks are in flight while a third is multiplied; the loads' offsets are constants plus a scalar, and only the chunk that holds the end
-// of K looks at it.  Bound by the matrix pipe and by the delivery of operands (64 rows for 1024 outputs) in about equal parts.  us, against one chunk in
-// flight and three or more waves to a tile: float32 [1024,1024]^2 33.4 -> 26.5, [1000,784] . [784,1000] 27.4 -> 22.6, [256,1024] . [1024,1024] 11.4 ->
-// 9.6 (against SmallDotKernel); float16 15.4 -> 10.5, 13.3 -> 11.0, 6.6 -> 5.1, [37,2048] . [2048,1000] 9.8 -> 6.1.
+// 16 x 16 outputs from 16 bytes of 16 rows of a and b, the k of a piece in any order as long as both operands keep to it.
 template <typename T>
+__device__ __forceinline__ void MfmaBlock(const Bytes16& a, const Bytes16& b, float4_t& acc) {
+    if constexpr (sizeof(T) == 2) {
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, a), __builtin_bit_cast(half8_t, b), acc, 0, 0, 0);
+    } else {
+        const float4_t af = __builtin_bit_cast(float4_t, a), bf = __builtin_bit_cast(float4_t, b);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(af[e], bf[e], acc, 0, 0, 0);
+    }
+}
+
+// Both operands in pieces; tiles of 32 rows and 16 * NB columns.  A wave takes chunks of 128 bytes per row: whole lines (8 lanes to a row, 8 rows to an
+// instruction), turned round in LDS of its own.  Two chunks are in flight while a third is multiplied; the loads' offsets are constants plus a scalar, and
+// only the chunk that holds the end of K looks at it.  Bound by the matrix pipe and by the delivery of operands (64 rows for 1024 outputs) in about equal
+// parts, and by tiles that are not dealt out evenly: hence the widths.  us, against one chunk in flight and three or more waves to a tile: float32
+// [1024,1024]^2 33.4 -> 26.7, [1000,784] . [784,1000] 27.4 -> 22.5, [256,1024] . [1024,1024] 11.4 -> 9.4 (against SmallDotKernel); float16 15.4 -> 10.7,
+// 13.3 -> 11.2, 6.6 -> 5.0, [37,2048] . [2048,1000] 9.8 -> 5.1.
+template <typename T, int NB>
 __global__ __launch_bounds__(64 * kSmallDotMaxWaves) __attribute__((amdgpu_waves_per_eu(2, 8))) void SmallDotLinesKernel(SmallDotArgs p) {
     constexpr int PL = 16 / sizeof(T);
     constexpr int KC = 8 * PL;  // k per chunk
     constexpr int kOut = 0x7fffffff;
+    constexpr int BL = 2 * NB;  // loads of b per chunk, 8 rows each
+    constexpr int kStage = (32 + 16 * NB) * kSmallDotPitch, kPitch = 16 * NB + 1;
     extern __shared__ __align__(16) char lds[];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: the loop below runs on scalar control flow
-    const int lr = lane & 31;
-    const int g = lane >> 5;
+    const int lr = lane & 15;
+    const int g = lane >> 4;
     const int piece = lane & 7, sub = lane >> 3;
     const int tiles = p.tiles_m * p.tiles_n;
     const int split = blockIdx.x / tiles;
@@ -290,14 +305,18 @@ __global__ __launch_bounds__(64 * kSmallDotMaxWaves) __attribute__((amdgpu_waves
     const int batch = blockIdx.y;
     const __amdgpu_buffer_rsrc_t ar = MakeRsrc(static_cast<const T*>(p.a) + batch * p.a_batch, p.a_bytes);
     const __amdgpu_buffer_rsrc_t br = MakeRsrc(p.b, p.b_bytes);
-    int a_line[4], b_line[4];
+    int a_line[4], b_line[BL];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        const int m = tm * 32 + j * 8 + sub, n = tn * 32 + j * 8 + sub;
+        const int m = tm * 32 + j * 8 + sub;
         a_line[j] = m < p.M ? static_cast<int>((m * p.a_row + piece * PL) * static_cast<int64_t>(sizeof(T))) : kOut;
+    }
+#pragma unroll
+    for (int j = 0; j < BL; ++j) {
+        const int n = tn * 16 * NB + j * 8 + sub;
         b_line[j] = n < p.N ? static_cast<int>((n * p.b_col + piece * PL) * static_cast<int64_t>(sizeof(T))) : kOut;
     }
-    char* const a_stage = lds + wave * 2 * kSmallDotStage;
+    char* const a_stage = lds + wave * kStage;
     char* const to = a_stage + sub * kSmallDotPitch + piece * 16;
     const char* const from = a_stage + lr * kSmallDotPitch + g * 16;
 
@@ -308,49 +327,51 @@ __global__ __launch_bounds__(64 * kSmallDotMaxWaves) __attribute__((amdgpu_waves
     const int per_wave = (max(s_end - s_begin, 0) + p.nw - 1) / p.nw;
     const int begin = s_begin + wave * per_wave, end = min(s_end, begin + per_wave);
 
-    float16_t acc;
+    float4_t acc[2][NB];
 #pragma unroll
-    for (int v = 0; v < 16; ++v) acc[v] = 0.f;
-    Bytes16 av[2][4], bv[2][4];
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) acc[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
+    Bytes16 av[2][4], bv[2][BL];
     auto load = [&](int st, int c) {
         if ((c + 1) * KC <= p.K) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                av[st][j] = __builtin_amdgcn_raw_buffer_load_b128(ar, a_line[j], c * 128, 0);
-                bv[st][j] = __builtin_amdgcn_raw_buffer_load_b128(br, b_line[j], c * 128, 0);
-            }
+            for (int j = 0; j < 4; ++j) av[st][j] = __builtin_amdgcn_raw_buffer_load_b128(ar, a_line[j], c * 128, 0);
+#pragma unroll
+            for (int j = 0; j < BL; ++j) bv[st][j] = __builtin_amdgcn_raw_buffer_load_b128(br, b_line[j], c * 128, 0);
         } else {  // pieces beyond K are not read
             const bool in = c * KC + piece * PL < p.K;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                av[st][j] = __builtin_amdgcn_raw_buffer_load_b128(ar, (in & (a_line[j] != kOut)) ? a_line[j] + c * 128 : kOut, 0, 0);
-                bv[st][j] = __builtin_amdgcn_raw_buffer_load_b128(br, (in & (b_line[j] != kOut)) ? b_line[j] + c * 128 : kOut, 0, 0);
-            }
+            for (int j = 0; j < 4; ++j) av[st][j] = __builtin_amdgcn_raw_buffer_load_b128(ar, (in & (a_line[j] != kOut)) ? a_line[j] + c * 128 : kOut, 0, 0);
+#pragma unroll
+            for (int j = 0; j < BL; ++j) bv[st][j] = __builtin_amdgcn_raw_buffer_load_b128(br, (in & (b_line[j] != kOut)) ? b_line[j] + c * 128 : kOut, 0, 0);
         }
     };
     auto multiply = [&](int st, int c, auto&& next) {
         if ((c + 1) * KC > p.K) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                av[st][j] = MaskPiece<T>(av[st][j], c * KC + piece * PL, p.K);
-                bv[st][j] = MaskPiece<T>(bv[st][j], c * KC + piece * PL, p.K);
-            }
+            for (int j = 0; j < 4; ++j) av[st][j] = MaskPiece<T>(av[st][j], c * KC + piece * PL, p.K);
+#pragma unroll
+            for (int j = 0; j < BL; ++j) bv[st][j] = MaskPiece<T>(bv[st][j], c * KC + piece * PL, p.K);
         }
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            *reinterpret_cast<Bytes16*>(to + j * 8 * kSmallDotPitch) = av[st][j];
-            *reinterpret_cast<Bytes16*>(to + kSmallDotStage + j * 8 * kSmallDotPitch) = bv[st][j];
-        }
+        for (int j = 0; j < 4; ++j) *reinterpret_cast<Bytes16*>(to + j * 8 * kSmallDotPitch) = av[st][j];
+#pragma unroll
+        for (int j = 0; j < BL; ++j) *reinterpret_cast<Bytes16*>(to + kSmallDotStage + j * 8 * kSmallDotPitch) = bv[st][j];
         next();
         __builtin_amdgcn_wave_barrier();
-        Bytes16 fa[4], fb[4];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            fa[q] = *reinterpret_cast<const Bytes16*>(from + q * 32);
-            fb[q] = *reinterpret_cast<const Bytes16*>(from + kSmallDotStage + q * 32);
+        for (int q = 0; q < 2; ++q) {  // pieces g and g + 4 of each row
+            Bytes16 fa[2], fb[NB];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) fa[i] = *reinterpret_cast<const Bytes16*>(from + i * 16 * kSmallDotPitch + q * 64);
+#pragma unroll
+            for (int j = 0; j < NB; ++j) fb[j] = *reinterpret_cast<const Bytes16*>(from + kSmallDotStage + j * 16 * kSmallDotPitch + q * 64);
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < NB; ++j) MfmaBlock<T>(fa[i], fb[j], acc[i][j]);
         }
-#pragma unroll
-        for (int q = 0; q < 4; ++q) MfmaTile<T>(fa[q], fb[q], acc);
         __builtin_amdgcn_wave_barrier();
     };
     if (begin < end) {
@@ -369,19 +390,24 @@ __global__ __launch_bounds__(64 * kSmallDotMaxWaves) __attribute__((amdgpu_waves
         if (c + 2 < end) multiply(0, c + 2, [] {});
     }
     __syncthreads();  // the staging areas become the partial tiles
-    // lane holds column lr, rows 8*(v/4) + 4*g + v%4
+    // lane holds column lr, rows 4 * g + v of each block
+    constexpr int kPart = 32 * kPitch;
     float* const part = reinterpret_cast<float*>(lds);
-    float* const mine = part + wave * kSmallDotPart;
+    float* const mine = part + wave * kPart;
 #pragma unroll
-    for (int v = 0; v < 16; ++v) mine[(8 * (v / 4) + 4 * g + (v % 4)) * 33 + lr] = acc[v];
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) mine[(i * 16 + 4 * g + v) * kPitch + j * 16 + lr] = acc[i][j][v];
     __syncthreads();
     T* out = static_cast<T*>(gridDim.y > 1 ? p.outs[batch] : p.out);
-    for (int e = tid; e < 32 * 32; e += 64 * p.nw) {
-        const int row = e >> 5, col = e & 31;
-        const int om = tm * 32 + row, on = tn * 32 + col;
+    for (int e = tid; e < 32 * 16 * NB; e += 64 * p.nw) {
+        const int row = e / (16 * NB), col = e - row * (16 * NB);
+        const int om = tm * 32 + row, on = tn * 16 * NB + col;
         if (om >= p.M || on >= p.N) continue;
         float s = 0.f;
-        for (int w = 0; w < p.nw; ++w) s += part[w * kSmallDotPart + row * 33 + col];
+        for (int w = 0; w < p.nw; ++w) s += part[w * kPart + row * kPitch + col];
         StoreTileElement<T>(p, split, out, om, on, s);
     }
 }

@@ -86,11 +86,32 @@ void LaunchSmallDotMixed(const SmallDotArgs& p, dim3 grid, int pieces, hipStream
     LaunchSmallDotPieces<T, AM, BM, 4>(p, grid, stream);
 }
 
-// Whether whole lines regrouped through LDS (SmallDotLinesKernel) beat loads straight into the MFMA layout (SmallDotKernel) for `groups` workgroups of
-// `k` terms each: once most compute units have a tile of some length, or a tile is long.  us, SmallDotKernel and lines: float32 128 tiles
-// of 784 terms 7.2 and 8.6, 164 of 650 7.1 and 8.2, 256 of 1024 11.4 and 9.6, 484 of 300 9.0 and 8.6; float16 64 of 2048 9.8 and 6.1, 128 of 1000 5.0
-// and 5.3, 484 of 300 4.7 and 5.6.
-bool TakesLines(int64_t groups, int64_t k, int item) { return (groups > NumCUs() * 3 / 4 && k * item > 7 * 128) || k >= 1536; }
+// Columns, in 16s, of the tiles of whole lines regrouped through LDS (SmallDotLinesKernel); 0: loads straight into the MFMA layout (SmallDotKernel) are
+// faster.  `rows` tiles of 32 rows, each of whose reductions of `k` terms `parts` workgroups share.  Tiles take the narrowest width that finds each of
+// them a compute unit, and long enough reductions: below, the detour through LDS outweighs the lines.  us, SmallDotKernel, then tiles of 16, 32, 48 and 64 columns:
+//   float32  [100,300] . [300,1000]  4.7  5.0  6.2              [100,1000] . [1000,1000]  8.5  7.4  9.1 11.3
+//            [256,800] . [800,1000]  9.4  9.3  9.0 11.2         [64,1300] . [1300,2600]  10.6 13.2 11.6        [256,1024] . [1024,1024] 11.4 10.1 9.4 11.5
+//            [128,300] . [300,2600]  6.9  7.6  8.0  8.4  9.6    [128,650] . [650,2600]   12.2 12.0 12.4 11.1 12.7
+//            [300,300] . [300,1500]  7.7  9.2  8.5 14.2 10.2    [300,650] . [650,1500]   13.9 14.7 13.2 19.1 13.7
+//   float16  [100,650] . [650,1000]  4.2  4.3  4.7              [37,2048] . [2048,1000]   9.7  5.1  6.1  7.3
+//            [128,300] . [300,2600]  4.2  4.9  7.9  5.5  6.5    [128,650] . [650,2600]    6.5  6.5  8.0  5.9  6.6
+//            [300,300] . [300,1500]  4.6  5.9  8.0  9.2  6.7    [500,1000] . [1000,1000]  9.5  8.8 10.3 11.3  8.3
+// 64 columns in float32: within 3 % of 32.  More tiles than compute units at any width: 484 of 300 terms 9.0 and 8.6 (float32, 32 columns), 4.7 and 5.6
+// (float16); [150,1024] . [1024,4096] 21.7 20.3 19.8 21.8 27.5, [1024,1024]^2 in float16 15.3 12.6 10.9 11.3 12.1.
+template <typename T>
+int LinesBlocks(int64_t rows, int64_t n, int64_t parts, int64_t k) {
+    constexpr bool kHalf = sizeof(T) == 2;
+    const int64_t cus = NumCUs(), bytes = k * static_cast<int64_t>(sizeof(T)), least = kHalf ? 800 : 1600;
+    auto groups = [&](int blocks) { return rows * ((n + 16 * blocks - 1) / (16 * blocks)) * parts; };
+    if (groups(1) <= cus) return bytes >= 1600 ? 1 : 0;
+    if (groups(2) <= cus) {
+        if (kHalf) return bytes >= 1600 ? 2 : 0;
+        return bytes >= 6144 || (bytes >= 4096 && groups(2) > cus * 3 / 4) ? 2 : 0;
+    }
+    if (groups(3) <= cus) return bytes >= least ? 3 : 0;
+    if (kHalf && groups(4) <= cus) return bytes >= least ? 4 : 0;
+    return bytes > (groups(2) > 2 * cus ? 7 * 128 : least) ? 2 : 0;
+}
 
 // Their waves: eight keep most loads in flight while a compute unit has one or two tiles (328 float32 tiles of 21 chunks: 12.3 us, 12.8 with four, 16.6
 // with two); beyond, what leaves the busiest SIMD the fewest chunks, fewer waves on near terms (626 tiles of 21 chunks: 17.6 us with two, 18.2 with three, 16.5 with four; 1252 of
@@ -113,18 +134,26 @@ void LaunchSmallDot(SmallDotArgs p, int a_mode, int b_mode, int batch, hipStream
     const dim3 grid(static_cast<unsigned>(tiles * p.ksplit), static_cast<unsigned>(batch));
     if (a_mode == kPieces && b_mode == kPieces) {
         const int chunks = ((p.K * static_cast<int>(sizeof(T)) + 127) / 128 + p.ksplit - 1) / p.ksplit;
-        const int64_t groups = tiles * p.ksplit * batch;
-        if (!TakesLines(groups, p.K / p.ksplit, sizeof(T))) {
-            hipLaunchKernelGGL((SmallDotKernel<T>), grid, dim3(512), 0, stream, p);
-            CheckLaunch("small_dot");
-            return;
+        auto lines = [&](auto blocks_tag) {
+            constexpr int NB = decltype(blocks_tag)::value, kWaveBytes = (32 + 16 * NB) * kSmallDotPitch;
+            p.tiles_n = (p.N + 16 * NB - 1) / (16 * NB);
+            const int64_t groups = static_cast<int64_t>(p.tiles_m) * p.tiles_n * p.ksplit;
+            p.nw = LinesWaves(groups * batch, chunks);
+            struct LinesTag {};
+            EnsureDynamicLds<LinesTag>(reinterpret_cast<const void*>(SmallDotLinesKernel<T, NB>), kSmallDotMaxWaves * kWaveBytes);
+            hipLaunchKernelGGL((SmallDotLinesKernel<T, NB>), dim3(static_cast<unsigned>(groups), static_cast<unsigned>(batch)), dim3(64 * p.nw), p.nw * kWaveBytes,
+                               stream, p);
+            CheckLaunch("small_dot_lines");
+        };
+        switch (LinesBlocks<T>(p.tiles_m, p.N, static_cast<int64_t>(p.ksplit) * batch, p.K / p.ksplit)) {
+            case 1: return lines(std::integral_constant<int, 1>{});
+            case 2: return lines(std::integral_constant<int, 2>{});
+            case 3: return lines(std::integral_constant<int, 3>{});
+            case 4:
+                if constexpr (sizeof(T) == 2) return lines(std::integral_constant<int, 4>{});
         }
-        p.nw = LinesWaves(groups, chunks);
-        constexpr int kWaveBytes = 2 * kSmallDotStage;
-        struct LinesTag {};
-        EnsureDynamicLds<LinesTag>(reinterpret_cast<const void*>(SmallDotLinesKernel<T>), kSmallDotMaxWaves * kWaveBytes);
-        hipLaunchKernelGGL((SmallDotLinesKernel<T>), grid, dim3(64 * p.nw), p.nw * kWaveBytes, stream, p);
-        CheckLaunch("small_dot_lines");
+        hipLaunchKernelGGL((SmallDotKernel<T>), grid, dim3(512), 0, stream, p);
+        CheckLaunch("small_dot");
         return;
     }
     // Elements come as they are used: chunks of 32 bytes, six of them in flight, beat whole lines ([32,1000] . [1000,2048] float16 14.3 -> 5.5 us,

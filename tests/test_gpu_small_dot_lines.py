@@ -1,4 +1,4 @@
-"""Small matrix products over whole 128-byte lines (SmallDotLinesKernel): edges of tiles, lines and 16-byte pieces, one wave to eight, split
+"""Small matrix products over whole 128-byte lines (SmallDotLinesKernel): edges of tiles of every width, lines and 16-byte pieces, one wave to eight, split
 reductions, and what lies behind an operand's rows."""
 import numpy as np
 import pytest
@@ -13,6 +13,7 @@ pytestmark = pytest.mark.gpu
     (5, 1536, 10), (33, 1538, 65), (64, 4099 * 2, 40),             # few long tiles, one of them split
     (512, 450, 512), (545, 458, 450), (800, 66 * 7, 33 * 32),      # one or two tiles to a compute unit
     (1025, 514, 1000), (1500, 322, 1100), (900, 70 * 8, 1500),     # more
+    (100, 802, 1001), (7, 1030, 17), (130, 802, 2390), (300, 450, 1489), (290, 514, 1300),  # 16, 48 and 64 columns
 ])
 def test_rows_in_pieces(dt, m, k, n):
     rng = np.random.default_rng(k)
