@@ -1327,18 +1327,19 @@ namespace {
 // reduction axis is not the unit-stride one (or whose rows are not dword-aligned) laid out anew, then the partial sums.
 struct GemmPpPlan {
     int slices = 0;  // 0: left to the other kernels
+    bool cols_a = false, cols_b = false;    // read k by k as they lie
     bool stage_a = false, stage_b = false;
     int64_t pitch = 0;  // of a staged row, elements
     size_t a_bytes = 0, b_bytes = 0, partial_bytes = 0;
     size_t Total() const { return a_bytes + b_bytes + partial_bytes; }
 };
 
-// The estimates, in us, are fits to measured products.  256 x 256 tiles: 0.85 for a chunk of 32 k, 5 for a tile's start and end, one tile at a time on
-// a compute unit, the result at 5 TB/s (nothing else runs meanwhile), partial sums written and read at 4 TB/s, staging at 3.5 TB/s.  The 128 x 128
-// kernel: 450 TFLOP/s on rows of 16-byte pieces, 350 of 8.  The 32 x 32 tiles of small outputs: 130, a third of it for operands read element by element.
-// The large tiles have to win by a fifth.  Against every choice on 84 products (28 shapes in three layouts) the one made is within 10 % of the best
-// for 62.  Farthest off: a round of large tiles that is not full is priced too high ([1793,642] . [642,2563] 45.8 us, 24.0 on large tiles), small
-// tiles over operands read element by element too (1024^3 with a row-major b 27.5 us, 15.8 on small tiles).
+// The estimates, in us, are fits to measured products (572 of this kernel, 232 of the others; 57 shapes of 60 to 10000 in every layout).  256 x 256 tiles: 0.54
+// for a chunk of 32 k, 0.76 when the whole chip fetches, 6.5 for a tile's start and end, one tile at a time on a compute unit, the result at 4.3 TB/s
+// (nothing else runs meanwhile), partial sums written and read at 7.3 TB/s; operands in an order of neither kind are staged at 3.5 TB/s.  The other
+// kernels, by the operands whose reduction axis is dense (both, one, none), for outputs small enough for 32 x 32 tiles and for larger ones: a start, the
+// operations, the bytes and the length of the reduction.  The one chosen takes 2 to 3 % longer than the best of all of them and all splits on
+// average; by more than 15 % for 6 of 116.
 GemmPpPlan PlanGemmPp(const hipcx_array* a, const hipcx_array* b, const hipcx_array* out) {
     GemmPpPlan pl;
     static const bool enabled = [] { const char* e = getenv("HIPCX_DOT_PP"); return e == nullptr || e[0] != '0'; }();
@@ -1355,22 +1356,32 @@ GemmPpPlan PlanGemmPp(const hipcx_array* a, const hipcx_array* b, const hipcx_ar
     auto fits = [&](const void* ptr, int64_t line, int64_t k_stride) {
         return k_stride == 2 && reinterpret_cast<uintptr_t>(ptr) % 4 == 0 && line % 4 == 0 && line >= 2 * k && 128 * line + 2 * k < (1LL << 30);
     };
+    auto fits_cols = [&](const void* ptr, int64_t line_stride, int64_t k_stride, int64_t lines) {
+        return line_stride == 2 && reinterpret_cast<uintptr_t>(ptr) % 4 == 0 && k_stride % 4 == 0 && k_stride >= 2 * lines && (k + 64) * k_stride < (1LL << 30);
+    };
     pl.stage_a = !fits(a->data, a->strides[0], a->strides[1]);
     pl.stage_b = !fits(b->data, b->strides[1], b->strides[0]);
-    const double flops = 2.0 * m * n * k, out_us = 2.0 * m * n / 5e6;
+    pl.cols_a = pl.stage_a && fits_cols(a->data, a->strides[0], a->strides[1], m);
+    pl.cols_b = pl.stage_b && fits_cols(b->data, b->strides[1], b->strides[0], n);
+    if (pl.cols_a) pl.stage_a = false;
+    if (pl.cols_b) pl.stage_b = false;
+    const double flops = 2.0 * m * n * k, bytes = 2.0 * (static_cast<double>(m) * n + static_cast<double>(m) * k + static_cast<double>(n) * k), outs = static_cast<double>(m) * n;
+    const int dense = (a->strides[1] == 2) + (b->strides[0] == 2);
+    struct Fit {
+        double start, flops, bytes, k;
+    };
+    static constexpr Fit kSmall[3] = {{3.6, 190e6, 1.6e6, 3.2e-3}, {4.0, 135e6, 3e6, 1.3e-3}, {3.6, 186e6, 14e6, 0.45e-3}};
+    static constexpr Fit kLarge[3] = {{17, 990e6, 2.8e6, 10e-3}, {15, 830e6, 4e6, 9e-3}, {12.6, 571e6, 1e9, 7e-3}};
+    const Fit& fit = (SmallDotShape(m, n, k) ? kSmall : kLarge)[dense];
+    double least = 0.95 * (fit.start + flops / fit.flops + bytes / fit.bytes + k * fit.k);
     auto stage_us = [&](bool needed, int64_t lines) { return needed ? 2.0 + 4.0 * lines * k / 3.5e6 : 0.0; };
-    const bool small = SmallDotShape(m, n, k), rows = a->strides[1] == 2 && b->strides[0] == 2;
-    const bool wide = rows && k % 8 == 0 && a->strides[0] % 16 == 0 && b->strides[1] % 16 == 0;
-    double other;
-    if (small) other = std::max(8.0, flops / (rows ? 130e6 : 45e6));
-    else other = 4.0 + out_us + flops / (!rows || wide ? 450e6 : 350e6) + stage_us(a->strides[1] != 2, m) + stage_us(b->strides[0] != 2, n);
-    // (on equal terms they may be level: most of the time of short reductions goes into the result)
-    double least = (wide && k % 32 == 0 && tiles >= (NumCUs() * 3) / 4 ? 1.05 : 0.8) * other;
+    const double staging = stage_us(pl.stage_a, m) + stage_us(pl.stage_b, n);
     for (int s = 1; s <= 16 && chunks / s >= 8 * (s > 1); ++s) {
         // every slice has work for the pipeline's prologue
-        if (chunks - (s - 1) * ((chunks + s - 1) / s) < gemm_pp::kMinK / 32) continue;
-        const int64_t rounds = (tiles * s + NumCUs() - 1) / NumCUs();
-        const double t = rounds * (((chunks + s - 1) / s) * 0.85 + 5.0) + (s > 1 ? 2.0 + 8.0 * s * m * n / 4e6 : out_us) + stage_us(pl.stage_a, m) + stage_us(pl.stage_b, n);
+        const int64_t each = (chunks + s - 1) / s, groups = tiles * s, rounds = (groups + NumCUs() - 1) / NumCUs();
+        if (chunks - (s - 1) * each < gemm_pp::kMinK / 32) continue;
+        const double chunk = 0.54 + 0.22 * std::min(1.0, static_cast<double>(groups) / NumCUs());
+        const double t = 2.5 + rounds * (each * chunk + 6.5) + (s > 1 ? 5.5 + 8.0 * s * outs / 7.3e6 : 2.0 * outs / 4.3e6) + staging;
         if (t < least) least = t, pl.slices = s;
     }
     pl.a_bytes = pl.stage_a ? RoundUpTo(static_cast<size_t>(m * pl.pitch * 2), 256) : 0;
@@ -1395,8 +1406,8 @@ bool TryGemmPp(const hipcx_array* a, const hipcx_array* b, const hipcx_array* bi
     p.M = static_cast<int>(M);
     p.N = static_cast<int>(N);
     p.K = static_cast<int>(K);
-    p.lda = static_cast<int>(a->strides[0] / 2);
-    p.ldb = static_cast<int>(b->strides[1] / 2);
+    p.lda = static_cast<int>(a->strides[space.cols_a ? 1 : 0] / 2);
+    p.ldb = static_cast<int>(b->strides[space.cols_b ? 0 : 1] / 2);
     p.ldc = static_cast<int>(out->strides[0] / 2);
     if (space.stage_a) {
         half_t* const to = reinterpret_cast<half_t*>(ws);
@@ -1420,15 +1431,21 @@ bool TryGemmPp(const hipcx_array* a, const hipcx_array* b, const hipcx_array* bi
     }
     ProfileScope prof(stream, 2.0 * static_cast<double>(M) * N * K, 2.0 * (static_cast<double>(M) * K + static_cast<double>(N) * K + static_cast<double>(M) * N));
     const unsigned grid = static_cast<unsigned>((static_cast<int64_t>(p.tiles_m) * p.tiles_n * slices + 7) / 8 * 8);
-    auto launch = [&](auto direct) {
-        constexpr bool DIRECT = decltype(direct)::value;
+    auto launch = [&](auto direct, auto cols_a, auto cols_b) {
+        constexpr bool DIRECT = decltype(direct)::value, A_COLS = decltype(cols_a)::value, B_COLS = decltype(cols_b)::value;
         struct GemmPpTag {};
-        EnsureDynamicLds<GemmPpTag>(reinterpret_cast<const void*>(gemm_pp::GemmPpKernel<DIRECT>), gemm_pp::kLdsBytes);
-        hipLaunchKernelGGL(gemm_pp::GemmPpKernel<DIRECT>, dim3(grid), dim3(512), gemm_pp::kLdsBytes, stream, p);
+        const auto kernel = gemm_pp::GemmPpKernel<DIRECT, A_COLS, B_COLS>;
+        EnsureDynamicLds<GemmPpTag>(reinterpret_cast<const void*>(kernel), gemm_pp::kLdsBytes);
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(512), gemm_pp::kLdsBytes, stream, p);
     };
     // short reductions: see the epilogue
-    if (slices == 1 && K <= 256 && N % 4 == 0 && p.ldc % 4 == 0 && Aligned(p.c, 8)) launch(std::true_type{});
-    else launch(std::false_type{});
+    const std::true_type yes{};
+    const std::false_type no{};
+    if (space.cols_a && space.cols_b) launch(no, yes, yes);
+    else if (space.cols_a) launch(no, yes, no);
+    else if (space.cols_b) launch(no, no, yes);
+    else if (slices == 1 && K <= 256 && N % 4 == 0 && p.ldc % 4 == 0 && Aligned(p.c, 8)) launch(yes, no, no);
+    else launch(no, no, no);
     CheckLaunch("gemm_pp");
     if (slices > 1) {
         const int64_t threads = M * ((N + 7) / 8);

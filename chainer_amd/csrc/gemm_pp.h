@@ -12,10 +12,12 @@
 // ahead, read the 12 fragments of the current chunk) and an MFMA phase (16 MFMAs on registers), half a period apart and
 // separated by workgroup barriers: while one wave of a SIMD multiplies, the other one feeds.
 // k may be any number: the last chunk is masked in registers; rows need dword alignment only.  Where tiles leave compute units idle the
-// reduction is split over `slices` workgroups, whose float sums GemmSumKernel adds up.
+// reduction is split over `slices` workgroups, whose float sums GemmSumKernel adds up.  An operand that lies k by k (the weights of a gradient, both
+// operands of a weight gradient) is loaded as it lies and turned round by transposing LDS reads.
 // Bound by the matrix pipes and, in short reductions, by writing c.  us, against 128 x 128 tiles over padded copies of the operands:
 // [4480,650] . [650,10000] 126 -> 95, [4480,10000] . [10000,650] 188 -> 115, [10000,4480] . [4480,650] with a and b transposed 198 -> 130;
-// [4096,4096]^2 126 (1089 TFLOP/s).
+// [4096,4096]^2 126 (1089 TFLOP/s).  Against copies with the reduction axis dense: [4480,10000] . [10000,650], b k by k, 104 -> 86; [10000,4480] .
+// [4480,650], a and b, 130 -> 85; [4096,4480] . [4480,1024], a and b, 116 -> 57; [4096,4096]^2 152 -> 125.
 // Tiles are ordered so that the 32 workgroups an XCD runs at a time cover `band` tile rows x 32 / band tile columns: they
 // share operand rows in that XCD's L2.
 #pragma once
@@ -33,7 +35,7 @@ struct GemmArgs {
     const half_t* b;
     half_t* c;
     int M, N, K;
-    int lda, ldb, ldc;  // elements; rows of a and b start at multiples of 4 bytes
+    int lda, ldb, ldc;  // elements; rows of a and b (their columns, where those are what is dense) start at multiples of 4 bytes
     int tiles_m, tiles_n;
     int slices;         // workgroups per tile along k
     int slice_chunks;   // chunks of 32 k of a slice (the last one may have fewer), at least kMinK / 32
@@ -56,7 +58,8 @@ struct __attribute__((packed, aligned(2))) OutPiece {  // 16 bytes of c, whose r
 };
 
 // DIRECT: c leaves straight from the registers (one slice, rows of c aligned to 8 bytes, N % 4 == 0).
-template <bool DIRECT>
+// A_COLS, B_COLS: the operand lies k by k, a[k][m] or b[k][n] with m or n dense (transposing LDS reads, ds_read_b64_tr_b16, turn it round).
+template <bool DIRECT, bool A_COLS = false, bool B_COLS = false>
 __global__ __launch_bounds__(512) void GemmPpKernel(GemmArgs p) {
     constexpr int NSTAGE = kStages, AHEAD = NSTAGE - 1;
     constexpr int TILE_B = 256 * 64;  // bytes of one operand tile in a stage
@@ -93,27 +96,36 @@ __global__ __launch_bounds__(512) void GemmPpKernel(GemmArgs p) {
     const int wm = wave & 1, wn = wave >> 1;
     const int r = lane & 31, h = lane >> 5;
 
-    // ---- global -> LDS loads: a wave instruction covers 16 rows x 64 bytes; lane = 4 * row + position ----
+    // ---- global -> LDS loads.  Rows: a wave instruction covers 16 rows x 64 bytes; lane = 4 * row + position.  Columns: two k of 256 elements, kept
+    // as they lie (stage[k][32 pieces of 8 elements]), 16-byte piece i of k at position i ^ (4 * (k & 3)): the four k that a transposing read
+    // combines then fall into four different 64-byte bank groups ----
     // what lies behind the last element of the last row is out of the buffers' bounds (an odd end shares its dword with 2 more bytes)
-    auto span = [&](int rows, int ld) { return ((static_cast<unsigned>(rows - 1) * static_cast<unsigned>(ld) + k_left) * 2u + 3u) & ~3u; };
-    const int4_t ra = RawRsrc(p.a + static_cast<int64_t>(m0) * p.lda + k0, span(min(p.M - m0, 256), p.lda));
-    const int4_t rb = RawRsrc(p.b + static_cast<int64_t>(n0) * p.ldb + k0, span(min(p.N - n0, 256), p.ldb));
+    auto span = [&](int rows, int ld, int cols) { return ((static_cast<unsigned>(rows - 1) * static_cast<unsigned>(ld) + cols) * 2u + 3u) & ~3u; };
+    const int rows_a = min(p.M - m0, 256), rows_b = min(p.N - n0, 256);
+    const int4_t ra = A_COLS ? RawRsrc(p.a + static_cast<int64_t>(k0) * p.lda + m0, span(k_left, p.lda, rows_a))
+                             : RawRsrc(p.a + static_cast<int64_t>(m0) * p.lda + k0, span(rows_a, p.lda, k_left));
+    const int4_t rb = B_COLS ? RawRsrc(p.b + static_cast<int64_t>(k0) * p.ldb + n0, span(k_left, p.ldb, rows_b))
+                             : RawRsrc(p.b + static_cast<int64_t>(n0) * p.ldb + k0, span(rows_b, p.ldb, k_left));
     int voa[LPO], vob[LPO];
 #pragma unroll
     for (int i = 0; i < LPO; ++i) {
         const int row = (wave * LPO + i) * 16 + (lane >> 2);
         const int piece = (lane & 3) ^ ((lane >> 4) & 3);  // (row >> 2) & 3 = (lane >> 4) & 3
-        voa[i] = (m0 + row < p.M) ? row * p.lda * 2 + piece * 16 : 0x7fffffff;  // beyond the buffer: zeros
-        vob[i] = (n0 + row < p.N) ? row * p.ldb * 2 + piece * 16 : 0x7fffffff;
+        const int k = (wave * LPO + i) * 2 + (lane >> 5), col = ((lane & 31) ^ (4 * (k & 3))) * 8;
+        // beyond the buffer: zeros (rows of k from K on are beyond it too)
+        if (A_COLS) voa[i] = col < rows_a ? (k * p.lda + col) * 2 : 0x7fffffff;
+        else voa[i] = row < rows_a ? row * p.lda * 2 + piece * 16 : 0x7fffffff;
+        if (B_COLS) vob[i] = col < rows_b ? (k * p.ldb + col) * 2 : 0x7fffffff;
+        else vob[i] = row < rows_b ? row * p.ldb * 2 + piece * 16 : 0x7fffffff;
     }
     const unsigned lds_base = static_cast<unsigned>(reinterpret_cast<uintptr_t>(lds));
+    const int step_a = A_COLS ? p.lda * 64 : 64, step_b = B_COLS ? p.ldb * 64 : 64;  // bytes of a chunk
     auto issue = [&](int c) {
         const unsigned st = lds_base + (c % NSTAGE) * STAGE_B + wave * LPO * 1024;
-        const int so = c * 64;
 #pragma unroll
-        for (int i = 0; i < LPO; ++i) LdsLoad16(ra, st + i * 1024, voa[i], so);
+        for (int i = 0; i < LPO; ++i) LdsLoad16(ra, st + i * 1024, voa[i], c * step_a);
 #pragma unroll
-        for (int i = 0; i < LPO; ++i) LdsLoad16(rb, st + TILE_B + i * 1024, vob[i], so);
+        for (int i = 0; i < LPO; ++i) LdsLoad16(rb, st + TILE_B + i * 1024, vob[i], c * step_b);
     };
 
     // ---- fragment addresses: rows of a are the MFMA column operand, rows of b the row operand, so that a lane ends up with
@@ -121,6 +133,11 @@ __global__ __launch_bounds__(512) void GemmPpKernel(GemmArgs p) {
     const int pos0 = h ^ ((r >> 2) & 3), pos1 = (2 + h) ^ ((r >> 2) & 3);
     const unsigned fa0 = lds_base + (wm * 128 + r) * 64 + pos0 * 16, fa1 = lds_base + (wm * 128 + r) * 64 + pos1 * 16;
     const unsigned fb0 = lds_base + TILE_B + (wn * 64 + r) * 64 + pos0 * 16, fb1 = lds_base + TILE_B + (wn * 64 + r) * 64 + pos1 * 16;
+
+    // columns: lane = 16 g + 4 q + s addresses elements 16 (g & 1) + 4 s .. + 3 of k = 8 (g >> 1) + q and receives element 16 (g & 1) + 4 q + s of four k
+    const int fg = lane >> 4, fq = (lane >> 2) & 3, fs = lane & 3;
+    const unsigned col0 = (8 * (fg >> 1) + fq) * 512 + (fs & 1) * 8;
+    const unsigned ca0 = col0 + ((16 * wm + 2 * (fg & 1) + (fs >> 1)) ^ (4 * fq)) * 16, cb0 = col0 + TILE_B + ((8 * wn + 2 * (fg & 1) + (fs >> 1)) ^ (4 * fq)) * 16;
 
     float16_t acc[4][2];
 #pragma unroll
@@ -131,29 +148,130 @@ __global__ __launch_bounds__(512) void GemmPpKernel(GemmArgs p) {
             for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
 
     Bytes16 fm[2][4], fn[2][2];
-    // All twelve fragment reads of a chunk and the wait for them in one statement: nothing touches the registers before the
+    // All fragment reads of a chunk and the wait for them in one statement: nothing touches the registers before the
     // data has landed.
     auto read_frags = [&](int c) {
         const unsigned so = (c % NSTAGE) * STAGE_B;
-        const unsigned a0 = fa0 + so, a1 = fa1 + so, b0 = fb0 + so, b1 = fb1 + so;
-        asm volatile(
-            "ds_read_b128 %0, %12\n\t"
-            "ds_read_b128 %1, %12 offset:2048\n\t"
-            "ds_read_b128 %2, %12 offset:4096\n\t"
-            "ds_read_b128 %3, %12 offset:6144\n\t"
-            "ds_read_b128 %4, %14\n\t"
-            "ds_read_b128 %5, %14 offset:2048\n\t"
-            "ds_read_b128 %6, %13\n\t"
-            "ds_read_b128 %7, %13 offset:2048\n\t"
-            "ds_read_b128 %8, %13 offset:4096\n\t"
-            "ds_read_b128 %9, %13 offset:6144\n\t"
-            "ds_read_b128 %10, %15\n\t"
-            "ds_read_b128 %11, %15 offset:2048\n\t"
-            "s_waitcnt lgkmcnt(0)"
-            : "=&v"(fm[0][0]), "=&v"(fm[0][1]), "=&v"(fm[0][2]), "=&v"(fm[0][3]), "=&v"(fn[0][0]), "=&v"(fn[0][1]), "=&v"(fm[1][0]), "=&v"(fm[1][1]),
-              "=&v"(fm[1][2]), "=&v"(fm[1][3]), "=&v"(fn[1][0]), "=&v"(fn[1][1])
-            : "v"(a0), "v"(a1), "v"(b0), "v"(b1)
-            : "memory");
+        Bytes8 am[2][4][2], bn[2][2][2];
+        const unsigned at = lds_base + so, a0 = A_COLS ? at + ca0 : fa0 + so, a1 = A_COLS ? at + (ca0 ^ 64) : fa1 + so, a2 = at + (ca0 ^ 128), a3 = at + (ca0 ^ 192);
+        const unsigned b0 = B_COLS ? at + cb0 : fb0 + so, b1 = B_COLS ? at + (cb0 ^ 64) : fb1 + so;
+        if constexpr (A_COLS && B_COLS) {
+            asm volatile(
+                "ds_read_b64_tr_b16 %0, %24\n\t"
+                "ds_read_b64_tr_b16 %1, %24 offset:2048\n\t"
+                "ds_read_b64_tr_b16 %2, %25\n\t"
+                "ds_read_b64_tr_b16 %3, %25 offset:2048\n\t"
+                "ds_read_b64_tr_b16 %4, %26\n\t"
+                "ds_read_b64_tr_b16 %5, %26 offset:2048\n\t"
+                "ds_read_b64_tr_b16 %6, %27\n\t"
+                "ds_read_b64_tr_b16 %7, %27 offset:2048\n\t"
+                "ds_read_b64_tr_b16 %8, %28\n\t"
+                "ds_read_b64_tr_b16 %9, %28 offset:2048\n\t"
+                "ds_read_b64_tr_b16 %10, %29\n\t"
+                "ds_read_b64_tr_b16 %11, %29 offset:2048\n\t"
+                "ds_read_b64_tr_b16 %12, %24 offset:8192\n\t"
+                "ds_read_b64_tr_b16 %13, %24 offset:10240\n\t"
+                "ds_read_b64_tr_b16 %14, %25 offset:8192\n\t"
+                "ds_read_b64_tr_b16 %15, %25 offset:10240\n\t"
+                "ds_read_b64_tr_b16 %16, %26 offset:8192\n\t"
+                "ds_read_b64_tr_b16 %17, %26 offset:10240\n\t"
+                "ds_read_b64_tr_b16 %18, %27 offset:8192\n\t"
+                "ds_read_b64_tr_b16 %19, %27 offset:10240\n\t"
+                "ds_read_b64_tr_b16 %20, %28 offset:8192\n\t"
+                "ds_read_b64_tr_b16 %21, %28 offset:10240\n\t"
+                "ds_read_b64_tr_b16 %22, %29 offset:8192\n\t"
+                "ds_read_b64_tr_b16 %23, %29 offset:10240\n\t"
+                "s_waitcnt lgkmcnt(0)"
+                : "=&v"(am[0][0][0]), "=&v"(am[0][0][1]), "=&v"(am[0][1][0]), "=&v"(am[0][1][1]), "=&v"(am[0][2][0]), "=&v"(am[0][2][1]),
+                  "=&v"(am[0][3][0]), "=&v"(am[0][3][1]), "=&v"(bn[0][0][0]), "=&v"(bn[0][0][1]), "=&v"(bn[0][1][0]), "=&v"(bn[0][1][1]),
+                  "=&v"(am[1][0][0]), "=&v"(am[1][0][1]), "=&v"(am[1][1][0]), "=&v"(am[1][1][1]), "=&v"(am[1][2][0]), "=&v"(am[1][2][1]),
+                  "=&v"(am[1][3][0]), "=&v"(am[1][3][1]), "=&v"(bn[1][0][0]), "=&v"(bn[1][0][1]), "=&v"(bn[1][1][0]), "=&v"(bn[1][1][1])
+                : "v"(a0), "v"(a1), "v"(a2), "v"(a3), "v"(b0), "v"(b1)
+                : "memory");
+        } else if constexpr (A_COLS) {
+            asm volatile(
+                "ds_read_b64_tr_b16 %0, %20\n\t"
+                "ds_read_b64_tr_b16 %1, %20 offset:2048\n\t"
+                "ds_read_b64_tr_b16 %2, %21\n\t"
+                "ds_read_b64_tr_b16 %3, %21 offset:2048\n\t"
+                "ds_read_b64_tr_b16 %4, %22\n\t"
+                "ds_read_b64_tr_b16 %5, %22 offset:2048\n\t"
+                "ds_read_b64_tr_b16 %6, %23\n\t"
+                "ds_read_b64_tr_b16 %7, %23 offset:2048\n\t"
+                "ds_read_b128 %8, %24\n\t"
+                "ds_read_b128 %9, %24 offset:2048\n\t"
+                "ds_read_b64_tr_b16 %10, %20 offset:8192\n\t"
+                "ds_read_b64_tr_b16 %11, %20 offset:10240\n\t"
+                "ds_read_b64_tr_b16 %12, %21 offset:8192\n\t"
+                "ds_read_b64_tr_b16 %13, %21 offset:10240\n\t"
+                "ds_read_b64_tr_b16 %14, %22 offset:8192\n\t"
+                "ds_read_b64_tr_b16 %15, %22 offset:10240\n\t"
+                "ds_read_b64_tr_b16 %16, %23 offset:8192\n\t"
+                "ds_read_b64_tr_b16 %17, %23 offset:10240\n\t"
+                "ds_read_b128 %18, %25\n\t"
+                "ds_read_b128 %19, %25 offset:2048\n\t"
+                "s_waitcnt lgkmcnt(0)"
+                : "=&v"(am[0][0][0]), "=&v"(am[0][0][1]), "=&v"(am[0][1][0]), "=&v"(am[0][1][1]), "=&v"(am[0][2][0]), "=&v"(am[0][2][1]),
+                  "=&v"(am[0][3][0]), "=&v"(am[0][3][1]), "=&v"(fn[0][0]), "=&v"(fn[0][1]), "=&v"(am[1][0][0]), "=&v"(am[1][0][1]),
+                  "=&v"(am[1][1][0]), "=&v"(am[1][1][1]), "=&v"(am[1][2][0]), "=&v"(am[1][2][1]), "=&v"(am[1][3][0]), "=&v"(am[1][3][1]),
+                  "=&v"(fn[1][0]), "=&v"(fn[1][1])
+                : "v"(a0), "v"(a1), "v"(a2), "v"(a3), "v"(b0), "v"(b1)
+                : "memory");
+        } else if constexpr (B_COLS) {
+            asm volatile(
+                "ds_read_b128 %0, %16\n\t"
+                "ds_read_b128 %1, %16 offset:2048\n\t"
+                "ds_read_b128 %2, %16 offset:4096\n\t"
+                "ds_read_b128 %3, %16 offset:6144\n\t"
+                "ds_read_b64_tr_b16 %4, %18\n\t"
+                "ds_read_b64_tr_b16 %5, %18 offset:2048\n\t"
+                "ds_read_b64_tr_b16 %6, %19\n\t"
+                "ds_read_b64_tr_b16 %7, %19 offset:2048\n\t"
+                "ds_read_b128 %8, %17\n\t"
+                "ds_read_b128 %9, %17 offset:2048\n\t"
+                "ds_read_b128 %10, %17 offset:4096\n\t"
+                "ds_read_b128 %11, %17 offset:6144\n\t"
+                "ds_read_b64_tr_b16 %12, %18 offset:8192\n\t"
+                "ds_read_b64_tr_b16 %13, %18 offset:10240\n\t"
+                "ds_read_b64_tr_b16 %14, %19 offset:8192\n\t"
+                "ds_read_b64_tr_b16 %15, %19 offset:10240\n\t"
+                "s_waitcnt lgkmcnt(0)"
+                : "=&v"(fm[0][0]), "=&v"(fm[0][1]), "=&v"(fm[0][2]), "=&v"(fm[0][3]), "=&v"(bn[0][0][0]), "=&v"(bn[0][0][1]),
+                  "=&v"(bn[0][1][0]), "=&v"(bn[0][1][1]), "=&v"(fm[1][0]), "=&v"(fm[1][1]), "=&v"(fm[1][2]), "=&v"(fm[1][3]),
+                  "=&v"(bn[1][0][0]), "=&v"(bn[1][0][1]), "=&v"(bn[1][1][0]), "=&v"(bn[1][1][1])
+                : "v"(a0), "v"(a1), "v"(b0), "v"(b1)
+                : "memory");
+        } else {
+            asm volatile(
+                "ds_read_b128 %0, %12\n\t"
+                "ds_read_b128 %1, %12 offset:2048\n\t"
+                "ds_read_b128 %2, %12 offset:4096\n\t"
+                "ds_read_b128 %3, %12 offset:6144\n\t"
+                "ds_read_b128 %4, %14\n\t"
+                "ds_read_b128 %5, %14 offset:2048\n\t"
+                "ds_read_b128 %6, %13\n\t"
+                "ds_read_b128 %7, %13 offset:2048\n\t"
+                "ds_read_b128 %8, %13 offset:4096\n\t"
+                "ds_read_b128 %9, %13 offset:6144\n\t"
+                "ds_read_b128 %10, %15\n\t"
+                "ds_read_b128 %11, %15 offset:2048\n\t"
+                "s_waitcnt lgkmcnt(0)"
+                : "=&v"(fm[0][0]), "=&v"(fm[0][1]), "=&v"(fm[0][2]), "=&v"(fm[0][3]), "=&v"(fn[0][0]), "=&v"(fn[0][1]), "=&v"(fm[1][0]),
+                  "=&v"(fm[1][1]), "=&v"(fm[1][2]), "=&v"(fm[1][3]), "=&v"(fn[1][0]), "=&v"(fn[1][1])
+                : "v"(a0), "v"(a1), "v"(b0), "v"(b1)
+                : "memory");
+        }
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if constexpr (A_COLS) fm[t][i] = Bytes16{am[t][i][0].x, am[t][i][0].y, am[t][i][1].x, am[t][i][1].y};
+            }
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                if constexpr (B_COLS) fn[t][j] = Bytes16{bn[t][j][0].x, bn[t][j][0].y, bn[t][j][1].x, bn[t][j][1].y};
+            }
+        }
     };
     auto compute = [&]() {
 #pragma unroll
