@@ -96,8 +96,9 @@ void LaunchSmallDotMixed(const SmallDotArgs& p, dim3 grid, int pieces, hipStream
 //   float16  [100,650] . [650,1000]  4.2  4.3  4.7              [37,2048] . [2048,1000]   9.7  5.1  6.1  7.3
 //            [128,300] . [300,2600]  4.2  4.9  7.9  5.5  6.5    [128,650] . [650,2600]    6.5  6.5  8.0  5.9  6.6
 //            [300,300] . [300,1500]  4.6  5.9  8.0  9.2  6.7    [500,1000] . [1000,1000]  9.5  8.8 10.3 11.3  8.3
-// 64 columns in float32: within 3 % of 32.  More tiles than compute units at any width: 484 of 300 terms 9.0 and 8.6 (float32, 32 columns), 4.7 and 5.6
-// (float16); [150,1024] . [1024,4096] 21.7 20.3 19.8 21.8 27.5, [1024,1024]^2 in float16 15.3 12.6 10.9 11.3 12.1.
+// 64 columns in float32: within 3 % of 32.  More tiles than compute units at any width, 32 and 48 columns: float32 [1024,1024]^2 23.6 26.8, float16
+// [1024,1024]^2 10.7 10.5, [700,1500] . [1500,900] 13.9 12.2, [800,2000] . [2000,800] 15.6 14.6; 484 tiles of 300 terms, SmallDotKernel and 32 columns: float32
+// 9.0 8.6, float16 4.7 5.6.  No width that pads the columns by a tenth more than 32 does ([2122,442] . [442,106] in float16 5.2 us, 6.0 by 48 columns).
 template <typename T>
 int LinesBlocks(int64_t rows, int64_t n, int64_t parts, int64_t k) {
     constexpr bool kHalf = sizeof(T) == 2;
@@ -108,16 +109,18 @@ int LinesBlocks(int64_t rows, int64_t n, int64_t parts, int64_t k) {
         if (kHalf) return bytes >= 1600 ? 2 : 0;
         return bytes >= 6144 || (bytes >= 4096 && groups(2) > cus * 3 / 4) ? 2 : 0;
     }
-    if (groups(3) <= cus) return bytes >= least ? 3 : 0;
-    if (kHalf && groups(4) <= cus) return bytes >= least ? 4 : 0;
-    return bytes > (groups(2) > 2 * cus ? 7 * 128 : least) ? 2 : 0;
+    auto fits = [&](int blocks) { return groups(blocks) <= cus && 10 * blocks * groups(blocks) <= 11 * 2 * groups(2); };
+    if (fits(3)) return bytes >= least ? 3 : 0;
+    if (kHalf && fits(4)) return bytes >= least ? 4 : 0;
+    if (bytes <= (groups(2) > 2 * cus ? 7 * 128 : least)) return 0;
+    return kHalf && 10 * 3 * groups(3) <= 11 * 2 * groups(2) ? 3 : 2;
 }
 
 // Their waves: eight keep most loads in flight while a compute unit has one or two tiles (328 float32 tiles of 21 chunks: 12.3 us, 12.8 with four, 16.6
-// with two); beyond, what leaves the busiest SIMD the fewest chunks, fewer waves on near terms (626 tiles of 21 chunks: 17.6 us with two, 18.2 with three, 16.5 with four; 1252 of
+// with two), or four for the lighter float16 ones beyond one ([150,1024] . [1024,4096] by 48 columns 9.6 -> 8.6 us); beyond, what leaves the busiest SIMD the fewest chunks, fewer waves on near terms (626 tiles of 21 chunks: 17.6 us with two, 18.2 with three, 16.5 with four; 1252 of
 // 21: 26.9, 26.5, 29.0; 1504 of 25: 34.1, 37.9, 35.3).
-int LinesWaves(int64_t groups, int chunks) {
-    if (groups <= 2 * NumCUs()) return std::min(kSmallDotMaxWaves, chunks);
+int LinesWaves(int64_t groups, int chunks, bool half) {
+    if (groups <= 2 * NumCUs()) return std::min(half && groups > NumCUs() ? 4 : kSmallDotMaxWaves, chunks);
     const int64_t per_unit = (groups + NumCUs() - 1) / NumCUs();
     auto cost = [&](int nw) { return (per_unit * nw + 3) / 4 * ((chunks + nw - 1) / nw); };
     int best = 2;
@@ -138,7 +141,7 @@ void LaunchSmallDot(SmallDotArgs p, int a_mode, int b_mode, int batch, hipStream
             constexpr int NB = decltype(blocks_tag)::value, kWaveBytes = (32 + 16 * NB) * kSmallDotPitch;
             p.tiles_n = (p.N + 16 * NB - 1) / (16 * NB);
             const int64_t groups = static_cast<int64_t>(p.tiles_m) * p.tiles_n * p.ksplit;
-            p.nw = LinesWaves(groups * batch, chunks);
+            p.nw = LinesWaves(groups * batch, chunks, sizeof(T) == 2);
             struct LinesTag {};
             EnsureDynamicLds<LinesTag>(reinterpret_cast<const void*>(SmallDotLinesKernel<T, NB>), kSmallDotMaxWaves * kWaveBytes);
             hipLaunchKernelGGL((SmallDotLinesKernel<T, NB>), dim3(static_cast<unsigned>(groups), static_cast<unsigned>(batch)), dim3(64 * p.nw), p.nw * kWaveBytes,
