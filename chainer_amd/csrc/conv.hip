@@ -1327,19 +1327,22 @@ namespace {
 // reduction axis is not the unit-stride one (or whose rows are not dword-aligned) laid out anew, then the partial sums.
 struct GemmPpPlan {
     int slices = 0;  // 0: left to the other kernels
-    bool cols_a = false, cols_b = false;    // read k by k as they lie
+    bool pair = false;                    // in tiles of half the width, two workgroups to a compute unit
+    bool cols_a = false, cols_b = false;  // read k by k as they lie
     bool stage_a = false, stage_b = false;
     int64_t pitch = 0;  // of a staged row, elements
     size_t a_bytes = 0, b_bytes = 0, partial_bytes = 0;
     size_t Total() const { return a_bytes + b_bytes + partial_bytes; }
 };
 
-// The estimates, in us, are fits to measured products (572 of this kernel, 232 of the others; 57 shapes of 60 to 10000 in every layout).  256 x 256 tiles: 0.54
-// for a chunk of 32 k, 0.76 when the whole chip fetches, 6.5 for a tile's start and end, one tile at a time on a compute unit, the result at 4.3 TB/s
-// (nothing else runs meanwhile), partial sums written and read at 7.3 TB/s; operands in an order of neither kind are staged at 3.5 TB/s.  The other
-// kernels, by the operands whose reduction axis is dense (both, one, none), for outputs small enough for 32 x 32 tiles and for larger ones: a start, the
-// operations, the bytes and the length of the reduction.  The one chosen takes 2 to 3 % longer than the best of all of them and all splits on
-// average; by more than 15 % for 6 of 116.
+// Outputs of 128 tiles of 128 x 128 and more always run here: the best split is within 1 % of the best of all kernels on average over 42 shapes, and at worst
+// 5 % slower than the others.  The estimates, in us, are fits to measured products (57 shapes of 60 to 10000, 572 measurements of this kernel in two
+// layouts, 150 of the small tiles in four).  256 x 256 tiles: 0.54 for a chunk of 32 k, 0.76 when the whole chip fetches, 6.5 for a tile's start and end,
+// one tile at a time on a compute unit, the result at 4.3 TB/s (nothing else runs meanwhile), partial sums written and read at 7.3 TB/s; operands in
+// an order of neither kind are staged at 3.5 TB/s.  Pairs: the same chunks at half the width, the result at 3.2 TB/s under the other tile's
+// work; over 512 terms the wide tiles' smaller operand traffic wins ([4480,650] . [650,10000] 103 and 118).  The small tiles, by the operands whose
+// reduction axis is dense (none, one, both): a start, the operations, the bytes and the length of the reduction; the choice against them is 3 % off the best
+// on average, by more than 15 % for 5 of 74.
 GemmPpPlan PlanGemmPp(const hipcx_array* a, const hipcx_array* b, const hipcx_array* out) {
     GemmPpPlan pl;
     static const bool enabled = [] { const char* e = getenv("HIPCX_DOT_PP"); return e == nullptr || e[0] != '0'; }();
@@ -1365,15 +1368,18 @@ GemmPpPlan PlanGemmPp(const hipcx_array* a, const hipcx_array* b, const hipcx_ar
     pl.cols_b = pl.stage_b && fits_cols(b->data, b->strides[1], b->strides[0], n);
     if (pl.cols_a) pl.stage_a = false;
     if (pl.cols_b) pl.stage_b = false;
-    const double flops = 2.0 * m * n * k, bytes = 2.0 * (static_cast<double>(m) * n + static_cast<double>(m) * k + static_cast<double>(n) * k), outs = static_cast<double>(m) * n;
-    const int dense = (a->strides[1] == 2) + (b->strides[0] == 2);
-    struct Fit {
-        double start, flops, bytes, k;
-    };
-    static constexpr Fit kSmall[3] = {{3.6, 190e6, 1.6e6, 3.2e-3}, {4.0, 135e6, 3e6, 1.3e-3}, {3.6, 186e6, 14e6, 0.45e-3}};
-    static constexpr Fit kLarge[3] = {{17, 990e6, 2.8e6, 10e-3}, {15, 830e6, 4e6, 9e-3}, {12.6, 571e6, 1e9, 7e-3}};
-    const Fit& fit = (SmallDotShape(m, n, k) ? kSmall : kLarge)[dense];
-    double least = 0.95 * (fit.start + flops / fit.flops + bytes / fit.bytes + k * fit.k);
+    const double outs = static_cast<double>(m) * n;
+    double least = 1e30;
+    if (SmallDotShape(m, n, k)) {
+        struct Fit {
+            double start, flops, bytes, k;
+        };
+        static constexpr Fit kFits[3] = {{3.6, 190e6, 1.6e6, 3.2e-3}, {4.0, 135e6, 3e6, 1.3e-3}, {3.6, 186e6, 14e6, 0.45e-3}};
+        const Fit& fit = kFits[(a->strides[1] == 2) + (b->strides[0] == 2)];
+        const double bytes = 2.0 * (outs + static_cast<double>(m) * k + static_cast<double>(n) * k);
+        const double serial = k < 5120 ? k : k / 4.0;  // (from there on they split the reduction too)
+        least = 0.95 * (fit.start + 2.0 * outs * k / fit.flops + bytes / fit.bytes + serial * fit.k);
+    }
     auto stage_us = [&](bool needed, int64_t lines) { return needed ? 2.0 + 4.0 * lines * k / 3.5e6 : 0.0; };
     const double staging = stage_us(pl.stage_a, m) + stage_us(pl.stage_b, n);
     for (int s = 1; s <= 16 && chunks / s >= 8 * (s > 1); ++s) {
@@ -1383,6 +1389,10 @@ GemmPpPlan PlanGemmPp(const hipcx_array* a, const hipcx_array* b, const hipcx_ar
         const double chunk = 0.54 + 0.22 * std::min(1.0, static_cast<double>(groups) / NumCUs());
         const double t = 2.5 + rounds * (each * chunk + 6.5) + (s > 1 ? 5.5 + 8.0 * s * outs / 7.3e6 : 2.0 * outs / 4.3e6) + staging;
         if (t < least) least = t, pl.slices = s;
+    }
+    if (k <= 512 && !pl.cols_a && !pl.cols_b) {
+        const double per_unit = static_cast<double>((m + 255) / 256 * ((n + 127) / 128)) / NumCUs();
+        if (6.5 + chunks * 0.53 * std::max(1.0, per_unit) + 2.0 * outs / 3.2e6 + staging < least) pl.slices = 1, pl.pair = true;
     }
     pl.a_bytes = pl.stage_a ? RoundUpTo(static_cast<size_t>(m * pl.pitch * 2), 256) : 0;
     pl.b_bytes = pl.stage_b ? RoundUpTo(static_cast<size_t>(n * pl.pitch * 2), 256) : 0;
@@ -1430,21 +1440,22 @@ bool TryGemmPp(const hipcx_array* a, const hipcx_array* b, const hipcx_array* bi
         p.bias_stride = bias->strides[0] / 2;
     }
     ProfileScope prof(stream, 2.0 * static_cast<double>(M) * N * K, 2.0 * (static_cast<double>(M) * K + static_cast<double>(N) * K + static_cast<double>(M) * N));
-    const unsigned grid = static_cast<unsigned>((static_cast<int64_t>(p.tiles_m) * p.tiles_n * slices + 7) / 8 * 8);
-    auto launch = [&](auto direct, auto cols_a, auto cols_b) {
-        constexpr bool DIRECT = decltype(direct)::value, A_COLS = decltype(cols_a)::value, B_COLS = decltype(cols_b)::value;
+    auto launch = [&](auto cols_a, auto cols_b, auto pair) {
+        constexpr bool A_COLS = decltype(cols_a)::value, B_COLS = decltype(cols_b)::value, PAIR = decltype(pair)::value;
+        constexpr int kLds = PAIR ? gemm_pp::kPairLdsBytes : gemm_pp::kLdsBytes;
         struct GemmPpTag {};
-        const auto kernel = gemm_pp::GemmPpKernel<DIRECT, A_COLS, B_COLS>;
-        EnsureDynamicLds<GemmPpTag>(reinterpret_cast<const void*>(kernel), gemm_pp::kLdsBytes);
-        hipLaunchKernelGGL(kernel, dim3(grid), dim3(512), gemm_pp::kLdsBytes, stream, p);
+        const auto kernel = gemm_pp::GemmPpKernel<A_COLS, B_COLS, PAIR>;
+        EnsureDynamicLds<GemmPpTag>(reinterpret_cast<const void*>(kernel), kLds);
+        if (PAIR) p.tiles_n = static_cast<int>((N + 127) / 128);
+        const unsigned grid = static_cast<unsigned>((static_cast<int64_t>(p.tiles_m) * p.tiles_n * slices + 7) / 8 * 8);
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(PAIR ? 256 : 512), kLds, stream, p);
     };
-    // short reductions: see the epilogue
     const std::true_type yes{};
     const std::false_type no{};
-    if (space.cols_a && space.cols_b) launch(no, yes, yes);
-    else if (space.cols_a) launch(no, yes, no);
-    else if (space.cols_b) launch(no, no, yes);
-    else if (slices == 1 && K <= 256 && N % 4 == 0 && p.ldc % 4 == 0 && Aligned(p.c, 8)) launch(yes, no, no);
+    if (space.cols_a && space.cols_b) launch(yes, yes, no);
+    else if (space.cols_a) launch(yes, no, no);
+    else if (space.cols_b) launch(no, yes, no);
+    else if (space.pair) launch(no, no, yes);
     else launch(no, no, no);
     CheckLaunch("gemm_pp");
     if (slices > 1) {

@@ -46,7 +46,7 @@ struct GemmArgs {
 };
 
 constexpr int kStages = 3;
-constexpr int kLdsBytes = kStages * 2 * 256 * 64;
+constexpr int kLdsBytes = kStages * 2 * 256 * 64, kPairLdsBytes = kStages * (256 + 128) * 64;
 constexpr int kMinK = 32 * (kStages - 1);  // the pipeline's prologue issues kStages - 1 chunks
 // Rows of a wave's 32 x 64 block on its way out, a float for partial sums: 16 bytes of padding keep the banks apart.
 constexpr int kOutPitch = 64 * 4 + 16;
@@ -57,15 +57,19 @@ struct __attribute__((packed, aligned(2))) OutPiece {  // 16 bytes of c, whose r
     T e[16 / sizeof(T)];
 };
 
-// DIRECT: c leaves straight from the registers (one slice, rows of c aligned to 8 bytes, N % 4 == 0).
 // A_COLS, B_COLS: the operand lies k by k, a[k][m] or b[k][n] with m or n dense (transposing LDS reads, ds_read_b64_tr_b16, turn it round).
-template <bool DIRECT, bool A_COLS = false, bool B_COLS = false>
-__global__ __launch_bounds__(512) void GemmPpKernel(GemmArgs p) {
+// PAIR: tiles of 256 x 128 by four waves, two workgroups to a compute unit: one's start and end run under the other's products, which in short reductions
+// is most of the time.  us, against one workgroup of eight waves (with the stores straight from the registers) and the 128 x 128 kernel: [8192,128] .
+// [128,8192] 125, 109, 54; [4480,256] . [256,10000] 98, 91, 54; [1500,64] . [64,3000] 28, 19, 10; [10000,300] . [300,5000] 86, 154, 82.
+template <bool A_COLS, bool B_COLS, bool PAIR>
+__global__ __launch_bounds__(PAIR ? 256 : 512, 2) void GemmPpKernel(GemmArgs p) {
+    static_assert(!PAIR || !(A_COLS || B_COLS), "pairs read rows");
     constexpr int NSTAGE = kStages, AHEAD = NSTAGE - 1;
-    constexpr int TILE_B = 256 * 64;  // bytes of one operand tile in a stage
-    constexpr int STAGE_B = 2 * TILE_B;
-    constexpr int LPO = 2;            // load instructions per operand, wave and chunk
-    constexpr int LPC = 2 * LPO;
+    constexpr int WAVES = PAIR ? 4 : 8, COLS = WAVES * 32;
+    constexpr int TILE_B = 256 * 64;  // bytes of a's tile in a stage
+    constexpr int STAGE_B = TILE_B + COLS * 64;
+    constexpr int LPA = 16 / WAVES, LPB = COLS / 16 / WAVES;  // load instructions per operand, wave and chunk
+    constexpr int LPC = LPA + LPB;
     extern __shared__ __align__(16) char lds[];
 
     // ---- tile of this workgroup: XCD x (workgroup ids go round-robin to the 8 XCDs) walks a contiguous range of the tile
@@ -88,7 +92,7 @@ __global__ __launch_bounds__(512) void GemmPpKernel(GemmArgs p) {
         tile_m = bi * p.band + rem % rows;
         tile_n = rem / rows;
     }
-    const int m0 = tile_m * 256, n0 = tile_n * 256;
+    const int m0 = tile_m * 256, n0 = tile_n * COLS;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -101,31 +105,34 @@ __global__ __launch_bounds__(512) void GemmPpKernel(GemmArgs p) {
     // combines then fall into four different 64-byte bank groups ----
     // what lies behind the last element of the last row is out of the buffers' bounds (an odd end shares its dword with 2 more bytes)
     auto span = [&](int rows, int ld, int cols) { return ((static_cast<unsigned>(rows - 1) * static_cast<unsigned>(ld) + cols) * 2u + 3u) & ~3u; };
-    const int rows_a = min(p.M - m0, 256), rows_b = min(p.N - n0, 256);
+    const int rows_a = min(p.M - m0, 256), rows_b = min(p.N - n0, COLS);
     const int4_t ra = A_COLS ? RawRsrc(p.a + static_cast<int64_t>(k0) * p.lda + m0, span(k_left, p.lda, rows_a))
                              : RawRsrc(p.a + static_cast<int64_t>(m0) * p.lda + k0, span(rows_a, p.lda, k_left));
     const int4_t rb = B_COLS ? RawRsrc(p.b + static_cast<int64_t>(k0) * p.ldb + n0, span(k_left, p.ldb, rows_b))
                              : RawRsrc(p.b + static_cast<int64_t>(n0) * p.ldb + k0, span(rows_b, p.ldb, k_left));
-    int voa[LPO], vob[LPO];
+    int voa[LPA], vob[LPB];
+    // beyond the buffer: zeros (rows of k from K on are beyond it too)
+    auto offsets = [&](auto cols_tag, auto& vo, int rows, int ld) {
+        constexpr int LPO = sizeof(vo) / sizeof(int);
 #pragma unroll
-    for (int i = 0; i < LPO; ++i) {
-        const int row = (wave * LPO + i) * 16 + (lane >> 2);
-        const int piece = (lane & 3) ^ ((lane >> 4) & 3);  // (row >> 2) & 3 = (lane >> 4) & 3
-        const int k = (wave * LPO + i) * 2 + (lane >> 5), col = ((lane & 31) ^ (4 * (k & 3))) * 8;
-        // beyond the buffer: zeros (rows of k from K on are beyond it too)
-        if (A_COLS) voa[i] = col < rows_a ? (k * p.lda + col) * 2 : 0x7fffffff;
-        else voa[i] = row < rows_a ? row * p.lda * 2 + piece * 16 : 0x7fffffff;
-        if (B_COLS) vob[i] = col < rows_b ? (k * p.ldb + col) * 2 : 0x7fffffff;
-        else vob[i] = row < rows_b ? row * p.ldb * 2 + piece * 16 : 0x7fffffff;
-    }
+        for (int i = 0; i < LPO; ++i) {
+            const int row = (wave * LPO + i) * 16 + (lane >> 2);
+            const int piece = (lane & 3) ^ ((lane >> 4) & 3);  // (row >> 2) & 3 = (lane >> 4) & 3
+            const int k = (wave * LPO + i) * 2 + (lane >> 5), col = ((lane & 31) ^ (4 * (k & 3))) * 8;
+            if constexpr (decltype(cols_tag)::value) vo[i] = col < rows ? (k * ld + col) * 2 : 0x7fffffff;
+            else vo[i] = row < rows ? row * ld * 2 + piece * 16 : 0x7fffffff;
+        }
+    };
+    offsets(std::integral_constant<bool, A_COLS>{}, voa, rows_a, p.lda);
+    offsets(std::integral_constant<bool, B_COLS>{}, vob, rows_b, p.ldb);
     const unsigned lds_base = static_cast<unsigned>(reinterpret_cast<uintptr_t>(lds));
     const int step_a = A_COLS ? p.lda * 64 : 64, step_b = B_COLS ? p.ldb * 64 : 64;  // bytes of a chunk
     auto issue = [&](int c) {
-        const unsigned st = lds_base + (c % NSTAGE) * STAGE_B + wave * LPO * 1024;
+        const unsigned st = lds_base + (c % NSTAGE) * STAGE_B;
 #pragma unroll
-        for (int i = 0; i < LPO; ++i) LdsLoad16(ra, st + i * 1024, voa[i], c * step_a);
+        for (int i = 0; i < LPA; ++i) LdsLoad16(ra, st + (wave * LPA + i) * 1024, voa[i], c * step_a);
 #pragma unroll
-        for (int i = 0; i < LPO; ++i) LdsLoad16(rb, st + TILE_B + i * 1024, vob[i], c * step_b);
+        for (int i = 0; i < LPB; ++i) LdsLoad16(rb, st + TILE_B + (wave * LPB + i) * 1024, vob[i], c * step_b);
     };
 
     // ---- fragment addresses: rows of a are the MFMA column operand, rows of b the row operand, so that a lane ends up with
@@ -304,12 +311,12 @@ __global__ __launch_bounds__(512) void GemmPpKernel(GemmArgs p) {
     for (int c = 0; c < AHEAD; ++c) issue(c);
     WaitVmcnt<(AHEAD - 1) * LPC>();  // this wave's share of chunk 0 has landed
     __builtin_amdgcn_s_barrier();
-    if (grp == 1) __builtin_amdgcn_s_barrier();  // the second group runs half a period behind
+    if (!PAIR && grp == 1) __builtin_amdgcn_s_barrier();  // the second group runs half a period behind
     auto iteration = [&](int c, auto issue_tag, auto wait_tag) {
         constexpr bool ISSUE = decltype(issue_tag)::value;
         constexpr int WAIT = decltype(wait_tag)::value;
         __builtin_amdgcn_sched_barrier(0);
-        if constexpr (ISSUE) issue(c + AHEAD);  // into the stage both groups finished reading a phase ago
+        if constexpr (ISSUE) issue(c + AHEAD);  // into the stage that everyone finished reading a phase ago
         read_frags(c);
         if constexpr (!ISSUE && WAIT == 0) {
             if (c * 32 + 32 > k_left) mask_tail(k_left - c * 32);
@@ -319,9 +326,11 @@ __global__ __launch_bounds__(512) void GemmPpKernel(GemmArgs p) {
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
         compute();
-        __builtin_amdgcn_sched_barrier(0);
-        __builtin_amdgcn_s_barrier();
-        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (!PAIR) {
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_sched_barrier(0);
+        }
     };
     int c = 0;
     for (; c + AHEAD < nc; ++c) iteration(c, std::true_type{}, std::integral_constant<int, (AHEAD - 1) * LPC>{});
@@ -331,37 +340,10 @@ __global__ __launch_bounds__(512) void GemmPpKernel(GemmArgs p) {
         iteration(c, std::false_type{}, std::integral_constant<int, (tt >= 1 ? tt - 1 : 0) * LPC>{});
         ++c;
     });
-    if (grp == 0) __builtin_amdgcn_s_barrier();
+    if (!PAIR && grp == 0) __builtin_amdgcn_s_barrier();
 
-    // ---- epilogue: lane holds m = r, n = 8 * (v / 4) + 4 * h + v % 4 of each 32 x 32 block.  DIRECT stores them as they are, 8 bytes each, and
-    // relies on the caches to put lines together; else the blocks pass through LDS (a piece per wave, free now), so that a row of 64 columns
-    // leaves in whole lines at any address.  That costs a tile about 1 us of latency and saves the traffic: [4480,650] . [650,10000] 100 -> 94 us,
-    // but [8192,128] . [128,8192], which has little else to do, 57 -> 61 ----
-    if constexpr (DIRECT) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int m = m0 + wm * 128 + i * 32 + r;
-            if (m >= p.M) continue;
-            half_t* const crow = p.c + static_cast<int64_t>(m) * p.ldc;
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const int n = n0 + wn * 64 + j * 32 + q * 8 + h * 4;
-                    if (n >= p.N) continue;  // N % 4 == 0: a group of four is inside or outside
-                    PVecH<4> o;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        float v = acc[i][j][q * 4 + e];
-                        if (p.bias != nullptr) v += static_cast<float>(p.bias[(n + e) * p.bias_stride]);
-                        o.e[e] = static_cast<half_t>(v);
-                    }
-                    *reinterpret_cast<PVecH<4>*>(crow + n) = o;
-                }
-            }
-        }
-        return;
-    }
+    // ---- epilogue: lane holds m = r, n = 8 * (v / 4) + 4 * h + v % 4 of each 32 x 32 block.  The blocks pass through LDS (a piece per wave, free now),
+    // so that a row of 64 columns leaves in whole lines at any address: [4480,650] . [650,10000] 100 -> 94 us against 8-byte stores ----
     char* const mine = lds + wave * 32 * kOutPitch;
     float bias[2][16];
     if (p.bias != nullptr && p.slices == 1) {  // one load for the wave's 64 columns, then to where the lanes need them

@@ -1,5 +1,5 @@
-"""Large float16 products whose operands lie k by k (GemmPpKernel's transposing reads): edges of the 256 x 256 tiles, of 32-wide chunks and of 8-element
-pieces, one slice and several, and what lies behind an operand's columns."""
+"""Large float16 products whose operands lie k by k (GemmPpKernel's transposing reads) and those of short reductions (tiles of 256 x 128): edges of the
+tiles, of 32-wide chunks and of 8-element pieces, one slice and several, and what lies behind an operand's rows or columns."""
 import numpy as np
 import pytest
 
@@ -26,3 +26,17 @@ def test_operands_that_lie_k_by_k(cols_a, cols_b, m, k, n):
     bt, btm = operand(n, cols_b)
     expected = am @ btm.T  # whole numbers below 2^24: exact in any order
     np.testing.assert_array_equal(chx.dot(a, bt.T).get(), expected.astype(np.float16))
+
+
+@pytest.mark.parametrize('m,k,n', [(2050, 66, 2306), (1300, 130, 1701), (4100, 450, 700), (1030, 512, 2051), (20000, 64, 130), (130, 95, 17000)])
+def test_short_reductions(m, k, n):
+    rng = np.random.default_rng(k)
+
+    def wide(lines):
+        a = np.full((lines, k + 3 - k % 2), np.nan, np.float16)[:, :(k + 3 - k % 2) // 2 * 2]
+        a[:, :k] = rng.integers(-2, 3, (lines, k))
+        return a
+
+    x, w, b = wide(m), wide(n), rng.integers(-8, 9, n).astype(np.float16)
+    got = chx.linear(chx.array(x)[:, :k], chx.array(w)[:, :k], chx.array(b)).get()
+    np.testing.assert_array_equal(got, (x[:, :k].astype(np.float32) @ w[:, :k].T.astype(np.float32) + b).astype(np.float16))  # exact in any order
