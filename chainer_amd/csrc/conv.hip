@@ -18,6 +18,7 @@
 #include "pw_conv.h"
 #include "small_conv.h"
 #include "stem_conv.h"
+#include "thin_conv.h"
 #include "dot_parts.h"
 
 namespace hipcx {
@@ -1159,7 +1160,7 @@ int hipcx_conv(const hipcx_array* x, const hipcx_array* w, const hipcx_array* b,
         if (out->dtype == HIPCX_FLOAT16) {
             RunConv<half_t>(x, w, b, pl, out, ws, st);
         } else if (out->dtype == HIPCX_FLOAT32) {
-            RunConv<float>(x, w, b, pl, out, ws, st);
+            if (!TryThinConv(x, w, b, stride, pad, out, st)) RunConv<float>(x, w, b, pl, out, ws, st);
         } else {
             RunConv<double>(x, w, b, pl, out, ws, st);
         }

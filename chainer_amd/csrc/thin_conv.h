@@ -1,0 +1,11 @@
+// float32 convolutions of few terms per output (the first layer of a network); the kernel: thin_conv.hip.
+#pragma once
+
+#include "common.h"
+
+namespace hipcx {
+
+// Runs the convolution if it is one of those: dense NCHW arrays, channels x filter of at most 32 terms.
+bool TryThinConv(const hipcx_array* x, const hipcx_array* w, const hipcx_array* b, const int64_t* stride, const int64_t* pad, const hipcx_array* out, hipStream_t stream);
+
+}  // namespace hipcx
