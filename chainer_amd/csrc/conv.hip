@@ -1158,7 +1158,7 @@ int hipcx_conv(const hipcx_array* x, const hipcx_array* w, const hipcx_array* b,
         }
         char* ws = static_cast<char*>(workspace);
         if (out->dtype == HIPCX_FLOAT16) {
-            RunConv<half_t>(x, w, b, pl, out, ws, st);
+            if (!TryThinConv(x, w, b, stride, pad, out, st)) RunConv<half_t>(x, w, b, pl, out, ws, st);
         } else if (out->dtype == HIPCX_FLOAT32) {
             if (!TryThinConv(x, w, b, stride, pad, out, st)) RunConv<float>(x, w, b, pl, out, ws, st);
         } else {

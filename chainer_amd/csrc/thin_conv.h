@@ -1,4 +1,4 @@
-// float32 convolutions of few terms per output (the first layer of a network); the kernel: thin_conv.hip.
+// float32 and float16 convolutions of few terms per output (the first layer of a network); the kernel: thin_conv.hip.
 #pragma once
 
 #include "common.h"

@@ -1,4 +1,4 @@
-// float32 convolutions whose outputs are sums of at most 32 terms: a network's first layer, 3 channels x 3 x 3.
+// float32 and float16 convolutions whose outputs are sums of at most 32 terms: a network's first layer, 3 channels x 3 x 3.
 //
 // Such a layer is its output: on the general kernel's 256 x 64 tiles, two steps long, the loads, the staging and the way out follow one another, after a
 // channels-last copy of x.  Here a wave owns 64 filters, whose terms stay in its registers, and walks blocks of 32 output pixels: a lane gathers the
@@ -6,6 +6,7 @@
 // of a plane each.  Neither LDS nor a barrier.  Bound by writing the result.  us, against the general
 // kernel and its copies: 256 images of 3 channels at 32^2, 3x3 into 64 62 -> 26, one image 23 -> 8; 256 of 1 at 28^2, 5x5 into 32 68 -> 22; 4 of 3 at 224^2
 // into 64 56 -> 24; 1x1, 256 of 32 at 16^2 into 256 41 -> 29.  Relative error against 64 bits 9.2e-8 (9.3e-8 before).
+// float16, the first and the third of these 44 -> 28 and 41 -> 24.
 #include <algorithm>
 
 #include "igemm.h"
@@ -19,11 +20,11 @@ namespace {
 constexpr int kOut = 0x7fffffff;  // an offset beyond any buffer: loads give zeros, stores are dropped
 
 struct ThinConvArgs {
-    const float* x;
-    const float* w;
-    const float* bias;
+    const void* x;
+    const void* w;
+    const void* bias;
     int64_t bias_stride;
-    float* out;
+    void* out;
     int C, H, W, K, R, S, OW, P;
     int stride_h, stride_w, pad_h, pad_w;
     int M;       // images * P
@@ -32,8 +33,14 @@ struct ThinConvArgs {
     FastDiv div_P, div_OW;
 };
 
+template <typename T>
+__device__ __forceinline__ float LoadFloat(__amdgpu_buffer_rsrc_t r, int element, bool in) {
+    if constexpr (sizeof(T) == 4) return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, in ? element * 4 : kOut, 0, 0));
+    else return static_cast<float>(__builtin_bit_cast(half_t, static_cast<unsigned short>(__builtin_amdgcn_raw_buffer_load_b16(r, in ? element * 2 : kOut, 0, 0))));
+}
+
 // STEPS: pairs of terms.
-template <int STEPS>
+template <typename T, int STEPS>
 __global__ __launch_bounds__(256, 3) void ThinConvKernel(ThinConvArgs p) {
     const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -52,7 +59,7 @@ __global__ __launch_bounds__(256, 3) void ThinConvKernel(ThinConvArgs p) {
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             const int n = n0 + j * 32 + r;
-            wf[j][k] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(wr, term < terms && n < p.K ? (n * terms + term) * 4 : kOut, 0, 0));
+            wf[j][k] = LoadFloat<T>(wr, n * terms + term, (term < terms) & (n < p.K));
         }
     }
     // lane holds pixel r, filters 8 * (v / 4) + 4 * h + v % 4 of each half
@@ -62,7 +69,7 @@ __global__ __launch_bounds__(256, 3) void ThinConvKernel(ThinConvArgs p) {
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
             const int n = n0 + j * 32 + 8 * (v / 4) + 4 * h + v % 4;
-            bias[j][v] = p.bias != nullptr && n < p.K ? p.bias[n * p.bias_stride] : 0.f;
+            bias[j][v] = p.bias != nullptr && n < p.K ? static_cast<float>(static_cast<const T*>(p.bias)[n * p.bias_stride]) : 0.f;
         }
     const bool whole = n0 + 64 <= p.K;
 
@@ -78,7 +85,7 @@ __global__ __launch_bounds__(256, 3) void ThinConvKernel(ThinConvArgs p) {
         for (int k = 0; k < STEPS; ++k) {
             const int yy = y + (at[k] >> 16), xx = x + (at[k] & 0xffff);
             const bool ok = in & (yy >= 0) & (yy < p.H) & (xx >= 0) & (xx < p.W);
-            xf[k] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(xr, ok ? (corner + off[k]) * 4 : kOut, 0, 0));
+            xf[k] = LoadFloat<T>(xr, corner + off[k], ok);
         }
         float16_t acc[2];
 #pragma unroll
@@ -89,16 +96,17 @@ __global__ __launch_bounds__(256, 3) void ThinConvKernel(ThinConvArgs p) {
         for (int k = 0; k < STEPS; ++k)
 #pragma unroll
             for (int j = 0; j < 2; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(wf[j][k], xf[k], acc[j], 0, 0, 0);
-        const int to = ((img * p.K + n0 + 4 * h) * p.P + px) * 4;
+        const int to = ((img * p.K + n0 + 4 * h) * p.P + px) * static_cast<int>(sizeof(T));
 #pragma unroll
         for (int j = 0; j < 2; ++j)
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
                 const int n = j * 32 + 8 * (v / 4) + v % 4;  // + 4 * h
-                const int o = in & (whole | (n0 + n + 4 * h < p.K)) ? to + n * p.P * 4 : kOut;
+                const int o = in & (whole | (n0 + n + 4 * h < p.K)) ? to + n * p.P * static_cast<int>(sizeof(T)) : kOut;
                 float s = acc[j][v];
                 if (p.bias != nullptr) s += bias[j][v];
-                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(s), outr, o, 0, 0);
+                if constexpr (sizeof(T) == 4) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(s), outr, o, 0, 0);
+                else __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(unsigned short, static_cast<half_t>(s)), outr, o, 0, 0);
             }
     }
 }
@@ -106,7 +114,7 @@ __global__ __launch_bounds__(256, 3) void ThinConvKernel(ThinConvArgs p) {
 }  // namespace
 
 bool TryThinConv(const hipcx_array* x, const hipcx_array* w, const hipcx_array* b, const int64_t* stride, const int64_t* pad, const hipcx_array* out, hipStream_t stream) {
-    if (out->dtype != HIPCX_FLOAT32 || !IsContiguous(x) || !IsContiguous(w) || !IsContiguous(out)) return false;
+    if ((out->dtype != HIPCX_FLOAT32 && out->dtype != HIPCX_FLOAT16) || !IsContiguous(x) || !IsContiguous(w) || !IsContiguous(out)) return false;
     const int64_t N = x->shape[0], C = x->shape[1], H = x->shape[2], W = x->shape[3], K = w->shape[0], R = w->shape[2], S = w->shape[3];
     const int64_t OH = out->shape[2], OW = out->shape[3], P = OH * OW, terms = C * R * S;
     // (from 16 filters on, a quarter of a wave's: 51 -> 24 us for 256 images of 3 channels at 32^2)
@@ -117,22 +125,28 @@ bool TryThinConv(const hipcx_array* x, const hipcx_array* w, const hipcx_array* 
     if (H >= 0x4000 || W >= 0x4000 || OH >= 0x4000 || OW >= 0x4000 || stride[0] >= 0x4000 || stride[1] >= 0x4000 || pad[0] >= 0x4000 || pad[1] >= 0x4000) return false;
     if (OH * stride[0] >= 0x3000 || OW * stride[1] >= 0x3000) return false;
     ThinConvArgs p{};
-    p.x = static_cast<const float*>(x->data), p.w = static_cast<const float*>(w->data), p.out = static_cast<float*>(out->data);
-    p.bias = b != nullptr ? static_cast<const float*>(b->data) : nullptr;
-    p.bias_stride = b != nullptr ? b->strides[0] / 4 : 0;
+    const int64_t it = ItemSize(out->dtype);
+    p.x = x->data, p.w = w->data, p.out = out->data;
+    p.bias = b != nullptr ? b->data : nullptr;
+    p.bias_stride = b != nullptr ? b->strides[0] / it : 0;
     p.C = static_cast<int>(C), p.H = static_cast<int>(H), p.W = static_cast<int>(W), p.K = static_cast<int>(K), p.R = static_cast<int>(R), p.S = static_cast<int>(S);
     p.OW = static_cast<int>(OW), p.P = static_cast<int>(P);
     p.stride_h = static_cast<int>(stride[0]), p.stride_w = static_cast<int>(stride[1]), p.pad_h = static_cast<int>(pad[0]), p.pad_w = static_cast<int>(pad[1]);
     p.M = static_cast<int>(N * P), p.blocks = (p.M + 31) / 32;
-    p.x_bytes = static_cast<unsigned>(N * C * H * W * 4), p.w_bytes = static_cast<unsigned>(K * terms * 4), p.out_bytes = static_cast<unsigned>(N * K * P * 4);
+    p.x_bytes = static_cast<unsigned>(N * C * H * W * it), p.w_bytes = static_cast<unsigned>(K * terms * it), p.out_bytes = static_cast<unsigned>(N * K * P * it);
     p.div_P = FastDiv(p.P), p.div_OW = FastDiv(p.OW);
     const int columns = static_cast<int>((K + 63) / 64);
     // three workgroups to a compute unit, as the registers allow
     const int64_t groups = std::min<int64_t>((p.blocks + 3) / 4, std::max<int64_t>(1, 3LL * NumCUs() / columns));
-    ProfileScope prof(stream, 2.0 * p.M * K * terms, 4.0 * (static_cast<double>(N) * C * H * W + static_cast<double>(K) * terms + static_cast<double>(p.M) * K));
+    ProfileScope prof(stream, 2.0 * p.M * K * terms, it * (static_cast<double>(N) * C * H * W + static_cast<double>(K) * terms + static_cast<double>(p.M) * K));
     const dim3 grid(static_cast<unsigned>(groups), static_cast<unsigned>(columns));
-    if (terms <= 16) hipLaunchKernelGGL(ThinConvKernel<8>, grid, dim3(256), 0, stream, p);
-    else hipLaunchKernelGGL(ThinConvKernel<16>, grid, dim3(256), 0, stream, p);
+    auto launch = [&](auto tag) {
+        using T = decltype(tag);
+        if (terms <= 16) hipLaunchKernelGGL((ThinConvKernel<T, 8>), grid, dim3(256), 0, stream, p);
+        else hipLaunchKernelGGL((ThinConvKernel<T, 16>), grid, dim3(256), 0, stream, p);
+    };
+    if (out->dtype == HIPCX_FLOAT16) launch(half_t{});
+    else launch(float{});
     CheckLaunch("thin_conv");
     return true;
 }

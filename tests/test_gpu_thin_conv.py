@@ -1,4 +1,4 @@
-"""float32 convolutions of at most 32 terms (thin_conv.hip): one term to 32, remainders of pixel blocks and of 64 filters, strides, padding, cover_all,
+"""Convolutions of at most 32 terms (thin_conv.hip): one term to 32, remainders of pixel blocks and of 64 filters, strides, padding, cover_all,
 rectangular filters and a bias, against the oracle."""
 import numpy as np
 import pytest
@@ -10,19 +10,20 @@ from helpers import assert_close
 pytestmark = pytest.mark.gpu
 
 
+@pytest.mark.parametrize('dt,tol', [('float32', 32 * 2.0 ** -23), ('float16', 2.0 ** -10)])  # 32 terms, each rounded twice at most; an ulp
 @pytest.mark.parametrize('n,c,h,w,k,kh,kw,stride,pad,cover_all', [
     (3, 3, 32, 32, 64, 3, 3, 1, 1, False), (2, 1, 28, 28, 20, 5, 5, 1, 0, False), (1, 1, 5, 5, 16, 1, 1, 1, 0, False), (2, 3, 9, 11, 130, 3, 3, 2, 1, True),
     (5, 2, 7, 13, 65, 4, 4, 3, 2, False), (2, 4, 6, 6, 33, 2, 4, 1, (3, 0), False), (1, 16, 3, 50, 70, 2, 1, (1, 2), 0, True), (7, 3, 1, 1, 96, 3, 3, 1, 1, False),
 ])
-def test_against_oracle(n, c, h, w, k, kh, kw, stride, pad, cover_all):
+def test_against_oracle(dt, tol, n, c, h, w, k, kh, kw, stride, pad, cover_all):
     rng = np.random.default_rng(c * h + w)
-    x, f = rng.standard_normal((n, c, h, w)).astype(np.float32), rng.standard_normal((k, c, kh, kw)).astype(np.float32)
-    bias = rng.standard_normal(k).astype(np.float32)
+    x, f = rng.standard_normal((n, c, h, w)).astype(dt), rng.standard_normal((k, c, kh, kw)).astype(dt)
+    bias = rng.standard_normal(k).astype(dt)
     for b in (None, bias):
         got = chx.conv(chx.array(x), chx.array(f), None if b is None else chx.array(b), stride, pad, cover_all).get()
-        assert_close(got, O.conv(x, f, b, stride, pad, cover_all), 32 * 2.0 ** -23, 'conv')  # 32 terms, each rounded twice at most
+        assert_close(got, O.conv(x, f, b, stride, pad, cover_all), tol, 'conv')
     # whole numbers: exact in any order
-    xi, fi = rng.integers(-3, 4, x.shape).astype(np.float32), rng.integers(-3, 4, f.shape).astype(np.float32)
+    xi, fi = rng.integers(-3, 4, x.shape).astype(dt), rng.integers(-3, 4, f.shape).astype(dt)
     np.testing.assert_array_equal(chx.conv(chx.array(xi), chx.array(fi), None, stride, pad, cover_all).get(), O.conv(xi, fi, None, stride, pad, cover_all))
 
 
