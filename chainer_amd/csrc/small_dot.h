@@ -3,12 +3,13 @@
 //
 // A workgroup owns one 32x32 tile of `out` (SmallDotLinesKernel: 16 to 64 columns); its waves split the reduction axis -- and, with ksplit > 1, so do several workgroups, whose
 // sums another kernel adds up -- each feeding the MFMA from global memory on its own (operands this small live in the caches), and
-// the partial tiles are summed through LDS.  Four kernels, by where the operands lie (chosen in TrySmallDot):
+// the partial tiles are summed through LDS.  Five kernels, by where the operands lie (chosen in TrySmallDot):
 //   SmallDotKernel        k is the unit-stride axis of both operands (Linear's x and W^T): straight from global memory, bound by the
 //                         latency of a few loads.
 //   SmallDotLinesKernel   the same for more or longer tiles: whole 128-byte lines regrouped through LDS.
 //   SmallDotMixedKernel   an operand whose k axis is not the unit-stride one (dG . Wh of a recurrent network, x^T . gy), or float16 rows
 //                         of odd pitch.
+//   SmallDotColumnsKernel float32, both operands with m and n as the unit-stride axes, of outputs that make a 64 x 64 tile per compute unit.
 //   SmallDotVectorKernel  M <= 4 (one image, one sentence): a wave per output column, K across the lanes, where the MFMA would work on
 //                         32 rows.
 // For float the reduction index is dealt to the v_mfma_f32_32x32x2_f32 steps so that a lane's four steps use four consecutive k (one
@@ -549,6 +550,86 @@ __global__ __launch_bounds__(64 * kSmallDotMaxWaves) __attribute__((amdgpu_waves
         float s = 0.f;
         for (int w = 0; w < p.nw; ++w) s += part[w * kSmallDotPart + row * 33 + col];
         StoreTileElement<T>(p, split, out, om, on, s);
+    }
+}
+
+// float32, both operands k by k with m and n dense (weight gradients x^T . gy): tiles of 64 x 64 by four waves that split the reduction.  A lane's 16 bytes of
+// one k are a term each of four v_mfma_f32_16x16x4_f32 operands whose rows are every fourth one: lines arrive whole, in the order the MFMA takes them,
+// without LDS.  Bound by the float pipe.  us, against elements in tiles of
+// 32 x 32: [700,2600]^T . [700,650] 43 -> 34, [1000,1000]^T . [1000,1000] 34 -> 30, [100,1000]^T . [100,1000] 10.0 -> 8.1.
+template <typename T>
+__global__ __launch_bounds__(256, 2) void SmallDotColumnsKernel(SmallDotArgs p) {
+    static_assert(sizeof(T) == 4);
+    constexpr int U = 4, KC = 4 * U;  // loads of an operand and k per stage
+    constexpr int kOut = 0x7fffffff;
+    constexpr int kPitch = 64 + 4, kPart = 64 * kPitch;
+    extern __shared__ __align__(16) char lds[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r = lane & 15, g = lane >> 4;
+    const int tiles = p.tiles_m * p.tiles_n;
+    const int split = blockIdx.x / tiles;
+    int tm, tn;
+    SmallDotTile(tiles, blockIdx.x - split * tiles, p.tiles_m, tm, tn);
+    const int batch = blockIdx.y;
+    const __amdgpu_buffer_rsrc_t ar = MakeRsrc(static_cast<const float*>(p.a) + batch * p.a_batch, p.a_bytes);
+    const __amdgpu_buffer_rsrc_t br = MakeRsrc(p.b, p.b_bytes);
+    const int m = tm * 64 + 4 * r, n = tn * 64 + 4 * r;
+    const unsigned a_step = static_cast<unsigned>(p.a_k * 4), b_step = static_cast<unsigned>(p.b_k * 4);
+
+    const int chunks = (p.K + KC - 1) / KC;
+    const int per_split = (chunks + p.ksplit - 1) / p.ksplit;
+    const int end = min(chunks, (split + 1) * per_split);
+    float4_t acc[4][4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int f = 0; f < 4; ++f) acc[e][f] = float4_t{0.f, 0.f, 0.f, 0.f};
+    Bytes16 av[2][U], bv[2][U];
+    auto load = [&](int st, int c) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int k = c * KC + u * 4 + g;
+            const bool in = (k < p.K) & (c < end);
+            av[st][u] = __builtin_amdgcn_raw_buffer_load_b128(ar, (in & (m < p.M)) ? static_cast<int>(k * a_step + m * 4) : kOut, 0, 0);
+            bv[st][u] = __builtin_amdgcn_raw_buffer_load_b128(br, (in & (n < p.N)) ? static_cast<int>(k * b_step + n * 4) : kOut, 0, 0);
+        }
+    };
+    auto multiply = [&](int st) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int f = 0; f < 4; ++f)
+                    acc[e][f] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(av[st][u][e]), __uint_as_float(bv[st][u][f]), acc[e][f], 0, 0, 0);
+    };
+    // the waves take every fourth chunk; what lies beyond the last one is loaded as zeros
+    int c = split * per_split + wave;
+    load(0, c);
+    for (; c < end; c += 8) {
+        load(1, c + 4);
+        multiply(0);
+        load(0, c + 8);
+        multiply(1);
+    }
+    // lane holds rows 4 * (4 * g + v) + e, columns 4 * r + f
+    float* const mine = reinterpret_cast<float*>(lds) + wave * kPart;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+            *reinterpret_cast<float4_t*>(mine + (16 * g + 4 * v + e) * kPitch + 4 * r) = float4_t{acc[e][0][v], acc[e][1][v], acc[e][2][v], acc[e][3][v]};
+    __syncthreads();
+    float* out = static_cast<float*>(gridDim.y > 1 ? p.outs[batch] : p.out);
+    const float* const part = reinterpret_cast<const float*>(lds);
+    for (int e = tid; e < 64 * 64; e += 256) {
+        const int row = e >> 6, col = e & 63, om = tm * 64 + row, on = tn * 64 + col;
+        if (om >= p.M || on >= p.N) continue;
+        float s = 0.f;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) s += part[w * kPart + row * kPitch + col];
+        StoreTileElement<float>(p, split, out, om, on, s);
     }
 }
 

@@ -159,6 +159,21 @@ void LaunchSmallDot(SmallDotArgs p, int a_mode, int b_mode, int batch, hipStream
         CheckLaunch("small_dot");
         return;
     }
+    if constexpr (sizeof(T) == 4) {
+        // Once 64 x 64 tiles occupy three quarters of the compute units; us, elements in 32 x 32 tiles and these: [700,650]^T . [700,650], 121 tiles, 15.0
+        // and 19.4, [100,784]^T . [100,1000], 208, 8.8 and 7.9, [64,1300]^T . [64,1300], 441, 11.3 and 10.6.
+        const int64_t squares = static_cast<int64_t>((p.M + 63) / 64) * ((p.N + 63) / 64) * p.ksplit * batch;
+        if (a_mode == kElements && b_mode == kElements && p.a_row == 1 && p.b_col == 1 && 4 * squares >= 3 * NumCUs()) {
+            constexpr int kLds = 4 * 64 * (64 + 4) * 4;
+            p.tiles_m = (p.M + 63) / 64, p.tiles_n = (p.N + 63) / 64;
+            struct ColumnsTag {};
+            EnsureDynamicLds<ColumnsTag>(reinterpret_cast<const void*>(SmallDotColumnsKernel<float>), kLds);
+            hipLaunchKernelGGL((SmallDotColumnsKernel<float>), dim3(static_cast<unsigned>(static_cast<int64_t>(p.tiles_m) * p.tiles_n * p.ksplit), static_cast<unsigned>(batch)),
+                               dim3(256), kLds, stream, p);
+            CheckLaunch("small_dot_columns");
+            return;
+        }
+    }
     // Elements come as they are used: chunks of 32 bytes, six of them in flight, beat whole lines ([32,1000] . [1000,2048] float16 14.3 -> 5.5 us,
     // [200,4000] . [4000,4000] 174 -> 51, [20,2600] . [2600,650] float32 13.4 -> 9.3); rows of odd pitch gain from whole lines at any size.
     const bool elements = a_mode == kElements || b_mode == kElements, odd = a_mode == kOddPieces || b_mode == kOddPieces;
