@@ -425,6 +425,8 @@ NchwPlan PlanNchw(const hipcx_array* x, const hipcx_array* w, const hipcx_array*
     const bool is1 = R == 1 && S == 1 && pad[0] == 0 && pad[1] == 0 && stride[0] == stride[1];
     const bool is3 = R == 3 && S == 3 && pad[0] == 1 && pad[1] == 1 && stride[0] == 1 && stride[1] == 1;
     if (!is1 && !is3) return pl;
+    // a 1x1 kernel reads pixel (oh, ow) * stride without a look at the plane's edges, which cover_all may put it beyond
+    if (is1 && ((OH - 1) * stride[0] >= H || (OW - 1) * stride[1] >= W)) return pl;
     const int64_t P = OH * OW;
     // Pixels per activation load.  Wider loads would be fewer, but a thread's transposed 16-byte groups go to LDS
     // NPX slots apart from its neighbour's, and beyond a 32-byte lane stride those writes serialise on LDS banks

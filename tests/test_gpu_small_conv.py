@@ -55,3 +55,18 @@ def test_filters_that_are_a_view(size):
     X, pad = chx.array(x), size // 2
     np.testing.assert_array_equal(chx.conv(X, view, None, 1, pad).get(), chx.conv(X, view.copy(), None, 1, pad).get())
     assert_close(chx.conv(X, view, None, 1, pad).get(), O.conv(x, f.transpose((1, 0, 2, 3))[:, :, ::-1, ::-1], None, 1, pad), 2e-3, 'conv')
+
+
+@pytest.mark.parametrize('n,c,h,w,k,stride', [(2, 32, 8, 8, 16, 2), (1, 64, 8, 9, 40, 3), (1, 32, 7, 8, 33, 2), (1, 32, 8, 7, 33, 2), (64, 64, 56, 56, 128, 2)])
+def test_cover_all_reaches_beyond_the_plane(n, c, h, w, k, stride):
+    """Outputs whose only pixel lies behind the last row or column are the bias (the last case has the size of NchwConvKernel's)."""
+    rng = np.random.default_rng(h)
+    x, f = rng.integers(-2, 3, (n, c, h, w)).astype(np.float16), rng.integers(-1, 2, (k, c, 1, 1)).astype(np.float16)
+    b = rng.integers(-3, 4, k).astype(np.float16)
+    X, F, B = chx.array(x), chx.array(f), chx.array(b)
+    expected = O.conv(x, f, b, stride, 0, True)
+    assert (expected[:, :, -1, -1] == b).all()
+    np.testing.assert_array_equal(chx.conv(X, F, B, stride, 0, True).get(), expected)
+    bn = [np.ones(k, np.float16) for _ in range(4)]
+    got = chx.conv_bn_act(X, F, B, stride, 0, True, [chx.array(a) for a in bn], 0.0, None, True).get()
+    np.testing.assert_array_equal(got, np.maximum(expected, 0))
