@@ -82,11 +82,12 @@ void LaunchShape(IGemmArgs<T> p, bool fast16, bool fast8, hipStream_t stream) {
     double x_elems = static_cast<double>(p.N) * (p.xsN > 0 ? p.xsN : 1);
     bool fits32 = x_elems < 2147483647.0 && static_cast<double>(p.K) * p.wsK < 2147483647.0;
     static const bool use_pipe = [] { const char* e = getenv("HIPCX_IGEMM_PIPE"); return e != nullptr && e[0] == '1'; }();
-    // float32 on the bfloat16 pipes wherever its layout allows.  us before -> after: [4480,650] . [650,10000] 593 -> 398, [4480,10000] . [10000,650]
-    // 704 -> 441, [4096,4096]^2 1123 -> 734, [8192,100] . [100,3000] 76 -> 47; 3x3 convolutions of 256 images 64 -> 64 at 32^2 234 -> 167,
-    // 128 -> 128 at 16^2 204 -> 148, 256 -> 256 at 8^2 224 -> 156.  Relative error (2-norm) against 64 bits: 4.57e-7 -> 3.89e-7, 1.04e-6 -> 9.3e-7,
-    // 1.15e-6 -> 1.0e-6, 1.8e-7 -> 1.5e-7; 4.24e-7 -> 3.57e-7, 5.88e-7 -> 5.02e-7, 8.07e-7 -> 6.96e-7.
-    // [8192,8] . [8,512] 11.6 -> 10.1, 5.4e-8 -> 3.1e-8.
+    // float32 on the bfloat16 pipes wherever its layout allows.  us, float pipe and these, and the relative errors (2-norm) against 64 bits:
+    //   [4480,650] . [650,10000]   600 and 400, 4.56e-7 and 1.45e-7     3x3 convolutions of 256 images:
+    //   [4480,10000] . [10000,650] 711 and 480, 1.03e-6 and 4.4e-7        64 -> 64 at 32^2   226 and 173, 4.26e-7 and 1.35e-7
+    //   [4096,4096]^2             1134 and 806, 1.15e-6 and 4.0e-7        128 -> 128 at 16^2 199 and 143, 5.91e-7 and 1.93e-7
+    //   [8192,512] . [512,2048]    169 and 122, 4.06e-7 and 1.28e-7       256 -> 256 at 8^2  220 and 159, 8.16e-7 and 2.72e-7
+    //   [8192,8] . [8,512]        12.1 and 10.6, 5.4e-8 and 2.8e-8
     static const bool use_split = [] { const char* e = getenv("HIPCX_IGEMM_SPLIT"); return e == nullptr || e[0] != '0'; }();
     bool split = false;
     if constexpr (sizeof(T) == 4) split = use_split && (fast16 || fast8) && IGemmSplit<WM, WN>(p, fast16 ? 16 : 8, PM, grid, stream);
@@ -1265,13 +1266,14 @@ int hipcx_conv_bn_act(const hipcx_array* x, const hipcx_array* w, const hipcx_ar
 namespace {
 // Matrix products with few 128x128 output tiles and a long reduction axis (weight gradients: M x N = filters, reduction = batch x
 // pixels): slices of the reduction run as separate workgroups.  Returns the number of slices (1: no split).
-int PlanSplitK(int64_t m, int64_t n, int64_t k, int dtype) {
+// `on_bf16`: on the split kernel for float32, which two workgroups to a compute unit fill ([4480,10000] . [10000,650] in three slices 523 us, in two 494).
+int PlanSplitK(int64_t m, int64_t n, int64_t k, int dtype, bool on_bf16) {
     static const bool enabled = [] { const char* e = getenv("HIPCX_DOT_SPLITK"); return e == nullptr || e[0] != '0'; }();
     if (!enabled || (dtype != HIPCX_FLOAT16 && dtype != HIPCX_FLOAT32)) return 1;
     const int64_t tiles = ((m + 127) / 128) * ((n + 127) / 128);
     const int64_t steps = k * ItemSize(dtype) / 128;  // reduction steps of 128 bytes per row
     if (k < 4096 || tiles > NumCUs() || m * n < 64 * 64 || steps < 16) return 1;  // up to one tile per compute unit: a second workgroup per unit still hides latency
-    int64_t s = (2 * NumCUs() + tiles - 1) / tiles;
+    int64_t s = on_bf16 ? 2 * NumCUs() / tiles : (2 * NumCUs() + tiles - 1) / tiles;
     static const int64_t min_steps = [] { const char* e = getenv("HIPCX_DOT_SPLITK_MINSTEPS"); int v = e ? atoi(e) : 0; return v >= 1 && v <= 4096 ? v : 8; }();
     if (s > steps / min_steps) s = steps / min_steps;  // a slice of fewer steps costs more in partial sums than it gains
     static const int64_t max_slices = [] { const char* e = getenv("HIPCX_DOT_SPLITK_MAX"); int v = e ? atoi(e) : 0; return v >= 2 && v <= 1024 ? v : 256; }();
@@ -1313,7 +1315,7 @@ DotStaging PlanDotStaging(const hipcx_array* a, const hipcx_array* b, const hipc
     // ([1000,8192]^T . [8192,1000] 217 -> 155 us, [1000,4500]^T . [4500,784] 117 -> 110; [500,8192]^T . [8192,500] would go from 60 to 74).
     const double flops = 2.0 * m * n * k;
     if (flops < 2e8) return st;
-    if (SmallDotShape(m, n, k) && !(out->dtype == HIPCX_FLOAT32 && flops >= 7e9 && PlanSplitK(m, n, k, out->dtype) > 1)) return st;
+    if (SmallDotShape(m, n, k) && !(out->dtype == HIPCX_FLOAT32 && flops >= 7e9 && PlanSplitK(m, n, k, out->dtype, true) > 1)) return st;
     const int64_t epv = 16 / it;
     st.kpad = (k + epv - 1) / epv * epv;
     // a changed pitch on one side needs the same (zero-padded) k extent on the other
@@ -1477,7 +1479,7 @@ bool TryGemmPp(const hipcx_array* a, const hipcx_array* b, const hipcx_array* bi
 int BatchedProductSlices(int64_t m, int64_t n, int64_t depth, int batch, int dtype) {
     const int64_t it = ItemSize(dtype);
     const int64_t steps_per = (depth * it + 127) / 128;
-    const int planned = PlanSplitK(m, n, depth * batch, dtype);
+    const int planned = PlanSplitK(m, n, depth * batch, dtype, false);
     const int64_t steps = steps_per * batch;
     return planned > steps ? static_cast<int>(steps) : planned;
 }
@@ -1645,7 +1647,7 @@ static int DotBias(const hipcx_array* a, const hipcx_array* b, const hipcx_array
         {
             const int64_t it = ItemSize(out->dtype);
             // slices from the extent the workspace query planned with; the partial sums lie behind the staged operands
-            const int planned = PlanSplitK(m, n, k_given, out->dtype);
+            const int planned = PlanSplitK(m, n, k_given, out->dtype, out->dtype == HIPCX_FLOAT32);
             if (planned > 1 && OperandIsFast(a->data, a->strides[0], a->strides[1], k, it) &&
                 OperandIsFast(b->data, b->strides[1], b->strides[0], k, it) && out->strides[0] >= 0 && out->strides[1] >= 0) {
                 const size_t offset = RoundUpTo(staged_bytes, 256);
@@ -1698,7 +1700,7 @@ size_t hipcx_dot_workspace_size(const hipcx_array* a, const hipcx_array* b, cons
             // the 128 x 128 tiles split the reduction of operands laid out (or staged) for them, else the small product's tiles do
             const bool fast = (st.a || OperandIsFast(a->data, a->strides[0], a->strides[1], k, it)) &&
                               (st.b || OperandIsFast(b->data, b->strides[1], b->strides[0], k, it));
-            if (fast) split = SplitKBytes(m, n, PlanSplitK(m, n, k, out->dtype));
+            if (fast) split = SplitKBytes(m, n, PlanSplitK(m, n, k, out->dtype, out->dtype == HIPCX_FLOAT32));
             if (split == 0 && !st.a && !st.b && a->dtype == out->dtype && b->dtype == out->dtype) split = SmallDotWorkspace(a, b, out->dtype);
         }
         const size_t need = RoundUpTo(st.a_bytes + st.b_bytes, 256) + split;

@@ -2,22 +2,22 @@
 //
 // v_mfma_f32_32x32x16_bf16 does sixteen times the multiply-adds of v_mfma_f32_32x32x2_f32 in a clock.  A float is the sum of three
 // bfloat16 numbers, exactly: x1 = bf16(x), x2 = bf16(x - x1), x3 = x - x1 - x2 (24 significant bits = 3 x 8; rounding to nearest leaves
-// remainders of at most half a unit, which have 16 and 8 bits).  Of the nine products of two such sums six are computed, smallest
-// first, x3 w1, x1 w3, x2 w2, x2 w1, x1 w2, x1 w1, into one float accumulator; what is left out is at most 2^-23 of x w and 2^-27 in the mean, below the
-// mean rounding of a float product, and of either sign.  A bfloat16 product is exact in float32, so the only roundings are the accumulator's, and those are
-// fewer than the float pipe's (six per 16 terms instead of one per term).  Against 64-bit sums the results are closer than the float pipe's: see
-// LaunchShape.
+// remainders of at most half a unit, which have 16 and 8 bits).  Of the nine products of two such sums all but x3 w3, at most 2^-34 of x w, are
+// computed.  A bfloat16 product is exact in float32; the matrix pipe's additions are not rounded to nearest (one product added to the sum of its
+// small parts may be off by a whole unit).  Hence two accumulators: x1 w1, whose 16 bits leave room for a few terms without any rounding and which
+// is rounded once for 16 terms, and the seven others, 2^-8 of it, whose roundings do not show; they are added at the end.  Largest relative error of
+// one term 5.98e-8 (5.96e-8 on the float pipe, rounded to nearest; 1.5e-7 with one accumulator and six products), 2-norm for two to eight terms
+// among zeros 2.6 to 2.8e-8 (3.1 to 5.4e-8; 4.1 to 8.2e-8), for more see LaunchShape.
 //
 // Where the split is not exact the tile is computed again on the float pipe, by the same workgroup: a sum that is not finite (an operand that
-// is infinite, NaN or beyond bfloat16's range, or a sum that overflowed), or a nonzero operand below 2^-110, whose last bits bfloat16 has no
-// numbers for (its least is 2^-133).
+// is infinite, NaN or beyond bfloat16's range, or a sum that overflowed), a nonzero sum so small that its parts' roundings to multiples of 2^-149 add
+// up, or a nonzero operand below 2^-110, whose last bits bfloat16 has no numbers for (its least is 2^-133).
 //
 // Layout: a workgroup's rows of x and w are split while they are staged, each element once, into three planes of LDS, 16 k at a time; a plane's
 // rows have 32 bytes, whose two pieces change places every eight rows, so that the staging writes and the fragment reads (16 bytes of 16 rows) both
-// use all banks.  12 fragment reads feed 24 MFMAs of a wave's 64 x 64 block.  The next step's rows are split into the other stage between the MFMAs of
-// the current one, with one barrier a step; 48 KiB for a 128 x 128 tile, three workgroups to a compute unit.
-// Bound by the MFMAs and the splitting together: at [6144,4096] . [4096,4096], 1.24 ms (166 TFLOP/s; 0.5 ms of MFMAs at their peak rate), a third of
-// the MFMAs take 0.82 ms, no loads 1.09, no staging writes 1.17, no fragment reads 1.13.
+// use all banks.  12 fragment reads feed 32 MFMAs of a wave's 64 x 64 block.  The next step's rows are split into the other stage between the MFMAs of
+// the current one, with one barrier a step; 48 KiB for a 128 x 128 tile, two workgroups to a compute unit, as the registers allow.
+// Bound by the MFMAs (at [4096,4096]^2 0.44 of 0.81 ms) and by the splitting.
 #include "igemm_split.h"
 
 #include <type_traits>
@@ -53,23 +53,30 @@ constexpr unsigned kSplitLeast = (17u << 24) - 1u;
 
 __device__ __forceinline__ unsigned SplitKey(unsigned bits) { return (bits << 1) - 1u; }
 
-// Whether all sums are finite: x * 0 is 0 for those only.
-__device__ __forceinline__ bool AllFinite(const float16_t (&acc)[2][2]) {
+// Sums from here on are not rounded to multiples of 2^-149 by their parts' additions.
+constexpr float kSplitLeastSum = 0x1p-120f;
+
+// Whether all sums are finite (x * 0 is 0 for those only) and none is a tiny one.
+__device__ __forceinline__ bool AllOrdinary(const float16_t (&acc)[2][2]) {
     bool all = true;
+    unsigned least = ~0u;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             float zero = 0.f;
 #pragma unroll
-            for (int v = 0; v < 16; ++v) zero += acc[i][j][v] * 0.f;
+            for (int v = 0; v < 16; ++v) {
+                zero += acc[i][j][v] * 0.f;
+                least = min(least, SplitKey(__float_as_uint(acc[i][j][v])));
+            }
             all &= zero == 0.f;
         }
-    return all;
+    return all & (least >= SplitKey(__float_as_uint(kSplitLeastSum)));
 }
 
 template <int WM, int WN, int LB, bool PM>
-__global__ __launch_bounds__(64 * WM * WN) void IGemmSplitKernel(IGemmArgs<float> p) {
+__global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2))) void IGemmSplitKernel(IGemmArgs<float> p) {
     constexpr int NT = 64 * WM * WN;
     constexpr int BM = 64 * WM;
     constexpr int BN = 64 * WN;
@@ -193,14 +200,14 @@ __global__ __launch_bounds__(64 * WM * WN) void IGemmSplitKernel(IGemmArgs<float
     const int lr = lane & 31, g = lane >> 5;
     const int xfrag = (wm * 64 + lr) * kSplitRow + (g ^ ((lr >> 3) & 1)) * 16;
     const int wfrag = (BM + wn * 64 + lr) * kSplitRow + (g ^ ((lr >> 3) & 1)) * 16;
-    float16_t acc[2][2];
+    float16_t acc[2][2], low[2][2];
     auto clear = [&] {
 #pragma unroll
         for (int i = 0; i < 2; ++i)
 #pragma unroll
             for (int j = 0; j < 2; ++j)
 #pragma unroll
-                for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+                for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f, low[i][j][v] = 0.f;
     };
     // One step: the fragments of stage kt & 1 are multiplied while the next step's rows, which have arrived in registers, are split into the other
     // stage and the loads of the step behind it go out.
@@ -216,22 +223,23 @@ __global__ __launch_bounds__(64 * WM * WN) void IGemmSplitKernel(IGemmArgs<float
             }
         if constexpr (decltype(split_tag)::value) split_tile(lds + (~kt & 1) * STAGE);
         if constexpr (decltype(load_tag)::value) load_tile();
-        constexpr int kX[6] = {2, 0, 1, 1, 0, 0}, kW[6] = {0, 2, 1, 0, 1, 0};
+        constexpr int kX[8] = {2, 1, 2, 0, 1, 1, 0, 0}, kW[8] = {1, 2, 0, 2, 1, 0, 1, 0};
 #pragma unroll
-        for (int c = 0; c < 6; ++c)
+        for (int c = 0; c < 8; ++c)
 #pragma unroll
             for (int ti = 0; ti < 2; ++ti)
 #pragma unroll
                 for (int tj = 0; tj < 2; ++tj) {
-                    if (PM) MfmaBf16(xf[kX[c]][ti], wf[kW[c]][tj], acc[ti][tj]);
-                    else MfmaBf16(wf[kW[c]][ti], xf[kX[c]][tj], acc[ti][tj]);
+                    float16_t& sum = c == 7 ? acc[ti][tj] : low[ti][tj];
+                    if (PM) MfmaBf16(xf[kX[c]][ti], wf[kW[c]][tj], sum);
+                    else MfmaBf16(wf[kW[c]][ti], xf[kX[c]][tj], sum);
                 }
         if constexpr (decltype(split_tag)::value) {
             __builtin_amdgcn_sched_group_barrier(0x100, 12, 0);
 #pragma unroll
-            for (int i = 0; i < 24; ++i) {
+            for (int i = 0; i < 32; ++i) {
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
                 if (i % 2 == 1) __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
             }
         }
@@ -258,7 +266,11 @@ __global__ __launch_bounds__(64 * WM * WN) void IGemmSplitKernel(IGemmArgs<float
         step(kt, false_type{}, false_type{});
     }
 
-    if (__syncthreads_or(least < kSplitLeast || !AllFinite(acc))) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] += low[i][j];
+    if (__syncthreads_or(least < kSplitLeast || !AllOrdinary(acc))) {
         clear();
         seek(kt_begin);
         for (int kt = kt_begin; kt < kt_end; ++kt) {

@@ -8,7 +8,7 @@ import chainer_amd as chx
 pytestmark = pytest.mark.gpu
 
 # A sum of K float products in any order, each and each partial sum rounded once, is within K 2^-24 of the sum of magnitudes (to first order); what the
-# split leaves out of a product is at most 2^-23 of it.
+# split leaves out of a product is at most 2^-34 of it.
 _EPS = 2.0 ** -24
 
 
@@ -87,3 +87,23 @@ def test_sums_that_overflow_in_part():
     got = chx.linear(chx.array(x), chx.array(w)).get()
     np.testing.assert_array_equal(got, np.full_like(got, x[0, 3] * w[0, 3]))
     assert np.isfinite(got).all()
+
+
+@pytest.mark.parametrize('scale', [0, -60, -99, -102])
+@pytest.mark.parametrize('terms,float_pipe', [(1, 2.53e-8), (2, 3.16e-8), (5, 4.39e-8)])
+def test_sums_of_few_terms_among_zeros(terms, float_pipe, scale):
+    """One term is rounded once: to half a unit, 2^-24 of it, and what the small parts' own roundings, units of 2^-7 of it at most, do to that.  With more,
+    the sum of the upper parts' products and the last addition round too.  Scaled down, the third parts of x are bfloat16's subnormal numbers."""
+    rng = np.random.default_rng(terms)
+    m, k, n = 2048, 64, 1024
+    x = np.zeros((m, k), np.float32)
+    for j in range(terms):
+        x[np.arange(m), (np.arange(m) * 7 + 11 * j) % k] = (rng.uniform(1, 2, m) * rng.choice([-1, 1], m)).astype(np.float32)
+    x *= np.float32(2.0 ** scale)
+    w = rng.uniform(1, 2, (n, k)).astype(np.float32)
+    got = chx.linear(chx.array(x), chx.array(w)).get().astype(np.float64)
+    exact, magnitude = x.astype(np.float64) @ w.T.astype(np.float64), np.abs(x).astype(np.float64) @ np.abs(w.T).astype(np.float64)
+    roundings = 1 + 2.0 ** -6 if terms == 1 else 2 * terms + 1  # (the matrix pipe's additions are off by a unit, two halves, at most)
+    assert (np.abs(got - exact) / magnitude).max() <= roundings * _EPS
+    # no farther off in the 2-norm than v_mfma_f32_32x32x2_f32, which rounds to nearest after every term
+    assert np.linalg.norm(got - exact) <= 1.01 * float_pipe * np.linalg.norm(exact)
