@@ -11,7 +11,8 @@
 //
 // Where the split is not exact the tile is computed again on the float pipe, by the same workgroup: a sum that is not finite (an operand that
 // is infinite, NaN or beyond bfloat16's range, or a sum that overflowed), a nonzero sum so small that its parts' roundings to multiples of 2^-149 add
-// up, or a nonzero operand below 2^-110, whose last bits bfloat16 has no numbers for (its least is 2^-133).
+// up, or a nonzero operand below 2^-110, whose last bits bfloat16 has no numbers for (its least is 2^-133), in a row whose sum is small enough
+// for those to count.
 //
 // Layout: a workgroup's rows of x and w are split while they are staged, each element once, into three planes of LDS, 16 k at a time; a plane's
 // rows have 32 bytes, whose two pieces change places every eight rows, so that the staging writes and the fragment reads (16 bytes of 16 rows) both
@@ -270,7 +271,64 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2)
     for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int j = 0; j < 2; ++j) acc[i][j] += low[i][j];
-    if (__syncthreads_or(least < kSplitLeast || !AllOrdinary(acc))) {
+    bool again = !AllOrdinary(acc);
+    if (__syncthreads_or(least < kSplitLeast)) {
+        // Operands lost at most 2^-134 each, which changes a sum by less than 2^-133 terms times the largest operand: by less than 2^-29 of it, an eighth of
+        // a rounding, from 2^-104 terms times that operand on.  The rows are read once more, to see which of them this is about.
+        constexpr int kDeep = 16 / (XCH + WCH);  // steps in flight
+        unsigned* const keys = reinterpret_cast<unsigned*>(lds);  // the least key of each row, then the waves' largest operands
+        unsigned row_least[XCH + WCH], most = 0;
+#pragma unroll
+        for (int i = 0; i < XCH + WCH; ++i) row_least[i] = ~0u;
+        seek(kt_begin);
+        for (int kt = kt_begin; kt < kt_end; kt += kDeep) {  // (what lies beyond kt_end may count too; beyond the last k are zeros)
+            Chunk rows[kDeep][XCH + WCH];
+#pragma unroll
+            for (int u = 0; u < kDeep; ++u) {
+                load_tile();
+#pragma unroll
+                for (int i = 0; i < XCH; ++i) rows[u][i] = xreg[i];
+#pragma unroll
+                for (int i = 0; i < WCH; ++i) rows[u][XCH + i] = wreg[i];
+            }
+#pragma unroll
+            for (int u = 0; u < kDeep; ++u)
+#pragma unroll
+                for (int i = 0; i < XCH + WCH; ++i)
+#pragma unroll
+                    for (int e = 0; e < EPC; ++e) {
+                        row_least[i] = min(row_least[i], SplitKey(rows[u][i][e]));
+                        most = max(most, rows[u][i][e] & 0x7fffffffu);
+                    }
+        }
+#pragma unroll
+        for (int i = 0; i < XCH + WCH; ++i) {
+#pragma unroll
+            for (int o = 1; o < CPR; o <<= 1) row_least[i] = min(row_least[i], static_cast<unsigned>(__shfl_xor(static_cast<int>(row_least[i]), o)));
+            if (kc == 0) keys[i < XCH ? row0 + i * RPP : BM + row0 + (i - XCH) * RPP] = row_least[i];
+        }
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) most = max(most, static_cast<unsigned>(__shfl_xor(static_cast<int>(most), o)));
+        if (lane == 0) keys[BM + BN + wave] = most;
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < WM * WN; ++i) most = max(most, keys[BM + BN + i]);
+        const float enough = 0x1p-104f * static_cast<float>((kt_end - kt_begin) * kSplitStep) * __uint_as_float(most);
+#pragma unroll
+        for (int ti = 0; ti < 2; ++ti)
+#pragma unroll
+            for (int tj = 0; tj < 2; ++tj) {
+                const int row_at = PM ? wm * 64 + ti * 32 : BM + wn * 64 + ti * 32, col_at = PM ? BM + wn * 64 + tj * 32 : wm * 64 + tj * 32;
+                const unsigned col = keys[col_at + lr];
+#pragma unroll
+                for (int v = 0; v < 16; ++v) {
+                    const unsigned row = keys[row_at + 8 * (v / 4) + 4 * g + v % 4];
+                    // (a sum over a row of zeros is zero)
+                    again |= (min(row, col) < kSplitLeast) & (max(row, col) != ~0u) & (fabsf(acc[ti][tj][v]) < enough);
+                }
+            }
+    }
+    if (__syncthreads_or(again)) {
         clear();
         seek(kt_begin);
         for (int kt = kt_begin; kt < kt_end; ++kt) {

@@ -107,3 +107,23 @@ def test_sums_of_few_terms_among_zeros(terms, float_pipe, scale):
     assert (np.abs(got - exact) / magnitude).max() <= roundings * _EPS
     # no farther off in the 2-norm than v_mfma_f32_32x32x2_f32, which rounds to nearest after every term
     assert np.linalg.norm(got - exact) <= 1.01 * float_pipe * np.linalg.norm(exact)
+
+
+def test_tiny_values_beside_ordinary_ones():
+    """Bits below 2^-133 are lost in the split, which counts only in sums that are as small."""
+    rng = np.random.default_rng(7)
+    m, k, n = 2100, 200, 1100
+    x, w = rng.standard_normal((m, k), dtype=np.float32), rng.standard_normal((n, k), dtype=np.float32)
+    tiny = (rng.standard_normal((m, k)) * 2.0 ** -116).astype(np.float32)
+    x[::3, 5] = tiny[::3, 5]      # among others
+    x[7::128] = tiny[7::128]      # rows of nothing else
+    x[9::128] = 0
+    x[9::128, 3] = tiny[9::128, 3]
+    x[11::128] = 0
+    w[4::200] *= np.float32(2.0 ** -112)
+    w[6::200] = 0
+    got = chx.linear(chx.array(x), chx.array(w)).get().astype(np.float64)
+    exact, magnitude = x.astype(np.float64) @ w.T.astype(np.float64), np.abs(x).astype(np.float64) @ np.abs(w.T).astype(np.float64)
+    # as in a sum of ordinary products; each product and sum also rounds to a multiple of 2^-149
+    np.testing.assert_array_less(np.abs(got - exact), (k + 4) * _EPS * magnitude + 2 * k * 2.0 ** -150)
+    assert (got[11::128] == 0).all() and (got[:, 6::200] == 0).all()
