@@ -1612,6 +1612,10 @@ static int DotBias(const hipcx_array* a, const hipcx_array* b, const hipcx_array
         size_t staged_bytes = 0;    // the front of the workspace that holds staged operands
         if (out->dtype == a->dtype && out->dtype == b->dtype) {
             DotStaging plan = PlanDotStaging(a, b, out);
+            if ((plan.a || plan.b) && SmallDotShape(m, n, k)) {  // without room for the copies and the partial sums their own kernel takes the operands as they lie
+                const size_t need = RoundUpTo(plan.a_bytes + plan.b_bytes, 256) + SplitKBytes(m, n, PlanSplitK(m, n, k, out->dtype, true));
+                if (workspace == nullptr || workspace_bytes < need || !Aligned(workspace, 16)) plan = DotStaging{};
+            }
             if (plan.a || plan.b) {
                 staged_bytes = plan.a_bytes + plan.b_bytes;
                 HIPCX_REQUIRE(workspace != nullptr && workspace_bytes >= plan.a_bytes + plan.b_bytes, HIPCX_CHAINERX_ERROR,

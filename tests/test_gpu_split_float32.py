@@ -4,6 +4,8 @@ import numpy as np
 import pytest
 
 import chainer_amd as chx
+from chainer_amd import _lib
+from chainer_amd._array import current_stream
 
 pytestmark = pytest.mark.gpu
 
@@ -127,3 +129,16 @@ def test_tiny_values_beside_ordinary_ones():
     # as in a sum of ordinary products; each product and sum also rounds to a multiple of 2^-149
     np.testing.assert_array_less(np.abs(got - exact), (k + 4) * _EPS * magnitude + 2 * k * 2.0 ** -150)
     assert (got[11::128] == 0).all() and (got[:, 6::200] == 0).all()
+
+
+@pytest.mark.parametrize('given', [0, 256, 1 << 24])
+def test_small_outputs_need_no_workspace(given):
+    """Transposed operands of a small output are copied for these kernels where there is room, and multiplied as they lie where there is not."""
+    rng = np.random.default_rng(2)
+    m, k, n = 1000, 4100, 900
+    x, g = rng.standard_normal((k, m), dtype=np.float32), rng.standard_normal((k, n), dtype=np.float32)
+    X, G, out = chx.array(x).T, chx.array(g), chx.zeros((m, n), np.float32)
+    assert _lib.load().hipcx_dot_workspace_size(X.desc(), G.desc(), out.desc()) > given
+    room = chx.zeros((max(given, 16),), np.uint8)
+    _lib.call('hipcx_dot', X.desc(), G.desc(), out.desc(), room.data_ptr if given else None, given, current_stream())
+    _check(out.get(), x.T, g.T)
