@@ -1312,16 +1312,21 @@ DotStaging PlanDotStaging(const hipcx_array* a, const hipcx_array* b, const hipc
     const bool b_fast = OperandIsFast(b->data, b->strides[1], b->strides[0], k, it);
     if (a_fast && b_fast) return st;
     // worth it only when the product is large against the copies; small outputs have their own kernel (any layout), which takes elements as they
-    // lie but at the float pipe's rate: from 7 GFLOP on a float32 product whose reduction is split is faster staged, on the bfloat16 pipes
-    // ([1000,8192]^T . [8192,1000] 217 -> 155 us, [1000,4500]^T . [4500,784] 117 -> 110; [500,8192]^T . [8192,500] would go from 60 to 74).
+    // lie but at the float pipe's rate: from 7 GFLOP on a float32 product whose reduction is split is faster staged, on the bfloat16 pipes, unless
+    // more lines are copied than the output is worth.  us, staged and not: [1000,8192]^T . [8192,1000], both copied, 160 and 190, [1000,4500]^T .
+    // [4500,784] 106 and 110, [512,16384]^T . [16384,512] 107 and 106, b alone 96 and 111; [600,60000]^T . [60000,100] 164 and 137, b alone 103 and 162.
     const double flops = 2.0 * m * n * k;
     if (flops < 2e8) return st;
-    if (SmallDotShape(m, n, k) && !(out->dtype == HIPCX_FLOAT32 && flops >= 7e9 && PlanSplitK(m, n, k, out->dtype, true) > 1)) return st;
-    const int64_t epv = 16 / it;
-    st.kpad = (k + epv - 1) / epv * epv;
+    const int64_t epv = 16 / it, kpad = (k + epv - 1) / epv * epv;
     // a changed pitch on one side needs the same (zero-padded) k extent on the other
-    st.a = !a_fast || st.kpad != k;
-    st.b = !b_fast || st.kpad != k;
+    const bool copy_a = !a_fast || kpad != k, copy_b = !b_fast || kpad != k;
+    if (SmallDotShape(m, n, k)) {
+        const int64_t lines = (copy_a ? m : 0) + (copy_b ? n : 0);
+        if (out->dtype != HIPCX_FLOAT32 || flops < 7e9 || m * n < 256 * lines || PlanSplitK(m, n, k, out->dtype, true) == 1) return st;
+    }
+    st.kpad = kpad;
+    st.a = copy_a;
+    st.b = copy_b;
     st.a_bytes = st.a ? RoundUpTo(static_cast<size_t>(m * st.kpad * it), 256) : 0;
     st.b_bytes = st.b ? RoundUpTo(static_cast<size_t>(n * st.kpad * it), 256) : 0;
     return st;

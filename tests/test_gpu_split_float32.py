@@ -142,3 +142,9 @@ def test_small_outputs_need_no_workspace(given):
     room = chx.zeros((max(given, 16),), np.uint8)
     _lib.call('hipcx_dot', X.desc(), G.desc(), out.desc(), room.data_ptr if given else None, given, current_stream())
     _check(out.get(), x.T, g.T)
+
+
+def test_narrow_outputs_are_not_worth_long_copies():
+    a, b, out = chx.zeros((60000, 600), np.float32), chx.zeros((60000, 100), np.float32), chx.zeros((600, 100), np.float32)
+    need = lambda x: _lib.load().hipcx_dot_workspace_size(x.desc(), b.desc(), out.desc())
+    assert need(a.T) < 4 * 60000 * 100 <= need(a.reshape((600, 60000)))
