@@ -373,6 +373,9 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2)
 template <int WM, int WN>
 bool IGemmSplit(const IGemmArgs<float>& p, int chunk_bytes, bool pm, dim3 grid, hipStream_t stream) {
     constexpr int BM = 64 * WM, BN = 64 * WN;
+    // A single tile of a few terms stays on the float pipe: bound by the launch and the first loads, it has a microsecond to gain ([6,40] . [40,64] 8.3 and
+    // 7.4 us) and keeps the sums, rounded to nearest term by term, that recurrent networks amplify.
+    if (p.tiles_m * p.tiles_n == 1 && p.Kg < 64) return false;
     if (p.batch > 0 || p.w_taps_s > 0 || p.xsN < 0 || p.xsH < 0 || p.xsW < 0 || p.wsK < 0) return false;
     if ((p.R > 1 || p.S > 1) && p.C % kSplitStep != 0) return false;  // a step would reach over several filter positions
     // the kernel's offsets from a tile's first image and first filter have 32 bits
