@@ -629,8 +629,11 @@ public:
         used_ += Round256(static_cast<size_t>(floats) * 4);
         return p;
     }
-    // everything after the pieces is scratch for the library calls; call once all pieces are taken
-    void StartScratch() { scratch_off_ = used_; }
+    // everything after the pieces is scratch for the library calls; call once all pieces are taken, before anything is launched
+    void StartScratch() {
+        scratch_off_ = used_;
+        CheckFits();
+    }
     size_t Need() const { return scratch_off_ + scratch_need_; }
     void CheckFits() const {
         HIPCX_REQUIRE(dry_ || Need() <= bytes_, HIPCX_CHAINERX_ERROR, "n_step_rnn workspace too small: need " + std::to_string(Need()) + " bytes");

@@ -139,3 +139,35 @@ def test_infinite_inputs_and_states(kind):
     assert_close(hy.get(), ref[0], 1e-5, 'hy')
     for y, r in zip(ys, ref[-1]):
         assert_close(y.get(), r, 1e-5, 'y')
+
+
+def _arguments(chx, kind, layers, in_size, units, lengths, seed):
+    """Arrays and descriptor pointers for direct calls of the C entries: (hx, cx, pointers of ws, bs, xs), and what they point to."""
+    from chainer_amd import routines
+    ws, bs, _, xs, hx, cx = _rnn_problem(np.random.default_rng(seed), kind, layers, False, in_size, units, lengths)
+    W, B, X = [chx.array(m) for g in ws for m in g], [chx.array(v) for g in bs for v in g], [chx.array(x) for x in xs]
+    return chx.array(hx), chx.array(cx), [routines._descriptor_pointers(a) for a in (W, B, X)], (W, B, X)
+
+
+@pytest.mark.parametrize('kind', ['lstm', 'gru', 'rnn'])
+@pytest.mark.parametrize('training', [0, 1])
+def test_workspace_too_small(kind, training):
+    """Refused before anything is written."""
+    import ctypes
+    import chainer_amd as chx
+    from chainer_amd import _lib, routines
+    from chainer_amd._array import current_stream
+    mode, units = {'gru': 0, 'lstm': 1, 'rnn': 2}[kind], 40
+    hx, cx, (pw, pb, px), (W, B, X) = _arguments(chx, kind, 2, 24, units, (4, 4, 3, 1), 3)
+    L, T = _lib.load(), len(X)
+    reserve = chx.zeros((L.hipcx_n_step_rnn_reserve_size(2, 0, mode, hx.desc(), px, T),), np.uint8) if training else None
+    need = L.hipcx_n_step_rnn_workspace_size(2, 0, mode, training, hx.desc(), px, T)
+    room = chx.array(np.full(need, 255, np.uint8))
+    hy, cy = chx.zeros(hx.shape, np.float32), chx.zeros(hx.shape, np.float32)
+    ys = [chx.zeros((x.shape[0], units), np.float32) for x in X]
+    for given in (256, 2048):
+        with pytest.raises(chx.ChainerxError, match='too small'):
+            _lib.call('hipcx_n_step_rnn', 2, 0, mode, 0, hx.desc(), cx.desc() if kind == 'lstm' else None, pw, pb, px, T, hy.desc(),
+                      cy.desc() if kind == 'lstm' else None, routines._descriptor_pointers(ys), ctypes.c_void_p(reserve.data_ptr) if training else None,
+                      reserve.nbytes if training else 0, ctypes.c_void_p(room.data_ptr), given, current_stream())
+    assert (room.get() == 255).all() and not any(y.get().any() for y in ys + [hy, cy])
