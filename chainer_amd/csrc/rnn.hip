@@ -708,12 +708,62 @@ float* PackInputWeights(Pass& pass, const RnnPlan& pl, const hipcx_array* const*
     return packed;
 }
 
-// An array's data where it is dense, else of a dense copy (there is always room for one: the caller's strides are not known to a dry run).
-const float* Dense(Pass& pass, const hipcx_array* a) {
+// The bytes that an array spans.
+struct Span {
+    uintptr_t begin, end;
+    const hipcx_array* array;
+};
+Span SpanOf(const hipcx_array* a) {
+    Span s{reinterpret_cast<uintptr_t>(a->data), reinterpret_cast<uintptr_t>(a->data) + 4, a};
+    for (int i = 0; i < a->ndim; ++i) {
+        const int64_t reach = (a->shape[i] - 1) * a->strides[i];
+        (reach < 0 ? s.begin : s.end) += static_cast<uintptr_t>(reach);
+    }
+    return s;
+}
+
+// Whether two arrays may share memory.  Matrices of dense rows with the same distance, as the steps of one batch-major array are, interleave.
+bool MayShare(const Span& a, const Span& b) {
+    if (a.end <= b.begin || b.end <= a.begin) return false;
+    const hipcx_array &x = *a.array, &y = *b.array;
+    if (x.ndim != 2 || y.ndim != 2 || x.strides[1] != 4 || y.strides[1] != 4 || x.strides[0] != y.strides[0] || x.strides[0] <= 0) return true;
+    const int64_t pitch = x.strides[0];
+    int64_t r = static_cast<int64_t>(b.begin - a.begin) % pitch;
+    if (r < 0) r += pitch;
+    return r < x.shape[1] * 4 || pitch - r < y.shape[1] * 4;
+}
+
+// Whether any of `outs` may share memory with another one of them or with one of `ins`.
+bool AnyShared(const std::vector<const hipcx_array*>& outs, const std::vector<const hipcx_array*>& ins) {
+    std::vector<Span> to, from;
+    for (const hipcx_array* a : outs) to.push_back(SpanOf(a));
+    for (const hipcx_array* a : ins) from.push_back(SpanOf(a));
+    std::sort(to.begin(), to.end(), [](const Span& a, const Span& b) { return a.begin < b.begin; });
+    bool apart = true;  // mostly the spans are disjoint
+    for (size_t i = 1; i < to.size(); ++i) apart = apart && to[i - 1].end <= to[i].begin;
+    for (size_t i = 0; i < from.size() && apart; ++i) {
+        const auto behind = std::lower_bound(to.begin(), to.end(), from[i].end, [](const Span& a, uintptr_t end) { return a.begin < end; });
+        apart = behind == to.begin() || std::prev(behind)->end <= from[i].begin;
+    }
+    if (apart) return false;
+    for (size_t i = 0; i < to.size(); ++i) {
+        for (size_t j = 0; j < i; ++j) {
+            if (MayShare(to[i], to[j])) return true;
+        }
+        for (const Span& f : from) {
+            if (MayShare(to[i], f)) return true;
+        }
+    }
+    return false;
+}
+
+// An array's data where it is dense and need not be copied, else of a dense copy (there is always room for one: the caller's strides are not known to a
+// dry run).
+const float* Dense(Pass& pass, const hipcx_array* a, bool copied = false) {
     int64_t n = 1;
     for (int i = 0; i < a->ndim; ++i) n *= a->shape[i];
     float* const copy = pass.Take(n);
-    if (pass.dry() || IsContiguous(a)) return static_cast<const float*>(a->data);
+    if (pass.dry() || (!copied && IsContiguous(a))) return static_cast<const float*>(a->data);
     pass.Copy(*a, a->ndim == 1 ? Vector(copy, n) : Matrix(copy, a->shape[0], a->shape[1], a->shape[1]));
     return copy;
 }
@@ -832,22 +882,37 @@ void RunForward(Pass& pass, const RnnPlan& pl, int activation, const hipcx_array
     float* const h0 = pass.Take(chains * B * H);
     std::vector<float*> wx_packed;
     for (int idx = 0; idx < chains && !narrow; ++idx) wx_packed.push_back(PackInputWeights(pass, pl, ws, idx));
+    // The steps read what earlier ones left in hy, cy and ys, and the caller's inputs where they are.  Results that share memory with each other (one
+    // scratch array for every ys[t]) or with an input are kept here until the end.
+    float *const y_own = pass.Take(rows * DH), *const h_own = pass.Take(chains * B * H), *const c_own = pl.mode == kLstm ? pass.Take(chains * B * H) : nullptr;
     pass.StartScratch();
+    bool own = false;
+    if (!pass.dry()) {
+        std::vector<const hipcx_array*> outs{hy}, ins{hx};
+        outs.insert(outs.end(), ys, ys + pl.T);
+        ins.insert(ins.end(), xs, xs + pl.T);
+        ins.insert(ins.end(), ws, ws + chains * 2 * pl.G);
+        ins.insert(ins.end(), bs, bs + chains * 2 * pl.G);
+        if (pl.mode == kLstm) outs.push_back(cy), ins.push_back(cx);
+        own = AnyShared(outs, ins);
+    }
+    auto h_state = [&](int idx) { return own ? Matrix(h_own + idx * B * H, B, H, H) : StateSlice(hy, idx); };
+    auto c_state = [&](int idx) { return own ? Matrix(c_own + idx * B * H, B, H, H) : StateSlice(cy, idx); };
     // the steps read rows of xs where they are if their columns are dense; the products over all steps need them in one array
     bool x_in_place = narrow;
     for (int t = 0; t < pl.T; ++t) x_in_place = x_in_place && (xs[t]->strides[1] == 4 || pl.I == 1) && xs[t]->strides[0] % 4 == 0;
     for (int t = 0; t < pl.T && !x_in_place; ++t) pass.Copy(*xs[t], Matrix(x_all + pl.row_start[t] * pl.I, pl.bt[t], pl.I, pl.I));
     for (int idx = 0; idx < chains; ++idx) {
         pass.Copy(StateSlice(hx, idx), Matrix(h0 + idx * B * H, B, H, H));
-        pass.Copy(StateSlice(hx, idx), StateSlice(hy, idx));
-        if (pl.mode == kLstm) pass.Copy(StateSlice(cx, idx), StateSlice(cy, idx));
+        pass.Copy(StateSlice(hx, idx), h_state(idx));
+        if (pl.mode == kLstm) pass.Copy(StateSlice(cx, idx), c_state(idx));
     }
     pass.FlushCopies();
     // output rows of layer l at step t, direction d's columns, and their stride
     auto y_at = [&](int l, int d, int t, int64_t* stride) {
-        if (l + 1 < pl.L) {
+        if (l + 1 < pl.L || own) {
             *stride = DH;
-            return y_buf[l] + pl.row_start[t] * DH + d * H;
+            return (l + 1 < pl.L ? y_buf[l] : y_own) + pl.row_start[t] * DH + d * H;
         }
         *stride = ys[t]->strides[0] / 4;
         return static_cast<float*>(ys[t]->data) + d * H;
@@ -879,7 +944,7 @@ void RunForward(Pass& pass, const RnnPlan& pl, int activation, const hipcx_array
                 j.prev_rows = static_cast<int>(std::min(bt, pl.bt[before]));
                 j.h_prev = y_at(l, d, before, &j.h_prev_stride);
                 if (const int64_t back = std::min(bt, seen[idx]); back > j.prev_rows) {  // rows that an earlier step held and the last one did not
-                    const hipcx_array state = StateSlice(hy, idx);
+                    const hipcx_array state = h_state(idx);
                     hipcx_array from = state;
                     from.data = static_cast<char*>(state.data) + j.prev_rows * state.strides[0];
                     from.shape[0] = back - j.prev_rows;
@@ -892,10 +957,10 @@ void RunForward(Pass& pass, const RnnPlan& pl, int activation, const hipcx_array
                 j.bx[g] = bx[idx * pl.G + g], j.bh[g] = bh[idx * pl.G + g];
             }
             j.y = y_at(l, d, t, &j.y_stride);
-            const hipcx_array h_out = StateSlice(hy, idx);
+            const hipcx_array h_out = h_state(idx);
             j.hy = static_cast<float*>(h_out.data), j.hy_row = h_out.strides[0] / 4, j.hy_col = h_out.strides[1] / 4;
             if (pl.mode == kLstm) {
-                const hipcx_array c_out = StateSlice(cy, idx);
+                const hipcx_array c_out = c_state(idx);
                 j.cy = static_cast<float*>(c_out.data), j.cy_row = c_out.strides[0] / 4, j.cy_col = c_out.strides[1] / 4;
             }
             if (reserve != nullptr) {
@@ -927,6 +992,23 @@ void RunForward(Pass& pass, const RnnPlan& pl, int activation, const hipcx_array
             ForEachTurn(pl, false, l, l, launch);
         }
     }
+    if (own) {  // one after the other: the last step's outputs and then the states are what is left where they share memory
+        auto hand_out = [&](const hipcx_array& from, const hipcx_array& to) {
+            pass.Copy(from, to);
+            pass.FlushCopies();
+        };
+        for (int d = 0; d < pl.D; ++d) {
+            for (int s = 0; s < pl.T; ++s) {
+                const int t = d == 0 ? s : pl.T - 1 - s;
+                hand_out(Matrix(y_own + pl.row_start[t] * DH + d * H, pl.bt[t], H, DH),
+                         Matrix(static_cast<float*>(ys[t]->data) + d * H, pl.bt[t], H, ys[t]->strides[0] / 4));
+            }
+        }
+        for (int idx = 0; idx < chains; ++idx) {
+            hand_out(h_state(idx), StateSlice(hy, idx));
+            if (pl.mode == kLstm) hand_out(c_state(idx), StateSlice(cy, idx));
+        }
+    }
     pass.CheckFits();
 }
 
@@ -949,11 +1031,16 @@ void RunBackward(Pass& pass, const RnnPlan& pl, int activation, const hipcx_arra
     const int together = wavefront ? pl.L : pl.D;  // layer-directions that advance together
     const int subs = BackSubs(pl, wavefront), splits = pl.G * subs;
     const int64_t most_rows = *std::max_element(pl.bt.begin(), pl.bt.end());
+    bool shared = false;  // gradients of a layer that overwrite the matrices of one below
+    if (!pass.dry()) {
+        std::vector<const hipcx_array*> outs(dws, dws + chains * 2 * pl.G);
+        shared = AnyShared(outs, std::vector<const hipcx_array*>(ws, ws + chains * 2 * pl.G));
+    }
     std::vector<const float*> wx, wh;
     for (int idx = 0; idx < chains; ++idx) {
         for (int g = 0; g < 2 * pl.G; ++g) {
-            if (g >= pl.G) wh.push_back(Dense(pass, ws[idx * 2 * pl.G + g]));
-            else wx.push_back(wavefront && idx > 0 ? Dense(pass, ws[idx * 2 * pl.G + g]) : nullptr);
+            if (g >= pl.G) wh.push_back(Dense(pass, ws[idx * 2 * pl.G + g], shared));
+            else wx.push_back(wavefront && idx > 0 ? Dense(pass, ws[idx * 2 * pl.G + g], shared) : nullptr);
         }
     }
     std::vector<float*> wx_packed(chains, nullptr);  // for the gradients of a layer's input over all steps

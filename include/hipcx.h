@@ -393,7 +393,9 @@ int hipcx_n_step_lstm(int n_layers, const hipcx_array* hx, const hipcx_array* cx
  *   Backward (RnnBackwardKernel::Call's grad lists): dhy (dcy: LSTM, may be NULL = zeros), dys[t] [B_t, D * H] (an entry may be NULL =
  *   zeros) -> dhx (dcx), dws / dbs shaped and ordered like ws / bs (C-contiguous), dxs[t] [B_t, in].
  *   Equal to the routine composition / its autograd gradients to float32 tolerance (sums in another order).  One-direction LSTM
- *   inference runs hipcx_n_step_lstm. */
+ *   inference of many units or rows runs hipcx_n_step_lstm (its workspace and speed; the results are the same to that tolerance).
+ *   hy, cy and ys may share memory with each other and with the inputs (one scratch array for every ys[t], ys[t] = xs[t]): what is
+ *   left there is the outputs of the last step, then hy, then cy.  Results that do not are written as the steps run, which is faster. */
 size_t hipcx_n_step_rnn_reserve_size(int n_layers, int bidirectional, int mode, const hipcx_array* hx, const hipcx_array* const* xs, int n_steps);
 size_t hipcx_n_step_rnn_workspace_size(int n_layers, int bidirectional, int mode, int training, const hipcx_array* hx, const hipcx_array* const* xs,
                                        int n_steps);

@@ -171,3 +171,54 @@ def test_workspace_too_small(kind, training):
                       cy.desc() if kind == 'lstm' else None, routines._descriptor_pointers(ys), ctypes.c_void_p(reserve.data_ptr) if training else None,
                       reserve.nbytes if training else 0, ctypes.c_void_p(room.data_ptr), given, current_stream())
     assert (room.get() == 255).all() and not any(y.get().any() for y in ys + [hy, cy])
+
+
+@pytest.mark.parametrize('kind', ['lstm', 'gru', 'rnn'])
+@pytest.mark.parametrize('layers,bidirectional,units,lengths', [(1, False, 33, (4, 4, 2)), (3, False, 40, (5, 3, 3, 1)), (2, True, 34, (4, 2, 2)), (2, True, 300, (3,) * 40)])
+@pytest.mark.parametrize('training', [0, 1])
+def test_results_that_share_memory(kind, layers, bidirectional, units, lengths, training):
+    """One scratch array for every ys[t], ys[t] in place of xs[t], new states in place of the old ones: the states are right, and what is left in shared
+    memory is what was written last.  Steps of one batch-major array interleave without sharing any."""
+    import ctypes
+    import chainer_amd as chx
+    from chainer_amd import _lib, routines
+    from chainer_amd._array import current_stream
+    d, mode, lstm = 2 if bidirectional else 1, {'gru': 0, 'lstm': 1, 'rnn': 2}[kind], kind == 'lstm'
+    ws, bs, _, xs, h, c = _rnn_problem(np.random.default_rng(units), kind, layers, bidirectional, d * units, units, lengths)
+    W, B, X = [chx.array(m) for g in ws for m in g], [chx.array(v) for g in bs for v in g], [chx.array(x) for x in xs]
+    hx, cx = chx.array(h), chx.array(c)
+    (hy, cy), ys, _ = chx.rnn(layers, hx, cx if lstm else None, [W[i * len(ws[0]):][:len(ws[0])] for i in range(len(ws))],
+                              [B[i * len(bs[0]):][:len(bs[0])] for i in range(len(bs))], X, bidirectional, kind, training=bool(training))
+    hy, cy, ys = hy.get(), cy.get() if lstm else None, [y.get() for y in ys]
+    L, T, pointers = _lib.load(), len(X), routines._descriptor_pointers
+    px = pointers(X)
+    need = L.hipcx_n_step_rnn_workspace_size(layers, int(bidirectional), mode, training, hx.desc(), px, T)
+    room = chx.zeros((need,), np.uint8)
+    reserve = chx.zeros((L.hipcx_n_step_rnn_reserve_size(layers, int(bidirectional), mode, hx.desc(), px, T),), np.uint8) if training else None
+
+    def run(h_in, c_in, x_in, h_out, c_out, y_out):
+        _lib.call('hipcx_n_step_rnn', layers, int(bidirectional), mode, 0, h_in.desc(), c_in.desc() if lstm else None, pointers(W), pointers(B), pointers(x_in), T,
+                  h_out.desc(), c_out.desc() if lstm else None, pointers(y_out), ctypes.c_void_p(reserve.data_ptr) if training else None,
+                  reserve.nbytes if training else 0, ctypes.c_void_p(room.data_ptr), need, current_stream())
+        np.testing.assert_array_equal(h_out.get(), hy)
+        if lstm:
+            np.testing.assert_array_equal(c_out.get(), cy)
+
+    new = lambda: (chx.zeros(hx.shape, np.float32), chx.zeros(hx.shape, np.float32))
+    scratch = chx.zeros(ys[0].shape, np.float32)
+    run(hx, cx, X, *new(), [scratch[:len(y)] for y in ys])
+    last = ys[-1][:, :units]  # the first direction's last step, and the second one's, which ends with step 0
+    np.testing.assert_array_equal(scratch.get()[:len(last), :units], last)
+    if bidirectional:
+        np.testing.assert_array_equal(scratch.get()[:, units:], ys[0][:, units:])
+    in_place = [x.copy() for x in X]
+    run(hx, cx, in_place, *new(), in_place)
+    for y, r in zip(in_place, ys):
+        np.testing.assert_array_equal(y.get(), r)
+    h2, c2 = hx.copy(), cx.copy()
+    run(h2, c2, X, h2, c2, [chx.zeros(y.shape, np.float32) for y in ys])
+    batch_major = chx.zeros((ys[0].shape[0], T, d * units), np.float32)
+    interleaved = [batch_major[:len(y), t] for t, y in enumerate(ys)]
+    run(hx, cx, X, *new(), interleaved)
+    for y, r in zip(interleaved, ys):
+        np.testing.assert_array_equal(y.get(), r)
