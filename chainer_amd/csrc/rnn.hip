@@ -9,6 +9,7 @@
 // steps from the last to the first on its own state.
 //   * Small launches take the products with the layer's input along; else they are one product  XW = X_all [rows, in] . Wx^T  over the rows of
 //     all steps of a layer (rows = sum of the steps' batch sizes).
+//   * Large steps are a library product  h . Wh^T  and a launch of cells (Wide); so are their gradients.
 //   * The state before a step is the output of the step before, where it lies; hy and cy are updated in place.
 //   * The outputs go to columns [d*H, (d+1)*H) of the layer's output rows, which are the next layer's input (the Concatenate of
 //     :398-404), or to the caller's ys[t] for the top layer.
@@ -84,6 +85,28 @@ __device__ __forceinline__ void KeepRun(Bytes16& v, int k, int K) {
     const int at = RunStart(k, K);
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[e] = (at + e >= k) & (at + e < K) ? v[e] : 0u;
+}
+
+// One unit of one row: x and h are the two sides' pre-activations with their biases (Linear(x), Linear(h)).  Returns the new state; `gates`, if not null, is
+// where its saved values go, H apart.
+template <int MODE, int G>
+__device__ __forceinline__ float RunCell(const float (&x)[G], const float (&h)[G], float h_old, float c_old, bool relu, float* gates, int H, float& c_new) {
+    auto pre = [&](int g) { return x[g] + h[g]; };
+    if constexpr (MODE == kLstm) {
+        const float gi = Sigmoid(pre(0)), gf = Sigmoid(pre(1)), gg = tanhf(pre(2)), go = Sigmoid(pre(3));
+        c_new = gg * gi + gf * c_old;
+        if (gates != nullptr) gates[0] = gi, gates[H] = gf, gates[2 * H] = gg, gates[3 * H] = go;
+        return go * tanhf(c_new);
+    } else if constexpr (MODE == kGru) {
+        const float gr = Sigmoid(pre(0)), gz = Sigmoid(pre(1));
+        const float gn = tanhf(x[2] + gr * h[2]);
+        if (gates != nullptr) gates[0] = gr, gates[H] = gz, gates[2 * H] = gn, gates[3 * H] = h[2];
+        return (1.0f - gz) * gn + gz * h_old;
+    } else {
+        const float h_new = relu ? fmaxf(pre(0), 0.0f) : tanhf(pre(0));
+        if (gates != nullptr) *gates = h_new;
+        return h_new;
+    }
 }
 
 // One step of one layer-direction.  Matrices are dense [units][columns], vectors dense.
@@ -279,40 +302,73 @@ __global__ __launch_bounds__(64 * kStepWaves) void RnnStepKernel(StepArgs p) {
 #pragma unroll
                 for (int w = 0; w < kStepWaves; ++w) sum[s][g] += part[(s * kStepWaves + w) * kPartFloats + at + g];
             }
-        if constexpr (MODE == kGru) {
-#pragma unroll
-            for (int g = 0; g < G; ++g) xw[i][g] += sum[0][g];
-        }
         const int64_t idx = static_cast<int64_t>(r) * H + u;
-        auto pre = [&](int g) { return (xw[i][g] + b_x[i][g]) + (sum[SIDES - 1][g] + b_h[i][g]); };  // Linear(x) + Linear(h)
-        float h_new;
+        float from_x[G], from_h[G], c_new = 0.f;
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            from_x[g] = (MODE == kGru ? xw[i][g] + sum[0][g] : xw[i][g]) + b_x[i][g];
+            from_h[g] = sum[SIDES - 1][g] + b_h[i][g];
+        }
+        float* const saved = gates != nullptr ? gates + (static_cast<int64_t>(r) * (G == 1 ? 1 : 4) * H + u) : nullptr;
+        const float h_new = RunCell<MODE, G>(from_x, from_h, h_old[i], c_old[i], p.relu != 0, saved, H, c_new);
         if constexpr (MODE == kLstm) {
-            const float gi = Sigmoid(pre(0)), gf = Sigmoid(pre(1)), gg = tanhf(pre(2)), go = Sigmoid(pre(3));
-            const float c_new = gg * gi + gf * c_old[i];
-            h_new = go * tanhf(c_new);
             cy[r * cy_row + u * cy_col] = c_new;
-            if (gates != nullptr) {
-                float* q = gates + static_cast<int64_t>(r) * 4 * H + u;
-                q[0] = gi, q[H] = gf, q[2 * H] = gg, q[3 * H] = go;
-                cprev[idx] = c_old[i];
-            }
-        } else if constexpr (MODE == kGru) {
-            const float gr = Sigmoid(pre(0)), gz = Sigmoid(pre(1));
-            const float hh = sum[SIDES - 1][2] + b_h[i][2];
-            const float gn = tanhf((xw[i][2] + b_x[i][2]) + gr * hh);
-            h_new = (1.0f - gz) * gn + gz * h_old[i];
-            if (gates != nullptr) {
-                float* q = gates + static_cast<int64_t>(r) * 4 * H + u;
-                q[0] = gr, q[H] = gz, q[2 * H] = gn, q[3 * H] = hh;
-            }
-        } else {
-            const float s = pre(0);
-            h_new = p.relu ? fmaxf(s, 0.0f) : tanhf(s);
-            if (gates != nullptr) gates[idx] = h_new;
+            if (gates != nullptr) cprev[idx] = c_old[i];
         }
         if (gates != nullptr) hprev[idx] = h_old[i];
         hy[r * hy_row + u * hy_col] = h_new;
         y[r * y_stride + u] = h_new;
+    }
+}
+
+// The cells of a step whose products are in memory, [bt][G*H]; states [B][H] are updated in place.
+struct CellJob {
+    int bt;
+    const float* xw;
+    const float* hw;
+    const float* bx[4];
+    const float* bh[4];
+    float* h;
+    float* c;  // (LSTM)
+    int64_t c_row, c_col;
+    float* y;
+    int64_t y_stride;
+    float* gates;  // as in StepJob
+    float* hprev;
+    float* cprev;
+};
+
+struct CellArgs {
+    int relu;
+    int H;
+    CellJob job[2];
+};
+
+template <int MODE>
+__global__ __launch_bounds__(256) void RnnCellKernel(CellArgs p) {
+    constexpr int G = MODE == kLstm ? 4 : (MODE == kGru ? 3 : 1);
+    const CellJob& j = p.job[blockIdx.y];
+    const int H = p.H, total = j.bt * H;
+    for (int idx = blockIdx.x * 256 + threadIdx.x; idx < total; idx += gridDim.x * 256) {
+        const int r = idx / H, u = idx - r * H;
+        float from_x[G], from_h[G], c_old = 0.f, c_new = 0.f;
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            const int64_t at = (static_cast<int64_t>(r) * G + g) * H + u;
+            from_x[g] = j.xw[at] + j.bx[g][u];
+            from_h[g] = j.hw[at] + j.bh[g][u];
+        }
+        const float h_old = j.h[idx];
+        if constexpr (MODE == kLstm) c_old = j.c[r * j.c_row + u * j.c_col];
+        float* const saved = j.gates != nullptr ? j.gates + (static_cast<int64_t>(r) * (G == 1 ? 1 : 4) * H + u) : nullptr;
+        const float h_new = RunCell<MODE, G>(from_x, from_h, h_old, c_old, p.relu != 0, saved, H, c_new);
+        if constexpr (MODE == kLstm) j.c[r * j.c_row + u * j.c_col] = c_new;
+        if (j.gates != nullptr) {
+            j.hprev[idx] = h_old;
+            if constexpr (MODE == kLstm) j.cprev[idx] = c_old;
+        }
+        j.h[idx] = h_new;
+        j.y[static_cast<int64_t>(r) * j.y_stride + u] = h_new;
     }
 }
 
@@ -699,12 +755,13 @@ private:
     std::vector<hipcx_array> copies_;
 };
 
-// The x-side matrices of a layer-direction stacked gate-major into [G*H][in]: rows [g*H, (g+1)*H) are ws[idx][g].
-float* PackInputWeights(Pass& pass, const RnnPlan& pl, const hipcx_array* const* ws, int idx) {
-    const int64_t in = pl.In(idx / pl.D);
-    float* const packed = pass.Take(pl.G * pl.H * in);
+// The matrices of a layer-direction's x side (first = 0) or h side (first = G) stacked gate-major into [G*H][columns]: rows [g*H, (g+1)*H) are
+// ws[idx][first + g].
+float* PackWeights(Pass& pass, const RnnPlan& pl, const hipcx_array* const* ws, int idx, int first) {
+    const int64_t columns = first == 0 ? pl.In(idx / pl.D) : pl.H;
+    float* const packed = pass.Take(pl.G * pl.H * columns);
     if (pass.dry()) return packed;
-    for (int g = 0; g < pl.G; ++g) pass.Copy(*ws[idx * 2 * pl.G + g], Matrix(packed + g * pl.H * in, pl.H, in, in));
+    for (int g = 0; g < pl.G; ++g) pass.Copy(*ws[idx * 2 * pl.G + first + g], Matrix(packed + g * pl.H * columns, pl.H, columns, columns));
     return packed;
 }
 
@@ -831,6 +888,18 @@ bool Narrow(const RnnPlan& pl) {
     return jobs <= kMaxJobs && rows * ((pl.H + units - 1) / units) * jobs <= most;
 }
 
+// Whether a step's products are library calls (on the bfloat16 pipes, in tiles of 128 x 128, where they are large), the x side's over all steps, with a
+// launch for the cells: from 1 G multiply-adds of the h side on, for GRU, whose steps work for a fourth gate, from 0.3.  Not for layers that run as a
+// wavefront.  us, forward and backward of 6 steps with as many inputs as units, one layer, steps and library calls:
+//   GRU  512 rows, 512 units  247 + 400, 177 + 373    LSTM  256 rows, 1024 units  364 + 626, 313 + 604    RNN 1024 rows, 1024 units 418 + 694, 337 + 697
+//        256,     1024        384 + 576, 277 + 539          1024,     512        378 + 741, 367 + 682         512,      2048       647 + 1053, 556 + 1027
+//        128,     2048        636 + 938, 463 + 931          1024,     1024     1178 + 2010, 850 + 1911
+//   and around the lines: GRU 256, 512 133 + 242, 127 + 246; LSTM 384, 768 308 + 691, 294 + 741; RNN 128, 2048 193 + 389, 215 + 367.
+bool Wide(const RnnPlan& pl) {
+    const double work = static_cast<double>(*std::max_element(pl.bt.begin(), pl.bt.end())) * pl.G * pl.H * pl.H;
+    return work >= (pl.mode == kGru ? 3e8 : 1e9) && (pl.L * pl.D == 1 || !Narrow(pl));
+}
+
 // f(jobs), for each launch of a pass: the (layer, direction, step) that it runs.  A direction's step s is time step s or T - 1 - s.
 struct Turn {
     int layer, direction, s;
@@ -861,11 +930,12 @@ void RunForward(Pass& pass, const RnnPlan& pl, int activation, const hipcx_array
                 const hipcx_array* const* ys, char* reserve) {
     const int64_t B = pl.B, H = pl.H, GH = pl.G * H, DH = pl.D * H, rows = pl.rows;
     const int chains = pl.L * pl.D;
-    const bool narrow = Narrow(pl), wavefront = narrow && pl.D == 1;
-    std::vector<const float*> wx, wh, bx, bh;
+    const bool wide = Wide(pl), narrow = Narrow(pl) && !wide, wavefront = narrow && pl.D == 1;
+    std::vector<const float*> wx, wh, bx, bh;  // (the steps read the x side's matrices of narrow networks only, and none of wide ones)
     for (int idx = 0; idx < chains; ++idx) {
         for (int g = 0; g < 2 * pl.G; ++g) {
-            (g < pl.G ? wx : wh).push_back(Dense(pass, ws[idx * 2 * pl.G + g]));
+            const bool read = g < pl.G ? narrow : !wide;
+            (g < pl.G ? wx : wh).push_back(read ? Dense(pass, ws[idx * 2 * pl.G + g]) : nullptr);
             (g < pl.G ? bx : bh).push_back(Dense(pass, bs[idx * 2 * pl.G + g]));
         }
     }
@@ -880,8 +950,11 @@ void RunForward(Pass& pass, const RnnPlan& pl, int activation, const hipcx_array
         for (int d = 0; d < pl.D; ++d) xw_all[d] = pass.Take(rows * GH);
     }
     float* const h0 = pass.Take(chains * B * H);
-    std::vector<float*> wx_packed;
-    for (int idx = 0; idx < chains && !narrow; ++idx) wx_packed.push_back(PackInputWeights(pass, pl, ws, idx));
+    std::vector<float*> wx_packed, wh_packed;
+    for (int idx = 0; idx < chains && !narrow; ++idx) wx_packed.push_back(PackWeights(pass, pl, ws, idx, 0));
+    for (int idx = 0; idx < chains && wide; ++idx) wh_packed.push_back(PackWeights(pass, pl, ws, idx, pl.G));
+    float* hw[2] = {nullptr, nullptr};
+    for (int d = 0; d < pl.D && wide; ++d) hw[d] = pass.Take(*std::max_element(pl.bt.begin(), pl.bt.end()) * GH);
     // The steps read what earlier ones left in hy, cy and ys, and the caller's inputs where they are.  Results that share memory with each other (one
     // scratch array for every ys[t]) or with an input are kept here until the end.
     float *const y_own = pass.Take(rows * DH), *const h_own = pass.Take(chains * B * H), *const c_own = pl.mode == kLstm ? pass.Take(chains * B * H) : nullptr;
@@ -979,6 +1052,40 @@ void RunForward(Pass& pass, const RnnPlan& pl, int activation, const hipcx_array
         });
         CheckLaunch("rnn_step");
     };
+    // the same for wide networks, whose states are in h0 until the end
+    auto launch_wide = [&](const std::vector<Turn>& turns) {
+        CellArgs a{};
+        a.relu = activation == 1;
+        a.H = static_cast<int>(H);
+        int64_t most = 0;
+        for (size_t i = 0; i < turns.size(); ++i) {
+            const int l = turns[i].layer, d = turns[i].direction, s = turns[i].s, idx = l * pl.D + d;
+            const int t = d == 0 ? s : pl.T - 1 - s;
+            const int64_t bt = pl.bt[t], r0 = pl.row_start[t];
+            pass.Dot(Matrix(h0 + idx * B * H, bt, H, H), Matrix(wh_packed[idx], H, GH, 1, H), Matrix(hw[d], bt, GH, GH));
+            CellJob& j = a.job[i];
+            j.bt = static_cast<int>(bt);
+            j.xw = xw_all[d] + r0 * GH, j.hw = hw[d];
+            for (int g = 0; g < pl.G; ++g) j.bx[g] = bx[idx * pl.G + g], j.bh[g] = bh[idx * pl.G + g];
+            j.h = h0 + idx * B * H;
+            if (pl.mode == kLstm) {
+                const hipcx_array c_out = c_state(idx);
+                j.c = static_cast<float*>(c_out.data), j.c_row = c_out.strides[0] / 4, j.c_col = c_out.strides[1] / 4;
+            }
+            j.y = y_at(l, d, t, &j.y_stride);
+            if (reserve != nullptr) {
+                j.gates = reinterpret_cast<float*>(reserve + pl.r_gates[idx]) + r0 * pl.GR * H;
+                j.hprev = reinterpret_cast<float*>(reserve + pl.r_hprev[idx]) + r0 * H;
+                j.cprev = pl.mode == kLstm ? reinterpret_cast<float*>(reserve + pl.r_cprev[idx]) + r0 * H : nullptr;
+            }
+            most = std::max(most, bt * H);
+        }
+        if (pass.dry()) return;
+        VisitMode(pl.mode, [&](auto mode) {
+            hipLaunchKernelGGL(RnnCellKernel<decltype(mode)::value>, dim3(CellBlocks(most), static_cast<unsigned>(turns.size())), dim3(256), 0, pass.hip_stream(), a);
+        });
+        CheckLaunch("rnn_cell");
+    };
     if (narrow) {
         ForEachTurn(pl, wavefront, 0, pl.L - 1, launch);
     } else {
@@ -989,8 +1096,13 @@ void RunForward(Pass& pass, const RnnPlan& pl, int activation, const hipcx_array
             for (int d = 0; d < pl.D; ++d) {
                 pass.Dot(Matrix(x_in, rows, in, in), Matrix(wx_packed[l * pl.D + d], in, GH, 1, in), Matrix(xw_all[d], rows, GH, GH));
             }
-            ForEachTurn(pl, false, l, l, launch);
+            if (wide) ForEachTurn(pl, false, l, l, launch_wide);
+            else ForEachTurn(pl, false, l, l, launch);
         }
+    }
+    if (wide) {
+        for (int idx = 0; idx < chains; ++idx) pass.Copy(Matrix(h0 + idx * B * H, B, H, H), h_state(idx));
+        pass.FlushCopies();
     }
     if (own) {  // one after the other: the last step's outputs and then the states are what is left where they share memory
         auto hand_out = [&](const hipcx_array& from, const hipcx_array& to) {
@@ -1027,9 +1139,9 @@ void RunBackward(Pass& pass, const RnnPlan& pl, int activation, const hipcx_arra
                  const hipcx_array* const* dxs) {
     const int64_t B = pl.B, H = pl.H, GH = pl.G * H, DH = pl.D * H, rows = pl.rows;
     const int chains = pl.L * pl.D;
-    const bool wavefront = Narrow(pl) && pl.D == 1;
+    const bool wide = Wide(pl), wavefront = Narrow(pl) && pl.D == 1 && !wide;
     const int together = wavefront ? pl.L : pl.D;  // layer-directions that advance together
-    const int subs = BackSubs(pl, wavefront), splits = pl.G * subs;
+    const int subs = BackSubs(pl, wavefront), splits = wide ? 1 : pl.G * subs;
     const int64_t most_rows = *std::max_element(pl.bt.begin(), pl.bt.end());
     bool shared = false;  // gradients of a layer that overwrite the matrices of one below
     if (!pass.dry()) {
@@ -1039,14 +1151,16 @@ void RunBackward(Pass& pass, const RnnPlan& pl, int activation, const hipcx_arra
     std::vector<const float*> wx, wh;
     for (int idx = 0; idx < chains; ++idx) {
         for (int g = 0; g < 2 * pl.G; ++g) {
-            if (g >= pl.G) wh.push_back(Dense(pass, ws[idx * 2 * pl.G + g], shared));
+            if (g >= pl.G) wh.push_back(wide ? nullptr : Dense(pass, ws[idx * 2 * pl.G + g], shared));
             else wx.push_back(wavefront && idx > 0 ? Dense(pass, ws[idx * 2 * pl.G + g], shared) : nullptr);
         }
     }
     std::vector<float*> wx_packed(chains, nullptr);  // for the gradients of a layer's input over all steps
     for (int idx = 0; idx < chains; ++idx) {
-        if (!wavefront || idx == 0) wx_packed[idx] = PackInputWeights(pass, pl, ws, idx);
+        if (!wavefront || idx == 0) wx_packed[idx] = PackWeights(pass, pl, ws, idx, 0);
     }
+    std::vector<float*> wh_packed;
+    for (int idx = 0; idx < chains && wide; ++idx) wh_packed.push_back(PackWeights(pass, pl, ws, idx, pl.G));
     float* x_all = pass.Take(rows * pl.I);
     float* dy_cur = pass.Take(rows * pl.max_in);   // gradient of the current layer's output rows [rows][D*H]
     float* dx_acc = pass.Take(rows * pl.max_in);   // gradient of its input rows [rows][in]
@@ -1130,7 +1244,11 @@ void RunBackward(Pass& pass, const RnnPlan& pl, int activation, const hipcx_arra
             most = std::max(most, (bt + 31) / 32 * ((H + 31) / 32 + (q.in + 31) / 32) * splits);
         }
         launch_cells(a, turns.size());
-        if (pass.dry()) return;
+        for (size_t n = 0; n < turns.size() && wide; ++n) {
+            const BackJob& q = b.job[n];
+            pass.Dot(Matrix(q.dgh, q.bt, GH, GH), Matrix(wh_packed[turns[n].layer * pl.D + turns[n].direction], GH, H, H), Matrix(q.dh_parts, q.bt, H, H));
+        }
+        if (pass.dry() || wide) return;
         hipLaunchKernelGGL(RnnBackKernel, dim3(static_cast<unsigned>(most), static_cast<unsigned>(turns.size())), dim3(64 * kStepWaves), 0,
                            pass.hip_stream(), b);
         CheckLaunch("rnn_back");

@@ -50,6 +50,11 @@ def _layer(kind, w, b, xs, h, c, reverse):
     ('gru', 5, False, 16, 24, (4, 4, 1)),
     ('rnn', 3, False, 40, 65, (65, 64, 3)),
     ('rnn', 2, True, 7, 33, (2, 2)),
+    ('gru', 1, False, 20, 513, (385, 384, 31)),           # steps whose products are library calls
+    ('gru', 2, True, 33, 512, (390, 385, 390)),
+    ('lstm', 1, False, 65, 520, (930, 929, 17)),
+    ('lstm', 2, True, 16, 510, (970, 961)),
+    ('rnn', 1, False, 30, 1030, (950, 945)),
 ])
 def test_against_autograd(kind, layers, bidirectional, in_size, units, batches):
     import chainer_amd as chx
