@@ -68,8 +68,8 @@ void LaunchShape(IGemmArgs<T> p, bool fast16, bool fast8, hipStream_t stream) {
     // wide products: a row of concurrent tiles would read more second-operand panels than an XCD's L2 holds
     static const int band_env = [] { const char* e = getenv("HIPCX_IGEMM_BAND"); return e != nullptr ? atoi(e) : 8; }();
     p.band = p.tiles_n > 16 ? band_env : 0;
-    static const bool pipe_env = [] { const char* e = getenv("HIPCX_IGEMM_PIPE"); return e != nullptr && e[0] == '1'; }();
-    if (PM || pipe_env || !(fast16 || fast8) || p.partial == nullptr) p.ksplit = 1;  // only the simple fast kernel splits the reduction
+    static const bool use_pipe = [] { const char* e = getenv("HIPCX_IGEMM_PIPE"); return e != nullptr && e[0] == '1'; }();
+    if (PM || use_pipe || !(fast16 || fast8) || p.partial == nullptr) p.ksplit = 1;  // only the simple fast kernel splits the reduction
     dim3 grid(per * 8, 1), block(64 * WM * WN);
     if (p.ksplit > 1 && total > 65535) p.ksplit = 1;  // never planned for that many tiles; the grid's y extent could not hold them
     if (p.ksplit > 1) grid = dim3(p.ksplit, static_cast<unsigned>(total));  // slices along x: see IGemmFastKernel
@@ -81,7 +81,8 @@ void LaunchShape(IGemmArgs<T> p, bool fast16, bool fast8, hipStream_t stream) {
     // the pipelined kernel indexes x and w with 32-bit element offsets
     double x_elems = static_cast<double>(p.N) * (p.xsN > 0 ? p.xsN : 1);
     bool fits32 = x_elems < 2147483647.0 && static_cast<double>(p.K) * p.wsK < 2147483647.0;
-    static const bool use_pipe = [] { const char* e = getenv("HIPCX_IGEMM_PIPE"); return e != nullptr && e[0] == '1'; }();
+    HIPCX_REQUIRE(p.batch == 0 || ((fast16 || fast8) && !PM), HIPCX_NOT_IMPLEMENTED_ERROR, "batched products need operands in the MFMA layout");
+    const bool pipe = (fast16 || fast8) && fits32 && use_pipe && p.batch == 0;
     // float32 on the bfloat16 pipes wherever its layout allows.  us, float pipe and these, and the relative errors (2-norm) against 64 bits:
     //   [4480,650] . [650,10000]   600 and 400, 4.56e-7 and 1.45e-7     3x3 convolutions of 256 images:
     //   [4480,10000] . [10000,650] 711 and 480, 1.03e-6 and 4.4e-7        64 -> 64 at 32^2   226 and 173, 4.26e-7 and 1.35e-7
@@ -91,9 +92,8 @@ void LaunchShape(IGemmArgs<T> p, bool fast16, bool fast8, hipStream_t stream) {
     // With operands below 2^-110 in every tile, whose rows are read once more, the first four take 528, 591, 973 and 149.
     static const bool use_split = [] { const char* e = getenv("HIPCX_IGEMM_SPLIT"); return e == nullptr || e[0] != '0'; }();
     bool split = false;
-    if constexpr (sizeof(T) == 4) split = use_split && (fast16 || fast8) && IGemmSplit<WM, WN>(p, fast16 ? 16 : 8, PM, grid, stream);
-    HIPCX_REQUIRE(p.batch == 0 || ((fast16 || fast8) && !PM), HIPCX_NOT_IMPLEMENTED_ERROR, "batched products need operands in the MFMA layout");
-    if ((fast16 || fast8) && fits32 && use_pipe && p.batch == 0) {
+    if constexpr (sizeof(T) == 4) split = use_split && !pipe && (fast16 || fast8) && IGemmSplit<WM, WN>(p, fast16 ? 16 : 8, PM, grid, stream);
+    if (pipe) {
         constexpr int lds_bytes = PipeLdsBytes<T, WM, WN, PM>();
         if (fast16) {
             auto kern = IGemmPipeKernel<T, WM, WN, 16, PM>;
