@@ -559,9 +559,25 @@ __global__ __launch_bounds__(256) void NchwRepackFiltersKernel(const half_t* w, 
     *reinterpret_cast<G*>(wp + idx * 8) = grp;
 }
 
+// The extents of a convolution that PlanNchw took.
+NchwConvArgs NchwExtents(const hipcx_array* x, const hipcx_array* w, const hipcx_array* out, const int64_t* stride) {
+    NchwConvArgs a{};
+    a.N = static_cast<int>(x->shape[0]);
+    a.C = static_cast<int>(x->shape[1]);
+    a.H = static_cast<int>(x->shape[2]);
+    a.W = static_cast<int>(x->shape[3]);
+    a.K = static_cast<int>(w->shape[0]);
+    a.OH = static_cast<int>(out->shape[2]);
+    a.OW = static_cast<int>(out->shape[3]);
+    a.stride = static_cast<int>(stride[0]);
+    a.P = a.OH * a.OW;
+    a.M = a.N * a.P;
+    return a;
+}
+
 void RunNchw(const hipcx_array* x, const hipcx_array* w, const hipcx_array* b, const NchwPlan& pl, const int64_t* stride,
              const hipcx_array* out, char* workspace, hipStream_t stream, const FusedTail& tail = FusedTail{}) {
-    NchwConvArgs a{};
+    NchwConvArgs a = NchwExtents(x, w, out, stride);
     a.bn_gamma = tail.gamma;
     a.bn_beta = tail.beta;
     a.bn_mean = tail.mean;
@@ -575,16 +591,6 @@ void RunNchw(const hipcx_array* x, const hipcx_array* w, const hipcx_array* b, c
     a.bias = b ? static_cast<const half_t*>(b->data) : nullptr;
     a.bias_stride = b ? b->strides[0] / 2 : 0;
     a.out = static_cast<half_t*>(out->data);
-    a.N = static_cast<int>(x->shape[0]);
-    a.C = static_cast<int>(x->shape[1]);
-    a.H = static_cast<int>(x->shape[2]);
-    a.W = static_cast<int>(x->shape[3]);
-    a.K = static_cast<int>(w->shape[0]);
-    a.OH = static_cast<int>(out->shape[2]);
-    a.OW = static_cast<int>(out->shape[3]);
-    a.stride = static_cast<int>(stride[0]);
-    a.P = a.OH * a.OW;
-    a.M = a.N * a.P;
     const int BM = 64 * pl.wpx, BN = 64 * pl.wch;
     a.tiles_m = (a.M + BM - 1) / BM;
     a.tiles_n = (a.K + BN - 1) / BN;
@@ -1117,9 +1123,9 @@ int hipcx_conv_route(const hipcx_array* x, const hipcx_array* w, const hipcx_arr
         if (x == nullptr || w == nullptr || out == nullptr || stride == nullptr || pad == nullptr) return -1;
         if (x->ndim != 4 || w->ndim != 4 || out->ndim != 4) return -1;
         if (PlanPw(x, w, b, out, stride, pad).ok) return 3;
-        if (PlanNchw(x, w, out, stride, pad).ok) return 1;
+        if (const NchwPlan pl = PlanNchw(x, w, out, stride, pad); pl.ok) return SmallConvTakes(NchwExtents(x, w, out, stride), pl.taps) ? 4 : 1;
         if (PlanStem(x, w, out, stride, pad).ok) return 2;
-        return 0;
+        return ThinConvTakes(x, w, stride, pad, out) ? 5 : 0;
     } catch (...) {
         return -1;
     }
@@ -1162,9 +1168,11 @@ int hipcx_conv(const hipcx_array* x, const hipcx_array* w, const hipcx_array* b,
         }
         char* ws = static_cast<char*>(workspace);
         if (out->dtype == HIPCX_FLOAT16) {
-            if (!TryThinConv(x, w, b, stride, pad, out, st)) RunConv<half_t>(x, w, b, pl, out, ws, st);
+            if (ThinConvTakes(x, w, stride, pad, out)) ThinConv(x, w, b, stride, pad, out, st);
+            else RunConv<half_t>(x, w, b, pl, out, ws, st);
         } else if (out->dtype == HIPCX_FLOAT32) {
-            if (!TryThinConv(x, w, b, stride, pad, out, st)) RunConv<float>(x, w, b, pl, out, ws, st);
+            if (ThinConvTakes(x, w, stride, pad, out)) ThinConv(x, w, b, stride, pad, out, st);
+            else RunConv<float>(x, w, b, pl, out, ws, st);
         } else {
             RunConv<double>(x, w, b, pl, out, ws, st);
         }

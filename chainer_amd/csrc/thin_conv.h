@@ -5,7 +5,9 @@
 
 namespace hipcx {
 
-// Runs the convolution if it is one of those: dense NCHW arrays, channels x filter of at most 32 terms.
-bool TryThinConv(const hipcx_array* x, const hipcx_array* w, const hipcx_array* b, const int64_t* stride, const int64_t* pad, const hipcx_array* out, hipStream_t stream);
+// Whether the convolution is one of those: dense NCHW arrays, channels x filter of at most 32 terms.
+bool ThinConvTakes(const hipcx_array* x, const hipcx_array* w, const int64_t* stride, const int64_t* pad, const hipcx_array* out);
+
+void ThinConv(const hipcx_array* x, const hipcx_array* w, const hipcx_array* b, const int64_t* stride, const int64_t* pad, const hipcx_array* out, hipStream_t stream);
 
 }  // namespace hipcx

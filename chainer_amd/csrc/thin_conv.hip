@@ -113,7 +113,7 @@ __global__ __launch_bounds__(256, 3) void ThinConvKernel(ThinConvArgs p) {
 
 }  // namespace
 
-bool TryThinConv(const hipcx_array* x, const hipcx_array* w, const hipcx_array* b, const int64_t* stride, const int64_t* pad, const hipcx_array* out, hipStream_t stream) {
+bool ThinConvTakes(const hipcx_array* x, const hipcx_array* w, const int64_t* stride, const int64_t* pad, const hipcx_array* out) {
     if ((out->dtype != HIPCX_FLOAT32 && out->dtype != HIPCX_FLOAT16) || !IsContiguous(x) || !IsContiguous(w) || !IsContiguous(out)) return false;
     const int64_t N = x->shape[0], C = x->shape[1], H = x->shape[2], W = x->shape[3], K = w->shape[0], R = w->shape[2], S = w->shape[3];
     const int64_t OH = out->shape[2], OW = out->shape[3], P = OH * OW, terms = C * R * S;
@@ -123,7 +123,12 @@ bool TryThinConv(const hipcx_array* x, const hipcx_array* w, const hipcx_array* 
     const double limit = 2147483000.0 / 4;
     if (static_cast<double>(N) * C * H * W >= limit || static_cast<double>(N) * (K + 64) * P >= limit || static_cast<double>(K) * terms >= limit) return false;
     if (H >= 0x4000 || W >= 0x4000 || OH >= 0x4000 || OW >= 0x4000 || stride[0] >= 0x4000 || stride[1] >= 0x4000 || pad[0] >= 0x4000 || pad[1] >= 0x4000) return false;
-    if (OH * stride[0] >= 0x3000 || OW * stride[1] >= 0x3000) return false;
+    return OH * stride[0] < 0x3000 && OW * stride[1] < 0x3000;
+}
+
+void ThinConv(const hipcx_array* x, const hipcx_array* w, const hipcx_array* b, const int64_t* stride, const int64_t* pad, const hipcx_array* out, hipStream_t stream) {
+    const int64_t N = x->shape[0], C = x->shape[1], H = x->shape[2], W = x->shape[3], K = w->shape[0], R = w->shape[2], S = w->shape[3];
+    const int64_t OH = out->shape[2], OW = out->shape[3], P = OH * OW, terms = C * R * S;
     ThinConvArgs p{};
     const int64_t it = ItemSize(out->dtype);
     p.x = x->data, p.w = w->data, p.out = out->data;
@@ -148,7 +153,6 @@ bool TryThinConv(const hipcx_array* x, const hipcx_array* w, const hipcx_array* 
     if (out->dtype == HIPCX_FLOAT16) launch(half_t{});
     else launch(float{});
     CheckLaunch("thin_conv");
-    return true;
 }
 
 }  // namespace hipcx

@@ -13,7 +13,8 @@ _CASES = [  # images, channels, height, width, filters, kernel, stride
     (1, 32, 7, 7, 64, 1, 1), (2, 96, 5, 3, 33, 1, 1), (1, 544, 14, 14, 40, 1, 1), (3, 64, 1, 1, 70, 1, 1), (1, 64, 9, 12, 100, 1, 2),
     (2, 32, 13, 8, 31, 1, 3), (1, 1024, 2, 2, 256, 1, 1), (1, 64, 30, 31, 128, 1, 1),
     (1, 16, 7, 7, 32, 3, 1), (2, 48, 14, 14, 33, 3, 1), (1, 144, 9, 5, 65, 3, 1), (3, 32, 2, 2, 40, 3, 1), (1, 64, 56, 56, 64, 3, 1),
-    (1, 32, 3, 62, 20, 3, 1), (1, 16, 40, 6, 16, 3, 1), (2, 512, 7, 7, 64, 3, 1), (1, 256, 1, 33, 8, 3, 1),
+    (1, 32, 3, 62, 20, 3, 1), (1, 16, 40, 6, 16, 3, 1), (2, 512, 7, 7, 64, 3, 1), (1, 256, 1, 34, 8, 3, 1),
+    (1, 256, 1, 33, 8, 3, 1),  # (beyond what the NCHW kernels plan for: the general kernel)
 ]
 
 
@@ -45,6 +46,15 @@ def test_special_values_stay_where_they_are(n, c, h, w, k, size, stride):
     f = np.ones((k, c, size, size), np.float16)
     pad = size // 2
     np.testing.assert_array_equal(chx.conv(chx.array(x), chx.array(f), None, stride, pad).get(), O.conv(x, f, None, stride, pad))
+
+
+def test_route():
+    """conv_route names these kernels, and the large tiles where those take over."""
+    def route(n, c, h, w, k, size, stride):
+        return chx.conv_route(chx.zeros((n, c, h, w), np.float16), chx.zeros((k, c, size, size), np.float16), None, stride, size // 2)
+
+    assert [route(*case) for case in _CASES] == [4] * (len(_CASES) - 1) + [0]
+    assert route(32, 64, 56, 56, 64, 3, 1) == route(32, 512, 28, 28, 256, 1, 2) == 1
 
 
 @pytest.mark.parametrize('size', [1, 3])

@@ -33,3 +33,11 @@ def test_special_values_stay_where_they_are():
     f = np.ones((24, 3, 3, 3), np.float32)
     f[5, 0, 1, 1] = -np.inf
     np.testing.assert_array_equal(chx.conv(chx.array(x), chx.array(f), None, 1, 1).get(), O.conv(x, f, None, 1, 1))
+
+
+@pytest.mark.parametrize('dt', ['float32', 'float16'])
+def test_route(dt):
+    x = chx.zeros((4, 3, 12, 12), dt)
+    assert chx.conv_route(x, chx.zeros((64, 3, 3, 3), dt), None, 1, 1) == 5
+    assert chx.conv_route(x, chx.zeros((64, 3, 4, 4), dt), None, 1, 1) == 0
+    assert chx.conv_route(x, chx.zeros((8, 3, 3, 3), dt), None, 1, 1) == 0
