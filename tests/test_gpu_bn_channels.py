@@ -12,7 +12,8 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize('dt', ['float32', 'float16'])
 @pytest.mark.parametrize('shape', [
     (1, 3, 1, 1), (2, 5, 3, 3), (21, 7, 7, 7), (3, 260, 25, 27), (42, 257, 7, 7), (5, 3, 14, 14), (33, 9, 14, 14),
-    (1, 2, 64, 128), (2, 2, 64, 128), (4, 2, 64, 128), (4, 3, 130, 126), (25, 256, 32, 128), (25, 2, 32, 128), (13, 1, 64, 128), (14, 2, 64, 128)])
+    (1, 2, 64, 128), (2, 2, 64, 128), (4, 2, 64, 128), (4, 3, 130, 126), (25, 256, 32, 128), (25, 2, 32, 128), (13, 1, 64, 128), (14, 2, 64, 128),
+    (7, 2, 64, 126), (2, 257, 62, 66)])
 def test_forward_and_gradient(dt, shape):
     rng = np.random.default_rng(shape[0] * shape[1])
     c = shape[1]

@@ -20,7 +20,8 @@ def _check(got, x, w):
     np.testing.assert_array_less(np.abs(got.astype(np.float64) - x @ w.T), bound)
 
 
-@pytest.mark.parametrize('m,k,n', [(2048, 64, 1024), (2049, 650, 1153), (1793, 66, 1025), (4000, 17 * 2, 700), (4097, 2, 640), (1500, 4098, 1300), (300, 4096, 300)])
+@pytest.mark.parametrize('m,k,n', [(2048, 64, 1024), (2049, 650, 1153), (1793, 66, 1025), (4000, 17 * 2, 700), (4097, 2, 640), (1500, 4098, 1300), (300, 4096, 300),
+                                   (20001, 66, 40), (20001, 64, 33), (100, 42, 90), (100, 36, 130)])
 def test_products(m, k, n):
     rng = np.random.default_rng(k)
     # magnitudes over thirty powers of two: every part of an operand matters
@@ -39,7 +40,8 @@ def test_reduction_of_transposed_operands_is_split():
 
 @pytest.mark.parametrize('shape,filters,kernel,stride,pad', [
     ((16, 16, 33, 31), 64, 3, 1, 1), ((16, 32, 17, 17), 130, 3, 2, 1), ((8, 48, 20, 20), 96, 5, 1, 2), ((64, 20, 28, 28), 72, 1, 1, 0),
-    ((3, 64, 40, 40), 256, (1, 3), 1, (0, 1)), ((40, 64, 9, 9), 70, 2, 1, 0)])
+    ((3, 64, 40, 40), 256, (1, 3), 1, (0, 1)), ((40, 64, 9, 9), 70, 2, 1, 0),
+    ((40, 48, 28, 28), 72, 1, 1, 0), ((30, 16, 25, 23), 130, 3, 1, 1)])
 def test_convolutions(shape, filters, kernel, stride, pad):
     rng = np.random.default_rng(filters)
     kh, kw = (kernel, kernel) if isinstance(kernel, int) else kernel
