@@ -1,7 +1,7 @@
 // out[m][n] = sum over b < batch, k < depth of a[b][m][k] * bt[b][n][k] in float16: the weight gradients of convolutions, whose outputs are a few
 // 128 x 128 tiles and whose reduction is every pixel of every image.
 //
-// The reduction is cut into chunks of 32 k of an image and split over `slices` workgroups per tile, whose float sums SplitKReduceKernel adds up.
+// The reduction is cut into chunks of 32 k of an image and split over `slices` workgroups per tile, whose float sums BatchedSumKernel adds up.
 // Operands come from far away (a tile's rows are read once) and a slice is a few dozen chunks, so what counts is loads in flight: they go to LDS
 // directly, three chunks ahead in a ring of four (64 KiB; two workgroups to a compute unit), and one barrier a
 // chunk hands a stage over.  LDS layout, swizzle and counted waits as in gemm_pp.h.  An image's last chunk is masked in registers, in both operands: what
@@ -263,7 +263,8 @@ void HalfProduct(const BatchedOperands& o, float* partial, int slices, hipStream
     p.a_bytes = static_cast<unsigned>(Bytes(o.M, o.a_row, o.a_slice, o));
     p.b_bytes = static_cast<unsigned>(Bytes(b_rows, o.b_row, o.b_slice, o) + 2 * last_b);
     const int64_t tiles = static_cast<int64_t>((o.M + 127) / 128) * p.tiles_n;
-    ProfileScope prof(stream, 2.0 * o.M * o.N * o.depth * o.batch, 2.0 * (static_cast<double>(o.M) * o.depth * o.batch + static_cast<double>(o.N) * o.depth * o.batch + static_cast<double>(o.M) * o.N));
+    const double terms = static_cast<double>(o.depth) * o.batch;
+    ProfileScope prof(stream, 2.0 * o.M * o.N * terms, 2.0 * (o.M * terms + o.N * terms + static_cast<double>(o.M) * o.N));
     struct BatchedProductTag {};
     EnsureDynamicLds<BatchedProductTag>(reinterpret_cast<const void*>(BatchedProductKernel), kRing * kStageBytes);
     hipLaunchKernelGGL(BatchedProductKernel, dim3(static_cast<unsigned>(tiles * slices)), dim3(256), kRing * kStageBytes, stream, p);

@@ -1,9 +1,10 @@
 // Matrix products with small outputs (batch-sized Linear layers, recurrent steps, weight gradients of small layers):
 // out[M,N] = a[M,K] . b[K,N] with so few elements that 128x128 tiles would occupy a handful of compute units.
 //
-// A workgroup owns one 32x32 tile of `out` (SmallDotLinesKernel: 16 to 64 columns); its waves split the reduction axis -- and, with ksplit > 1, so do several workgroups, whose
-// sums another kernel adds up -- each feeding the MFMA from global memory on its own (operands this small live in the caches), and
-// the partial tiles are summed through LDS.  Five kernels, by where the operands lie (chosen in TrySmallDot):
+// A workgroup owns one 32x32 tile of `out` (SmallDotLinesKernel: 16 to 64 columns, SmallDotColumnsKernel: 64x64); its waves split the reduction
+// axis -- and, with ksplit > 1, so do several workgroups, whose sums another kernel adds up -- each feeding the MFMA from global memory on its own
+// (operands this small live in the caches), and the partial tiles are summed through LDS.  Five kernels, by where the operands lie (chosen in
+// LaunchSmallDot, the last one in PlanSmallDot):
 //   SmallDotKernel        k is the unit-stride axis of both operands (Linear's x and W^T): straight from global memory, bound by the
 //                         latency of a few loads.
 //   SmallDotLinesKernel   the same for more or longer tiles: whole 128-byte lines regrouped through LDS.

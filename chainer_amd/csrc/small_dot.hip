@@ -88,17 +88,10 @@ void LaunchSmallDotMixed(const SmallDotArgs& p, dim3 grid, int pieces, hipStream
 
 // Columns, in 16s, of the tiles of whole lines regrouped through LDS (SmallDotLinesKernel); 0: loads straight into the MFMA layout (SmallDotKernel) are
 // faster.  `rows` tiles of 32 rows, each of whose reductions of `k` terms `parts` workgroups share.  Tiles take the narrowest width that finds each of
-// them a compute unit, and long enough reductions: below, the detour through LDS outweighs the lines.  us, SmallDotKernel, then tiles of 16, 32, 48 and 64 columns:
-//   float32  [100,300] . [300,1000]  4.7  5.0  6.2              [100,1000] . [1000,1000]  8.5  7.4  9.1 11.3
-//            [256,800] . [800,1000]  9.4  9.3  9.0 11.2         [64,1300] . [1300,2600]  10.6 13.2 11.6        [256,1024] . [1024,1024] 11.4 10.1 9.4 11.5
-//            [128,300] . [300,2600]  6.9  7.6  8.0  8.4  9.6    [128,650] . [650,2600]   12.2 12.0 12.4 11.1 12.7
-//            [300,300] . [300,1500]  7.7  9.2  8.5 14.2 10.2    [300,650] . [650,1500]   13.9 14.7 13.2 19.1 13.7
-//   float16  [100,650] . [650,1000]  4.2  4.3  4.7              [37,2048] . [2048,1000]   9.7  5.1  6.1  7.3
-//            [128,300] . [300,2600]  4.2  4.9  7.9  5.5  6.5    [128,650] . [650,2600]    6.5  6.5  8.0  5.9  6.6
-//            [300,300] . [300,1500]  4.6  5.9  8.0  9.2  6.7    [500,1000] . [1000,1000]  9.5  8.8 10.3 11.3  8.3
-// 64 columns in float32: within 3 % of 32.  More tiles than compute units at any width, 32 and 48 columns: float32 [1024,1024]^2 23.6 26.8, float16
-// [1024,1024]^2 10.7 10.5, [700,1500] . [1500,900] 13.9 12.2, [800,2000] . [2000,800] 15.6 14.6; 484 tiles of 300 terms, SmallDotKernel and 32 columns: float32
-// 9.0 8.6, float16 4.7 5.6.  No width that pads the columns by a tenth more than 32 does ([2122,442] . [442,106] in float16 5.2 us, 6.0 by 48 columns).
+// them a compute unit, and long enough reductions: below, the detour through LDS outweighs the lines.  us, SmallDotKernel, then tiles of 16, 32, 48 and 64
+// columns (more of them: profiles/matrix_product_plans.txt): float32 [100,1000] . [1000,1000] 8.5 7.4 9.1 11.3, [128,650] . [650,2600] 12.2 12.0 12.4 11.1
+// 12.7, [100,300] . [300,1000] 4.7 5.0 6.2; float16 [37,2048] . [2048,1000] 9.7 5.1 6.1 7.3, [500,1000] . [1000,1000] 9.5 8.8 10.3 11.3 8.3.  No width that
+// pads the columns by a tenth more than 32 does ([2122,442] . [442,106] in float16 5.2 us, 6.0 by 48 columns).
 template <typename T>
 int LinesBlocks(int64_t rows, int64_t n, int64_t parts, int64_t k) {
     constexpr bool kHalf = sizeof(T) == 2;
@@ -117,8 +110,9 @@ int LinesBlocks(int64_t rows, int64_t n, int64_t parts, int64_t k) {
 }
 
 // Their waves: eight keep most loads in flight while a compute unit has one or two tiles (328 float32 tiles of 21 chunks: 12.3 us, 12.8 with four, 16.6
-// with two), or four for the lighter float16 ones beyond one ([150,1024] . [1024,4096] by 48 columns 9.6 -> 8.6 us); beyond, what leaves the busiest SIMD the fewest chunks, fewer waves on near terms (626 tiles of 21 chunks: 17.6 us with two, 18.2 with three, 16.5 with four; 1252 of
-// 21: 26.9, 26.5, 29.0; 1504 of 25: 34.1, 37.9, 35.3).
+// with two), or four for the lighter float16 ones beyond one ([150,1024] . [1024,4096] by 48 columns 9.6 -> 8.6 us); beyond, what leaves the busiest SIMD
+// the fewest chunks, fewer waves on near terms (626 tiles of 21 chunks: 17.6 us with two, 18.2 with three, 16.5 with four; 1252 of 21: 26.9, 26.5, 29.0;
+// 1504 of 25: 34.1, 37.9, 35.3).
 int LinesWaves(int64_t groups, int chunks, bool half) {
     if (groups <= 2 * NumCUs()) return std::min(half && groups > NumCUs() ? 4 : kSmallDotMaxWaves, chunks);
     const int64_t per_unit = (groups + NumCUs() - 1) / NumCUs();
