@@ -419,11 +419,11 @@ def section_families(chx, oracle, with_cpu):
         ('take float32 [10000,650] by [128,35]', r'TakeRowsKernel', lambda: chx.take(table, ids, 0), 2 * 128 * 35 * 650 * 4 + 128 * 35 * 4, 0, 1),
         ('dot float32 [100,784].[784,1000] (config 1)', r'SmallDot', lambda: chx.dot(a1, w1.T), (100 * 784 + 784 * 1000 + 100 * 1000) * 4, 2.0 * 100 * 784 * 1000, 1),
         ('dot float32 [128,650].[650,2600] (config 5 gates)', r'SmallDot', lambda: chx.dot(a5, w5.T), (128 * 650 + 650 * 2600 + 128 * 2600) * 4, 2.0 * 128 * 650 * 2600, 1),
-        ('dot float32 [4480,650].[650,10000] (config 5 output layer)', r'IGemmFastKernel<float', lambda: chx.dot(a5o, w5o.T),
+        ('dot float32 [4480,650].[650,10000] (config 5 output layer)', r'IGemmSplitKernel', lambda: chx.dot(a5o, w5o.T),
          (4480 * 650 + 650 * 10000 + 4480 * 10000) * 4, 2.0 * 4480 * 650 * 10000, 1),
         ('dot float16 [128,2048].[2048,1000] (config 4 classifier)', r'SmallDot', lambda: chx.dot(a4, w4.T), (128 * 2048 + 2048 * 1000 + 128 * 1000) * 2, 2.0 * 128 * 2048 * 1000, 1),
         ('dot float16 [4096,4096].[4096,4096] (calibration)', r'GemmPpKernel', lambda: chx.dot(ag, wg.T), 3 * 4096 * 4096 * 2, 2.0 * 4096 ** 3, 1),
-        ('conv float32 3x3 [256,64,32,32] -> 64 (config 3)', r'IGemmFastKernel<float', lambda: chx.conv(cx, cw, None, 1, 1),
+        ('conv float32 3x3 [256,64,32,32] -> 64 (config 3)', r'IGemmSplitKernel', lambda: chx.conv(cx, cw, None, 1, 1),
          (2 * 256 * 64 * 32 * 32 + 64 * 64 * 9) * 4, 2.0 * 256 * 32 * 32 * 64 * 64 * 9, 1),
         ('conv float16 1x1 [128,512,28,28] -> 128', r'PwConvKernel', lambda: chx.conv(px, pw), (128 * 512 * 784 + 128 * 512 + 128 * 128 * 784) * 2, 2.0 * 128 * 784 * 128 * 512, 1),
         ('n_step_lstm float32 2 layers x 35 steps, batch 128, 650 units (RnnKernel entry)', r'LstmStepKernel',
