@@ -2,12 +2,13 @@
 //
 // v_mfma_f32_32x32x16_bf16 does sixteen times the multiply-adds of v_mfma_f32_32x32x2_f32 in a clock.  A float is the sum of three
 // bfloat16 numbers, exactly: x1 = bf16(x), x2 = bf16(x - x1), x3 = x - x1 - x2 (24 significant bits = 3 x 8; rounding to nearest leaves
-// remainders of at most half a unit, which have 16 and 8 bits).  Of the nine products of two such sums all but x3 w3, at most 2^-34 of x w, are
-// computed.  A bfloat16 product is exact in float32; the matrix pipe's additions are not rounded to nearest (one product added to the sum of its
-// small parts may be off by a whole unit).  Hence two accumulators: x1 w1, whose 16 bits leave room for a few terms without any rounding and which
-// is rounded once for 16 terms, and the seven others, 2^-8 of it, whose roundings do not show; they are added at the end.  Largest relative error of
-// one term 5.98e-8 (5.96e-8 on the float pipe, rounded to nearest; 1.5e-7 with one accumulator and six products), 2-norm for two to eight terms
-// among zeros 2.6 to 2.8e-8 (3.1 to 5.4e-8; 4.1 to 8.2e-8), for more see LaunchShape.
+// remainders of at most half a unit, which have 16 and 8 bits; such splits are published, e.g. Henry, Tang and Heinecke, ARITH 2019).  Of the
+// nine products of two such sums all but x3 w3, at most 2^-34 of x w, are computed.  A bfloat16 product is exact in float32; the matrix pipe's
+// additions are not rounded to nearest (one product added to the sum of its small parts may be off by a whole unit).  Hence two accumulators:
+// x1 w1, whose 16 bits leave room for a few terms without any rounding and which is rounded once for 16 terms, and the seven others, 2^-8 of it,
+// whose roundings do not show; they are added at the end.  Largest relative error of one term 5.98e-8 (5.96e-8 on the float pipe, rounded to
+// nearest; 1.5e-7 with one accumulator and six products), 2-norm for two to eight terms among zeros 2.6 to 2.8e-8 (3.1 to 5.4e-8; 4.1 to
+// 8.2e-8), for more see LaunchShape.
 //
 // Where the split is not exact the tile is computed again on the float pipe, by the same workgroup: a sum that is not finite (an operand that
 // is infinite, NaN or beyond bfloat16's range, or a sum that overflowed), a nonzero sum so small that its parts' roundings to multiples of 2^-149 add

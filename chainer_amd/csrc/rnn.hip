@@ -959,15 +959,21 @@ void RunForward(Pass& pass, const RnnPlan& pl, int activation, const hipcx_array
     // scratch array for every ys[t]) or with an input are kept here until the end.
     float *const y_own = pass.Take(rows * DH), *const h_own = pass.Take(chains * B * H), *const c_own = pl.mode == kLstm ? pass.Take(chains * B * H) : nullptr;
     pass.StartScratch();
-    bool own = false;
+    bool own = false, in_order = false;
     if (!pass.dry()) {
-        std::vector<const hipcx_array*> outs{hy}, ins{hx};
+        auto same = [](const hipcx_array* a, const hipcx_array* b) { return a->data == b->data && std::equal(a->strides, a->strides + 3, b->strides); };
+        std::vector<const hipcx_array*> outs{hy}, ins;
+        if (!same(hx, hy)) ins.push_back(hx);  // (a state that is updated in place is copied onto itself)
         outs.insert(outs.end(), ys, ys + pl.T);
         ins.insert(ins.end(), xs, xs + pl.T);
         ins.insert(ins.end(), ws, ws + chains * 2 * pl.G);
         ins.insert(ins.end(), bs, bs + chains * 2 * pl.G);
-        if (pl.mode == kLstm) outs.push_back(cy), ins.push_back(cx);
+        if (pl.mode == kLstm) {
+            outs.push_back(cy);
+            if (!same(cx, cy)) ins.push_back(cx);
+        }
         own = AnyShared(outs, ins);
+        in_order = own && AnyShared(outs, {});
     }
     auto h_state = [&](int idx) { return own ? Matrix(h_own + idx * B * H, B, H, H) : StateSlice(hy, idx); };
     auto c_state = [&](int idx) { return own ? Matrix(c_own + idx * B * H, B, H, H) : StateSlice(cy, idx); };
@@ -1104,10 +1110,10 @@ void RunForward(Pass& pass, const RnnPlan& pl, int activation, const hipcx_array
         for (int idx = 0; idx < chains; ++idx) pass.Copy(Matrix(h0 + idx * B * H, B, H, H), h_state(idx));
         pass.FlushCopies();
     }
-    if (own) {  // one after the other: the last step's outputs and then the states are what is left where they share memory
+    if (own) {  // where they share memory one after the other: the last step's outputs and then the states are what is left
         auto hand_out = [&](const hipcx_array& from, const hipcx_array& to) {
             pass.Copy(from, to);
-            pass.FlushCopies();
+            if (in_order) pass.FlushCopies();
         };
         for (int d = 0; d < pl.D; ++d) {
             for (int s = 0; s < pl.T; ++s) {
@@ -1120,6 +1126,7 @@ void RunForward(Pass& pass, const RnnPlan& pl, int activation, const hipcx_array
             hand_out(h_state(idx), StateSlice(hy, idx));
             if (pl.mode == kLstm) hand_out(c_state(idx), StateSlice(cy, idx));
         }
+        pass.FlushCopies();
     }
     pass.CheckFits();
 }

@@ -222,6 +222,8 @@ def test_results_that_share_memory(kind, layers, bidirectional, units, lengths, 
         np.testing.assert_array_equal(y.get(), r)
     h2, c2 = hx.copy(), cx.copy()
     run(h2, c2, X, h2, c2, [chx.zeros(y.shape, np.float32) for y in ys])
+    h2, c2 = hx.copy(), cx.copy()
+    run(h2, c2, X, c2, h2, [chx.zeros(y.shape, np.float32) for y in ys])
     batch_major = chx.zeros((ys[0].shape[0], T, d * units), np.float32)
     interleaved = [batch_major[:len(y), t] for t, y in enumerate(ys)]
     run(hx, cx, X, *new(), interleaved)
