@@ -113,24 +113,43 @@ def test_sums_of_few_terms_among_zeros(terms, float_pipe, scale):
     assert np.linalg.norm(got - exact) <= 1.01 * float_pipe * np.linalg.norm(exact)
 
 
+def _tiny(rng, shape):
+    """Values below 2^-120: their third parts, and of most the second, are beyond bfloat16's least number, 2^-133."""
+    return (rng.uniform(0.5, 1, shape) * rng.choice([-1, 1], shape) * 2.0 ** -120).astype(np.float32)
+
+
 def test_tiny_values_beside_ordinary_ones():
     """Bits below 2^-133 are lost in the split, which counts only in sums that are as small."""
     rng = np.random.default_rng(7)
     m, k, n = 2100, 200, 1100
     x, w = rng.standard_normal((m, k), dtype=np.float32), rng.standard_normal((n, k), dtype=np.float32)
-    tiny = (rng.standard_normal((m, k)) * 2.0 ** -116).astype(np.float32)
+    tiny = _tiny(rng, (m, k))
     x[::3, 5] = tiny[::3, 5]      # among others
     x[7::128] = tiny[7::128]      # rows of nothing else
     x[9::128] = 0
     x[9::128, 3] = tiny[9::128, 3]
     x[11::128] = 0
-    w[4::200] *= np.float32(2.0 ** -112)
+    w[4::200] = _tiny(rng, w[4::200].shape)
     w[6::200] = 0
     got = chx.linear(chx.array(x), chx.array(w)).get().astype(np.float64)
     exact, magnitude = x.astype(np.float64) @ w.T.astype(np.float64), np.abs(x).astype(np.float64) @ np.abs(w.T).astype(np.float64)
     # as in a sum of ordinary products; each product and sum also rounds to a multiple of 2^-149
     np.testing.assert_array_less(np.abs(got - exact), (k + 4) * _EPS * magnitude + 2 * k * 2.0 ** -150)
     assert (got[11::128] == 0).all() and (got[:, 6::200] == 0).all()
+
+
+@pytest.mark.parametrize('filters', [40, 130])  # tiles of 256 x 64 and 128 x 128, pixels first
+def test_tiny_pixels_and_filters(filters):
+    rng = np.random.default_rng(filters)
+    n, c, h, w = 30, 48, 27, 29
+    x = rng.standard_normal((n, h, w, c), dtype=np.float32).reshape(-1, c)
+    f = rng.standard_normal((filters, c), dtype=np.float32)
+    x[5::97] = _tiny(rng, x[5::97].shape)
+    f[3::31] = _tiny(rng, f[3::31].shape)
+    got = chx.conv(chx.array(np.ascontiguousarray(x.reshape(n, h, w, c).transpose(0, 3, 1, 2))), chx.array(f.reshape(filters, c, 1, 1))).get()
+    got = got.transpose(0, 2, 3, 1).reshape(-1, filters).astype(np.float64)
+    exact, magnitude = x.astype(np.float64) @ f.T.astype(np.float64), np.abs(x).astype(np.float64) @ np.abs(f.T).astype(np.float64)
+    np.testing.assert_array_less(np.abs(got - exact), (c + 4) * _EPS * magnitude + 2 * c * 2.0 ** -150)
 
 
 @pytest.mark.parametrize('given', [0, 256, 1 << 24])
