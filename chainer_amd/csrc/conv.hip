@@ -1328,7 +1328,8 @@ DotStaging PlanDotStaging(const hipcx_array* a, const hipcx_array* b, const hipc
     const int64_t epv = 16 / it, kpad = (k + epv - 1) / epv * epv;
     // a changed pitch on one side needs the same (zero-padded) k extent on the other
     const bool copy_a = !a_fast || kpad != k, copy_b = !b_fast || kpad != k;
-    if (SmallDotShape(m, n, k)) {
+    const bool reversed = a->strides[0] < 0 || a->strides[1] < 0 || b->strides[0] < 0 || b->strides[1] < 0;  // which the small product's kernels do not take
+    if (SmallDotShape(m, n, k) && !(k < 64 && reversed)) {
         const int64_t lines = (copy_a ? m : 0) + (copy_b ? n : 0);
         if (out->dtype != HIPCX_FLOAT32 || flops < 7e9 || m * n < 256 * lines || PlanSplitK(m, n, k, out->dtype, true) == 1) return st;
     }

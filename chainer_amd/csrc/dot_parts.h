@@ -5,7 +5,7 @@
 
 namespace hipcx {
 
-// Whether an [m,k] . [k,n] product is small: fewer than 128 tiles of 128 x 128.
+// Whether an [m,k] . [k,n] product is small: fewer than 128 tiles of 128 x 128, 256 for fewer than 64 terms.
 bool SmallDotShape(int64_t m, int64_t n, int64_t k);
 
 // Bytes of partial sums that TrySmallDot would use.

@@ -8,7 +8,11 @@
 
 namespace hipcx {
 
-bool SmallDotShape(int64_t m, int64_t n, int64_t k) { return ((m + 127) / 128) * ((n + 127) / 128) < 128 && k >= 64; }
+// Fewer tiles of 128 x 128 than keep the chip busy; up to 256 for fewer than 64 terms, where larger tiles are bound by copying operands into their layout.  us,
+// without and with these kernels: [64,33] . [33,64] float32 35 and 4.1, [20,50] . [50,8789] 33 and 4.2, float16 30 and 3.9, [128,63] . [63,2600] 41 and 4.6 (one
+// element after another, or a wave to a tile); [352,35] . [35,8653], 204 tiles, 23 and 13.5, float16 23 and 17; beyond, 288 tiles of [3000,33] . [33,1500], 18.2 and
+// 18.9, float16 17.3 and 23.7.
+bool SmallDotShape(int64_t m, int64_t n, int64_t k) { return ((m + 127) / 128) * ((n + 127) / 128) < (k >= 64 ? 128 : 256); }
 
 namespace {
 
@@ -191,6 +195,16 @@ void LaunchSmallDot(SmallDotArgs p, int a_mode, int b_mode, int batch, hipStream
     if constexpr (sizeof(T) == 2) with_a(std::integral_constant<int, kOddPieces>{});
 }
 
+// Rows of a and columns of b of whole 8-byte granules, k dense: what IGemmFastKernel and IGemmSplitKernel read.
+template <typename T>
+bool LiesForTiles(const hipcx_array* a, const hipcx_array* b) {
+    const int64_t it = sizeof(T), k = a->shape[1];
+    auto lies = [&](const void* ptr, int64_t line, int64_t k_stride) {
+        return k_stride == it && line % 8 == 0 && k * it % 8 == 0 && reinterpret_cast<uintptr_t>(ptr) % 8 == 0;
+    };
+    return lies(a->data, a->strides[0], a->strides[1]) && lies(b->data, b->strides[1], b->strides[0]);
+}
+
 // Which kernel of small_dot.h takes a product.
 enum SmallDotPath { kNoSmallDot, kSmallDotVector, kSmallDotTiles, kSmallDotWhole };  // (whole: tiles whose reduction is not split)
 
@@ -199,6 +213,12 @@ SmallDotPath PlanSmallDot(const hipcx_array* a, const hipcx_array* b, SmallDotAr
     static const bool enabled = [] { const char* e = getenv("HIPCX_SMALL_DOT"); return e == nullptr || e[0] != '0'; }();
     const int64_t M = a->shape[0], K = a->shape[1], N = b->shape[1];
     if (!enabled || !SmallDotShape(M, N, K) || !SmallDotOperands<T>(a, b, p, a_mode, b_mode)) return kNoSmallDot;
+    if (K < 64 && LiesForTiles<T>(a, b)) {
+        // The tiles of 128 x 128 read these operands as they lie.  float16: [1000,32] . [32,1000] 7.9 us there and 5.0 here, [8192,8] . [8,512] (256 of them) 8.7 and
+        // 13.2.  float32: 6 to 10 us there and 3 to 6 here, but with errors of 2.8e-8 to 4.6e-8 (2-norm, 8 to 50 terms; bfloat16 parts) and 5.4e-8 to 7.7e-8; a
+        // single tile is summed term by term there, which recurrent networks that amplify rounding are held to.
+        if (sizeof(T) == 4 || ((M + 127) / 128) * ((N + 127) / 128) >= 128) return kNoSmallDot;
+    }
     if (*a_mode != kPieces || *b_mode != kPieces) return kSmallDotTiles;
     if (M <= 4) return kSmallDotVector;
     return 2.0 * M * N * K >= 1e9 ? kSmallDotWhole : kSmallDotTiles;  // enough tiles, or enough of them long, to keep the chip busy
