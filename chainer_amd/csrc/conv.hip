@@ -8,6 +8,7 @@
 #include <utility>
 #include <vector>
 
+#include "direct_conv.h"
 #include "gemm_pp.h"
 #include "igemm.h"
 #include "igemm_pipe.h"
@@ -1125,7 +1126,8 @@ int hipcx_conv_route(const hipcx_array* x, const hipcx_array* w, const hipcx_arr
         if (PlanPw(x, w, b, out, stride, pad).ok) return 3;
         if (const NchwPlan pl = PlanNchw(x, w, out, stride, pad); pl.ok) return SmallConvTakes(NchwExtents(x, w, out, stride), pl.taps) ? 4 : 1;
         if (PlanStem(x, w, out, stride, pad).ok) return 2;
-        return ThinConvTakes(x, w, stride, pad, out) ? 5 : 0;
+        if (ThinConvTakes(x, w, stride, pad, out)) return 5;
+        return DirectConvTakes(x, w, stride, pad, out) ? 6 : 0;
     } catch (...) {
         return -1;
     }
@@ -1172,6 +1174,7 @@ int hipcx_conv(const hipcx_array* x, const hipcx_array* w, const hipcx_array* b,
             else RunConv<half_t>(x, w, b, pl, out, ws, st);
         } else if (out->dtype == HIPCX_FLOAT32) {
             if (ThinConvTakes(x, w, stride, pad, out)) ThinConv(x, w, b, stride, pad, out, st);
+            else if (DirectConvTakes(x, w, stride, pad, out)) DirectConv(x, w, b, out, st);
             else RunConv<float>(x, w, b, pl, out, ws, st);
         } else {
             RunConv<double>(x, w, b, pl, out, ws, st);

@@ -752,7 +752,8 @@ def _spatial_out(x, n, c, h, w, dtype):
 def conv_route(x, w, b=None, stride=1, pad=0, cover_all=False):
     """Which kernel family `conv` runs for these arguments (hipcx_conv_route): 0 general implicit GEMM, 1 float16 NCHW kernels
     with 128-wide tiles, 2 the 7x7 / 2 stem kernel, 3 the float16 1x1 kernel with LDS-direct operand loads, 4 the float16 kernel for
-    few output pixels, 5 the kernel for sums of at most 32 terms.  For tests and benchmarks; not part of the ChainerX routine surface."""
+    few output pixels, 5 the kernel for sums of at most 32 terms, 6 the float32 3x3 kernel for few output tiles.  For tests and benchmarks;
+    not part of the ChainerX routine surface."""
     stride, pad = _pair(stride), _pair(pad)
     dt = result_type(x, w, b) if b is not None else result_type(x, w)
     oh = conv_out_dim(x.shape[2], w.shape[2], stride[0], pad[0], cover_all)
