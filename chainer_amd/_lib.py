@@ -219,6 +219,9 @@ SIGNATURES = {
     'hipcx_fixed_batch_norm': (_INT, [_A, _A, _A, _A, _A, _S, _I8P, _INT, _A, _V]),
     'hipcx_batch_norm_workspace_size': (_SZ, [_A, _I8P, _INT]),
     'hipcx_batch_norm': (_INT, [_A, _A, _A, _A, _A, _S, _S, _I8P, _INT, _A, _A, _A, _V, _SZ, _V]),
+    'hipcx_batch_norm_relu': (_INT, [_A, _A, _A, _A, _A, _S, _S, _I8P, _INT, _A, _A, _A, _A, _A, _V, _SZ, _V]),
+    'hipcx_batch_norm_relu_grad': (_INT, [_A, _A, _A, _A, _A, _A, _I8P, _INT, _A, _A, _A, _V, _SZ, _V]),
+    'hipcx_add_relu_grad': (_INT, [_A, _A, _A, _A, _V]),
     'hipcx_batch_norm_grad': (_INT, [_A, _A, _A, _A, _A, _I8P, _INT, _A, _A, _A, _V, _SZ, _V]),
     'hipcx_solve_workspace_size': (_SZ, [_A]),
     'hipcx_solve': (_INT, [_A, _A, _A, _V, _SZ, ctypes.POINTER(ctypes.c_int32), _V]),

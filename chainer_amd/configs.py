@@ -232,7 +232,7 @@ class DeviceTrainOps:
     def __init__(self, chx):
         self.c = chx
         for name in ('conv', 'relu', 'max_pool', 'average_pool', 'linear', 'log_softmax', 'exp', 'add', 'subtract', 'multiply', 'sum',
-                     'max_pool_grad', 'average_pool_grad', 'conv_transpose', 'dot', 'batch_norm_grad'):
+                     'max_pool_grad', 'average_pool_grad', 'conv_transpose', 'dot', 'batch_norm_grad', 'batch_norm_relu_grad', 'add_relu_grad'):
             setattr(self, name, getattr(chx, name))
         self.array = chx.array
         self.get = lambda a: a.get()
@@ -254,19 +254,33 @@ class DeviceTrainOps:
     def scale(self, a, s):
         return self.c.multiply(a, s)
 
+    def batch_norm_relu(self, x, gamma, beta, rm, rv, residual=None):
+        return self.c.batch_norm_relu(x, gamma, beta, rm, rv, BN_EPS, 0.9, None, residual)
 
-def _unit_forward(F, x, w, bn, stride, pad, relu):
-    """conv -> batch norm (batch statistics, running statistics updated in place) -> optional ReLU; returns (y, saved)."""
+
+def _unit_forward(F, x, w, bn, stride, pad, relu, residual=None):
+    """conv -> batch norm (batch statistics, running statistics updated in place) -> optional sum with `residual` -> optional ReLU; returns
+    (y, the sum or None, saved).  `F` may supply batch norm and ReLU as one routine."""
     c = F.conv(x, w, None, stride, pad)
-    b, state = F.batch_norm(c, bn['gamma'], bn['beta'], bn['mean'], bn['var'])
-    y = F.relu(b) if relu else b
-    return y, (x, w, bn, stride, pad, c, state, b if relu else None)
+    total = None
+    if relu and hasattr(F, 'batch_norm_relu'):
+        y, total, state = F.batch_norm_relu(c, bn['gamma'], bn['beta'], bn['mean'], bn['var'], residual)
+        pre = None
+    else:
+        pre, state = F.batch_norm(c, bn['gamma'], bn['beta'], bn['mean'], bn['var'])
+        if residual is not None:
+            total = F.add(pre, residual)
+        y = F.relu(pre if total is None else total) if relu else pre
+    return y, total, (x, w, bn, stride, pad, c, state, relu and residual is None, pre)
 
 
 def _unit_backward(F, saved, gy, grads, need_gx=True):
-    x, w, bn, stride, pad, c, state, pre = saved
-    g = F.relu_grad(pre, gy) if pre is not None else gy
-    gc, ggamma, gbeta = F.batch_norm_grad(c, bn['gamma'], g, state)
+    """`gy`: gradient of the unit's result, of the sum where there is a residual."""
+    x, w, bn, stride, pad, c, state, relu, pre = saved
+    if relu and pre is None:
+        gc, ggamma, gbeta = F.batch_norm_relu_grad(c, bn['gamma'], bn['beta'], gy, state)
+    else:
+        gc, ggamma, gbeta = F.batch_norm_grad(c, bn['gamma'], F.relu_grad(pre, gy) if relu else gy, state)
     grads.append((bn, 'gamma', ggamma))
     grads.append((bn, 'beta', gbeta))
     grads.append((w, None, F.conv_grad_weight(w, x, gc, stride, pad)))
@@ -277,21 +291,19 @@ def resnet50_train_step(F, p, x, t, lr=0.01):
     """One SGD step on softmax cross entropy (mean over the batch); updates `p` in place and returns the loss array."""
     n = x.shape[0]
     # ---- forward ----
-    h0, s_stem = _unit_forward(F, x, p['conv1'], p['bn1'], 2, 3, True)
+    h0, _, s_stem = _unit_forward(F, x, p['conv1'], p['bn1'], 2, 3, True)
     h = F.max_pool(h0, 3, 2, 1, False)
     tape = []
     for si, stage in enumerate(p['stages']):
         for bi, blk in enumerate(stage):
             stride = 2 if (bi == 0 and si > 0) else 1
-            a, s1 = _unit_forward(F, h, blk['conv1'], blk['bn1'], stride, 0, True)
-            b, s2 = _unit_forward(F, a, blk['conv2'], blk['bn2'], 1, 1, True)
-            c, s3 = _unit_forward(F, b, blk['conv3'], blk['bn3'], 1, 0, False)
+            a, _, s1 = _unit_forward(F, h, blk['conv1'], blk['bn1'], stride, 0, True)
+            b, _, s2 = _unit_forward(F, a, blk['conv2'], blk['bn2'], 1, 1, True)
             if 'conv4' in blk:
-                sc, s4 = _unit_forward(F, h, blk['conv4'], blk['bn4'], stride, 0, False)
+                sc, _, s4 = _unit_forward(F, h, blk['conv4'], blk['bn4'], stride, 0, False)
             else:
                 sc, s4 = h, None
-            pre = F.add(c, sc)
-            h = F.relu(pre)
+            h, pre, s3 = _unit_forward(F, b, blk['conv3'], blk['bn3'], 1, 0, True, sc)
             tape.append((s1, s2, s3, s4, pre))
     pooled = F.average_pool(h, h.shape[2], 1, 0, 'zero')
     feat = pooled.reshape((n, -1))
@@ -305,25 +317,31 @@ def resnet50_train_step(F, p, x, t, lr=0.01):
     g_fc_w = F.dot(dlogits.T, feat)
     g_fc_b = F.sum(dlogits, 0)
     gh = F.average_pool_grad(h, F.dot(dlogits, p['fc_w']).reshape(pooled.shape), h.shape[2], 1, 0, 'zero')
+    shortcut = None  # gh is a sum whose other part is this
     for (s1, s2, s3, s4, pre) in reversed(tape):
-        g = F.relu_grad(pre, gh)
+        if shortcut is None:
+            g = F.relu_grad(pre, gh)
+        elif hasattr(F, 'add_relu_grad'):
+            g = F.add_relu_grad(pre, gh, shortcut)
+        else:
+            g = F.relu_grad(pre, F.add(gh, shortcut))
         gb = _unit_backward(F, s3, g, grads)
         ga = _unit_backward(F, s2, gb, grads)
-        gx = _unit_backward(F, s1, ga, grads)
-        gh = F.add(gx, _unit_backward(F, s4, g, grads) if s4 is not None else g)
-    g0 = F.max_pool_grad(h0, gh, 3, 2, 1)
+        gh = _unit_backward(F, s1, ga, grads)
+        shortcut = _unit_backward(F, s4, g, grads) if s4 is not None else g
+    g0 = F.max_pool_grad(h0, F.add(gh, shortcut), 3, 2, 1)
     _unit_backward(F, s_stem, g0, grads, need_gx=False)
     # ---- SGD ----
+    grads += [(p, 'fc_w', g_fc_w), (p, 'fc_b', g_fc_b)]
+    params = [container if key is None else container[key] for container, key, _ in grads]
+    new = [F.subtract(old, F.scale(g.reshape(old.shape), lr)) for old, (_, _, g) in zip(params, grads)]
     updates = {}
-    for container, key, g in grads:
+    for (container, key, _), a in zip(grads, new):
         if key is None:
-            updates[id(container)] = F.subtract(container, F.scale(g, lr))
+            updates[id(container)] = a
         else:
-            container[key] = F.subtract(container[key], F.scale(g.reshape(container[key].shape), lr))
-
+            container[key] = a
     _replace_leaves(p, updates)  # filters are values of dicts: replace them where they live
-    p['fc_w'] = F.subtract(p['fc_w'], F.scale(g_fc_w, lr))
-    p['fc_b'] = F.subtract(p['fc_b'], F.scale(g_fc_b, lr))
     return loss
 
 

@@ -71,9 +71,18 @@ struct BnStatArgs {
     int S;
     int state_in_array_dtype;  // see LoadState
     int64_t mean_stride, inv_stride;
+    const void* gamma;  // MODE 3
+    const void* beta;
+    int64_t gamma_stride, beta_stride;
 };
 
-// MODE 0: sum x.  MODE 1: sum (x - mean)^2.  MODE 2: sum g and sum g * (x - mean) * inv_std.
+// Whether Relu passes a gradient on where batch norm made a value of x_hat: not where that, as the array held it, is below zero.
+template <typename T, typename P, typename C>
+__device__ __forceinline__ bool ReluPasses(C x_hat, C gamma, C beta) {
+    return !(static_cast<C>(static_cast<T>(Rnd<P>(x_hat * gamma) + beta)) < C(0));
+}
+
+// MODE 0: sum x.  MODE 1: sum (x - mean)^2.  MODE 2: sum g and sum g * (x - mean) * inv_std.  MODE 3: the same of what Relu passes of g.
 template <typename T, typename P, int MODE, int VEC>
 __global__ __launch_bounds__(kBnTrainThreads) void BnStatKernel(BnStatArgs p) {
     using C = compute_t<T>;
@@ -83,7 +92,9 @@ __global__ __launch_bounds__(kBnTrainThreads) void BnStatKernel(BnStatArgs p) {
     const T* g = static_cast<const T*>(p.g);
     C m = C(0), is = C(1);
     if (MODE >= 1) m = LoadState<T, P>(p.mean, c, p.state_in_array_dtype, p.mean_stride);
-    if (MODE == 2) is = LoadState<T, P>(p.inv_std, c, p.state_in_array_dtype, p.inv_stride);
+    if (MODE >= 2) is = LoadState<T, P>(p.inv_std, c, p.state_in_array_dtype, p.inv_stride);
+    C gamma = C(0), beta = C(0);
+    if (MODE == 3) gamma = static_cast<C>(static_cast<const P*>(p.gamma)[c * p.gamma_stride]), beta = static_cast<C>(static_cast<const P*>(p.beta)[c * p.beta_stride]);
     C a0 = C(0), a1 = C(0);
     // The slice's images n = s, s + S, ... times the plane's vectors form one index space shared out over the threads, so that
     // planes shorter than the workgroup (14x14, 7x7) keep every lane busy.  32-bit index arithmetic: the host checks N * L < 2^31.
@@ -95,7 +106,7 @@ __global__ __launch_bounds__(kBnTrainThreads) void BnStatKernel(BnStatArgs p) {
         const int64_t base = (static_cast<int64_t>(s + j * p.S) * p.C + c) * p.L + static_cast<int64_t>(v) * VEC;
         Vec<T, VEC> xv = *reinterpret_cast<const Vec<T, VEC>*>(x + base);
         Vec<T, VEC> gv;
-        if (MODE == 2) gv = *reinterpret_cast<const Vec<T, VEC>*>(g + base);
+        if (MODE >= 2) gv = *reinterpret_cast<const Vec<T, VEC>*>(g + base);
 #pragma unroll
         for (int e = 0; e < VEC; ++e) {
             C xe = static_cast<C>(xv.v[e]);
@@ -105,14 +116,16 @@ __global__ __launch_bounds__(kBnTrainThreads) void BnStatKernel(BnStatArgs p) {
                 C d = Rnd<P>(xe - m);
                 a0 += Rnd<P>(d * d);
             } else {
+                const C x_hat = Rnd<P>(Rnd<P>(xe - m) * is);
                 C ge = static_cast<C>(gv.v[e]);
+                if (MODE == 3 && !ReluPasses<T, P>(x_hat, gamma, beta)) ge = C(0);
                 a0 += ge;
-                a1 += Rnd<P>(ge * Rnd<P>(Rnd<P>(xe - m) * is));
+                a1 += Rnd<P>(ge * x_hat);
             }
         }
     }
     C r0 = BlockSum<C>(a0, lds);
-    C r1 = MODE == 2 ? BlockSum<C>(a1, lds) : C(0);
+    C r1 = MODE >= 2 ? BlockSum<C>(a1, lds) : C(0);
     if (threadIdx.x == 0) {
         C* out = static_cast<C*>(p.partial) + (static_cast<int64_t>(c) * p.S + s) * 2;
         out[0] = r0;
@@ -197,6 +210,8 @@ struct BnApplyArgs {
     double count;
     int state_in_array_dtype;  // see LoadState
     int64_t mean_stride, inv_stride;
+    const void* residual;  // RELU, forward: added before Relu; may be null
+    void* sum;             // RELU, forward: where that sum goes; null with residual
 };
 
 // Gradient finish: ggamma = sum g * x_hat, gbeta = sum g, one thread per channel; leaves both as compute-type values at partial[c][0].
@@ -217,9 +232,25 @@ __global__ __launch_bounds__(256) void BnGradFinishKernel(BnApplyArgs p) {
     static_cast<P*>(p.ggamma)[c * p.gg_stride] = static_cast<P>(sgx);
 }
 
+// Relu of a vector of results, or of its sum with the residual's at element `at`, which is stored too.
+template <typename T, int VEC>
+__device__ __forceinline__ Vec<T, VEC> AddRelu(const BnApplyArgs& p, Vec<T, VEC> o, int64_t at) {
+    using C = compute_t<T>;
+    if (p.residual != nullptr) {
+        const Vec<T, VEC> r = *reinterpret_cast<const Vec<T, VEC>*>(static_cast<const T*>(p.residual) + at);
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) o.v[e] = static_cast<T>(static_cast<C>(o.v[e]) + static_cast<C>(r.v[e]));
+        *reinterpret_cast<Vec<T, VEC>*>(static_cast<T*>(p.sum) + at) = o;
+    }
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) o.v[e] = static_cast<C>(o.v[e]) < C(0) ? static_cast<T>(C(0)) : o.v[e];
+    return o;
+}
+
 // GRAD false: out = ((x - mean) * inv_std) * gamma + beta.
 // GRAD true:  gx = (gamma * inv_std) * (g - (x_hat * ggamma + gbeta) / count)   (CX/routines/normalization.cc:232-246).
-template <typename T, typename P, bool GRAD, int VEC>
+// RELU: Relu of it, or of its sum with another array, and the gradient through both.
+template <typename T, typename P, bool GRAD, int VEC, bool RELU>
 __global__ __launch_bounds__(256) void BnApplyKernel(BnApplyArgs p) {
     using C = compute_t<T>;
     const T* x = static_cast<const T*>(p.x);
@@ -261,12 +292,19 @@ __global__ __launch_bounds__(256) void BnApplyKernel(BnApplyArgs p) {
             }
             Vec<T, VEC> gv = *reinterpret_cast<const Vec<T, VEC>*>(g + v * VEC);
             const C scale = Rnd<P>(ga * is), scale2 = Rnd<P>(ga2 * is2);
+            C be = C(0), be2 = C(0);
+            if constexpr (RELU) {
+                be = static_cast<C>(static_cast<const P*>(p.beta)[c * p.beta_stride]);
+                be2 = split ? static_cast<C>(static_cast<const P*>(p.beta)[c2 * p.beta_stride]) : be;
+            }
 #pragma unroll
             for (int e = 0; e < VEC; ++e) {
                 const bool second = e >= split_at;
                 C x_hat = Rnd<P>(Rnd<P>(static_cast<C>(xv.v[e]) - (second ? m2 : m)) * (second ? is2 : is));
                 C t = Rnd<P>(Rnd<P>(Rnd<P>(x_hat * (second ? ggamma2 : ggamma)) + (second ? gbeta2 : gbeta)) * inv_n);
-                o.v[e] = static_cast<T>((second ? scale2 : scale) * Rnd<P>(static_cast<C>(gv.v[e]) - t));
+                C ge = static_cast<C>(gv.v[e]);
+                if (RELU && !ReluPasses<T, P>(x_hat, second ? ga2 : ga, second ? be2 : be)) ge = C(0);
+                o.v[e] = static_cast<T>((second ? scale2 : scale) * Rnd<P>(ge - t));
             }
         } else {
             const C be = static_cast<C>(static_cast<const P*>(p.beta)[c * p.beta_stride]);
@@ -277,6 +315,7 @@ __global__ __launch_bounds__(256) void BnApplyKernel(BnApplyArgs p) {
                 C t = Rnd<P>(Rnd<P>(static_cast<C>(xv.v[e]) - (second ? m2 : m)) * (second ? is2 : is));
                 o.v[e] = static_cast<T>(Rnd<P>(t * (second ? ga2 : ga)) + (second ? be2 : be));
             }
+            if constexpr (RELU) o = AddRelu<T, VEC>(p, o, v * VEC);
         }
         *reinterpret_cast<Vec<T, VEC>*>(out + v * VEC) = o;
     }
@@ -288,6 +327,9 @@ __global__ __launch_bounds__(256) void BnApplyKernel(BnApplyArgs p) {
 // repeat its last vector, so that none is conditional, and count as nothing.  Bound by memory and, for small channels, by the latency of a load and
 // two sums over the workgroup.  us, forward / gradient, float16 with float32 parameters: [32,256,14,14] 14.1 / 9.9 -> 4.8 / 4.9, [32,512,28,28] 27.0 /
 // 26.0 -> 13.2 / 19.3, [32,256,56,56] 42.5 / 42.6 -> 21.0 / 36.7, [2,64,56,56] 15.3 / 10.4 -> 5.1 / 5.1.
+// RELU saves the passes of the element-wise kernels behind (forward two, with a residual three) and in front (gradient three: the sign comes from x, not from an
+// array kept for it).  us with launch gaps, separate kernels and this, [32,256,56,56] forward 47 -> 34, with a residual 71 -> 45, gradient 60 -> 43; a ResNet-50
+// training step at batch 32 6670 -> 5950.
 // ---------------------------------------------------------------------------------------------
 template <typename C, int THREADS>
 __device__ __forceinline__ C BlockTotal(C v, C* lds) {  // the same for every thread
@@ -326,7 +368,7 @@ __device__ __forceinline__ void Forget(V& v) {
     v = __builtin_bit_cast(V, r);
 }
 
-template <typename T, typename P, int VEC, int NV, int THREADS>
+template <typename T, typename P, int VEC, int NV, int THREADS, bool RELU>
 __global__ __launch_bounds__(THREADS) void BnChannelKernel(BnFinishArgs f, BnApplyArgs p, int N) {
     using C = compute_t<T>;
     __shared__ C lds[THREADS / 64];
@@ -378,11 +420,14 @@ __global__ __launch_bounds__(THREADS) void BnChannelKernel(BnFinishArgs f, BnApp
             const C t = Rnd<P>(Rnd<P>(static_cast<C>(xv[i].v[e]) - mean) * inv_std);
             o.v[e] = static_cast<T>(Rnd<P>(t * gamma) + beta);
         }
-        if (i < own) *reinterpret_cast<Vec<T, VEC>*>(out + off[i]) = o;
+        if (i < own) {
+            if constexpr (RELU) o = AddRelu<T, VEC>(p, o, off[i]);
+            *reinterpret_cast<Vec<T, VEC>*>(out + off[i]) = o;
+        }
     }
 }
 
-template <typename T, typename P, int VEC, int NV, int THREADS>
+template <typename T, typename P, int VEC, int NV, int THREADS, bool RELU>
 __global__ __launch_bounds__(THREADS) void BnChannelGradKernel(BnApplyArgs p, int N) {
     using C = compute_t<T>;
     __shared__ C lds[THREADS / 64];
@@ -400,18 +445,24 @@ __global__ __launch_bounds__(THREADS) void BnChannelGradKernel(BnApplyArgs p, in
     }
     const C m = LoadState<T, P>(p.mean, c, p.state_in_array_dtype, p.mean_stride), is = LoadState<T, P>(p.inv_std, c, p.state_in_array_dtype, p.inv_stride);
     const C gamma = static_cast<C>(static_cast<const P*>(p.gamma)[c * p.gamma_stride]);
+    C beta = C(0);
+    if constexpr (RELU) beta = static_cast<C>(static_cast<const P*>(p.beta)[c * p.beta_stride]);
     C a0 = C(0), a1 = C(0);
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
+        Forget(xv[i]), Forget(gv[i]);  // one vector after another: taken up together they need more registers than there are
         C t0 = C(0), t1 = C(0);
 #pragma unroll
         for (int e = 0; e < VEC; ++e) {
-            const C ge = static_cast<C>(gv[i].v[e]);
+            const C x_hat = Rnd<P>(Rnd<P>(static_cast<C>(xv[i].v[e]) - m) * is);
+            C ge = static_cast<C>(gv[i].v[e]);
+            if (RELU && !ReluPasses<T, P>(x_hat, gamma, beta)) ge = C(0);
             t0 += ge;
-            t1 += Rnd<P>(ge * Rnd<P>(Rnd<P>(static_cast<C>(xv[i].v[e]) - m) * is));
+            t1 += Rnd<P>(ge * x_hat);
         }
         a0 += i < own ? t0 : C(0);
         a1 += i < own ? t1 : C(0);
+        asm volatile("" : "+v"(a0), "+v"(a1));
     }
     const C sg = BlockTotal<C, THREADS>(a0, lds), sgx = BlockTotal<C, THREADS>(a1, lds);
     if (threadIdx.x == 0) {
@@ -429,7 +480,9 @@ __global__ __launch_bounds__(THREADS) void BnChannelGradKernel(BnApplyArgs p, in
         for (int e = 0; e < VEC; ++e) {
             const C x_hat = Rnd<P>(Rnd<P>(static_cast<C>(xv[i].v[e]) - m) * is);
             const C t = Rnd<P>(Rnd<P>(Rnd<P>(x_hat * ggamma) + gbeta) * inv_n);
-            o.v[e] = static_cast<T>(scale * Rnd<P>(static_cast<C>(gv[i].v[e]) - t));
+            C ge = static_cast<C>(gv[i].v[e]);
+            if (RELU && !ReluPasses<T, P>(x_hat, gamma, beta)) ge = C(0);
+            o.v[e] = static_cast<T>(scale * Rnd<P>(ge - t));
         }
         if (i < own) *reinterpret_cast<Vec<T, VEC>*>(out + off[i]) = o;
     }
@@ -547,7 +600,7 @@ void LaunchStat(const BnStatArgs& a, int width, hipStream_t stream) {
     CheckLaunch("batch_norm statistics");
 }
 
-template <typename T, typename P, bool GRAD>
+template <typename T, typename P, bool GRAD, bool RELU>
 void LaunchApply(const BnApplyArgs& a, bool vec, hipStream_t stream) {
     constexpr int VEC = 16 / sizeof(T);
     int64_t nvec = a.total / (vec ? VEC : 1);
@@ -556,9 +609,9 @@ void LaunchApply(const BnApplyArgs& a, bool vec, hipStream_t stream) {
     if (blocks > cap) blocks = cap;
     if (blocks < 1) blocks = 1;
     if (vec) {
-        hipLaunchKernelGGL((BnApplyKernel<T, P, GRAD, VEC>), dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, a);
+        hipLaunchKernelGGL((BnApplyKernel<T, P, GRAD, VEC, RELU>), dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, a);
     } else {
-        hipLaunchKernelGGL((BnApplyKernel<T, P, GRAD, 1>), dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, a);
+        hipLaunchKernelGGL((BnApplyKernel<T, P, GRAD, 1, RELU>), dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, a);
     }
     CheckLaunch("batch_norm apply");
 }
@@ -597,6 +650,163 @@ void CheckWorkspace(void* workspace, size_t workspace_bytes, size_t need) {
     HIPCX_REQUIRE(reinterpret_cast<uintptr_t>(workspace) % 16 == 0, HIPCX_CHAINERX_ERROR, "workspace must be 16-byte aligned");
 }
 
+// BatchNorm; RELU: Relu of it, or of its sum with `residual` (may be null), which goes to `total`.
+template <bool RELU>
+int BatchNorm(const hipcx_array* x, const hipcx_array* gamma, const hipcx_array* beta, const hipcx_array* running_mean, const hipcx_array* running_var,
+              hipcx_scalar eps, hipcx_scalar decay, const int8_t* axis, int naxis, const hipcx_array* residual, const hipcx_array* total_out, const hipcx_array* out,
+              const hipcx_array* mean_out, const hipcx_array* inv_std_out, void* workspace, size_t workspace_bytes, void* stream) {
+    return Guard([&] {
+        BnTrainGeom g = MakeGeom(x, axis, naxis);
+        ValidateArray(out, "out");
+        HIPCX_REQUIRE(out->dtype == x->dtype && SameShape(x, out) && IsContiguous(out), HIPCX_NOT_IMPLEMENTED_ERROR,
+                      "hip batch_norm: out must be C-contiguous with x's shape and dtype");
+        if (residual != nullptr) {
+            ValidateArray(residual, "residual");
+            ValidateArray(total_out, "total");
+            for (const hipcx_array* y : {residual, total_out}) {
+                HIPCX_REQUIRE(y->dtype == x->dtype && SameShape(x, y) && IsContiguous(y), HIPCX_NOT_IMPLEMENTED_ERROR,
+                              "hip batch_norm_relu: residual and total must be C-contiguous with x's shape and dtype");
+            }
+        }
+        BnFinishArgs f{};
+        BnApplyArgs a{};
+        const int pd = ParamDtype(x, gamma);
+        a.gamma_stride = ChannelStride(gamma, x, "gamma", pd);
+        a.beta_stride = ChannelStride(beta, x, "beta", pd);
+        f.rm_stride = ChannelStride(running_mean, x, "running_mean", pd);
+        f.rv_stride = ChannelStride(running_var, x, "running_var", pd);
+        f.mo_stride = ChannelStride(mean_out, x, "mean_out", pd);
+        f.io_stride = ChannelStride(inv_std_out, x, "inv_std_out", pd);
+        const int64_t total = static_cast<int64_t>(g.N) * g.C * g.L;
+        if (total == 0) return;
+        CheckWorkspace(workspace, workspace_bytes, TrainWorkspace(g));
+        char* ws = static_cast<char*>(workspace);
+        const size_t vec_bytes = RoundUpTo(static_cast<size_t>(g.C) * g.csize, 16);
+        void* mean_c = ws;
+        void* inv_c = ws + vec_bytes;
+        void* partial = ws + 2 * vec_bytes;
+        hipStream_t st = AsStream(stream);
+        HIPCX_REQUIRE(total < (int64_t{1} << 31), HIPCX_NOT_IMPLEMENTED_ERROR, "hip batch_norm: array too large for the dedicated kernels");
+        const BnWidths widths = PickWidths(g.L, total, ItemSize(x->dtype), {x->data, out->data, residual != nullptr ? residual->data : nullptr, residual != nullptr ? total_out->data : nullptr});
+        BnStatArgs s{};
+        s.x = x->data;
+        s.mean = mean_c;
+        s.inv_std = inv_c;
+        s.partial = partial;
+        s.N = g.N, s.C = g.C, s.L = g.L, s.S = g.S;
+        f.partial = partial;
+        f.mean = mean_c;
+        f.inv_std = inv_c;
+        f.mean_out = mean_out->data;
+        f.inv_std_out = inv_std_out->data;
+        f.running_mean = running_mean->data;
+        f.running_var = running_var->data;
+        f.C = g.C, f.S = g.S;
+        f.count = static_cast<double>(g.N) * static_cast<double>(g.L);
+        f.eps = ScalarTo<double>(eps);
+        f.decay = ScalarTo<double>(decay);
+        a.x = x->data;
+        a.out = out->data;
+        a.residual = residual != nullptr ? residual->data : nullptr;
+        a.sum = residual != nullptr ? total_out->data : nullptr;
+        a.mean = mean_c;
+        a.inv_std = inv_c;
+        a.gamma = gamma->data;
+        a.beta = beta->data;
+        a.C = g.C, a.S = g.S, a.L = g.L, a.total = total;
+        a.count = f.count;
+        const unsigned cblocks = static_cast<unsigned>((g.C + 255) / 256);
+        VisitBnDtypes(x->dtype, pd, [&](auto tag, auto ptag) {
+            using T = typename decltype(tag)::type;
+            using P = typename decltype(ptag)::type;
+            const bool done = VisitChannelShape<T, false>(g, widths.stat, [&](auto vec, auto nv, auto threads) {
+                hipLaunchKernelGGL((BnChannelKernel<T, P, decltype(vec)::value, decltype(nv)::value, decltype(threads)::value, RELU>),
+                                   dim3(static_cast<unsigned>(g.C)), dim3(decltype(threads)::value), 0, st, f, a, g.N);
+                CheckLaunch("batch_norm channels");
+            });
+            if (done) return;
+            LaunchStat<T, P, 0>(s, widths.stat, st);
+            hipLaunchKernelGGL((BnFinishKernel<T, P, 0>), dim3(cblocks), dim3(256), 0, st, f);
+            LaunchStat<T, P, 1>(s, widths.stat, st);
+            hipLaunchKernelGGL((BnFinishKernel<T, P, 1>), dim3(cblocks), dim3(256), 0, st, f);
+            CheckLaunch("batch_norm finish");
+            LaunchApply<T, P, false, RELU>(a, widths.apply, st);
+        });
+    });
+}
+
+// BatchNormGrad; RELU: of BatchNorm with Relu behind it, whose sign is computed again from x, gamma and beta.
+template <bool RELU>
+int BatchNormGrad(const hipcx_array* x, const hipcx_array* gamma, const hipcx_array* beta, const hipcx_array* gout, const hipcx_array* mean,
+                  const hipcx_array* inv_std, const int8_t* axis, int naxis, const hipcx_array* gx, const hipcx_array* ggamma, const hipcx_array* gbeta,
+                  void* workspace, size_t workspace_bytes, void* stream) {
+    return Guard([&] {
+        BnTrainGeom g = MakeGeom(x, axis, naxis);
+        ValidateArray(gout, "gout");
+        ValidateArray(gx, "gx");
+        HIPCX_REQUIRE(gout->dtype == x->dtype && SameShape(x, gout) && IsContiguous(gout), HIPCX_NOT_IMPLEMENTED_ERROR,
+                      "hip batch_norm_grad: gout must be C-contiguous with x's shape and dtype");
+        HIPCX_REQUIRE(gx->dtype == x->dtype && SameShape(x, gx) && IsContiguous(gx), HIPCX_NOT_IMPLEMENTED_ERROR,
+                      "hip batch_norm_grad: gx must be C-contiguous with x's shape and dtype");
+        BnApplyArgs a{};
+        const int pd = ParamDtype(x, gamma);
+        a.gamma_stride = ChannelStride(gamma, x, "gamma", pd);
+        if constexpr (RELU) a.beta_stride = ChannelStride(beta, x, "beta", pd);
+        a.gg_stride = ChannelStride(ggamma, x, "ggamma", pd);
+        a.gb_stride = ChannelStride(gbeta, x, "gbeta", pd);
+        const int64_t mean_stride = ChannelStride(mean, x, "mean", pd);
+        const int64_t inv_stride = ChannelStride(inv_std, x, "inv_std", pd);
+        const int64_t total = static_cast<int64_t>(g.N) * g.C * g.L;
+        if (total == 0) return;
+        CheckWorkspace(workspace, workspace_bytes, TrainWorkspace(g));
+        char* ws = static_cast<char*>(workspace);
+        const size_t vec_bytes = RoundUpTo(static_cast<size_t>(g.C) * g.csize, 16);
+        void* partial = ws + 2 * vec_bytes;  // the same layout as the forward's workspace; the state vectors before it stay unused here
+        hipStream_t st = AsStream(stream);
+        HIPCX_REQUIRE(total < (int64_t{1} << 31), HIPCX_NOT_IMPLEMENTED_ERROR, "hip batch_norm_grad: array too large for the dedicated kernels");
+        const BnWidths widths = PickWidths(g.L, total, ItemSize(x->dtype), {x->data, gout->data, gx->data});
+        BnStatArgs s{};
+        s.x = x->data;
+        s.g = gout->data;
+        s.mean = mean->data;  // the state as BatchNorm handed it out, read in place
+        s.inv_std = inv_std->data;
+        s.state_in_array_dtype = 1;
+        s.mean_stride = mean_stride, s.inv_stride = inv_stride;
+        s.partial = partial;
+        s.N = g.N, s.C = g.C, s.L = g.L, s.S = g.S;
+        a.x = x->data;
+        a.g = gout->data;
+        a.out = gx->data;
+        a.mean = mean->data;
+        a.inv_std = inv_std->data;
+        a.state_in_array_dtype = 1;
+        a.mean_stride = mean_stride, a.inv_stride = inv_stride;
+        a.gamma = s.gamma = gamma->data;
+        if constexpr (RELU) a.beta = s.beta = beta->data;
+        s.gamma_stride = a.gamma_stride, s.beta_stride = a.beta_stride;
+        a.partial = partial;
+        a.ggamma = ggamma->data;
+        a.gbeta = gbeta->data;
+        a.C = g.C, a.S = g.S, a.L = g.L, a.total = total;
+        a.count = static_cast<double>(g.N) * static_cast<double>(g.L);
+        const unsigned cblocks = static_cast<unsigned>((g.C + 255) / 256);
+        VisitBnDtypes(x->dtype, pd, [&](auto tag, auto ptag) {
+            using T = typename decltype(tag)::type;
+            using P = typename decltype(ptag)::type;
+            const bool done = VisitChannelShape<T, true>(g, widths.stat, [&](auto vec, auto nv, auto threads) {
+                hipLaunchKernelGGL((BnChannelGradKernel<T, P, decltype(vec)::value, decltype(nv)::value, decltype(threads)::value, RELU>),
+                                   dim3(static_cast<unsigned>(g.C)), dim3(decltype(threads)::value), 0, st, a, g.N);
+                CheckLaunch("batch_norm_grad channels");
+            });
+            if (done) return;
+            LaunchStat<T, P, RELU ? 3 : 2>(s, widths.stat, st);
+            hipLaunchKernelGGL((BnGradFinishKernel<T, P>), dim3(cblocks), dim3(256), 0, st, a);
+            CheckLaunch("batch_norm_grad finish");
+            LaunchApply<T, P, true, RELU>(a, widths.apply, st);
+        });
+    });
+}
+
 }  // namespace
 }  // namespace hipcx
 
@@ -633,141 +843,28 @@ int hipcx_batch_norm(const hipcx_array* x, const hipcx_array* gamma, const hipcx
                      const hipcx_array* running_var, hipcx_scalar eps, hipcx_scalar decay, const int8_t* axis, int naxis,
                      const hipcx_array* out, const hipcx_array* mean_out, const hipcx_array* inv_std_out, void* workspace,
                      size_t workspace_bytes, void* stream) {
-    return Guard([&] {
-        BnTrainGeom g = MakeGeom(x, axis, naxis);
-        ValidateArray(out, "out");
-        HIPCX_REQUIRE(out->dtype == x->dtype && SameShape(x, out) && IsContiguous(out), HIPCX_NOT_IMPLEMENTED_ERROR,
-                      "hip batch_norm: out must be C-contiguous with x's shape and dtype");
-        BnFinishArgs f{};
-        BnApplyArgs a{};
-        const int pd = ParamDtype(x, gamma);
-        a.gamma_stride = ChannelStride(gamma, x, "gamma", pd);
-        a.beta_stride = ChannelStride(beta, x, "beta", pd);
-        f.rm_stride = ChannelStride(running_mean, x, "running_mean", pd);
-        f.rv_stride = ChannelStride(running_var, x, "running_var", pd);
-        f.mo_stride = ChannelStride(mean_out, x, "mean_out", pd);
-        f.io_stride = ChannelStride(inv_std_out, x, "inv_std_out", pd);
-        const int64_t total = static_cast<int64_t>(g.N) * g.C * g.L;
-        if (total == 0) return;
-        CheckWorkspace(workspace, workspace_bytes, TrainWorkspace(g));
-        char* ws = static_cast<char*>(workspace);
-        const size_t vec_bytes = RoundUpTo(static_cast<size_t>(g.C) * g.csize, 16);
-        void* mean_c = ws;
-        void* inv_c = ws + vec_bytes;
-        void* partial = ws + 2 * vec_bytes;
-        hipStream_t st = AsStream(stream);
-        HIPCX_REQUIRE(total < (int64_t{1} << 31), HIPCX_NOT_IMPLEMENTED_ERROR, "hip batch_norm: array too large for the dedicated kernels");
-        const BnWidths widths = PickWidths(g.L, total, ItemSize(x->dtype), {x->data, out->data});
-        BnStatArgs s{};
-        s.x = x->data;
-        s.mean = mean_c;
-        s.inv_std = inv_c;
-        s.partial = partial;
-        s.N = g.N, s.C = g.C, s.L = g.L, s.S = g.S;
-        f.partial = partial;
-        f.mean = mean_c;
-        f.inv_std = inv_c;
-        f.mean_out = mean_out->data;
-        f.inv_std_out = inv_std_out->data;
-        f.running_mean = running_mean->data;
-        f.running_var = running_var->data;
-        f.C = g.C, f.S = g.S;
-        f.count = static_cast<double>(g.N) * static_cast<double>(g.L);
-        f.eps = ScalarTo<double>(eps);
-        f.decay = ScalarTo<double>(decay);
-        a.x = x->data;
-        a.out = out->data;
-        a.mean = mean_c;
-        a.inv_std = inv_c;
-        a.gamma = gamma->data;
-        a.beta = beta->data;
-        a.C = g.C, a.S = g.S, a.L = g.L, a.total = total;
-        a.count = f.count;
-        const unsigned cblocks = static_cast<unsigned>((g.C + 255) / 256);
-        VisitBnDtypes(x->dtype, pd, [&](auto tag, auto ptag) {
-            using T = typename decltype(tag)::type;
-            using P = typename decltype(ptag)::type;
-            const bool done = VisitChannelShape<T, false>(g, widths.stat, [&](auto vec, auto nv, auto threads) {
-                hipLaunchKernelGGL((BnChannelKernel<T, P, decltype(vec)::value, decltype(nv)::value, decltype(threads)::value>),
-                                   dim3(static_cast<unsigned>(g.C)), dim3(decltype(threads)::value), 0, st, f, a, g.N);
-                CheckLaunch("batch_norm channels");
-            });
-            if (done) return;
-            LaunchStat<T, P, 0>(s, widths.stat, st);
-            hipLaunchKernelGGL((BnFinishKernel<T, P, 0>), dim3(cblocks), dim3(256), 0, st, f);
-            LaunchStat<T, P, 1>(s, widths.stat, st);
-            hipLaunchKernelGGL((BnFinishKernel<T, P, 1>), dim3(cblocks), dim3(256), 0, st, f);
-            CheckLaunch("batch_norm finish");
-            LaunchApply<T, P, false>(a, widths.apply, st);
-        });
-    });
+    return BatchNorm<false>(x, gamma, beta, running_mean, running_var, eps, decay, axis, naxis, nullptr, nullptr, out, mean_out, inv_std_out, workspace, workspace_bytes,
+                            stream);
+}
+
+int hipcx_batch_norm_relu(const hipcx_array* x, const hipcx_array* gamma, const hipcx_array* beta, const hipcx_array* running_mean,
+                          const hipcx_array* running_var, hipcx_scalar eps, hipcx_scalar decay, const int8_t* axis, int naxis, const hipcx_array* residual,
+                          const hipcx_array* total, const hipcx_array* out, const hipcx_array* mean_out, const hipcx_array* inv_std_out, void* workspace,
+                          size_t workspace_bytes, void* stream) {
+    return BatchNorm<true>(x, gamma, beta, running_mean, running_var, eps, decay, axis, naxis, residual, total, out, mean_out, inv_std_out, workspace, workspace_bytes,
+                           stream);
 }
 
 int hipcx_batch_norm_grad(const hipcx_array* x, const hipcx_array* gamma, const hipcx_array* gout, const hipcx_array* mean,
                           const hipcx_array* inv_std, const int8_t* axis, int naxis, const hipcx_array* gx, const hipcx_array* ggamma,
                           const hipcx_array* gbeta, void* workspace, size_t workspace_bytes, void* stream) {
-    return Guard([&] {
-        BnTrainGeom g = MakeGeom(x, axis, naxis);
-        ValidateArray(gout, "gout");
-        ValidateArray(gx, "gx");
-        HIPCX_REQUIRE(gout->dtype == x->dtype && SameShape(x, gout) && IsContiguous(gout), HIPCX_NOT_IMPLEMENTED_ERROR,
-                      "hip batch_norm_grad: gout must be C-contiguous with x's shape and dtype");
-        HIPCX_REQUIRE(gx->dtype == x->dtype && SameShape(x, gx) && IsContiguous(gx), HIPCX_NOT_IMPLEMENTED_ERROR,
-                      "hip batch_norm_grad: gx must be C-contiguous with x's shape and dtype");
-        BnApplyArgs a{};
-        const int pd = ParamDtype(x, gamma);
-        a.gamma_stride = ChannelStride(gamma, x, "gamma", pd);
-        a.gg_stride = ChannelStride(ggamma, x, "ggamma", pd);
-        a.gb_stride = ChannelStride(gbeta, x, "gbeta", pd);
-        const int64_t mean_stride = ChannelStride(mean, x, "mean", pd);
-        const int64_t inv_stride = ChannelStride(inv_std, x, "inv_std", pd);
-        const int64_t total = static_cast<int64_t>(g.N) * g.C * g.L;
-        if (total == 0) return;
-        CheckWorkspace(workspace, workspace_bytes, TrainWorkspace(g));
-        char* ws = static_cast<char*>(workspace);
-        const size_t vec_bytes = RoundUpTo(static_cast<size_t>(g.C) * g.csize, 16);
-        void* partial = ws + 2 * vec_bytes;  // the same layout as the forward's workspace; the state vectors before it stay unused here
-        hipStream_t st = AsStream(stream);
-        HIPCX_REQUIRE(total < (int64_t{1} << 31), HIPCX_NOT_IMPLEMENTED_ERROR, "hip batch_norm_grad: array too large for the dedicated kernels");
-        const BnWidths widths = PickWidths(g.L, total, ItemSize(x->dtype), {x->data, gout->data, gx->data});
-        BnStatArgs s{};
-        s.x = x->data;
-        s.g = gout->data;
-        s.mean = mean->data;  // the state as BatchNorm handed it out, read in place
-        s.inv_std = inv_std->data;
-        s.state_in_array_dtype = 1;
-        s.mean_stride = mean_stride, s.inv_stride = inv_stride;
-        s.partial = partial;
-        s.N = g.N, s.C = g.C, s.L = g.L, s.S = g.S;
-        a.x = x->data;
-        a.g = gout->data;
-        a.out = gx->data;
-        a.mean = mean->data;
-        a.inv_std = inv_std->data;
-        a.state_in_array_dtype = 1;
-        a.mean_stride = mean_stride, a.inv_stride = inv_stride;
-        a.gamma = gamma->data;
-        a.partial = partial;
-        a.ggamma = ggamma->data;
-        a.gbeta = gbeta->data;
-        a.C = g.C, a.S = g.S, a.L = g.L, a.total = total;
-        a.count = static_cast<double>(g.N) * static_cast<double>(g.L);
-        const unsigned cblocks = static_cast<unsigned>((g.C + 255) / 256);
-        VisitBnDtypes(x->dtype, pd, [&](auto tag, auto ptag) {
-            using T = typename decltype(tag)::type;
-            using P = typename decltype(ptag)::type;
-            const bool done = VisitChannelShape<T, true>(g, widths.stat, [&](auto vec, auto nv, auto threads) {
-                hipLaunchKernelGGL((BnChannelGradKernel<T, P, decltype(vec)::value, decltype(nv)::value, decltype(threads)::value>),
-                                   dim3(static_cast<unsigned>(g.C)), dim3(decltype(threads)::value), 0, st, a, g.N);
-                CheckLaunch("batch_norm_grad channels");
-            });
-            if (done) return;
-            LaunchStat<T, P, 2>(s, widths.stat, st);
-            hipLaunchKernelGGL((BnGradFinishKernel<T, P>), dim3(cblocks), dim3(256), 0, st, a);
-            CheckLaunch("batch_norm_grad finish");
-            LaunchApply<T, P, true>(a, widths.apply, st);
-        });
-    });
+    return BatchNormGrad<false>(x, gamma, nullptr, gout, mean, inv_std, axis, naxis, gx, ggamma, gbeta, workspace, workspace_bytes, stream);
+}
+
+int hipcx_batch_norm_relu_grad(const hipcx_array* x, const hipcx_array* gamma, const hipcx_array* beta, const hipcx_array* gout, const hipcx_array* mean,
+                               const hipcx_array* inv_std, const int8_t* axis, int naxis, const hipcx_array* gx, const hipcx_array* ggamma,
+                               const hipcx_array* gbeta, void* workspace, size_t workspace_bytes, void* stream) {
+    return BatchNormGrad<true>(x, gamma, beta, gout, mean, inv_std, axis, naxis, gx, ggamma, gbeta, workspace, workspace_bytes, stream);
 }
 
 }  // extern "C"

@@ -119,6 +119,18 @@ void RunSelectASSA(const hipcx_array* x1, hipcx_scalar x2, hipcx_scalar pos, con
     });
 }
 
+// Relu's gradient on x of a sum of two: x < 0 ? 0 : g1 + g2, the sum rounded as an array holds it.
+template <typename T>
+struct AddReluGrad {
+    using In = T;
+    using Out = T;
+    static constexpr int kNumIn = 3;
+    static constexpr bool kNeedsIndex = false;
+    __device__ __forceinline__ compute_t<T> operator()(compute_t<T> x, compute_t<T> g1, compute_t<T> g2, compute_t<T>, int64_t) const {
+        return x < compute_t<T>(0) ? compute_t<T>(0) : static_cast<compute_t<T>>(static_cast<T>(g1 + g2));
+    }
+};
+
 enum class Cmp { kEq, kNe, kGt, kGe };
 
 template <typename T, Cmp C>
@@ -182,6 +194,14 @@ int hipcx_if_greater_else_aaaa(const hipcx_array* x1, const hipcx_array* x2, con
             using T = typename decltype(tag)::type;
             LaunchElementwise(p, SelectGreaterAAAA<T>{}, AsStream(stream));
         });
+    });
+}
+int hipcx_add_relu_grad(const hipcx_array* x, const hipcx_array* g1, const hipcx_array* g2, const hipcx_array* out, void* stream) {
+    return Guard([&] {
+        EwPlan p = MakeEwPlan({out, x, g1, g2});
+        HIPCX_REQUIRE(x->dtype == out->dtype && g1->dtype == out->dtype && g2->dtype == out->dtype, HIPCX_DTYPE_ERROR,
+                      "operand dtype differs from out dtype (cast with hipcx_copy first)");
+        VisitFloatDtype(out->dtype, [&](auto tag) { LaunchElementwise(p, AddReluGrad<typename decltype(tag)::type>{}, AsStream(stream)); });
     });
 }
 int hipcx_equal(const hipcx_array* x1, const hipcx_array* x2, const hipcx_array* out, void* stream) {

@@ -219,6 +219,21 @@ HOST_FN(IfLessElse) {
     HOST_CATCH(nullptr);
 }
 
+// IfLessElse(x, 0, 0, Add(g1, g2)) of float arrays of one shape and dtype in one kernel, or None.
+HOST_FN(AddReluGrad) {
+    HOST_TRY;
+    HOST_ARGS("add_relu_grad", 3, "x", "g1", "g2");
+    Array *x = AsArray(arg[0], "x"), *g1 = AsArray(arg[1], "g1"), *g2 = AsArray(arg[2], "g2");
+    for (const Array* g : {g1, g2}) {
+        if (!IsFloat(x->d.dtype) || g->d.dtype != x->d.dtype || !ShapeIs(g, x->d.ndim, x->d.shape)) Py_RETURN_NONE;
+    }
+    Ref out = EmptyLike(x, x->d.dtype);
+    void* stream = Stream();
+    Call([&] { return hipcx_add_relu_grad(&x->d, &g1->d, &g2->d, out.d(), stream); });
+    return out.release();
+    HOST_CATCH(nullptr);
+}
+
 HOST_FN(IfGreaterElse) {
     HOST_TRY;
     HOST_ARGS("if_greater_else", 4, "x1", "x2", "pos", "neg");
@@ -995,10 +1010,11 @@ int BnAxes(PyObject* axis, int ndim, int8_t* axes) {
 }
 
 // BatchNorm in training mode through hipcx_batch_norm -> (out, (mean, inv_std, beta dtype)), or None for calls the dedicated
-// kernels do not take.
+// kernels do not take.  `relu`: Relu of it, or of its sum with `residual`, through hipcx_batch_norm_relu -> (out, sum or None, state).
 HOST_FN(BatchNormDirect) {
     HOST_TRY;
-    HOST_ARGS("batch_norm", 5, "x", "gamma", "beta", "running_mean", "running_var", "eps", "decay", "axis");
+    HOST_ARGS("batch_norm", 5, "x", "gamma", "beta", "running_mean", "running_var", "eps", "decay", "axis", "relu", "residual");
+    const bool relu = Given(arg[8]) && PyObject_IsTrue(arg[8]) == 1;
     Array* a[5];
     for (int i = 0; i < 5; ++i) {
         a[i] = AsArray(arg[i], "argument");
@@ -1008,6 +1024,8 @@ HOST_FN(BatchNormDirect) {
     int8_t axes[HIPCX_MAX_NDIM];
     const int n_axes = BnAxes(arg[7], x->d.ndim, axes);
     if (!BnKernelApplies(x, axes, n_axes, {a[1], a[2], a[3], a[4]})) Py_RETURN_NONE;
+    Array* residual = Given(arg[9]) ? AsArray(arg[9], "residual") : nullptr;
+    if (residual != nullptr && (residual->d.dtype != x->d.dtype || !ShapeIs(residual, x->d.ndim, x->d.shape) || !IsContiguous(residual->d))) Py_RETURN_NONE;
     int64_t reduced[HIPCX_MAX_NDIM];
     std::copy(x->d.shape, x->d.shape + x->d.ndim, reduced);
     for (int i = 0; i < n_axes; ++i) reduced[axes[i]] = 1;
@@ -1028,6 +1046,16 @@ HOST_FN(BatchNormDirect) {
     Ref out = EmptyLike(x, x->d.dtype), mean = Empty(x->d.ndim, reduced, interm), inv_std = Empty(x->d.ndim, reduced, interm);
     Workspace ws(hipcx_batch_norm_workspace_size(&x->d, axes, n_axes));
     void* stream = Stream();
+    if (relu) {
+        Ref total = residual != nullptr ? EmptyLike(x, x->d.dtype) : Ref();
+        Call([&] {
+            return hipcx_batch_norm_relu(&x->d, &p[0], &p[1], &p[2], &p[3], eps, decay, axes, n_axes, residual != nullptr ? &residual->d : nullptr, total.d(),
+                                         out.d(), mean.d(), inv_std.d(), ws.ptr, ws.bytes, stream);
+        });
+        Ref state(PyTuple_Pack(3, mean.get(), inv_std.get(), a[2]->dtype));
+        if (!state) throw PyError();
+        return PyTuple_Pack(3, out.get(), total ? total.get() : Py_None, state.get());
+    }
     Call([&] {
         return hipcx_batch_norm(&x->d, &p[0], &p[1], &p[2], &p[3], eps, decay, axes, n_axes, out.d(), mean.d(), inv_std.d(), ws.ptr, ws.bytes, stream);
     });
@@ -1040,22 +1068,23 @@ HOST_FN(BatchNormDirect) {
 // GenericBatchNormGradKernel through hipcx_batch_norm_grad -> (gx, ggamma, gbeta), or None.
 HOST_FN(BatchNormGradDirect) {
     HOST_TRY;
-    HOST_ARGS("batch_norm_grad", 6, "x", "gamma", "gout", "x_mean", "x_inv_std", "beta_dtype", "axis");
+    HOST_ARGS("batch_norm_grad", 6, "x", "gamma", "gout", "x_mean", "x_inv_std", "beta_dtype", "axis", "relu_beta");
     Array *x = AsArray(arg[0], "x"), *gamma = AsArray(arg[1], "gamma"), *gout = AsArray(arg[2], "gout");
+    Array* beta = Given(arg[7]) ? AsArray(arg[7], "beta") : nullptr;  // the gradient of Relu's input, through hipcx_batch_norm_relu_grad
     Array *mean = AsArray(arg[3], "x_mean"), *inv_std = AsArray(arg[4], "x_inv_std");
     int8_t axes[HIPCX_MAX_NDIM];
     const int n_axes = BnAxes(arg[6], x->d.ndim, axes);
     if (!BnKernelApplies(x, axes, n_axes, {gamma, mean, inv_std}) || gout->d.dtype != x->d.dtype || !ShapeIs(gout, x->d.ndim, x->d.shape) ||
-        !IsContiguous(gout->d) || DtypeCode(arg[5]) != gamma->d.dtype) {
+        !IsContiguous(gout->d) || DtypeCode(arg[5]) != gamma->d.dtype || (beta != nullptr && beta->d.dtype != gamma->d.dtype)) {
         Py_RETURN_NONE;
     }
     int64_t reduced[HIPCX_MAX_NDIM];
     std::copy(x->d.shape, x->d.shape + x->d.ndim, reduced);
     for (int i = 0; i < n_axes; ++i) reduced[axes[i]] = 1;
-    Array* in[3] = {gamma, mean, inv_std};
-    hipcx_array p[3];
-    Ref keep[3];
-    for (int i = 0; i < 3; ++i) {
+    Array* in[4] = {gamma, mean, inv_std, beta};
+    hipcx_array p[4];
+    Ref keep[4];
+    for (int i = 0; i < (beta != nullptr ? 4 : 3); ++i) {
         if (Size(in[i]) != x->d.shape[1]) {
             Raise(HIPCX_DIMENSION_ERROR, "cannot reshape array of size %lld into %lld channels", static_cast<long long>(Size(in[i])), static_cast<long long>(x->d.shape[1]));
         }
@@ -1066,7 +1095,12 @@ HOST_FN(BatchNormGradDirect) {
     const hipcx_array gg = Reshaped(ggamma.arr(), x->d.ndim, reduced, &unused[0]), gb = Reshaped(gbeta.arr(), x->d.ndim, reduced, &unused[1]);
     Workspace ws(hipcx_batch_norm_workspace_size(&x->d, axes, n_axes));
     void* stream = Stream();
-    Call([&] { return hipcx_batch_norm_grad(&x->d, &p[0], &gout->d, &p[1], &p[2], axes, n_axes, gx.d(), &gg, &gb, ws.ptr, ws.bytes, stream); });
+    Call([&] {
+        if (beta != nullptr) {
+            return hipcx_batch_norm_relu_grad(&x->d, &p[0], &p[3], &gout->d, &p[1], &p[2], axes, n_axes, gx.d(), &gg, &gb, ws.ptr, ws.bytes, stream);
+        }
+        return hipcx_batch_norm_grad(&x->d, &p[0], &gout->d, &p[1], &p[2], axes, n_axes, gx.d(), &gg, &gb, ws.ptr, ws.bytes, stream);
+    });
     return PyTuple_Pack(3, gx.get(), ggamma.get(), gbeta.get());
     HOST_CATCH(nullptr);
 }
@@ -1310,6 +1344,7 @@ PyMethodDef kRoutines[] = {
         ROUTINE("average_pool_grad_2d", AveragePoolGrad2d, nullptr),
         ROUTINE("conv_grad_weight_2d", ConvGradWeight2d, nullptr),
         ROUTINE("conv_transpose_2d", ConvTranspose2d, nullptr),
+        ROUTINE("add_relu_grad_direct", AddReluGrad, nullptr),
         ROUTINE("batch_norm_direct", BatchNormDirect, nullptr),
         ROUTINE("batch_norm_grad_direct", BatchNormGradDirect, nullptr),
         ROUTINE("take_deferred", TakeDeferred, nullptr),

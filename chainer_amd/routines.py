@@ -1250,6 +1250,39 @@ def batch_norm_grad(x, gamma, gout, state, axis=None):
             gbeta.astype(beta_dtype, False).reshape(gamma.shape))
 
 
+def batch_norm_relu(x, gamma, beta, running_mean, running_var, eps=2e-5, decay=0.9, axis=None, residual=None):
+    """relu(b), or relu(total) with total = add(b, residual), where b is what `batch_norm` returns: one kernel call, the same values.  An addition to the
+    reference's routines, for training loops that ask for it.  Returns (out, total or None, state)."""
+    if not COMPOSE_BATCH_NORM:
+        direct = _host.batch_norm_direct(x, gamma, beta, running_mean, running_var, eps, decay, axis, True, residual)
+        if direct is not None:
+            return direct
+    b, state = batch_norm(x, gamma, beta, running_mean, running_var, eps, decay, axis)
+    total = None if residual is None else add(b, residual)
+    return relu(b if total is None else total), total, state
+
+
+def batch_norm_relu_grad(x, gamma, beta, gout, state, axis=None):
+    """`batch_norm_grad` of `gout` where batch norm's result b is not below zero, the gradient of relu(b); b is computed again from x."""
+    x_mean, x_inv_std, beta_dtype = state
+    if not COMPOSE_BATCH_NORM:
+        direct = _host.batch_norm_grad_direct(x, gamma, gout, x_mean, x_inv_std, beta_dtype, axis, beta)
+        if direct is not None:
+            return direct
+    axes = _sorted_axes((0,) + tuple(range(2, x.ndim)) if axis is None else axis, x.ndim)
+    red_shape = tuple(1 if i in axes else d for i, d in enumerate(x.shape))
+    interm = x_mean.dtype
+    g, bt = gamma.reshape(red_shape).astype(interm, False), beta.reshape(red_shape).astype(interm, False)
+    b = add(multiply(multiply(subtract(x.astype(interm, False), x_mean), x_inv_std), g), bt).astype(x.dtype, False)
+    return batch_norm_grad(x, gamma, if_less_else(b, 0, 0, gout), state, axis)
+
+
+def add_relu_grad(x, g1, g2):
+    """if_less_else(x, 0, 0, add(g1, g2)), the gradient of relu(x) where two of its uses meet, in one kernel call where the arrays are alike."""
+    direct = _host.add_relu_grad_direct(x, g1, g2)
+    return if_less_else(x, 0, 0, add(g1, g2)) if direct is None else direct
+
+
 # True: pooling gradients run as the native backend's Im2Col / ArgMax / Col2Im composition instead of the dedicated kernels (tests
 # compare the two bit for bit).
 COMPOSE_POOL_GRADIENTS = False

@@ -178,6 +178,8 @@ int hipcx_if_greater_else_assa(const hipcx_array* x1, hipcx_scalar x2, hipcx_sca
                                const hipcx_array* out, void* stream);         /* IfGreaterElseASSAKernel misc.h:43 */
 int hipcx_if_greater_else_aaaa(const hipcx_array* x1, const hipcx_array* x2, const hipcx_array* pos, const hipcx_array* neg,
                                const hipcx_array* out, void* stream);         /* IfGreaterElseAAAAKernel misc.h:48 */
+/* out = x < 0 ? 0 : g1 + g2 (floating point): Add (CX/kernels/arithmetic.h) and Relu's gradient IfLessElse(x, 0, 0, g) in one pass, the sum rounded in between. */
+int hipcx_add_relu_grad(const hipcx_array* x, const hipcx_array* g1, const hipcx_array* g2, const hipcx_array* out, void* stream);
 
 /* ---- logic: CX/kernels/logic.h (inputs share one dtype, out is bool) ---- */
 int hipcx_equal(const hipcx_array* x1, const hipcx_array* x2, const hipcx_array* out, void* stream);          /* EqualKernel :9 */
@@ -523,6 +525,16 @@ int hipcx_batch_norm(const hipcx_array* x, const hipcx_array* gamma, const hipcx
 int hipcx_batch_norm_grad(const hipcx_array* x, const hipcx_array* gamma, const hipcx_array* gout, const hipcx_array* mean,
                           const hipcx_array* inv_std, const int8_t* axis, int naxis, const hipcx_array* gx, const hipcx_array* ggamma,
                           const hipcx_array* gbeta, void* workspace, size_t workspace_bytes, void* stream);
+/* The same with Relu behind it, for training loops that say so (the reference issues the kernels one by one): out = Relu(b), or Relu(total) with total = b + residual
+ * if residual is not null, where b is what hipcx_batch_norm writes; every value is rounded where the kernels' arrays would hold it.  The gradient takes gout of
+ * Relu(b) and gives what IfLessElse(b, 0, 0, gout) and hipcx_batch_norm_grad give; b is computed again.  residual, total: C-contiguous like x. */
+int hipcx_batch_norm_relu(const hipcx_array* x, const hipcx_array* gamma, const hipcx_array* beta, const hipcx_array* running_mean,
+                          const hipcx_array* running_var, hipcx_scalar eps, hipcx_scalar decay, const int8_t* axis, int naxis, const hipcx_array* residual,
+                          const hipcx_array* total, const hipcx_array* out, const hipcx_array* mean_out, const hipcx_array* inv_std_out, void* workspace,
+                          size_t workspace_bytes, void* stream);
+int hipcx_batch_norm_relu_grad(const hipcx_array* x, const hipcx_array* gamma, const hipcx_array* beta, const hipcx_array* gout, const hipcx_array* mean,
+                               const hipcx_array* inv_std, const int8_t* axis, int naxis, const hipcx_array* gx, const hipcx_array* ggamma,
+                               const hipcx_array* gbeta, void* workspace, size_t workspace_bytes, void* stream);
 
 /* ---- pooling: CX/kernels/pooling.h:29,83 (NCHW logical layout, any strides; x[N,C,d_1..d_n] with n values per window parameter:
  * the dedicated kernels are the 2-D ones, n = 1 runs them over an extent of one, n >= 3 a plain one-thread-per-output kernel with
