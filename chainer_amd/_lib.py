@@ -149,6 +149,7 @@ SIGNATURES = {
     'hipcx_greater': (_INT, [_A, _A, _A, _V]),
     'hipcx_greater_equal': (_INT, [_A, _A, _A, _V]),
     'hipcx_copy': (_INT, [_A, _A, _V]),
+    'hipcx_update_many': (_INT, [ctypes.POINTER(_A), ctypes.POINTER(_A), _S, ctypes.POINTER(_A), _INT, _V]),
     'hipcx_copy_many': (_INT, [ctypes.POINTER(_A), ctypes.POINTER(_A), _INT, _V]),
     'hipcx_fill': (_INT, [_A, _S, _V]),
     'hipcx_arange': (_INT, [_S, _S, _A, _V]),

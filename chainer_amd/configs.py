@@ -232,7 +232,7 @@ class DeviceTrainOps:
     def __init__(self, chx):
         self.c = chx
         for name in ('conv', 'relu', 'max_pool', 'average_pool', 'linear', 'log_softmax', 'exp', 'add', 'subtract', 'multiply', 'sum',
-                     'max_pool_grad', 'average_pool_grad', 'conv_transpose', 'dot', 'batch_norm_grad', 'batch_norm_relu_grad', 'add_relu_grad'):
+                     'max_pool_grad', 'average_pool_grad', 'conv_transpose', 'dot', 'batch_norm_grad', 'batch_norm_relu_grad', 'add_relu_grad', 'sgd_update'):
             setattr(self, name, getattr(chx, name))
         self.array = chx.array
         self.get = lambda a: a.get()
@@ -334,7 +334,10 @@ def resnet50_train_step(F, p, x, t, lr=0.01):
     # ---- SGD ----
     grads += [(p, 'fc_w', g_fc_w), (p, 'fc_b', g_fc_b)]
     params = [container if key is None else container[key] for container, key, _ in grads]
-    new = [F.subtract(old, F.scale(g.reshape(old.shape), lr)) for old, (_, _, g) in zip(params, grads)]
+    if hasattr(F, 'sgd_update'):
+        new = F.sgd_update(params, [g for _, _, g in grads], lr)
+    else:
+        new = [F.subtract(old, F.scale(g.reshape(old.shape), lr)) for old, (_, _, g) in zip(params, grads)]
     updates = {}
     for (container, key, _), a in zip(grads, new):
         if key is None:

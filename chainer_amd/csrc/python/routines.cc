@@ -1105,6 +1105,38 @@ HOST_FN(BatchNormGradDirect) {
     HOST_CATCH(nullptr);
 }
 
+// x - g * s for every array x and its g, which is taken in x's shape; None for other than float arrays of one dtype each.
+HOST_FN(SgdUpdate) {
+    HOST_TRY;
+    HOST_ARGS("sgd_update", 3, "params", "grads", "lr");
+    std::vector<Ref> xs = Sequence(arg[0]), gs = Sequence(arg[1]);
+    if (xs.size() != gs.size()) Raise(HIPCX_DIMENSION_ERROR, "sgd_update: one gradient per parameter is needed");
+    if (!IsScalar(arg[2])) Py_RETURN_NONE;
+    for (size_t i = 0; i < xs.size(); ++i) {
+        const Array *x = xs[i].arr(), *g = gs[i].arr();
+        if (!IsFloat(x->d.dtype) || g->d.dtype != x->d.dtype || Size(g) != Size(x)) Py_RETURN_NONE;
+    }
+    const hipcx_scalar lr = ToScalar(arg[2]);
+    Ref list(PyList_New(static_cast<Py_ssize_t>(xs.size())));
+    if (!list) throw PyError();
+    std::vector<Ref> keep(xs.size());
+    std::vector<hipcx_array> g_views(xs.size());
+    std::vector<const hipcx_array*> x_ptrs, g_ptrs, out_ptrs;
+    for (size_t i = 0; i < xs.size(); ++i) {
+        Array* x = xs[i].arr();
+        g_views[i] = Reshaped(gs[i].arr(), x->d.ndim, x->d.shape, &keep[i]);
+        Ref out = EmptyLike(x, x->d.dtype);
+        x_ptrs.push_back(&x->d);
+        g_ptrs.push_back(&g_views[i]);
+        out_ptrs.push_back(out.d());
+        PyList_SET_ITEM(list.get(), static_cast<Py_ssize_t>(i), out.release());
+    }
+    void* stream = Stream();
+    Call([&] { return hipcx_update_many(x_ptrs.data(), g_ptrs.data(), lr, out_ptrs.data(), static_cast<int>(xs.size()), stream); });
+    return list.release();
+    HOST_CATCH(nullptr);
+}
+
 // ---------------------------------------------------------------------------------------------
 // indexing
 // ---------------------------------------------------------------------------------------------
@@ -1344,6 +1376,7 @@ PyMethodDef kRoutines[] = {
         ROUTINE("average_pool_grad_2d", AveragePoolGrad2d, nullptr),
         ROUTINE("conv_grad_weight_2d", ConvGradWeight2d, nullptr),
         ROUTINE("conv_transpose_2d", ConvTranspose2d, nullptr),
+        ROUTINE("sgd_update_direct", SgdUpdate, nullptr),
         ROUTINE("add_relu_grad_direct", AddReluGrad, nullptr),
         ROUTINE("batch_norm_direct", BatchNormDirect, nullptr),
         ROUTINE("batch_norm_grad_direct", BatchNormGradDirect, nullptr),

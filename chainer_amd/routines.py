@@ -1283,6 +1283,14 @@ def add_relu_grad(x, g1, g2):
     return if_less_else(x, 0, 0, add(g1, g2)) if direct is None else direct
 
 
+def sgd_update(params, grads, lr):
+    """[p - g.reshape(p.shape) * lr for every parameter and its gradient], rounded like `multiply` and `subtract`, in one kernel call for up to 112 arrays of a
+    dtype: an addition to the reference's routines, whose optimizers issue two kernels per parameter (chainer/optimizers/sgd.py:39-57)."""
+    params, grads = list(params), list(grads)
+    direct = _host.sgd_update_direct(params, grads, lr)
+    return [subtract(p, multiply(g.reshape(p.shape), lr)) for p, g in zip(params, grads)] if direct is None else direct
+
+
 # True: pooling gradients run as the native backend's Im2Col / ArgMax / Col2Im composition instead of the dedicated kernels (tests
 # compare the two bit for bit).
 COMPOSE_POOL_GRADIENTS = False

@@ -190,6 +190,10 @@ int hipcx_greater_equal(const hipcx_array* x1, const hipcx_array* x2, const hipc
 /* ---- creation: CX/kernels/creation.h, misc.h ---- */
 int hipcx_copy(const hipcx_array* a, const hipcx_array* out, void* stream);                       /* CopyKernel creation.h:16 (dtype-casting) */
 int hipcx_copy_many(const hipcx_array* const* as, const hipcx_array* const* outs, int n, void* stream);  /* n copies, none of which reads what another writes */
+/* outs[i] = xs[i] - gs[i] * scale, i < n: the parameter updates of gradient descent, rounded to the arrays' (floating point) dtype after the product and after
+ * the difference like MultiplyASKernel and SubtractKernel (CX/kernels/arithmetic.h), float16 and float32 arrays in one launch for up to 112 of them.  No out may
+ * overlap another array of the call. */
+int hipcx_update_many(const hipcx_array* const* xs, const hipcx_array* const* gs, hipcx_scalar scale, const hipcx_array* const* outs, int n, void* stream);
 int hipcx_fill(const hipcx_array* out, hipcx_scalar value, void* stream);                         /* FillKernel misc.h:9 */
 int hipcx_arange(hipcx_scalar start, hipcx_scalar step, const hipcx_array* out, void* stream);    /* ArangeKernel creation.h:11 */
 

@@ -1,4 +1,4 @@
-"""Batch norm with Relu behind it and its gradient, and the sum of two gradients before Relu's: each against the routines that it stands
+"""Batch norm with Relu behind it and its gradient, the sum of two gradients before Relu's, and updates of many parameters: each against the routines that it stands
 for, bit for bit, in the layouts of the kernels that take a channel in registers, of those that do not, and of none."""
 import numpy as np
 import pytest
@@ -72,3 +72,24 @@ def test_add_relu_grad(dt):
         X, A, B = (chx.array(v) if order is None else chx.array(v).transpose(*order) for v in (x, a, b))
         same(chx.add_relu_grad(X, A, B), chx.if_less_else(X, 0, 0, chx.add(A, B)))
     same(chx.add_relu_grad(chx.array(x), chx.array(a[:, :1]), chx.array(b)), chx.if_less_else(chx.array(x), 0, 0, chx.add(chx.array(a[:, :1]), chx.array(b))))
+
+
+@pytest.mark.parametrize('sizes', [[1], [0, 7, 8, 9], [255 * 8 + 3, 256 * 8, 4096 * 8 + 1], list(range(1, 240)), [5 << 20, 3, (6 << 20) + 5]])
+def test_sgd_update(sizes):
+    rng = np.random.default_rng(len(sizes))
+    for dts in (['float16'], ['float32'], ['float16', 'float32', 'float64']):
+        ps, gs = [], []
+        for i, n in enumerate(sizes):
+            dt = dts[i % len(dts)]
+            wide = chx.array(rng.standard_normal(n + 3).astype(dt))
+            ps.append(wide[i % 3:i % 3 + n])  # starts at any element
+            gs.append(chx.array(rng.standard_normal((1, n)).astype(dt)))
+        for lr in (0.01, 2):
+            for p, g, got in zip(ps, gs, chx.sgd_update(ps, gs, lr)):
+                same(got, chx.subtract(p, chx.multiply(g.reshape(p.shape), lr)))
+    # other layouts and types that promote
+    p, g = chx.array(rng.standard_normal((40, 30)).astype('float16')).T, chx.array(rng.standard_normal((30, 40)).astype('float16'))
+    same(chx.sgd_update([p], [g], 0.5)[0], chx.subtract(p, chx.multiply(g, 0.5)))
+    same(chx.sgd_update([p], [g.astype('float32')], 0.5)[0], chx.subtract(p, chx.multiply(g.astype('float32'), 0.5)))
+    with pytest.raises(chx.DimensionError):
+        chx.sgd_update([p], [g, g], 0.5)
