@@ -15,6 +15,7 @@
 #include "igemm_split.h"
 #include "launch_profile.h"
 #include "layout_kernels.h"
+#include "mid_conv.h"
 #include "nchw_conv.h"
 #include "pw_conv.h"
 #include "small_conv.h"
@@ -687,6 +688,7 @@ void RunNchw(const hipcx_array* x, const hipcx_array* w, const hipcx_array* b, c
     double flops = 2.0 * a.M * a.K * RS * a.C;
     double bytes = 2.0 * (static_cast<double>(a.N) * a.C * a.H * a.W + static_cast<double>(a.K) * RS * a.C + static_cast<double>(a.M) * a.K);
     ProfileScope prof(stream, flops, bytes);
+    if (MidConvTakes(a, pl.taps)) return MidConv(a, stream);
     const int key = (pl.ksplit - 1) * 1000000 + (pl.ck / 16) * 100000 + pl.taps * 10000 + pl.wpx * 1000 + pl.wch * 100 + pl.npx * 10 + pl.maxi;
     // single-pixel 1x1 kernels exist with and without dword loads
 #define HIPCX_NCHW_LAUNCH(TAPS, WPX, WCH, CK, NPX, MAXI, KSPLIT)                                          \
@@ -1168,7 +1170,10 @@ int hipcx_conv_route(const hipcx_array* x, const hipcx_array* w, const hipcx_arr
         if (x == nullptr || w == nullptr || out == nullptr || stride == nullptr || pad == nullptr) return -1;
         if (x->ndim != 4 || w->ndim != 4 || out->ndim != 4) return -1;
         if (PlanPw(x, w, b, out, stride, pad).ok) return 3;
-        if (const NchwPlan pl = PlanNchw(x, w, out, stride, pad); pl.ok) return SmallConvTakes(NchwExtents(x, w, out, stride), pl.taps) ? 4 : 1;
+        if (const NchwPlan pl = PlanNchw(x, w, out, stride, pad); pl.ok) {
+            const NchwConvArgs a = NchwExtents(x, w, out, stride);
+            return SmallConvTakes(a, pl.taps) ? 4 : MidConvTakes(a, pl.taps) ? 7 : 1;
+        }
         if (PlanStem(x, w, out, stride, pad).ok) return 2;
         if (ThinConvTakes(x, w, stride, pad, out)) return 5;
         return DirectConvTakes(x, w, stride, pad, out) ? 6 : 0;

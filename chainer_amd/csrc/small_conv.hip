@@ -10,6 +10,8 @@
 // 1024 -> 256 at 14^2 13.0 -> 5.4, 2048 -> 512 at 7^2 29.9 -> 11.9, 1024 -> 2048 at 14^2 with stride 2 18.6 -> 8.0.
 #include <algorithm>
 
+#include "mid_conv.h"
+#include "pixel_pairs.h"
 #include "small_conv.h"
 #include "small_dot.h"
 
@@ -25,13 +27,6 @@ constexpr int kRow1 = 32 * 2 + 16;
 // 3x3: a filter's 16 channels x 9 taps; a pixel's 16 channels.
 constexpr int kFilter3 = 16 * 9 * 2, kRow3 = kFilter3 + 16, kPixel3 = 32;
 
-// Halves `sel` of {hi, lo}: the low or high half of lo first, then of hi.
-template <bool LO_HIGH, bool HI_HIGH>
-__device__ __forceinline__ unsigned PickHalves(unsigned lo, unsigned hi) {
-    constexpr unsigned sel = (LO_HIGH ? 0x0302u : 0x0100u) | ((HI_HIGH ? 0x0706u : 0x0504u) << 16);
-    return __builtin_amdgcn_perm(hi, lo, sel);
-}
-
 struct SmallConvArgs {
     NchwConvArgs c;
     int nw;
@@ -39,15 +34,6 @@ struct SmallConvArgs {
     int pairs;     // 3x3: pairs of pixels in a patch
     int wave_lds;
 };
-
-// The two pixels' 16-byte groups of 8 channels from 8 dwords, one channel's pair of pixels each.
-__device__ __forceinline__ void TurnPairs(const unsigned (&v)[8], Bytes16& first, Bytes16& second) {
-#pragma unroll
-    for (int d = 0; d < 4; ++d) {
-        first[d] = PickHalves<false, false>(v[2 * d], v[2 * d + 1]);
-        second[d] = PickHalves<true, true>(v[2 * d], v[2 * d + 1]);
-    }
-}
 
 // SINGLE (1x1): pixels are loaded one by one, as planes of an odd size and strides above 1 ask for.
 template <int TAPS, bool SINGLE>
@@ -281,10 +267,13 @@ SmallConvArgs Plan(const NchwConvArgs& a, int taps) {
 // batch this small): up to 1.5 + C / 300 to a compute unit for 3x3 filters, 1.6 for strides above 1, 2 for odd planes, 2 + 110 / C else.  us, large tiles
 // and this kernel, around the lines: 3x3 64 channels at 56^2 392 workgroups 14.4 and 8.5, 784 14.5 and 15.2; 256 at 14^2 448 23.4 and 17.3, 672 23.8 and
 // 24.9; 512 at 7^2 768 51 and 33; 1x1 1024 -> 256 at 14^2 448 14.2 and 10.1, 672 14.2 and 16.4; 64 -> 64 at 56^2 784 5.1 and 4.8, 1568 5.3 and 5.8;
-// 2048 -> 512 at 7^2 512 33.5 and 23.8, 768 33.6 and 37.5; stride 2, 256 -> 512 at 56^2 400 7.5 and 5.9, 512 -> 256 at 28^2 448 10.7 and 13.9.
+// (for 3x3 the first figure is what NchwConvKernel takes; beyond one workgroup to a compute unit MidConvKernel is faster than both, us, this kernel and that:
+// 512 channels at 7^2 256 12.8 and 18.1, 384 22.0 and 18.7; 256 at 14^2 224 10.0 and 13.0, 336 17.4 and 13.2; 128 at 28^2 200 7.9 and 10.4, 400 13.7 and
+// 10.5; 64 at 56^2 392 8.9 and 9.7.)  1x1 2048 -> 512 at 7^2 512 33.5 and 23.8, 768 33.6 and 37.5; stride 2, 256 -> 512 at 56^2 400 7.5 and 5.9, 512 -> 256 at 28^2 448 10.7 and 13.9.
 bool SmallConvTakes(const NchwConvArgs& a, int taps) {
     const double groups = static_cast<double>((a.P + 31) / 32) * a.N * ((a.K + 31) / 32) / NumCUs();
     if (taps == 9) {
+        if (MidConvTakes(a, taps) && groups > (a.C < 128 ? 1.6 : 1.0)) return false;
         return groups <= 1.5 + a.C / 300.0 && PatchPairs(a) * 2 <= 4 * 64 && a.H * a.W >= 2;  // the patch of a tile is loaded in four passes at most
     }
     return groups <= (a.stride > 1 ? 1.6 : (a.P % 2 != 0 ? 2.0 : 2.0 + 110.0 / a.C));

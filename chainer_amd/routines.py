@@ -752,8 +752,8 @@ def _spatial_out(x, n, c, h, w, dtype):
 def conv_route(x, w, b=None, stride=1, pad=0, cover_all=False):
     """Which kernel family `conv` runs for these arguments (hipcx_conv_route): 0 general implicit GEMM, 1 float16 NCHW kernels
     with 128-wide tiles, 2 the 7x7 / 2 stem kernel, 3 the float16 1x1 kernel with LDS-direct operand loads, 4 the float16 kernel for
-    few output pixels, 5 the kernel for sums of at most 32 terms, 6 the float32 3x3 kernel for few output tiles.  For tests and benchmarks;
-    not part of the ChainerX routine surface."""
+    few output pixels, 5 the kernel for sums of at most 32 terms, 6 the float32 3x3 kernel for few output tiles, 7 the float16
+    3x3 kernel for a few hundred 64 x 64 tiles.  For tests and benchmarks; not part of the ChainerX routine surface."""
     stride, pad = _pair(stride), _pair(pad)
     dt = result_type(x, w, b) if b is not None else result_type(x, w)
     oh = conv_out_dim(x.shape[2], w.shape[2], stride[0], pad[0], cover_all)
@@ -1285,7 +1285,7 @@ def add_relu_grad(x, g1, g2):
 
 def sgd_update(params, grads, lr):
     """[p - g.reshape(p.shape) * lr for every parameter and its gradient], rounded like `multiply` and `subtract`, in one kernel call for up to 112 arrays of a
-    dtype: an addition to the reference's routines, whose optimizers issue two kernels per parameter (chainer/optimizers/sgd.py:39-57)."""
+    dtype: an addition to the reference's routines, whose optimizers issue two kernels per parameter (chainer/optimizers/sgd.py)."""
     params, grads = list(params), list(grads)
     direct = _host.sgd_update_direct(params, grads, lr)
     return [subtract(p, multiply(g.reshape(p.shape), lr)) for p, g in zip(params, grads)] if direct is None else direct
