@@ -560,6 +560,87 @@ __global__ __launch_bounds__(kRowThreads) void RowReduceKernel(ReduceGeom g, int
     }
 }
 
+// Rows of at most 4 * S * MAXI elements, one dense run each: S lanes to a row, which they hold in registers, 256 / S rows to a workgroup.  A workgroup to a row
+// (above) and a thread to a row (GenericReduceKernel, uncoalesced) are bounded by the starts of workgroups and by their loads.  The same tree: a lane's group of
+// four -> chunk (8 lanes) -> node (S lanes) of an iteration -> the aligned tree of the iterations' nodes.  Bytes bound the long ones, the
+// starts of workgroups and the tree's lane moves the short ones; sum/argmax of float32 in us, before and after: 64000 x 300 58/70 -> 15/19, 5775 x 122 19/21 -> 5/5.5,
+// 50000 x 1001 51/62 -> 32/35 (one read: 34 at 5.8 TB/s), 16000 x 2000 23.4/27.6 -> 22.5/26.2.
+constexpr int kShortRowIters = 8;
+template <typename Impl, int S>
+__global__ __launch_bounds__(256) void ShortRowReduceKernel(ReduceGeom g, int64_t row0, int iters) {
+    using R = typename Impl::Row;
+    using In = typename R::In;
+    using Acc = typename R::Acc;
+    using Op = ReduceOp<R, false>;
+    const int lane = threadIdx.x & 63, l = threadIdx.x % S, seg_lane = lane & 7;
+    const int64_t row = row0 + static_cast<int64_t>(blockIdx.x) * (256 / S) + threadIdx.x / S;
+    int64_t in_off, out_off;
+    OutOffsets(g, min(row, g.n_out - 1), in_off, out_off);
+    const In* const x = reinterpret_cast<const In*>(g.in + in_off);
+    const int L = static_cast<int>(g.red_len), G = L / 4, k_last = (G - 1) / 8;  // (G > 0)
+    Group4<In> q[kShortRowIters];
+#pragma unroll
+    for (int it = 0; it < kShortRowIters; ++it) {
+        if (it < iters) q[it] = LoadGroup(x + min(it * S + l, G - 1) * 4);
+    }
+    In rest[3];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) rest[j] = x[min(G * 4 + j, L - 1)];
+    Acc node[kShortRowIters];
+#pragma unroll
+    for (int it = 0; it < kShortRowIters; ++it) {
+        node[it] = R::Empty();
+        if (it >= iters) continue;
+        const int grp = it * S + l, chunk = grp >> 3, local = grp * 4;
+        Acc p0 = R::Map(q[it].v[0], local);
+        R::Reduce(R::Map(q[it].v[1], local + 1), p0);
+        Acc p1 = R::Map(q[it].v[2], local + 2);
+        R::Reduce(R::Map(q[it].v[3], local + 3), p1);
+        R::Reduce(p1, p0);
+        Acc gv = grp < G ? p0 : R::Empty();
+        Acc acc = R::Identity();
+        auto each = [&](auto&& f) {
+            f(std::integral_constant<int, 1>()), f(std::integral_constant<int, 2>()), f(std::integral_constant<int, 3>()), f(std::integral_constant<int, 4>());
+            f(std::integral_constant<int, 5>()), f(std::integral_constant<int, 6>()), f(std::integral_constant<int, 7>());
+        };
+        if constexpr (R::kSerialFold) {
+            R::Reduce(gv, acc);
+            each([&](auto j) { R::Reduce(FromLaneAbove<decltype(j)::value>(gv), acc); });
+        } else {
+            R::MaskLaterNan(gv, seg_lane == 0);
+            R::Reduce(gv, acc);
+            R::Reduce(FromLaneAbove<1>(acc), acc);
+            R::Reduce(FromLaneAbove<2>(acc), acc);
+            R::Reduce(FromLaneAbove<4>(acc), acc);
+        }
+        if (chunk == k_last) {  // it also folds the leftover elements, in order
+#pragma unroll
+            for (int j = 0; j < 3; ++j) {
+                if (G * 4 + j < L) R::Reduce(R::Map(rest[j], G * 4 + j), acc);
+            }
+        }
+        if (chunk > k_last) acc = R::Empty();
+        if constexpr (S >= 16) MergeLaneAbove<Op, 8>(acc);
+        auto merge_far = [&](int distance) {
+            Acc later = R::Shfl(acc, lane + distance);
+            R::Reduce(acc, later);
+            acc = later;
+        };
+        if constexpr (S >= 32) merge_far(16);
+        if constexpr (S >= 64) merge_far(32);
+        node[it] = acc;
+    }
+#pragma unroll
+    for (int s = 1; s < kShortRowIters; s <<= 1) {
+#pragma unroll
+        for (int i = 0; i < kShortRowIters; i += 2 * s) {
+            R::Reduce(node[i], node[i + s]);
+            node[i] = node[i + s];
+        }
+    }
+    if (row < g.n_out && l == 0) *reinterpret_cast<typename Impl::Out*>(g.out + out_off) = Impl::MapOut(Impl::FromRow(node[0], 0));
+}
+
 // second pass: tree over the per-block partials of each row (blocks_per_row <= kMaxPartials)
 template <typename Impl>
 __global__ __launch_bounds__(kRowThreads) void RowFinalizeKernel(ReduceGeom g, int64_t row0, int blocks_per_row, const void* partials) {
@@ -857,6 +938,7 @@ struct ReducePlan {
     bool row_path = false;
     int64_t span = 0;
     int blocks_per_row = 1;
+    int short_lanes = 0;  // row path: not 0: ShortRowReduceKernel with that many lanes to a row
     size_t acc_size = 0;
     bool column_path = false;
     int col_vec = 1;      // outputs per thread: 16 bytes of the innermost kept axis, or 1
@@ -968,6 +1050,17 @@ ReducePlan MakePlan(const hipcx_array* a, const int8_t* axis, int naxis, const h
             pl.blocks_per_row = static_cast<int>(bpr);
         }
     }
+    // Short rows: below 256 elements the other choice is a thread to a row, which is uncoalesced but needs no lanes to talk to each other: it is the faster one
+    // under 20 elements (200000 rows of 10 float32: 4.9 against 6.2 us; of 20: 11.3 against 6.2) unless the rows are too few for that to matter (5000 of 10: 3.4
+    // against 2.4).  From 256 on it is a workgroup to a row, which is ahead as long as rows leave compute units idle (333 rows of 1001: 3.1 against 3.3 us, argmax
+    // 3.7 against 5.2; 1000 of 500: 3.4 against 3.2, 3.9 against 3.8; 2000 of 1001: 4.4 against 3.6, 5.2 against 5.5).
+    const int lanes = g.red_len <= 8 * 4 * kShortRowIters ? 8 : g.red_len <= 32 * 4 * kShortRowIters ? 32 : 64;
+    if (one_run && g.red_len >= (g.n_out <= 8192 ? 8 : 20) && g.red_len <= 64 * 4 * kShortRowIters && g.n_out < (1LL << 31) &&
+        (g.red_len < 256 || g.n_out >= 32 * lanes)) {
+        pl.row_path = true;
+        pl.blocks_per_row = 1;
+        pl.short_lanes = lanes;
+    }
     // Column path: one strided reduced axis of at least a chunk (below that a thread per output reads its few rows itself).
     if (!pl.row_path && g.n_red == 1 && g.red_stride[0] != it && g.red_len >= 32 && g.n_out > 0 && g.n_out < (1LL << 28)) {
         const int64_t chunks = (g.red_len / 4 + 7) / 8;
@@ -1029,6 +1122,18 @@ void Run(const hipcx_array* a, const int8_t* axis, int naxis, const hipcx_array*
         HIPCX_REQUIRE(need == 0 || reinterpret_cast<uintptr_t>(workspace) % 16 == 0, HIPCX_CHAINERX_ERROR,
                       "workspace must be 16-byte aligned");
         const int64_t rows = std::max<int64_t>(1, kBlocksPerLaunch / pl.blocks_per_row);  // of one launch
+        if (pl.short_lanes > 0) {
+            const int64_t per_block = 256 / pl.short_lanes;
+            const int iters = static_cast<int>((g.red_len / 4 + pl.short_lanes - 1) / pl.short_lanes);
+            for (int64_t r0 = 0; r0 < g.n_out; r0 += kBlocksPerLaunch * per_block) {
+                const dim3 grid(static_cast<unsigned>(std::min(kBlocksPerLaunch, (g.n_out - r0 + per_block - 1) / per_block)));
+                if (pl.short_lanes == 8) hipLaunchKernelGGL((ShortRowReduceKernel<Impl, 8>), grid, dim3(256), 0, stream, g, r0, iters);
+                else if (pl.short_lanes == 32) hipLaunchKernelGGL((ShortRowReduceKernel<Impl, 32>), grid, dim3(256), 0, stream, g, r0, iters);
+                else hipLaunchKernelGGL((ShortRowReduceKernel<Impl, 64>), grid, dim3(256), 0, stream, g, r0, iters);
+                CheckLaunch("short_row_reduce");
+            }
+            return;
+        }
         for (int64_t r0 = 0; r0 < g.n_out; r0 += rows) {
             const int64_t count = std::min(rows, g.n_out - r0);
             const dim3 grid(static_cast<unsigned>(count * pl.blocks_per_row)), block(kRowThreads);
