@@ -71,59 +71,79 @@ struct alignas(sizeof(T) * V) Pack {
     T e[V];
 };
 
-// ---- LogSoftmax, rows that fit in registers: one workgroup per row, VPT packs of V elements per thread ----
+// 16 bytes at any address: rows of odd length start anywhere, and the hardware takes vector accesses there too.
+template <typename T, int V>
+__device__ __forceinline__ Pack<T, V> LoadPack(const T* p) {
+    Pack<T, V> v;
+    __builtin_memcpy(&v, p, sizeof(v));
+    return v;
+}
+template <typename T, int V>
+__device__ __forceinline__ void StorePack(T* p, const Pack<T, V>& v) {
+    __builtin_memcpy(p, &v, sizeof(v));
+}
+
+// ---- LogSoftmax, rows that fit in registers: a workgroup of 256 to a row, or a wave to each of four, VPT packs of 16 bytes per thread.  The row's last
+// pack moves back over its neighbour's elements, which are counted once and written twice with the same values: no access is conditional.
+// Bound by its bytes where rows are many: float32/float16 in us, rows taken element by element before, 64000 x 300 74/53 -> 31/31.5, 50000 x 1001 122/129 -> 73/43
+// (a read and a write: 69/35), 5398 x 1158 23.8 -> 14.7; by its start where they are few: 333 x 1001 3.1. ----
 template <typename T, int NT, int VPT>
-__global__ __launch_bounds__(NT) void LogSoftmaxRowKernel(const T* x, T* out, int64_t n, int64_t x_row, int64_t o_row, int vec_ok) {
+__global__ __launch_bounds__(256) void LogSoftmaxRowKernel(const T* x, T* out, int64_t rows, int n, int64_t x_row, int64_t o_row) {
     using C = compute_t<T>;
     constexpr int V = 16 / sizeof(T);
-    __shared__ C scratch[NT / 64];
-    const T* xr = x + static_cast<int64_t>(blockIdx.x) * x_row;
-    T* orow = out + static_cast<int64_t>(blockIdx.x) * o_row;
-    C v[VPT][V];
-    const C lowest = -INFINITY;
-    C m = lowest;
-#pragma unroll
-    for (int i = 0; i < VPT; ++i) {
-        const int64_t e0 = (static_cast<int64_t>(i) * NT + threadIdx.x) * V;
-        if (vec_ok && e0 + V <= n) {
-            Pack<T, V> p = *reinterpret_cast<const Pack<T, V>*>(xr + e0);
-#pragma unroll
-            for (int j = 0; j < V; ++j) v[i][j] = static_cast<C>(p.e[j]);
+    __shared__ C scratch[4];
+    const int t = threadIdx.x % NT;
+    const int64_t row = static_cast<int64_t>(blockIdx.x) * (256 / NT) + threadIdx.x / NT;
+    if (NT == 64 && row >= rows) return;  // a whole wave
+    auto reduce = [&](C v, auto is_max) {
+        constexpr bool MAX = decltype(is_max)::value;
+        if constexpr (NT == 256) {
+            return BlockReduce<C, 256, MAX>(v, scratch);
         } else {
 #pragma unroll
-            for (int j = 0; j < V; ++j) v[i][j] = e0 + j < n ? static_cast<C>(xr[e0 + j]) : lowest;
+            for (int d = 32; d >= 1; d >>= 1) {
+                const C o = static_cast<C>(__shfl_xor(v, d, 64));
+                v = MAX ? MaxNan(v, o) : v + o;
+            }
+            return v;
         }
-#pragma unroll
-        for (int j = 0; j < V; ++j) {
-            if (e0 + j < n) m = MaxNan(m, v[i][j]);
-        }
-    }
-    m = BlockReduce<C, NT, true>(m, scratch);
-    C s = 0;
+    };
+    const T* xr = x + row * x_row;
+    T* orow = out + row * o_row;
+    Pack<T, V> v[VPT];
+    int at[VPT], skip[VPT];  // of a pack, elements of the one in front
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
-        const int64_t e0 = (static_cast<int64_t>(i) * NT + threadIdx.x) * V;
+        const int e0 = (i * NT + t) * V;
+        at[i] = min(e0, n - V);
+        skip[i] = e0 - at[i];
+        v[i] = LoadPack<T, V>(xr + at[i]);
+    }
+    C m = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < VPT; ++i)
 #pragma unroll
         for (int j = 0; j < V; ++j) {
-            if (e0 + j < n) s += ExpOf<C>(v[i][j] - m);
+            if (j >= skip[i]) m = MaxNan(m, static_cast<C>(v[i].e[j]));
         }
-    }
-    s = BlockReduce<C, NT, false>(s, scratch);
+    m = reduce(m, std::true_type{});
+    C s = 0;
+#pragma unroll
+    for (int i = 0; i < VPT; ++i)
+#pragma unroll
+        for (int j = 0; j < V; ++j) {
+            const C e = ExpOf<C>(static_cast<C>(v[i].e[j]) - m);
+            s += j >= skip[i] ? e : C(0);
+        }
+    s = reduce(s, std::false_type{});
     const C lse = m + LogOf<C>(s);
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
-        const int64_t e0 = (static_cast<int64_t>(i) * NT + threadIdx.x) * V;
-        if (vec_ok && e0 + V <= n) {
-            Pack<T, V> p;
+        if (skip[i] >= V) continue;
+        Pack<T, V> p;
 #pragma unroll
-            for (int j = 0; j < V; ++j) p.e[j] = static_cast<T>(v[i][j] - lse);
-            *reinterpret_cast<Pack<T, V>*>(orow + e0) = p;
-        } else {
-#pragma unroll
-            for (int j = 0; j < V; ++j) {
-                if (e0 + j < n) orow[e0 + j] = static_cast<T>(v[i][j] - lse);
-            }
-        }
+        for (int j = 0; j < V; ++j) p.e[j] = static_cast<T>(static_cast<C>(v[i].e[j]) - lse);
+        StorePack<T, V>(orow + at[i], p);
     }
 }
 
@@ -167,36 +187,33 @@ __global__ __launch_bounds__(256) void LogSoftmaxShortRowKernel(const T* x, T* o
 // segments, then rewrites its own segment ----
 constexpr int kSegThreads = 256;
 
-// A segment is walked in packs of 16 bytes when rows start on 16-byte boundaries (seg_len is a multiple of the pack size).
+// A segment in packs of 16 bytes, wherever it starts, its last elements one by one.
 template <typename T, typename F>
-__device__ __forceinline__ void ForSegment(const T* xr, int64_t lo, int64_t hi, int vec_ok, F&& f) {
+__device__ __forceinline__ void ForSegment(const T* xr, int64_t lo, int64_t hi, F&& f) {
     constexpr int V = 16 / sizeof(T);
-    if (vec_ok) {
-        const int64_t full = lo + (hi - lo) / V * V;
-        for (int64_t e = lo + static_cast<int64_t>(threadIdx.x) * V; e < full; e += kSegThreads * V) {
-            Pack<T, V> p = *reinterpret_cast<const Pack<T, V>*>(xr + e);
+    const int64_t full = lo + (hi - lo) / V * V;
+#pragma unroll 4
+    for (int64_t e = lo + static_cast<int64_t>(threadIdx.x) * V; e < full; e += kSegThreads * V) {
+        const Pack<T, V> p = LoadPack<T, V>(xr + e);
 #pragma unroll
-            for (int j = 0; j < V; ++j) f(e + j, p.e[j]);
-        }
-        for (int64_t e = full + threadIdx.x; e < hi; e += kSegThreads) f(e, xr[e]);
-    } else {
-        for (int64_t e = lo + threadIdx.x; e < hi; e += kSegThreads) f(e, xr[e]);
+        for (int j = 0; j < V; ++j) f(p.e[j]);
     }
+    for (int64_t e = full + threadIdx.x; e < hi; e += kSegThreads) f(xr[e]);
 }
 
 template <typename T>
 __global__ __launch_bounds__(kSegThreads) void LogSoftmaxPartialKernel(const T* x, compute_t<T>* part, int64_t n, int64_t x_row, int64_t seg_len,
-                                                                       int nseg, int vec_ok) {
+                                                                       int nseg) {
     using C = compute_t<T>;
     __shared__ C scratch[kSegThreads / 64];
     const int row = blockIdx.x / nseg, seg = blockIdx.x - row * nseg;
     const T* xr = x + static_cast<int64_t>(row) * x_row;
     const int64_t lo = seg * seg_len, hi = min(n, lo + seg_len);
     C m = -INFINITY;
-    ForSegment<T>(xr, lo, hi, vec_ok, [&](int64_t, T v) { m = MaxNan(m, static_cast<C>(v)); });
+    ForSegment<T>(xr, lo, hi, [&](T v) { m = MaxNan(m, static_cast<C>(v)); });
     m = BlockReduce<C, kSegThreads, true>(m, scratch);
     C s = 0;
-    ForSegment<T>(xr, lo, hi, vec_ok, [&](int64_t, T v) { s += ExpOf<C>(static_cast<C>(v) - m); });  // second walk hits L2
+    ForSegment<T>(xr, lo, hi, [&](T v) { s += ExpOf<C>(static_cast<C>(v) - m); });  // second walk hits L2
     s = BlockReduce<C, kSegThreads, false>(s, scratch);
     // a segment of -inf only: its terms are exp(-inf - rowmax) = 0 unless the whole row is -inf (then 0 * exp(NaN) = NaN below,
     // which is what the chain gives for such a row)
@@ -209,7 +226,7 @@ __global__ __launch_bounds__(kSegThreads) void LogSoftmaxPartialKernel(const T* 
 
 template <typename T>
 __global__ __launch_bounds__(kSegThreads) void LogSoftmaxApplyKernel(const T* x, T* out, const compute_t<T>* part, int64_t n, int64_t x_row,
-                                                                     int64_t o_row, int64_t seg_len, int nseg, int vec_ok) {
+                                                                     int64_t o_row, int64_t seg_len, int nseg) {
     using C = compute_t<T>;
     constexpr int V = 16 / sizeof(T);
     __shared__ C scratch[kSegThreads / 64];
@@ -228,18 +245,15 @@ __global__ __launch_bounds__(kSegThreads) void LogSoftmaxApplyKernel(const T* x,
     const T* xr = x + static_cast<int64_t>(row) * x_row;
     T* orow = out + static_cast<int64_t>(row) * o_row;
     const int64_t lo = seg * seg_len, hi = min(n, lo + seg_len);
-    if (vec_ok) {
-        const int64_t full = lo + (hi - lo) / V * V;
-        for (int64_t e = lo + static_cast<int64_t>(threadIdx.x) * V; e < full; e += kSegThreads * V) {
-            Pack<T, V> p = *reinterpret_cast<const Pack<T, V>*>(xr + e);
+    const int64_t full = lo + (hi - lo) / V * V;
+#pragma unroll 4
+    for (int64_t e = lo + static_cast<int64_t>(threadIdx.x) * V; e < full; e += kSegThreads * V) {
+        Pack<T, V> p = LoadPack<T, V>(xr + e);
 #pragma unroll
-            for (int j = 0; j < V; ++j) p.e[j] = static_cast<T>(static_cast<C>(p.e[j]) - lse);
-            *reinterpret_cast<Pack<T, V>*>(orow + e) = p;
-        }
-        for (int64_t e = full + threadIdx.x; e < hi; e += kSegThreads) orow[e] = static_cast<T>(static_cast<C>(xr[e]) - lse);
-    } else {
-        for (int64_t e = lo + threadIdx.x; e < hi; e += kSegThreads) orow[e] = static_cast<T>(static_cast<C>(xr[e]) - lse);
+        for (int j = 0; j < V; ++j) p.e[j] = static_cast<T>(static_cast<C>(p.e[j]) - lse);
+        StorePack<T, V>(orow + e, p);
     }
+    for (int64_t e = full + threadIdx.x; e < hi; e += kSegThreads) orow[e] = static_cast<T>(static_cast<C>(xr[e]) - lse);
 }
 
 constexpr int64_t kRowInRegisters = 16384 * 4;  // bytes of a row the register kernel holds (256 threads x 16 packs x 16 bytes)
@@ -267,49 +281,82 @@ LsmShape CheckLogSoftmax(const hipcx_array* x, const hipcx_array* out) {
 // these take several launches, each of them far longer than its start.
 constexpr int64_t kRowsPerLaunch = int64_t{1} << 21;
 
+// Elements of a segment of rows of n: rows that are few are cut into more of them, two workgroups to a compute unit, of at least 16 KiB: a row of
+// 64 KiB segments kept one compute unit busy for each (7 x 70001 float32: 33 us, 9.5 now; 3 x 1000000: 19.5, 13.3; 100000: 16.3, 9.3).
+int64_t LogSoftmaxSegment(int64_t rows, int64_t n, int64_t it) {
+    const int64_t want = std::max<int64_t>(1, 2 * NumCUs() / rows), most = kSegmentBytes / it, least = kSegmentBytes / 4 / it;
+    return std::min(most, std::max(least, ((n + want - 1) / want + 15) / 16 * 16));
+}
+// Whether rows go through segments: those beyond a workgroup's registers, and 16-bit ones as long as these in elements that are too few to occupy the chip
+// (20 x 30000 float16: 8.9 us, 12.8 in registers; 37 x 20011: 9.8 and 10.3; 64 x 16000: 11.1 and 9.1).
+bool LogSoftmaxInSegments(int64_t rows, int64_t n, int64_t it) {
+    return n * it > kRowInRegisters || (rows <= 64 && n > kRowInRegisters / 4);
+}
+
 template <typename T>
 void RunLogSoftmax(const T* xp, T* op, const LsmShape& sh, void* workspace, size_t workspace_bytes, hipStream_t stream) {
     constexpr int V = 16 / sizeof(T);
-    const int vec_ok = reinterpret_cast<uintptr_t>(xp) % 16 == 0 && reinterpret_cast<uintptr_t>(op) % 16 == 0 && sh.x_row % V == 0 && sh.o_row % V == 0;
+    constexpr int64_t it = sizeof(T);
     const int64_t packs = (sh.n + V - 1) / V;
-    const unsigned rows = static_cast<unsigned>(sh.rows);
     auto short_rows = [&](auto lpr) {
         constexpr int LPR = decltype(lpr)::value;
         const int64_t blocks = (sh.rows + 256 / LPR - 1) / (256 / LPR);
         hipLaunchKernelGGL((LogSoftmaxShortRowKernel<T, LPR>), dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, xp, op, sh.rows,
                            static_cast<int>(sh.n), sh.x_row, sh.o_row);
     };
+    auto rows = [&](auto threads, auto per_thread) {
+        constexpr int NT = decltype(threads)::value, VPT = decltype(per_thread)::value;
+        const int64_t blocks = (sh.rows + 256 / NT - 1) / (256 / NT);
+        hipLaunchKernelGGL((LogSoftmaxRowKernel<T, NT, VPT>), dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, xp, op, sh.rows, static_cast<int>(sh.n),
+                           sh.x_row, sh.o_row);
+    };
+    auto segments = [&](int64_t seg_len) { return (sh.n + seg_len - 1) / seg_len; };
+    auto bytes = [&](int64_t nseg) { return static_cast<size_t>(sh.rows * nseg) * 2 * sizeof(compute_t<T>); };
+    int64_t seg_len = LogSoftmaxSegment(sh.rows, sh.n, it);
+    bool cut = LogSoftmaxInSegments(sh.rows, sh.n, it);
+    if (cut && (workspace == nullptr || workspace_bytes < bytes(segments(seg_len)))) {  // the fewest that do, then
+        seg_len = kSegmentBytes / it;
+        cut = sh.n * it > kRowInRegisters;
+    }
+    using std::integral_constant;
+    const bool many = sh.rows >= 2048;  // workgroups of four waves to a row otherwise (3000 x 1000: 6.2 us, 7.0 with them; 1500 x 2000: 7.1, 6.4)
     // up to four elements to a lane: beyond 128 of them a row fills a wave with 16-byte loads
     if (sh.n <= 16) {
-        short_rows(std::integral_constant<int, 4>{});
+        short_rows(integral_constant<int, 4>{});
     } else if (sh.n <= 64) {
-        short_rows(std::integral_constant<int, 16>{});
+        short_rows(integral_constant<int, 16>{});
     } else if (sh.n <= 128) {
-        short_rows(std::integral_constant<int, 32>{});
-    } else if (packs <= 64) {
-        hipLaunchKernelGGL((LogSoftmaxRowKernel<T, 64, 1>), dim3(rows), dim3(64), 0, stream, xp, op, sh.n, sh.x_row, sh.o_row, vec_ok);
-    } else if (packs <= 256) {
-        hipLaunchKernelGGL((LogSoftmaxRowKernel<T, 256, 1>), dim3(rows), dim3(256), 0, stream, xp, op, sh.n, sh.x_row, sh.o_row, vec_ok);
-    } else if (packs <= 256 * 4) {
-        hipLaunchKernelGGL((LogSoftmaxRowKernel<T, 256, 4>), dim3(rows), dim3(256), 0, stream, xp, op, sh.n, sh.x_row, sh.o_row, vec_ok);
-    } else if (packs <= 256 * 10) {
-        hipLaunchKernelGGL((LogSoftmaxRowKernel<T, 256, 10>), dim3(rows), dim3(256), 0, stream, xp, op, sh.n, sh.x_row, sh.o_row, vec_ok);
-    } else if (packs <= 256 * 16) {
-        hipLaunchKernelGGL((LogSoftmaxRowKernel<T, 256, 16>), dim3(rows), dim3(256), 0, stream, xp, op, sh.n, sh.x_row, sh.o_row, vec_ok);
-    } else {
-        const int64_t seg_len = kSegmentBytes / static_cast<int64_t>(sizeof(T));
-        const int64_t nseg = (sh.n + seg_len - 1) / seg_len;
+        short_rows(integral_constant<int, 32>{});
+    } else if (cut) {
+        const int64_t nseg = segments(seg_len);
         HIPCX_REQUIRE(sh.rows * nseg < (1LL << 31), HIPCX_NOT_IMPLEMENTED_ERROR, "log_softmax: problem too large for one launch");
-        const size_t need = static_cast<size_t>(sh.rows * nseg) * 2 * sizeof(compute_t<T>);
+        const size_t need = bytes(nseg);
         HIPCX_REQUIRE(workspace != nullptr && workspace_bytes >= need, HIPCX_CHAINERX_ERROR,
                       "log_softmax: workspace of " + std::to_string(need) + " bytes required");
         auto* part = static_cast<compute_t<T>*>(workspace);
         const unsigned blocks = static_cast<unsigned>(sh.rows * nseg);
-        hipLaunchKernelGGL(LogSoftmaxPartialKernel<T>, dim3(blocks), dim3(kSegThreads), 0, stream, xp, part, sh.n, sh.x_row, seg_len,
-                           static_cast<int>(nseg), vec_ok);
+        hipLaunchKernelGGL(LogSoftmaxPartialKernel<T>, dim3(blocks), dim3(kSegThreads), 0, stream, xp, part, sh.n, sh.x_row, seg_len, static_cast<int>(nseg));
         CheckLaunch("log_softmax_partial");
         hipLaunchKernelGGL(LogSoftmaxApplyKernel<T>, dim3(blocks), dim3(kSegThreads), 0, stream, xp, op, part, sh.n, sh.x_row, sh.o_row, seg_len,
-                           static_cast<int>(nseg), vec_ok);
+                           static_cast<int>(nseg));
+    } else if (packs <= 64) {
+        rows(integral_constant<int, 64>{}, integral_constant<int, 1>{});
+    } else if (many && packs <= 128) {
+        rows(integral_constant<int, 64>{}, integral_constant<int, 2>{});
+    } else if (many && packs <= 256) {
+        rows(integral_constant<int, 64>{}, integral_constant<int, 4>{});
+    } else if (many && packs <= 512) {
+        rows(integral_constant<int, 64>{}, integral_constant<int, 8>{});
+    } else if (packs <= 256) {
+        rows(integral_constant<int, 256>{}, integral_constant<int, 1>{});
+    } else if (packs <= 256 * 2) {
+        rows(integral_constant<int, 256>{}, integral_constant<int, 2>{});
+    } else if (packs <= 256 * 4) {
+        rows(integral_constant<int, 256>{}, integral_constant<int, 4>{});
+    } else if (packs <= 256 * 10) {
+        rows(integral_constant<int, 256>{}, integral_constant<int, 10>{});
+    } else {
+        rows(integral_constant<int, 256>{}, integral_constant<int, 16>{});
     }
     CheckLaunch("log_softmax");
 }
@@ -704,8 +751,8 @@ extern "C" {
 size_t hipcx_log_softmax_workspace_size(const hipcx_array* x) {
     if (x == nullptr || x->ndim != 2 || !IsFloatDtype(x->dtype)) return 0;
     const int64_t it = ItemSize(x->dtype);
-    if (x->shape[1] * it <= kRowInRegisters) return 0;
-    const int64_t seg_len = kSegmentBytes / it;
+    if (x->shape[0] == 0 || !LogSoftmaxInSegments(x->shape[0], x->shape[1], it)) return 0;
+    const int64_t seg_len = LogSoftmaxSegment(x->shape[0], x->shape[1], it);
     const int64_t nseg = (x->shape[1] + seg_len - 1) / seg_len;
     return static_cast<size_t>(x->shape[0] * nseg) * 2 * (x->dtype == HIPCX_FLOAT64 ? 8 : 4);
 }

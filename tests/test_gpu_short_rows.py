@@ -1,9 +1,12 @@
-"""Reductions of short rows, several of which share a workgroup: bit for bit the oracle's tree."""
+"""Reductions and log-softmax of short rows: several rows to a workgroup, or a wave or workgroup that holds one in registers.
+
+Reductions are bit for bit the oracle's tree.  log-softmax is x - (m + log(sum exp(x - m))): the chain of the same type on the oracle differs by the rounding of
+its own steps, which the float tolerance of the other log-softmax tests covers."""
 import numpy as np
 import pytest
 
 from oracle import native as O
-from helpers import assert_exact
+from helpers import assert_close, assert_exact
 
 pytestmark = pytest.mark.gpu
 
@@ -38,3 +41,30 @@ def test_outputs_of_two_axes():
     X = chx.array(x)
     assert_exact(chx.sum(X, 2).get(), O.sum(x, 2), 'sum')
     assert_exact(chx.argmax(X[:, 3:90, 5:], 2).get(), O.argmax(x[:, 3:90, 5:], 2), 'argmax of a slice')
+
+
+@pytest.mark.parametrize('dt', ['float16', 'float32', 'float64'])
+@pytest.mark.parametrize('rows,n', [(5, 129), (2047, 255), (2048, 257), (2049, 511), (2050, 1023), (2048, 1025), (2051, 2047), (2048, 4095), (3, 4097), (70, 10241),
+                                    (64, 16385), (65, 16385), (1, 32769), (2, 70001)])
+def test_log_softmax(dt, rows, n):
+    import chainer_amd as chx
+    x = (np.random.default_rng(rows + n).standard_normal((rows, n + 1)) * 3).astype(dt)
+    x[rows // 2, n // 3] = 60000 if dt == 'float16' else 1e30
+    X = chx.array(x)
+    assert_close(chx.log_softmax_fused(X).get(), O.log_softmax(x, 1), None, 'rows')
+    x = x[:, 1:]
+    assert_close(chx.log_softmax_fused(X[:, 1:]).get(), O.log_softmax(x, 1), None, 'rows that start anywhere')
+
+
+def test_log_softmax_in_place_and_in_a_smaller_workspace():
+    import chainer_amd as chx
+    rng = np.random.default_rng(4)
+    for rows, n in ((2100, 1001), (3, 2001), (2, 20001), (1, 100003)):
+        x = rng.standard_normal((rows, n)).astype('float32')
+        X = chx.array(x)
+        ref = chx.log_softmax_fused(X).get()
+        need = -(-n // (64 * 1024 // 4)) * rows * 2 * 4 if n > 16384 else 0  # what segments of 64 KiB take
+        ws = chx.empty((max(need, 1),), 'uint8')
+        chx._lib.call('hipcx_log_softmax', X.desc(), X.desc(), ws.data_ptr if need else None, need, chx.routines.current_stream())
+        # other segments add the exponentials in another order: a few roundings of a sum, of which the logarithm is taken
+        assert_close(X.get(), ref, 1e-5, 'in place %d x %d' % (rows, n))
