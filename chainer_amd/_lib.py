@@ -195,6 +195,8 @@ SIGNATURES = {
     'hipcx_log_softmax_workspace_size': (_SZ, [_A]),
     'hipcx_log_softmax': (_INT, [_A, _A, _V, _SZ, _V]),
     'hipcx_lstm_cell': (_INT, [_A, _A, _A, _A, _V]),
+    'hipcx_lstm_step_supported': (_INT, [_A, _A, _A, _A, _A, _A]),
+    'hipcx_lstm_step': (_INT, [_A, _A, _A, _A, _A, _A, _A, _A, _V]),
     'hipcx_softmax_cross_entropy_workspace_size': (_SZ, [_A]),
     'hipcx_softmax_cross_entropy': (_INT, [_A, _A, _A, _V, _SZ, _V]),
     'hipcx_profile_start': (_INT, []),

@@ -418,8 +418,11 @@ def lstm_lm_forward(F, p, ids, zeros, take_mode=None, fused=False):
     for t in range(seq):
         x = F.take(p['embed'], ids[:, t], 0, take_mode)
         for li, layer in enumerate(p['layers']):
-            gates = F.add(F.linear(x, layer['up_w'], layer['up_b']), F.linear(hs[li], layer['lat_w']))
-            hs[li], cs[li] = lstm(cs[li], gates)
+            if hasattr(F, 'lstm_step'):
+                hs[li], cs[li] = F.lstm_step(cs[li], x, layer['up_w'], layer['up_b'], hs[li], layer['lat_w'])
+            else:
+                gates = F.add(F.linear(x, layer['up_w'], layer['up_b']), F.linear(hs[li], layer['lat_w']))
+                hs[li], cs[li] = lstm(cs[li], gates)
             x = hs[li]
         y = F.linear(x, p['out_w'], p['out_b'])
     return log_softmax(y, 1), hs, cs

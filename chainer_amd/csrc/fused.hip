@@ -10,6 +10,7 @@
 #include <algorithm>
 
 #include "common.h"
+#include "lstm_cell.h"
 
 namespace hipcx {
 namespace {
@@ -24,12 +25,6 @@ __device__ __forceinline__ C LogOf(C v) {
     if constexpr (std::is_same_v<C, float>) return logf(v);
     else return log(v);
 }
-template <typename C>
-__device__ __forceinline__ C TanhOf(C v) {
-    if constexpr (std::is_same_v<C, float>) return tanhf(v);
-    else return tanh(v);
-}
-
 // AMax's update (native/native_device/statistics.cc:27-48): NaN wins, otherwise strictly greater.
 template <typename C>
 __device__ __forceinline__ C MaxNan(C acc, C v) {
@@ -727,16 +722,8 @@ __global__ __launch_bounds__(256) void LstmCellKernel(const T* c, const T* x, T*
 #pragma unroll
         for (int k = 0; k < 4; ++k) g[k] = static_cast<C>(xg[k]);
     }
-    // Sigmoid as the routine composes it (CX/routines/activation.cc:74-78): Reciprocal(1 + Exp(-x)) with Reciprocal = 1 / x
-    auto sigmoid = [](C v) { return C(1) / (C(1) + ExpOf<C>(-v)); };
-    // (the float16 chain rounds after every kernel; here the values stay in float until the two stores)
-    const C a = TanhOf<C>(g[0]);
-    const C i = sigmoid(g[1]);
-    const C f = sigmoid(g[2]);
-    const C o = sigmoid(g[3]);
-    const C cprev = static_cast<C>(c[b * c_row + j]);
-    const C cn = a * i + f * cprev;
-    const C h = o * TanhOf<C>(cn);
+    C cn;
+    const C h = LstmCell<C>(g, static_cast<C>(c[b * c_row + j]), cn);
     c_out[b * co_row + j] = static_cast<T>(cn);
     h_out[b * h_row + j] = static_cast<T>(h);
 }

@@ -1227,6 +1227,21 @@ HOST_FN(LstmCell) {
     HOST_CATCH(nullptr);
 }
 
+// A step of an LSTM link through hipcx_lstm_step, or None for the calls to compose.
+HOST_FN(LstmStep) {
+    HOST_TRY;
+    HOST_ARGS("lstm_step", 6, "c", "x", "wx", "bx", "h", "wh");
+    Array *c = AsArray(arg[0], "c"), *x = AsArray(arg[1], "x"), *wx = AsArray(arg[2], "wx"), *bx = Given(arg[3]) ? AsArray(arg[3], "bx") : nullptr;
+    Array *h = AsArray(arg[4], "h"), *wh = AsArray(arg[5], "wh");
+    const hipcx_array* const bias = bx != nullptr ? &bx->d : nullptr;
+    if (hipcx_lstm_step_supported(&c->d, &x->d, &wx->d, bias, &h->d, &wh->d) == 0) Py_RETURN_NONE;
+    Ref new_h = EmptyLike(c, c->d.dtype), new_c = EmptyLike(c, c->d.dtype);
+    void* stream = Stream();
+    Call([&] { return hipcx_lstm_step(&c->d, &x->d, &wx->d, bias, &h->d, &wh->d, new_h.d(), new_c.d(), stream); });
+    return PyTuple_Pack(2, new_h.get(), new_c.get());
+    HOST_CATCH(nullptr);
+}
+
 // ---------------------------------------------------------------------------------------------
 // recurrent networks
 // ---------------------------------------------------------------------------------------------
@@ -1384,6 +1399,7 @@ PyMethodDef kRoutines[] = {
         ROUTINE("log_softmax_direct", LogSoftmaxDirect, nullptr),
         ROUTINE("softmax_cross_entropy_direct", SoftmaxCrossEntropyDirect, nullptr),
         ROUTINE("lstm_cell", LstmCell, nullptr),
+        ROUTINE("lstm_step_direct", LstmStep, nullptr),
         ROUTINE("rnn_forward", RnnForward, nullptr),
         ROUTINE("rnn_backward", RnnBackward, nullptr),
         {nullptr, nullptr, 0, nullptr}};

@@ -1441,6 +1441,13 @@ def lstm_fused(c, x):
     return lstm(c, x)
 
 
+def lstm_step(c, x, upward_w, upward_b, h, lateral_w):
+    """(h, c) of lstm(c, add(linear(x, upward_w, upward_b), linear(h, lateral_w))), a step of L.LSTM (chainer/links/rnn/lstm.py:119-144), in one kernel call where
+    the batch and the layer are of the sizes that gain by it."""
+    direct = _host.lstm_step_direct(c, x, upward_w, upward_b, h, lateral_w)
+    return lstm(c, add(linear(x, upward_w, upward_b), linear(h, lateral_w))) if direct is None else direct
+
+
 def clipped_relu(x, z):
     """ClippedRelu = Minimum(Maximum(0, x), z) (CX/routines/activation.cc:51-55)."""
     return minimum(maximum(x.astype(_math_result_dtype(x.dtype), False), 0), z)

@@ -419,6 +419,15 @@ int hipcx_n_step_rnn_backward(int n_layers, int bidirectional, int mode, int act
 size_t hipcx_log_softmax_workspace_size(const hipcx_array* x);
 int hipcx_log_softmax(const hipcx_array* x, const hipcx_array* out, void* workspace, size_t workspace_bytes, void* stream);
 int hipcx_lstm_cell(const hipcx_array* c, const hipcx_array* x, const hipcx_array* h_out, const hipcx_array* c_out, void* stream);
+/* hipcx_lstm_step: hipcx_lstm_cell of c and Linear(x, wx, bx) + Linear(h, wh), a step of the L.LSTM link
+ *   (chainer/links/rnn/lstm.py:119-144), in one launch.  c, h, h_out, c_out [B, H]; x [B, in]; wx [4H, in], wh [4H, H] with gate k of
+ *   unit j in row 4j+k; bx [4H] or NULL.  float32 and float16, the gates' sums in float or double, rounded once.  h_out shares no
+ *   memory with x or h; c_out may be c.  hipcx_lstm_step_supported: 1 for the calls that it takes (dense rows of 16 bytes or more,
+ *   sizes at which one launch is the faster way), 0 for those to compose. */
+int hipcx_lstm_step_supported(const hipcx_array* c, const hipcx_array* x, const hipcx_array* wx, const hipcx_array* bx, const hipcx_array* h,
+                              const hipcx_array* wh);
+int hipcx_lstm_step(const hipcx_array* c, const hipcx_array* x, const hipcx_array* wx, const hipcx_array* bx, const hipcx_array* h,
+                    const hipcx_array* wh, const hipcx_array* h_out, const hipcx_array* c_out, void* stream);
 /* hipcx_softmax_cross_entropy: F.softmax_cross_entropy for chainerx arrays (chainer/functions/loss/softmax_cross_entropy.py:123-130:
  *   LogSoftmax, a one-hot mask from Equal(t[:, None], Arange(n)), -sum(score * mask) / sum(mask); about 15 kernels) as one kernel, or
  *   two for large batches.  x [B, n] float, dense along axis 1; t [B], an integer dtype that can hold n - 1; out: one element of x's
