@@ -1,13 +1,14 @@
 // Matrix products with small outputs (batch-sized Linear layers, recurrent steps, weight gradients of small layers):
 // out[M,N] = a[M,K] . b[K,N] with so few elements that 128x128 tiles would occupy a handful of compute units.
 //
-// A workgroup owns one 32x32 tile of `out` (SmallDotLinesKernel: 16 to 64 columns, SmallDotColumnsKernel: 64x64); its waves split the reduction
+// A workgroup owns one 32x32 tile of `out` (SmallDotLinesKernel: 16 to 64 columns, SmallDotSquaresKernel: 64 x 32 to 64 x 80, SmallDotColumnsKernel: 64x64); its waves split the reduction
 // axis -- and, with ksplit > 1, so do several workgroups, whose sums another kernel adds up -- each feeding the MFMA from global memory on its own
-// (operands this small live in the caches), and the partial tiles are summed through LDS.  Five kernels, by where the operands lie (chosen in
+// (operands this small live in the caches), and the partial tiles are summed through LDS.  Six kernels, by where the operands lie (chosen in
 // LaunchSmallDot, the last one in PlanSmallDot):
 //   SmallDotKernel        k is the unit-stride axis of both operands (Linear's x and W^T): straight from global memory, bound by the
 //                         latency of a few loads.
 //   SmallDotLinesKernel   the same for more or longer tiles: whole 128-byte lines regrouped through LDS.
+//   SmallDotSquaresKernel the same once 64 rows to a tile fill the chip: whole lines into LDS that the waves share.
 //   SmallDotMixedKernel   an operand whose k axis is not the unit-stride one (dG . Wh of a recurrent network, x^T . gy), or float16 rows
 //                         of odd pitch.
 //   SmallDotColumnsKernel float32, both operands with m and n as the unit-stride axes, of outputs that make a 64 x 64 tile per compute unit.
@@ -411,6 +412,166 @@ __global__ __launch_bounds__(64 * kSmallDotMaxWaves) __attribute__((amdgpu_waves
         float s = 0.f;
         for (int w = 0; w < p.nw; ++w) s += part[w * kPart + row * kPitch + col];
         StoreTileElement<T>(p, split, out, om, on, s);
+    }
+}
+
+// Tiles of 64 rows and 16 * NB columns, both operands in pieces.  The eight waves take 32 rows each of a quarter of a chunk's k; chunks of 256 bytes per
+// row go through LDS that they share (two buffers, one barrier a chunk): while one is multiplied, the fragments of the next come out of LDS, the one after
+// goes there, and one more is on its way.  A chunk's products start from zero and are
+// added up by chunk, so that a chain is 16 terms: the error is half of that of tiles whose waves add up all of their terms ([128,650] . [650,10000] 1.07e-7 of the
+// norm, 2.68e-7; [670,3324] . [3324,2007] 1.6e-7, 7.3e-7).  Bound by the matrix pipe, 1.2 us of a chunk's 1.5 at five blocks, and by 5 us of launch, first loads
+// and sums; fragments read twice as often (16 rows to a wave) or what is not a product after the products, instead of between them, cost 3 us of 25.
+// Against SmallDotLinesKernel: float32 [128,650] . [650,10000] 28.1 -> 24.8 us (11.5 of matrix work), [1000,784] . [784,1000] 24.2 -> 22.3, float16
+// [1903,2408] . [2408,452] 28.6 -> 19.7.
+constexpr int kSquaresPitch = 256 + 16;  // bytes of a row in LDS: 16 rows' pieces start in different banks
+template <typename T, int NB>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void SmallDotSquaresKernel(SmallDotArgs p) {
+    constexpr int PL = 16 / sizeof(T);
+    constexpr int KC = 16 * PL;  // k per chunk
+    constexpr int kOut = 0x7fffffff;
+    constexpr int BL = (NB + 1) / 2;  // loads of b per chunk and thread, 32 rows each in all
+    constexpr int kStage = (64 + 32 * BL) * kSquaresPitch, kPitch = 16 * NB + 1;
+    extern __shared__ __align__(16) char lds[];
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lr = lane & 15, g = lane >> 4;
+    int tm, tn;
+    SmallDotTile(p.tiles_m * p.tiles_n, blockIdx.x, p.tiles_m, tm, tn);
+    const __amdgpu_buffer_rsrc_t ar = MakeRsrc(static_cast<const T*>(p.a), p.a_bytes);
+    const __amdgpu_buffer_rsrc_t br = MakeRsrc(p.b, p.b_bytes);
+    const int row_in = tid >> 4, k_in = (tid & 15) * PL;  // of this thread's loads
+    int a_line[2], b_line[BL];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const int m = tm * 64 + j * 32 + row_in;
+        a_line[j] = m < p.M ? static_cast<int>((m * p.a_row + k_in) * static_cast<int64_t>(sizeof(T))) : kOut;
+    }
+#pragma unroll
+    for (int j = 0; j < BL; ++j) {
+        const int row = j * 32 + row_in, n = tn * 16 * NB + row;
+        b_line[j] = row < 16 * NB && n < p.N ? static_cast<int>((n * p.b_col + k_in) * static_cast<int64_t>(sizeof(T))) : kOut;
+    }
+    char* const to = lds + row_in * kSquaresPitch + (tid & 15) * 16;
+    const int rows = wave & 1, quarter = wave >> 1;
+    const char* const from = lds + lr * kSquaresPitch + quarter * 64 + g * 16;
+
+    float4_t acc[2][NB], terms[2][NB];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) acc[i][j] = terms[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
+    const int chunks = (p.K + KC - 1) / KC;
+    Bytes16 av[2], bv[BL], fa[2][2], fb[2][NB];
+    auto load = [&](int c) {  // (pieces beyond K are not read)
+        const bool in = c * KC + k_in < p.K;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) av[j] = __builtin_amdgcn_raw_buffer_load_b128(ar, (in & (a_line[j] != kOut)) ? a_line[j] + c * 256 : kOut, 0, 0);
+#pragma unroll
+        for (int j = 0; j < BL; ++j) bv[j] = __builtin_amdgcn_raw_buffer_load_b128(br, (in & (b_line[j] != kOut)) ? b_line[j] + c * 256 : kOut, 0, 0);
+    };
+    auto store = [&](int c, auto whole) {
+        if (!decltype(whole)::value && (c + 1) * KC > p.K) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j) av[j] = MaskPiece<T>(av[j], c * KC + k_in, p.K);
+#pragma unroll
+            for (int j = 0; j < BL; ++j) bv[j] = MaskPiece<T>(bv[j], c * KC + k_in, p.K);
+        }
+        char* const at = to + (c & 1) * kStage;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) *reinterpret_cast<Bytes16*>(at + j * 32 * kSquaresPitch) = av[j];
+#pragma unroll
+        for (int j = 0; j < BL; ++j) *reinterpret_cast<Bytes16*>(at + (64 + j * 32) * kSquaresPitch) = bv[j];
+    };
+    auto read = [&](int st, int c) {
+        const char* const at = from + (c & 1) * kStage;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) fa[st][i] = *reinterpret_cast<const Bytes16*>(at + (rows * 32 + i * 16) * kSquaresPitch);
+#pragma unroll
+        for (int j = 0; j < NB; ++j) fb[st][j] = *reinterpret_cast<const Bytes16*>(at + (64 + j * 16) * kSquaresPitch);
+    };
+    // `whole`: c + 2 lies inside K
+    auto step = [&](auto parity, int c, auto whole) {
+        constexpr int S = decltype(parity)::value;
+        constexpr bool kWhole = decltype(whole)::value;
+        read(S ^ 1, c + 1);
+        store(c + 2, whole);
+        load(c + 3);
+        if (kWhole || c * KC + quarter * (KC / 4) < p.K) {
+#pragma unroll
+            for (int e = 0; e < (sizeof(T) == 4 ? 4 : 1); ++e)
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int j = 0; j < NB; ++j) {
+                        if (e == 0) {  // the chunk before's
+                            acc[i][j] += terms[i][j];
+                            terms[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
+                        }
+                        if constexpr (sizeof(T) == 4) {
+                            terms[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(fa[S][i][e]), __uint_as_float(fb[S][j][e]), terms[i][j], 0, 0, 0);
+                        } else {
+                            MfmaBlock<T>(fa[S][i], fb[S][j], terms[i][j]);
+                        }
+                    }
+        }
+        if constexpr (kWhole) {  // what is not a product goes between them, under the matrix pipe
+            constexpr int kProducts = sizeof(T) == 4 && NB >= 4 ? 2 : 1;
+#pragma unroll
+            for (int i = 0; i < 2 + NB; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x8, kProducts, 0);
+                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            }
+#pragma unroll
+            for (int i = 0; i < 2 + BL; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x8, kProducts, 0);
+                __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
+            }
+#pragma unroll
+            for (int i = 0; i < 2 + BL; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x8, kProducts, 0);
+                __builtin_amdgcn_sched_group_barrier(0x20, 1, 0);
+            }
+        }
+        __syncthreads();
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    load(0);
+    store(0, std::false_type{});
+    load(1);
+    __syncthreads();
+    read(0, 0);
+    store(1, std::false_type{});
+    load(2);
+    __syncthreads();
+    __builtin_amdgcn_sched_barrier(0);
+    int c = 0;
+    for (; (c + 4) * KC <= p.K; c += 2) {
+        step(std::integral_constant<int, 0>{}, c, std::true_type{});
+        step(std::integral_constant<int, 1>{}, c + 1, std::true_type{});
+    }
+    for (; c < chunks; c += 2) {
+        step(std::integral_constant<int, 0>{}, c, std::false_type{});
+        if (c + 1 < chunks) step(std::integral_constant<int, 1>{}, c + 1, std::false_type{});
+    }
+    // lane holds column lr, rows 4 * g + v of each block
+    constexpr int kPart = 64 * kPitch;
+    float* const part = reinterpret_cast<float*>(lds);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) part[quarter * kPart + (rows * 32 + i * 16 + 4 * g + v) * kPitch + j * 16 + lr] = acc[i][j][v] + terms[i][j][v];
+    __syncthreads();
+    T* const out = static_cast<T*>(p.out);
+    for (int e = tid; e < 64 * 16 * NB; e += 512) {
+        const int row = e / (16 * NB), col = e - row * (16 * NB);
+        const int om = tm * 64 + row, on = tn * 16 * NB + col;
+        if (om >= p.M || on >= p.N) continue;
+        const float* const s = part + row * kPitch + col;
+        StoreDot<T>(p, out, om, on, (s[0] + s[kPart]) + (s[2 * kPart] + s[3 * kPart]));
     }
 }
 

@@ -128,6 +128,31 @@ int LinesWaves(int64_t groups, int chunks, bool half) {
     return std::min(best, chunks);
 }
 
+// Columns, in 16s, of the tiles of 64 rows (SmallDotSquaresKernel); 0: other tiles are faster.  They read each operand half as often as 32 rows do, but one of them
+// occupies a compute unit, so it takes outputs that fill one round of them (float32: or two) and enough terms for the kernel's slow start.  Of 128 products of 66 to
+// 4084 terms these are the 42 that gain 1 to 52 %, 12 in the middle; us, without and with them: float32 [128,650] . [650,10000] (0.98 of a round) 28.1 24.8,
+// [512,1000] . [1000,1000] (0.98) 17.8 15.6, [143,1682] . [1682,3773] (0.69) 34.1 31.6, [670,3324] . [3324,2007] (0.86 of two) 126 107; float16
+// [1782,2632] . [2632,471] (0.80) 30.3 19.9, [99,1654] . [1654,5651] (0.71) 15.6 12.5.  Beside the lines: float32 [135,932] . [932,3209] (0.55) 17.4 20.2,
+// [308,262] . [262,1617] 8.2 8.7, [467,788] . [788,3290] (0.73 of two) 40.4 41.2, float16 [994,424] . [424,807] (0.77) 8.4 8.8, [814,378] . [378,1580] (0.82 of two)
+// 10.1 13.2.
+template <typename T>
+int SquaresBlocks(int64_t m, int64_t n, int64_t k) {
+    if (k < (sizeof(T) == 4 ? 300 : 470)) return 0;
+    int best = 0;
+    double most = 0;
+    for (int rounds = 1; rounds <= (sizeof(T) == 4 ? 2 : 1); ++rounds) {
+        for (int blocks = 2; blocks <= 5; ++blocks) {
+            const int64_t groups = (m + 63) / 64 * ((n + 16 * blocks - 1) / (16 * blocks));
+            if (groups > rounds * NumCUs()) continue;
+            const double filled = static_cast<double>(m) * n / (64.0 * 16 * blocks * rounds * NumCUs());
+            if (filled >= (rounds == 1 ? 0.65 : 0.8) && filled > most) best = blocks, most = filled;
+            break;  // wider tiles only leave more idle
+        }
+        if (best > 0) return best;
+    }
+    return 0;
+}
+
 // `batch` products (SmallDotArgs::outs) of p.ksplit workgroups per tile.
 template <typename T>
 void LaunchSmallDot(SmallDotArgs p, int a_mode, int b_mode, int batch, hipStream_t stream) {
@@ -146,6 +171,21 @@ void LaunchSmallDot(SmallDotArgs p, int a_mode, int b_mode, int batch, hipStream
                                stream, p);
             CheckLaunch("small_dot_lines");
         };
+        const int square_blocks = p.ksplit == 1 && batch == 1 ? SquaresBlocks<T>(p.M, p.N, p.K) : 0;
+        auto squares = [&](auto blocks_tag) {
+            constexpr int NB = decltype(blocks_tag)::value, kLds = std::max(2 * (64 + (NB + 1) / 2 * 32) * kSquaresPitch, 4 * 64 * (16 * NB + 1) * 4);
+            p.tiles_m = (p.M + 63) / 64, p.tiles_n = (p.N + 16 * NB - 1) / (16 * NB);
+            struct SquaresTag {};
+            EnsureDynamicLds<SquaresTag>(reinterpret_cast<const void*>(SmallDotSquaresKernel<T, NB>), kLds);
+            hipLaunchKernelGGL((SmallDotSquaresKernel<T, NB>), dim3(static_cast<unsigned>(p.tiles_m * p.tiles_n)), dim3(512), kLds, stream, p);
+            CheckLaunch("small_dot_squares");
+        };
+        switch (square_blocks) {
+            case 2: return squares(std::integral_constant<int, 2>{});
+            case 3: return squares(std::integral_constant<int, 3>{});
+            case 4: return squares(std::integral_constant<int, 4>{});
+            case 5: return squares(std::integral_constant<int, 5>{});
+        }
         switch (LinesBlocks<T>(p.tiles_m, p.N, static_cast<int64_t>(p.ksplit) * batch, p.K / p.ksplit)) {
             case 1: return lines(std::integral_constant<int, 1>{});
             case 2: return lines(std::integral_constant<int, 2>{});
