@@ -125,18 +125,11 @@ __global__ __launch_bounds__(512) void LstmStepKernel(LstmStepArgs p) {
     };
     auto multiply = [&](int st, int c, auto&& next) {
         if ((c + 1) * KC > K) {
-            const int skip = c * KC + piece * PL - (K - PL);  // elements that another piece holds
-            auto keep = [&](Bytes16 v) {
-                using Piece = __attribute__((ext_vector_type(PL))) std::conditional_t<sizeof(T) == 4, unsigned, unsigned short>;
-                Piece e = __builtin_bit_cast(Piece, v);
+            const int early = PieceEarly<T>(c * KC + piece * PL, K);
 #pragma unroll
-                for (int i = 0; i < PL; ++i) e[i] = i < skip ? 0 : e[i];
-                return __builtin_bit_cast(Bytes16, e);
-            };
+            for (int j = 0; j < AL; ++j) av[st][j] = KeepPiece<T>(av[st][j], early);
 #pragma unroll
-            for (int j = 0; j < AL; ++j) av[st][j] = keep(av[st][j]);
-#pragma unroll
-            for (int j = 0; j < BL; ++j) wv[st][j] = keep(wv[st][j]);
+            for (int j = 0; j < BL; ++j) wv[st][j] = KeepPiece<T>(wv[st][j], early);
         }
 #pragma unroll
         for (int j = 0; j < AL; ++j) *reinterpret_cast<Bytes16*>(to + j * 8 * kSmallDotPitch) = av[st][j];

@@ -9,11 +9,10 @@
 //                         latency of a few loads.
 //   SmallDotLinesKernel   the same for more or longer tiles: whole 128-byte lines regrouped through LDS.
 //   SmallDotSquaresKernel the same once 64 rows to a tile fill the chip: whole lines into LDS that the waves share.
-//   SmallDotMixedKernel   an operand whose k axis is not the unit-stride one (dG . Wh of a recurrent network, x^T . gy), or float16 rows
-//                         of odd pitch.
+//   SmallDotMixedKernel   an operand whose k axis is not the unit-stride one (dG . Wh of a recurrent network, x^T . gy).
 //   SmallDotColumnsKernel float32, both operands with m and n as the unit-stride axes, of outputs that make a 64 x 64 tile per compute unit.
 //   SmallDotVectorKernel  M <= 4 (one image, one sentence): a wave per output column, K across the lanes, where the MFMA would work on
-//                         32 rows.
+//                         32 rows (float16: of few columns).
 // For float the reduction index is dealt to the v_mfma_f32_32x32x2_f32 steps so that a lane's four steps use four consecutive k (one
 // 16-byte load when k is the contiguous axis of the operand); for float16 a lane's v_mfma_f32_32x32x16_f16 operand is 8 consecutive k.
 // Rows / columns beyond M / N and the tail of K are served as zeros by the buffer bounds check or explicit masks.
@@ -268,6 +267,23 @@ __device__ __forceinline__ Bytes16 MaskPiece(Bytes16 v, int k, int K) {
     return v;
 }
 
+// A piece that reaches beyond the end of its row is read from the row's last 16 bytes instead: rows may then start and end anywhere, as long as they are 16
+// bytes long.  Elements by which that is early, of the piece at `k`; they are another piece's.
+template <typename T>
+__device__ __forceinline__ int PieceEarly(int k, int K) {
+    return max(0, k - (K - static_cast<int>(16 / sizeof(T))));
+}
+// The piece without them.
+template <typename T>
+__device__ __forceinline__ Bytes16 KeepPiece(Bytes16 v, int early) {
+    constexpr int PL = 16 / sizeof(T);
+    using Piece = __attribute__((ext_vector_type(PL))) std::conditional_t<sizeof(T) == 4, unsigned, unsigned short>;
+    Piece e = __builtin_bit_cast(Piece, v);
+#pragma unroll
+    for (int i = 0; i < PL; ++i) e[i] = i < early ? 0 : e[i];
+    return __builtin_bit_cast(Bytes16, e);
+}
+
 // 16 x 16 outputs from 16 bytes of 16 rows of a and b, the k of a piece in any order as long as both operands keep to it.
 template <typename T>
 __device__ __forceinline__ void MfmaBlock(const Bytes16& a, const Bytes16& b, float4_t& acc) {
@@ -342,20 +358,21 @@ __global__ __launch_bounds__(64 * kSmallDotMaxWaves) __attribute__((amdgpu_waves
             for (int j = 0; j < 4; ++j) av[st][j] = __builtin_amdgcn_raw_buffer_load_b128(ar, a_line[j], c * 128, 0);
 #pragma unroll
             for (int j = 0; j < BL; ++j) bv[st][j] = __builtin_amdgcn_raw_buffer_load_b128(br, b_line[j], c * 128, 0);
-        } else {  // pieces beyond K are not read
-            const bool in = c * KC + piece * PL < p.K;
+        } else {
+            const int at = c * 128 - PieceEarly<T>(c * KC + piece * PL, p.K) * static_cast<int>(sizeof(T));
 #pragma unroll
-            for (int j = 0; j < 4; ++j) av[st][j] = __builtin_amdgcn_raw_buffer_load_b128(ar, (in & (a_line[j] != kOut)) ? a_line[j] + c * 128 : kOut, 0, 0);
+            for (int j = 0; j < 4; ++j) av[st][j] = __builtin_amdgcn_raw_buffer_load_b128(ar, a_line[j] != kOut ? a_line[j] + at : kOut, 0, 0);
 #pragma unroll
-            for (int j = 0; j < BL; ++j) bv[st][j] = __builtin_amdgcn_raw_buffer_load_b128(br, (in & (b_line[j] != kOut)) ? b_line[j] + c * 128 : kOut, 0, 0);
+            for (int j = 0; j < BL; ++j) bv[st][j] = __builtin_amdgcn_raw_buffer_load_b128(br, b_line[j] != kOut ? b_line[j] + at : kOut, 0, 0);
         }
     };
     auto multiply = [&](int st, int c, auto&& next) {
         if ((c + 1) * KC > p.K) {
+            const int early = PieceEarly<T>(c * KC + piece * PL, p.K);
 #pragma unroll
-            for (int j = 0; j < 4; ++j) av[st][j] = MaskPiece<T>(av[st][j], c * KC + piece * PL, p.K);
+            for (int j = 0; j < 4; ++j) av[st][j] = KeepPiece<T>(av[st][j], early);
 #pragma unroll
-            for (int j = 0; j < BL; ++j) bv[st][j] = MaskPiece<T>(bv[st][j], c * KC + piece * PL, p.K);
+            for (int j = 0; j < BL; ++j) bv[st][j] = KeepPiece<T>(bv[st][j], early);
         }
 #pragma unroll
         for (int j = 0; j < 4; ++j) *reinterpret_cast<Bytes16*>(to + j * 8 * kSmallDotPitch) = av[st][j];
@@ -464,19 +481,26 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         for (int j = 0; j < NB; ++j) acc[i][j] = terms[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
     const int chunks = (p.K + KC - 1) / KC;
     Bytes16 av[2], bv[BL], fa[2][2], fb[2][NB];
-    auto load = [&](int c) {  // (pieces beyond K are not read)
-        const bool in = c * KC + k_in < p.K;
+    auto load = [&](int c) {
+        int at = c * 256;
+        bool in = true;
+        if constexpr (sizeof(T) == 2) at -= PieceEarly<T>(c * KC + k_in, p.K) * static_cast<int>(sizeof(T));
+        else in = c * KC + k_in < p.K;  // (their rows are whole dwords: what lies behind them is masked, what is behind the array reads as zeros)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) av[j] = __builtin_amdgcn_raw_buffer_load_b128(ar, (in & (a_line[j] != kOut)) ? a_line[j] + c * 256 : kOut, 0, 0);
+        for (int j = 0; j < 2; ++j) av[j] = __builtin_amdgcn_raw_buffer_load_b128(ar, (in & (a_line[j] != kOut)) ? a_line[j] + at : kOut, 0, 0);
 #pragma unroll
-        for (int j = 0; j < BL; ++j) bv[j] = __builtin_amdgcn_raw_buffer_load_b128(br, (in & (b_line[j] != kOut)) ? b_line[j] + c * 256 : kOut, 0, 0);
+        for (int j = 0; j < BL; ++j) bv[j] = __builtin_amdgcn_raw_buffer_load_b128(br, (in & (b_line[j] != kOut)) ? b_line[j] + at : kOut, 0, 0);
     };
     auto store = [&](int c, auto whole) {
         if (!decltype(whole)::value && (c + 1) * KC > p.K) {
+            auto keep = [&](Bytes16 v) {
+                if constexpr (sizeof(T) == 2) return KeepPiece<T>(v, PieceEarly<T>(c * KC + k_in, p.K));
+                else return MaskPiece<T>(v, c * KC + k_in, p.K);
+            };
 #pragma unroll
-            for (int j = 0; j < 2; ++j) av[j] = MaskPiece<T>(av[j], c * KC + k_in, p.K);
+            for (int j = 0; j < 2; ++j) av[j] = keep(av[j]);
 #pragma unroll
-            for (int j = 0; j < BL; ++j) bv[j] = MaskPiece<T>(bv[j], c * KC + k_in, p.K);
+            for (int j = 0; j < BL; ++j) bv[j] = keep(bv[j]);
         }
         char* const at = to + (c & 1) * kStage;
 #pragma unroll

@@ -82,12 +82,11 @@ void LaunchSmallDotPieces(const SmallDotArgs& p, dim3 grid, hipStream_t stream) 
     CheckLaunch("small_dot_mixed");
 }
 
+// Elements come as they are used: chunks of 32 bytes, six of them in flight, beat whole lines ([32,1000] . [1000,2048] float16 14.3 -> 5.5 us,
+// [200,4000] . [4000,4000] 174 -> 51, [20,2600] . [2600,650] float32 13.4 -> 9.3); rows of odd pitch gain from whole lines at any size.
 template <typename T, int AM, int BM>
-void LaunchSmallDotMixed(const SmallDotArgs& p, dim3 grid, int pieces, hipStream_t stream) {
-    if constexpr (AM != kOddPieces && BM != kOddPieces) {
-        if (pieces == 1) return LaunchSmallDotPieces<T, AM, BM, 1>(p, grid, stream);
-    }
-    LaunchSmallDotPieces<T, AM, BM, 4>(p, grid, stream);
+void LaunchSmallDotMixed(const SmallDotArgs& p, dim3 grid, hipStream_t stream) {
+    LaunchSmallDotPieces<T, AM, BM, AM != kOddPieces && BM != kOddPieces ? 1 : 4>(p, grid, stream);
 }
 
 // Columns, in 16s, of the tiles of whole lines regrouped through LDS (SmallDotLinesKernel); 0: loads straight into the MFMA layout (SmallDotKernel) are
@@ -158,7 +157,7 @@ template <typename T>
 void LaunchSmallDot(SmallDotArgs p, int a_mode, int b_mode, int batch, hipStream_t stream) {
     const int64_t tiles = static_cast<int64_t>(p.tiles_m) * p.tiles_n;
     const dim3 grid(static_cast<unsigned>(tiles * p.ksplit), static_cast<unsigned>(batch));
-    if (a_mode == kPieces && b_mode == kPieces) {
+    if (a_mode != kElements && b_mode != kElements && p.K >= 16 / static_cast<int>(sizeof(T))) {
         const int chunks = ((p.K * static_cast<int>(sizeof(T)) + 127) / 128 + p.ksplit - 1) / p.ksplit;
         auto lines = [&](auto blocks_tag) {
             constexpr int NB = decltype(blocks_tag)::value, kWaveBytes = (32 + 16 * NB) * kSmallDotPitch;
@@ -186,13 +185,24 @@ void LaunchSmallDot(SmallDotArgs p, int a_mode, int b_mode, int batch, hipStream
             case 4: return squares(std::integral_constant<int, 4>{});
             case 5: return squares(std::integral_constant<int, 5>{});
         }
-        switch (LinesBlocks<T>(p.tiles_m, p.N, static_cast<int64_t>(p.ksplit) * batch, p.K / p.ksplit)) {
+        int blocks = LinesBlocks<T>(p.tiles_m, p.N, static_cast<int64_t>(p.ksplit) * batch, p.K / p.ksplit);
+        // SmallDotKernel reads beyond the end of a row, which does not do for the last one of an odd pitch.  us, by elements where a piece does not fit, and so:
+        // [20,651] . [651,2600] 6.3 4.8, [64,33] . [33,500] 7.7 5.5, [128,101] . [101,3000] 7.5 5.4; in tiles of 32 columns 5.7, 7.3, 6.7.  Other widths take these
+        // rows as well: [1000,785] . [785,1000] 26.1 12.1 (784 terms 10.9), [37,801] . [801,1000] 7.3 5.2.
+        if (blocks == 0 && (a_mode == kOddPieces || b_mode == kOddPieces)) blocks = 1;
+        switch (blocks) {
             case 1: return lines(std::integral_constant<int, 1>{});
             case 2: return lines(std::integral_constant<int, 2>{});
             case 3: return lines(std::integral_constant<int, 3>{});
             case 4:
                 if constexpr (sizeof(T) == 2) return lines(std::integral_constant<int, 4>{});
         }
+        if (a_mode == kPieces && b_mode == kPieces) {
+            hipLaunchKernelGGL((SmallDotKernel<T>), grid, dim3(512), 0, stream, p);
+            CheckLaunch("small_dot");
+            return;
+        }
+    } else if (a_mode == kPieces && b_mode == kPieces) {
         hipLaunchKernelGGL((SmallDotKernel<T>), grid, dim3(512), 0, stream, p);
         CheckLaunch("small_dot");
         return;
@@ -212,27 +222,20 @@ void LaunchSmallDot(SmallDotArgs p, int a_mode, int b_mode, int batch, hipStream
             return;
         }
     }
-    // Elements come as they are used: chunks of 32 bytes, six of them in flight, beat whole lines ([32,1000] . [1000,2048] float16 14.3 -> 5.5 us,
-    // [200,4000] . [4000,4000] 174 -> 51, [20,2600] . [2600,650] float32 13.4 -> 9.3); rows of odd pitch gain from whole lines at any size.
-    const bool elements = a_mode == kElements || b_mode == kElements, odd = a_mode == kOddPieces || b_mode == kOddPieces;
-    const int pieces = elements && !odd ? 1 : 4;
+    if (a_mode != kElements && b_mode != kElements) a_mode = b_mode = kElements;  // (fewer terms than a piece holds)
     // eight waves keep more loads in flight; four, one per SIMD, once there is a workgroup for every compute unit
-    const int chunk = pieces == 1 ? 32 : 128, chunks = (p.K * static_cast<int>(sizeof(T)) + chunk - 1) / chunk;
+    const int chunk = a_mode == kOddPieces || b_mode == kOddPieces ? 128 : 32, chunks = (p.K * static_cast<int>(sizeof(T)) + chunk - 1) / chunk;
     const int per_split = (chunks + p.ksplit - 1) / p.ksplit;
     const int most = static_cast<int>(grid.x) * batch <= NumCUs() ? kSmallDotMaxWaves : 4;
     const int per_wave = (per_split + most - 1) / most;
     p.nw = (per_split + per_wave - 1) / per_wave;
-    auto with_a = [&](auto a_tag) {
-        constexpr int AM = decltype(a_tag)::value;
-        if (b_mode == kElements) return LaunchSmallDotMixed<T, AM, kElements>(p, grid, pieces, stream);
-        if constexpr (sizeof(T) == 2) {
-            if (b_mode == kOddPieces) return LaunchSmallDotMixed<T, AM, kOddPieces>(p, grid, pieces, stream);
-        }
-        if constexpr (AM != kPieces) LaunchSmallDotMixed<T, AM, kPieces>(p, grid, pieces, stream);
-    };
-    if (a_mode == kPieces) return with_a(std::integral_constant<int, kPieces>{});
-    if (a_mode == kElements) return with_a(std::integral_constant<int, kElements>{});
-    if constexpr (sizeof(T) == 2) with_a(std::integral_constant<int, kOddPieces>{});
+    if (a_mode == kPieces) return LaunchSmallDotMixed<T, kPieces, kElements>(p, grid, stream);
+    if (b_mode == kPieces) return LaunchSmallDotMixed<T, kElements, kPieces>(p, grid, stream);
+    if constexpr (sizeof(T) == 2) {
+        if (a_mode == kOddPieces) return LaunchSmallDotMixed<T, kOddPieces, kElements>(p, grid, stream);
+        if (b_mode == kOddPieces) return LaunchSmallDotMixed<T, kElements, kOddPieces>(p, grid, stream);
+    }
+    LaunchSmallDotMixed<T, kElements, kElements>(p, grid, stream);
 }
 
 // Rows of a and columns of b of whole 8-byte granules, k dense: what IGemmFastKernel and IGemmSplitKernel read.
@@ -260,7 +263,10 @@ SmallDotPath PlanSmallDot(const hipcx_array* a, const hipcx_array* b, SmallDotAr
         if (sizeof(T) == 4 || ((M + 127) / 128) * ((N + 127) / 128) >= 128) return kNoSmallDot;
     }
     if (*a_mode != kPieces || *b_mode != kPieces) return kSmallDotTiles;
-    if (M <= 4) return kSmallDotVector;
+    // A wave to a column: float32 whatever its size, whose lanes' sums are short.  float16, whose products cost two conversions each there, where the columns are few and
+    // so are the rows, or the terms are many; us, tiles and waves: [1,1000] . [1000,1000] 4.7 3.6, [2,2048] . [2048,2048] 5.7 4.6, [4,4096] . [4096,1000] 7.5
+    // 6.6; [4,332] . [332,3333] 3.7 8.0, [4,1000] . [1000,10000] 6.2 14.8, [1,1000] . [1000,10000] 6.1 7.1, [4,1000] . [1000,1000] 4.7 4.9.
+    if (M <= 4 && (sizeof(T) == 4 || (N <= 2560 && (M <= 2 || K >= 3072)))) return kSmallDotVector;
     return 2.0 * M * N * K >= 1e9 ? kSmallDotWhole : kSmallDotTiles;  // enough tiles, or enough of them long, to keep the chip busy
 }
 

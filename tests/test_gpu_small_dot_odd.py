@@ -1,0 +1,32 @@
+"""float16 matrix products over rows that start and end anywhere, and of up to four rows: at the edges of pieces, tiles and the rule for few rows."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def check(chx, x, w, X, W, what):
+    got = chx.dot(X, W.T).get().astype('float64')
+    x64, w64 = x.astype('float64'), w.astype('float64')
+    ref = x64 @ w64.T
+    # one rounding to 2^-11 of the result, float sums of exact products in chains of at most all the terms, float16's smallest step
+    bound = 2.0 ** -11 * np.abs(ref) + (x.shape[1] + 40) * 2.0 ** -24 * (np.abs(x64) @ np.abs(w64).T) + 2.0 ** -24
+    assert (np.abs(got - ref) <= bound).all(), (what, np.max(np.abs(got - ref) / bound))
+
+
+@pytest.mark.parametrize('m,k,n', [(5, 1, 7), (6, 7, 9), (1, 9, 40), (3, 15, 33), (64, 33, 500), (33, 65, 47), (20, 651, 2600), (37, 801, 1000), (128, 333, 5000),
+                                   (500, 501, 500), (150, 1023, 2049), (1000, 785, 1000), (300, 4001, 300), (129, 771, 9985), (2, 1001, 1000),
+                                   (2, 1000, 2560), (2, 1000, 2561), (3, 3072, 1000), (3, 3070, 1000), (4, 332, 3333), (1, 64, 10000)])
+def test_products(m, k, n):
+    import chainer_amd as chx
+    rng = np.random.default_rng(m + k + n)
+    x, w = [rng.standard_normal(s).astype('float16') for s in ((m, k + 1), (n, k + 1))]
+    X, W = chx.array(x), chx.array(w)
+    x[0, -1] = w[0, -1] = x[-1, 0] = w[-1, 0] = np.nan  # what lies beside the operands
+    X, W = chx.array(x), chx.array(w)
+    ok = np.s_[1:-1] if m > 2 else np.s_[:0]
+    x2, w2 = np.ascontiguousarray(np.nan_to_num(x[:, :k])), np.ascontiguousarray(np.nan_to_num(w[:, :k]))
+    check(chx, x2, w2, chx.array(x2), chx.array(w2), 'dense')
+    check(chx, x[ok, :k], w[1:-1, :k], X[ok, :k], W[1:-1, :k], 'rows of a wider array')
+    check(chx, x[ok, 1:], w[1:-1, 1:], X[ok, 1:], W[1:-1, 1:], 'rows that start at odd elements')
+    check(chx, x[ok, 1:], w[1:-1, :k], X[ok, 1:], W[1:-1, :k], 'one of each')
