@@ -934,6 +934,26 @@ ConvPlan PlanConv(const hipcx_array* x, const hipcx_array* w, const int64_t* str
     return pl;
 }
 
+// DirectConv reads dense filters: those, or a copy of views (the flipped ones of a transposed convolution) in the room that the general kernel has for one.
+bool DirectFilters(const hipcx_array* w, const ConvPlan& pl) {
+    return IsContiguous(w) || pl.w_bytes >= static_cast<size_t>(TotalSize(w)) * sizeof(float);
+}
+
+void RunDirect(const hipcx_array* x, const hipcx_array* w, const hipcx_array* b, const hipcx_array* out, char* ws, hipStream_t stream) {
+    hipcx_array dense = *w;
+    if (!IsContiguous(w)) {
+        dense.data = ws;
+        int64_t step = sizeof(float);
+        for (int d = 3; d >= 0; --d) {
+            dense.strides[d] = step;
+            step *= dense.shape[d];
+        }
+        const int rc = hipcx_copy(w, &dense, stream);
+        HIPCX_REQUIRE(rc == HIPCX_OK, rc, hipcx_last_error());
+    }
+    DirectConv(x, &dense, b, out, stream);
+}
+
 // Repacks w[K,C,R,S] (any strides) into dense [K][R][S][Cpad] (zero-filled padding) with strided Copy launches.
 void RepackFilters(const hipcx_array* w, int Cpad, void* dst, hipStream_t stream) {
     int64_t it = ItemSize(w->dtype);
@@ -1176,7 +1196,7 @@ int hipcx_conv_route(const hipcx_array* x, const hipcx_array* w, const hipcx_arr
         }
         if (PlanStem(x, w, out, stride, pad).ok) return 2;
         if (ThinConvTakes(x, w, stride, pad, out)) return 5;
-        return DirectConvTakes(x, w, stride, pad, out) ? 6 : 0;
+        return DirectConvTakes(x, w, stride, pad, out) && DirectFilters(w, PlanConv(x, w, stride, pad)) ? 6 : 0;
     } catch (...) {
         return -1;
     }
@@ -1223,7 +1243,7 @@ int hipcx_conv(const hipcx_array* x, const hipcx_array* w, const hipcx_array* b,
             else RunConv<half_t>(x, w, b, pl, out, ws, st);
         } else if (out->dtype == HIPCX_FLOAT32) {
             if (ThinConvTakes(x, w, stride, pad, out)) ThinConv(x, w, b, stride, pad, out, st);
-            else if (DirectConvTakes(x, w, stride, pad, out)) DirectConv(x, w, b, out, st);
+            else if (DirectConvTakes(x, w, stride, pad, out) && DirectFilters(w, pl)) RunDirect(x, w, b, out, ws, st);
             else RunConv<float>(x, w, b, pl, out, ws, st);
         } else {
             RunConv<double>(x, w, b, pl, out, ws, st);

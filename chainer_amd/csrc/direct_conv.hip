@@ -188,7 +188,7 @@ int64_t Tiles(int64_t pixels, int64_t filters) { return ((pixels + 31) / 32) * (
 
 bool DirectConvTakes(const hipcx_array* x, const hipcx_array* w, const int64_t* stride, const int64_t* pad, const hipcx_array* out) {
     static const bool enabled = [] { const char* e = getenv("HIPCX_CONV_DIRECT"); return e == nullptr || e[0] != '0'; }();
-    if (!enabled || out->dtype != HIPCX_FLOAT32 || !IsContiguous(x) || !IsContiguous(w) || !IsContiguous(out)) return false;
+    if (!enabled || out->dtype != HIPCX_FLOAT32 || !IsContiguous(x) || !IsContiguous(out)) return false;
     const int64_t N = x->shape[0], C = x->shape[1], P = x->shape[2] * x->shape[3], K = w->shape[0];
     // Beyond, the large tiles of the split operands (igemm_split.hip) catch up, copies of x and w included.  us there and here: 64 -> 64 at 32^2, 96 images 87 and 80,
     // 128 images (8192 tiles) 96 and 105; 128 -> 128 at 16^2, 96 images (3072) 88 and 82, 112 images 94 and 101; 256 -> 256 at 8^2, 160 images (2560) 145 and

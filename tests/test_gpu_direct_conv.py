@@ -52,3 +52,13 @@ def test_limits_of_the_route():
     assert route(2, 12, 8, 64) == 0 and route(2, 8, 8, 64, stride=2) == 0 and route(2, 8, 8, 64, pad=0) == 0 and route(2, 8, 8, 64, size=5) == 0
     x = chx.zeros((2, 8, 9, 8), np.float32)
     assert chx.conv_route(x[:, :, 1:], chx.zeros((64, 8, 3, 3), np.float32), None, 1, 1) == 0
+
+
+def test_filters_that_are_a_view_are_copied():
+    rng = np.random.default_rng(5)
+    x, f = rng.standard_normal((2, 16, 9, 8), dtype=np.float32), rng.standard_normal((16, 24, 3, 3), dtype=np.float32)
+    flipped = chx.array(f)[:, :, ::-1, ::-1].transpose((1, 0, 2, 3))
+    assert chx.conv_route(chx.array(x), flipped, None, 1, 1) == 6
+    dense = chx.conv(chx.array(x), flipped.copy(), None, 1, 1).get()
+    np.testing.assert_array_equal(chx.conv(chx.array(x), flipped, None, 1, 1).get(), dense)
+    np.testing.assert_array_equal(chx.conv_transpose(chx.array(x), chx.array(f), None, 1, 1).get(), dense)
