@@ -13,9 +13,10 @@ struct BatchedOperands {
     half_t* out;  // dense [M][N]
     int M, N, depth, batch;
     int64_t a_row, a_slice, b_row, b_slice;
-    // taps_s > 0: row j of bt_b is a window of a larger array: j = (c, r, s), c = j / (taps_r * taps_s), starts at b + c * b_row + r * r_stride + s * s_stride
+    // taps_s > 0: row j of bt_b is a window of a larger array: j = (c, r, s), c = j / (taps_r * taps_s), starts at b + c * b_row + r * r_stride + s % 2 * s_stride +
+    // s / 2 * s_pair_stride
     int taps_r, taps_s;
-    int64_t r_stride, s_stride;
+    int64_t r_stride, s_stride, s_pair_stride;
 };
 
 // Workgroups per tile along the reduction; slices > 1 need slices * m * n floats of partial sums.

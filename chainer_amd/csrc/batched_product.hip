@@ -57,7 +57,8 @@ __global__ __launch_bounds__(256) void BatchedProductKernel(ProductArgs p) {
         int64_t b_row = static_cast<int64_t>(n) * o.b_row;
         if (o.taps_s > 0) {
             const int taps = o.taps_r * o.taps_s, c = n / taps, t = n - c * taps, tr = t / o.taps_s;
-            b_row = c * o.b_row + tr * o.r_stride + (t - tr * o.taps_s) * o.s_stride;
+            const int ts = t - tr * o.taps_s;
+            b_row = c * o.b_row + tr * o.r_stride + (ts & 1) * o.s_stride + (ts >> 1) * o.s_pair_stride;
         }
         voa[i] = m < o.M ? static_cast<int>(m * o.a_row * 2) + piece * 16 : kOut;
         vob[i] = n < o.N ? static_cast<int>(b_row * 2) + piece * 16 : kOut;
@@ -223,6 +224,14 @@ __global__ __launch_bounds__(256) void BatchedSumKernel(const float* partial, ha
     }
 }
 
+// Where the last window of a row begins.
+double LastTap(const BatchedOperands& o) {
+    if (o.taps_s <= 0) return 0.0;
+    const int last = o.taps_s - 1;
+    const double even = static_cast<double>(last / 2) * o.s_pair_stride, odd = last > 0 ? static_cast<double>(o.s_stride) + (last - 1) / 2 * static_cast<double>(o.s_pair_stride) : 0.0;
+    return (o.taps_r - 1.0) * o.r_stride + std::max(even, odd);
+}
+
 double Bytes(int64_t rows, int64_t row, int64_t slice, const BatchedOperands& o) { return 2.0 * ((rows - 1.0) * row + (o.batch - 1.0) * slice + o.depth); }
 
 }  // namespace
@@ -241,12 +250,12 @@ int HalfProductSlices(int64_t m, int64_t n, int64_t depth, int64_t batch) {
 }
 
 bool HalfProductApplies(const BatchedOperands& o) {
-    const double last_b = o.taps_s > 0 ? (o.taps_r - 1.0) * o.r_stride + (o.taps_s - 1.0) * o.s_stride : 0.0;
+    const double last_b = LastTap(o);
     const int64_t b_rows = o.taps_s > 0 ? o.N / (o.taps_r * o.taps_s) : o.N;
     const double limit = 2147483000.0;
     const int64_t tiles = ((static_cast<int64_t>(o.M) + 127) / 128) * ((static_cast<int64_t>(o.N) + 127) / 128);
     const int64_t odd = static_cast<int64_t>(reinterpret_cast<uintptr_t>(o.a) | reinterpret_cast<uintptr_t>(o.b)) / 2 | o.depth | o.a_row | o.a_slice | o.b_row |
-                        o.b_slice | o.r_stride | o.s_stride;
+                        o.b_slice | o.r_stride | o.s_stride | o.s_pair_stride;
     return o.depth >= 32 && odd % 2 == 0 && tiles < (1 << 14) && Bytes(o.M, o.a_row, o.a_slice, o) < limit && Bytes(b_rows, o.b_row, o.b_slice, o) + 2 * last_b < limit &&
            static_cast<double>(o.M) * o.N < limit;
 }
@@ -259,7 +268,7 @@ void HalfProduct(const BatchedOperands& o, float* partial, int slices, hipStream
     p.chunks_per_image = (o.depth + 31) / 32;
     p.tiles_n = (o.N + 127) / 128;
     const int64_t b_rows = o.taps_s > 0 ? o.N / (o.taps_r * o.taps_s) : o.N;
-    const double last_b = o.taps_s > 0 ? (o.taps_r - 1.0) * o.r_stride + (o.taps_s - 1.0) * o.s_stride : 0.0;
+    const double last_b = LastTap(o);
     p.a_bytes = static_cast<unsigned>(Bytes(o.M, o.a_row, o.a_slice, o));
     p.b_bytes = static_cast<unsigned>(Bytes(b_rows, o.b_row, o.b_slice, o) + 2 * last_b);
     const int64_t tiles = static_cast<int64_t>((o.M + 127) / 128) * p.tiles_n;

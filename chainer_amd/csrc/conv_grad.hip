@@ -8,16 +8,18 @@
 // and then gw[k][(c, r, s)] = Dot(gy_t, col_t^T), which for these shapes (few output tiles, long reduction) runs with the
 // reduction split over workgroups.
 //
-// Filters larger than 1x1 at stride 1 (float16 / float32) avoid the kh*kw-fold Im2Col: x is written kw times as zero-padded planes
-// whose rows are Wp = W + 2*pw rounded up to a 16-byte granule, copy s shifted left by s elements, and gy once with its rows
-// padded to Wp with zeros.  On that common grid tap (r, s) of channel c is the window of copy s that starts r rows down, so
-//     gw[k][c][r][s] = sum_n sum_q gy_p[n][k][q] * x_s[s][n][c][q + r*Wp],   q over OH*Wp
+// Filters larger than 1x1 at stride 1 (float16 / float32) avoid the kh*kw-fold Im2Col: x is written as zero-padded planes of rows of Wp elements, several
+// copies of them shifted left by one element each, and gy once with its rows padded to Wp with zeros.  On that common grid tap (r, s) of channel c is a
+// window of one of the copies, so
+//     gw[k][c][r][s] = sum_n sum_q gy_p[n][k][q] * x_p[n][c][q + r*Wp + s],   q over OH*Wp
 // is one accumulated matrix product per image whose right-hand rows alias windows of the copies; the zero columns of gy_p cancel
-// the products that wrap around a row end.  A non-finite x value would meet a zero of gy_p in windows the reference never
-// multiplies it into (0 * inf = NaN in filter taps that stay finite there), so the copy kernel flags every input channel that holds
-// an inf or NaN and, after the product, GradWeightChannelFixupKernel computes the flagged channels' filter taps again the
+// the products that wrap around a row end.  In float16 the product reads at any even element: two copies serve every s, and rows are as long as x's with
+// the padding of one side (the next row's stands in for the other), rounded up to even.  Otherwise there are kw copies and rows are whole 16-byte
+// granules with both paddings.  A non-finite x value would meet a zero of gy_p in windows the reference never
+// multiplies it into (0 * inf = NaN in filter taps that stay finite there), so the copy kernel flags every plane of x that holds
+// an inf or NaN and, after the product, GradWeightChannelFixupKernel computes the filter taps of those planes' channels again the
 // reference's way (the sum over the Im2Col windows, padding multiplied as zeros).  With finite data that kernel's workgroups read
-// one flag each and exit.
+// a channel's flags each and exit.
 #include "batched_product.h"
 #include "common.h"
 
@@ -118,16 +120,22 @@ __global__ __launch_bounds__(256) void TransposeNKKernel(GradWeightArgs p, int64
     }
 }
 
-struct ShiftedArgs {
-    const void* x;
-    const void* gy;
-    void* xs;   // [kw][N*C][Hp*Wp]
-    void* gyp;  // [N*K][OH*Wp]
-    int* nonfinite;  // [C]: set to 1 for channels of x that hold an inf or NaN (cleared by PaddedRowsKernel, which runs first)
-    int planes_x, planes_gy;  // N*C, N*K
-    int C;
-    int H, W, OH, OW, Hp, Wp, ph, pw, kw;
+// Planes [H][W] and where they lie in planes of rows of Wp elements: from row ph and column pw on, zeros around them.
+struct PlaneSet {
+    const void* from;
+    void* to;  // [copies][planes][pitch]: copy s holds the plane's element q + s at q
+    int planes, H, W, ph, pw, copies;
+    int pitch;  // a multiple of 16 bytes
 };
+
+struct PlanesArgs {
+    PlaneSet set[2];  // x, gy
+    int Wp;
+    int* nonfinite;  // [planes of x]: whether it holds an inf or NaN
+    int each;        // planes of a workgroup, kMostPlanes at most
+    int64_t blocks_x, blocks;
+};
+constexpr int kMostPlanes = 64;
 
 template <typename T>
 __device__ __forceinline__ bool NonFinite(T v) {
@@ -138,66 +146,68 @@ __device__ __forceinline__ bool NonFinite(T v) {
     }
 }
 
-// xs[s][plane][q] = padded x[plane][q + s]; one thread writes VEC consecutive q.
-template <typename T, int VEC>
-__global__ __launch_bounds__(256) void ShiftedPlanesKernel(ShiftedArgs p, unsigned total) {
-    const T* x = static_cast<const T*>(p.x);
-    T* xs = static_cast<T*>(p.xs);
-    const unsigned per_plane = static_cast<unsigned>(p.Hp * p.Wp / VEC);
-    for (unsigned idx = blockIdx.x * 256u + threadIdx.x; idx < total; idx += gridDim.x * 256u) {
-        unsigned t = idx / per_plane;
-        const unsigned qv = idx - t * per_plane;
-        const unsigned s = t / static_cast<unsigned>(p.planes_x);
-        const unsigned plane = t - s * static_cast<unsigned>(p.planes_x);
-        const T* src = x + static_cast<int64_t>(plane) * p.H * p.W;
-        GVec<T, VEC> out;
-        int q = static_cast<int>(qv) * VEC + static_cast<int>(s);
-        int hp = q / p.Wp, wp = q - hp * p.Wp;
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) {
-            const int ih = hp - p.ph, iw = wp - p.pw;
-            out.v[e] = (ih >= 0 && ih < p.H && iw >= 0 && iw < p.W) ? src[ih * p.W + iw] : T(0);  // rows past Hp fail ih < H
-            if (++wp == p.Wp) wp = 0, ++hp;
+// Both sets in one pass.  A workgroup takes a few whole planes, whose pieces of 16 bytes are dealt out to its threads; a piece's elements are gathered
+// once, and each further copy takes one more.  Bound by the gathers, an element a lane; 64 threads to a plane, of which the 33 pieces of a 14 x 14 one
+// use half, make the whole call of 256 channels, 32 images, 38.9 us instead of 35.8.  us of the call in float16, three copies of rows of whole granules from
+// two kernels and now, 32 images: 64 channels at 56^2 61 -> 53, 128 at 28^2 42 -> 38, 256 at 14^2 37.7 -> 35.8, 512 at 7^2 54 -> 39.
+template <typename T>
+__global__ __launch_bounds__(256) void PlanesKernel(PlanesArgs p) {
+    constexpr int E = 16 / sizeof(T);
+    __shared__ int flags[kMostPlanes];
+    for (int64_t block = blockIdx.x; block < p.blocks; block += gridDim.x) {
+        const bool of_x = block < p.blocks_x;
+        const PlaneSet& o = p.set[of_x ? 0 : 1];
+        const int64_t plane0 = (of_x ? block : block - p.blocks_x) * p.each;
+        const int planes = static_cast<int>(min(static_cast<int64_t>(p.each), o.planes - plane0)), pieces = o.pitch / E;
+        if (of_x) {
+            if (threadIdx.x < kMostPlanes) flags[threadIdx.x] = 0;
+            __syncthreads();
         }
-        *reinterpret_cast<GVec<T, VEC>*>(xs + static_cast<int64_t>(idx) * VEC) = out;
-        if (s == 0) {  // copy 0 holds every element of x
+        for (int i = threadIdx.x; i < planes * pieces; i += 256) {
+            const int local = static_cast<unsigned>(i) / static_cast<unsigned>(pieces), q = (i - local * pieces) * E;
+            const int64_t plane = plane0 + local;
+            const T* const from = static_cast<const T*>(o.from) + plane * o.H * o.W;
+            T* const to = static_cast<T*>(o.to) + plane * o.pitch + q;
+            int row = static_cast<unsigned>(q) / static_cast<unsigned>(p.Wp), col = q - row * p.Wp;
+            auto next = [&] {
+                const int h = row - o.ph, w = col - o.pw;
+                const bool inside = h >= 0 && h < o.H && w >= 0 && w < o.W;
+                const T v = from[inside ? h * o.W + w : 0];
+                if (++col == p.Wp) col = 0, ++row;
+                return inside ? v : T(0);
+            };
+            GVec<T, E> out;
+#pragma unroll
+            for (int e = 0; e < E; ++e) out.v[e] = next();
             bool bad = false;
 #pragma unroll
-            for (int e = 0; e < VEC; ++e) bad |= NonFinite<T>(out.v[e]);
-            if (bad) p.nonfinite[plane % static_cast<unsigned>(p.C)] = 1;
-        }
-        if (idx + gridDim.x * 256u < idx) break;  // the next index would wrap
-    }
-}
-
-// gyp[plane][oh][w] = gy[plane][oh][w] for w < OW, 0 up to Wp.
-template <typename T, int VEC>
-__global__ __launch_bounds__(256) void PaddedRowsKernel(ShiftedArgs p, unsigned total) {
-    const T* gy = static_cast<const T*>(p.gy);
-    T* gyp = static_cast<T*>(p.gyp);
-    const unsigned per_row = static_cast<unsigned>(p.Wp / VEC);
-    if (blockIdx.x == 0) {
-        for (int c = threadIdx.x; c < p.C; c += 256) p.nonfinite[c] = 0;
-    }
-    for (unsigned idx = blockIdx.x * 256u + threadIdx.x; idx < total; idx += gridDim.x * 256u) {
-        const unsigned row = idx / per_row;  // plane * OH + oh: rows of gy are OW apart
-        const int w0 = static_cast<int>(idx - row * per_row) * VEC;
-        const T* src = gy + static_cast<int64_t>(row) * p.OW;
-        GVec<T, VEC> out;
+            for (int e = 0; e < E; ++e) bad |= NonFinite<T>(out.v[e]);
+            if (of_x && bad) flags[local] = 1;
+            *reinterpret_cast<GVec<T, E>*>(to) = out;
+            for (int s = 1; s < o.copies; ++s) {
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) out.v[e] = w0 + e < p.OW ? src[w0 + e] : T(0);
-        *reinterpret_cast<GVec<T, VEC>*>(gyp + static_cast<int64_t>(idx) * VEC) = out;
-        if (idx + gridDim.x * 256u < idx) break;
+                for (int e = 0; e + 1 < E; ++e) out.v[e] = out.v[e + 1];
+                out.v[E - 1] = next();
+                *reinterpret_cast<GVec<T, E>*>(to + static_cast<int64_t>(s) * o.planes * o.pitch) = out;
+            }
+        }
+        if (of_x) {
+            __syncthreads();
+            if (threadIdx.x < planes) p.nonfinite[plane0 + threadIdx.x] = flags[threadIdx.x];
+            __syncthreads();
+        }
     }
 }
 
-// Filter taps of the input channels flagged in `nonfinite`, summed the reference's way: gw[k][c][r][s] = sum over (n, oh, ow) of
+// Filter taps of the input channels of the planes flagged in `nonfinite`, summed the reference's way: gw[k][c][r][s] = sum over (n, oh, ow) of
 // gy[n][k][oh][ow] * col, col = x[n][c][oh*sh - ph + r][ow*sw - pw + s] or the padding's zero (still multiplied, as TensorDot
 // multiplies Im2Col's zeros: CX/native/native_device/conv.cc:91-124).  Grid (C, slices); a wave per output, lanes over the sum.
 template <typename T>
 __global__ __launch_bounds__(256) void GradWeightChannelFixupKernel(GradWeightArgs p, const int* nonfinite, T* gw) {
     const int c = blockIdx.x;
-    if (nonfinite[c] == 0) return;
+    int any = 0;
+    for (int n = threadIdx.x; n < p.N; n += 256) any |= nonfinite[static_cast<int64_t>(n) * p.C + c];
+    if (__syncthreads_or(any) == 0) return;
     const T* x = static_cast<const T*>(p.x);
     const T* gy = static_cast<const T*>(p.gy);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -345,13 +355,13 @@ struct Product {
 };
 
 Product PlanProduct(const void* a, int64_t a_row, int64_t a_slice, const void* b, int64_t b_row, int64_t b_slice, int64_t m, int64_t n, int64_t depth, int64_t batch,
-                    void* out, int dtype, int taps_r = 0, int taps_s = 0, int64_t r_stride = 0, int64_t s_stride = 0) {
+                    void* out, int dtype, int taps_r = 0, int taps_s = 0, int64_t r_stride = 0, int64_t s_stride = 0, int64_t s_pair_stride = 0) {
     Product pr;
     BatchedOperands& o = pr.o;
     o.a = static_cast<const half_t*>(a), o.b = static_cast<const half_t*>(b), o.out = static_cast<half_t*>(out);
     o.M = static_cast<int>(m), o.N = static_cast<int>(n), o.depth = static_cast<int>(depth), o.batch = static_cast<int>(batch);
     o.a_row = a_row, o.a_slice = a_slice, o.b_row = b_row, o.b_slice = b_slice;
-    o.taps_r = taps_r, o.taps_s = taps_s, o.r_stride = r_stride, o.s_stride = s_stride;
+    o.taps_r = taps_r, o.taps_s = taps_s, o.r_stride = r_stride, o.s_stride = s_stride, o.s_pair_stride = s_pair_stride;
     pr.dtype = dtype;
     pr.half = dtype == HIPCX_FLOAT16 && std::max(std::max(m, n), depth) < (1LL << 31) && HalfProductApplies(o);
     if (pr.half) {
@@ -394,40 +404,53 @@ bool DirectPointwise(const GradWeightPlan& pl, const Product& pr, const hipcx_ar
 // Filters larger than 1x1 at stride 1: shifted zero-padded copies of x instead of Im2Col (see the top of the file).
 struct ShiftedPlan {
     bool ok = false;
-    ShiftedArgs a{};
-    int64_t depth = 0, plane = 0;  // OH*Wp; Hp*Wp
-    size_t xs_bytes = 0, gyp_bytes = 0, partial_bytes = 0, flag_bytes = 0;
+    PlanesArgs a{};
+    Product product;  // (of null operands)
+    size_t xs_bytes = 0, gyp_bytes = 0, flag_bytes = 0;
 };
 
 Product ShiftedProduct(const ShiftedPlan& sp, const GradWeightArgs& g, void* gw, int dtype) {
-    return PlanProduct(sp.a.gyp, sp.depth, g.K * sp.depth, sp.a.xs, sp.plane, g.C * sp.plane, g.K, static_cast<int64_t>(g.C) * g.kh * g.kw, sp.depth, g.N, gw, dtype, g.kh,
-                       g.kw, sp.a.Wp, static_cast<int64_t>(g.N) * g.C * sp.plane);
+    const PlaneSet &x = sp.a.set[0], &gy = sp.a.set[1];
+    const int64_t copy = static_cast<int64_t>(x.planes) * x.pitch;
+    return PlanProduct(gy.to, gy.pitch, static_cast<int64_t>(g.K) * gy.pitch, x.to, x.pitch, static_cast<int64_t>(g.C) * x.pitch, g.K,
+                       static_cast<int64_t>(g.C) * g.kh * g.kw, static_cast<int64_t>(g.OH) * sp.a.Wp, g.N, gw, dtype, g.kh, g.kw, sp.a.Wp, copy,
+                       x.copies == g.kw ? 2 * copy : 2);
 }
 
-ShiftedPlan PlanShifted(const GradWeightPlan& pl, int dtype) {
+// `pairs`: two copies, rows rounded up to an even width, for the float16 product; false: kw copies of rows of whole granules.
+ShiftedPlan PlanShifted(const GradWeightPlan& pl, int dtype, bool pairs) {
     ShiftedPlan sp;
     static const bool enabled = [] { const char* e = getenv("HIPCX_GRAD_WEIGHT_SHIFTED"); return e == nullptr || e[0] != '0'; }();
     const GradWeightArgs& g = pl.a;
     if (!enabled || (dtype != HIPCX_FLOAT16 && dtype != HIPCX_FLOAT32)) return sp;
     if (g.sh != 1 || g.sw != 1 || g.kh * g.kw == 1) return sp;
     if (g.OH != g.H + 2 * g.ph - g.kh + 1 || g.OW != g.W + 2 * g.pw - g.kw + 1) return sp;  // cover_all adds nothing at stride 1
-    const int64_t it = ItemSize(dtype), epc = 16 / it;
-    const int64_t Wp = (g.W + 2 * g.pw + epc - 1) / epc * epc, Hp = g.H + 2 * g.ph;
-    // worth it when the kw copies are smaller than the kh*kw-fold Im2Col
-    if (g.kw * Hp * Wp * g.C >= static_cast<int64_t>(g.kh) * g.kw * g.OH * g.OW * g.C) return sp;
-    const int64_t xs_elems = static_cast<int64_t>(g.kw) * g.N * g.C * Hp * Wp, gyp_elems = static_cast<int64_t>(g.N) * g.K * g.OH * Wp;
-    if (xs_elems / epc >= (1LL << 32) || gyp_elems / epc >= (1LL << 32)) return sp;  // 32-bit vector indices in the copy kernels
-    sp.a.planes_x = g.N * g.C, sp.a.planes_gy = g.N * g.K;
-    sp.a.H = g.H, sp.a.W = g.W, sp.a.OH = g.OH, sp.a.OW = g.OW, sp.a.Hp = static_cast<int>(Hp), sp.a.Wp = static_cast<int>(Wp);
-    sp.a.ph = g.ph, sp.a.pw = g.pw, sp.a.kw = g.kw, sp.a.C = g.C;
-    sp.flag_bytes = RoundUp256(static_cast<size_t>(g.C) * sizeof(int));
-    sp.depth = g.OH * Wp;
-    sp.plane = Hp * Wp;
-    sp.xs_bytes = RoundUp256(static_cast<size_t>(xs_elems * it));
-    sp.gyp_bytes = RoundUp256(static_cast<size_t>(gyp_elems * it));
-    sp.partial_bytes = ShiftedProduct(sp, g, nullptr, dtype).partial_bytes;
-    sp.ok = true;
+    const int64_t N = g.N, it = ItemSize(dtype), epc = 16 / it, pw = g.pw, W = g.W;
+    const int64_t Wp = pairs ? (std::max<int64_t>(W + pw, g.OW) + 1) / 2 * 2 : (W + 2 * pw + epc - 1) / epc * epc;
+    const int64_t Hp = g.H + 2 * static_cast<int64_t>(g.ph), copies = pairs ? std::min(g.kw, 2) : g.kw;
+    // windows of a pair's copies start up to kw - 1 elements later than those of copies of their own, and end as much later
+    const int64_t pitch_x = (Hp * Wp + (pairs ? (g.kw - 1) / 2 * 2 : 0) + epc - 1) / epc * epc, pitch_gy = (g.OH * Wp + epc - 1) / epc * epc;
+    // worth it when the copies are smaller than the kh*kw-fold Im2Col
+    if (copies * pitch_x >= static_cast<int64_t>(g.kh) * g.kw * g.OH * g.OW) return sp;
+    const int64_t most = int64_t{1} << 31;
+    if (static_cast<int64_t>(g.H) * W == 0 || pitch_x + 256 * epc >= most || N * g.C >= most || N * g.K >= most) return sp;  // (the copy kernel's 32-bit indices)
+    sp.a.set[0] = PlaneSet{g.x, nullptr, static_cast<int>(N * g.C), g.H, g.W, g.ph, g.pw, static_cast<int>(copies), static_cast<int>(pitch_x)};
+    sp.a.set[1] = PlaneSet{g.gy, nullptr, static_cast<int>(N * g.K), g.OH, g.OW, 0, 0, 1, static_cast<int>(pitch_gy)};
+    sp.a.Wp = static_cast<int>(Wp);
+    sp.flag_bytes = RoundUp256(static_cast<size_t>(N * g.C) * sizeof(int));
+    sp.xs_bytes = RoundUp256(static_cast<size_t>(copies * N * g.C * pitch_x * it));
+    sp.gyp_bytes = RoundUp256(static_cast<size_t>(N * g.K * pitch_gy * it));
+    sp.product = ShiftedProduct(sp, g, nullptr, dtype);
+    sp.ok = !pairs || sp.product.half;
     return sp;
+}
+
+ShiftedPlan PlanShifted(const GradWeightPlan& pl, int dtype) {
+    if (dtype == HIPCX_FLOAT16) {
+        const ShiftedPlan sp = PlanShifted(pl, dtype, true);
+        if (sp.ok) return sp;
+    }
+    return PlanShifted(pl, dtype, false);
 }
 
 // The product of the staged operands, whose rows are the pixels of all images.  float16 of an even number of pixels only, and of 1 GFLOP or 2048 pixels at
@@ -442,16 +465,13 @@ Product StagedProduct(const GradWeightPlan& pl, void* gw, int dtype) {
 }
 
 template <typename T>
-void RunShiftedCopies(const ShiftedArgs& a, hipStream_t stream) {
-    constexpr int VEC = 16 / sizeof(T);
-    const int64_t cap = static_cast<int64_t>(NumCUs()) * 32;
-    auto grid = [&](int64_t n) { int64_t b = (n + 255) / 256; return dim3(static_cast<unsigned>(b > cap ? cap : (b < 1 ? 1 : b))); };
-    const int64_t total_gy = static_cast<int64_t>(a.planes_gy) * a.OH * (a.Wp / VEC);
-    hipLaunchKernelGGL((PaddedRowsKernel<T, VEC>), grid(total_gy), dim3(256), 0, stream, a, static_cast<unsigned>(total_gy));  // clears the flags
-    CheckLaunch("padded rows (weight gradient)");
-    const int64_t total_x = static_cast<int64_t>(a.kw) * a.planes_x * (a.Hp * a.Wp / VEC);
-    hipLaunchKernelGGL((ShiftedPlanesKernel<T, VEC>), grid(total_x), dim3(256), 0, stream, a, static_cast<unsigned>(total_x));  // sets them
-    CheckLaunch("shifted planes (weight gradient)");
+void RunPlanes(PlanesArgs a, hipStream_t stream) {
+    // two pieces to a thread, or a plane
+    a.each = std::max(1, std::min(kMostPlanes, 512 / (a.set[0].pitch / static_cast<int>(16 / sizeof(T)))));
+    a.blocks_x = (a.set[0].planes + int64_t{a.each} - 1) / a.each;
+    a.blocks = a.blocks_x + (a.set[1].planes + int64_t{a.each} - 1) / a.each;
+    hipLaunchKernelGGL((PlanesKernel<T>), dim3(static_cast<unsigned>(std::min<int64_t>(a.blocks, 1 << 22))), dim3(256), 0, stream, a);
+    CheckLaunch("padded planes (weight gradient)");
 }
 
 template <typename T>
@@ -480,7 +500,7 @@ size_t hipcx_conv_grad_weight_workspace_size(const hipcx_array* x, const hipcx_a
         const size_t direct = std::max(in_place.partial_bytes, BatchedProductPartialBytes(pl.a.K, pl.a.C, pixels, pl.a.N, gw->dtype)) + 256;
         const size_t staged = pl.col_bytes + pl.gyt_bytes + std::max(hipcx_dot_workspace_size(&pl.gy_t, &pl.col_view, &out), copied.half ? copied.partial_bytes : 0);
         const ShiftedPlan sp = PlanShifted(pl, gw->dtype);
-        const size_t shifted = sp.ok ? sp.xs_bytes + sp.gyp_bytes + sp.partial_bytes + sp.flag_bytes + 256 : 0;
+        const size_t shifted = sp.ok ? sp.xs_bytes + sp.gyp_bytes + sp.product.partial_bytes + sp.flag_bytes + 256 : 0;
         return std::max(std::max(direct, staged), shifted);
     } catch (...) {
         return 0;
@@ -513,16 +533,15 @@ int hipcx_conv_grad_weight(const hipcx_array* x, const hipcx_array* gy, const in
         }
         ShiftedPlan sp = PlanShifted(pl, gw->dtype);
         if (sp.ok && reinterpret_cast<uintptr_t>(workspace) % 16 == 0 && reinterpret_cast<uintptr_t>(gw->data) % 16 == 0) {
-            const size_t need = sp.xs_bytes + sp.gyp_bytes + sp.partial_bytes + sp.flag_bytes;
+            const size_t need = sp.xs_bytes + sp.gyp_bytes + sp.product.partial_bytes + sp.flag_bytes;
             HIPCX_REQUIRE(workspace != nullptr && workspace_bytes >= need, HIPCX_CHAINERX_ERROR,
                           "conv_grad_weight workspace too small: need " + std::to_string(need) + " bytes");
             char* ws = static_cast<char*>(workspace);
-            sp.a.x = x->data, sp.a.gy = gy->data;
-            sp.a.xs = ws, sp.a.gyp = ws + sp.xs_bytes;
-            sp.a.nonfinite = reinterpret_cast<int*>(ws + sp.xs_bytes + sp.gyp_bytes + sp.partial_bytes);
+            sp.a.set[0].to = ws, sp.a.set[1].to = ws + sp.xs_bytes;
+            sp.a.nonfinite = reinterpret_cast<int*>(ws + sp.xs_bytes + sp.gyp_bytes + sp.product.partial_bytes);
             hipStream_t st = AsStream(stream);
-            if (gw->dtype == HIPCX_FLOAT16) RunShiftedCopies<half_t>(sp.a, st);
-            else RunShiftedCopies<float>(sp.a, st);
+            if (gw->dtype == HIPCX_FLOAT16) RunPlanes<half_t>(sp.a, st);
+            else RunPlanes<float>(sp.a, st);
             const GradWeightArgs& g = pl.a;
             RunProduct(ShiftedProduct(sp, g, gw->data, gw->dtype), ws + sp.xs_bytes + sp.gyp_bytes, st);
             if (gw->dtype == HIPCX_FLOAT16) RunChannelFixup<half_t>(g, sp.a.nonfinite, gw->data, st);
