@@ -321,7 +321,7 @@ def section_train(chx, oracle, with_cpu):
         flops = 3.0 * cfg.resnet50_flops(batch)
         emit(section='train', op='ResNet-50 training step, float16 (batch norm parameters float32)', batch=batch, eager_ms=round(eager * 1e3, 2),
              graph_replay_ms=round(graph * 1e3, 2), img_per_s_graph=round(batch / graph, 1), TFLOPs_graph=round(flops / graph / 1e12, 1),
-             note='3x the forward flops (forward, data gradient, weight gradient); eager time includes ~1500 Python-issued kernel calls')
+             note='3x the forward flops (forward, data gradient, weight gradient); eager time includes ~530 Python-issued kernel calls')
         del pd
 
 
