@@ -10,8 +10,8 @@ namespace hipcx {
 
 // Fewer tiles of 128 x 128 than keep the chip busy; up to 256 for fewer than 64 terms, where larger tiles are bound by copying operands into their layout.  us,
 // without and with these kernels: [64,33] . [33,64] float32 35 and 4.1, [20,50] . [50,8789] 33 and 4.2, float16 30 and 3.9, [128,63] . [63,2600] 41 and 4.6 (one
-// element after another, or a wave to a tile); [352,35] . [35,8653], 204 tiles, 23 and 13.5, float16 23 and 17; beyond, 288 tiles of [3000,33] . [33,1500], 18.2 and
-// 18.9, float16 17.3 and 23.7.
+// element after another, or a wave to a tile); [352,35] . [35,8653], 204 tiles, float16 23 and 17 (float32 of that size is staged, see PlanDotStaging); beyond, 288
+// tiles of [3000,33] . [33,1500], 18.2 and 18.9, float16 17.3 and 23.7.
 bool SmallDotShape(int64_t m, int64_t n, int64_t k) { return ((m + 127) / 128) * ((n + 127) / 128) < (k >= 64 ? 128 : 256); }
 
 namespace {
@@ -326,6 +326,7 @@ bool DotSeveral(const hipcx_array* a0, int64_t a_distance, const hipcx_array* b,
     SmallDotArgs p{};
     int a_mode = 0, b_mode = 0;
     if (n > kSmallDotMaxBatch || !SmallDotShape(M, N, K) || SmallDotSplit(M, N, K, HIPCX_FLOAT32) > 1) return false;
+    if (K < 64 && 2.0 * M * N * K >= 2e8) return false;  // one by one they run on the bfloat16 parts, with half the error (PlanDotStaging)
     if (!SmallDotOperands<float>(a0, b, &p, &a_mode, &b_mode)) return false;
     for (int i = 0; i < n; ++i) {
         if (outs[i]->strides[0] != outs[0]->strides[0] || outs[i]->strides[1] != outs[0]->strides[1]) return false;

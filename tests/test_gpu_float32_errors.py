@@ -1,0 +1,28 @@
+"""float32 results against 64 bits where a call could run on kernels of different accuracy: the 2-norm of the error over that of the result."""
+import numpy as np
+import pytest
+
+import chainer_amd as chx
+
+pytestmark = pytest.mark.gpu
+
+
+def relative(got, ref):
+    return np.linalg.norm(got - ref) / np.linalg.norm(ref)
+
+
+def layouts(a, b):
+    """a . b in every order of both."""
+    for x in (chx.array(a), chx.array(np.ascontiguousarray(a.T)).T):
+        for y in (chx.array(b), chx.array(np.ascontiguousarray(b.T)).T):
+            yield chx.dot(x, y).get()
+
+
+@pytest.mark.parametrize('m,k,n', [(352, 35, 8653), (1500, 57, 1500), (1501, 47, 1700), (2000, 62, 1300), (1400, 63, 1700)])
+def test_large_products_of_few_terms(m, k, n):
+    rng = np.random.default_rng(k)
+    a, b = rng.standard_normal((m, k), dtype=np.float32), rng.standard_normal((k, n), dtype=np.float32)
+    ref = a.astype(np.float64) @ b
+    # sums of bfloat16 parts, 4.0e-8 to 4.9e-8 for 35 to 63 terms; chains of float additions have 7.0e-8 and more
+    for got in layouts(a, b):
+        assert relative(got, ref) < 5.5e-8
