@@ -265,8 +265,9 @@ SmallDotPath PlanSmallDot(const hipcx_array* a, const hipcx_array* b, SmallDotAr
     if (*a_mode != kPieces || *b_mode != kPieces) return kSmallDotTiles;
     // A wave to a column: float32 whatever its size, whose lanes' sums are short.  float16, whose products cost two conversions each there, where the columns are few and
     // so are the rows, or the terms are many; us, tiles and waves: [1,1000] . [1000,1000] 4.7 3.6, [2,2048] . [2048,2048] 5.7 4.6, [4,4096] . [4096,1000] 7.5
-    // 6.6; [4,332] . [332,3333] 3.7 8.0, [4,1000] . [1000,10000] 6.2 14.8, [1,1000] . [1000,10000] 6.1 7.1, [4,1000] . [1000,1000] 4.7 4.9.
-    if (M <= 4 && (sizeof(T) == 4 || (N <= 2560 && (M <= 2 || K >= 3072)))) return kSmallDotVector;
+    // 6.6; [4,332] . [332,3333] 3.7 8.0, [4,1000] . [1000,10000] 6.2 14.8, [1,1000] . [1000,10000] 6.1 7.1, [4,1000] . [1000,1000] 4.7 4.9.  Not for few terms in
+    // float32: a product is rounded before it is added there, 4.4e-8 of the norm for three terms where a chain of the matrix pipe has 3.7e-8.
+    if (M <= 4 && (sizeof(T) == 4 ? K >= 64 : N <= 2560 && (M <= 2 || K >= 3072))) return kSmallDotVector;
     return 2.0 * M * N * K >= 1e9 ? kSmallDotWhole : kSmallDotTiles;  // enough tiles, or enough of them long, to keep the chip busy
 }
 
