@@ -47,3 +47,13 @@ def test_few_rows_of_few_terms(m, k):
     most = relative(chain(a, b), ref) * 1.001 + 1e-12
     for got in layouts(a, b):
         assert relative(got, ref) <= most
+
+
+@pytest.mark.parametrize('m', [1, 5, 40, 300])
+def test_nine_terms(m):
+    rng = np.random.default_rng(m)
+    a, b = rng.standard_normal((m, 9), dtype=np.float32), rng.standard_normal((9, 20000), dtype=np.float32)
+    ref = a.astype(np.float64) @ b
+    most = relative(chain(a, b), ref) * 1.001
+    for got in layouts(a, b):
+        assert relative(got, ref) <= most
