@@ -211,9 +211,10 @@ void LaunchSmallDot(SmallDotArgs p, int a_mode, int b_mode, int batch, hipStream
     }
     if constexpr (sizeof(T) == 4) {
         // Once 64 x 64 tiles occupy three quarters of the compute units; us, elements in 32 x 32 tiles and these: [700,650]^T . [700,650], 121 tiles, 15.0
-        // and 19.4, [100,784]^T . [100,1000], 208, 8.8 and 7.9, [64,1300]^T . [64,1300], 441, 11.3 and 10.6.
+        // and 19.4, [100,784]^T . [100,1000], 208, 8.8 and 7.9, [64,1300]^T . [64,1300], 441, 11.3 and 10.6.  Not for fewer than 64
+        // terms, these and elements: [20,2000]^T . [20,1900] 18.5 and 16.4, [12,1000]^T . [12,1000] 7.5 and 5.5, [35,650]^T . [35,1300] 7.5 and 6.0.
         const int64_t squares = static_cast<int64_t>((p.M + 63) / 64) * ((p.N + 63) / 64) * p.ksplit * batch;
-        if (a_mode == kElements && b_mode == kElements && p.a_row == 1 && p.b_col == 1 && 4 * squares >= 3 * NumCUs()) {
+        if (p.K >= 64 && a_mode == kElements && b_mode == kElements && p.a_row == 1 && p.b_col == 1 && 4 * squares >= 3 * NumCUs()) {
             constexpr int kLds = 4 * 64 * (64 + 4) * 4;
             p.tiles_m = (p.M + 63) / 64, p.tiles_n = (p.N + 63) / 64;
             struct ColumnsTag {};

@@ -57,3 +57,12 @@ def test_nine_terms(m):
     most = relative(chain(a, b), ref) * 1.001
     for got in layouts(a, b):
         assert relative(got, ref) <= most
+
+
+@pytest.mark.parametrize('m,k,n', [(1000, 6, 1100), (4000, 8, 328)])
+def test_both_operands_k_by_k(m, k, n):
+    rng = np.random.default_rng(m)
+    a, b = rng.standard_normal((m, k), dtype=np.float32), rng.standard_normal((k, n), dtype=np.float32)
+    ref = a.astype(np.float64) @ b
+    got = chx.dot(chx.array(np.ascontiguousarray(a.T)).T, chx.array(b)).get()
+    assert relative(got, ref) <= relative(chain(a, b), ref) * 1.001
