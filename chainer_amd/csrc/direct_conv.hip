@@ -6,7 +6,9 @@
 // which are computed once (the channel is a scalar offset); the filters of eight channels, 288 bytes in a row, go through LDS, rows of 74 floats so that the
 // 32 rows lie in the even banks and the next channel's terms in the odd ones.  A chunk of eight channels is in flight while the one before is multiplied:
 // 36 v_mfma_f32_32x32x2_f32.  Sums of 36 terms are added up separately, which keeps the error of long sums below the split operands': 2-norm against 64 bits
-// for 576, 1152 and 2304 terms 9.6e-8 to 9.9e-8, 1.0e-7 to 1.15e-7 and 1.1e-7 to 1.3e-7 (there 1.0e-7, 1.5e-7 and 2.1e-7).
+// for 576, 1152 and 2304 terms 1.21e-7 to 1.24e-7, 1.23e-7 to 1.26e-7 and 1.29e-7 to 1.34e-7 (there 1.31e-7 to 1.33e-7, 1.85e-7 to 1.9e-7 and 2.7e-7), for 8, 24, 40 and
+// 56 channels, which have no split operands there, 1.1e-7 to 1.2e-7 (1.5e-7 to 3.9e-7).  At 16, 32 and 48 channels the split operands are ahead of such sums, 6.7e-8,
+// 9.3e-8 and 1.15e-7 against 1.13e-7 to 1.21e-7: chains of at most 10 terms, or of 18, are added up in double there, 6.2e-8, 8.1e-8 and 8.1e-8.
 // Bound by the float pipe from a few hundred tiles on (0.74 of it at 4096), before by the latency of a wave's share.  us, general kernel with its copies and
 // this one, 64 -> 64 at 32^2, 128 -> 128 at 16^2 and 256 -> 256 at 8^2: one image 53, 93, 174 and 6.7, 10.7, 16.0; 16 images 50, 95, 176 and 17.9, 17.2, 18.5; 64
 // images 70, 79, 181 and 55, 56, 62.
@@ -44,8 +46,9 @@ struct DirectConvArgs {
     FastDiv div_P, div_W;
 };
 
-// PW waves of a workgroup take 32 pixels each, with the same 32 filters; KS such groups share the channels.
-template <int PW, int KS>
+// PW waves of a workgroup take 32 pixels each, with the same 32 filters; KS such groups share the channels.  CHAIN > 0: chains of that many taps of two
+// channels, and of the rest of the nine, added up in double.
+template <int PW, int KS, int CHAIN>
 __global__ __launch_bounds__(64 * PW * KS) __attribute__((amdgpu_waves_per_eu(2))) void DirectConvKernel(DirectConvArgs p) {
     constexpr int kGroup = 64 * PW;  // threads that share filters
     constexpr int kStagePieces = 32 * kPieces;
@@ -118,9 +121,15 @@ __global__ __launch_bounds__(64 * PW * KS) __attribute__((amdgpu_waves_per_eu(2)
         else __builtin_amdgcn_wave_barrier();  // (filters of its own)
     };
 
-    float16_t sum, acc;
+    constexpr bool DOUBLE = CHAIN > 0;
+    using Sum = std::conditional_t<DOUBLE, double, float>;
+    using Sum16 = __attribute__((ext_vector_type(16))) Sum;
+    Sum16 sum = {};
+    float16_t acc[DOUBLE ? 2 : 1] = {};  // two chains in turn: one is added up while the other grows
+    auto add_up = [&](int chain) {
 #pragma unroll
-    for (int v = 0; v < 16; ++v) sum[v] = 0.f;
+        for (int v = 0; v < 16; ++v) sum[v] += static_cast<Sum>(acc[chain][v]);
+    };
     const int chunks = p.C / kChunk, rounds = (chunks + KS - 1) / KS, own = (chunks - ks + KS - 1) / KS;
     auto multiply = [&](int i, auto next_tag) {
         const int c = (ks + i * KS) * kChunk;
@@ -130,10 +139,13 @@ __global__ __launch_bounds__(64 * PW * KS) __attribute__((amdgpu_waves_per_eu(2)
 #pragma unroll
             for (int k = 0; k < kTaps; ++k) {
                 const float16_t zero = {};
-                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(from[j * 2 * kTaps + k], b[j][k], j % 2 == 0 && k == 0 ? zero : acc, 0, 0, 0);
+                const int chain = DOUBLE ? (CHAIN < kTaps ? k >= CHAIN : j % 2) : 0;
+                const bool first = DOUBLE ? k == 0 || k == CHAIN : j % 2 == 0 && k == 0;
+                acc[chain] = __builtin_amdgcn_mfma_f32_32x32x2f32(from[j * 2 * kTaps + k], b[j][k], first ? zero : acc[chain], 0, 0, 0);
+                if (DOUBLE && first) add_up(1 - chain);
             }
             if constexpr (decltype(next_tag)::value) load_x(j, c + KS * kChunk + 2 * j);
-            if (j % 2 == 1) sum += acc;
+            if (!DOUBLE && j % 2 == 1) add_up(0);
         }
     };
     if (own > 0) {
@@ -156,31 +168,37 @@ __global__ __launch_bounds__(64 * PW * KS) __attribute__((amdgpu_waves_per_eu(2)
     }
 
     // lane holds pixel r, filters 8 * (v / 4) + 4 * g + v % 4; each wave adds up its share of them
+    if (DOUBLE) add_up(1);
     constexpr int kShare = 16 / KS;
     __syncthreads();  // the staging areas become partial sums
+    Sum* const parts = reinterpret_cast<Sum*>(lds);
 #pragma unroll
-    for (int v = 0; v < 16; ++v) lds[(wave * 16 + v) * 64 + lane] = sum[v];
+    for (int v = 0; v < 16; ++v) parts[(wave * 16 + v) * 64 + lane] = sum[v];
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < kShare; ++i) {
         const int v = ks * kShare + i, row = 8 * (v / 4) + v % 4, n = n0 + row + 4 * g;
-        float s = 0.f;
+        Sum total = 0;
 #pragma unroll
-        for (int k = 0; k < KS; ++k) s += lds[((k * PW + pw) * 16 + v) * 64 + lane];
+        for (int k = 0; k < KS; ++k) total += parts[((k * PW + pw) * 16 + v) * 64 + lane];
+        float s = static_cast<float>(total);
         if (p.bias != nullptr) s += n < p.K ? p.bias[n * p.bias_stride] : 0.f;
         __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(s), outr, (in & (n < p.K)) ? to + row * plane : kOut, 0, 0);
     }
 }
 
-template <int PW, int KS>
+template <int PW, int KS, int CHAIN>
 void Launch(DirectConvArgs p, hipStream_t stream) {
-    constexpr int kLds = std::max(KS * 2 * 32 * kPitch, KS * PW * 16 * 64) * 4;
+    constexpr int kLds = std::max(KS * 2 * 32 * kPitch * 4, KS * PW * 16 * 64 * (CHAIN > 0 ? 8 : 4));
     p.tiles_f = (p.K + 31) / 32, p.tiles_p = (p.M + 32 * PW - 1) / (32 * PW);
     struct DirectConvTag {};
-    EnsureDynamicLds<DirectConvTag>(reinterpret_cast<const void*>(DirectConvKernel<PW, KS>), kLds);
-    hipLaunchKernelGGL((DirectConvKernel<PW, KS>), dim3(static_cast<unsigned>(p.tiles_f) * p.tiles_p), dim3(64 * PW * KS), kLds, stream, p);
+    EnsureDynamicLds<DirectConvTag>(reinterpret_cast<const void*>(DirectConvKernel<PW, KS, CHAIN>), kLds);
+    hipLaunchKernelGGL((DirectConvKernel<PW, KS, CHAIN>), dim3(static_cast<unsigned>(p.tiles_f) * p.tiles_p), dim3(64 * PW * KS), kLds, stream, p);
     CheckLaunch("direct_conv");
 }
+
+// Where the split operands of the general kernel, which takes whole groups of 16 channels, have less error than chains of 36 terms.
+bool SumsInDouble(int64_t channels) { return channels % 16 == 0 && channels < 64; }
 
 int64_t Tiles(int64_t pixels, int64_t filters) { return ((pixels + 31) / 32) * ((filters + 31) / 32); }
 
@@ -193,7 +211,10 @@ bool DirectConvTakes(const hipcx_array* x, const hipcx_array* w, const int64_t* 
     // Beyond, the large tiles of the split operands (igemm_split.hip) catch up, copies of x and w included.  us there and here: 64 -> 64 at 32^2, 96 images 87 and 80,
     // 128 images (8192 tiles) 96 and 105; 128 -> 128 at 16^2, 96 images (3072) 88 and 82, 112 images 94 and 101; 256 -> 256 at 8^2, 160 images (2560) 145 and
     // 145, 200 images 152 and 185.
-    if (Tiles(N * P, K) > (K <= 64 ? 24 : 12) * NumCUs()) return false;
+    // Half to two thirds of that where sums are in double, whose additions bound the kernel: 64 filters, 12 and 16 tiles to a compute unit, 16 channels 25.8 and 23.0,
+    // 27.7 and 29.6, 32 channels 35.5 and 30.0, 40.6 and 38.7; 128 filters, 8 and 12, 21.8 and 17.0, 23.3 and 24.4, 48 channels 36.2 and 27.7, 38.3 and 39.5.
+    const int most = SumsInDouble(C) ? (K <= 64 ? 12 : 8) : (K <= 64 ? 24 : 12);
+    if (Tiles(N * P, K) > most * NumCUs()) return false;
     if (w->shape[2] != 3 || w->shape[3] != 3 || stride[0] != 1 || stride[1] != 1 || pad[0] != 1 || pad[1] != 1) return false;
     if (out->shape[2] != x->shape[2] || out->shape[3] != x->shape[3] || C % kChunk != 0 || C == 0) return false;
     // 32-bit offsets from a tile's first image
@@ -215,9 +236,15 @@ void DirectConv(const hipcx_array* x, const hipcx_array* w, const hipcx_array* b
     // images (256 tiles) 7.4 10.3 16.2, 6 images 12.2 10.7 16.5, 12 images 18.1 19.2 17.4, 64 images 84 73 55; 256 -> 256 at 8^2, 16 images (256 tiles)
     // 18.5 26.9 57, 48 images 50 53 61, 80 images 81 78 96, 128 images 128 105 104.
     const int64_t tiles = Tiles(p.M, K), cus = NumCUs();
-    if (tiles <= cus) Launch<1, 8>(p, stream);
-    else if (tiles <= (C >= 128 ? 6 : 2) * cus) Launch<2, 4>(p, stream);
-    else Launch<4, 2>(p, stream);
+    auto run = [&](auto taps) {
+        constexpr int CHAIN = decltype(taps)::value;
+        if (tiles <= cus) Launch<1, 8, CHAIN>(p, stream);
+        else if (tiles <= (C >= 128 ? 6 : 2) * cus) Launch<2, 4, CHAIN>(p, stream);
+        else Launch<4, 2, CHAIN>(p, stream);
+    };
+    if (!SumsInDouble(C)) run(std::integral_constant<int, 0>{});
+    else if (C == 16) run(std::integral_constant<int, 5>{});
+    else run(std::integral_constant<int, kTaps>{});
 }
 
 }  // namespace hipcx

@@ -66,3 +66,26 @@ def test_both_operands_k_by_k(m, k, n):
     ref = a.astype(np.float64) @ b
     got = chx.dot(chx.array(np.ascontiguousarray(a.T)).T, chx.array(b)).get()
     assert relative(got, ref) <= relative(chain(a, b), ref) * 1.001
+
+
+@pytest.mark.parametrize('images', [2, 16, 48])  # eight, four and two groups of waves to a tile's channels
+@pytest.mark.parametrize('c,bound', [(16, 6.4e-8), (32, 8.8e-8), (48, 1.09e-7)])  # what the general kernel's split operands have at least
+def test_convolutions_of_few_channels(c, bound, images):
+    rng = np.random.default_rng(c)
+    x, f = rng.standard_normal((images, c, 32, 32), dtype=np.float32), rng.standard_normal((33, c, 3, 3), dtype=np.float32)
+    if images < 48:
+        assert chx.conv_route(chx.array(x), chx.array(f), None, 1, 1) == 6
+    few = x[::max(1, images // 2)][:2].astype(np.float64)
+    padded = np.pad(few, ((0, 0), (0, 0), (1, 1), (1, 1)))
+    ref = sum(np.tensordot(f[:, :, r, s].astype(np.float64), padded[:, :, r:r + 32, s:s + 32], (1, 1)).transpose(1, 0, 2, 3) for r in range(3) for s in range(3))
+    got = chx.conv(chx.array(x), chx.array(f), None, 1, 1).get()[::max(1, images // 2)][:2]
+    assert relative(got, ref) < bound
+
+
+def test_convolutions_of_few_channels_leave_to_the_general_kernel_earlier():
+    def route(n, c, k):
+        return chx.conv_route(chx.zeros((n, c, 8, 8), np.float32), chx.zeros((k, c, 3, 3), np.float32), None, 1, 1)
+    for c in (16, 32, 48):
+        assert route(3 * 256, c, 64) == 6 and route(3 * 256 + 1, c, 64) == 0  # 12 tiles of 32 x 32 to a compute unit, 256 of these
+        assert route(4 * 64, c, 128) == 6 and route(4 * 64 + 1, c, 128) == 0    # 8
+    assert route(3 * 256 + 1, 64, 64) == 6
