@@ -206,12 +206,24 @@ __global__ __launch_bounds__(512) void LstmStepKernel(LstmStepArgs p) {
     static_cast<T*>(p.h_out)[m * p.h_out_row + u] = static_cast<T>(h);
 }
 
+constexpr int kExactTerms = 64;  // float32 reductions of fewer terms are summed in double
+
 int64_t StepTiles(int64_t rows, int64_t units, int blocks) { return (rows + 31) / 32 * ((units + 4 * blocks - 1) / (4 * blocks)); }
 
 // Up to four (float16: six) tiles of 32 rows and 16 units to a compute unit: beyond, the tiles of a large product read each operand less often.  us, the four
 // calls and one, float32: 768 x 650 units, 3.8 tiles, 90.7, 85.5; 4096 x 128, 4, 50.9, 25.6; 1024 x 650, 5.1, 116, 123; 512 x 2048, 8, 282, 336.  float16: 1024 x 650
 // 64.7, 49.9; 2048 x 300, 4.8, 41.0, 28.7; 1024 x 1024, 8, 69.4, 75.1; 512 x 2048 94.4, 111.
-bool StepTakes(int64_t rows, int64_t units, int dtype) { return StepTiles(rows, units, 4) <= (dtype == HIPCX_FLOAT32 ? 4 : 6) * NumCUs(); }
+// And up to a number of terms, over the rounds of tiles that a compute unit takes: the separate products split theirs over workgroups, or run in larger tiles.
+// float32 (rounds x terms): 445 x 567 of 594 inputs (2322) 43.1, 37.6; 57 x 79 of 3388 (3467) 15.3, 15.0; 52 x 168 of 5347 (5515) 22.3, 21.3; 886 x 419 of 2576
+// (8985) 112, 114; 107 x 112 of 9223 (9335) 30.2, 35.7; 169 x 1537 of 7891 (28284) 217, 285.  float16: 245 x 1465 of 238 (5109) 40.7, 31.3; 144 x 948 of 2967 (7830)
+// 35.3, 37.5; 606 x 9 of 9241 (9250) 19.5, 22.0; 3003 x 184 of 7054 (36190) 83, 149.  In double, in tiles of 4 units: 8192 x 16 (128) 23.8, 10.5; 4096 x 50 (700) 37.8,
+// 15.8; 32 x 15 of 940 (955) 12.3, 10.1; 3 x 27 of 975 (1002) 9.8, 10.2; 508 x 319 of 23 (1710) 20.9, 22.2; 128 x 2048 of 50 (16784) 66, 116.
+bool StepTakes(int64_t rows, int64_t units, int64_t inputs, int dtype) {
+    if (StepTiles(rows, units, 4) > (dtype == HIPCX_FLOAT32 ? 4 : 6) * NumCUs()) return false;
+    const bool exact = dtype == HIPCX_FLOAT32 && std::min(inputs, units) < kExactTerms;
+    const int64_t rounds = (StepTiles(rows, units, exact ? 1 : 4) + NumCUs() - 1) / NumCUs();
+    return rounds * (inputs + units) <= (exact ? 960 : dtype == HIPCX_FLOAT32 ? 5300 : 7800);
+}
 
 template <typename T>
 void RunLstmStep(LstmStepArgs& p, hipStream_t stream) {
@@ -229,7 +241,7 @@ void RunLstmStep(LstmStepArgs& p, hipStream_t stream) {
     using One = integral_constant<int, 1>;
     using Two = integral_constant<int, 2>;
     if constexpr (sizeof(T) == 4) {
-        if (std::min(p.side[0].K, p.side[1].K) < 64) return run(0.0, One{}, Two{});
+        if (std::min(p.side[0].K, p.side[1].K) < kExactTerms) return run(0.0, One{}, Two{});
     }
     int nb = 4;  // the narrowest tiles that find each of them a compute unit
     for (int b = 3; b >= 1; --b) {
@@ -263,7 +275,7 @@ int hipcx_lstm_step_supported(const hipcx_array* c, const hipcx_array* x, const 
     if (c == nullptr || x == nullptr || wx == nullptr || h == nullptr || wh == nullptr) return 0;
     if ((c->dtype != HIPCX_FLOAT32 && c->dtype != HIPCX_FLOAT16) || c->ndim != 2 || x->ndim != 2) return 0;
     const int64_t M = c->shape[0], H = c->shape[1], piece = 16 / ItemSize(c->dtype);
-    if (M < 1 || H < 1 || H >= (1 << 28) || !StepTakes(M, H, c->dtype)) return 0;
+    if (M < 1 || H < 1 || H >= (1 << 28) || !StepTakes(M, H, x->shape[1], c->dtype)) return 0;
     return StepRows(c, M, H, c->dtype, 1) && StepRows(x, M, x->shape[1], c->dtype, piece) && StepRows(h, M, H, c->dtype, piece) &&
            StepRows(wx, 4 * H, x->shape[1], c->dtype, piece) && StepRows(wh, 4 * H, H, c->dtype, piece) &&
            (bx == nullptr || (bx->ndim == 1 && bx->dtype == c->dtype && bx->shape[0] == 4 * H && bx->strides[0] % ItemSize(c->dtype) == 0));

@@ -63,3 +63,17 @@ def test_views_special_values_and_what_is_composed(dt):
         chx.lstm_step(C, X, WX[4:], B[4:], H, WH[4:])
     with pytest.raises(chx.DtypeError):
         chx.lstm_step(C, X.astype('float64'), WX, B, H, WH)
+
+
+@pytest.mark.parametrize('dt,rows,n_in,units,taken', [
+    ('float32', 128, 650, 650, True), ('float32', 768, 650, 650, True), ('float32', 1024, 650, 650, False),  # rounds of tiles x terms: 1300, 5200; too many tiles
+    ('float32', 20, 5000, 300, True), ('float32', 20, 5001, 300, False),                                    # 5300 terms in one round
+    ('float16', 20, 7500, 300, True), ('float16', 20, 7501, 300, False),                                    # 7800
+    ('float32', 32, 910, 50, True), ('float32', 32, 911, 50, False), ('float16', 32, 911, 50, True),        # 960, in double
+    ('float32', 4096, 50, 50, True), ('float32', 8192, 63, 63, False), ('float32', 128, 50, 2048, False),   # 700, 2016, 16784
+    ('float32', 4, 3, 20, False), ('float16', 4, 20, 7, False)])                                            # rows shorter than 16 bytes
+def test_what_is_taken(dt, rows, n_in, units, taken):
+    import chainer_amd as chx
+    from chainer_amd import _host
+    c, x, wx, b, h, wh = [chx.zeros(s, dt) for s in ((rows, units), (rows, n_in), (4 * units, n_in), (4 * units,), (rows, units), (4 * units, units))]
+    assert (_host.lstm_step_direct(c, x, wx, b, h, wh) is not None) == taken
