@@ -430,8 +430,9 @@ ShiftedPlan PlanShifted(const GradWeightPlan& pl, int dtype, bool pairs) {
     const int64_t Hp = g.H + 2 * static_cast<int64_t>(g.ph), copies = pairs ? std::min(g.kw, 2) : g.kw;
     // windows of a pair's copies start up to kw - 1 elements later than those of copies of their own, and end as much later
     const int64_t pitch_x = (Hp * Wp + (pairs ? (g.kw - 1) / 2 * 2 : 0) + epc - 1) / epc * epc, pitch_gy = (g.OH * Wp + epc - 1) / epc * epc;
-    // worth it when the copies are smaller than the kh*kw-fold Im2Col
-    if (copies * pitch_x >= static_cast<int64_t>(g.kh) * g.kw * g.OH * g.OW) return sp;
+    // worth it when kw copies of rows of whole granules are smaller than the kh*kw-fold Im2Col, also where it is two copies of shorter rows: small planes and
+    // filters are faster as one Dot.  us, Im2Col and two copies: 2x2 on 7 x 7 8.7 and 15.8, 3x3 on 9 x 3 10.5 and 19.1, 5x5 on 13 x 3 99 and 214.
+    if (g.kw * Hp * ((W + 2 * pw + epc - 1) / epc * epc) >= static_cast<int64_t>(g.kh) * g.kw * g.OH * g.OW) return sp;
     const int64_t most = int64_t{1} << 31;
     if (static_cast<int64_t>(g.H) * W == 0 || pitch_x + 256 * epc >= most || N * g.C >= most || N * g.K >= most) return sp;  // (the copy kernel's 32-bit indices)
     sp.a.set[0] = PlaneSet{g.x, nullptr, static_cast<int>(N * g.C), g.H, g.W, g.ph, g.pw, static_cast<int>(copies), static_cast<int>(pitch_x)};
