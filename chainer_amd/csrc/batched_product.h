@@ -20,7 +20,7 @@ struct BatchedOperands {
 };
 
 // Workgroups per tile along the reduction; slices > 1 need slices * m * n floats of partial sums.
-int HalfProductSlices(int64_t m, int64_t n, int64_t depth, int64_t batch);
+int HalfProductSlices(const BatchedOperands& o);
 
 // Whether the operands' alignment, spans and extents are within what the kernel addresses.  Null operands: every address is taken to be aligned.
 bool HalfProductApplies(const BatchedOperands& o);

@@ -238,13 +238,15 @@ double Bytes(int64_t rows, int64_t row, int64_t slice, const BatchedOperands& o)
 
 // One workgroup to a compute unit (its ring then has the unit's whole bandwidth; two: 4 % slower, three: 8 %), two where one each would leave more than a
 // quarter of the chip idle (144 tiles of 3x3 of 512 channels on 7 x 7: 73 -> 56 us).  Slices of 8 chunks at least: of 4, the sum outweighs the
-// shorter loops (458 against 426 us over ResNet-50's shapes at batch 8); 16 is the same.  Multiples of 8, for the L2s.
-int HalfProductSlices(int64_t m, int64_t n, int64_t depth, int64_t batch) {
-    const int64_t tiles = std::max<int64_t>(1, ((m + 127) / 128) * ((n + 127) / 128)), chunks = (depth + 31) / 32 * batch;
+// shorter loops (458 against 426 us over ResNet-50's shapes at batch 8); 16 is the same.  Multiples of 8, for the L2s.  Windows of a larger array make eight
+// slices or more of 6 chunks already, which their tight rows of 14 would otherwise turn into half as many of the double length (24 images of 11 x 11, 50
+// filters, 15 slices of 8: 11.3 us in 8, 9.0 in 16; 1x1 filters of 970 channels on 16 x 16 gain nothing, 16.1 and 18.3).
+int HalfProductSlices(const BatchedOperands& o) {
+    const int64_t tiles = std::max<int64_t>(1, ((int64_t{o.M} + 127) / 128) * ((int64_t{o.N} + 127) / 128)), chunks = (int64_t{o.depth} + 31) / 32 * o.batch;
     const int64_t cus = NumCUs();
     int64_t s = cus / tiles;
     if (s * tiles < cus * 3 / 4) s = 2 * cus / tiles;
-    s = std::min(s, chunks / 8);
+    s = std::min(s, o.taps_s > 0 && chunks / 6 >= 8 ? chunks / 6 : chunks / 8);
     if (s >= 8) s = s / 8 * 8;
     return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(s, 256)));
 }

@@ -131,11 +131,21 @@ struct PlaneSet {
 struct PlanesArgs {
     PlaneSet set[2];  // x, gy
     int Wp;
-    int* nonfinite;  // [planes of x]: whether it holds an inf or NaN
-    int each;        // planes of a workgroup, kMostPlanes at most
+    int* nonfinite;  // [channels][images][parts]: whether that part of a plane of x holds an inf or NaN
+    int images, channels;
+    bool pairs;       // float16: rows of gy hold two elements or more and its copy's an even number
+    int each;         // planes of a workgroup, kMostPlanes at most
+    int parts, share;  // workgroups to a plane, where each is 1, and pieces that each of them takes
     int64_t blocks_x, blocks;
 };
 constexpr int kMostPlanes = 64;
+
+struct __attribute__((packed, aligned(2))) AnyDword {
+    unsigned v;
+};
+struct alignas(16) Dwords {
+    unsigned v[4];
+};
 
 template <typename T>
 __device__ __forceinline__ bool NonFinite(T v) {
@@ -146,10 +156,12 @@ __device__ __forceinline__ bool NonFinite(T v) {
     }
 }
 
-// Both sets in one pass.  A workgroup takes a few whole planes, whose pieces of 16 bytes are dealt out to its threads; a piece's elements are gathered
-// once, and each further copy takes one more.  Bound by the gathers, an element a lane; 64 threads to a plane, of which the 33 pieces of a 14 x 14 one
-// use half, make the whole call of 256 channels, 32 images, 38.9 us instead of 35.8.  us of the call in float16, three copies of rows of whole granules from
-// two kernels and now, 32 images: 64 channels at 56^2 61 -> 53, 128 at 28^2 42 -> 38, 256 at 14^2 37.7 -> 35.8, 512 at 7^2 54 -> 39.
+// Both sets in one pass.  A workgroup takes a few whole planes or a part of one, whose pieces of 16 bytes are dealt out to its threads; a piece's elements are
+// gathered once, and each further copy takes one more, which is asked for with the rest.  Bound by the gathers, an element of x or two of gy a lane (324 channels of
+// gy, 17 images of 60^2, element by element 26.3 us, 17.0 so), and by their latency where planes are few: two pieces to a thread and no parts of planes made
+// 6 images of 80 to 125 channels on 5 x 5 18.0 us instead of 16.5, 2 of 41 to 12 on 62 x 62 20.1 instead of 15.5.  64 threads to a plane, of which the 33 pieces
+// of a 14 x 14 one use half, make the whole call of 256 channels, 32 images, 38.9 us instead of 35.8.  us of the call in float16, three copies of rows of whole
+// granules from two kernels and now, 32 images: 64 channels at 56^2 62 -> 52, 128 at 28^2 43 -> 39, 256 at 14^2 38 -> 35, 512 at 7^2 55 -> 37.
 template <typename T>
 __global__ __launch_bounds__(256) void PlanesKernel(PlanesArgs p) {
     constexpr int E = 16 / sizeof(T);
@@ -157,18 +169,38 @@ __global__ __launch_bounds__(256) void PlanesKernel(PlanesArgs p) {
     for (int64_t block = blockIdx.x; block < p.blocks; block += gridDim.x) {
         const bool of_x = block < p.blocks_x;
         const PlaneSet& o = p.set[of_x ? 0 : 1];
-        const int64_t plane0 = (of_x ? block : block - p.blocks_x) * p.each;
+        const int64_t own = of_x ? block : block - p.blocks_x;
+        const int64_t plane0 = p.parts > 1 ? static_cast<unsigned>(own) / static_cast<unsigned>(p.parts) : own * p.each;
         const int planes = static_cast<int>(min(static_cast<int64_t>(p.each), o.planes - plane0)), pieces = o.pitch / E;
+        int begin = 0, end = planes * pieces, part = 0;
+        if (p.parts > 1) {  // (of one plane)
+            part = static_cast<int>(own - plane0 * p.parts);
+            begin = part * p.share, end = min(pieces, begin + p.share);
+        }
         if (of_x) {
             if (threadIdx.x < kMostPlanes) flags[threadIdx.x] = 0;
             __syncthreads();
         }
-        for (int i = threadIdx.x; i < planes * pieces; i += 256) {
+        for (int i = begin + threadIdx.x; i < end; i += 256) {
             const int local = static_cast<unsigned>(i) / static_cast<unsigned>(pieces), q = (i - local * pieces) * E;
             const int64_t plane = plane0 + local;
             const T* const from = static_cast<const T*>(o.from) + plane * o.H * o.W;
             T* const to = static_cast<T*>(o.to) + plane * o.pitch + q;
             int row = static_cast<unsigned>(q) / static_cast<unsigned>(p.Wp), col = q - row * p.Wp;
+            if constexpr (sizeof(T) == 2) {
+                if (!of_x && p.pairs) {  // rows of an even pitch without padding in front: both elements of a dword lie in one row
+                    Dwords out;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const bool inside = row < o.H && col < o.W, alone = col + 1 == o.W;  // (nothing behind an odd row's last element is read)
+                        const unsigned v = reinterpret_cast<const AnyDword*>(from + (inside ? row * o.W + col - alone : 0))->v >> (alone ? 16 : 0);
+                        out.v[e] = inside ? v : 0u;
+                        if ((col += 2) == p.Wp) col = 0, ++row;
+                    }
+                    *reinterpret_cast<Dwords*>(to) = out;
+                    continue;
+                }
+            }
             auto next = [&] {
                 const int h = row - o.ph, w = col - o.pw;
                 const bool inside = h >= 0 && h < o.H && w >= 0 && w < o.W;
@@ -179,6 +211,7 @@ __global__ __launch_bounds__(256) void PlanesKernel(PlanesArgs p) {
             GVec<T, E> out;
 #pragma unroll
             for (int e = 0; e < E; ++e) out.v[e] = next();
+            T more = o.copies > 1 ? next() : T(0);
             bool bad = false;
 #pragma unroll
             for (int e = 0; e < E; ++e) bad |= NonFinite<T>(out.v[e]);
@@ -187,13 +220,17 @@ __global__ __launch_bounds__(256) void PlanesKernel(PlanesArgs p) {
             for (int s = 1; s < o.copies; ++s) {
 #pragma unroll
                 for (int e = 0; e + 1 < E; ++e) out.v[e] = out.v[e + 1];
-                out.v[E - 1] = next();
+                out.v[E - 1] = more;
                 *reinterpret_cast<GVec<T, E>*>(to + static_cast<int64_t>(s) * o.planes * o.pitch) = out;
+                if (s + 1 < o.copies) more = next();
             }
         }
         if (of_x) {
             __syncthreads();
-            if (threadIdx.x < planes) p.nonfinite[plane0 + threadIdx.x] = flags[threadIdx.x];
+            if (threadIdx.x < planes) {
+                const int plane = static_cast<int>(plane0) + threadIdx.x, n = plane / p.channels;
+                p.nonfinite[(static_cast<int64_t>(plane - n * p.channels) * p.images + n) * p.parts + part] = flags[threadIdx.x];
+            }
             __syncthreads();
         }
     }
@@ -203,14 +240,15 @@ __global__ __launch_bounds__(256) void PlanesKernel(PlanesArgs p) {
 // gy[n][k][oh][ow] * col, col = x[n][c][oh*sh - ph + r][ow*sw - pw + s] or the padding's zero (still multiplied, as TensorDot
 // multiplies Im2Col's zeros: CX/native/native_device/conv.cc:91-124).  Grid (C, slices); a wave per output, lanes over the sum.
 template <typename T>
-__global__ __launch_bounds__(256) void GradWeightChannelFixupKernel(GradWeightArgs p, const int* nonfinite, T* gw) {
+__global__ __launch_bounds__(256) void GradWeightChannelFixupKernel(GradWeightArgs p, const int* nonfinite, int parts, T* gw) {
     const int c = blockIdx.x;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t flags = static_cast<int64_t>(p.N) * parts;
     int any = 0;
-    for (int n = threadIdx.x; n < p.N; n += 256) any |= nonfinite[static_cast<int64_t>(n) * p.C + c];
-    if (__syncthreads_or(any) == 0) return;
+    for (int64_t i = lane; i < flags; i += 64) any |= nonfinite[c * flags + i];
+    if (__ballot(any) == 0) return;  // (a wave)
     const T* x = static_cast<const T*>(p.x);
     const T* gy = static_cast<const T*>(p.gy);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int taps = p.kh * p.kw, outputs = p.K * taps;
     const int64_t plane = static_cast<int64_t>(p.OH) * p.OW, total = plane * p.N;
     for (int o = blockIdx.y * 4 + wave; o < outputs; o += gridDim.y * 4) {
@@ -365,7 +403,7 @@ Product PlanProduct(const void* a, int64_t a_row, int64_t a_slice, const void* b
     pr.dtype = dtype;
     pr.half = dtype == HIPCX_FLOAT16 && std::max(std::max(m, n), depth) < (1LL << 31) && HalfProductApplies(o);
     if (pr.half) {
-        const int slices = HalfProductSlices(m, n, depth, batch);
+        const int slices = HalfProductSlices(o);
         pr.partial_bytes = slices > 1 ? static_cast<size_t>(slices) * m * n * sizeof(float) : 0;
     } else {
         pr.partial_bytes = BatchedProductPartialBytes(m, n, depth, o.batch, dtype);
@@ -376,7 +414,7 @@ Product PlanProduct(const void* a, int64_t a_row, int64_t a_slice, const void* b
 void RunProduct(const Product& pr, void* partial, hipStream_t stream) {
     const BatchedOperands& o = pr.o;
     float* const sums = pr.partial_bytes ? static_cast<float*>(partial) : nullptr;
-    if (pr.half) HalfProduct(o, sums, HalfProductSlices(o.M, o.N, o.depth, o.batch), stream);
+    if (pr.half) HalfProduct(o, sums, HalfProductSlices(o), stream);
     else LaunchBatchedProduct(pr.dtype, o.a, o.a_row, o.a_slice, o.b, o.b_row, o.b_slice, o.M, o.N, o.depth, o.batch, o.out, sums, stream, o.taps_r, o.taps_s, o.r_stride, o.s_stride);
 }
 
@@ -438,7 +476,16 @@ ShiftedPlan PlanShifted(const GradWeightPlan& pl, int dtype, bool pairs) {
     sp.a.set[0] = PlaneSet{g.x, nullptr, static_cast<int>(N * g.C), g.H, g.W, g.ph, g.pw, static_cast<int>(copies), static_cast<int>(pitch_x)};
     sp.a.set[1] = PlaneSet{g.gy, nullptr, static_cast<int>(N * g.K), g.OH, g.OW, 0, 0, 1, static_cast<int>(pitch_gy)};
     sp.a.Wp = static_cast<int>(Wp);
-    sp.flag_bytes = RoundUp256(static_cast<size_t>(N * g.C) * sizeof(int));
+    sp.a.images = g.N, sp.a.channels = g.C;
+    sp.a.pairs = Wp % 2 == 0 && g.OW >= 2;
+    // A piece to a thread: planes together, or less where that leaves compute units without a workgroup, or parts of a plane; two pieces once the chip is full.
+    const int64_t pieces = pitch_x / epc, planes = N * (static_cast<int64_t>(g.C) + g.K), cus = NumCUs();
+    sp.a.each = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>({kMostPlanes, (planes * pieces >= 4096 * cus ? 512 : 256) / pieces, planes / cus})));
+    sp.a.parts = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>((pieces + 255) / 256, 8 * cus / planes)));
+    sp.a.share = static_cast<int>((pieces + sp.a.parts - 1) / sp.a.parts);
+    sp.a.blocks_x = (sp.a.set[0].planes + int64_t{sp.a.each} - 1) / sp.a.each * sp.a.parts;
+    sp.a.blocks = sp.a.blocks_x + (sp.a.set[1].planes + int64_t{sp.a.each} - 1) / sp.a.each * sp.a.parts;
+    sp.flag_bytes = RoundUp256(static_cast<size_t>(N * g.C) * sp.a.parts * sizeof(int));
     sp.xs_bytes = RoundUp256(static_cast<size_t>(copies * N * g.C * pitch_x * it));
     sp.gyp_bytes = RoundUp256(static_cast<size_t>(N * g.K * pitch_gy * it));
     sp.product = ShiftedProduct(sp, g, nullptr, dtype);
@@ -466,21 +513,17 @@ Product StagedProduct(const GradWeightPlan& pl, void* gw, int dtype) {
 }
 
 template <typename T>
-void RunPlanes(PlanesArgs a, hipStream_t stream) {
-    // two pieces to a thread, or a plane
-    a.each = std::max(1, std::min(kMostPlanes, 512 / (a.set[0].pitch / static_cast<int>(16 / sizeof(T)))));
-    a.blocks_x = (a.set[0].planes + int64_t{a.each} - 1) / a.each;
-    a.blocks = a.blocks_x + (a.set[1].planes + int64_t{a.each} - 1) / a.each;
+void RunPlanes(const PlanesArgs& a, hipStream_t stream) {
     hipLaunchKernelGGL((PlanesKernel<T>), dim3(static_cast<unsigned>(std::min<int64_t>(a.blocks, 1 << 22))), dim3(256), 0, stream, a);
     CheckLaunch("padded planes (weight gradient)");
 }
 
 template <typename T>
-void RunChannelFixup(const GradWeightArgs& g, const int* nonfinite, void* gw, hipStream_t stream) {
+void RunChannelFixup(const GradWeightArgs& g, const PlanesArgs& planes, void* gw, hipStream_t stream) {
     const int outputs = g.K * g.kh * g.kw;
     const int slices = std::max(1, std::min(outputs / 4, 16));
     hipLaunchKernelGGL((GradWeightChannelFixupKernel<T>), dim3(static_cast<unsigned>(g.C), static_cast<unsigned>(slices)), dim3(256), 0, stream, g,
-                       nonfinite, static_cast<T*>(gw));
+                       planes.nonfinite, planes.parts, static_cast<T*>(gw));
     CheckLaunch("non-finite channels (weight gradient)");
 }
 }  // namespace
@@ -545,8 +588,8 @@ int hipcx_conv_grad_weight(const hipcx_array* x, const hipcx_array* gy, const in
             else RunPlanes<float>(sp.a, st);
             const GradWeightArgs& g = pl.a;
             RunProduct(ShiftedProduct(sp, g, gw->data, gw->dtype), ws + sp.xs_bytes + sp.gyp_bytes, st);
-            if (gw->dtype == HIPCX_FLOAT16) RunChannelFixup<half_t>(g, sp.a.nonfinite, gw->data, st);
-            else RunChannelFixup<float>(g, sp.a.nonfinite, gw->data, st);
+            if (gw->dtype == HIPCX_FLOAT16) RunChannelFixup<half_t>(g, sp.a, gw->data, st);
+            else RunChannelFixup<float>(g, sp.a, gw->data, st);
             return;
         }
         const size_t dot_bytes = hipcx_dot_workspace_size(&pl.gy_t, &pl.col_view, &out);

@@ -28,3 +28,21 @@ def test_against_oracle(n, c, h, w, k, size, pad, dtype):
     x[n - 1, 0, 0, 0], x[0, c - 1, h - 1, w - 1] = np.inf, np.nan
     gw = chx.conv_grad_weight(dtype, shape, chx.array(x), chx.array(gy), 1, pad, False).get()
     np.testing.assert_array_equal(gw, O.conv_grad_weight(shape, x, gy, 1, pad, False))
+
+
+@pytest.mark.parametrize('dtype', ['float16', 'float32'])
+@pytest.mark.parametrize('n,c,h,w,k,size,pad', [
+    (1, 2, 70, 131, 3, (3, 3), (1, 1)), (2, 1, 129, 64, 5, (3, 3), (0, 1)),   # several workgroups to a plane
+    (2, 3, 40, 41, 90, (3, 3), (1, 1)), (2, 3, 40, 40, 90, (2, 3), (1, 0)),   # rows of gy of an odd and of an even number
+    (3, 5, 90, 3, 4, (3, 3), (1, 0)), (3, 5, 90, 3, 4, (3, 2), (1, 0)),       # of one and of two
+    (65, 3, 7, 7, 4, (3, 3), (1, 1)), (130, 40, 7, 7, 30, (3, 3), (1, 1))])   # more flags of a channel than lanes; two pieces to a thread
+def test_parts_of_planes_and_rows_of_gy(n, c, h, w, k, size, pad, dtype):
+    test_against_oracle(n, c, h, w, k, size, pad, dtype)
+    # the last part of the last plane flags its channel
+    rng = np.random.default_rng(w)
+    shape = (k, c) + size
+    x = rng.integers(-1, 2, (n, c, h, w)).astype(dtype)
+    gy = rng.integers(-1, 2, (n, k, h + 2 * pad[0] - size[0] + 1, w + 2 * pad[1] - size[1] + 1)).astype(dtype)
+    x[n - 1, c - 1, h - 1, w - 1] = np.inf
+    gw = chx.conv_grad_weight(dtype, shape, chx.array(x), chx.array(gy), 1, pad, False).get()
+    np.testing.assert_array_equal(gw, O.conv_grad_weight(shape, x, gy, 1, pad, False))
