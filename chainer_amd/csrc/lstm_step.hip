@@ -57,19 +57,21 @@ struct LstmStepArgs {
 // lines turned round in LDS of its own, two of them in flight while a third is multiplied (three and four: equal or slower, [512,650] float32 78 us
 // against 62).  Rows beyond M and columns beyond 4H repeat the last one (nobody reads what comes of them); the pieces that reach beyond the end of K
 // are read from its last 16 bytes, without what the one before them holds.  Loads take any address, so odd pitches of float16 need no kernel of their own.
-// Sums: 16 (8 for few rows) products to a chain, the chains of a chunk, the chunks, the waves, so that no case has a larger error than the separate calls
+// Sums: 16 (8 for few rows or few terms) products to a chain, the chains of a chunk, the chunks, the waves, so that no case has a larger error than the separate calls
 // (2-norm of the error of h and c, against 64 bits, separate calls and this: 128 x 650 units 1.06e-7, 6.8e-8, 1 x 650 5.2e-8, 5.1e-8, 2 x 77 of 129 inputs
 // 4.57e-8, 4.56e-8); Acc = double for reductions of fewer than 64 terms, whose separate products are exact but for a rounding.
 // Bound by the matrix pipe and by the delivery of operands at 128 rows, by the latency of launch, first loads and sums below.  us, the four calls and this,
 // back to back on the device: 128 x 650 units float32 27.7, 18.6 (7.1 of MFMA on 220 compute units), float16 17.3, 8.9; 20 x 650 15.6, 8.8; 1 x 650 9.7, 6.8; 1 x 50
 // 22.5, 4.3; float16 of an odd number of units, 37 x 77 of 129 inputs 15.2, 4.6.
-template <typename T, typename Acc, int NB, int RB>
+template <typename T, typename Acc, int NB, int RB, int CH>
 __global__ __launch_bounds__(512) void LstmStepKernel(LstmStepArgs p) {
     constexpr int PL = 16 / sizeof(T);
     constexpr int KC = 8 * PL;  // k per chunk
     using Acc4 = std::conditional_t<sizeof(Acc) == 8, double4_t, float4_t>;
     constexpr bool kExact = sizeof(Acc) == 8;
-    constexpr int CH = sizeof(T) == 4 && RB == 1 && !kExact ? 4 : 2;  // chains of additions that a chunk makes
+    static_assert(CH == 2 || (CH == 4 && sizeof(T) == 4 && !kExact));  // chains of additions that a chunk makes
+    constexpr bool kHalves = CH == 4 && RB == 2;  // whose chains are added up by half a chunk: there are no registers for all of them
+    constexpr int kKept = kHalves ? 2 : CH;
     constexpr int AL = 2 * RB, BL = 2 * NB;  // loads of a and w per chunk, 8 rows each
     constexpr int kRowsOfW = 16 * RB * kSmallDotPitch, kStage = kRowsOfW + 16 * NB * kSmallDotPitch, kPitch = 16 * NB + 4;
     extern __shared__ __align__(16) char lds[];
@@ -137,7 +139,7 @@ __global__ __launch_bounds__(512) void LstmStepKernel(LstmStepArgs p) {
         for (int j = 0; j < BL; ++j) *reinterpret_cast<Bytes16*>(to + kRowsOfW + j * 8 * kSmallDotPitch) = wv[st][j];
         next();
         __builtin_amdgcn_wave_barrier();
-        Acc4 terms[CH][RB][NB];
+        Acc4 terms[kKept][RB][NB];
 #pragma unroll
         for (int q = 0; q < 2; ++q) {  // pieces g and g + 4 of each row
             Bytes16 fa[RB], fb[NB];
@@ -152,16 +154,17 @@ __global__ __launch_bounds__(512) void LstmStepKernel(LstmStepArgs p) {
                     Acc4 t[CH / 2];
                     Terms<T>(fa[i], fb[j], t);
 #pragma unroll
-                    for (int e = 0; e < CH / 2; ++e) terms[q * CH / 2 + e][i][j] = t[e];
+                    for (int e = 0; e < CH / 2; ++e) terms[(kHalves ? 0 : q * CH / 2) + e][i][j] = t[e];
+                }
+            if (!kHalves && q == 0) continue;
+#pragma unroll
+            for (int i = 0; i < RB; ++i)
+#pragma unroll
+                for (int j = 0; j < NB; ++j) {
+                    if constexpr (kKept == 2) acc[i][j] += terms[0][i][j] + terms[1][i][j];
+                    else acc[i][j] += (terms[0][i][j] + terms[1][i][j]) + (terms[2][i][j] + terms[3][i][j]);
                 }
         }
-#pragma unroll
-        for (int i = 0; i < RB; ++i)
-#pragma unroll
-            for (int j = 0; j < NB; ++j) {
-                if constexpr (CH == 2) acc[i][j] += terms[0][i][j] + terms[1][i][j];
-                else acc[i][j] += (terms[0][i][j] + terms[1][i][j]) + (terms[2][i][j] + terms[3][i][j]);
-            }
         __builtin_amdgcn_wave_barrier();
     };
     if (begin < end) {
@@ -227,19 +230,29 @@ bool StepTakes(int64_t rows, int64_t units, int64_t inputs, int dtype) {
 
 template <typename T>
 void RunLstmStep(LstmStepArgs& p, hipStream_t stream) {
-    auto run = [&](auto acc, auto blocks, auto row_blocks) {
+    auto launch = [&](auto acc, auto blocks, auto row_blocks, auto chains) {
         using Acc = decltype(acc);
-        constexpr int NB = decltype(blocks)::value, RB = decltype(row_blocks)::value, kLds = 8 * 16 * (RB + NB) * kSmallDotPitch;
+        constexpr int NB = decltype(blocks)::value, RB = decltype(row_blocks)::value, CH = decltype(chains)::value, kLds = 8 * 16 * (RB + NB) * kSmallDotPitch;
         static_assert(kLds >= 8 * 16 * RB * (16 * NB + 4) * static_cast<int>(sizeof(Acc)), "the sums fit the staging areas");
         p.tiles_m = (p.M + 16 * RB - 1) / (16 * RB), p.tiles_n = (p.H + 4 * NB - 1) / (4 * NB);
         struct StepTag {};
-        EnsureDynamicLds<StepTag>(reinterpret_cast<const void*>(LstmStepKernel<T, Acc, NB, RB>), kLds);
-        hipLaunchKernelGGL((LstmStepKernel<T, Acc, NB, RB>), dim3(static_cast<unsigned>(p.tiles_m * p.tiles_n)), dim3(512), kLds, stream, p);
+        EnsureDynamicLds<StepTag>(reinterpret_cast<const void*>(LstmStepKernel<T, Acc, NB, RB, CH>), kLds);
+        hipLaunchKernelGGL((LstmStepKernel<T, Acc, NB, RB, CH>), dim3(static_cast<unsigned>(p.tiles_m * p.tiles_n)), dim3(512), kLds, stream, p);
         CheckLaunch("lstm_step");
     };
     using std::integral_constant;
     using One = integral_constant<int, 1>;
     using Two = integral_constant<int, 2>;
+    using Four = integral_constant<int, 4>;
+    // float32: chains of 8 terms for few rows, whose separate products are summed in short chains, and for few terms, of 16 else.  2-norm of the error of h, 64 rows, the
+    // separate calls and chains of 16 and 8: 64 units of 64 inputs 9.6e-8, 9.9e-8, 9.3e-8; 97 1.02e-7, 1.03e-7, 9.6e-8; 200 1.19e-7, 1.05e-7.  us, 16 and 8: 128 rows of 100 units 4.26 and 4.34, 4096 25.9 and 26.6.
+    const bool short_chains = std::min(p.side[0].K, p.side[1].K) < 128;
+    auto run = [&](auto acc, auto blocks, auto row_blocks) {
+        if constexpr (sizeof(T) == 4 && std::is_same_v<decltype(acc), float>) {
+            if (decltype(row_blocks)::value == 1 || short_chains) return launch(acc, blocks, row_blocks, Four{});
+        }
+        if constexpr (sizeof(T) == 2 || std::is_same_v<decltype(acc), double> || decltype(row_blocks)::value == 2) launch(acc, blocks, row_blocks, Two{});
+    };
     if constexpr (sizeof(T) == 4) {
         if (std::min(p.side[0].K, p.side[1].K) < kExactTerms) return run(0.0, One{}, Two{});
     }

@@ -77,3 +77,18 @@ def test_what_is_taken(dt, rows, n_in, units, taken):
     from chainer_amd import _host
     c, x, wx, b, h, wh = [chx.zeros(s, dt) for s in ((rows, units), (rows, n_in), (4 * units, n_in), (4 * units,), (rows, units), (4 * units, units))]
     assert (_host.lstm_step_direct(c, x, wx, b, h, wh) is not None) == taken
+
+
+@pytest.mark.parametrize('units', [64, 97, 127, 300])
+@pytest.mark.parametrize('rows', [16, 1024])
+def test_error_is_not_above_the_separate_calls(rows, units):
+    import chainer_amd as chx
+    wrong, composed = 0.0, 0.0
+    for seed in range(1024 // rows):
+        c, x, wx, b, h, wh = arrays(np.random.default_rng(seed), 'float32', rows, units, units)
+        C, X, WX, B, H, WH = [chx.array(a) for a in (c, x, wx, b, h, wh)]
+        ref = reference(c, x, wx, b, h, wh)
+        for g, s, r in zip(chx.lstm_step(C, X, WX, B, H, WH), chx.lstm(C, chx.add(chx.linear(X, WX, B), chx.linear(H, WH))), ref):
+            wrong += np.sum((g.get() - r) ** 2)
+            composed += np.sum((s.get() - r) ** 2)
+    assert wrong <= composed * 1.01  # sums over 65536 elements and more: 0.4 % of chance in either
