@@ -227,12 +227,17 @@ def resnet50_forward_fused(F, p, x):
 # `F` supplies the kernels: DeviceTrainOps below for the device, an adapter over the CPU oracle in the tests.
 # ---------------------------------------------------------------------------------------------
 class DeviceTrainOps:
-    """The call shapes resnet50_train_step uses, over the chainer_amd routines."""
+    """The call shapes resnet50_train_step uses, over the chainer_amd routines.  ``fused``: with batch norm and ReLU, ReLU's gradient
+    of a sum, and the updates as one routine each; False: the reference's routines one by one, same bits."""
 
-    def __init__(self, chx):
+    def __init__(self, chx, fused=True):
         self.c = chx
-        for name in ('conv', 'relu', 'max_pool', 'average_pool', 'linear', 'log_softmax', 'exp', 'add', 'subtract', 'multiply', 'sum',
-                     'max_pool_grad', 'average_pool_grad', 'conv_transpose', 'dot', 'batch_norm_grad', 'batch_norm_relu_grad', 'add_relu_grad', 'sgd_update'):
+        names = ('conv', 'relu', 'max_pool', 'average_pool', 'linear', 'log_softmax', 'exp', 'add', 'subtract', 'multiply', 'sum',
+                 'max_pool_grad', 'average_pool_grad', 'conv_transpose', 'dot', 'batch_norm_grad')
+        if fused:
+            names += ('batch_norm_relu_grad', 'add_relu_grad', 'sgd_update')
+            self.batch_norm_relu = self._batch_norm_relu
+        for name in names:
             setattr(self, name, getattr(chx, name))
         self.array = chx.array
         self.get = lambda a: a.get()
@@ -254,7 +259,7 @@ class DeviceTrainOps:
     def scale(self, a, s):
         return self.c.multiply(a, s)
 
-    def batch_norm_relu(self, x, gamma, beta, rm, rv, residual=None):
+    def _batch_norm_relu(self, x, gamma, beta, rm, rv, residual=None):
         return self.c.batch_norm_relu(x, gamma, beta, rm, rv, BN_EPS, 0.9, None, residual)
 
 
@@ -403,10 +408,14 @@ def lstm_lm_input(seed=5, batch=128, seq=35, vocab=10000):
     return _rng(seed + 1000).integers(0, vocab, (batch, seq)).astype(np.int32)
 
 
-def lstm_lm_forward(F, p, ids, zeros, take_mode=None, fused=False):
+def lstm_lm_forward(F, p, ids, zeros, take_mode=None, fused=False, step=None):
     """Runs the sequence; returns log-probabilities of the last step and the final (h, c) of both layers.
-    ``zeros(shape, dtype)`` makes the initial state on the same backend as ``F``.  ``fused`` calls ``F.lstm_fused`` and
-    ``F.log_softmax_fused``, which run the kernels that ``F.lstm`` and ``F.log_softmax`` of this backend run for these arrays."""
+    ``zeros(shape, dtype)`` makes the initial state on the same backend as ``F``.  ``step``: a layer's time step is one call of
+    ``F.lstm_step``, in which float16 gates are not rounded, instead of two of ``F.linear``, ``F.add`` and the cell's; None: where ``F``
+    has that routine, unless ``fused`` asks for a cell.  ``fused`` calls ``F.lstm_fused`` and ``F.log_softmax_fused``, which run the
+    kernels that ``F.lstm`` and ``F.log_softmax`` of this backend run for these arrays."""
+    if step is None:
+        step = hasattr(F, 'lstm_step') and not fused
     lstm = F.lstm_fused if fused else F.lstm
     log_softmax = F.log_softmax_fused if fused else F.log_softmax
     batch, seq = ids.shape
@@ -418,7 +427,7 @@ def lstm_lm_forward(F, p, ids, zeros, take_mode=None, fused=False):
     for t in range(seq):
         x = F.take(p['embed'], ids[:, t], 0, take_mode)
         for li, layer in enumerate(p['layers']):
-            if hasattr(F, 'lstm_step'):
+            if step:
                 hs[li], cs[li] = F.lstm_step(cs[li], x, layer['up_w'], layer['up_b'], hs[li], layer['lat_w'])
             else:
                 gates = F.add(F.linear(x, layer['up_w'], layer['up_b']), F.linear(hs[li], layer['lat_w']))

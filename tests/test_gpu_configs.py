@@ -73,3 +73,18 @@ def test_lstm_language_model():
     o2, h2, _ = cfg.lstm_lm_forward(O, p, ids, np.zeros)
     assert_close(o1.get(), o2, 1e-5, 'full-size log-probabilities', elementwise=True)
     assert_exact(chx.argmax(o1, 1).get(), O.argmax(o2, 1), 'full-size predictions')
+
+
+@pytest.mark.parametrize('vocab,units,batch,seq', [(1000, 64, 8, 5), (10000, 650, 128, 2)])
+@pytest.mark.parametrize('arguments', [{'step': False}, {'fused': True}, {'step': True}])
+def test_lstm_language_model_by_either_step(vocab, units, batch, seq, arguments):
+    """Linear, linear, add and the cell as separate calls, and as the one call that the default is, against the oracle."""
+    import chainer_amd as chx
+    from chainer_amd import configs as cfg
+    p = cfg.lstm_lm_params(vocab=vocab, units=units)
+    ids = cfg.lstm_lm_input(batch=batch, seq=seq, vocab=vocab)
+    o1, h1, c1 = cfg.lstm_lm_forward(chx, to_dev(chx, cfg, p), chx.array(ids), chx.zeros, **arguments)
+    o2, h2, c2 = cfg.lstm_lm_forward(O, p, ids, np.zeros)
+    assert_close(o1.get(), o2, 1e-5, 'log-probabilities', elementwise=True)
+    for a, r in zip(h1 + c1, h2 + c2):
+        assert_close(a.get(), r, 1e-5, 'states')

@@ -172,3 +172,22 @@ def test_resnet_training_step_matches_the_oracle():
     compare(pd, po, '')
     changed = np.abs(np.asarray(po['conv1']) - p0['conv1']).max()
     assert changed > 0, 'the step must have updated the first filters'
+
+
+def test_resnet_training_step_is_the_same_one_routine_at_a_time():
+    """configs.resnet50_train_step with the reference's routines one by one gives the bits of the fused ones: loss, updated parameters and statistics."""
+    import chainer_amd as chx
+    from chainer_amd import configs as cfg
+    results = []
+    for fused in (True, False):
+        p = cfg.tree_map(chx.array, cfg.resnet50_params_mixed(seed=3))
+        ops = cfg.DeviceTrainOps(chx, fused)
+        assert all(hasattr(ops, name) == fused for name in ('batch_norm_relu', 'batch_norm_relu_grad', 'add_relu_grad', 'sgd_update'))
+        leaves = []
+        x, t = chx.array(cfg.resnet50_input(3, 3, size=64)), chx.array(np.arange(3, dtype=np.int32))
+        leaves.append(cfg.resnet50_train_step(ops, p, x, t, 0.05).get())
+        cfg.tree_map(lambda a: leaves.append(a.get()), p)
+        results.append(leaves)
+    assert len(results[0]) == len(results[1]) > 161
+    for a, b in zip(*results):
+        np.testing.assert_array_equal(a, b)
