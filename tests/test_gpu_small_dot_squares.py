@@ -46,3 +46,13 @@ def test_views_and_special_values(dt):
     bad = np.zeros(got.shape, bool)
     bad[5], bad[:, 77] = True, True
     assert np.isnan(got[5]).all() and (~np.isfinite(got[:, 77])).all() and np.isfinite(got[~bad]).all()
+
+
+@pytest.mark.parametrize('m,k,n', [(128, 650, 10000), (512, 1000, 1000), (670, 3324, 2007), (994, 385, 807)])
+def test_error_of_chains_of_sixteen(m, k, n):
+    """Only these tiles sum float32 in chains of 16 products: 1.0e-7 to 1.6e-7 of the norm, where one chain to a wave has 2.7e-7 and 7.3e-7 at 650 and 3324 terms."""
+    import chainer_amd as chx
+    rng = np.random.default_rng(k)
+    x, w = rng.standard_normal((m, k), dtype=np.float32), rng.standard_normal((n, k), dtype=np.float32)
+    ref = x.astype('float64') @ w.astype('float64').T
+    assert np.linalg.norm(chx.linear(chx.array(x), chx.array(w), None).get() - ref) < 1.8e-7 * np.linalg.norm(ref)

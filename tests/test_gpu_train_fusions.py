@@ -93,3 +93,29 @@ def test_sgd_update(sizes):
     same(chx.sgd_update([p], [g.astype('float32')], 0.5)[0], chx.subtract(p, chx.multiply(g.astype('float32'), 0.5)))
     with pytest.raises(chx.DimensionError):
         chx.sgd_update([p], [g, g], 0.5)
+
+
+@pytest.mark.parametrize('dt,pt', [('float32', 'float32'), ('float16', 'float32'), ('float16', 'float16'), ('float64', 'float64')])
+@pytest.mark.parametrize('shape', SHAPES)
+def test_batch_norm_relu_is_one_call(dt, pt, shape):
+    """Arrays of the tests above run on the dedicated kernels, not on the routines that they are compared with."""
+    from chainer_amd import _host
+    c = shape[1]
+    x, r, g, (gamma, beta, mean, var) = chx.zeros(shape, dt), chx.zeros(shape, dt), chx.zeros(shape, dt), [chx.ones((c,), pt) for _ in range(4)]
+    for residual in (None, r):
+        y, total, state = _host.batch_norm_direct(x, gamma, beta, mean, var, 2e-5, 0.9, None, True, residual)
+        assert y.shape == shape and (total is None) == (residual is None)
+    assert len(_host.batch_norm_grad_direct(x, gamma, g, *state, None, beta)) == 3
+
+
+def test_which_calls_are_composed():
+    from chainer_amd import _host
+    x, p = chx.zeros((5, 6, 7, 4), 'float32'), [chx.ones((6,), 'float32') for _ in range(4)]
+    y = chx.zeros((5, 7, 4, 6), 'float32').transpose(0, 3, 1, 2)
+    state = _host.batch_norm_direct(x, *p, 2e-5, 0.9, None, True, None)[2]
+    assert _host.batch_norm_direct(y, *p, 2e-5, 0.9, None, True, None) is None and _host.batch_norm_direct(x, *p, 2e-5, 0.9, None, True, y) is None
+    assert _host.batch_norm_grad_direct(x, p[0], y, *state, None, p[1]) is None and _host.batch_norm_grad_direct(x, p[0], x, *state, None, p[1].astype('float64')) is None
+    assert _host.add_relu_grad_direct(x, x, x) is not None and _host.add_relu_grad_direct(y, x[:, :, :, ::-1], x) is not None
+    assert _host.add_relu_grad_direct(x, x[:, :1], x) is None and _host.add_relu_grad_direct(x, x.astype('float16'), x) is None
+    assert len(_host.sgd_update_direct([x, y], [x, x.reshape((-1,))], 0.5)) == 2 and _host.sgd_update_direct([], [], 0.5) == []
+    assert _host.sgd_update_direct([x], [x.astype('float16')], 0.5) is None and _host.sgd_update_direct([x], [x], x[0, 0, 0, 0]) is None
