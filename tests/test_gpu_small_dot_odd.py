@@ -30,3 +30,16 @@ def test_products(m, k, n):
     check(chx, x[ok, :k], w[1:-1, :k], X[ok, :k], W[1:-1, :k], 'rows of a wider array')
     check(chx, x[ok, 1:], w[1:-1, 1:], X[ok, 1:], W[1:-1, 1:], 'rows that start at odd elements')
     check(chx, x[ok, 1:], w[1:-1, :k], X[ok, 1:], W[1:-1, :k], 'one of each')
+
+
+@pytest.mark.parametrize('m,k,n', [(1, 8, 40), (1, 9, 40), (2, 15, 33), (2, 1001, 1000), (2, 1000, 2560), (2, 1000, 2561), (1, 64, 10000), (1, 771, 2559), (3, 3071, 1000)])
+def test_few_rows_between_what_is_not_a_number(m, k, n):
+    import chainer_amd as chx
+    rng = np.random.default_rng(m + k + n)
+    for first_x, first_w in ((0, 0), (1, 1), (1, 0), (0, 1)):  # even and odd elements
+        x, w = [np.full((rows + 2, k + 2), np.nan, 'float16') for rows in (m, n)]
+        of_x, of_w = np.s_[1:-1, first_x:first_x + k], np.s_[1:-1, first_w:first_w + k]
+        x[of_x], w[of_w] = [rng.standard_normal((rows, k)).astype('float16') for rows in (m, n)]
+        X, W = chx.array(x)[of_x], chx.array(w)[of_w]
+        assert X.shape == (m, k) and W.shape == (n, k)
+        check(chx, x[of_x], w[of_w], X, W, 'starts %d and %d' % (first_x, first_w))
