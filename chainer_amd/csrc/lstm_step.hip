@@ -244,8 +244,9 @@ void RunLstmStep(LstmStepArgs& p, hipStream_t stream) {
     using One = integral_constant<int, 1>;
     using Two = integral_constant<int, 2>;
     using Four = integral_constant<int, 4>;
-    // float32: chains of 8 terms for few rows, whose separate products are summed in short chains, and for few terms, of 16 else.  2-norm of the error of h, 64 rows, the
-    // separate calls and chains of 16 and 8: 64 units of 64 inputs 9.6e-8, 9.9e-8, 9.3e-8; 97 1.02e-7, 1.03e-7, 9.6e-8; 200 1.19e-7, 1.05e-7.  us, 16 and 8: 128 rows of 100 units 4.26 and 4.34, 4096 25.9 and 26.6.
+    // float32: chains of 8 terms for few rows, whose separate products are summed in short chains, and for few terms, of 16 else.  2-norm of the error of h, 64 rows,
+    // the separate calls and chains of 16 and 8: 64 units of 64 inputs 9.6e-8, 9.9e-8, 9.3e-8; 97 of 97 1.02e-7, 1.03e-7, 9.6e-8; 200 of 200, in chains of 16, 1.19e-7,
+    // 1.05e-7.  us, 16 and 8: 128 rows of 100 units 4.26 and 4.34, 4096 of 127 25.9 and 26.6.
     const bool short_chains = std::min(p.side[0].K, p.side[1].K) < 128;
     auto run = [&](auto acc, auto blocks, auto row_blocks) {
         if constexpr (sizeof(T) == 4 && std::is_same_v<decltype(acc), float>) {

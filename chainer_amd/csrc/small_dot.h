@@ -599,16 +599,17 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
 }
 
-// The reduction is dealt out in chunks of 128 bytes per row.  Pieces are loaded as whole lines
-// and turned round through a piece of LDS that belongs to the wave (no barrier); elements come as they are used.  Two chunks are in flight
-// while a third is multiplied.  [20,2600] . [2600,650] float32, row-major b: 34 -> 9.3 us (several workgroups per tile and the pass over
-// their sums included), [64,333] . [333,777] float16 8.5 -> 6.4.
-template <typename T, int AM, int BM, int P>
+// At least one operand element by element.  The reduction is dealt out in chunks of 32 bytes per row, which come as they are used, six of them in flight, or, where
+// the other operand's are float16 rows of odd pitch, of 128 bytes, two in flight: these are loaded as whole lines and turned round through a piece of LDS that
+// belongs to the wave (no barrier).  [20,2600] . [2600,650] float32, row-major b: 34 -> 9.3 us (several workgroups per tile and the pass over their sums included).
+template <typename T, int AM, int BM>
 __global__ __launch_bounds__(64 * kSmallDotMaxWaves) __attribute__((amdgpu_waves_per_eu(3, 8))) void SmallDotMixedKernel(SmallDotArgs p) {
+    static_assert(AM == kElements || BM == kElements);
     constexpr int PL = 16 / sizeof(T);
+    constexpr bool A_LDS = AM == kOddPieces, B_LDS = BM == kOddPieces;
+    constexpr int P = A_LDS || B_LDS ? 4 : 1;
     constexpr int KC = 2 * P * PL;      // k per chunk
     constexpr int D = P == 1 ? 6 : 2;   // chunks in flight
-    constexpr bool A_LDS = P == 4 && AM != kElements, B_LDS = P == 4 && BM != kElements;
     extern __shared__ __align__(16) char lds[];
 
     const int tid = threadIdx.x;
@@ -633,7 +634,7 @@ __global__ __launch_bounds__(64 * kSmallDotMaxWaves) __attribute__((amdgpu_waves
         a_line[j] = line_of(tm * 32 + (A_LDS ? j * 8 + sub : lr), p.M, p.a_row);
         b_line[j] = line_of(tn * 32 + (B_LDS ? j * 8 + sub : lr), p.N, p.b_col);
     }
-    char* const stage = lds + wave * ((A_LDS ? kSmallDotStage : 0) + (B_LDS ? kSmallDotStage : 0));
+    char* const stage = lds + wave * kSmallDotStage;
 
     // this wave's chunks
     const int chunks = (p.K + KC - 1) / KC;
@@ -648,7 +649,7 @@ __global__ __launch_bounds__(64 * kSmallDotMaxWaves) __attribute__((amdgpu_waves
     SmallDotShare<P> av[D], bv[D];
     auto load_operand = [&](auto mode_tag, SmallDotShare<P>& x, __amdgpu_buffer_rsrc_t r, const int (&line)[4], int ks, int c) {
         constexpr int MODE = decltype(mode_tag)::value;
-        constexpr bool LDS = P == 4 && MODE != kElements;
+        constexpr bool LDS = MODE == kOddPieces;
         const int k0 = c * KC + (LDS ? piece * PL : g * P * PL);
         if (MODE == kPieces || (MODE == kOddPieces && (c + 1) * KC <= p.K)) {
 #pragma unroll
@@ -663,38 +664,31 @@ __global__ __launch_bounds__(64 * kSmallDotMaxWaves) __attribute__((amdgpu_waves
         load_operand(std::integral_constant<int, BM>{}, bv[i], br, b_line, b_ks, c);
     };
     // the chunk in the MFMA layout: lane (lr, g) holds pieces g * P .. of its row
-    auto arrange = [&](auto mode_tag, SmallDotShare<P>& x, char* area, int c) {
+    auto arrange = [&](auto mode_tag, SmallDotShare<P>& x, int c) {
         constexpr int MODE = decltype(mode_tag)::value;
-        constexpr bool LDS = P == 4 && MODE != kElements;
-        if (MODE == kPieces && (c + 1) * KC > p.K) {
-            const int k0 = c * KC + (LDS ? piece * PL : g * P * PL);
+        if (MODE == kPieces && (c + 1) * KC > p.K) x.v[0] = MaskPiece<T>(x.v[0], c * KC + g * PL, p.K);
+        if constexpr (MODE == kOddPieces) {
 #pragma unroll
-            for (int j = 0; j < P; ++j) x.v[j] = MaskPiece<T>(x.v[j], k0 + (LDS ? 0 : j * PL), p.K);
-        }
-        if constexpr (LDS) {
-#pragma unroll
-            for (int j = 0; j < P; ++j) *reinterpret_cast<Bytes16*>(area + (j * 8 + sub) * kSmallDotPitch + piece * 16) = x.v[j];
+            for (int j = 0; j < P; ++j) *reinterpret_cast<Bytes16*>(stage + (j * 8 + sub) * kSmallDotPitch + piece * 16) = x.v[j];
         }
     };
-    auto fragment = [&](bool in_lds, const SmallDotShare<P>& x, const char* area, int j) {
-        return in_lds ? *reinterpret_cast<const Bytes16*>(area + lr * kSmallDotPitch + (g * P + j) * 16) : x.v[j];
+    auto fragment = [&](bool in_lds, const SmallDotShare<P>& x, int j) {
+        return in_lds ? *reinterpret_cast<const Bytes16*>(stage + lr * kSmallDotPitch + (g * P + j) * 16) : x.v[j];
     };
     auto multiply = [&](int i, int c, auto&& next) {
-        char* const b_area = stage + (A_LDS ? kSmallDotStage : 0);
-        arrange(std::integral_constant<int, AM>{}, av[i], stage, c);
-        arrange(std::integral_constant<int, BM>{}, bv[i], b_area, c);
+        arrange(std::integral_constant<int, AM>{}, av[i], c);
+        arrange(std::integral_constant<int, BM>{}, bv[i], c);
         if constexpr (A_LDS || B_LDS) __builtin_amdgcn_wave_barrier();
         Bytes16 fa[P], fb[P];
 #pragma unroll
         for (int j = 0; j < P; ++j) {
-            fa[j] = fragment(A_LDS, av[i], stage, j);
-            fb[j] = fragment(B_LDS, bv[i], b_area, j);
+            fa[j] = fragment(A_LDS, av[i], j);
+            fb[j] = fragment(B_LDS, bv[i], j);
         }
-        if constexpr (A_LDS && B_LDS) next();  // (else the registers of a chunk are its fragments)
         if constexpr (A_LDS || B_LDS) __builtin_amdgcn_wave_barrier();
 #pragma unroll
         for (int j = 0; j < P; ++j) MfmaTile<T>(fa[j], fb[j], acc);
-        if constexpr (!(A_LDS && B_LDS)) next();
+        next();  // (into the registers that were this chunk's fragments)
     };
     if (begin < end) {
 #pragma unroll

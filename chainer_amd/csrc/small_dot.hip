@@ -73,20 +73,15 @@ bool SmallDotOperands(const hipcx_array* a, const hipcx_array* b, SmallDotArgs* 
     return true;
 }
 
-template <typename T, int AM, int BM, int P>
-void LaunchSmallDotPieces(const SmallDotArgs& p, dim3 grid, hipStream_t stream) {
-    constexpr int kWaveBytes = std::max<int>((P == 4) * ((AM != kElements) + (BM != kElements)) * kSmallDotStage, kSmallDotPart * sizeof(float));
-    struct SmallDotTag {};
-    EnsureDynamicLds<SmallDotTag>(reinterpret_cast<const void*>(SmallDotMixedKernel<T, AM, BM, P>), kSmallDotMaxWaves * kWaveBytes);
-    hipLaunchKernelGGL((SmallDotMixedKernel<T, AM, BM, P>), grid, dim3(64 * p.nw), p.nw * kWaveBytes, stream, p);
-    CheckLaunch("small_dot_mixed");
-}
-
 // Elements come as they are used: chunks of 32 bytes, six of them in flight, beat whole lines ([32,1000] . [1000,2048] float16 14.3 -> 5.5 us,
 // [200,4000] . [4000,4000] 174 -> 51, [20,2600] . [2600,650] float32 13.4 -> 9.3); rows of odd pitch gain from whole lines at any size.
 template <typename T, int AM, int BM>
 void LaunchSmallDotMixed(const SmallDotArgs& p, dim3 grid, hipStream_t stream) {
-    LaunchSmallDotPieces<T, AM, BM, AM != kOddPieces && BM != kOddPieces ? 1 : 4>(p, grid, stream);
+    constexpr int kWaveBytes = std::max<int>(AM == kOddPieces || BM == kOddPieces ? kSmallDotStage : 0, kSmallDotPart * sizeof(float));
+    struct SmallDotTag {};
+    EnsureDynamicLds<SmallDotTag>(reinterpret_cast<const void*>(SmallDotMixedKernel<T, AM, BM>), kSmallDotMaxWaves * kWaveBytes);
+    hipLaunchKernelGGL((SmallDotMixedKernel<T, AM, BM>), grid, dim3(64 * p.nw), p.nw * kWaveBytes, stream, p);
+    CheckLaunch("small_dot_mixed");
 }
 
 // Columns, in 16s, of the tiles of whole lines regrouped through LDS (SmallDotLinesKernel); 0: loads straight into the MFMA layout (SmallDotKernel) are
