@@ -359,7 +359,10 @@ __global__ __launch_bounds__(64 * kSmallDotMaxWaves) __attribute__((amdgpu_waves
 #pragma unroll
             for (int j = 0; j < BL; ++j) bv[st][j] = __builtin_amdgcn_raw_buffer_load_b128(br, b_line[j], c * 128, 0);
         } else {
-            const int at = c * 128 - PieceEarly<T>(c * KC + piece * PL, p.K) * static_cast<int>(sizeof(T));
+            int at = c * 128;
+            bool in = true;
+            if constexpr (sizeof(T) == 2) at -= PieceEarly<T>(c * KC + piece * PL, p.K) * static_cast<int>(sizeof(T));
+            else in = c * KC + piece * PL < p.K;  // (rows of whole dwords: pieces beyond K are not read, what lies behind it in one is masked)
 #pragma unroll
             for (int j = 0; j < 4; ++j) av[st][j] = __builtin_amdgcn_raw_buffer_load_b128(ar, a_line[j] != kOut ? a_line[j] + at : kOut, 0, 0);
 #pragma unroll
@@ -368,7 +371,12 @@ __global__ __launch_bounds__(64 * kSmallDotMaxWaves) __attribute__((amdgpu_waves
     };
     auto multiply = [&](int st, int c, auto&& next) {
         if ((c + 1) * KC > p.K) {
-            const int early = PieceEarly<T>(c * KC + piece * PL, p.K);
+            auto keep = [&](Bytes16 v) {
+                // float32 by masks: by early pieces it takes 146 registers with two blocks, not 128, and a compute unit has no room for a second workgroup of eight waves
+                // ([135,896] . [896,3209] 13.8 us, 16.3)
+                if constexpr (sizeof(T) == 2) return KeepPiece<T>(v, PieceEarly<T>(c * KC + piece * PL, p.K));
+                else return MaskPiece<T>(v, c * KC + piece * PL, p.K);
+            };
 #pragma unroll
             for (int j = 0; j < 4; ++j) av[st][j] = KeepPiece<T>(av[st][j], early);
 #pragma unroll
