@@ -12,7 +12,7 @@
 //   SmallDotMixedKernel   an operand whose k axis is not the unit-stride one (dG . Wh of a recurrent network, x^T . gy).
 //   SmallDotColumnsKernel float32, both operands with m and n as the unit-stride axes, of outputs that make a 64 x 64 tile per compute unit.
 //   SmallDotVectorKernel  M <= 4 (one image, one sentence): a wave per output column, K across the lanes, where the MFMA would work on
-//                         32 rows (float16: of few columns).
+//                         32 rows (float16: of few columns or many terms).
 // For float the reduction index is dealt to the v_mfma_f32_32x32x2_f32 steps so that a lane's four steps use four consecutive k (one
 // 16-byte load when k is the contiguous axis of the operand); for float16 a lane's v_mfma_f32_32x32x16_f16 operand is 8 consecutive k.
 // Rows / columns beyond M / N and the tail of K are served as zeros by the buffer bounds check or explicit masks.
@@ -364,9 +364,9 @@ __global__ __launch_bounds__(64 * kSmallDotMaxWaves) __attribute__((amdgpu_waves
             if constexpr (sizeof(T) == 2) at -= PieceEarly<T>(c * KC + piece * PL, p.K) * static_cast<int>(sizeof(T));
             else in = c * KC + piece * PL < p.K;  // (rows of whole dwords: pieces beyond K are not read, what lies behind it in one is masked)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) av[st][j] = __builtin_amdgcn_raw_buffer_load_b128(ar, a_line[j] != kOut ? a_line[j] + at : kOut, 0, 0);
+            for (int j = 0; j < 4; ++j) av[st][j] = __builtin_amdgcn_raw_buffer_load_b128(ar, (in & (a_line[j] != kOut)) ? a_line[j] + at : kOut, 0, 0);
 #pragma unroll
-            for (int j = 0; j < BL; ++j) bv[st][j] = __builtin_amdgcn_raw_buffer_load_b128(br, b_line[j] != kOut ? b_line[j] + at : kOut, 0, 0);
+            for (int j = 0; j < BL; ++j) bv[st][j] = __builtin_amdgcn_raw_buffer_load_b128(br, (in & (b_line[j] != kOut)) ? b_line[j] + at : kOut, 0, 0);
         }
     };
     auto multiply = [&](int st, int c, auto&& next) {
@@ -378,9 +378,9 @@ __global__ __launch_bounds__(64 * kSmallDotMaxWaves) __attribute__((amdgpu_waves
                 else return MaskPiece<T>(v, c * KC + piece * PL, p.K);
             };
 #pragma unroll
-            for (int j = 0; j < 4; ++j) av[st][j] = KeepPiece<T>(av[st][j], early);
+            for (int j = 0; j < 4; ++j) av[st][j] = keep(av[st][j]);
 #pragma unroll
-            for (int j = 0; j < BL; ++j) bv[st][j] = KeepPiece<T>(bv[st][j], early);
+            for (int j = 0; j < BL; ++j) bv[st][j] = keep(bv[st][j]);
         }
 #pragma unroll
         for (int j = 0; j < 4; ++j) *reinterpret_cast<Bytes16*>(to + j * 8 * kSmallDotPitch) = av[st][j];

@@ -261,11 +261,15 @@ SmallDotPath PlanSmallDot(const hipcx_array* a, const hipcx_array* b, SmallDotAr
         if (sizeof(T) == 4 || ((M + 127) / 128) * ((N + 127) / 128) >= 128) return kNoSmallDot;
     }
     if (*a_mode != kPieces || *b_mode != kPieces) return kSmallDotTiles;
-    // A wave to a column: float32 whatever its size, whose lanes' sums are short.  float16, whose products cost two conversions each there, where the columns are few and
-    // so are the rows, or the terms are many; us, tiles and waves: [1,1000] . [1000,1000] 4.7 3.6, [2,2048] . [2048,2048] 5.7 4.6, [4,4096] . [4096,1000] 7.5
-    // 6.6; [4,332] . [332,3333] 3.7 8.0, [4,1000] . [1000,10000] 6.2 14.8, [1,1000] . [1000,10000] 6.1 7.1, [4,1000] . [1000,1000] 4.7 4.9.  Not for few terms in
-    // float32: a product is rounded before it is added there, 4.4e-8 of the norm for three terms where a chain of the matrix pipe has 3.7e-8.
-    if (M <= 4 && (sizeof(T) == 4 ? K >= 64 : N <= 2560 && (M <= 2 || K >= 3072))) return kSmallDotVector;
+    if (M <= 4) {
+        // A wave to a column.  float32 whatever its size, whose lanes' sums are short, but not few terms: a product is rounded before it is added there, 4.4e-8 of the norm
+        // for three terms where a chain of the matrix pipe has 3.7e-8.  float16, whose products cost two conversions each there and which the tiles take as fast for ten
+        // thousand columns as for one thousand, where the columns are few or the terms many.  us, tiles and waves, one row: [1,512] . [512,3000] 3.8 3.8, [1,1000] . [1000,5000]
+        // 4.7 4.5, 6000 columns 4.7 4.8, 10000 5.5 6.4, [1,2048] . [2048,10000] 9.2 8.6; two: [2,1000] . [1000,2561] 4.3 4.6, [2,2048] . [2048,4000] 5.3 5.2, 6000 6.1 6.5;
+        // four: [4,1000] . [1000,1000] 4.2 4.2, [4,2048] . [2048,1000] 5.1 4.2, 2000 5.2 5.3, [4,3000] . [3000,500] 5.9 5.6, 2000 6.0 7.7, [4,332] . [332,3333] 3.3 7.1.
+        const int64_t most = sizeof(T) == 4 ? (K >= 64 ? N : 0) : M > 2 ? (K >= 2048 ? 1280 : 0) : std::max<int64_t>(2560, M == 1 ? 28 * K / 5 : 5 * K / 2);
+        if (N <= most) return kSmallDotVector;
+    }
     return 2.0 * M * N * K >= 1e9 ? kSmallDotWhole : kSmallDotTiles;  // enough tiles, or enough of them long, to keep the chip busy
 }
 

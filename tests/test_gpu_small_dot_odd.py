@@ -43,3 +43,12 @@ def test_few_rows_between_what_is_not_a_number(m, k, n):
         X, W = chx.array(x)[of_x], chx.array(w)[of_w]
         assert X.shape == (m, k) and W.shape == (n, k)
         check(chx, x[of_x], w[of_w], X, W, 'starts %d and %d' % (first_x, first_w))
+
+
+@pytest.mark.parametrize('m,k,n', [(1, 1000, 5600), (1, 1000, 5601), (1, 457, 2560), (1, 457, 2561), (2, 1030, 2575), (2, 1030, 2576), (3, 2048, 1280), (4, 2048, 1281),
+                                   (4, 2047, 700), (3, 2047, 1281), (4, 3072, 2001)])
+def test_limits_of_the_rule_for_few_rows(m, k, n):
+    import chainer_amd as chx
+    rng = np.random.default_rng(m + k + n)
+    x, w = [rng.standard_normal((rows, k)).astype('float16') for rows in (m, n)]
+    check(chx, x, w, chx.array(x), chx.array(w), 'dense')
