@@ -471,15 +471,15 @@ ShiftedPlan PlanShifted(const GradWeightPlan& pl, int dtype, bool pairs) {
     // worth it when kw copies of rows of whole granules are smaller than the kh*kw-fold Im2Col, also where it is two copies of shorter rows: small planes and
     // filters are faster as one Dot.  us, Im2Col and two copies: 2x2 on 7 x 7 8.7 and 15.8, 3x3 on 9 x 3 10.5 and 19.1, 5x5 on 13 x 3 99 and 214.
     if (g.kw * Hp * ((W + 2 * pw + epc - 1) / epc * epc) >= static_cast<int64_t>(g.kh) * g.kw * g.OH * g.OW) return sp;
-    const int64_t most = int64_t{1} << 31;
-    if (static_cast<int64_t>(g.H) * W == 0 || pitch_x + 256 * epc >= most || N * g.C >= most || N * g.K >= most) return sp;  // (the copy kernel's 32-bit indices)
+    const int64_t most = int64_t{1} << 31, planes = N * (static_cast<int64_t>(g.C) + g.K);
+    if (static_cast<int64_t>(g.H) * W == 0 || planes == 0 || pitch_x + 256 * epc >= most || N * g.C >= most || N * g.K >= most) return sp;  // (the copy kernel's 32-bit indices)
     sp.a.set[0] = PlaneSet{g.x, nullptr, static_cast<int>(N * g.C), g.H, g.W, g.ph, g.pw, static_cast<int>(copies), static_cast<int>(pitch_x)};
     sp.a.set[1] = PlaneSet{g.gy, nullptr, static_cast<int>(N * g.K), g.OH, g.OW, 0, 0, 1, static_cast<int>(pitch_gy)};
     sp.a.Wp = static_cast<int>(Wp);
     sp.a.images = g.N, sp.a.channels = g.C;
     sp.a.pairs = Wp % 2 == 0 && g.OW >= 2;
     // A piece to a thread: planes together, or less where that leaves compute units without a workgroup, or parts of a plane; two pieces once the chip is full.
-    const int64_t pieces = pitch_x / epc, planes = N * (static_cast<int64_t>(g.C) + g.K), cus = NumCUs();
+    const int64_t pieces = pitch_x / epc, cus = NumCUs();
     sp.a.each = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>({kMostPlanes, (planes * pieces >= 4096 * cus ? 512 : 256) / pieces, planes / cus})));
     sp.a.parts = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>((pieces + 255) / 256, 8 * cus / planes)));
     sp.a.share = static_cast<int>((pieces + sp.a.parts - 1) / sp.a.parts);
