@@ -1189,6 +1189,7 @@ int hipcx_conv_route(const hipcx_array* x, const hipcx_array* w, const hipcx_arr
     try {
         if (x == nullptr || w == nullptr || out == nullptr || stride == nullptr || pad == nullptr) return -1;
         if (x->ndim != 4 || w->ndim != 4 || out->ndim != 4) return -1;
+        if (TotalSize(out) == 0) return 0;  // nothing runs
         if (PlanPw(x, w, b, out, stride, pad).ok) return 3;
         if (const NchwPlan pl = PlanNchw(x, w, out, stride, pad); pl.ok) {
             const NchwConvArgs a = NchwExtents(x, w, out, stride);

@@ -35,6 +35,7 @@ print(sorted(answers))
 @pytest.mark.parametrize('question,answers', [
     ('lib.hipcx_conv_grad_weight_workspace_size(x, y, filters, one, pad, 0) >= 0', '[True]'),
     ('lib.hipcx_conv_workspace_size(x, filters, y) >= 0', '[True]'),
+    ('lib.hipcx_conv_route(x, filters, None, one, pad, y) if 0 in (n, k, h, w) else 0', '[0]'),
 ])
 def test_empty_arrays(question, answers):
     done = subprocess.run([sys.executable, '-c', ASK % question], cwd=ROOT, capture_output=True, text=True)
