@@ -56,16 +56,17 @@ bool SmallDotOperands(const hipcx_array* a, const hipcx_array* b, SmallDotArgs* 
     p->b_col = b->strides[1] / it;
     int64_t a_span = ((M - 1) * p->a_row + (K - 1) * p->a_k + 1) * it, b_span = ((K - 1) * p->b_k + (N - 1) * p->b_col + 1) * it;
     if (a_span >= (1LL << 31) - 256 || b_span >= (1LL << 31) - 256) return false;
-    auto mode = [&](const void* ptr, int64_t k_stride, int64_t line_stride, int64_t* span) {
+    // (the stride of an axis of length one says nothing: a reshaped row may have any)
+    auto mode = [&](const void* ptr, int64_t k_stride, int64_t lines, int64_t line_stride, int64_t* span) {
         if (k_stride != 1 && K > 1) return static_cast<int>(kElements);
-        if (reinterpret_cast<uintptr_t>(ptr) % 4 == 0 && line_stride * it % 4 == 0) {
+        if (reinterpret_cast<uintptr_t>(ptr) % 4 == 0 && (lines == 1 || line_stride * it % 4 == 0)) {
             *span = (*span + 3) / 4 * 4;  // a last half element shares its (aligned) dword with the two bytes behind it
             return static_cast<int>(kPieces);
         }
         return static_cast<int>(kOddPieces);
     };
-    *a_mode = mode(a->data, p->a_k, p->a_row, &a_span);
-    *b_mode = mode(b->data, p->b_k, p->b_col, &b_span);
+    *a_mode = mode(a->data, p->a_k, M, p->a_row, &a_span);
+    *b_mode = mode(b->data, p->b_k, N, p->b_col, &b_span);
     p->a_bytes = static_cast<unsigned>(a_span);
     p->b_bytes = static_cast<unsigned>(b_span);
     p->tiles_m = static_cast<int>((M + 31) / 32);

@@ -52,3 +52,19 @@ def test_limits_of_the_rule_for_few_rows(m, k, n):
     rng = np.random.default_rng(m + k + n)
     x, w = [rng.standard_normal((rows, k)).astype('float16') for rows in (m, n)]
     check(chx, x, w, chx.array(x), chx.array(w), 'dense')
+
+
+@pytest.mark.parametrize('k,n', [(2048, 1000), (1000, 2560), (1000, 5600), (2048, 1), (1001, 1), (7, 1)])
+def test_stride_of_a_single_row_or_column_says_nothing(k, n):
+    import chainer_amd as chx
+    rng = np.random.default_rng(k + n)
+    x, w = rng.standard_normal((1, k)).astype('float16'), rng.standard_normal((n, k)).astype('float16')
+    X, W = chx.array(np.pad(x, ((0, 0), (0, 1 + k % 2))))[:, :k], chx.array(np.pad(w, ((0, 0), (0, 2 - k % 2))))[:, :k]  # rows of even pitch
+    rows = [chx.array(x.reshape(1, k, 1, 1)).reshape((1, k)), chx.array(x), X]
+    assert len({r.strides for r in rows}) > 1
+    columns = [W] if n > 1 else [W, chx.array(w), chx.array(w.reshape(1, k, 1, 1)).reshape((1, k))]
+    expect = chx.dot(X, W.T).get()
+    check(chx, x, w, X, W, 'even pitch')
+    for r in rows:
+        for c in columns:  # the same kernel: the same bits
+            np.testing.assert_array_equal(chx.dot(r, c.T).get(), expect)
