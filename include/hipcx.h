@@ -318,7 +318,7 @@ int64_t hipcx_conv_out_dim(int64_t in_dim, int64_t kernel_size, int64_t stride, 
  * (CX/native/native_device/conv.cc:78-84), which this entry also accepts as `out`. */
 size_t hipcx_conv_workspace_size(const hipcx_array* x, const hipcx_array* w, const hipcx_array* out);
 /* Which kernel family hipcx_conv runs for these arguments (no counterpart in the reference: for tests and benchmarks that must
- * know that a specialised kernel, not the general one, produced a result).  0: general implicit GEMM (any dtype / layout);
+ * know that a specialised kernel, not the general one, produced a result).  0: general implicit GEMM (any dtype / layout), or an empty result;
  * 1: float16 NCHW kernels with 128-wide tiles; 2: float16 7x7 / 2 stem kernel; 3: float16 1x1 / stride 1 kernel that loads its
  * operands straight into LDS and walks 256 x 128 tiles; 4: float16 NCHW kernel for few output pixels, 32 x 32 tiles; 5: float32 and
  * float16 kernel for sums of at most 32 terms; 6: float32 3x3 kernel for few output tiles, NCHW read in place; 7: float16 NCHW 3x3
